@@ -44,6 +44,24 @@ def test_selective_scan_forms(new, ctx, Ch, N, heads, groups):
     torch.testing.assert_close(a["ssm_state"], b["ssm_state"], atol=1e-4, rtol=1e-4)
 
 
+@pytest.mark.parametrize("Ch,N,heads", [(1024, 16, 0), (256, 128, 4)])
+def test_continued_sequences_of_many_chunks(Ch, N, heads):
+    # the first chunk starts from the slot into which the last one leaves its state, here as soon as it has walked one token
+    new, ctx = [97, 129, 161, 225, 257], [4, 1, 0, 9, 3]
+    a = _scan_inputs(new, ctx, Ch, N, heads, 1, torch.float32, 11)
+    names = ("u", "delta", "A", "B", "C", "D", "z", "delta_bias", "ssm_state")
+    b = {k: v.clone() if isinstance(v, torch.Tensor) else v for k, v in a.items()}
+    want = R.selective_scan(*(b[k] for k in names), b["query_start_loc"], b["seq_lens"], b["block_table"])
+    first = a["ssm_state"].clone()
+    ys = []
+    for _ in range(3):
+        a["ssm_state"].copy_(first)
+        ys.append(ops.selective_scan(**a, max_query_len=max(new)))
+        torch.testing.assert_close(a["ssm_state"], b["ssm_state"], atol=1e-4, rtol=1e-4)
+    torch.testing.assert_close(ys[0], want, atol=3e-4, rtol=1e-4)          # as in test_selective_scan_forms
+    assert torch.equal(ys[0], ys[1]) and torch.equal(ys[0], ys[2])
+
+
 def test_rows_off_a_pair_boundary_take_the_plain_form():
     new, ctx = [130, 4], [0, 1]
     a = _scan_inputs(new, ctx, 64, 16, 0, 1, torch.bfloat16, 3, offset=1)

@@ -277,6 +277,8 @@ __global__ __launch_bounds__(256) void scan_combine_kernel(float* __restrict__ w
 // states' B and C serves eight updates.  NL = N / 16 lanes share the states of a pair, lane q of them the groups of four
 // q, q + NL, q + 2 NL, q + 3 NL: their state accesses are contiguous.
 // A chunk's product of decays is exp2(a * sum of dt): the workspace holds the sum, not the product.
+// The output pass of several chunks reads its start states from the workspace alone: the last chunk leaves its end state in
+// the request's slot while the first one may not have begun, so the carry kernel puts the slot's state aside first.
 // Bound by vector issue: per state and token exp2 (4 slots), its argument, two for the state and one for y.
 // 3325 tokens of 8192 channels x 16 states, three sequences: both passes 637 -> 320 us (the exponentials alone are 90);
 // 1100 tokens of 64 heads x 64 x 128 states: 990 -> 283 with the convolution.
@@ -292,7 +294,9 @@ struct ScanArgs {
   const int *qsl, *seq_lens, *block_table;
   long bt_stride, u_stride, d_stride, b_stride, c_stride, z_stride, o_stride;
   int Ch, dt_div, group_ch, softplus, chunk, tile;      // tile: tokens staged at a time
-  float *ws_dt, *ws_h;                                  // [S, chunks, Ch] sums of dt; [S, chunks, Ch, N] states
+  // [S, chunks, Ch] sums of dt; [S, chunks, Ch, N] states: of a sequence's chunks but the last their end states, in the last
+  // one's place the state that the sequence starts from
+  float *ws_dt, *ws_h;
 };
 constexpr int SCAN_LDS = 8192;                          // floats of staged B and C
 
@@ -330,6 +334,8 @@ __global__ __launch_bounds__(256) void scan_pairs_kernel(ScanArgs p) {
       const int at = v * N + 4 * j * NL;
       if (!ASC) a[v][j] = *reinterpret_cast<const f32x4*>(p.A + (long)c * N + 4 * part + at) * LOG2E;
       if (MODE == 2 && kch > 0) h[v][j] = *reinterpret_cast<const f32x4*>(p.ws_h + (wc - p.Ch) * N + 4 * part + at);
+      else if (MODE == 2 && from_state && nch > 1)
+        h[v][j] = *reinterpret_cast<const f32x4*>(p.ws_h + (wc + (long)(nch - 1) * p.Ch) * N + 4 * part + at);
       else h[v][j] = from_state ? *reinterpret_cast<const f32x4*>(hp + at) : f32x4{0, 0, 0, 0};
     }
   const float dv[2] = {p.D ? p.D[e0] : 0.f, p.D ? p.D[e1] : 0.f};
@@ -454,19 +460,24 @@ __global__ __launch_bounds__(256) void scan_pairs_kernel(ScanArgs p) {
 }
 
 // One thread per (sequence, channel, four states): walk the chunks, leaving in chunk k's place its TRUE end state, which is
-// where chunk k + 1 starts.  (The first chunk's is true already.)
+// where chunk k + 1 starts.  (The first chunk's is true already.)  The last chunk's place, which has no end state yet, takes
+// the state that the sequence continues from.
 template <bool ASC>
 __global__ __launch_bounds__(256) void scan_carry_kernel(ScanArgs p, int N, int nchunks) {
   const int s = blockIdx.y;
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
   const int c = (int)(i / (N / 4)), n = (int)(i % (N / 4)) * 4;
-  if (c >= p.Ch || p.seq_lens[s] <= 0) return;
-  const int nc = (p.qsl[s + 1] - p.qsl[s] + p.chunk - 1) / p.chunk;
+  const int sl = p.seq_lens[s];
+  if (c >= p.Ch || sl <= 0) return;
+  const int L = p.qsl[s + 1] - p.qsl[s], nc = (L + p.chunk - 1) / p.chunk;
   f32x4 a;
   if (ASC) { const float v = p.A[c / p.dt_div] * LOG2E; a = f32x4{v, v, v, v}; }
   else a = *reinterpret_cast<const f32x4*>(p.A + (long)c * N + n) * LOG2E;
   f32x4 h = {0, 0, 0, 0};
   const long w0 = (long)s * nchunks * p.Ch + c;
+  if (nc > 1 && sl - L > 0)
+    *reinterpret_cast<f32x4*>(p.ws_h + (w0 + (long)(nc - 1) * p.Ch) * N + n) =
+        *reinterpret_cast<const f32x4*>(p.state + ((long)p.block_table[s * p.bt_stride] * p.Ch + c) * N + n);
   constexpr int U = 8;                                  // chunks in flight
   for (int k0 = 0; k0 < nc - 1; k0 += U) {
     f32x4 loc[U];
