@@ -62,6 +62,20 @@ def test_continued_sequences_of_many_chunks(Ch, N, heads):
     assert torch.equal(ys[0], ys[1]) and torch.equal(ys[0], ys[2])
 
 
+@pytest.mark.parametrize("Ch,N,heads,offset", [(520, 16, 0, 0), (96, 64, 12, 0), (7, 16, 0, 0), (64, 16, 0, 1)])
+@pytest.mark.parametrize("new,ctx,hint", [([40, 3, 700], [0, 5, 2], None),          # the argument left out
+                                          ([2, 0, 1, 0], [3, 4, 0, 0], None),       # ... and few rows: the one-token form
+                                          ([900, 300], [1, 0], 128), ([900, 300], [1, 0], 256)])
+def test_a_length_hint_that_is_too_small(new, ctx, hint, Ch, N, heads, offset):
+    a = _scan_inputs(new, ctx, Ch, N, heads, 1, torch.float32, 5, offset)
+    names = ("u", "delta", "A", "B", "C", "D", "z", "delta_bias", "ssm_state")
+    b = {k: v.clone() if isinstance(v, torch.Tensor) else v for k, v in a.items()}
+    y = ops.selective_scan(**a, **({} if hint is None else dict(max_query_len=hint)))
+    want = R.selective_scan(*(b[k] for k in names), b["query_start_loc"], b["seq_lens"], b["block_table"])
+    torch.testing.assert_close(y, want, atol=3e-4, rtol=1e-4)              # as in test_selective_scan_forms
+    torch.testing.assert_close(a["ssm_state"], b["ssm_state"], atol=1e-4, rtol=1e-4)
+
+
 def test_rows_off_a_pair_boundary_take_the_plain_form():
     new, ctx = [130, 4], [0, 1]
     a = _scan_inputs(new, ctx, 64, 16, 0, 1, torch.bfloat16, 3, offset=1)

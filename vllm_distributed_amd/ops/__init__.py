@@ -1402,7 +1402,8 @@ def selective_scan(u: torch.Tensor, delta: torch.Tensor, A: torch.Tensor, B: tor
     """Selective state-space scan over a ragged batch with carried state.
     u, z [T, Ch]; delta [T, Ch] (Mamba) or [T, heads] (Mamba-2: one step size per head);
     A fp32 [Ch, N] or [heads]; B, C [T, groups * N]; D, delta_bias fp32 with delta's width;
-    ssm_state fp32 [slots, Ch, N], updated in place.  Returns y * silu(z) (y when z is None)."""
+    ssm_state fp32 [slots, Ch, N], updated in place.  Returns y * silu(z) (y when z is None).
+    ``max_query_len`` (the most new tokens of a sequence) is a hint: results do not depend on it."""
     if not _dev(u):
         return R.selective_scan(u, delta, A, B, C, D, z, delta_bias, ssm_state, query_start_loc, seq_lens,
                                 block_table, softplus, num_groups)
@@ -1423,7 +1424,8 @@ def selective_scan(u: torch.Tensor, delta: torch.Tensor, A: torch.Tensor, B: tor
     rep, gch, eb = Ch // E, Ch // num_groups, u.element_size()
     # one token per sequence, or channels in pairs that share B and C (and lie on a pair's boundary in every row);
     # what the pair kernel stages of B and C for a workgroup's channels has to fit its 8192 floats
-    step = max_query_len <= 1
+    # (a batch of two rows a sequence and more is one of prompts, whatever the hint says)
+    step = max_query_len <= 1 and T < 2 * S
     wgch = 512 * 16 // Nst
     paired = ssm_state.data_ptr() % 16 == 0 and A.data_ptr() % (16 if A.dim() == 2 else 4) == 0 and (step or (
         Ch % 2 == 0 and gch % 2 == 0 and (rep == 1 or rep % 2 == 0)

@@ -194,7 +194,7 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(
   if (MODE != 0) {
     ta = t0 + blockIdx.z * chunk;
     if (ta >= tb) return;
-    tb = min(tb, ta + chunk);
+    if (blockIdx.z + 1 < gridDim.z) tb = min(tb, ta + chunk);      // (the last chunk of the grid takes all that is left)
     ws_off = ((((long)s * gridDim.z + blockIdx.z) * C + c) * N) + part * 16;
   }
   float* hp = ssm_state + ((long)block_table[s * bt_stride] * C + c) * N + part * 16;
@@ -261,7 +261,7 @@ __global__ __launch_bounds__(256) void scan_combine_kernel(float* __restrict__ w
   const int L = qsl[s + 1] - qsl[s];
   float* hp = ssm_state + (long)block_table[s * bt_stride] * CN + i;
   float h = (sl - L > 0) ? *hp : 0.f;
-  const int nc = (L + chunk - 1) / chunk;
+  const int nc = min((L + chunk - 1) / chunk, nchunks);
   for (int k = 0; k < nc; ++k) {
     const long off = ((long)s * nchunks + k) * CN + i;
     const float p = ws_p[off];
@@ -311,10 +311,12 @@ __global__ __launch_bounds__(256) void scan_pairs_kernel(ScanArgs p) {
   const int sl = p.seq_lens[s];
   if (sl <= 0) return;
   const int t0 = p.qsl[s], L = p.qsl[s + 1] - t0;
-  const int nch = MODE == 0 ? 1 : (L + p.chunk - 1) / p.chunk, kch = MODE == 0 ? 0 : blockIdx.z;
+  const int nch = MODE == 0 ? 1 : min((L + p.chunk - 1) / p.chunk, (int)gridDim.z), kch = MODE == 0 ? 0 : blockIdx.z;
   if (kch >= nch || (MODE == 1 && kch == nch - 1)) return;       // (the last chunk's end state falls out of its output pass)
-  const int ta = MODE == 0 ? 0 : kch * p.chunk, tb = MODE == 0 ? L : min(L, ta + p.chunk);
-  const bool last = kch == nch - 1, from_state = sl - L > 0 && kch == 0;
+  // (the grid is sized by what the caller says is the longest: a sequence's last chunk takes all that is left)
+  const bool last = kch == nch - 1;
+  const int ta = MODE == 0 ? 0 : kch * p.chunk, tb = last ? L : ta + p.chunk;
+  const bool from_state = sl - L > 0 && kch == 0;
   const int cw = blockIdx.x * WGCH, g0 = cw / p.group_ch;
   const int span = (min(cw + WGCH, p.Ch) - 1) / p.group_ch - g0 + 1;       // B / C groups of this workgroup's channels
   const int part = threadIdx.x % NL;
@@ -469,7 +471,7 @@ __global__ __launch_bounds__(256) void scan_carry_kernel(ScanArgs p, int N, int 
   const int c = (int)(i / (N / 4)), n = (int)(i % (N / 4)) * 4;
   const int sl = p.seq_lens[s];
   if (c >= p.Ch || sl <= 0) return;
-  const int L = p.qsl[s + 1] - p.qsl[s], nc = (L + p.chunk - 1) / p.chunk;
+  const int L = p.qsl[s + 1] - p.qsl[s], nc = min((L + p.chunk - 1) / p.chunk, nchunks);
   f32x4 a;
   if (ASC) { const float v = p.A[c / p.dt_div] * LOG2E; a = f32x4{v, v, v, v}; }
   else a = *reinterpret_cast<const f32x4*>(p.A + (long)c * N + n) * LOG2E;
@@ -499,15 +501,16 @@ __global__ __launch_bounds__(256) void scan_carry_kernel(ScanArgs p, int N, int 
   }
 }
 
-// One token per sequence: the state read and written is all there is (118 sequences of 4096 x 128 states, 495 MB,
-// with the convolution: 118 us).  A lane owns four states, a wave one contiguous KB of them, and eight of those are in flight.
+// One token per sequence (or few): the state read and written is all there is (118 sequences of
+// 4096 x 128 states, 495 MB, with the convolution: 118 us).  A lane owns four states, a wave one contiguous KB of them, and
+// eight of those are in flight.
 template <typename T, int N, bool ASC>
 __global__ __launch_bounds__(256) void scan_step_kernel(ScanArgs p) {
   constexpr int Q = N / 4, CW = 64 / Q, K = 8;          // lanes per channel, channels per KB
   const int s = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int sl = p.seq_lens[s];
   if (sl <= 0) return;
-  const int t = p.qsl[s], L = p.qsl[s + 1] - t;
+  const int t0 = p.qsl[s], L = p.qsl[s + 1] - t0;
   if (L <= 0) return;
   const bool has_init = sl - L > 0;
   const int q = lane % Q, c0 = (blockIdx.x * 4 + wave) * (CW * K) + lane / Q;
@@ -518,10 +521,7 @@ __global__ __launch_bounds__(256) void scan_step_kernel(ScanArgs p) {
     const int c = c0 + k * CW;
     h[k] = has_init && c < p.Ch ? *reinterpret_cast<const f32x4*>(hp + (long)c * N) : f32x4{0, 0, 0, 0};
   }
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const int c = c0 + k * CW;
-    if (c >= p.Ch) break;                               // whole channels: the lanes of one leave together
+  auto token = [&](int t, int c, f32x4 hk) {             // whole channels: the lanes of one come here together
     const int e = c / p.dt_div;
     float dt = (float)((const T*)p.delta)[(long)t * p.d_stride + e] + (p.delta_bias ? p.delta_bias[e] : 0.f);
     if (p.softplus) dt = softplus_f(dt);
@@ -535,20 +535,32 @@ __global__ __launch_bounds__(256) void scan_step_kernel(ScanArgs p) {
     float y = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      h[k][i] = fmaf(__builtin_amdgcn_exp2f(dt * (a[i] * LOG2E)), h[k][i], dx * (float)bp[i]);
-      y = fmaf((float)cp[i], h[k][i], y);
+      hk[i] = fmaf(__builtin_amdgcn_exp2f(dt * (a[i] * LOG2E)), hk[i], dx * (float)bp[i]);
+      y = fmaf((float)cp[i], hk[i], y);
     }
-    *reinterpret_cast<f32x4*>(hp + (long)c * N) = h[k];
+    *reinterpret_cast<f32x4*>(hp + (long)c * N) = hk;
     y = group_sum<Q>(y);
     if (q == 0) {
       y += (p.D ? p.D[e] : 0.f) * x;
       if (p.z) y *= silu_f((float)((const T*)p.z)[(long)t * p.z_stride + c]);
       ((T*)p.out)[(long)t * p.o_stride + c] = (T)y;
     }
+  };
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int c = c0 + k * CW;
+    if (c >= p.Ch) break;
+    token(t0, c, h[k]);
+  }
+  // further tokens of a sequence, rare here: each lane's own states again from memory
+#pragma unroll 1
+  for (int i = K; i < K * L; ++i) {
+    const int c = c0 + i % K * CW;
+    if (c < p.Ch) token(t0 + i / K, c, *reinterpret_cast<const f32x4*>(hp + (long)c * N));
   }
 }
 
-// step: every sequence has at most one new token; otherwise channels in pairs (the caller checks that pairs share B, C and
+// step: the sequences have one new token each (none and several are right too); otherwise channels in pairs (the caller checks that pairs share B, C and
 // are aligned).  nchunks > 1: ws_dt [S, nchunks, C] and ws_h [S, nchunks, C, N].
 VDA_EXPORT int vda_selective_scan_pairs(void* out, const void* u, const void* delta, const float* A, const void* Bm,
                                         const void* Cm, const float* D, const void* z, const float* delta_bias,
