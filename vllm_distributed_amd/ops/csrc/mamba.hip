@@ -61,7 +61,8 @@ __global__ __launch_bounds__(256) void causal_conv1d_kernel(
   if (sl <= 0) return;
   const int t0 = qsl[s], L = qsl[s + 1] - t0;
   const bool has_init = sl - L > 0;
-  const int cs = blockIdx.z * chunk, ce = min(L, cs + chunk);
+  // (the grid is sized by what the caller says is the longest: its last chunk takes all that is left)
+  const int cs = blockIdx.z * chunk, ce = blockIdx.z + 1 < gridDim.z ? min(L, cs + chunk) : L;
   if (cs > 0 && cs >= L) return;
   T* st = conv_state + ((long)block_table[s * bt_stride] * C + c) * (W - 1);
   auto load = [&](int t) { return *reinterpret_cast<const vec_t*>(x + (long)(t0 + t) * x_stride + c); };
