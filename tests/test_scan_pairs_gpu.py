@@ -99,7 +99,7 @@ def test_conv_chunk_edges(W, C, offset):
     table = torch.randperm(9, generator=g)[:7, None].int().to(DEV)
     st2 = state.clone()
     want = R.causal_conv1d(x, w, b, st2, qsl, lens, table)
-    for longest in (max(new), 1, 40):                                        # a hint only: results do not depend on it
+    for longest in (max(new), 1, 9, 40):                                       # a hint only: results do not depend on it
         st = state.clone()
         y = ops.causal_conv1d(x, w, b, st, qsl, lens, table, longest)
         torch.testing.assert_close(y, want, atol=1e-5, rtol=1e-5)
