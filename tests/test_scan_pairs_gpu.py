@@ -104,3 +104,18 @@ def test_conv_chunk_edges(W, C, offset):
         y = ops.causal_conv1d(x, w, b, st, qsl, lens, table, longest)
         torch.testing.assert_close(y, want, atol=1e-5, rtol=1e-5)
         assert torch.equal(st, st2)
+
+
+@pytest.mark.parametrize("Ch,repeat,form", [(520, 1, "vda_selective_scan"), (4104, 5, "vda_selective_scan_pairs")])
+def test_short_sequences_take_the_form_that_fills_the_chip(monkeypatch, Ch, repeat, form):
+    new, ctx = [31, 32, 33, 1, 0] * repeat, [0, 3, 0, 4, 0] * repeat
+    a = _scan_inputs(new, ctx, Ch, 16, 0, 1, torch.float32, 2)
+    names = ("u", "delta", "A", "B", "C", "D", "z", "delta_bias", "ssm_state")
+    b = {k: v.clone() if isinstance(v, torch.Tensor) else v for k, v in a.items()}
+    called, call = [], ops.N.call
+    monkeypatch.setattr(ops.N, "call", lambda name, *args: (called.append(name), call(name, *args))[1])
+    y = ops.selective_scan(**a, max_query_len=33)
+    assert called == [form]
+    want = R.selective_scan(*(b[k] for k in names), b["query_start_loc"], b["seq_lens"], b["block_table"])
+    torch.testing.assert_close(y, want, atol=3e-4, rtol=1e-4)              # as in test_selective_scan_forms
+    torch.testing.assert_close(a["ssm_state"], b["ssm_state"], atol=1e-4, rtol=1e-4)

@@ -1432,6 +1432,12 @@ def selective_scan(u: torch.Tensor, delta: torch.Tensor, A: torch.Tensor, B: tor
         and 2 * Nst * min(-(-wgch // gch) + 1, -(-Ch // gch)) <= 8192
         and all(t.stride(0) % 2 == 0 and t.data_ptr() % (2 * eb) == 0
                 for t in (u, out) + ((delta,) if rep == 1 else ()) + ((z,) if z is not None else ()))))
+    # In one pass (below 96 tokens) pairs leave half as many lanes, each with twice the work: where 16 states a channel are less
+    # than 640 waves of pairs, the plain form is ahead (us, plain / pairs: 1 sequence of 40 tokens 31 / 41, 16 of 17 with
+    # 4096 channels, 512 waves, 20 / 25; 64 of 40 with 1536, 768 waves, 56 / 51).  More states share lanes in both forms
+    # and gain by the staged B and C at any size.
+    if paired and not step and Nst == 16 and max_query_len < envs.VDA_SCAN_CHUNK_MIN_TOKENS and S * Ch < 640 * 128:
+        paired = False
     chunk, nchunks, ws_p, ws_h = 0, 1, None, None
     # (seven prompts of 82 tokens on average, 4096 x 16: 140 us in one pass, 82 in chunks of 32; the plain form pays later)
     if max_query_len >= envs.VDA_SCAN_CHUNK_MIN_TOKENS and (paired or max_query_len >= 256):
