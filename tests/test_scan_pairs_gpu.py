@@ -119,3 +119,22 @@ def test_short_sequences_take_the_form_that_fills_the_chip(monkeypatch, Ch, repe
     want = R.selective_scan(*(b[k] for k in names), b["query_start_loc"], b["seq_lens"], b["block_table"])
     torch.testing.assert_close(y, want, atol=3e-4, rtol=1e-4)              # as in test_selective_scan_forms
     torch.testing.assert_close(a["ssm_state"], b["ssm_state"], atol=1e-4, rtol=1e-4)
+
+
+@pytest.mark.parametrize("setting,tokens,offset,chunked", [(None, 200, 1, False), (None, 256, 1, True), ("64", 80, 1, True),
+                                                          ("64", 80, 0, True), ("512", 300, 0, False), ("512", 300, 1, False)])
+def test_the_chunk_setting_holds_for_both_forms(monkeypatch, setting, tokens, offset, chunked):
+    monkeypatch.delenv("VDA_SCAN_CHUNK_MIN_TOKENS", raising=False)
+    if setting is not None:
+        monkeypatch.setenv("VDA_SCAN_CHUNK_MIN_TOKENS", setting)
+    a = _scan_inputs([tokens, 5], [0, 2], 64, 16, 0, 1, torch.float32, 4, offset)
+    names = ("u", "delta", "A", "B", "C", "D", "z", "delta_bias", "ssm_state")
+    b = {k: v.clone() if isinstance(v, torch.Tensor) else v for k, v in a.items()}
+    called, call = [], ops.N.call
+    monkeypatch.setattr(ops.N, "call", lambda name, *args: (called.append((name, args[-5])), call(name, *args))[1])
+    y = ops.selective_scan(**a, max_query_len=tokens)
+    (name, nchunks), = called
+    assert (nchunks > 1) == chunked, called
+    want = R.selective_scan(*(b[k] for k in names), b["query_start_loc"], b["seq_lens"], b["block_table"])
+    torch.testing.assert_close(y, want, atol=3e-4, rtol=1e-4)              # as in test_selective_scan_forms
+    torch.testing.assert_close(a["ssm_state"], b["ssm_state"], atol=1e-4, rtol=1e-4)

@@ -93,7 +93,8 @@ _REGISTRY: dict[str, tuple[Callable[[str], Any], Any]] = {
     "VDA_GEMM_SELECTIONS": (str, None),          # CSV of library-GEMM algorithm choices; "off" disables
     "VDA_DISABLE_SKINNY_GEMM": (_bool, False),
     "VDA_LORA_KERNEL_MAX_TOKENS": (int, 1024),   # multi-LoRA: batches up to this many rows use the fused shrink/expand kernels
-    "VDA_SCAN_CHUNK_MIN_TOKENS": (int, 96),      # state-space scan: sequences of at least this many new tokens run chunk-parallel
+    # state-space scan: sequences of at least this many new tokens run chunk-parallel (unset: 96 where channels go in pairs, else 256)
+    "VDA_SCAN_CHUNK_MIN_TOKENS": (int, None),
     "VDA_W4_SKINNY_MAX_M": (int, 32),            # W4A16: rows served by the packed-weight skinny kernel
     "VDA_CB4_SKINNY_MAX_M": (int, 64),           # 4-bit code-book weights (NF4 / FP4 / NVFP4): rows served by the skinny kernel
     "VDA_GGUF_PACKED": (_bool, True),            # GGUF: keep 4- / 5- / 8-bit block codes packed (False: expand to 16 bit at load)

@@ -1436,11 +1436,13 @@ def selective_scan(u: torch.Tensor, delta: torch.Tensor, A: torch.Tensor, B: tor
     # than 640 waves of pairs, the plain form is ahead (us, plain / pairs: 1 sequence of 40 tokens 31 / 41, 16 of 17 with
     # 4096 channels, 512 waves, 20 / 25; 64 of 40 with 1536, 768 waves, 56 / 51).  More states share lanes in both forms
     # and gain by the staged B and C at any size.
-    if paired and not step and Nst == 16 and max_query_len < envs.VDA_SCAN_CHUNK_MIN_TOKENS and S * Ch < 640 * 128:
+    set_min = envs.VDA_SCAN_CHUNK_MIN_TOKENS
+    if paired and not step and Nst == 16 and max_query_len < (96 if set_min is None else set_min) and S * Ch < 640 * 128:
         paired = False
     chunk, nchunks, ws_p, ws_h = 0, 1, None, None
-    # (seven prompts of 82 tokens on average, 4096 x 16: 140 us in one pass, 82 in chunks of 32; the plain form pays later)
-    if max_query_len >= envs.VDA_SCAN_CHUNK_MIN_TOKENS and (paired or max_query_len >= 256):
+    # unless the setting says otherwise, from 96 tokens on in pairs (seven prompts of 82 tokens on average, 4096 x 16: 140 us in
+    # one pass, 82 in chunks of 32), from 256 on in the plain form, where more passes over more states pay later
+    if max_query_len >= ((96 if paired else 256) if set_min is None else set_min):
         # lanes per channel: N / 16, or as many for a pair of them
         least = 32 if paired else 64
         want = -(-524288 // (S * (Ch // (2 if paired else 1)) * (Nst // 16)))
