@@ -16,6 +16,13 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
+@pytest.fixture(autouse=True)
+def at_any_cost(request, monkeypatch):
+    """The kernel's tests take it wherever it can run, also where its tiles would leave the chip idle."""
+    if "cost" not in request.node.name:
+        monkeypatch.setattr(ops, "_moe_wide_pays", lambda *a: True)
+
+
 def _routing(counts, k, g):
     """ids [T, k] in which expert e appears counts[e] times (in mixed order; -1 fills the last token)."""
     ids = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])
@@ -44,7 +51,6 @@ def test_wide_tiles(monkeypatch, dt, counts, k, H, I, gated):
     tw = torch.rand(T, k, generator=g).to(DEV) + 0.1
     ids = ids.to(DEV)
     assert ops._moe_wide_ok(x, w13, w2, T * k)
-    print(f"\ncase {counts[:6]} k {k} H {H} I {I}", flush=True)
     out = ops.fused_moe(x, w13, w2, tw, ids, gated=gated).double()
     ref = torch.zeros(T, H, dtype=torch.float64, device=DEV)
     for e in range(E):
@@ -82,3 +88,30 @@ def test_rule_and_the_other_tiles_agree(monkeypatch):
         lim = 2 * 2.0 ** -9 * other.float().norm(dim=1, keepdim=True)
         assert bool(((out.float() - other.float()).abs() <= lim).all())
     assert took == {128: False, 129: True, 232: True, 233: False, 351: False, 352: True, 600: True}
+
+
+@pytest.mark.parametrize("E,k,H,I,rows,wide", [(8, 2, 1024, 512, 360, False),        # fewer tiles than CUs
+                                               (32, 4, 1024, 512, 160, False),       # one round of either
+                                               (64, 8, 1024, 512, 160, True), (64, 8, 1024, 512, 440, True)])
+def test_the_cost_of_rounds_decides(monkeypatch, E, k, H, I, rows, wide):
+    """By the launch that is made; and the result is that of the other tiles (see above)."""
+    monkeypatch.setenv("VDA_MOE_GROUPED_MAX_PAIRS", "0")
+    g = torch.Generator().manual_seed(rows)
+    T = rows * E // k
+    gd = torch.Generator(device=DEV).manual_seed(rows)
+    w13 = (torch.randn(E, 2 * I, H, generator=gd, device=DEV) * 0.08).to(torch.bfloat16)
+    w2 = (torch.randn(E, H, I, generator=gd, device=DEV) * 0.08).to(torch.bfloat16)
+    x = torch.randn(T, H, generator=g).to(torch.bfloat16).to(DEV)
+    tw, ids = ops.moe_topk_softmax(torch.randn(T, E, generator=g).to(DEV), k)
+    out, took, call = [], [], ops.N.call
+    for force in (None, True, False):
+        with monkeypatch.context() as m:
+            if force is not None:
+                m.setattr(ops, "_moe_wide_pays", lambda *a: force)
+            m.setattr(ops.N, "call", lambda name, *a: (took.append(a[-6]) if name == "vda_tile_gemm" else None, call(name, *a))[1])
+            out.append(ops.fused_moe(x, w13, w2, tw, ids).float())
+    assert took == [256 if wide else 128] * 2 + [256] * 2 + [128] * 2
+    # pairs' rows round to bfloat16 in both, k of them are summed: 2 u of a pair's row each, of k rows of random sign
+    lim = 2 * 2.0 ** -9 * k * out[2].norm(dim=1, keepdim=True)
+    assert bool(((out[1] - out[2]).abs() <= lim).all())
+    assert torch.equal(out[0], out[1 if wide else 2])

@@ -8,6 +8,8 @@ KV cache layout used throughout:
 """
 from __future__ import annotations
 
+import functools
+import math
 from typing import Optional
 
 import torch
@@ -1134,16 +1136,31 @@ def moe_align_tiles(topk_ids: torch.Tensor, E: int, rows_per_tile: int):
 
 
 def _moe_wide_ok(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, pairs: int) -> bool:
-    """Do 16-bit experts take 256 x 256 tiles?  From 129 rows an expert on, except between 233 and 351, where most experts
-    are cut into one whole tile and one that is nearly empty.  Layer times in us, 128-row tiles / 256-row tiles: 16 experts
-    4096 x 6400 with 160 rows 795 / 735, 240 rows 888 / 923, 300 rows 1117 / 1159, 360 rows 1218 / 1182, 512 rows
-    1663 / 1510; 64 experts 2048 x 1024 with 160 rows 328 / 312, 270 rows 427 / 470, 360 rows 498 / 479, 512 rows
-    634 / 582.  (Eight experts 4096 x 14336 gain there too, 1277 / 1146 at 300 rows; 60 experts lose.)  The kernel's
-    offsets inside an operand are 32-bit."""
+    """Can 16-bit experts gain by 256 x 256 tiles?  From 129 rows an expert on, except between 233 and 351, where most experts
+    are cut into one whole tile and one that is nearly empty (60 experts 2048 x 1408 with 300 rows: 541 us on 128-row tiles, 620
+    on these; 64 experts 2048 x 1024 436 / 460; eight experts 4096 x 14336, whose rounds come out even, 1292 / 1161).  The
+    kernel's offsets inside an operand are 32-bit."""
     rows = pairs / w13.shape[0]
     return (w13.dtype != torch.float8_e4m3fn and rows > 128 and not 232 < rows < 352
             and max(max(x.stride(0), x.shape[1]) * x.shape[0], w2.shape[2] * pairs, w13.shape[1] * w13.shape[2],
                     w2.shape[1] * w2.shape[2]) < 1 << 31)
+
+
+@functools.lru_cache(maxsize=1024)
+def _moe_wide_pays(pairs: int, E: int, n1: int, k1: int, n2: int, k2: int) -> bool:
+    """Do 256 x 256 tiles cost less than 128 x 256 ones, for ``pairs`` rows over E experts in products [rows, k] x [k, n tiles]?
+    A CU holds one tile at a time: a product takes rounds of 256 tiles (whole ones; beyond two rounds their ends overlap) of
+    K steps each, and a round of wide tiles costs 1.65 of the others (1.6 .. 1.9 where both fill their rounds).  An expert's rows
+    are its share and a standard deviation.  Layer times in us, 128-row tiles / 256-row tiles: 64 experts 2048 x 1024 with 160 rows
+    each 322 / 305, 440 rows 561 / 492, 500 rows 618 / 575; 8 experts
+    4096 x 14336 with 440 rows 1522 / 1260, 200 rows 834 / 917; 8 experts 1024 x 512, whose tiles leave CUs idle, with 360
+    rows 52 / 72.  Of 195 such points in the range above, this takes 93; four of them lose more than 2 %, the worst 7 %."""
+    rows = pairs / E
+
+    def cost(rows_per_tile: int) -> float:
+        m_tiles = E * math.ceil((rows + math.sqrt(rows)) / rows_per_tile)
+        return sum(k * (-(-m_tiles * n // 256) if m_tiles * n <= 512 else m_tiles * n / 256) for n, k in ((n1, k1), (n2, k2)))
+    return 1.65 * cost(256) < cost(128)
 
 
 def _moe_tiled(x, w13, w2, topk_w, topk_ids, w13_scale, w2_scale, block_scales: bool = False,
@@ -1160,7 +1177,8 @@ def _moe_tiled(x, w13, w2, topk_w, topk_ids, w13_scale, w2_scale, block_scales: 
     I = I2 // 2 if gated else I2
     P_ = T * k
     dev = x.device
-    rows = 256 if _moe_wide_ok(x, w13, w2, P_) else _tile_rows(P_ / E)
+    wide = _moe_wide_ok(x, w13, w2, P_) and _moe_wide_pays(P_, E, -(-I // (128 if gated else 256)), H, -(-H // 256), I)
+    rows = 256 if wide else _tile_rows(P_ / E)
     sorted_ids, _, tiles, max_tiles = moe_align_tiles(topk_ids, E, rows)
     te, tb, tend, ntl = (tiles[:max_tiles], tiles[max_tiles:2 * max_tiles], tiles[2 * max_tiles:3 * max_tiles],
                          tiles[3 * max_tiles:])
