@@ -81,3 +81,29 @@ def test_split_rows_of_nothing_but_masked_tokens():
     k = torch.tensor([0, 5, 0, 5], dtype=torch.int32, device=DEV)
     p = torch.tensor([1.0, 1.0, 0.5, 0.5], device=DEV)
     assert ops.sample(x, None, k, p).tolist() == [0, 0, 0, 0]
+
+
+# a row of 8191 is walked by one workgroup, the same row and a masked entry by several; more rows than one set of launches takes;
+# counts beyond the list's length, with and without a fraction
+@pytest.mark.parametrize("S,high", [(600, 60), (24, 8191)])
+@pytest.mark.parametrize("shape", ["model", "ties", "masked", "infinite"])
+def test_both_forms_draw_the_same(S, high, shape):
+    g = torch.Generator().manual_seed(S + len(shape))
+    V = 8191
+    x = torch.randn(S, V, generator=g) * 2.0
+    if shape == "ties":
+        x = (x * 2).round() / 2
+    elif shape == "masked":
+        x[:, 100:] = torch.where(torch.rand(S, V - 100, generator=g) < 0.7, -float("inf"), x[:, 100:])
+    elif shape == "infinite":
+        x[::2, 5] = float("inf")
+        x[::3, 9] = torch.finfo(torch.float32).min
+    r = torch.arange(S)
+    temp = 0.4 + torch.rand(S, generator=g)
+    k = torch.where(r % 2 == 1, torch.randint(high // 2, high, (S,), generator=g), 0).to(torch.int32)
+    p = torch.where(r % 4 >= 2, 0.3 + 0.69 * torch.rand(S, generator=g), 1.0)
+    mp = torch.where(r % 5 == 4, 0.02, 0.0)
+    seeds = torch.randint(0, 2 ** 62, (S,), generator=g)
+    args = [t.to(DEV) for t in (temp, k, p, mp, seeds)]
+    wide = torch.cat([x, torch.full((S, 1), -float("inf"))], 1)
+    assert torch.equal(ops.sample(wide.to(DEV), *args), ops.sample(x.to(DEV), *args))

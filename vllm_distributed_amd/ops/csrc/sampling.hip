@@ -113,12 +113,15 @@ __device__ __forceinline__ void pick_bin(const unsigned long long* hist, unsigne
   }
 }
 
-// keeps the compiler from folding the multiplication behind ``v`` into what is done with it: a weight is the same
-// number wherever it is computed
+// keeps the compiler from folding the operation behind ``v`` into what is done with it.  Several kernels compute a scaled
+// logit, its weight, its bin and its noise, each from other registers; what one counts another must find, so every step
+// of these is rounded by itself, wherever it is compiled.
 __device__ __forceinline__ float opaque(float v) { asm("" : "+v"(v)); return v; }
+// 1 / temperature
+__device__ __forceinline__ float inverse(float t) { return opaque(__builtin_amdgcn_rcpf(t)); }
 // exp(z - zmax) as a 32.32 fixed-point number
 __device__ __forceinline__ unsigned long long fixed_weight(float z, float zmax) {
-  return (unsigned long long)(__expf(opaque(z) - zmax) * 4294967296.f);
+  return (unsigned long long)(__expf(opaque(opaque(z) - zmax)) * 4294967296.f);
 }
 
 // One radix descent over n entries; at(i) is entry i's scaled logit.  weight(i) = 1 (COUNT) or exp(z_i - zmax) for
@@ -159,7 +162,7 @@ __device__ uint32_t radix_threshold(At at, int n, float zmax, float target, unsi
 __device__ __forceinline__ float noisy(float z, uint64_t seed, int i) {
   const uint32_t rnd = mix32(seed * 0x9E3779B97F4A7C15ULL + (uint64_t)i + 0x632BE59BD9B4E019ULL);
   const float u = ((float)(rnd >> 8) + 0.5f) * (1.f / 16777216.f);     // (0, 1)
-  return z - __logf(-__logf(u));
+  return opaque(z) - opaque(__logf(-__logf(u)));
 }
 
 struct SampleArgs {
@@ -187,7 +190,7 @@ __device__ void sample_row(const SampleArgs& p, int rowi, float zmax_known, bool
     if (threadIdx.x == 0) p.out[rowi] = a.i;
     return;
   }
-  const float inv_t = 1.f / temp;
+  const float inv_t = inverse(temp);
   float zmax = zmax_known;
   if (!know_max) {
     float mx = -INFINITY;
@@ -237,7 +240,8 @@ __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs p) {
 //            that bin's entries (top-k and top-p together: all entries down to it)
 //   finish   the exact threshold key among the collected entries, the draw among them, and the row's winner
 // A row whose bin overflows the list (thousands of equal logits) is done by its finish workgroup alone, the way of the
-// short rows.  The result is that of the one-workgroup form: the bins are monotone in the key and sums are integers.
+// short rows.  The result is that of the one-workgroup form: the bins are monotone in the key, sums are integers, and each
+// number is rounded alike in every kernel (opaque).
 constexpr int SPLIT_BINS = 2048;      // bin 0: the maximum; the last: -inf; the last but one: beyond the span
 constexpr int SPLIT_LIST = 4096;      // collected entries of a row
 constexpr int SPLIT_MAX_G = 64;
@@ -264,7 +268,7 @@ __device__ __forceinline__ SplitFilter split_filter(const SampleArgs& p, int row
   SplitFilter f;
   const float temp = p.temperature ? p.temperature[rowi] : 1.f;
   f.greedy = temp < 1e-5f;
-  f.inv_t = f.greedy ? 1.f : 1.f / temp;
+  f.inv_t = f.greedy ? 1.f : inverse(temp);
   const int k = p.top_k ? p.top_k[rowi] : 0;
   f.k = k > 0 && k < p.V ? k : 0;
   f.tp = p.top_p ? p.top_p[rowi] : 1.f;
@@ -308,12 +312,12 @@ __device__ __forceinline__ SplitScale split_scale(const SplitRow* ws, int G) {
   mn = -wave_max(-mn);
   // weights below 2^-32 of the largest are zero: 22.2; a k-th largest entry further down lands in the last bins
   const float span = fminf(fmaxf(mx - mn, 1e-3f), 24.f);
-  return {mx, (float)(SPLIT_BINS - 2) / span};
+  return {mx, opaque((float)(SPLIT_BINS - 2) * opaque(__builtin_amdgcn_rcpf(span)))};
 }
 // a function of the scaled logit that never decreases as it falls
 __device__ __forceinline__ int split_bin(float z, SplitScale sc) {
   if (z == -INFINITY) return SPLIT_BINS - 1;
-  return (int)fminf(fmaxf((sc.zmax - opaque(z)) * sc.per, 0.f), (float)(SPLIT_BINS - 2));
+  return (int)fminf(fmaxf(opaque(opaque(sc.zmax - opaque(z)) * sc.per), 0.f), (float)(SPLIT_BINS - 2));
 }
 
 __global__ __launch_bounds__(1024) void split_stats_kernel(SampleArgs p, SplitRow* ws_rows, int row0) {
