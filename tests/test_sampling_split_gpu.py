@@ -107,3 +107,19 @@ def test_both_forms_draw_the_same(S, high, shape):
     args = [t.to(DEV) for t in (temp, k, p, mp, seeds)]
     wide = torch.cat([x, torch.full((S, 1), -float("inf"))], 1)
     assert torch.equal(ops.sample(wide.to(DEV), *args), ops.sample(x.to(DEV), *args))
+
+
+@pytest.mark.parametrize("S,V,split", [(3, 24575, False), (3, 24576, True), (33, 40959, False), (33, 40960, True),
+                                       (257, 65535, False), (257, 65536, True)])
+def test_unfiltered_rows(S, V, split):
+    """Draws without top-k and top-p are spread over workgroups from longer rows on; temperature, min-p and greedy rows."""
+    assert (ops.N.lib().vda_sample_workspace(S, V, 0) > 0) == split and ops.N.lib().vda_sample_workspace(S, V, 1) > 0
+    g = torch.Generator().manual_seed(V)
+    x = (torch.randn(S, V, generator=g) * 2.0).to(DEV)
+    temp = (0.4 + torch.rand(S, generator=g)).masked_fill_(torch.arange(S) % 3 == 2, 0.0).to(DEV)
+    mp = torch.where(torch.arange(S) % 5 == 4, 0.02, 0.0).to(DEV)
+    seeds = torch.randint(0, 2 ** 62, (S,), generator=g).to(DEV)
+    got = ops.sample(x, temp, None, None, mp, seeds)
+    off = torch.ones(S, device=DEV)                                          # a top-p that filters nothing: the other form
+    assert torch.equal(got, ops.sample(x, temp, None, off, mp, seeds))
+    assert torch.equal(got[2::3], x[2::3].argmax(1))

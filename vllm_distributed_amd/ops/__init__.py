@@ -439,7 +439,7 @@ def sample(logits: torch.Tensor, temperature=None, top_k=None, top_p=None, min_p
     assert logits.dtype == torch.float32
     S, V = logits.shape
     out = torch.empty(S, dtype=torch.long, device=logits.device)
-    ws_bytes = N.lib().vda_sample_workspace(S, V)
+    ws_bytes = N.lib().vda_sample_workspace(S, V, int(top_k is not None or top_p is not None))
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=logits.device) if ws_bytes else None
     N.call("vda_sample", logits.data_ptr(), out.data_ptr(), N.ptr(temperature), N.ptr(top_k), N.ptr(top_p),
            N.ptr(min_p), N.ptr(seeds), S, V, logits.stride(0), N.ptr(ws), ws_bytes, N.stream())

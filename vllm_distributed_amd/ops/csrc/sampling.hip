@@ -4,8 +4,8 @@
 //     counting (or summing fixed-point weights) per bin: no sort, and no dependence on the order of the lanes;
 //   * the draw is Gumbel-argmax (argmax of z_i + g_i, g_i ~ Gumbel(0,1)), which is
 //     exactly a sample from softmax(z) restricted to the kept tokens.
-// Vocabularies of SPLIT_MIN_V entries and more spread every row over several workgroups (the split kernels below);
-// shorter rows are walked by one workgroup each.
+// Long vocabularies spread every row over several workgroups (the split kernels below; split_min_v says from which length
+// on); shorter rows are walked by one workgroup each.
 // Reference behaviour: vllm/v1/sample/sampler.py, ops/topk_topp_sampler.py,
 // csrc/sampler.cu (apply_repetition_penalties_).
 #include "common.h"
@@ -116,7 +116,11 @@ __device__ __forceinline__ void pick_bin(const unsigned long long* hist, unsigne
 // keeps the compiler from folding the operation behind ``v`` into what is done with it.  Several kernels compute a scaled
 // logit, its weight, its bin and its noise, each from other registers; what one counts another must find, so every step
 // of these is rounded by itself, wherever it is compiled.
-__device__ __forceinline__ float opaque(float v) { asm("" : "+v"(v)); return v; }
+// (noconvergent: loops with it can still be unrolled.)
+__device__ __forceinline__ float opaque(float v) {
+  [[clang::noconvergent]] asm("" : "+v"(v));
+  return v;
+}
 // 1 / temperature
 __device__ __forceinline__ float inverse(float t) { return opaque(__builtin_amdgcn_rcpf(t)); }
 // exp(z - zmax) as a 32.32 fixed-point number
@@ -124,7 +128,7 @@ __device__ __forceinline__ unsigned long long fixed_weight(float z, float zmax) 
   return (unsigned long long)(__expf(opaque(opaque(z) - zmax)) * 4294967296.f);
 }
 
-// One radix descent over n entries; at(i) is entry i's scaled logit.  weight(i) = 1 (COUNT) or exp(z_i - zmax) for
+// One radix descent by 1024 threads over n entries; at(i) is entry i's scaled logit.  weight(i) = 1 (COUNT) or exp(z_i - zmax) for
 // keys >= floor_key; target = a number of entries (COUNT), a fraction of the total weight (target_w = 0), or the
 // weight target_w.  Returns the key u* with  W{key >= u*} >= target  and  W{key > u*} < target.  Weights are
 // accumulated as 32.32 fixed-point integers: integer addition does not depend on the order in which the lanes'
@@ -138,9 +142,9 @@ __device__ uint32_t radix_threshold(At at, int n, float zmax, float target, unsi
   unsigned long long remaining = COUNT ? (unsigned long long)target : target_w;
   for (int pass = 0; pass < 4; ++pass) {
     const int shift = 24 - 8 * pass;
-    for (int b = threadIdx.x; b < 256; b += blockDim.x) hist[b] = 0ull;
+    for (int b = threadIdx.x; b < 256; b += 1024) hist[b] = 0ull;
     __syncthreads();
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    for (int i = threadIdx.x; i < n; i += 1024) {
       const float z = at(i);
       const uint32_t k = fkey(z);
       if (k < floor_key) continue;
@@ -177,7 +181,7 @@ struct SampleArgs {
   long stride;
 };
 
-// One row by one workgroup.
+// One row by one workgroup of 1024.
 __device__ void sample_row(const SampleArgs& p, int rowi, float zmax_known, bool know_max, float* red, float* rv, int* ri,
                            unsigned long long* hist, uint32_t* s_sel, unsigned long long* s_rem) {
   const float* row = p.logits + (long)rowi * p.stride;
@@ -185,7 +189,7 @@ __device__ void sample_row(const SampleArgs& p, int rowi, float zmax_known, bool
   const float temp = p.temperature ? p.temperature[rowi] : 1.f;
   if (temp < 1e-5f) {
     ArgMax a{-INFINITY, 0x7fffffff};
-    for (int i = threadIdx.x; i < V; i += blockDim.x) a = amax2(a, ArgMax{row[i], i});
+    for (int i = threadIdx.x; i < V; i += 1024) a = amax2(a, ArgMax{row[i], i});
     a = block_argmax(a, rv, ri);
     if (threadIdx.x == 0) p.out[rowi] = a.i;
     return;
@@ -194,7 +198,7 @@ __device__ void sample_row(const SampleArgs& p, int rowi, float zmax_known, bool
   float zmax = zmax_known;
   if (!know_max) {
     float mx = -INFINITY;
-    for (int i = threadIdx.x; i < V; i += blockDim.x) mx = fmaxf(mx, row[i] * inv_t);
+    for (int i = threadIdx.x; i < V; i += 1024) mx = fmaxf(mx, row[i] * inv_t);
     zmax = block_max(mx, red);
   }
   auto at = [&](int i) { return row[i] * inv_t; };
@@ -210,7 +214,7 @@ __device__ void sample_row(const SampleArgs& p, int rowi, float zmax_known, bool
 
   const uint64_t seed = (uint64_t)(p.seeds ? p.seeds[rowi] : 0);
   ArgMax a{-INFINITY, 0x7fffffff};
-  for (int i = threadIdx.x; i < V; i += blockDim.x) {
+  for (int i = threadIdx.x; i < V; i += 1024) {
     const float z = at(i);
     if (fkey(z) >= thr) a = amax2(a, ArgMax{noisy(z, seed, i), i});
   }
@@ -246,6 +250,13 @@ constexpr int SPLIT_BINS = 2048;      // bin 0: the maximum; the last: -inf; the
 constexpr int SPLIT_LIST = 4096;      // collected entries of a row
 constexpr int SPLIT_MAX_G = 64;
 constexpr int SPLIT_MIN_V = 8192;     // shorter rows: the launches cost more than the one-workgroup form's passes
+// Without top-k and top-p the one-workgroup form walks a row twice, not ten times, and many rows fill the chip by themselves:
+// the launches pay from longer rows on.  Kernel times in us, one workgroup a row / several, draws (greedy rows): 8 x 16384
+// 11.9 / 13.0 (5.5 / 8.1), 8 x 32000 19.4 / 13.2 (7.9 / 8.1), 64 x 32000 19.9 / 17.7 (8.1 / 10.2), 256 x 50257 44.7 / 41.9, 600 x 50257
+// 82.9 / 99.7 (39.5 / 45.6), 600 x 65536 107 / 106.
+static int split_min_v(int S, bool filtered) {
+  return filtered ? SPLIT_MIN_V : S <= 32 ? 24576 : S <= 256 ? 40960 : 65536;
+}
 constexpr int SPLIT_ROWS = 512;       // rows of one set of launches (bounds the workspace)
 
 struct SplitRow {                     // workspace of one row
@@ -573,9 +584,9 @@ VDA_EXPORT int vda_argmax(const void* logits, long* out, int S, int V, long stri
   return 0;
 }
 
-// bytes of workspace that vda_sample wants for rows of V entries (0: none)
-VDA_EXPORT long vda_sample_workspace(int S, int V) {
-  return V < SPLIT_MIN_V ? 0 : (long)sizeof(SplitRow) * (S < SPLIT_ROWS ? S : SPLIT_ROWS);
+// bytes of workspace that vda_sample wants for rows of V entries, with top_k or top_p (filtered) or without (0: none)
+VDA_EXPORT long vda_sample_workspace(int S, int V, int filtered) {
+  return V < split_min_v(S, filtered) ? 0 : (long)sizeof(SplitRow) * (S < SPLIT_ROWS ? S : SPLIT_ROWS);
 }
 
 VDA_EXPORT int vda_sample(const float* logits, long* out, const float* temperature, const int* top_k,
@@ -583,19 +594,20 @@ VDA_EXPORT int vda_sample(const float* logits, long* out, const float* temperatu
                           void* workspace, long workspace_bytes, hipStream_t st) {
   if (S == 0) return 0;
   const SampleArgs p{logits, out, temperature, top_k, top_p, min_p, seeds, V, stride};
-  if (V < SPLIT_MIN_V) {
+  const bool filtered = top_k || top_p;
+  if (V < split_min_v(S, filtered)) {
     hipLaunchKernelGGL(sample_kernel, dim3(S), dim3(1024), 0, st, p);
     VDA_CHECK_LAUNCH();
     return 0;
   }
-  if (!workspace || workspace_bytes < vda_sample_workspace(S, V)) return -1;
+  if (!workspace || workspace_bytes < vda_sample_workspace(S, V, filtered)) return -1;
   SplitRow* ws = (SplitRow*)workspace;
   for (int row0 = 0; row0 < S; row0 += SPLIT_ROWS) {
     const int rows = min(S - row0, SPLIT_ROWS);
     // two workgroups of 1024 threads per CU, at least a float4 for every thread
     const int G = max(1, min(min((512 + rows - 1) / rows, (V + 4095) / 4096), SPLIT_MAX_G));
     hipLaunchKernelGGL(split_stats_kernel, dim3(G, rows), dim3(1024), 0, st, p, ws, row0);
-    if (top_k || top_p) hipLaunchKernelGGL(split_bins_kernel, dim3(G, rows), dim3(1024), 0, st, p, ws, row0);
+    if (filtered) hipLaunchKernelGGL(split_bins_kernel, dim3(G, rows), dim3(1024), 0, st, p, ws, row0);
     hipLaunchKernelGGL(split_collect_kernel, dim3(G, rows), dim3(1024), 0, st, p, ws, row0);
     hipLaunchKernelGGL(split_finish_kernel, dim3(rows), dim3(1024), 0, st, p, ws, row0, G);
   }

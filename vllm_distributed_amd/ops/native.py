@@ -49,7 +49,7 @@ _SIGS = {
     "vda_set_prefill_wide_min_wgs": [L],
     "vda_merge_attn_states": [P, P, P, P, P, P, I, I, I, I, P],
     "vda_argmax": [P, P, I, I, L, I, P],
-    "vda_sample_workspace": [I, I],
+    "vda_sample_workspace": [I, I, I],
     "vda_sample": [P, P, P, P, P, P, P, I, I, L, P, L, P],
     "vda_topk_topp_mask": [P, P, P, P, I, I, L, P],
     "vda_apply_penalties": [P, P, P, P, P, P, I, I, L, P],
