@@ -73,3 +73,12 @@ def test_masks_and_several_tokens(D, Hq, Hkv, kw, fp8):
 def test_longest_first(S, Hkv, nsplit):
     lens = [(EDGES * 20)[i] if i % 3 else 200 for i in range(S)]
     _check(lens, [1] * S, 2 * Hkv, Hkv, 128, 16, torch.bfloat16, True, nsplit)
+
+
+# grids above 512 workgroups: lengths alike (their own order), all within an eighth but one, and rows without keys
+@pytest.mark.parametrize("S", [65, 129, 256])
+@pytest.mark.parametrize("lens", [lambda i, S: 130, lambda i, S: 128 + i % 9, lambda i, S: 600 if i == S - 1 else 130,
+                                  lambda i, S: 0 if i % 5 == 1 else 77])
+def test_order_of_large_batches(S, lens):
+    lens = [lens(i, S) for i in range(S)]
+    _check(lens, [1] * S, 16, 8, 128, 16, torch.bfloat16, S == 129, 1)

@@ -229,9 +229,9 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(AttnParams p) {
 // registers until the product takes them: the next step's keys are requested as soon as the scores have used this step's, its
 // values as soon as the outputs have, and page numbers a step before that, so that no load waits for another.
 //
-// What it measured (us, before -> after): 183 sequences of 525 .. 3675 keys, 64 / 8 heads of 128, e4m3 cache 257 -> 160 (4.9 TB/s);
-// 128 of 375 .. 2625, 32 / 8 heads, bf16 174 -> 146 (5.4 TB/s); 64 of 500 .. 3500, 16 / 8 heads of 256 308 -> 203; 5 of some
-// 390 keys 13.0 -> 11.7.  Of the first, 203 without the order of sequences below; held to the 168 registers of three
+// What it measured (us, before -> after): 183 sequences of 525 .. 3675 keys, 64 / 8 heads of 128, e4m3 cache 257 -> 148 (5.3 TB/s),
+// 16-bit 310 -> 271; 256 of 1100, 64 / 8 heads, e4m3 160 -> 113, 16-bit 206 -> 200 (5.8 TB/s), of 300 keys 70 -> 64; 64 of
+// 500 .. 3500, 16 / 8 heads of 256 308 -> 203; 5 of some 390 keys 13.0 -> 11.7.  Of the first, 203 without the order of sequences below; held to the 168 registers of three
 // waves per SIMD it spills 15 and takes 177.  Non-temporal loads: e4m3 rows 6 % faster, 16-bit ones, of which a lane's pieces share
 // lines, up to 60 % slower.
 constexpr unsigned DECODE_RANKED = 512;    // two workgroups per CU are resident
@@ -250,25 +250,37 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(AttnParams p) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, g = lane >> 4;
   // Workgroup -> (sequence, part, kv head), heads fastest.  A grid larger than the chip holds takes its sequences longest
-  // first (rank by counting): a long one that starts last would run alone.
+  // first: a long one that starts last would run alone.  Every wave finds its own, the blockIdx.z-th largest of the lengths,
+  // bit by bit: no barrier, and no more than some 25 dependent counts before the first key (counting ranks over LDS took
+  // 256 of 300 keys, 64 / 8 heads, from 70 to 90 us).  Lengths within an eighth of the first one's stay in their order.
   const int kvh = blockIdx.x, part = blockIdx.y;
   int seq = blockIdx.z;
+  int qs = p.q_start_loc[seq], q_end = p.q_start_loc[seq + 1], seq_len = p.seq_lens[seq];
   if (gridDim.x * gridDim.y * gridDim.z > DECODE_RANKED && p.num_seqs <= 256) {
-    __shared__ int s_len[256];
-    __shared__ int s_seq;
-    const int tid = threadIdx.x, mine = tid < p.num_seqs ? p.seq_lens[tid] : -1;
-    s_len[tid] = mine;
-    __syncthreads();
-    int rank = 0;
-    for (int i = 0; i < p.num_seqs; ++i) rank += s_len[i] > mine || (s_len[i] == mine && i < tid);
-    if (tid < p.num_seqs && rank == seq) s_seq = tid;
-    __syncthreads();
-    seq = __builtin_amdgcn_readfirstlane(s_seq);
+    const int base = p.seq_lens[0], bits = min(32 - __clz(p.max_blocks * BS), 22);
+    int key[4];                                         // length, then the first of the batch; no two alike
+    bool differs = false;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int at = lane + 64 * i, len = p.seq_lens[min(at, p.num_seqs - 1)];
+      differs |= abs(len - base) > base >> 3;
+      key[i] = at < p.num_seqs ? min(max(len, 0), (1 << bits) - 1) << 8 | (255 - at) : -1;
+    }
+    if (__any(differs)) {
+      int found = 0;                                    // the largest number that more than blockIdx.z keys reach
+      for (int bit = bits + 7; bit >= 0; --bit) {
+        const int next = found | 1 << bit;
+        int reach = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) reach += __popcll(__ballot(key[i] >= next));
+        if (reach > (int)blockIdx.z) found = next;
+      }
+      seq = 255 - (found & 255);
+      qs = p.q_start_loc[seq]; q_end = p.q_start_loc[seq + 1]; seq_len = p.seq_lens[seq];
+    }
   }
   const int G = p.Hq / p.Hkv;
-  const int qs = p.q_start_loc[seq];
-  const int q_len = p.q_start_loc[seq + 1] - qs;
-  const int seq_len = p.seq_lens[seq];
+  const int q_len = q_end - qs;
   if (q_len <= 0) return;
   const int ctx = seq_len - q_len;        // keys that precede the first query token
   const int* bt = p.block_table + (long)seq * p.max_blocks;
