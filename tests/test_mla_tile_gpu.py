@@ -69,3 +69,32 @@ def test_growing_scores_rescale_the_sums():
     ops.mla_attention(out, q, kc, vt, table, lens, starts, 0.5, 3, 1)
     want = R.mla_attention(q, kc, vt, table, lens, starts, 0.5)
     torch.testing.assert_close(out.float(), want.float(), atol=12 * 2.0 ** -9, rtol=2.0 ** -8)
+
+
+@pytest.mark.parametrize("H", [16, 128])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float8_e4m3fn])
+def test_rows_without_keys(H, dtype):
+    """Padded sequences (no keys) among others, with pieces: their rows are merged from what was written for them alone.  Tokens
+    before their sequence's first key (fewer keys than new tokens), in one piece and in several: zero."""
+    kc, vt, table, lens, starts = _batch([1, 1, 1], [40, 700, 2100], 16, dtype, 8)
+    lens[1] = 0
+    q = torch.randn(3, H, DK, device=DEV).to(torch.bfloat16)
+    out = torch.full((3, H, DV), float("nan"), device=DEV, dtype=torch.bfloat16)
+    for fill in (float("inf"), 0.0, -1.0):               # whatever the pieces' workspace held before
+        torch.full((3 * H * 16 * (DV + 1) * 2,), fill, device=DEV)
+        ops.mla_attention(out, q, kc, vt, table, lens, starts, 192 ** -0.5, 1, 8)
+        assert bool((out[1] == 0).all())
+    live = torch.tensor([0, 2], device=DEV)
+    want = R.mla_attention(q[live], kc, vt, table[live], lens[live], torch.tensor([0, 1, 2], dtype=torch.int32, device=DEV), 192 ** -0.5)
+    torch.testing.assert_close(out[live].float(), want.float(), atol=12 * 2.0 ** -9, rtol=2.0 ** -8)
+    for total, width in (([9, 40], 4), ([9, 900], 90)):  # a table of one piece, and of several
+        kc, vt, table, lens, starts = _batch([20, 3], [20, total[1]], 16, dtype, 9)
+        lens[0] = total[0]
+        wide = torch.zeros((2, width), dtype=torch.int32, device=DEV)
+        wide[:, :min(width, table.shape[1])] = table[:, :width]
+        q = torch.randn(23, H, DK, device=DEV).to(torch.bfloat16)
+        out = torch.full((23, H, DV), float("nan"), device=DEV, dtype=torch.bfloat16)
+        ops.mla_attention(out, q, kc, vt, wide, lens, starts, 192 ** -0.5, 20, 1)
+        assert bool((out[:11] == 0).all()) and bool(out.isfinite().all())
+        want = R.mla_attention(q[11:], kc, vt, wide, lens, torch.tensor([0, 9, 12], dtype=torch.int32, device=DEV), 192 ** -0.5)
+        torch.testing.assert_close(out[11:].float(), want.float(), atol=12 * 2.0 ** -9, rtol=2.0 ** -8)
