@@ -98,3 +98,26 @@ def test_rows_without_keys(H, dtype):
         assert bool((out[:11] == 0).all()) and bool(out.isfinite().all())
         want = R.mla_attention(q[11:], kc, vt, wide, lens, torch.tensor([0, 9, 12], dtype=torch.int32, device=DEV), 192 ** -0.5)
         torch.testing.assert_close(out[11:].float(), want.float(), atol=12 * 2.0 ** -9, rtol=2.0 ** -8)
+
+
+@pytest.mark.parametrize("H,new,dtype", [(16, 1, torch.bfloat16), (128, 1, torch.float16), (40, 3, torch.bfloat16),
+                                         (16, 1, torch.float8_e4m3fn)])
+def test_a_sequence_does_not_see_its_neighbours_lengths(H, new, dtype):
+    """Where its keys are cut depends on the batch's size and the table's width, not on how long the others are: the same bits."""
+    S, width = 5, 300
+    qd = torch.bfloat16 if dtype == torch.float8_e4m3fn else dtype
+    first = None
+    for others in ([40, 50, 60, 70], [4000, 3500, 4100, 2900], [1, 0, 2000, 3]):
+        total = [new + 1700] + [new + t if t else 0 for t in others]
+        kc, vt, table, lens, starts = _batch([new] * S, total, 16, dtype, 3)
+        g = torch.Generator().manual_seed(4)
+        rows = torch.randn(total[0], DK, generator=g).to(DEV).to(kc.dtype)
+        pos = torch.arange(total[0], device=DEV)
+        kc[table[0, pos // 16].long(), pos % 16] = rows
+        wide = torch.zeros((S, width), dtype=torch.int32, device=DEV)
+        wide[:, :table.shape[1]] = table
+        q = torch.randn(new, H, DK, generator=g).to(qd).to(DEV).repeat(S, 1, 1)
+        out = torch.empty(S * new, H, DV, device=DEV, dtype=qd)
+        ops.mla_attention(out, q, kc, kc[..., :DV].transpose(1, 2).contiguous(), wide, lens, starts, 192 ** -0.5, new, 8)
+        first = out[:new].clone() if first is None else first
+        assert torch.equal(out[:new], first)

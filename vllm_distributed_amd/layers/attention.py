@@ -499,7 +499,8 @@ class MLAAttention(nn.Module):
         S = md.num_decode_seqs + md.num_prefill_seqs
         # few query tokens per sequence: split the keys further so the launch fills the chip.  The factor
         # depends on the batch size and the model's maximum length only, so eager steps and captured
-        # graphs of one batch size compute identical sums.
+        # graphs of one batch size compute identical sums.  (Rows of 576 values choose their own factor, from the same
+        # sizes and, per sequence, from its own length.)
         nsplit = 1
         if md.max_query_len <= 4:
             nsplit = ops.decode_num_splits(S * max(self.num_heads // 16, 1), 1, self.max_model_len)

@@ -404,8 +404,9 @@ def mla_attention(out: torch.Tensor, q: torch.Tensor, kc: torch.Tensor, vt: torc
         return out
     assert sink is None or (sink.dtype == torch.float32 and sink.is_contiguous() and sink.numel() == H)
     part_out = part_lse = None
-    # the kernels of some sizes cut the keys by the batch's real lengths and say themselves into how many parts at most
-    # (one where a table holds no more than a part's 128 keys: not worth the question, 1 us of a 22 us call)
+    # the kernels of some sizes cut a sequence's keys by its real length and say themselves into how many parts at most
+    # (one where a table holds no more than a part's 128 keys: not worth the question, 1 us of a 22 us call; an engine's
+    # tables hold more unless its longest request is that short)
     if num_splits > 1 or block_table.stride(0) * kc.shape[1] > 128:
         num_splits = N.lib().vda_mla_splits(seq_lens.shape[0], T, H, DK, kc.shape[1], block_table.stride(0),
                                             max(int(max_query_len), 1), float(scale), num_splits)
