@@ -1150,18 +1150,29 @@ def _moe_wide_ok(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, pairs: in
 @functools.lru_cache(maxsize=1024)
 def _moe_wide_pays(pairs: int, E: int, n1: int, k1: int, n2: int, k2: int) -> bool:
     """Do 256 x 256 tiles cost less than 128 x 256 ones, for ``pairs`` rows over E experts in products [rows, k] x [k, n tiles]?
-    A CU holds one tile at a time: a product takes rounds of 256 tiles (whole ones; beyond two rounds their ends overlap) of
-    K steps each, and a round of wide tiles costs 1.65 of the others (1.6 .. 1.9 where both fill their rounds).  An expert's rows
-    are its share and a standard deviation.  Layer times in us, 128-row tiles / 256-row tiles: 64 experts 2048 x 1024 with 160 rows
+    A CU holds one tile at a time: a product takes rounds of 256 tiles (whole ones while they are few; later their ends overlap)
+    of K steps each, and a round of wide tiles costs 1.65 of the others (1.6 .. 1.9 where both fill their rounds).  Both
+    estimates of the tiles have to say so: every expert takes its share of rows and a standard deviation, and the number to be
+    expected, where one expert in 64 that exceeds 256 rows opens a round (64 experts 2048 x 1024 with 219 rows each 341 us on
+    128-row tiles, 328 on these; with 225 378 / 414).  Layer times in us, 128-row tiles / 256-row tiles: 64 experts 2048 x 1024 with 160 rows
     each 322 / 305, 440 rows 561 / 492, 500 rows 618 / 575; 8 experts
     4096 x 14336 with 440 rows 1522 / 1260, 200 rows 834 / 917; 8 experts 1024 x 512, whose tiles leave CUs idle, with 360
-    rows 52 / 72.  Of 195 such points in the range above, this takes 93; four of them lose more than 2 %, the worst 7 %."""
+    rows 52 / 72; 16 experts 2048 x 1408 with 620 rows 282 / 312.  Of 200 such points in the range above (9 layers, 135 .. 1025
+    rows) this takes 107; three of them lose more than 2 %, the worst 4.3 %."""
     rows = pairs / E
+    sd = math.sqrt(rows)
 
-    def cost(rows_per_tile: int) -> float:
-        m_tiles = E * math.ceil((rows + math.sqrt(rows)) / rows_per_tile)
-        return sum(k * (-(-m_tiles * n // 256) if m_tiles * n <= 512 else m_tiles * n / 256) for n, k in ((n1, k1), (n2, k2)))
-    return 1.65 * cost(256) < cost(128)
+    def pays(tiles, whole_rounds: int) -> bool:
+        def cost(rows_per_tile: int) -> float:
+            m_tiles = tiles(rows_per_tile)
+            return sum(k * (-(-m_tiles * n // 256) if m_tiles * n <= 256 * whole_rounds else m_tiles * n / 256)
+                       for n, k in ((n1, k1), (n2, k2)))
+        return 1.65 * cost(256) < cost(128)
+
+    def expected(rows_per_tile: int) -> int:             # an expert opens tile j if it has more than j tiles' rows
+        return round(E * sum(math.erfc((j * rows_per_tile - rows) / sd / math.sqrt(2)) / 2
+                             for j in range(int(rows // rows_per_tile) + 3)))
+    return pays(lambda r: E * math.ceil((rows + sd) / r), 2) and pays(expected, 4)
 
 
 def _moe_tiled(x, w13, w2, topk_w, topk_ids, w13_scale, w2_scale, block_scales: bool = False,
