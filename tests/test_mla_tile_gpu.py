@@ -143,3 +143,18 @@ def test_error_is_that_of_rounding_the_result(new, total, H, dtype, fp8):
         at += n
     off, rounding = (out.double() - want).norm(), (want.to(dtype).double() - want).norm()
     assert float(off / rounding) < 1.02
+
+
+@pytest.mark.parametrize("new,keys,H", [(1, 9000, 16), (1, 2049, 128), (3, 4100, 16)])
+def test_one_long_sequence_in_many_pieces(new, keys, H):
+    """Alone in its batch a sequence is cut into up to 64 pieces; behind a table that could hold far more, too."""
+    kc, vt, table, lens, starts = _batch([new], [keys], 16, torch.bfloat16, 12)
+    wide = torch.zeros((1, 2048), dtype=torch.int32, device=DEV)
+    wide[:, :table.shape[1]] = table
+    blocks = -(-new * H // (128 if new * H > 32 else 32))
+    assert ops.N.lib().vda_mla_splits(1, new, H, DK, 16, 2048, new, 192 ** -0.5, 1) == 64 and blocks <= 2
+    q = torch.randn(new, H, DK, device=DEV).to(torch.bfloat16)
+    out = torch.empty(new, H, DV, device=DEV, dtype=torch.bfloat16)
+    ops.mla_attention(out, q, kc, vt, wide, lens, starts, 192 ** -0.5, new, 1)
+    want = R.mla_attention(q, kc, vt, wide, lens, starts, 192 ** -0.5)
+    torch.testing.assert_close(out.float(), want.float(), atol=12 * 2.0 ** -9, rtol=2.0 ** -8)

@@ -411,22 +411,30 @@ __global__ __launch_bounds__(64) void mla_reduce_kernel(T* out, const float* par
   float W = w_mine;
 #pragma unroll
   for (int o_ = 32; o_ > 0; o_ >>= 1) W += __shfl_xor(W, o_, 64);
-  // four neighbouring values a load, and four partitions' loads in flight
+  // four neighbouring values a load, and eight partitions' loads in flight (one row of 64 partitions is a chain of round trips:
+  // two in flight, each behind a branch on its weight, took 24 us)
   using V4 = typename Vec<T>::v4;
-  constexpr int PER = (DV / 4 + 63) / 64;
+  constexpr int PER = (DV / 4 + 63) / 64, U = 8;
   f32x4 o[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) o[i] = f32x4{0, 0, 0, 0};
-#pragma unroll 4
-  for (int s = 0; s < nsplit; ++s) {
-    const float w = __shfl(w_mine, s, 64);
-    if (w == 0.f) continue;
-    const float* po = part_out + (th * nsplit + s) * DV;
+  for (uint64_t left = __ballot(w_mine != 0.f); left;) {
+    f32x4 v[U][PER];
+    float w[U];
+    const int s0 = __builtin_ctzll(left);
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int d = 4 * (lane + 64 * i);
-      if (d < DV) o[i] += w * *reinterpret_cast<const f32x4*>(po + d);
+    for (int k = 0; k < U; ++k) {
+      const int s = left ? __builtin_ctzll(left) : s0;               // (past the last one: the first of these again, weightless)
+      w[k] = left ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w_mine), s)) : 0.f;
+      left &= left - 1;
+      const float* po = part_out + (th * nsplit + s) * DV;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) v[k][i] = *reinterpret_cast<const f32x4*>(po + min(4 * (lane + 64 * i), DV - 4));
     }
+#pragma unroll
+    for (int k = 0; k < U; ++k)
+#pragma unroll
+      for (int i = 0; i < PER; ++i) o[i] += w[k] * v[k][i];
   }
   const float inv = W > 0.f ? 1.f / W : 0.f;
   const long tok = th / H, head = th % H;
