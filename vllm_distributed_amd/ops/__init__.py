@@ -390,6 +390,13 @@ def mla_cache_write(kv_c: torch.Tensor, k_pe: torch.Tensor, kc: torch.Tensor, vt
            N.dt(kv_c.dtype), int(kc.dtype == torch.float8_e4m3fn), float(kv_scale), N.stream())
 
 
+@functools.lru_cache(maxsize=1024)
+def _mla_splits(S: int, T: int, H: int, DK: int, page: int, width: int, max_q: int, scale: float, num_splits: int) -> int:
+    """Parts that a sequence's keys can be cut into: the kernels of some sizes cut by a sequence's real length and say themselves
+    how many there are at most, from the sizes alone (so the answer is kept: asking is 1 us of a 22 us call)."""
+    return N.lib().vda_mla_splits(S, T, H, DK, page, width, max_q, scale, num_splits)
+
+
 def mla_attention(out: torch.Tensor, q: torch.Tensor, kc: torch.Tensor, vt: torch.Tensor, block_table: torch.Tensor,
                   seq_lens: torch.Tensor, q_start_loc: torch.Tensor, scale: float, max_query_len: int,
                   num_splits: int = 1, kv_scale: float = 1.0, window: int = 0,
@@ -403,20 +410,17 @@ def mla_attention(out: torch.Tensor, q: torch.Tensor, kc: torch.Tensor, vt: torc
         out.copy_(R.mla_attention(q, kc, vt, block_table, seq_lens, q_start_loc, scale, kv_scale, window, sink))
         return out
     assert sink is None or (sink.dtype == torch.float32 and sink.is_contiguous() and sink.numel() == H)
+    max_q = max(int(max_query_len), 1)
+    num_splits = _mla_splits(seq_lens.shape[0], T, H, DK, kc.shape[1], block_table.stride(0), max_q, float(scale), num_splits)
     part_out = part_lse = None
-    # the kernels of some sizes cut a sequence's keys by its real length and say themselves into how many parts at most
-    # (one where a table holds no more than a part's 128 keys: not worth the question, 1 us of a 22 us call; an engine's
-    # tables hold more unless its longest request is that short)
-    if num_splits > 1 or block_table.stride(0) * kc.shape[1] > 128:
-        num_splits = N.lib().vda_mla_splits(seq_lens.shape[0], T, H, DK, kc.shape[1], block_table.stride(0),
-                                            max(int(max_query_len), 1), float(scale), num_splits)
-    if num_splits > 1:
-        part_out = torch.empty((T, H, num_splits, DV), dtype=torch.float32, device=q.device)
-        part_lse = torch.empty((T, H, num_splits), dtype=torch.float32, device=q.device)
+    if num_splits > 1:                                   # the parts' rows, then their weights (one allocation, 1 us a call less than two)
+        part = torch.empty(T * H * num_splits * (DV + 1), dtype=torch.float32, device=q.device)
+        part_out = part.data_ptr()
+        part_lse = part_out + 4 * T * H * num_splits * DV
     assert q.stride(2) == 1 and q.stride(1) == DK and out.stride(2) == 1 and out.stride(1) == DV
     N.call("vda_mla_attention", out.data_ptr(), q.data_ptr(), kc.data_ptr(), vt.data_ptr(), block_table.data_ptr(),
-           seq_lens.data_ptr(), q_start_loc.data_ptr(), N.ptr(part_out), N.ptr(part_lse), seq_lens.shape[0], T, H, DK,
-           DV, kc.shape[1], block_table.stride(0), num_splits, max(int(max_query_len), 1), q.stride(0),
+           seq_lens.data_ptr(), q_start_loc.data_ptr(), part_out, part_lse, seq_lens.shape[0], T, H, DK,
+           DV, kc.shape[1], block_table.stride(0), num_splits, max_q, q.stride(0),
            out.stride(0), scale, N.dt(q.dtype), int(kc.dtype == torch.float8_e4m3fn), float(kv_scale), int(window),
            N.ptr(sink), N.stream())
     return out
