@@ -158,3 +158,17 @@ def test_one_long_sequence_in_many_pieces(new, keys, H):
     ops.mla_attention(out, q, kc, vt, wide, lens, starts, 192 ** -0.5, new, 1)
     want = R.mla_attention(q, kc, vt, wide, lens, starts, 192 ** -0.5)
     torch.testing.assert_close(out.float(), want.float(), atol=12 * 2.0 ** -9, rtol=2.0 ** -8)
+
+
+@pytest.mark.parametrize("page,scale", [(8, 192 ** -0.5), (24, 192 ** -0.5), (16, -(192 ** -0.5))])
+@pytest.mark.parametrize("new,total,H", [([1, 1], [40, 700], 16), ([5, 70], [5, 130], 16)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_what_the_tiles_do_not_take(page, scale, new, total, H, fp8):
+    """Pages off a power of two or below 16 tokens, and scales below zero, stay with the kernels of mla.hip."""
+    kc, vt, table, lens, starts = _batch(new, total, page, torch.float8_e4m3fn if fp8 else torch.bfloat16, 13)
+    q = torch.randn(sum(new), H, DK, device=DEV).to(torch.bfloat16)
+    out = torch.empty(sum(new), H, DV, device=DEV, dtype=torch.bfloat16)
+    for splits in (1, 3):
+        ops.mla_attention(out, q, kc, vt, table, lens, starts, scale, max(new), splits)
+        want = R.mla_attention(q, kc, vt, table, lens, starts, scale)
+        torch.testing.assert_close(out.float(), want.float(), atol=12 * 2.0 ** -9, rtol=2.0 ** -8)

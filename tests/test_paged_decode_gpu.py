@@ -36,7 +36,6 @@ def _check(lens, new, Hq, Hkv, D, BS, dt, fp8, nsplit, **kw):
     starts = torch.tensor([0] + new).cumsum(0).to(torch.int32).to(DEV)
     sl, table = torch.tensor(lens, dtype=torch.int32, device=DEV), table.to(DEV)
     out = torch.empty(T, Hq, D, dtype=dt, device=DEV)
-    print(f"\ncase S {S} D {D} BS {BS} fp8 {fp8} nsplit {nsplit} {kw}", flush=True)
     ops.paged_attention_decode(out, q, kc, vc, table, sl, starts, D ** -0.5, num_splits=nsplit, max_q_len=max(new),
                                k_scale=ks, v_scale=vs, **kw)
     chunk = kw.pop("chunk", 0)

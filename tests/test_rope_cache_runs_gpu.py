@@ -54,7 +54,6 @@ def test_runs(dt, runs, BS, Hq, Hkv, D, rot, neox, fp8):
     ks, vs = (0.5, 0.25) if fp8 else (1.0, 1.0)
     want = qkv.clone()
     q, k, v = want[:, :Hq * D], want[:, Hq * D:(Hq + Hkv) * D], want[:, (Hq + Hkv) * D:]
-    print(f"\ncase {runs[:3]} BS {BS} D {D} rot {rot}", flush=True)
     ops.rope_and_cache(pos, qkv, cs, kc, vc, slots, rot, D, Hq, Hkv, neox, ks, vs)
     R.rotary_embedding(pos, q, k, cs, rot, D, neox)
     u = 2.0 ** (-7 if dt == torch.bfloat16 else -10)

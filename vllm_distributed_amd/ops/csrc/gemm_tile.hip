@@ -323,7 +323,7 @@ __global__ __launch_bounds__(512, 1) void tile_gemm_kernel(const TileGemmArgs a)
 // that every reader of unit u + 1 passes first.  LDS image as above but with f(r) = (r >> 1) & 7: a lane reads
 // one chunk, 4 h + g, per row and half.  What bounds it is the chip's power at this density: dense products of this K run
 // at 1.1 (kernels here) to 1.4 PFLOP/s (library).
-// 8 experts 4096 x 14336, top 2, whole layer: 4099 tokens 3419 -> 3057 us (0.95 PFLOP/s with rows that exist), 3200 tokens
+// 8 experts 4096 x 14336, top 2, whole layer: 4099 tokens 3290 -> 2940 us (0.98 PFLOP/s with rows that exist), 3200 tokens
 // 2741 -> 2234; 16 experts 4096 x 6400, 5600 tokens 2076 -> 1746.
 template <typename T, int EPI>
 __global__ __launch_bounds__(512, 1) void moe_wide_gemm_kernel(const TileGemmArgs a) {

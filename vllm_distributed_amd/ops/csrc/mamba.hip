@@ -14,7 +14,8 @@ __device__ __forceinline__ float silu_f(float v) { return v / (1.f + __expf(-v))
 constexpr float LOG2E = 1.4426950408889634f, LOG2E_LO = 1.925963033500e-8f, LN2 = 0.6931471805599453f;
 // log(1 + e^v) = max(v, 0) + log(1 + e^-|v|).  The exponential's argument keeps its rounding error (e^v alone loses 1e-6 of
 // a step size at v = -15), and log(1 + e) the part of e that 1 + e rounds away (Kahan's correction, (e - d) / u).  About
-// 25 instructions where log1pf takes over 60; within 1.2e-7 of the 64-bit value for all v (log1pf of e^v: 1e-6).
+// 25 instructions where log1pf takes over 60; relative error at most 2.6e-7 between -87 and 80 (two million v in each of six
+// ranges, with correctly rounded exponential, logarithm and reciprocal; log1pf of e^v: 1e-6), zero below, where e^v is subnormal.
 __device__ __forceinline__ float softplus_f(float v) {
   const float t = fmaxf(-fabsf(v), -100.f);
   float p = t * LOG2E;

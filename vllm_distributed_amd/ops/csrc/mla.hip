@@ -474,7 +474,9 @@ static int launch_mla(const MlaParams& p, int S, int T_tokens, int max_q, bool f
   return 0;
 }
 
-// (a tile's halves of 16 rows lie in one page each; the tile kernel takes maxima before it scales)
+// Rows of 576 values go to mla_tile.hip wherever the engine's page sizes (16, 32, 64) and a softmax scale above zero are
+// given: a tile's halves of 16 rows lie in one page each there, and maxima are taken before they are scaled.  The kernels above
+// keep what else this entry point accepts for such rows: pages of other multiples of 8 tokens, scales of zero and below.
 static bool mla_takes_tiles(int DK, int BS, float scale) {
   return DK == 576 && BS >= 16 && (BS & (BS - 1)) == 0 && scale > 0.f;
 }
@@ -506,7 +508,7 @@ VDA_EXPORT int vda_mla_attention(void* out, const void* q, const void* kc, const
   p.scale = scale * (kv_fp8 ? kv_scale : 1.f); p.v_scale = kv_fp8 ? kv_scale : 1.f;
   p.window = window > 0 ? window : 0;
   p.sink = sink;
-  if (mla_takes_tiles(DK, BS, scale) && p.scale > 0.f) {
+  if (mla_takes_tiles(DK, BS, scale) && p.scale > 0.f) {              // (vt is not read)
     const MlaTilePlan plan = mla_tile_plan(S, T_tokens, H, BS, max_blocks, max_q);
     if (nsplit != plan.nsplit) return -4;
     const int rc = mla_tile_launch(p, plan, S, dtype, kv_fp8 != 0, st);
