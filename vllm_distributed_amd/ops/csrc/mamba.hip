@@ -222,27 +222,43 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(
   const float dv = D ? D[e] : 0.f;
   const float db = delta_bias ? delta_bias[e] : 0.f;
   const long bc_off = (long)(c / group_ch) * N + part * 16;
+  // the next token's inputs are on their way while this one's are worked on (past the end: the last token's again)
+  T nd, nu, nz = (T)0.f, nb[16], nc[16];
+  auto fetch = [&](int t) {
+    nd = delta[(long)t * d_stride + e];
+    nu = u[(long)t * u_stride + c];
+    if (MODE != 1 && z) nz = z[(long)t * z_stride + c];
+#pragma unroll
+    for (int n = 0; n < 16; ++n) nb[n] = Bm[(long)t * b_stride + bc_off + n];
+    if (MODE != 1) {
+#pragma unroll
+      for (int n = 0; n < 16; ++n) nc[n] = Cm[(long)t * c_stride + bc_off + n];
+    }
+  };
+  if (ta < tb) fetch(ta);
   for (int t = ta; t < tb; ++t) {
-    float dt = (float)delta[(long)t * d_stride + e] + db;
+    float dt = (float)nd + db;
+    const float x = (float)nu, zt = (float)nz;
+    T bt[16], ct[16];
+#pragma unroll
+    for (int n = 0; n < 16; ++n) { bt[n] = nb[n]; if (MODE != 1) ct[n] = nc[n]; }
+    fetch(min(t + 1, tb - 1));
     if (softplus) dt = softplus_f(dt);
-    const float x = (float)u[(long)t * u_stride + c];
     const float dx = dt * x;
-    const T* bp = Bm + (long)t * b_stride + bc_off;
-    const T* cp = Cm + (long)t * c_stride + bc_off;
     float y = 0.f;
 #pragma unroll
     for (int n = 0; n < 16; ++n) {
       const float dec = __expf(dt * a[n]);
-      h[n] = dec * h[n] + dx * (float)bp[n];
+      h[n] = dec * h[n] + dx * (float)bt[n];
       if (MODE == 1) pr[n] *= dec;
-      else y += (float)cp[n] * h[n];
+      else y += (float)ct[n] * h[n];
     }
     if (MODE != 1) {
 #pragma unroll
       for (int o = NL / 2; o > 0; o >>= 1) y += __shfl_xor(y, o, 64);
       if (part == 0) {
         y += dv * x;
-        if (z) y *= silu_f((float)z[(long)t * z_stride + c]);
+        if (z) y *= silu_f(zt);
         out[(long)t * o_stride + c] = (T)y;
       }
     }
