@@ -530,10 +530,13 @@ __global__ __launch_bounds__(256) void scan_carry_kernel(ScanArgs p, int N, int 
 
 // One token per sequence (or few): the state read and written is all there is (118 sequences of
 // 4096 x 128 states, 495 MB, with the convolution: 118 us).  A lane owns four states, a wave one contiguous KB of them, and
-// eight of those are in flight.
-template <typename T, int N, bool ASC>
+// K of those are in flight: eight where the states are many.  Few are a chain of trips to memory, so there two are taken by a wave
+// and all their inputs are asked for before the first store, which the compiler moves no load across (one sequence of
+// 4096 x 16 states 8.3 us with eight, 6.2 in the plain form; SCAN_FEW says how many are few).
+template <typename T, int N, bool ASC, int K>
 __global__ __launch_bounds__(256) void scan_step_kernel(ScanArgs p) {
-  constexpr int Q = N / 4, CW = 64 / Q, K = 8;          // lanes per channel, channels per KB
+  constexpr int Q = N / 4, CW = 64 / Q;                 // lanes per channel, channels per KB
+  constexpr bool AHEAD = K <= 2;
   const int s = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int sl = p.seq_lens[s];
   if (sl <= 0) return;
@@ -548,44 +551,63 @@ __global__ __launch_bounds__(256) void scan_step_kernel(ScanArgs p) {
     const int c = c0 + k * CW;
     h[k] = has_init && c < p.Ch ? *reinterpret_cast<const f32x4*>(hp + (long)c * N) : f32x4{0, 0, 0, 0};
   }
-  auto token = [&](int t, int c, f32x4 hk) {             // whole channels: the lanes of one come here together
+  // one channel's inputs of a token, and what is done with them (whole channels: the lanes of one come here together)
+  struct In { T delta, u, z, b[4], c[4]; float bias, d; f32x4 a; };
+  auto load = [&](int t, int c) {
+    In in;
     const int e = c / p.dt_div;
-    float dt = (float)((const T*)p.delta)[(long)t * p.d_stride + e] + (p.delta_bias ? p.delta_bias[e] : 0.f);
-    if (p.softplus) dt = softplus_f(dt);
-    const float x = (float)((const T*)p.u)[(long)t * p.u_stride + c], dx = dt * x;
+    in.delta = ((const T*)p.delta)[(long)t * p.d_stride + e];
+    in.u = ((const T*)p.u)[(long)t * p.u_stride + c];
+    in.z = p.z ? ((const T*)p.z)[(long)t * p.z_stride + c] : (T)0.f;
+    in.bias = p.delta_bias ? p.delta_bias[e] : 0.f;
+    in.d = p.D ? p.D[e] : 0.f;
     const long g = (long)(c / p.group_ch) * N + 4 * q;
-    const T* bp = (const T*)p.B + (long)t * p.b_stride + g;
-    const T* cp = (const T*)p.C + (long)t * p.c_stride + g;
-    f32x4 a;
-    if (ASC) { const float v = p.A[e]; a = f32x4{v, v, v, v}; }
-    else a = *reinterpret_cast<const f32x4*>(p.A + (long)c * N + 4 * q);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      in.b[i] = ((const T*)p.B)[(long)t * p.b_stride + g + i];
+      in.c[i] = ((const T*)p.C)[(long)t * p.c_stride + g + i];
+    }
+    if (ASC) { const float v = p.A[e]; in.a = f32x4{v, v, v, v}; }
+    else in.a = *reinterpret_cast<const f32x4*>(p.A + (long)c * N + 4 * q);
+    return in;
+  };
+  auto token = [&](int t, int c, f32x4 hk, const In& in) {
+    float dt = (float)in.delta + in.bias;
+    if (p.softplus) dt = softplus_f(dt);
+    const float x = (float)in.u, dx = dt * x;
     float y = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      hk[i] = fmaf(__builtin_amdgcn_exp2f(dt * (a[i] * LOG2E)), hk[i], dx * (float)bp[i]);
-      y = fmaf((float)cp[i], hk[i], y);
+      hk[i] = fmaf(__builtin_amdgcn_exp2f(dt * (in.a[i] * LOG2E)), hk[i], dx * (float)in.b[i]);
+      y = fmaf((float)in.c[i], hk[i], y);
     }
     *reinterpret_cast<f32x4*>(hp + (long)c * N) = hk;
     y = group_sum<Q>(y);
     if (q == 0) {
-      y += (p.D ? p.D[e] : 0.f) * x;
-      if (p.z) y *= silu_f((float)((const T*)p.z)[(long)t * p.z_stride + c]);
+      y += in.d * x;
+      if (p.z) y *= silu_f((float)in.z);
       ((T*)p.out)[(long)t * p.o_stride + c] = (T)y;
     }
   };
+  In in[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    if (AHEAD) in[k] = load(t0, min(c0 + k * CW, p.Ch - 1));
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int c = c0 + k * CW;
     if (c >= p.Ch) break;
-    token(t0, c, h[k]);
+    token(t0, c, h[k], AHEAD ? in[k] : load(t0, c));
   }
   // further tokens of a sequence, rare here: each lane's own states again from memory
 #pragma unroll 1
   for (int i = K; i < K * L; ++i) {
     const int c = c0 + i % K * CW;
-    if (c < p.Ch) token(t0 + i / K, c, *reinterpret_cast<const f32x4*>(hp + (long)c * N));
+    if (c < p.Ch) token(t0 + i / K, c, *reinterpret_cast<const f32x4*>(hp + (long)c * N), load(t0 + i / K, c));
   }
 }
+
+constexpr long SCAN_FEW = 5L << 20;                     // states of a one-token step (20 MB)
 
 // step: the sequences have one new token each (none and several are right too); otherwise channels in pairs (the caller checks that pairs share B, C and
 // are aligned).  nchunks > 1: ws_dt [S, nchunks, C] and ws_h [S, nchunks, C, N].
@@ -608,11 +630,13 @@ VDA_EXPORT int vda_selective_scan_pairs(void* out, const void* u, const void* de
   p.tile = SCAN_LDS / (2 * N * span);
   p.tile = p.tile > 64 ? 64 : p.tile > nl ? p.tile / nl * nl : p.tile;     // (whole blocks of tokens where they fit)
   const dim3 block(256), grid((C + wgch - 1) / wgch, S, nchunks > 1 ? nchunks : 1);
-  const int step_ch = 4 * 8 * (256 / N);
+  const bool few = (long)S * C * N < SCAN_FEW;
+  const int step_ch = 4 * (few ? 2 : 8) * (256 / N);
   const dim3 grid_step((C + step_ch - 1) / step_ch, S);
   const dim3 grid_carry((unsigned)(((long)C * (N / 4) + 255) / 256), S);
 #define K(TT, NN, AA) do {                                                                                              \
-    if (step) hipLaunchKernelGGL((scan_step_kernel<TT, NN, AA>), grid_step, block, 0, st, p);                              \
+    if (step && few) hipLaunchKernelGGL((scan_step_kernel<TT, NN, AA, 2>), grid_step, block, 0, st, p);                    \
+    else if (step) hipLaunchKernelGGL((scan_step_kernel<TT, NN, AA, 8>), grid_step, block, 0, st, p);                      \
     else if (nchunks <= 1) hipLaunchKernelGGL((scan_pairs_kernel<TT, NN, 0, AA>), grid, block, 0, st, p);                  \
     else {                                                                                                                 \
       hipLaunchKernelGGL((scan_pairs_kernel<TT, NN, 1, AA>), grid, block, 0, st, p);                                       \
