@@ -121,6 +121,44 @@ def test_short_sequences_take_the_form_that_fills_the_chip(monkeypatch, Ch, repe
     torch.testing.assert_close(a["ssm_state"], b["ssm_state"], atol=1e-4, rtol=1e-4)
 
 
+@pytest.mark.parametrize("Ch,N,heads,repeat,longest,form", [(1024, 128, 16, 3, 33, "vda_selective_scan"), (1024, 128, 16, 4, 33, "vda_selective_scan_pairs"),
+                                                            (1024, 256, 16, 2, 33, "vda_selective_scan_pairs"), (1024, 128, 16, 1, 8, "vda_selective_scan"),
+                                                            (1024, 128, 16, 2, 8, "vda_selective_scan_pairs"), (64, 64, 2, 1, 33, "vda_selective_scan_pairs")])
+def test_wide_states_of_few_short_sequences(monkeypatch, Ch, N, heads, repeat, longest, form):
+    """As above for 64, 128 and 256 states a channel, where lanes of 16 states count."""
+    new, ctx = [longest - 2, longest - 1, longest, 1, 0] * repeat, [0, 3, 0, 4, 0] * repeat
+    a = _scan_inputs(new, ctx, Ch, N, heads, 1, torch.float32, 3)
+    names = ("u", "delta", "A", "B", "C", "D", "z", "delta_bias", "ssm_state")
+    b = {k: v.clone() if isinstance(v, torch.Tensor) else v for k, v in a.items()}
+    called, call = [], ops.N.call
+    monkeypatch.setattr(ops.N, "call", lambda name, *args: (called.append(name), call(name, *args))[1])
+    y = ops.selective_scan(**a, max_query_len=longest)
+    assert called == [form]
+    want = R.selective_scan(*(b[k] for k in names), b["query_start_loc"], b["seq_lens"], b["block_table"])
+    # as in test_selective_scan_forms, with N / 16 as many terms in a sum
+    torch.testing.assert_close(y, want, atol=3e-4 * (N // 16) ** 0.5, rtol=1e-4)
+    torch.testing.assert_close(a["ssm_state"], b["ssm_state"], atol=1e-4, rtol=1e-4)
+
+
+@pytest.mark.parametrize("Ch,N,S", [(16, 16, 3), (70, 16, 2), (4096, 16, 79), (4096, 16, 80), (4096, 16, 81), (33, 128, 3), (2048, 64, 39), (2048, 64, 41),
+                                    (66, 256, 2)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_one_token_of_few_and_of_many_sequences(Ch, N, S, dtype):
+    """Both splits of the one-token kernel, on either side of where they change (5 Mi states) and where channels end inside a wave."""
+    new, ctx = [1] * S, [i % 3 for i in range(S)]
+    a = _scan_inputs(new, ctx, Ch, N, 0 if N == 16 else 1 if Ch % 2 else 2, 1, dtype, 6)
+    names = ("u", "delta", "A", "B", "C", "D", "z", "delta_bias", "ssm_state")
+    b = {k: v.clone() if isinstance(v, torch.Tensor) else v for k, v in a.items()}
+    y = ops.selective_scan(**a, max_query_len=1)
+    want = R.selective_scan(*(b[k] for k in names), b["query_start_loc"], b["seq_lens"], b["block_table"])
+    tol = 3e-4 * max(N // 16, 1) ** 0.5
+    if dtype == torch.float32:
+        torch.testing.assert_close(y, want, atol=tol, rtol=1e-4)
+    else:                                                                   # the reference sums in fp32 as well; one rounding each: 2^-8
+        torch.testing.assert_close(y.float(), want.float(), atol=tol, rtol=2.0 ** -7)
+    torch.testing.assert_close(a["ssm_state"], b["ssm_state"], atol=1e-4, rtol=1e-4)
+
+
 @pytest.mark.parametrize("setting,tokens,offset,chunked", [(None, 200, 1, False), (None, 256, 1, True), ("64", 80, 1, True),
                                                           ("64", 80, 0, True), ("512", 300, 0, False), ("512", 300, 1, False)])
 def test_the_chunk_setting_holds_for_both_forms(monkeypatch, setting, tokens, offset, chunked):

@@ -1466,13 +1466,15 @@ def selective_scan(u: torch.Tensor, delta: torch.Tensor, A: torch.Tensor, B: tor
         and 2 * Nst * min(-(-wgch // gch) + 1, -(-Ch // gch)) <= 8192
         and all(t.stride(0) % 2 == 0 and t.data_ptr() % (2 * eb) == 0
                 for t in (u, out) + ((delta,) if rep == 1 else ()) + ((z,) if z is not None else ()))))
-    # In one pass (below 96 tokens) pairs leave half as many lanes, each with twice the work: where 16 states a channel are less
-    # than 640 waves of pairs, the plain form is ahead (us, plain / pairs: 1 sequence of 40 tokens 31 / 41, 16 of 17 with
-    # 4096 channels, 512 waves, 20 / 25; 64 of 40 with 1536, 768 waves, 56 / 51).  More states share lanes in both forms
-    # and gain by the staged B and C at any size.
+    # In one pass (below 96 tokens) pairs leave half as many lanes, each with twice the work: with few of them the plain form is
+    # ahead, whose lanes of 16 states are counted here.  Scan times in us, plain / pairs: 16 states a channel, one sequence of 40 tokens
+    # before its inputs came a token ahead 31 / 41, 24 of 43 tokens at most with 4096 channels (98 304 lanes) 41 / 47 since, 64
+    # (262 144) 63 / 60, of 8 tokens at most 22.0 / 18.6; 128 states, 43 tokens: 4 of 4096 (131 072) 35 / 39, six 46 / 39; 3 tokens:
+    # two 6.0 / 7.6, three 8.3 / 8.0.  32 and 64 states gain by the staged B and C at any size (one sequence of 2048 x 64, 20
+    # tokens, 16.7 / 15.5).
     set_min = envs.VDA_SCAN_CHUNK_MIN_TOKENS
-    if paired and not step and Nst == 16 and max_query_len < (96 if set_min is None else set_min) and S * Ch < 640 * 128:
-        paired = False
+    if paired and not step and Nst not in (32, 64) and max_query_len < (96 if set_min is None else set_min):
+        paired = S * Ch * (Nst // 16) >= (163840 if Nst > 16 and max_query_len > 8 else 81920)
     chunk, nchunks, ws_p, ws_h = 0, 1, None, None
     # unless the setting says otherwise, from 96 tokens on in pairs (seven prompts of 82 tokens on average, 4096 x 16: 140 us in
     # one pass, 82 in chunks of 32), from 256 on in the plain form, where more passes over more states pay later
