@@ -235,6 +235,7 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(AttnParams p) {
 // waves per SIMD it spills 15 and takes 177.  Non-temporal loads: e4m3 rows 6 % faster, 16-bit ones, of which a lane's pieces share
 // lines, up to 60 % slower.
 constexpr unsigned DECODE_RANKED = 512;    // two workgroups per CU are resident
+constexpr int DECODE_APART = 256;          // keys
 template <typename T, int D, int BS, int NCT, bool F8>
 __global__ __launch_bounds__(256) void paged_decode_kernel(AttnParams p) {
   using V8 = typename Vec<T>::v8;
@@ -252,7 +253,9 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(AttnParams p) {
   // Workgroup -> (sequence, part, kv head), heads fastest.  A grid larger than the chip holds takes its sequences longest
   // first: a long one that starts last would run alone.  Every wave finds its own, the blockIdx.z-th largest of the lengths,
   // bit by bit: no barrier, and no more than some 25 dependent counts before the first key (counting ranks over LDS took
-  // 256 of 300 keys, 64 / 8 heads, from 70 to 90 us).  Lengths within an eighth of the first one's stay in their order.
+  // 256 of 300 keys, 64 / 8 heads, from 70 to 90 us).  Lengths within an eighth or 256 keys of the first one's stay in their order: a
+  // workgroup of few keys costs less than looking for it (250 of 12 .. 87 keys, 32 / 8 heads, 31.5 us in order of length, 28.4 in the
+  // batch's; e4m3 33.4 / 30.2).
   const int kvh = blockIdx.x, part = blockIdx.y;
   int seq = blockIdx.z;
   int qs = p.q_start_loc[seq], q_end = p.q_start_loc[seq + 1], seq_len = p.seq_lens[seq];
@@ -263,7 +266,7 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(AttnParams p) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int at = lane + 64 * i, len = p.seq_lens[min(at, p.num_seqs - 1)];
-      differs |= abs(len - base) > base >> 3;
+      differs |= abs(len - base) > max(base >> 3, DECODE_APART);
       key[i] = at < p.num_seqs ? min(max(len, 0), (1 << bits) - 1) << 8 | (255 - at) : -1;
     }
     if (__any(differs)) {
