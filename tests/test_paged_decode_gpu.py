@@ -81,3 +81,10 @@ def test_longest_first(S, Hkv, nsplit):
 def test_order_of_large_batches(S, lens):
     lens = [lens(i, S) for i in range(S)]
     _check(lens, [1] * S, 16, 8, 128, 16, torch.bfloat16, S == 129, 1)
+
+
+# the merge of the parts: one wave's last count, four waves' first, the most; parts with and without keys
+@pytest.mark.parametrize("nsplit", [2, 8, 9, 64])
+@pytest.mark.parametrize("D", [64, 96, 128, 192, 256])
+def test_merge_of_parts(D, nsplit):
+    _check([1, 40, 300, 2100, 0], [1] * 5, 6, 2, D, 16, torch.bfloat16, False, nsplit)
