@@ -176,3 +176,40 @@ def test_the_chunk_setting_holds_for_both_forms(monkeypatch, setting, tokens, of
     want = R.selective_scan(*(b[k] for k in names), b["query_start_loc"], b["seq_lens"], b["block_table"])
     torch.testing.assert_close(y, want, atol=3e-4, rtol=1e-4)              # as in test_selective_scan_forms
     torch.testing.assert_close(a["ssm_state"], b["ssm_state"], atol=1e-4, rtol=1e-4)
+
+
+@pytest.mark.parametrize("Ch,groups,offset", [(64, 1, 0), (64, 2, 0), (72, 1, 0), (36, 1, 1), (7, 1, 0), (260, 1, 2)])
+@pytest.mark.parametrize("new,ctx", [([96, 1, 8, 9, 0], [0, 4, 0, 1, 0]),            # eight tokens at a time, tiles of 32
+                                     ([31, 32, 33, 130], [2, 0, 1, 0]), ([64, 65, 97, 2], [0, 5, 0, 3])])
+@pytest.mark.parametrize("chunks", [False, True])
+def test_two_states_a_lane(monkeypatch, new, ctx, Ch, groups, offset, chunks):
+    # channels that do not fill a workgroup, rows that are read one value at a time, chunks of one tile (the setting asks for them)
+    if chunks:
+        monkeypatch.setenv("VDA_SCAN_CHUNK_MIN_TOKENS", "96")
+    a = _scan_inputs(new, ctx, Ch, 16, 0, groups, torch.float32, Ch + len(new), offset)
+    if not offset:
+        a = {k: v.contiguous() if isinstance(v, torch.Tensor) else v for k, v in a.items()}
+    names = ("u", "delta", "A", "B", "C", "D", "z", "delta_bias", "ssm_state")
+    b = {k: v.clone() if isinstance(v, torch.Tensor) else v for k, v in a.items()}
+    called, call = [], ops.N.call
+    monkeypatch.setattr(ops.N, "call", lambda name, *args: (called.append((name, args[27], args[29])), call(name, *args))[1])
+    y = ops.selective_scan(**a, max_query_len=max(new))
+    assert called == [("vda_selective_scan_pairs", 2, -(-max(new) // 32) if chunks else 1)]
+    want = R.selective_scan(*(b[k] for k in names), b["query_start_loc"], b["seq_lens"], b["block_table"], num_groups=groups)
+    torch.testing.assert_close(y, want, atol=3e-4, rtol=1e-4)              # as in test_selective_scan_forms
+    torch.testing.assert_close(a["ssm_state"], b["ssm_state"], atol=1e-4, rtol=1e-4)
+
+
+@pytest.mark.parametrize("left_out", ["z", "D", "delta_bias"])
+def test_two_states_a_lane_without(left_out):
+    a = _scan_inputs([100, 3], [0, 2], 64, 16, 0, 1, torch.bfloat16, 9)
+    a[left_out] = None
+    if left_out == "D":                                                    # step sizes as they are: none below zero
+        a["delta"], a["delta_bias"] = a["delta"].abs(), a["delta_bias"].abs() * 0.1
+    names = ("u", "delta", "A", "B", "C", "D", "z", "delta_bias", "ssm_state")
+    b = {k: v.clone() if isinstance(v, torch.Tensor) else v for k, v in a.items()}
+    y = ops.selective_scan(**a, softplus=False, max_query_len=100) if left_out == "D" else ops.selective_scan(**a, max_query_len=100)
+    want = R.selective_scan(*(b[k] for k in names), b["query_start_loc"], b["seq_lens"], b["block_table"], softplus=left_out != "D")
+    # one bf16 rounding of y
+    torch.testing.assert_close(y.float(), want.float(), atol=0.05, rtol=2 ** -7)
+    torch.testing.assert_close(a["ssm_state"], b["ssm_state"], atol=1e-4, rtol=1e-4)

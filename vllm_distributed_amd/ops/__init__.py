@@ -1473,15 +1473,28 @@ def selective_scan(u: torch.Tensor, delta: torch.Tensor, A: torch.Tensor, B: tor
     # two 6.0 / 7.6, three 8.3 / 8.0.  32 and 64 states gain by the staged B and C at any size (one sequence of 2048 x 64, 20
     # tokens, 16.7 / 15.5).
     set_min = envs.VDA_SCAN_CHUNK_MIN_TOKENS
-    if paired and not step and Nst not in (32, 64) and max_query_len < (96 if set_min is None else set_min):
+    few_tokens = max_query_len < (96 if set_min is None else set_min)
+    if paired and not step and Nst not in (32, 64) and few_tokens:
         paired = S * Ch * (Nst // 16) >= (163840 if Nst > 16 and max_query_len > 8 else 81920)
+    # Two states a lane (Mamba: 16 of them, a decay rate each, a step size per channel): one pass where pairs take two.  A
+    # workgroup's setup and its tile of 32 tokens want some tokens to work on: pairs / this, 128 sequences of 20 tokens at most
+    # x 8192 channels 89 / 125 us, of 34 x 4096 80 / 79, 100 of 43 x 4096 87 / 75, 64 of 51 69 / 56, three of 1558 x 8192 300 / 163.
+    lanes = not step and Nst == 16 and A.dim() == 2 and rep == 1 and (num_groups == 1 or gch % 32 == 0) \
+        and ssm_state.data_ptr() % 16 == 0 and A.data_ptr() % 16 == 0 and (not few_tokens or paired and max_query_len >= 40)
+    paired = paired or lanes
     chunk, nchunks, ws_p, ws_h = 0, 1, None, None
     # unless the setting says otherwise, from 96 tokens on in pairs (seven prompts of 82 tokens on average, 4096 x 16: 140 us in
-    # one pass, 82 in chunks of 32), from 256 on in the plain form, where more passes over more states pay later
-    if max_query_len >= ((96 if paired else 256) if set_min is None else set_min):
+    # one pass, 82 in chunks of 32), from 256 on in the plain form, where more passes over more states pay later, and with
+    # two states a lane, whose waves (eight channels each) are only cut where they leave SIMDs with less than two: us in one
+    # pass / cut, 4096 channels: 241 tokens 32 / 32, 402 43 / 33, 1609 148 / 70; 8192: 322 tokens 31 / 37, 1609 155 / 119;
+    # 16384 channels and sequences: 1212 tokens 126 / 128; 24576: 1558 tokens 163 / 206
+    if max_query_len >= ((96 if paired and not lanes else 256) if set_min is None else set_min):
         # lanes per channel: N / 16, or as many for a pair of them
         least = 32 if paired else 64
-        want = -(-524288 // (S * (Ch // (2 if paired else 1)) * (Nst // 16)))
+        if lanes:
+            want = -(-65536 // (S * Ch)) if S * Ch < 16384 else 1
+        else:
+            want = -(-524288 // (S * (Ch // (2 if paired else 1)) * (Nst // 16)))
         if want > 1:
             chunk = max(least, -(-(-(-max_query_len // want)) // least) * least)
             nchunks = -(-max_query_len // chunk)
@@ -1494,7 +1507,7 @@ def selective_scan(u: torch.Tensor, delta: torch.Tensor, A: torch.Tensor, B: tor
             u.stride(0), delta.stride(0), B.stride(0), C.stride(0), z.stride(0) if z is not None else 0, out.stride(0),
             rep, int(A.dim() == 1), gch, int(softplus))
     if paired:
-        N.call("vda_selective_scan_pairs", *args, int(step), chunk, nchunks, N.ptr(ws_p), N.ptr(ws_h), N.dt(u.dtype), N.stream())
+        N.call("vda_selective_scan_pairs", *args, 2 if lanes else int(step), chunk, nchunks, N.ptr(ws_p), N.ptr(ws_h), N.dt(u.dtype), N.stream())
     else:
         N.call("vda_selective_scan", *args, chunk, nchunks, N.ptr(ws_p), N.ptr(ws_h), N.dt(u.dtype), N.stream())
     return out

@@ -307,7 +307,7 @@ __global__ __launch_bounds__(256) void scan_combine_kernel(float* __restrict__ w
 // The output pass of several chunks reads its start states from the workspace alone: the last chunk leaves its end state in
 // the request's slot while the first one may not have begun, so the carry kernel puts the slot's state aside first.
 // Bound by vector issue: per state and token exp2 (4 slots), its argument, two for the state and one for y.
-// 3325 tokens of 8192 channels x 16 states, three sequences: both passes 637 -> 320 us (the exponentials alone are 90);
+// 3325 tokens of 8192 channels x 16 states, three sequences: both passes 637 -> 320 us;
 // 1100 tokens of 64 heads x 64 x 128 states: 990 -> 283 with the convolution.
 struct ScanArgs {
   void* out;
@@ -488,6 +488,167 @@ __global__ __launch_bounds__(256) void scan_pairs_kernel(ScanArgs p) {
   }
 }
 
+// ---- selective scan, two states a lane ---------------------------------------------------------------------------------
+// 16 states with decay rates of their own (Mamba): eight lanes share a channel, two states each, so that three prompts of 8192
+// channels are 3072 waves and walk their tokens in one pass where the pairs above took two.  A SIMD issues at its full rate from
+// two waves on (one alone: every 8 cycles instead of 4, measured), which is what chunks are still made for where sequences
+// and channels are few.
+// Everything that a (token, channel) needs once is done while a tile of 32 tokens x 32 channels is staged: a thread takes four
+// channels of a token, applies the softplus and leaves (dt, dt * u) in LDS; the gate and D join when the tile's sums come
+// back through LDS.  The recurrence itself then reads two LDS words a token, B and C of its two states beside each other.
+// The sums over a channel's eight lanes are transposed ones: of eight tokens' partial sums each lane sends the half that its
+// partner finishes, 21 instructions for eight tokens instead of 24 additions and eight selections, and lane k ends with token k's.
+// Per state and token: exp2 (two issue slots), its argument, two for the state, one for y: 69 us for 3325 tokens of 8192 channels
+// x 16 states at the full rate, with the sums and the staging about twice that: 298 (pairs) -> 163 us; 16 sequences of 323 tokens
+// at most 291 -> 126; one of 1609 169 -> 119, with 4096 channels 105 -> 70.
+constexpr int LN_TT = 32, LN_CH = 32, LN_YS = 40;       // tokens and channels of a tile; floats between two tokens' sums
+template <typename T> __device__ __forceinline__ void load_few(const T* p, float (&v)[4], bool vec, int last) {
+  typedef T v4_t __attribute__((ext_vector_type(4)));
+  if (vec) {
+    const v4_t q = *reinterpret_cast<const v4_t*>(p);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = (float)q[i];
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = (float)p[min(i, last)];
+  }
+}
+// a chunk's MODE, as in the pairs above; vec: rows of four channels may be read and written at once
+template <typename T, int MODE>
+__global__ __launch_bounds__(256) void scan_lanes_kernel(ScanArgs p, int vec) {
+  constexpr int N = 16;
+  typedef T v4_t __attribute__((ext_vector_type(4)));
+  __shared__ __attribute__((aligned(16))) float dd[LN_TT][LN_CH][2], bc[LN_TT][8][4], ys[LN_TT][LN_YS];
+  const int s = blockIdx.y;
+  const int sl = p.seq_lens[s];
+  if (sl <= 0) return;
+  const int t0 = p.qsl[s], L = p.qsl[s + 1] - t0;
+  const int nch = MODE == 0 ? 1 : min((L + p.chunk - 1) / p.chunk, (int)gridDim.z), kch = MODE == 0 ? 0 : blockIdx.z;
+  if (kch >= nch || (MODE == 1 && kch == nch - 1)) return;
+  const bool last = kch == nch - 1;
+  const int ta = MODE == 0 ? 0 : kch * p.chunk, tb = last ? L : ta + p.chunk;
+  if (ta >= tb) return;
+  const bool from_state = sl - L > 0 && kch == 0;
+  // neighbouring workgroups share lines of 128 bytes: they go to one XCD (workgroups are dealt to the eight in turn)
+  const int nb = gridDim.x, cb = nb % 8 ? (int)blockIdx.x : (int)(blockIdx.x % 8) * (nb / 8) + (int)(blockIdx.x / 8);
+  const int cw = cb * LN_CH;
+  const int lane = threadIdx.x & 63, q = lane & 7, mych = (threadIdx.x >> 6) * 8 + (lane >> 3);
+  const int c = min(cw + mych, p.Ch - 1);
+  const bool mine = cw + mych < p.Ch;
+  float* hp = p.state + ((long)p.block_table[s * p.bt_stride] * p.Ch + c) * N + 2 * q;
+  const long wc = ((long)s * gridDim.z + kch) * p.Ch + c;
+  f32x2 a = *reinterpret_cast<const f32x2*>(p.A + (long)c * N + 2 * q), h = {0, 0};
+  a[0] *= LOG2E;
+  a[1] *= LOG2E;
+  if (MODE == 2 && kch > 0) h = *reinterpret_cast<const f32x2*>(p.ws_h + (wc - p.Ch) * N + 2 * q);
+  else if (MODE == 2 && from_state && nch > 1) h = *reinterpret_cast<const f32x2*>(p.ws_h + (wc + (long)(nch - 1) * p.Ch) * N + 2 * q);
+  else if (from_state) h = *reinterpret_cast<const f32x2*>(hp);
+
+  // staging: this thread's token of a tile, its four channels, and its two states' B and C
+  const int st = threadIdx.x >> 3, sc = 4 * (threadIdx.x & 7), c4 = min(cw + sc, p.Ch - 1), left = p.Ch - 1 - c4;
+  const long g = (long)(cw / p.group_ch) * N + 2 * (threadIdx.x & 7);
+  const T* U = (const T*)p.u + (long)t0 * p.u_stride + c4;
+  const T* Dt = (const T*)p.delta + (long)t0 * p.d_stride + c4;
+  const T* Z = p.z ? (const T*)p.z + (long)t0 * p.z_stride + c4 : nullptr;
+  const T* B = (const T*)p.B + (long)t0 * p.b_stride + g;
+  const T* C = (const T*)p.C + (long)t0 * p.c_stride + g;
+  T* O = (T*)p.out + (long)t0 * p.o_stride + c4;
+  float dv[4], db[4], nd[4], nu[4], nz[4] = {0, 0, 0, 0}, nbc[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    dv[i] = p.D ? p.D[c4 + min(i, left)] : 0.f;
+    db[i] = p.delta_bias ? p.delta_bias[c4 + min(i, left)] : 0.f;
+  }
+  auto fetch = [&](int tt) {
+    const long t = tt + st;
+    if (t >= tb) return;
+    load_few(Dt + t * p.d_stride, nd, vec, left);
+    load_few(U + t * p.u_stride, nu, vec, left);
+    if (MODE != 1 && Z) load_few(Z + t * p.z_stride, nz, vec, left);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      nbc[i] = (float)B[t * p.b_stride + i];
+      nbc[2 + i] = MODE != 1 ? (float)C[t * p.c_stride + i] : 0.f;
+    }
+  };
+  fetch(ta);
+  float sdt[4] = {0, 0, 0, 0};
+  for (int tt = ta; tt < tb; tt += LN_TT) {
+    const bool there = tt + st < tb;                    // no token: the state stays as it is
+    float cu[4], cz[4];
+    f32x4 w[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}}, wb = {0, 0, 0, 0};
+    if (there) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float dt = nd[i] + db[i];
+        if (p.softplus) dt = softplus_f(dt);
+        if (MODE == 1) sdt[i] += dt;
+        cu[i] = nu[i];
+        cz[i] = nz[i];
+        w[i >> 1][2 * (i & 1)] = dt;
+        w[i >> 1][2 * (i & 1) + 1] = dt * nu[i];
+        wb[i] = nbc[i];
+      }
+    }
+    *reinterpret_cast<f32x4*>(&dd[st][sc][0]) = w[0];
+    *reinterpret_cast<f32x4*>(&dd[st][sc + 2][0]) = w[1];
+    *reinterpret_cast<f32x4*>(&bc[st][threadIdx.x & 7][0]) = wb;
+    __syncthreads();
+    if (tt + LN_TT < tb) fetch(tt + LN_TT);             // under this tile's arithmetic
+    const int nt = min(LN_TT, tb - tt);
+    for (int tk = 0; tk < nt; tk += 8) {
+      float y[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const f32x2 d = *reinterpret_cast<const f32x2*>(&dd[tk + k][mych][0]);
+        const f32x4 b = *reinterpret_cast<const f32x4*>(&bc[tk + k][q][0]);
+        h[0] = fmaf(__builtin_amdgcn_exp2f(d[0] * a[0]), h[0], d[1] * b[0]);
+        h[1] = fmaf(__builtin_amdgcn_exp2f(d[0] * a[1]), h[1], d[1] * b[1]);
+        y[k] = fmaf(b[3], h[1], b[2] * h[0]);
+      }
+      if (MODE != 1) {
+        auto meet = [](float keep, float send, auto ctrl) {
+          return keep + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(send), decltype(ctrl)::value, 0xf, 0xf, true));
+        };
+        const bool b2 = q & 4, b1 = q & 2, b0 = q & 1;
+        float y4[4], y2[2];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) y4[k] = meet(b2 ? y[k + 4] : y[k], b2 ? y[k] : y[k + 4], std::integral_constant<int, 0x141>());
+#pragma unroll
+        for (int k = 0; k < 2; ++k) y2[k] = meet(b1 ? y4[k + 2] : y4[k], b1 ? y4[k] : y4[k + 2], std::integral_constant<int, 0x1b>());
+        ys[tk + q][mych] = meet(b0 ? y2[1] : y2[0], b0 ? y2[0] : y2[1], std::integral_constant<int, 0xb1>());
+      }
+    }
+    __syncthreads();
+    if (MODE != 1 && there && cw + sc < p.Ch) {
+      const f32x4 y = *reinterpret_cast<const f32x4*>(&ys[st][sc]);
+      v4_t o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float v = fmaf(dv[i], cu[i], y[i]);
+        o[i] = (T)(Z ? v * silu_f(cz[i]) : v);
+      }
+      T* to = O + (long)(tt + st) * p.o_stride;
+      if (vec) *reinterpret_cast<v4_t*>(to) = o;
+      else
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (i <= left) to[i] = o[i];
+    }
+  }
+  if (MODE == 1) {                                      // a channel's sum of dt: over the 32 threads that staged its tokens
+    __syncthreads();
+    *reinterpret_cast<f32x4*>(&ys[st][sc]) = f32x4{sdt[0], sdt[1], sdt[2], sdt[3]};
+    __syncthreads();
+    if (threadIdx.x < LN_CH && cw + (int)threadIdx.x < p.Ch) {
+      float sum = 0.f;
+      for (int t = 0; t < LN_TT; ++t) sum += ys[t][threadIdx.x];
+      p.ws_dt[((long)s * gridDim.z + kch) * p.Ch + cw + threadIdx.x] = sum;
+    }
+  }
+  if (mine && (MODE == 1 || last)) *reinterpret_cast<f32x2*>(MODE == 1 ? p.ws_h + wc * N + 2 * q : hp) = h;
+}
+
 // One thread per (sequence, channel, four states): walk the chunks, leaving in chunk k's place its TRUE end state, which is
 // where chunk k + 1 starts.  (The first chunk's is true already.)  The last chunk's place, which has no end state yet, takes
 // the state that the sequence continues from.
@@ -609,21 +770,23 @@ __global__ __launch_bounds__(256) void scan_step_kernel(ScanArgs p) {
 
 constexpr long SCAN_FEW = 5L << 20;                     // states of a one-token step (20 MB)
 
-// step: the sequences have one new token each (none and several are right too); otherwise channels in pairs (the caller checks that pairs share B, C and
-// are aligned).  nchunks > 1: ws_dt [S, nchunks, C] and ws_h [S, nchunks, C, N].
+// form 1: the sequences have one new token each (none and several are right too); 2: two states a lane (16 of them, a rate each, a step size per
+// channel, 32 channels on a boundary of 32 share B and C); 0: channels in pairs (the caller checks that pairs share B, C and are aligned).  nchunks > 1: ws_dt [S, nchunks, C] and ws_h [S, nchunks, C, N].
 VDA_EXPORT int vda_selective_scan_pairs(void* out, const void* u, const void* delta, const float* A, const void* Bm,
                                         const void* Cm, const float* D, const void* z, const float* delta_bias,
                                         float* ssm_state, const int* qsl, const int* seq_lens, const int* block_table,
                                         long bt_stride, int S, int C, int N, long u_stride, long d_stride, long b_stride,
                                         long c_stride, long z_stride, long o_stride, int dt_div, int a_scalar,
-                                        int group_ch, int softplus, int step, int chunk, int nchunks, float* ws_dt,
+                                        int group_ch, int softplus, int form, int chunk, int nchunks, float* ws_dt,
                                         float* ws_h, int dtype, hipStream_t st) {
   if (S <= 0 || C <= 0) return 0;
   if (N != 16 && N != 32 && N != 64 && N != 128 && N != 256) return -1;
   if (dt_div < 1 || group_ch < 1) return -2;
+  const bool step = form == 1, lanes = form == 2;
+  if (lanes && (N != 16 || a_scalar || dt_div != 1 || (group_ch < C && group_ch % LN_CH))) return -4;
   const int nl = N / 16, wgch = 512 / nl;
   const int span = min((wgch + group_ch - 1) / group_ch + 1, (C + group_ch - 1) / group_ch);
-  if (!step && ((C & 1) || (group_ch & 1) || (dt_div > 1 && (dt_div & 1)) || 2 * N * span > SCAN_LDS)) return -4;
+  if (form == 0 && ((C & 1) || (group_ch & 1) || (dt_div > 1 && (dt_div & 1)) || 2 * N * span > SCAN_LDS)) return -4;
   if (nchunks > 1 && (!ws_dt || !ws_h || chunk < 1)) return -4;
   ScanArgs p{out, u, delta, A, Bm, Cm, D, z, delta_bias, ssm_state, qsl, seq_lens, block_table, bt_stride, u_stride, d_stride,
              b_stride, c_stride, z_stride, o_stride, C, dt_div, group_ch, softplus, chunk, 0, ws_dt, ws_h};
@@ -634,6 +797,17 @@ VDA_EXPORT int vda_selective_scan_pairs(void* out, const void* u, const void* de
   const int step_ch = 4 * (few ? 2 : 8) * (256 / N);
   const dim3 grid_step((C + step_ch - 1) / step_ch, S);
   const dim3 grid_carry((unsigned)(((long)C * (N / 4) + 255) / 256), S);
+  const long eb = dtype == VDA_F32 ? 4 : 2;
+  const auto apart = [&](const void* at, long stride) { return stride % 4 == 0 && (uintptr_t)at % (4 * eb) == 0; };
+  const int vec = C % 4 == 0 && apart(u, u_stride) && apart(delta, d_stride) && (!z || apart(z, z_stride)) && apart(out, o_stride);
+  const dim3 grid_lanes((C + LN_CH - 1) / LN_CH, S, nchunks > 1 ? nchunks : 1);
+#define K2(TT) do {                                                                                                     \
+    if (nchunks <= 1) hipLaunchKernelGGL((scan_lanes_kernel<TT, 0>), grid_lanes, block, 0, st, p, vec);                  \
+    else {                                                                                                                 \
+      hipLaunchKernelGGL((scan_lanes_kernel<TT, 1>), grid_lanes, block, 0, st, p, vec);                                    \
+      hipLaunchKernelGGL((scan_carry_kernel<false>), grid_carry, block, 0, st, p, N, nchunks);                             \
+      hipLaunchKernelGGL((scan_lanes_kernel<TT, 2>), grid_lanes, block, 0, st, p, vec);                                    \
+    } } while (0)
 #define K(TT, NN, AA) do {                                                                                              \
     if (step && few) hipLaunchKernelGGL((scan_step_kernel<TT, NN, AA, 2>), grid_step, block, 0, st, p);                    \
     else if (step) hipLaunchKernelGGL((scan_step_kernel<TT, NN, AA, 8>), grid_step, block, 0, st, p);                      \
@@ -644,7 +818,7 @@ VDA_EXPORT int vda_selective_scan_pairs(void* out, const void* u, const void* de
       hipLaunchKernelGGL((scan_pairs_kernel<TT, NN, 2, AA>), grid, block, 0, st, p);                                       \
     } } while (0)
 #define BYA(TT, NN) do { if (a_scalar) K(TT, NN, true); else K(TT, NN, false); } while (0)
-#define RUN(TT) do { if (N == 16) BYA(TT, 16); else if (N == 32) BYA(TT, 32); else if (N == 64) BYA(TT, 64);              \
+#define RUN(TT) do { if (lanes) K2(TT); else if (N == 16) BYA(TT, 16); else if (N == 32) BYA(TT, 32); else if (N == 64) BYA(TT, 64); \
                      else if (N == 128) BYA(TT, 128); else BYA(TT, 256); } while (0)
   if (dtype == VDA_BF16) RUN(bf16_t);
   else if (dtype == VDA_F16) RUN(f16_t);
@@ -653,6 +827,7 @@ VDA_EXPORT int vda_selective_scan_pairs(void* out, const void* u, const void* de
 #undef RUN
 #undef BYA
 #undef K
+#undef K2
   VDA_CHECK_LAUNCH();
   return 0;
 }
