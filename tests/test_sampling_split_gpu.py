@@ -123,3 +123,41 @@ def test_unfiltered_rows(S, V, split):
     off = torch.ones(S, device=DEV)                                          # a top-p that filters nothing: the other form
     assert torch.equal(got, ops.sample(x, temp, None, off, mp, seeds))
     assert torch.equal(got[2::3], x[2::3].argmax(1))
+
+
+@pytest.mark.parametrize("high", [250, 300, 520])
+def test_lists_of_about_256_entries(high):
+    """Collected entries around the number up to which they are ranked; beyond, the radix descent."""
+    test_both_forms_draw_the_same(24, high, "model")
+
+
+def test_shares_beyond_what_a_sum_holds():
+    """One workgroup a row of 66001 entries, most of them the maximum: their weights are summed in two goes."""
+    g = torch.Generator().manual_seed(3)
+    S, V = 300, 66001
+    x = torch.randn(S, V, generator=g) * 2.0
+    x[:4] = 0.0
+    x[:4, ::8] = -1.0 - torch.rand(4, 8251, generator=g)
+    p = torch.where(torch.arange(S) % 3 == 2, 1.0, 0.3 + 0.69 * torch.rand(S, generator=g))
+    k = torch.where(torch.arange(S) % 4 == 1, 50, 0).to(torch.int32)
+    seeds = torch.randint(0, 2 ** 62, (S,), generator=g)
+    few = [t.to(DEV) for t in (x[:8], k[:8], p[:8], seeds[:8])]              # 17 workgroups a row
+    got = ops.sample(x.to(DEV), None, k.to(DEV), p.to(DEV), None, seeds.to(DEV))
+    assert torch.equal(got[:8], ops.sample(few[0], None, few[1], few[2], None, few[3]))
+    assert all(float(x[s, int(got[s])]) == 0.0 for s in range(2))            # top-p below the maxima's share of 0.95
+
+
+def test_hash_whose_upper_word_changes_along_a_row():
+    """Seeds that put the carry into the upper word of the noise's hash inside the row, and at a share's edges."""
+    V, inverse = 40000, pow(0x9E3779B97F4A7C15, -1, 2 ** 64)
+    seeds = []
+    for at in (0, 1, 2047, 2048, 20001, V - 1):                             # the first token with the next upper word
+        base = (0x12345678 << 32) - at
+        seed = (base - 0x632BE59BD9B4E019) * inverse % 2 ** 64
+        seeds.append(seed - 2 ** 64 if seed >= 2 ** 63 else seed)
+    x = torch.randn(len(seeds), V, generator=torch.Generator().manual_seed(1)) * 0.1
+    for p in (1.0, 0.7):
+        got = ops.sample(x.to(DEV), None, None, torch.full((len(seeds),), p, device=DEV), None, torch.tensor(seeds, device=DEV)).cpu()
+        for s, seed in enumerate(seeds):
+            sure, may = _scores(x[s], 1.0, 0, p, 0.0, seed % 2 ** 64)
+            assert may[int(got[s])] >= sure.max() - 2.0 ** -14               # as above

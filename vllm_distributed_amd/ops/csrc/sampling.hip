@@ -124,8 +124,11 @@ __device__ __forceinline__ float opaque(float v) {
 // 1 / temperature
 __device__ __forceinline__ float inverse(float t) { return opaque(__builtin_amdgcn_rcpf(t)); }
 // exp(z - zmax) as a 32.32 fixed-point number
+// (at most 1: a conversion to 32 bits, which saturates, and one more for the largest entry; to 64 bits it is ten instructions)
 __device__ __forceinline__ unsigned long long fixed_weight(float z, float zmax) {
-  return (unsigned long long)(__expf(opaque(opaque(z) - zmax)) * 4294967296.f);
+  const float w = __expf(opaque(opaque(z) - zmax)) * 4294967296.f;
+  const uint32_t low = (uint32_t)fminf(w, 4294967040.f);
+  return w >= 4294967296.f ? 1ull << 32 : (unsigned long long)low;
 }
 
 // One radix descent by 1024 threads over n entries; at(i) is entry i's scaled logit.  weight(i) = 1 (COUNT) or exp(z_i - zmax) for
@@ -162,11 +165,39 @@ __device__ uint32_t radix_threshold(At at, int n, float zmax, float target, unsi
   return prefix;
 }
 
-// z_i + Gumbel noise: the noise is a function of the row's seed and the token alone
-__device__ __forceinline__ float noisy(float z, uint64_t seed, int i) {
-  const uint32_t rnd = mix32(seed * 0x9E3779B97F4A7C15ULL + (uint64_t)i + 0x632BE59BD9B4E019ULL);
-  const float u = ((float)(rnd >> 8) + 0.5f) * (1.f / 16777216.f);     // (0, 1)
-  return opaque(z) - opaque(__logf(-__logf(u)));
+// z_i + Gumbel noise: the noise is a function of the row's seed and the token alone.  (The logarithms' arguments are at least
+// 2^-25 or zero, so the bare instruction does.)
+__device__ __forceinline__ float gumbel(float z, uint32_t rnd) {
+  const float u = ((float)(rnd >> 8) + 0.5f) * (1.f / 16777216.f);     // (0, 1]
+  const float e = -(__builtin_amdgcn_logf(u) * 0.6931471805599453f);
+  return opaque(z) - opaque(__builtin_amdgcn_logf(e) * 0.6931471805599453f);
+}
+__device__ __forceinline__ uint64_t noise_base(uint64_t seed) { return seed * 0x9E3779B97F4A7C15ULL + 0x632BE59BD9B4E019ULL; }
+__device__ __forceinline__ float noisy(float z, uint64_t seed, int i) { return gumbel(z, mix32(noise_base(seed) + (uint64_t)i)); }
+// The same for tokens a .. b - 1 between which the upper word of the hash's start does not change (SAME): its part of the hash is
+// worked out once, a seventh of the instructions that a token costs.
+struct Noise {
+  uint64_t base;
+  uint32_t lo, hi_shifted, hi_times;
+  bool same;
+};
+__device__ __forceinline__ Noise noise_of(uint64_t seed, int a, int b) {
+  Noise n;
+  n.base = noise_base(seed);
+  const uint64_t first = n.base + (uint64_t)a;
+  n.lo = (uint32_t)n.base;
+  n.hi_shifted = (uint32_t)(first >> 33);
+  n.hi_times = (uint32_t)(first >> 32) * 0xed558ccdu;
+  n.same = a < b && (uint32_t)((n.base + (uint64_t)(b - 1)) >> 32) == (uint32_t)(first >> 32);
+  return n;
+}
+template <bool SAME>
+__device__ __forceinline__ float noisy(float z, const Noise& n, int i) {
+  if (!SAME) return gumbel(z, mix32(n.base + (uint64_t)i));
+  const uint32_t lo = (n.lo + (uint32_t)i) ^ n.hi_shifted;               // (mix32's steps, word by word)
+  uint64_t x = (uint64_t)lo * 0xed558ccdu + ((uint64_t)(lo * 0xff51afd7u + n.hi_times) << 32);
+  x ^= x >> 33; x *= 0xc4ceb9fe1a85ec53ULL; x ^= x >> 33;
+  return gumbel(z, (uint32_t)(x >> 16));
 }
 
 struct SampleArgs {
@@ -235,18 +266,23 @@ __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs p) {
 // ---- rows over several workgroups --------------------------------------------------------------------------------
 // One workgroup per row spends up to ten passes over 0.5 MB (V = 128256) on one CU, most of the time in LDS atomics that
 // all hit the few leading bytes real logits share: 447 us for 61 rows of V = 128256, 73 us for one.  Here a row takes G
-// workgroups and four launches, 59 us and 16 us (of the 59: 11 + 17 + 17 + 14; bins and collect bound by LDS atomics and the
-// noise's 64-bit hash, finish by its barriers; two workgroups a CU: G for 256 or 2048 in all is 72 and 75 us):
+// workgroups and four launches, 51 us and 17 us (of the 51: 8 + 12 + 21 + 10; 256 rows of 151936 136: 26 + 33 + 66 + 12):
 //   stats    the row's maximum and smallest finite value (argmax of a greedy row)
 //   bins     counts (top-k) or fixed-point weights (top-p) in SPLIT_BINS bins that are LINEAR between the maximum and the
-//            smallest value: neighbouring lanes hit different bins, and a bin holds a few hundred entries
+//            smallest value: neighbouring lanes hit different bins, and a bin holds a few hundred entries; rows without a
+//            filter draw among half of their entries
 //   collect  draws among the entries above the bin in which the running sum reaches the target, and collects
 //            that bin's entries (top-k and top-p together: all entries down to it)
 //   finish   the exact threshold key among the collected entries, the draw among them, and the row's winner
+// Bound by the noise's 64-bit hash (45 issue slots an entry) where many entries are drawn from, by trips to memory of a
+// microsecond each elsewhere.  A fifth less than a form (62 us; 203 for 256 rows of 151936) that let the entries beyond the span meet in one bin's
+// atomic (92 us of the 203), hashed the upper word anew for every entry, left the filterless rows' draws to the collecting launch,
+// listed entries with a memory atomic each and always took the radix descent at the end.  One launch for collect and
+// finish, the row's last workgroup finishing it, is no way: the fences it needs took it from 20 to 155 us.
 // A row whose bin overflows the list (thousands of equal logits) is done by its finish workgroup alone, the way of the
 // short rows.  The result is that of the one-workgroup form: the bins are monotone in the key, sums are integers, and each
 // number is rounded alike in every kernel (opaque).
-constexpr int SPLIT_BINS = 2048;      // bin 0: the maximum; the last: -inf; the last but one: beyond the span
+constexpr int SPLIT_BINS = 2048;      // bin 0: the maximum; the last: -inf; the last but one: beyond the span (two per thread)
 constexpr int SPLIT_LIST = 4096;      // collected entries of a row
 constexpr int SPLIT_MAX_G = 64;
 constexpr int SPLIT_MIN_V = 8192;     // shorter rows: the launches cost more than the one-workgroup form's passes
@@ -299,14 +335,34 @@ __device__ __forceinline__ SplitChunk split_chunk(const float* row, int V, int G
   c.vec = (reinterpret_cast<uintptr_t>(row) & 15) == 0;
   return c;
 }
+// Sixteen entries a thread are on their way at once; the first of them (``ahead``) since before anything else is known of
+// the row: every trip to what another kernel has just written costs about a microsecond.
+constexpr int SPLIT_AHEAD = 4;
+struct SplitAhead { f32x4 v[SPLIT_AHEAD]; };
+__device__ __forceinline__ SplitAhead split_ahead(const float* row, SplitChunk c, int from) {
+  SplitAhead h;
+  const int nv = c.a + ((c.b - c.a) & ~3);
+#pragma unroll
+  for (int u = 0; u < SPLIT_AHEAD; ++u) {
+    const int i = from + 4 * (int)threadIdx.x + 4096 * u;
+    h.v[u] = c.vec && i < nv ? *reinterpret_cast<const f32x4*>(row + i) : f32x4{0, 0, 0, 0};
+  }
+  return h;
+}
 template <typename F>
-__device__ __forceinline__ void split_walk(const float* row, SplitChunk c, F f) {
+__device__ __forceinline__ void split_walk(const float* row, SplitChunk c, SplitAhead h, F f) {
   if (c.vec) {
     const int nv = c.a + ((c.b - c.a) & ~3);
-    for (int i = c.a + 4 * threadIdx.x; i < nv; i += 4096) {
-      const f32x4 v = *reinterpret_cast<const f32x4*>(row + i);
+    for (int from = c.a; from < nv;) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) f(v[j], i + j);
+      for (int u = 0; u < SPLIT_AHEAD; ++u) {
+        const int i = from + 4 * (int)threadIdx.x + 4096 * u;
+        if (i >= nv) break;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) f(h.v[u][j], i + j);
+      }
+      from += 4096 * SPLIT_AHEAD;
+      if (from < nv) h = split_ahead(row, c, from);
     }
     for (int i = nv + threadIdx.x; i < c.b; i += 1024) f(row[i], i);
   } else {
@@ -316,19 +372,26 @@ __device__ __forceinline__ void split_walk(const float* row, SplitChunk c, F f) 
 
 // the row's maximum and the width of its bins, from the workgroups' partial results; every thread returns the same
 struct SplitScale { float zmax, per; };
-__device__ __forceinline__ SplitScale split_scale(const SplitRow* ws, int G) {
+// (split_parts asks for them)
+__device__ __forceinline__ f32x2 split_parts(const SplitRow* ws, int G) {
   const int lane = threadIdx.x & 63;
-  float mx = lane < G ? ws->part_max[lane] : -INFINITY, mn = lane < G ? ws->part_min[lane] : INFINITY;
+  return lane < G ? f32x2{ws->part_max[lane], ws->part_min[lane]} : f32x2{-INFINITY, INFINITY};
+}
+__device__ __forceinline__ SplitScale split_scale(f32x2 parts) {
+  float mx = parts[0], mn = parts[1];
   mx = wave_max(mx);
   mn = -wave_max(-mn);
   // weights below 2^-32 of the largest are zero: 22.2; a k-th largest entry further down lands in the last bins
   const float span = fminf(fmaxf(mx - mn, 1e-3f), 24.f);
   return {mx, opaque((float)(SPLIT_BINS - 2) * opaque(__builtin_amdgcn_rcpf(span)))};
 }
-// a function of the scaled logit that never decreases as it falls
+// functions of the scaled logit that never decrease as it falls
+__device__ __forceinline__ float split_place(float z, SplitScale sc) {
+  return fmaxf(opaque(opaque(sc.zmax - opaque(z)) * sc.per), 0.f);
+}
 __device__ __forceinline__ int split_bin(float z, SplitScale sc) {
   if (z == -INFINITY) return SPLIT_BINS - 1;
-  return (int)fminf(fmaxf(opaque(opaque(sc.zmax - opaque(z)) * sc.per), 0.f), (float)(SPLIT_BINS - 2));
+  return (int)fminf(split_place(z, sc), (float)(SPLIT_BINS - 2));
 }
 
 __global__ __launch_bounds__(1024) void split_stats_kernel(SampleArgs p, SplitRow* ws_rows, int row0) {
@@ -340,17 +403,18 @@ __global__ __launch_bounds__(1024) void split_stats_kernel(SampleArgs p, SplitRo
   const float* row = p.logits + (long)rowi * p.stride;
   for (int b = blockIdx.x * 1024 + threadIdx.x; b < SPLIT_BINS; b += G * 1024) ws->hist[b] = 0ull;
   if (blockIdx.x == 0 && threadIdx.x == 0) ws->count = 0u;
-  const SplitFilter f = split_filter(p, rowi);
   const SplitChunk c = split_chunk(row, p.V, G);
+  const SplitAhead ahead = split_ahead(row, c, c.a);
+  const SplitFilter f = split_filter(p, rowi);
   if (f.greedy) {
     ArgMax a{-INFINITY, 0x7fffffff};
-    split_walk(row, c, [&](float v, int i) { a = amax2(a, ArgMax{v, i}); });
+    split_walk(row, c, ahead, [&](float v, int i) { a = amax2(a, ArgMax{v, i}); });
     a = block_argmax(a, rv, ri);
     if (threadIdx.x == 0) { ws->part_v[blockIdx.x] = a.v; ws->part_i[blockIdx.x] = a.i; }
     return;
   }
   float mx = -INFINITY, mn = INFINITY;
-  split_walk(row, c, [&](float v, int) {
+  split_walk(row, c, ahead, [&](float v, int) {
     const float z = v * f.inv_t;
     mx = fmaxf(mx, z);
     if (z > -INFINITY) mn = fminf(mn, z);
@@ -360,39 +424,107 @@ __global__ __launch_bounds__(1024) void split_stats_kernel(SampleArgs p, SplitRo
   if (threadIdx.x == 0) { ws->part_max[blockIdx.x] = mx; ws->part_min[blockIdx.x] = mn; }
 }
 
+// a thread walks its share in order: the first of equals stays
+__device__ __forceinline__ void later(ArgMax& a, float v, int i) {
+  if (v > a.v) { a.v = v; a.i = i; }
+}
+// the best of a share's entries that are drawn from without a filter
+template <bool SAME>
+__device__ __forceinline__ ArgMax split_draw_as(float inv_t, uint32_t floor_key, const float* row, SplitChunk c, const SplitAhead& ahead,
+                                                const Noise& n) {
+  ArgMax a{-INFINITY, 0x7fffffff};
+  if (floor_key) {
+    split_walk(row, c, ahead, [&](float v, int i) {
+      const float z = v * inv_t;
+      if (fkey(z) >= floor_key) later(a, noisy<SAME>(z, n, i), i);
+    });
+  } else {
+    split_walk(row, c, ahead, [&](float v, int i) { later(a, noisy<SAME>(v * inv_t, n, i), i); });
+  }
+  return a;
+}
+__device__ __forceinline__ ArgMax split_draw(const SampleArgs& p, const SplitFilter& f, const SplitScale& sc, int rowi, const float* row,
+                                             SplitChunk c, const SplitAhead& ahead) {
+  const uint32_t floor_key = f.mp > 0.f ? fkey(sc.zmax + __logf(f.mp)) : 0u;
+  const Noise n = noise_of((uint64_t)(p.seeds ? p.seeds[rowi] : 0), c.a, c.b);
+  return n.same ? split_draw_as<true>(f.inv_t, floor_key, row, c, ahead, n) : split_draw_as<false>(f.inv_t, floor_key, row, c, ahead, n);
+}
+// A row without top-k and top-p has no bins to fill, but noise for every entry, which costs more than all that a filtered row
+// asks for: it draws among the first half of each share here and among the second in the next launch.
+__device__ __forceinline__ int split_half(SplitChunk c) { return c.a + (((c.b - c.a) / 2) & ~3); }
+
+// Sums in two 32-bit words, each of which 65535 entries cannot overflow: 16 bits of a weight each (the upper one up to 65536,
+// and mostly zero).  A 64-bit LDS atomic of a wave costs three times a 32-bit one.
+constexpr int SPLIT_SUMMED = 65532;
 __global__ __launch_bounds__(1024) void split_bins_kernel(SampleArgs p, SplitRow* ws_rows, int row0) {
-  __shared__ unsigned long long hist[SPLIT_BINS];
+  __shared__ uint32_t low[SPLIT_BINS], high[SPLIT_BINS];
+  __shared__ float rv[16];
+  __shared__ int ri[16];
   const int rowi = row0 + blockIdx.y;
   SplitRow* ws = ws_rows + blockIdx.y;
-  const SplitFilter f = split_filter(p, rowi);
-  if (f.greedy || f.mode == MODE_NONE) return;
   const float* row = p.logits + (long)rowi * p.stride;
-  for (int b = threadIdx.x; b < SPLIT_BINS; b += 1024) hist[b] = 0ull;
-  __syncthreads();
-  const SplitScale sc = split_scale(ws, gridDim.x);
-  const SplitChunk c = split_chunk(row, p.V, gridDim.x);
-  if (f.k) {
-    split_walk(row, c, [&](float v, int) { atomicAdd(&hist[split_bin(v * f.inv_t, sc)], 1ull); });
-  } else {
-    split_walk(row, c, [&](float v, int) {
-      const float z = v * f.inv_t;
-      const unsigned long long w = fixed_weight(z, sc.zmax);
-      if (w) atomicAdd(&hist[split_bin(z, sc)], w);
-    });
+  SplitChunk c = split_chunk(row, p.V, gridDim.x);
+  SplitAhead ahead = split_ahead(row, c, c.a);
+  const f32x2 parts = split_parts(ws, gridDim.x);
+  const SplitFilter f = split_filter(p, rowi);
+  if (f.greedy) return;
+  const SplitScale sc = split_scale(parts);
+  if (f.mode == MODE_NONE) {
+    c.b = split_half(c);
+    ArgMax a = split_draw(p, f, sc, rowi, row, c, ahead);
+    a = block_argmax(a, rv, ri);
+    if (threadIdx.x == 0) { ws->part_v[blockIdx.x] = a.v; ws->part_i[blockIdx.x] = a.i; }
+    return;
   }
-  __syncthreads();
-  for (int b = threadIdx.x; b < SPLIT_BINS; b += 1024)
-    if (hist[b]) atomicAdd(&ws->hist[b], hist[b]);
+  const int end = c.b;
+  for (;;) {
+#pragma unroll
+    for (int b = threadIdx.x; b < SPLIT_BINS; b += 1024) { low[b] = 0u; high[b] = 0u; }
+    __syncthreads();
+    c.b = min(c.a + SPLIT_SUMMED, end);
+    if (f.k) {
+      // most of a row far below its maximum, or masked, is one bin: lanes that meet there wait for each other
+      uint32_t beyond = 0u, masked = 0u;
+      split_walk(row, c, ahead, [&](float v, int) {
+        const int b = split_bin(v * f.inv_t, sc);
+        beyond += b == SPLIT_BINS - 2;
+        masked += b == SPLIT_BINS - 1;
+        if (b < SPLIT_BINS - 2) atomicAdd(&low[b], 1u);
+      });
+      if (beyond) atomicAdd(&low[SPLIT_BINS - 2], beyond);
+      if (masked) atomicAdd(&low[SPLIT_BINS - 1], masked);
+    } else {
+      split_walk(row, c, ahead, [&](float v, int) {
+        const float z = v * f.inv_t;
+        const unsigned long long w = fixed_weight(z, sc.zmax);
+        const int b = split_bin(z, sc);
+        const uint32_t lo = (uint32_t)w & 0xffffu, hi = (uint32_t)(w >> 16);
+        if (lo) atomicAdd(&low[b], lo);
+        if (hi) atomicAdd(&high[b], hi);
+      });
+    }
+    __syncthreads();
+#pragma unroll
+    for (int b = threadIdx.x; b < SPLIT_BINS; b += 1024) {
+      const unsigned long long sum = ((unsigned long long)high[b] << 16) + low[b];
+      if (sum) atomicAdd(&ws->hist[b], sum);
+    }
+    c.a = c.b;
+    if (c.a >= end) return;
+    ahead = split_ahead(row, SplitChunk{c.a, min(c.a + SPLIT_SUMMED, end), c.vec}, c.a);
+    __syncthreads();
+  }
 }
 
 // Where the running sum over the bins reaches the target: the bin, what is left of the target there, and (counts)
 // how many entries it and all before it hold.  bin -1: no weight at all, nothing is filtered.
 struct SplitCut { int bin; unsigned long long rem, upto; };
-__device__ __forceinline__ SplitCut split_cut(const SplitRow* ws, const SplitFilter& f, unsigned long long* s_wave /*[16]*/,
+// w: the sums of the two bins that are this thread's.
+typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ SplitCut split_cut(u64x2 w, const SplitFilter& f, unsigned long long* s_wave /*[16]*/,
                                               SplitCut* s_cut) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const unsigned long long w0 = ws->hist[2 * threadIdx.x], w1 = ws->hist[2 * threadIdx.x + 1];
-  unsigned long long cum = w0 + w1;
+  unsigned long long cum = w[0] + w[1];
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
     const unsigned long long up = __shfl_up(cum, o, 64);
@@ -403,9 +535,9 @@ __device__ __forceinline__ SplitCut split_cut(const SplitRow* ws, const SplitFil
   __syncthreads();
   unsigned long long total = 0ull;
 #pragma unroll
-  for (int w = 0; w < 16; ++w) {
-    if (w < wid) cum += s_wave[w];
-    total += s_wave[w];
+  for (int i = 0; i < 16; ++i) {
+    if (i < wid) cum += s_wave[i];
+    total += s_wave[i];
   }
   unsigned long long remaining;
   if (f.k) remaining = (unsigned long long)f.k;
@@ -413,16 +545,16 @@ __device__ __forceinline__ SplitCut split_cut(const SplitRow* ws, const SplitFil
     remaining = (unsigned long long)((double)f.tp * (double)total);
     if (remaining < 1ull) remaining = 1ull;
   }
-  const unsigned long long before = cum - w0 - w1;
-  if (w0 > 0ull && before < remaining && before + w0 >= remaining)
-    *s_cut = SplitCut{2 * (int)threadIdx.x, remaining - before, before + w0};
-  else if (w1 > 0ull && before + w0 < remaining && cum >= remaining)
-    *s_cut = SplitCut{2 * (int)threadIdx.x + 1, remaining - before - w0, cum};
+  const unsigned long long before = cum - w[0] - w[1];
+  if (w[0] > 0ull && before < remaining && before + w[0] >= remaining)
+    *s_cut = SplitCut{2 * (int)threadIdx.x, remaining - before, before + w[0]};
+  else if (w[1] > 0ull && before + w[0] < remaining && cum >= remaining)
+    *s_cut = SplitCut{2 * (int)threadIdx.x + 1, remaining - before - w[0], cum};
   __syncthreads();
   return *s_cut;
 }
 
-// Rows that their finish workgroup does by itself: counts that say before collecting that the list is too short
+// Rows that one workgroup finishes by itself: counts that say before collecting that the list is too short
 // (top-k and top-p together list everything down to the cut, without the -inf entries), and rows of nothing but -inf.
 __device__ __forceinline__ bool split_alone(const SplitFilter& f, const SplitCut& cut, const SplitScale& sc) {
   if (sc.zmax == -INFINITY) return true;
@@ -431,51 +563,112 @@ __device__ __forceinline__ bool split_alone(const SplitFilter& f, const SplitCut
   return n > (unsigned long long)SPLIT_LIST;
 }
 
-__global__ __launch_bounds__(1024) void split_collect_kernel(SampleArgs p, SplitRow* ws_rows, int row0) {
+// The same threshold as radix_threshold over a list of 256 at most, in one go: four threads an entry sum what lies above it.
+// The key is the lowest of those above which less than the target lies (0 where there is no weight at all).
+template <bool COUNT>
+__device__ uint32_t ranked_threshold(const uint2* list, const unsigned long long* weight, int n, unsigned long long target,
+                                     float fraction, uint32_t floor_key, uint32_t* s_key) {
+  const int i = threadIdx.x >> 2;
+  if (threadIdx.x == 0) *s_key = 0xffffffffu;
+  const uint32_t key = i < n ? list[i].x : 0u;
+  unsigned long long above = 0ull, total = 0ull;
+  if (i < n) {
+#pragma unroll 4
+    for (int j = threadIdx.x & 3; j < n; j += 4) {
+      const uint32_t k = list[j].x;
+      const unsigned long long w = COUNT ? 1ull : weight[j];
+      above += k > key ? w : 0ull;
+      if (!COUNT) total += k >= floor_key ? w : 0ull;
+    }
+  }
+#pragma unroll
+  for (int o = 1; o < 4; o <<= 1) {
+    above += __shfl_xor(above, o, 64);
+    if (!COUNT) total += __shfl_xor(total, o, 64);
+  }
+  if (!COUNT && fraction >= 0.f) {
+    target = (unsigned long long)((double)fraction * (double)total);
+    if (target < 1ull) target = 1ull;
+  }
+  const bool in = i < n && key >= floor_key && above < target && (COUNT || weight[i] > 0ull);
+  uint32_t lowest = in ? key : 0xffffffffu;
+#pragma unroll
+  for (int o = 4; o < 64; o <<= 1) lowest = min(lowest, (uint32_t)__shfl_xor((int)lowest, o, 64));
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0 && lowest != 0xffffffffu) atomicMin(s_key, lowest);
+  __syncthreads();
+  const uint32_t found = *s_key;
+  __syncthreads();
+  return found == 0xffffffffu ? 0u : found;
+}
+
+__global__ __launch_bounds__(1024) void split_collect_kernel(SampleArgs p, SplitRow* ws_rows, int row0, int half_drawn) {
   __shared__ float rv[16];
   __shared__ int ri[16];
   __shared__ unsigned long long s_wave[16];
   __shared__ SplitCut s_cut;
+  __shared__ uint32_t s_count, s_base;
+  __shared__ uint2 list[SPLIT_LIST];
   const int rowi = row0 + blockIdx.y;
   SplitRow* ws = ws_rows + blockIdx.y;
+  const float* row = p.logits + (long)rowi * p.stride;
+  SplitChunk c = split_chunk(row, p.V, gridDim.x);
+  const int half = split_half(c);
+  const SplitAhead ahead = split_ahead(row, c, c.a);
+  const f32x2 parts = split_parts(ws, gridDim.x);
+  const u64x2 bin_sum = reinterpret_cast<const u64x2*>(ws->hist)[threadIdx.x];
   const SplitFilter f = split_filter(p, rowi);
   if (f.greedy) return;
-  const float* row = p.logits + (long)rowi * p.stride;
-  const SplitScale sc = split_scale(ws, gridDim.x);
-  SplitCut cut{-1, 0ull, 0ull};
-  if (f.mode != MODE_NONE) cut = split_cut(ws, f, s_wave, &s_cut);
-  const bool all = f.mode == MODE_ALL;
-  // a count that reaches the -inf entries keeps every other one: none of them needs to be listed
-  const bool keeps_all = cut.bin < 0 || cut.bin == SPLIT_BINS - 1;
-  const int draw_to = all ? 0 : keeps_all ? SPLIT_BINS : cut.bin;         // bins below are drawn from here
-  const int list_from = all ? 0 : keeps_all ? SPLIT_BINS : cut.bin;       // bins list_from .. list_to are collected
-  const int list_to = cut.bin == SPLIT_BINS - 1 ? SPLIT_BINS - 2 : cut.bin;
-  const uint32_t floor_key = f.mp > 0.f ? fkey(sc.zmax + __logf(f.mp)) : 0u;
-  const uint64_t seed = (uint64_t)(p.seeds ? p.seeds[rowi] : 0);
+  const SplitScale sc = split_scale(parts);
   ArgMax a{-INFINITY, 0x7fffffff};
-  if (!split_alone(f, cut, sc))
-    split_walk(row, split_chunk(row, p.V, gridDim.x), [&](float v, int i) {
-      const float z = v * f.inv_t;
-      if (f.mode != MODE_NONE) {
-        const int b = split_bin(z, sc);
-        if (b >= list_from && b <= list_to) {
-          // one atomic for the lanes that came here together
-          const unsigned long long here = __ballot(1);
-          const int lane = threadIdx.x & 63, first = __ffsll(here) - 1;
-          uint32_t at = 0u;
-          if (lane == first) at = atomicAdd(&ws->count, (uint32_t)__popcll(here));
-          at = __shfl(at, first, 64) + (uint32_t)__popcll(here & ((1ull << lane) - 1ull));
-          if (at < (uint32_t)SPLIT_LIST) ws->list[at] = make_uint2(fkey(z), (uint32_t)i);
-          return;
+  if (f.mode == MODE_NONE) {
+    if (half_drawn) c.a = half;
+    a = split_draw(p, f, sc, rowi, row, c, half_drawn ? split_ahead(row, c, c.a) : ahead);
+    if (half_drawn && threadIdx.x == 0) a = amax2(a, ArgMax{ws->part_v[blockIdx.x], ws->part_i[blockIdx.x]});
+  } else {
+    if (threadIdx.x == 0) s_count = 0u;
+    const SplitCut cut = split_cut(bin_sum, f, s_wave, &s_cut);
+    const bool all = f.mode == MODE_ALL;
+    // a count that reaches the -inf entries keeps every other one: none of them needs to be listed
+    const bool keeps_all = cut.bin < 0 || cut.bin == SPLIT_BINS - 1;
+    // Bins below draw_to are drawn from here, bins list_from .. list_to are collected: in places between bins, as split_bin has
+    // them ahead of its rounding down (-inf entries and those beyond the span share the place at infinity)
+    const float draw_to = all ? 0.f : keeps_all ? INFINITY : (float)cut.bin;
+    const float list_from = all ? 0.f : keeps_all ? NAN : (float)cut.bin;
+    const bool beyond = cut.bin >= SPLIT_BINS - 2;
+    const float list_end = beyond ? INFINITY : (float)(cut.bin + 1);
+    const uint32_t floor_key = f.mp > 0.f ? fkey(sc.zmax + __logf(f.mp)) : 0u;
+    const Noise noise = noise_of((uint64_t)(p.seeds ? p.seeds[rowi] : 0), c.a, c.b);
+    auto walk = [&](auto same) {
+      split_walk(row, c, ahead, [&](float v, int i) {
+        const float z = v * f.inv_t, at = split_place(z, sc);
+        if (at < draw_to) {
+          if (!floor_key || fkey(z) >= floor_key) later(a, noisy<decltype(same)::value>(z, noise, i), i);
+        } else if (at >= list_from && (at < list_end || (beyond && z != -INFINITY))) {
+          const uint32_t to = atomicAdd(&s_count, 1u);
+          if (to < (uint32_t)SPLIT_LIST) list[to] = make_uint2(fkey(z), (uint32_t)i);
         }
-        if (b >= draw_to) return;
+      });
+    };
+    if (!split_alone(f, cut, sc)) {
+      if (noise.same) walk(std::true_type());
+      else walk(std::false_type());
+      // this share's entries behind those of others: one atomic on the row's count
+      __syncthreads();
+      const uint32_t n = s_count;
+      if (n > 0u) {
+        if (threadIdx.x == 0) s_base = atomicAdd(&ws->count, n);
+        __syncthreads();
+        const uint32_t base = s_base;
+        for (uint32_t i = threadIdx.x; i < n && base + i < (uint32_t)SPLIT_LIST; i += 1024) ws->list[base + i] = list[i];
       }
-      if (fkey(z) >= floor_key) a = amax2(a, ArgMax{noisy(z, seed, i), i});
-    });
+    }
+  }
   a = block_argmax(a, rv, ri);
   if (threadIdx.x == 0) { ws->part_v[blockIdx.x] = a.v; ws->part_i[blockIdx.x] = a.i; }
 }
 
+constexpr int SPLIT_RANKED = 256;     // entries; more take the radix descent (its LDS histogram holds the weights of these)
 __global__ __launch_bounds__(1024) void split_finish_kernel(SampleArgs p, SplitRow* ws_rows, int row0, int G) {
   __shared__ float red[16];
   __shared__ float rv[16];
@@ -487,21 +680,26 @@ __global__ __launch_bounds__(1024) void split_finish_kernel(SampleArgs p, SplitR
   __shared__ uint2 list[SPLIT_LIST];
   const int rowi = row0 + blockIdx.x;
   SplitRow* ws = ws_rows + blockIdx.x;
-  const SplitFilter f = split_filter(p, rowi);
+  // everything that may be wanted in one trip (list entries past the count: nobody's)
+  const f32x2 parts = split_parts(ws, G);
+  const u64x2 bin_sum = reinterpret_cast<const u64x2*>(ws->hist)[threadIdx.x];
+  const uint2 entry = ws->list[threadIdx.x];
+  const uint32_t n = ws->count;
   ArgMax a{-INFINITY, 0x7fffffff};
   if ((int)threadIdx.x < G) a = ArgMax{ws->part_v[threadIdx.x], ws->part_i[threadIdx.x]};
+  const SplitFilter f = split_filter(p, rowi);
   if (!f.greedy) {
-    const SplitScale sc = split_scale(ws, G);
+    const SplitScale sc = split_scale(parts);
     SplitCut cut{-1, 0ull, 0ull};
-    if (f.mode != MODE_NONE) cut = split_cut(ws, f, s_wave, &s_cut);
+    if (f.mode != MODE_NONE) cut = split_cut(bin_sum, f, s_wave, &s_cut);
     const bool all = f.mode == MODE_ALL;
-    const uint32_t n = ws->count;
     if (n > (uint32_t)SPLIT_LIST || split_alone(f, cut, sc)) {
       sample_row(p, rowi, sc.zmax, true, red, rv, ri, hist, &s_sel, &s_rem);
       return;
     }
     if (n > 0u) {
-      for (uint32_t i = threadIdx.x; i < n; i += 1024) list[i] = ws->list[i];
+      list[threadIdx.x] = entry;
+      for (uint32_t i = threadIdx.x + 1024; i < n; i += 1024) list[i] = ws->list[i];
       __syncthreads();
       auto at = [&](int i) {
         const uint32_t key = list[i].x;
@@ -509,10 +707,17 @@ __global__ __launch_bounds__(1024) void split_finish_kernel(SampleArgs p, SplitR
       };
       uint32_t thr = 0;
       // the list starts with what lies above the cut bin (all) or with that bin
-      if (f.k && cut.bin != SPLIT_BINS - 1)
-        thr = radix_threshold<true>(at, (int)n, sc.zmax, all ? (float)f.k : (float)cut.rem, 0ull, 0u, hist, &s_sel, &s_rem);
-      if (f.tp < 1.f)
-        thr = max(thr, radix_threshold<false>(at, (int)n, sc.zmax, f.tp, all ? 0ull : cut.rem, thr, hist, &s_sel, &s_rem));
+      const bool counts = f.k && cut.bin != SPLIT_BINS - 1, weighs = f.tp < 1.f;
+      if (n <= (uint32_t)SPLIT_RANKED) {
+        if (weighs && threadIdx.x < n) hist[threadIdx.x] = fixed_weight(at(threadIdx.x), sc.zmax);
+        __syncthreads();
+        if (counts) thr = ranked_threshold<true>(list, hist, (int)n, all ? (unsigned long long)f.k : cut.rem, -1.f, 0u, &s_sel);
+        if (weighs) thr = max(thr, ranked_threshold<false>(list, hist, (int)n, cut.rem, all ? f.tp : -1.f, thr, &s_sel));
+      } else {
+        if (counts) thr = radix_threshold<true>(at, (int)n, sc.zmax, all ? (float)f.k : (float)cut.rem, 0ull, 0u, hist, &s_sel, &s_rem);
+        if (weighs)
+          thr = max(thr, radix_threshold<false>(at, (int)n, sc.zmax, f.tp, all ? 0ull : cut.rem, thr, hist, &s_sel, &s_rem));
+      }
       if (f.mp > 0.f) thr = max(thr, fkey(sc.zmax + __logf(f.mp)));
       const uint64_t seed = (uint64_t)(p.seeds ? p.seeds[rowi] : 0);
       for (uint32_t i = threadIdx.x; i < n; i += 1024)
@@ -604,11 +809,12 @@ VDA_EXPORT int vda_sample(const float* logits, long* out, const float* temperatu
   SplitRow* ws = (SplitRow*)workspace;
   for (int row0 = 0; row0 < S; row0 += SPLIT_ROWS) {
     const int rows = min(S - row0, SPLIT_ROWS);
-    // two workgroups of 1024 threads per CU, at least a float4 for every thread
-    const int G = max(1, min(min((512 + rows - 1) / rows, (V + 4095) / 4096), SPLIT_MAX_G));
+    // two workgroups of 1024 threads per CU and no more (61 rows in nine parts are 549, and the last 37 cost as much as all the
+    // others), at least a float4 for every thread
+    const int G = max(1, min(min(512 / rows, (V + 4095) / 4096), SPLIT_MAX_G));
     hipLaunchKernelGGL(split_stats_kernel, dim3(G, rows), dim3(1024), 0, st, p, ws, row0);
     if (filtered) hipLaunchKernelGGL(split_bins_kernel, dim3(G, rows), dim3(1024), 0, st, p, ws, row0);
-    hipLaunchKernelGGL(split_collect_kernel, dim3(G, rows), dim3(1024), 0, st, p, ws, row0);
+    hipLaunchKernelGGL(split_collect_kernel, dim3(G, rows), dim3(1024), 0, st, p, ws, row0, (int)filtered);
     hipLaunchKernelGGL(split_finish_kernel, dim3(rows), dim3(1024), 0, st, p, ws, row0, G);
   }
   VDA_CHECK_LAUNCH();
