@@ -168,15 +168,22 @@ _HASHED = (
 )
 
 
+_RAW_NAME = {name: os.environ.encodekey(name) for name in _REGISTRY}
+
+
 def __getattr__(name: str) -> Any:
     try:
         parser, default = _REGISTRY[name]
     except KeyError:
         raise AttributeError(f"unknown environment knob {name!r}") from None
-    raw = os.environ.get(name)
-    if raw is None:
-        return default
-    return parser(raw)
+    # the mapping behind os.environ: every launch reads a switch or two, and a miss costs os.environ.get an exception (0.6 us,
+    # 0.1 this way)
+    try:
+        raw = os.environ._data.get(_RAW_NAME[name])
+    except AttributeError:                               # something else in os.environ's place
+        raw = os.environ.get(name)
+        return default if raw is None else parser(raw)
+    return default if raw is None else parser(os.environ.decodevalue(raw))
 
 
 def __dir__() -> list[str]:

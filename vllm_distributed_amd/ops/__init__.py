@@ -264,13 +264,14 @@ def paged_attention_decode(out, q, k_cache, v_cache, block_table, seq_lens, q_st
     part_out = part_lse = None
     if num_splits > 1:
         if workspace is not None:
-            part_out, part_lse = workspace
-        else:
-            part_out = torch.empty((T, Hq, num_splits, D), dtype=torch.float32, device=q.device)
-            part_lse = torch.empty((T, Hq, num_splits), dtype=torch.float32, device=q.device)
+            part_out, part_lse = workspace[0].data_ptr(), workspace[1].data_ptr()
+        else:                                            # the parts' rows, then their weights: an allocation is 1.5 us
+            part = torch.empty(T * Hq * num_splits * (D + 1), dtype=torch.float32, device=q.device)
+            part_out = part.data_ptr()
+            part_lse = part_out + 4 * T * Hq * num_splits * D
     N.call("vda_paged_attention_decode", out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-           block_table.data_ptr(), seq_lens.data_ptr(), q_start_loc.data_ptr(), N.ptr(alibi), N.ptr(part_out),
-           N.ptr(part_lse), S, T, Hq, k_cache.shape[1], D, k_cache.shape[2], block_table.stride(0), num_splits,
+           block_table.data_ptr(), seq_lens.data_ptr(), q_start_loc.data_ptr(), N.ptr(alibi), part_out,
+           part_lse, S, T, Hq, k_cache.shape[1], D, k_cache.shape[2], block_table.stride(0), num_splits,
            max_q_len, q.stride(0), out.stride(0), scale, softcap, window, N.dt(q.dtype), _kv_fp8(k_cache), k_scale,
            v_scale, N.ptr(sink), int(chunk), int(v_shift), *_dist_bias_args(dist_bias, Hq), N.stream())
     return out
@@ -1387,23 +1388,25 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, topk_w: torc
     dev = x.device
     ids = topk_ids.contiguous()
     tw = topk_w.contiguous()
-    sorted_ids = torch.empty(T * k, dtype=torch.int32, device=dev)
-    offsets = torch.empty(E + 1, dtype=torch.int32, device=dev)
-    st = N.stream()
-    N.call("vda_moe_align", sorted_ids.data_ptr(), offsets.data_ptr(), ids.data_ptr(), T * k, E, st)
-    inter = torch.empty((T * k, I), dtype=x.dtype, device=dev)
-    out2 = torch.empty((T * k, H), dtype=x.dtype, device=dev)
+    # what passes between the launches, in one allocation (1.5 us each): both products' rows, the sorted pairs, the experts' offsets
+    st, eb, n = N.stream(), x.element_size(), T * k
+    scratch = torch.empty(n * (I + H) * eb + 4 * (n + E + 1), dtype=torch.uint8, device=dev)
+    inter = scratch.data_ptr()
+    out2 = inter + n * I * eb
+    sorted_ids = out2 + n * H * eb
+    offsets = sorted_ids + 4 * n
+    N.call("vda_moe_align", sorted_ids, offsets, ids.data_ptr(), n, E, st)
     out = torch.empty((T, H), dtype=x.dtype, device=dev)
     wd = N.dt(w13.dtype)
     # one expert can receive at most one slot of every token
     max_pairs = T
-    N.call("vda_moe_gate_up", inter.data_ptr(), x.data_ptr(), w13.data_ptr(), N.ptr(w13_scale), sorted_ids.data_ptr(),
-           offsets.data_ptr(), E, I, H, k, max_pairs, x.stride(0), N.dt(x.dtype), wd,
-           int(moe_rows_form(T * k, E, I, w13.element_size())), N.ACT[activation], float(act_limit), st)
-    N.call("vda_moe_down", out2.data_ptr(), inter.data_ptr(), w2.data_ptr(), N.ptr(w2_scale), tw.data_ptr(),
-           sorted_ids.data_ptr(), offsets.data_ptr(), E, H, I, max_pairs, N.dt(x.dtype), wd,
-           int(moe_rows_form(T * k, E, H, w2.element_size())), st)
-    N.call("vda_moe_sum", out.data_ptr(), out2.data_ptr(), ids.data_ptr(), T, H, k, out.stride(0), N.dt(x.dtype), st)
+    N.call("vda_moe_gate_up", inter, x.data_ptr(), w13.data_ptr(), N.ptr(w13_scale), sorted_ids,
+           offsets, E, I, H, k, max_pairs, x.stride(0), N.dt(x.dtype), wd,
+           int(moe_rows_form(n, E, I, w13.element_size())), N.ACT[activation], float(act_limit), st)
+    N.call("vda_moe_down", out2, inter, w2.data_ptr(), N.ptr(w2_scale), tw.data_ptr(),
+           sorted_ids, offsets, E, H, I, max_pairs, N.dt(x.dtype), wd,
+           int(moe_rows_form(n, E, H, w2.element_size())), st)
+    N.call("vda_moe_sum", out.data_ptr(), out2, ids.data_ptr(), T, H, k, out.stride(0), N.dt(x.dtype), st)
     return out
 
 

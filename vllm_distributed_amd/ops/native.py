@@ -165,7 +165,9 @@ def register(name: str, sig: list) -> None:
 
 
 def stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream of the current device.  Its handle alone: ``torch.cuda.current_stream()`` builds an object around it, which
+    takes 2.7 us of a launch's 9, this 0.2."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def dt(t: torch.dtype) -> int:
