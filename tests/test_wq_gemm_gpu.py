@@ -328,3 +328,36 @@ def test_codebook4_k_splits(N, K, G):
         torch.cuda.synchronize()
         ref = x.float() @ deq.t()
         assert (out.float() - ref).abs().max().item() < 2e-2 * ref.abs().max().item() + 2e-2
+
+
+# K over a workgroup's waves: waves without a step (K = 128), slices of unequal length, groups that a slice cuts, rows that do not
+# fill a fragment, the last row counts of the rule and the first beyond
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M", [1, 5, 10, 11, 13, 16, 17])
+@pytest.mark.parametrize("N,K,G", [(32, 128, 128), (36, 640, 64), (100, 1152, 128), (44, 768, 256), (64, 1024, 1024), (260, 9216, 128)])
+def test_wq_slices(dtype, bits, M, N, K, G):
+    from vllm_distributed_amd import ops
+    torch.manual_seed(M * 11 + N + bits)
+    x = (torch.rand(M, K + 8, device="cuda") * 2 - 1).to(dtype)[:, :K]
+    qw, scales, zeros, sz, deq = _quantised(N, K, G, bits, dtype)
+    bias = torch.randn(N, device="cuda").to(dtype)
+    ref = x.float() @ deq.to(dtype).float().t() + bias.float()
+    got = ops.wq_gemm(x, qw, sz, G, bits, bias).float()
+    # sums of K products below about 1 each over sqrt(K); one rounding of the result, and of each widened weight where it is scaled
+    # in 16 bits (which the reference rounds too, and the unscaled form does not)
+    u = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    assert (got - ref).abs().max().item() <= 2 * u * ref.abs().max().item() + 4 * u
+
+
+def test_wq_slices_of_many_rows():
+    """8-bit weights of so many rows that the other kernel would fill the chip."""
+    from vllm_distributed_amd import ops
+    torch.manual_seed(5)
+    N, K, G = 49160, 256, 128
+    x = (torch.rand(4, K, device="cuda") * 2 - 1).to(torch.bfloat16)
+    qw, scales, zeros, sz, deq = _quantised(N, K, G, 8, torch.bfloat16)
+    ref = x.float() @ deq.to(torch.bfloat16).float().t()
+    for rows in (4, 3):
+        got = ops.wq_gemm(x[:rows], qw, sz, G, 8).float()
+        assert (got - ref[:rows]).abs().max().item() <= 2 ** -7 * ref.abs().max().item() + 2 ** -6

@@ -228,7 +228,7 @@ __global__ __launch_bounds__(256 * WM, WM == 1 ? 2 : 1) void wq_stream_kernel(co
   const DenseGemmArgs& a = wa.d;
   constexpr int WAVES = 4 * WM;
   constexpr int SX = 4;                                // activation ring depth (filled three steps ahead)
-  constexpr int DW = BITS == 4 && !(POST && MT16 >= 4) ? 8 : 4;   // weight steps in registers
+  constexpr int DW = 4;                                // weight steps in registers (eight: 57344 x 8192 in 4 bits 66 us, four 62)
   static_assert(!POST || BITS == 4, "unscaled operands exist for 4-bit weights only");
   constexpr int NQ = BITS / 4;                         // 16-byte loads per fragment and step
   constexpr int LW = 2 * NQ + 2;                       // vector-memory operations of one weight step
@@ -249,6 +249,18 @@ __global__ __launch_bounds__(256 * WM, WM == 1 ? 2 : 1) void wq_stream_kernel(co
   const int nk_all = a.K >> 7;
   const int kt0 = blockIdx.y * a.units_per_split;
   const int nk = min(a.units_per_split, nk_all - kt0);           // >= 1 by the host's choice of splits
+  // Where this workgroup starts: at a group's first step, another one for each workgroup.  Rows are a power of two apart in most
+  // models: with all workgroups at the same column of their rows, what they read falls on few memory channels (13 activation
+  // rows, 57344 x 8192: 4 bits 71.6 -> 66.1 us, 8 bits 112 -> 104).
+  int turn = 0;
+  {
+    const int per = wa.gshift <= 2 ? 1 : 1 << (wa.gshift - 2);   // steps of a group
+    if (a.splits == 1 && wa.gshift < 30 && nk % per == 0) turn = (int)(blockIdx.x * 5u % (unsigned)(nk / per)) * per;
+  }
+  auto at_step = [&](int kt) {                                   // past the end: any step
+    const int t = min(kt, nk - 1) + turn;
+    return t < nk ? t : t - nk;
+  };
 
   const uint8_t* wp[2];
   const uint8_t* sp[2];
@@ -267,7 +279,7 @@ __global__ __launch_bounds__(256 * WM, WM == 1 ? 2 : 1) void wq_stream_kernel(co
     xp[j] = reinterpret_cast<const uint8_t*>(a.x) + row * a.x_stride * 2 + (long)kt0 * 256 + (((tid & 15) ^ (tau & 15)) << 4);
   }
   auto fill = [&](int kt) {          // ring slot kt % 4 <- K step min(kt, nk - 1)
-    const long ko = (long)min(kt, nk - 1) * 256;
+    const long ko = (long)at_step(kt) * 256;
     uint8_t* dst = lds + (kt & 3) * XB + wave * 1024;
 #pragma unroll
     for (int j = 0; j < P; ++j) glds16(xp[j] + ko, dst + j * WAVES * 1024);
@@ -276,7 +288,7 @@ __global__ __launch_bounds__(256 * WM, WM == 1 ? 2 : 1) void wq_stream_kernel(co
   typename std::conditional<POST, i32x4, uint32_t>::type sreg[DW][2];
   const long plane = (long)a.N * 4;
   auto wload = [&](int u, int kt) {
-    const int kk = min(kt, nk - 1);
+    const int kk = at_step(kt);
     const long so = (long)((((kt0 + kk) << 2) + g) >> wa.gshift) * plane;
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
@@ -345,7 +357,7 @@ __global__ __launch_bounds__(256 * WM, WM == 1 ? 2 : 1) void wq_stream_kernel(co
               xsum[nt] = mfma16(ones, xf, xsum[nt]);
             }
           }
-          const int here = (kt0 + kt) << 2;
+          const int here = (kt0 + at_step(kt)) << 2;
           if ((here >> wa.gshift) != ((here + 4) >> wa.gshift) || kt + 1 == nk) {   // the group ends with this step
 #pragma unroll
             for (int mt = 0; mt < 2; ++mt) {
@@ -431,6 +443,180 @@ __global__ __launch_bounds__(256 * WM, WM == 1 ? 2 : 1) void wq_stream_kernel(co
   }
 }
 
+// ---- decode, fewer weight rows than fill the chip: K over the waves of a workgroup --------------------------
+// Up to 16 activation rows.  The kernel above splits K over workgroups there, and the sum of the parts is a launch of its own
+// (5 us and a gap of 2, of 20 in all).  Here a workgroup owns 32 weight rows and its KS waves a slice of K each: nothing is shared until
+// the waves' sums meet in LDS, so there is no barrier in the loop, and the activations, a few rows that the L2 holds, go
+// straight to registers.  Operands, steps of 128 elements and the unscaled form (POST) are the ones above.  Behind a step's
+// arithmetic its registers take the activations two steps ahead and the weights four ahead (plain loads, which the
+// compiler counts: were they inline assembly, a build that has to spill would spill what has not arrived).
+// Bound by the memory system's latency and by activations from the L2, of which a wave of 32 weight rows reads M / 8 (4 bits) bytes
+// a byte of weights.  us, K over workgroups -> this: 8192 x 8192 in 4 bits, 2 rows 21.0 -> 12.9, 16 rows 21.9 -> 17.3, in 8 bits, 9
+// rows 25.4 -> 17.8; 28672 x 4096, 9 rows 32.3 -> 27.4, in 8 bits 43.6 -> 35.3; 6144 x 4096 16 -> 10.6.  Twice the steps in
+// flight 34.8 and 19.7 for the second and the fourth of these, eight waves 20.8 for the second.
+constexpr int WQ_KS = 4;
+// Longer rows of many activations lose: 8192 x 28672 in 4 bits, 1 / 10 / 13 / 16 rows 40.4 -> 34.4 / 41.4 -> 41.5 / 41.9 -> 45.0 / 42.1
+// -> 48.8; 4096 x 14336, 9 / 13 / 16 rows 22.6 -> 20.7 / 23.2 -> 23.5 / 22.6 -> 25.6; in 8 bits 9 / 16 rows 27.1 -> 25.2 / 27.2 -> 30.0.
+// Where workgroups of 128 weight rows fill the chip, the kernel above has no parts to sum (57344 x 8192 in 4 bits, 1 / 13
+// rows 61.8 / 61.9 there, 65.6 / 90.2 here), but for 8 bits and very few rows: 98.7 there, 88.6 here.
+static bool wq_slices_pay(int M, int N, int K, int bits) {
+  const bool fills = (N + 127) / 128 * 4 >= 512 * 3;
+  return M <= 16 && (fills ? bits == 8 && M <= 4 : K <= 8192 || M <= (bits == 4 ? 10 : 12));
+}
+template <typename T, int BITS, bool POST>
+__global__ __launch_bounds__(64 * WQ_KS, 2) void wq_slices_kernel(const WqGemmArgs wa) {
+  using V8 = typename Vec<T>::v8;
+  using V4 = typename Vec<T>::v4;
+  const DenseGemmArgs& a = wa.d;
+  constexpr int KS = WQ_KS, DW = 4, XD = 2;
+  constexpr int NQ = BITS / 4, STEPB = 16 * BITS;
+  __shared__ f32x4 sums[KS][2][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int r = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * 32;
+  const int nk_all = a.K >> 7;
+  const int kt0 = (int)((long)nk_all * wave / KS), nk = (int)((long)nk_all * (wave + 1) / KS) - kt0;
+
+  const uint8_t* wp[2];
+  const uint8_t* sp[2];
+#pragma unroll
+  for (int mt = 0; mt < 2; ++mt) {
+    const int row = min(n0 + 16 * mt + r, a.N - 1);
+    wp[mt] = reinterpret_cast<const uint8_t*>(a.w) + (long)row * ((long)a.K * BITS / 8) + (long)kt0 * STEPB + g * (STEPB / 4);
+    sp[mt] = reinterpret_cast<const uint8_t*>(wa.sz) + (POST ? (long)min(n0 + 16 * mt + 4 * g, a.N - 4) * 4 : (long)row * 4);
+  }
+  const uint8_t* xp = reinterpret_cast<const uint8_t*>(a.x) + (long)min(r, a.M - 1) * a.x_stride * 2 + (long)kt0 * 256 + g * 64;
+  i32x4 wreg[DW][2][NQ], xreg[XD][4];
+  using Pairs = typename std::conditional<POST, i32x4, uint32_t>::type;
+  Pairs sreg[DW][2];
+  const long plane = (long)a.N * 4;
+  auto xload = [&](int u, int kt) {
+    const i32x4* p = reinterpret_cast<const i32x4*>(xp + (long)min(kt, nk - 1) * 256);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) xreg[u][j] = p[j];
+  };
+  auto wload = [&](int u, int kt) {
+    const int kk = min(kt, nk - 1);
+    const long so = (long)((((kt0 + kk) << 2) + g) >> wa.gshift) * plane;
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) wreg[u][mt][q] = reinterpret_cast<const i32x4*>(wp[mt] + (long)kk * STEPB)[q];
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) sreg[u][mt] = *reinterpret_cast<const Pairs*>(sp[mt] + so);
+  };
+
+  f32x4 acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}}, part[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}}, xsum = {0, 0, 0, 0};
+  V8 ones;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ones[i] = (T)1.f;
+  if (nk > 0) {
+    // in the loop's own order
+#pragma unroll
+    for (int u = 0; u < DW - XD; ++u) wload(u, u);
+#pragma unroll
+    for (int u = 0; u < XD; ++u) { xload(u, u); wload(DW - XD + u, DW - XD + u); }
+    for (int kb = 0; kb < nk; kb += DW) {
+#pragma unroll
+      for (int u = 0; u < DW; ++u) {
+        const int kt = kb + u;
+        if (kt < nk) {
+          float sc[2], nz[2];
+          if constexpr (!POST) {
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt) {
+              const V4 pv = __builtin_bit_cast(V4, u32x2{sreg[u][mt], 0u});
+              sc[mt] = (float)pv[0];
+              nz[mt] = -(float)pv[1] * sc[mt];
+            }
+          }
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const V8 xf = __builtin_bit_cast(V8, xreg[u % XD][j]);
+            V8 wf[2];
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt) {
+              if constexpr (POST) {
+                const uint32_t w = (uint32_t)wreg[u][mt][0][j];
+                const u32x4 d = {(w & 0x000F000Fu) | WqMagic<T>::OR, ((w >> 4) & 0x000F000Fu) | WqMagic<T>::OR,
+                                 ((w >> 8) & 0x000F000Fu) | WqMagic<T>::OR, ((w >> 12) & 0x000F000Fu) | WqMagic<T>::OR};
+                wf[mt] = __builtin_bit_cast(V8, d);
+              } else {
+                uint32_t q[2];
+                if (BITS == 4) { q[0] = (uint32_t)wreg[u][mt][0][j]; q[1] = 0u; }
+                else { q[0] = (uint32_t)wreg[u][mt][(2 * j) >> 2][(2 * j) & 3]; q[1] = (uint32_t)wreg[u][mt][(2 * j + 1) >> 2][(2 * j + 1) & 3]; }
+                wf[mt] = wq_expand<T, BITS>(q, sc[mt], nz[mt]);
+              }
+            }
+            if constexpr (POST) {
+              part[0] = mfma16(wf[0], xf, part[0]);
+              part[1] = mfma16(wf[1], xf, part[1]);
+              xsum = mfma16(ones, xf, xsum);
+            } else {
+              acc[0] = mfma16(wf[0], xf, acc[0]);
+              acc[1] = mfma16(wf[1], xf, acc[1]);
+            }
+          }
+          if constexpr (POST) {
+            const int here = (kt0 + kt) << 2;
+            if ((here >> wa.gshift) != ((here + 4) >> wa.gshift) || kt + 1 == nk) {   // the group, or what this wave has of it, ends
+#pragma unroll
+              for (int mt = 0; mt < 2; ++mt) {
+                const V8 pv = __builtin_bit_cast(V8, sreg[u][mt]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                  const float s = (float)pv[2 * i], zb = (float)pv[2 * i + 1] + WqMagic<T>::BIAS;
+                  acc[mt][i] = fmaf(s, fmaf(-zb, xsum[i], part[mt][i]), acc[mt][i]);
+                  part[mt][i] = 0.f;
+                }
+              }
+              xsum = f32x4{0, 0, 0, 0};
+            }
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        xload(u % XD, kt + XD);
+        wload(u, kt + DW);
+      }
+    }
+  }
+  sums[wave][0][lane] = acc[0];
+  sums[wave][1][lane] = acc[1];
+  __syncthreads();
+  if (threadIdx.x >= 128) return;
+  // out[token r][n0 + 16 mt + 4 g + i]
+  const int mt = threadIdx.x >> 6, n = n0 + 16 * mt + 4 * g;
+  if (r >= a.M || n >= a.N) return;
+  f32x4 v = sums[0][mt][lane];
+#pragma unroll
+  for (int w = 1; w < KS; ++w) v += sums[w][mt][lane];
+  T* op = reinterpret_cast<T*>(a.out) + (long)r * a.out_stride;
+  V4 o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (a.bias && n + i < a.N) v[i] += (float)reinterpret_cast<const T*>(a.bias)[n + i];
+    o[i] = (T)v[i];
+  }
+  if (n + 3 < a.N && a.out_stride % 4 == 0) *reinterpret_cast<V4*>(op + n) = o;
+  else
+    for (int i = 0; i < 4; ++i) if (n + i < a.N) op[n + i] = o[i];
+}
+
+template <typename T, int BITS>
+static int launch_wq_slices(const WqGemmArgs& wa, hipStream_t st) {
+  const DenseGemmArgs& a = wa.d;
+  const dim3 grid((unsigned)((a.N + 31) / 32));
+  if constexpr (BITS == 4) {
+    if (!wa.per_element && wa.group % 128 == 0 && a.N % 4 == 0) {
+      hipLaunchKernelGGL((wq_slices_kernel<T, 4, true>), grid, dim3(64 * WQ_KS), 0, st, wa);
+      return 0;
+    }
+  }
+  hipLaunchKernelGGL((wq_slices_kernel<T, BITS, false>), grid, dim3(64 * WQ_KS), 0, st, wa);
+  return 0;
+}
+
 template <typename T, int BITS>
 static int launch_wq_stream(const WqGemmArgs& wa, hipStream_t st) {
   const DenseGemmArgs& a = wa.d;
@@ -504,6 +690,12 @@ VDA_EXPORT int vda_wq_gemm(void* out, const void* x, const void* qw, const void*
     const int nk = K >> 7;
     const int groups = (N + 127) / 128;
     const int slots = M <= 64 ? 512 : 256;
+    if (variant == 0 && splits < 1 && wq_slices_pay(M, N, K, bits)) {
+      rc = dtype == VDA_BF16 ? (bits == 4 ? launch_wq_slices<bf16_t, 4>(wa, st) : launch_wq_slices<bf16_t, 8>(wa, st))
+                             : (bits == 4 ? launch_wq_slices<f16_t, 4>(wa, st) : launch_wq_slices<f16_t, 8>(wa, st));
+      VDA_CHECK_LAUNCH();
+      return rc;
+    }
     if (splits < 1) {
       splits = 1;
       if (groups * 4 < slots * 3) splits = (slots + groups - 1) / groups;
