@@ -1105,12 +1105,15 @@ class ModelRunner:
 
         # ---- logits + sampling ------------------------------------------------
         spec_sched = so.scheduled_spec_decode_tokens
+        taps = None
         if spec_sched and self.rejection_sampler is not None:
             out = self._sample_with_spec(so, hidden, req_ids, rows, n_sched, cu, S)
         else:
             self._to_dev(self.logits_indices, logits_idx)
             sample_hidden = hidden[self.logits_indices[:S]]
             logits = self._compute_logits(sample_hidden, logits_idx[:S])
+            if so.logit_taps:                # on their way to the host before anything changes them
+                taps = self._start_taps(so, hidden, req_ids, n_sched, cu, logits, logits_idx[:S])
             if envs.VLLM_COMPUTE_NANS_IN_LOGITS:
                 self._last_nans = {r: int(x) for r, x in zip(req_ids, logits.isnan().sum(-1).tolist())}
             if so.grammar_bitmask is not None:
@@ -1160,7 +1163,7 @@ class ModelRunner:
             failed_recving=failed_recving,
             num_nans_in_logits=getattr(self, "_last_nans", None))
         if so.logit_taps:
-            result.tapped_logits = self._tap_logits(so, hidden, req_ids, n_sched, cu)
+            result.tapped_logits = self._collect_taps(taps or self._start_taps(so, hidden, req_ids, n_sched, cu))
         if tmd is not None and not tk_plain:
             get_tknp_group().broadcast_object(result, src=0)
         return result
@@ -1354,8 +1357,9 @@ class ModelRunner:
             out[rid] = LogprobsLists(ids.tolist(), lps.tolist(), ranks.tolist())
         return out
 
-    def _tap_logits(self, so, hidden, req_ids, n_sched, cu) -> dict:
-        """Full-vocabulary fp32 logits at the positions ``so.logit_taps`` names, per request, on the host."""
+    def _start_taps(self, so, hidden, req_ids, n_sched, cu, logits=None, logits_idx=None):
+        """Queue the full-vocabulary fp32 logits at the positions ``so.logit_taps`` names for the host.  ``logits``: those of the
+        rows ``logits_idx``, which are not worked out a second time where they are the ones that are asked for."""
         idx, spans = [], {}
         for i, rid in enumerate(req_ids):
             taps = so.logit_taps.get(rid)
@@ -1366,10 +1370,25 @@ class ModelRunner:
             spans[rid] = (len(idx), len(idx) + len(taps))
             idx.extend(int(cu[i]) + int(t) for t in taps)
         if not idx:
-            return {}
-        sel = torch.tensor(idx, dtype=torch.int64, device=self.device)
-        logits = self._compute_logits(hidden[sel], np.asarray(idx)).float().cpu().numpy()
-        return {rid: logits[a:b] for rid, (a, b) in spans.items()}
+            return None, spans, None
+        if logits is None or idx != logits_idx.tolist():
+            sel = torch.tensor(idx, dtype=torch.int64, device=self.device)
+            logits = self._compute_logits(hidden[sel], np.asarray(idx))
+        rows = torch.empty(logits.shape, dtype=torch.float32, pin_memory=self.pin)
+        rows.copy_(logits.float() if self.is_gpu else logits, non_blocking=True)
+        done = None
+        if self.is_gpu:
+            done = torch.cuda.Event()
+            done.record()
+        return rows, spans, done
+
+    @staticmethod
+    def _collect_taps(started) -> dict:
+        """Per request, on the host."""
+        rows, spans, done = started
+        if done is not None:
+            done.synchronize()
+        return {rid: rows[a:b].numpy() for rid, (a, b) in spans.items()}
 
     def _compute_logits(self, hidden_rows: torch.Tensor, index: np.ndarray) -> torch.Tensor:
         """Logits of rows ``index`` of this step's tokens (the index tells LoRA which adapter each row uses)."""
