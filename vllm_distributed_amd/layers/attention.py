@@ -133,7 +133,8 @@ class Attention(nn.Module):
             ops.paged_attention_prefill(out[ndt:e], q[ndt:e], src.k_cache, src.v_cache, md.block_table[nd:nd + n_pre],
                                         md.seq_lens[nd:nd + n_pre], md.prefill_query_start_loc, self.scale,
                                         window=self.sliding_window, softcap=self.softcap, alibi=self.alibi_slopes,
-                                        k_scale=ksc, v_scale=vsc, causal=self.causal, max_q_len=md.max_query_len)
+                                        k_scale=ksc, v_scale=vsc, causal=self.causal, max_q_len=md.max_query_len,
+                                        max_kv_len=md.max_seq_len)
         if n < T:
             out[n:].zero_()
         return out.view(T, Hq * D)
@@ -214,7 +215,7 @@ class Attention(nn.Module):
                                             sl[nd:nd + n_pre], pqsl, self.scale,
                                             window=self.sliding_window, softcap=self.softcap, alibi=self.alibi_slopes,
                                             k_scale=ksc, v_scale=vsc, causal=self.causal,
-                                            max_q_len=md.max_query_len)
+                                            max_q_len=md.max_query_len, max_kv_len=md.max_seq_len)
         if conn is not None:
             conn.save_kv_layer(self.layer_name, (self.k_cache, self.v_cache), md)
         return out.view(T, qs)

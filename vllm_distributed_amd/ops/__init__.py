@@ -301,12 +301,15 @@ def paged_attention_prefill(out, q, k_cache, v_cache, block_table, seq_lens, q_s
                             window: int = 0, softcap: float = 0.0, alibi: Optional[torch.Tensor] = None,
                             k_scale: float = 1.0, v_scale: float = 1.0, causal: bool = True,
                             return_lse: bool = False, max_q_len: int = 0, sink: Optional[torch.Tensor] = None,
-                            chunk: int = 0, v_shift: int = 0, dist_bias: Optional[torch.Tensor] = None):
+                            chunk: int = 0, v_shift: int = 0, dist_bias: Optional[torch.Tensor] = None,
+                            max_kv_len: int = 0):
     """Varlen attention of new tokens against the paged cache.  ``causal=False``: every query token sees
     all ``seq_lens[s]`` keys of its sequence (encoder models, the shared-prefix pass of cascade
     attention).  ``return_lse``: also return the log-sum-exp [Hq, T] (natural log) of every row.
     ``max_q_len``: the longest query run of the batch when the caller knows it on the host (0 = unknown);
-    the wide kernel then starts the longest causal tiles of all sequences first."""
+    the wide kernel then starts the longest causal tiles of all sequences first.  ``max_kv_len``: the most keys of a
+    sequence when the caller knows it on the host (0: what the block table can hold); few query rows over long
+    sequences are cut along their keys by it."""
     T, Hq, D = q.shape
     if not _dev(q):
         # options of the device kernels (see the decode form)
@@ -317,11 +320,23 @@ def paged_attention_prefill(out, q, k_cache, v_cache, block_table, seq_lens, q_s
         out.copy_(o)
         return (out, lse) if return_lse else out
     lse = torch.full((Hq, T), float("-inf"), dtype=torch.float32, device=q.device) if return_lse else None
+    Hkv, page = k_cache.shape[1], k_cache.shape[2]
+    part_out, part_lse, parts = None, None, 1
+    if not return_lse:
+        keys = block_table.shape[1] * page                 # that a tile of 128 rows at most can see
+        for bound in (max_kv_len, window + 128 if window > 0 else 0, chunk + 128 if chunk > 0 else 0):
+            keys = min(keys, bound) if bound > 0 else keys
+        parts = N.lib().vda_prefill_parts(seq_lens.shape[0], T, Hq, Hkv, D, int(max_q_len), keys)
+        if parts > 1:
+            part = torch.empty(T * Hq * parts * (D + 1), dtype=torch.float32, device=q.device)
+            part_out = part.data_ptr()
+            part_lse = part_out + 4 * T * Hq * parts * D
     N.call("vda_paged_attention_prefill", out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
            block_table.data_ptr(), seq_lens.data_ptr(), q_start_loc.data_ptr(), N.ptr(alibi), seq_lens.shape[0], T,
-           Hq, k_cache.shape[1], D, k_cache.shape[2], block_table.stride(0), q.stride(0), out.stride(0), scale,
+           Hq, Hkv, D, page, block_table.stride(0), q.stride(0), out.stride(0), scale,
            softcap, window, N.dt(q.dtype), _kv_fp8(k_cache), k_scale, v_scale, int(bool(causal)), N.ptr(lse),
-           int(max_q_len), N.ptr(sink), int(chunk), int(v_shift), *_dist_bias_args(dist_bias, Hq), N.stream())
+           int(max_q_len), N.ptr(sink), int(chunk), int(v_shift), *_dist_bias_args(dist_bias, Hq), part_out, part_lse, parts,
+           N.stream())
     return (out, lse) if return_lse else out
 
 

@@ -22,6 +22,50 @@
 // Nothing goes through LDS except the final cross-wave merge of the decode form.
 #include "attention.h"
 
+// Which sequence and query tokens a prompt's workgroup owns: tiles of sequence s lie in [qsl[s] / q_tile + s, qsl[s + 1] / q_tile
+// + s + 1).  The lanes look at 64 sequences at once and hand out what they have read: one trip to memory where a binary
+// search makes one for each of its steps and two more.
+struct QueryTile { int seq, q0, qs, q_len, seq_len; };
+__device__ __forceinline__ QueryTile query_tile(const AttnParams& p, int tile) {
+  const int lane = threadIdx.x & 63;
+  QueryTile t{0, 0, 0, 0, 0};
+  for (int base = 0; base < p.num_seqs; base += 64) {
+    const int i = min(base + lane, p.num_seqs - 1);
+    const int start = p.q_start_loc[i], end = p.q_start_loc[i + 1], len = p.seq_lens[i];
+    const int n = __popcll(__ballot(base + lane < p.num_seqs && start / p.q_tile + i <= tile));
+    if (n > 0) {
+      t.seq = base + n - 1;
+      t.qs = __builtin_amdgcn_readlane(start, n - 1);
+      t.q_len = __builtin_amdgcn_readlane(end, n - 1) - t.qs;
+      t.seq_len = __builtin_amdgcn_readlane(len, n - 1);
+    }
+    if (n < 64) break;
+  }
+  t.q0 = (tile - (t.qs / p.q_tile + t.seq)) * p.q_tile;
+  return t;
+}
+
+// Prompts whose query tiles do not fill the chip: part blockIdx.z of gridDim.z of a tile's 32-key steps (prefill_parts says
+// how many), whose results attn_reduce_kernel merges.
+__device__ __forceinline__ void key_part(const AttnParams& p, int& step_lo, int& step_hi) {
+  if (p.nsplit <= 1) return;
+  const int per = (max(step_hi - step_lo, 0) + p.nsplit - 1) / p.nsplit;
+  step_lo += blockIdx.z * per;
+  step_hi = min(step_hi, step_lo + per);
+}
+// a lane's values 16 n + 4 g of one (token, head), as that part's row and its log2-domain weight
+template <int D>
+__device__ __forceinline__ void store_part(const AttnParams& p, long tok, int head, int g, const f32x4 (&acc)[D / 16], float inv,
+                                           float m, float l) {
+  const long at = (tok * p.Hq + head) * p.nsplit + blockIdx.z;
+  if (l > 0.f) {                                          // (a part without keys is left out by its weight)
+    float* po = p.part_out + at * D + 4 * g;
+#pragma unroll
+    for (int n = 0; n < D / 16; ++n) *reinterpret_cast<f32x4*>(po + 16 * n) = acc[n] * inv;
+  }
+  if (g == 0) p.part_lse[at] = l > 0.f ? m + log2f(l) : -INFINITY;
+}
+
 template <typename T, int D, int BS, int NCT, bool F8>
 __global__ __launch_bounds__(256) void paged_attn_kernel(AttnParams p) {
   using V8 = typename Vec<T>::v8;
@@ -36,18 +80,8 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(AttnParams p) {
   const int kvh = blockIdx.y;
   const int G = p.Hq / p.Hkv;
 
-  // ---- which sequence / query tokens does this workgroup own ----------------
-  // tiles of sequence s live in [qsl[s]/QT + s, qsl[s+1]/QT + s + 1): find s
-  const int tile = blockIdx.x;
-  int seq = 0, last = p.num_seqs;
-  while (seq < last) {
-    int mid = (seq + last + 1) >> 1;
-    if (mid < p.num_seqs && p.q_start_loc[mid] / p.q_tile + mid <= tile) seq = mid; else last = mid - 1;
-  }
-  const int q0 = (tile - (p.q_start_loc[seq] / p.q_tile + seq)) * p.q_tile;
-  const int qs = p.q_start_loc[seq];
-  const int q_len = p.q_start_loc[seq + 1] - qs;
-  const int seq_len = p.seq_lens[seq];
+  const QueryTile own = query_tile(p, blockIdx.x);
+  const int seq = own.seq, q0 = own.q0, qs = own.qs, q_len = own.q_len, seq_len = own.seq_len;
   if (q0 >= q_len) return;
   const int ctx = seq_len - q_len;        // keys that precede the first query token
   const int* bt = p.block_table + (long)seq * p.max_blocks;
@@ -91,12 +125,14 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(AttnParams p) {
     wave_hi = max(wave_hi, __shfl_xor(wave_hi, o, 64));
     wave_lo = min(wave_lo, __shfl_xor(wave_lo, o, 64));
   }
-  const int step_lo = wave_hi > 0 ? wave_lo / 32 : 0, step_hi = (wave_hi + 31) / 32;
+  int step_lo = wave_hi > 0 ? wave_lo / 32 : 0, step_hi = (wave_hi + 31) / 32;
+  key_part(p, step_lo, step_hi);
 
   float m[NCT], l[NCT];
   f32x4 acc[NCT][NT];
 #pragma unroll
   for (int ct = 0; ct < NCT; ++ct) {
+    if (blockIdx.z > 0) sink_m[ct] = -INFINITY;           // (a sink joins once)
     m[ct] = sink_m[ct]; l[ct] = (sink_m[ct] != -INFINITY && g == 0) ? 1.f : 0.f;
 #pragma unroll
     for (int n = 0; n < NT; ++n) acc[ct][n] = f32x4{0, 0, 0, 0};
@@ -207,6 +243,10 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(AttnParams p) {
     const int c = wave * COLS + ct * 16 + r;
     const int head = kvh * G + c % G;
     const float inv = l[ct] > 0.f ? p.v_scale / l[ct] : 0.f;
+    if (p.nsplit > 1) {
+      store_part<D>(p, col_off[ct], head, g, acc[ct], inv, m[ct], l[ct]);
+      continue;
+    }
     T* op = (T*)p.out + col_off[ct] * p.out_stride + (long)head * D + 4 * g;
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
@@ -557,9 +597,6 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(AttnParams p) {
 // every wave then reads its MFMA operands from LDS.  16-byte pieces are XOR-swizzled so that the eight
 // lanes served per LDS cycle hit eight different bank groups for both the row-per-lane K reads and the
 // d-row-per-lane V reads.
-#ifndef PREFILL_REG_STAGES
-#define PREFILL_REG_STAGES 1
-#endif
 #ifndef PREFILL_WGS_PER_CU
 #define PREFILL_WGS_PER_CU 2
 #endif
@@ -592,17 +629,8 @@ __global__ __launch_bounds__(256, PREFILL_WGS_PER_CU) void paged_prefill_lds_ker
   const int kvh = SPARSE ? blockIdx.y / (p.Hq / p.Hkv) : blockIdx.y;
   const int head0 = SPARSE ? blockIdx.y : kvh * G;        // first query head of this workgroup's columns
 
-  const int tile = blockIdx.x;
-  int lo = 0, hi = p.num_seqs;
-  while (lo < hi) {
-    int mid = (lo + hi + 1) >> 1;
-    if (mid < p.num_seqs && p.q_start_loc[mid] / p.q_tile + mid <= tile) lo = mid; else hi = mid - 1;
-  }
-  const int seq = lo;
-  const int q0 = (tile - (p.q_start_loc[seq] / p.q_tile + seq)) * p.q_tile;
-  const int qs = p.q_start_loc[seq];
-  const int q_len = p.q_start_loc[seq + 1] - qs;
-  const int seq_len = p.seq_lens[seq];
+  const QueryTile own = query_tile(p, blockIdx.x);
+  const int seq = own.seq, q0 = own.q0, qs = own.qs, q_len = own.q_len, seq_len = own.seq_len;
   if (q0 >= q_len) return;                  // uniform over the workgroup
   const int ctx = seq_len - q_len;
   const int* bt = p.block_table + (long)seq * p.max_blocks;
@@ -644,7 +672,12 @@ __global__ __launch_bounds__(256, PREFILL_WGS_PER_CU) void paged_prefill_lds_ker
   const int wg_hi = p.causal ? ctx + qt_end : seq_len;
   int wg_lo = p.window > 0 ? max(0, ctx + q0 + 1 - p.window) : 0;
   if (p.chunk > 0 && p.causal) wg_lo = max(wg_lo, (ctx + q0) / p.chunk * p.chunk);
-  const int step_lo = wg_lo / 32, step_hi = (wg_hi + 31) / 32;
+  int step_lo = wg_lo / 32, step_hi = (wg_hi + 31) / 32;
+  if constexpr (!SPARSE) {
+    key_part(p, step_lo, step_hi);
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct) sink_m[ct] = blockIdx.z > 0 ? -INFINITY : sink_m[ct];   // (a sink joins once)
+  }
 
   __shared__ unsigned bm[SPARSE ? SPARSE_BM_WORDS : 1];
   if constexpr (SPARSE) {
@@ -686,36 +719,37 @@ __global__ __launch_bounds__(256, PREFILL_WGS_PER_CU) void paged_prefill_lds_ker
   const CT* kc = (const CT*)p.k_cache;
   const CT* vc = (const CT*)p.v_cache;
 
-  // Two register stages: tile t+2 is requested from memory while tile t is consumed and tile t+1 (requested one
-  // iteration earlier) moves from registers into the other LDS buffer -- a full iteration of latency cover.
-  V8 rkA[KPT], rvA[VPT];
-#if PREFILL_REG_STAGES == 2
-  V8 rkB[KPT], rvB[VPT];
-#endif
+  V8 rk[KPT], rv[VPT];
+  unsigned pk[KPT], pv[VPT];                    // page numbers, asked for a tile before what lies in the pages
   // Address arithmetic kept in 32 bits except for the one block-number x block-stride product (a single
   // v_mad_u64_u32): offsets inside a block fit 32 bits by construction.
   const unsigned blk_stride = (unsigned)p.Hkv * BS * D;          // elements per K cache block
   const unsigned v_blk_stride = (unsigned)(p.Hkv >> p.v_shift) * D * BS;     // per V cache block (fewer heads when shared)
   const unsigned k_head = (unsigned)kvh * BS * D, v_head = (unsigned)(kvh >> p.v_shift) * D * BS;
-  auto gload = [&](int step, V8 (&rk)[KPT], V8 (&rv)[VPT]) {
+  auto pages = [&](int step) {
+    const int tb = step * 32;
+#pragma unroll
+    for (int i = 0; i < KPT; ++i) pk[i] = (unsigned)bt[max(min((tb + (tid + 256 * i) / KCH) / BS, nblk_valid - 1), 0)];
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) pv[i] = (unsigned)bt[max(min((tb + 8 * ((tid + 256 * i) & 3)) / BS, nblk_valid - 1), 0)];
+  };
+  auto gload = [&](int step) {
     const int tb = step * 32;
 #pragma unroll
     for (int i = 0; i < KPT; ++i) {
       const int pi = tid + 256 * i;
       const int key = pi / KCH, ch = pi % KCH;
       const int tok = tb + key;
-      const unsigned blk = (unsigned)bt[max(min(tok / BS, nblk_valid - 1), 0)];
       const unsigned off = k_head + (unsigned)(tok % BS) * D + ch * 8;
-      rk[i] = KVLoad<T, F8>::ld(kc + (size_t)blk * blk_stride + off);
+      rk[i] = KVLoad<T, F8>::ld(kc + (size_t)pk[i] * blk_stride + off);
     }
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
       const int pi = tid + 256 * i;
       const int d = pi >> 2, c = pi & 3;
       const int tok = tb + 8 * c;
-      const unsigned blk = (unsigned)bt[max(min(tok / BS, nblk_valid - 1), 0)];
       const unsigned off = v_head + (unsigned)d * BS + (tok % BS);
-      rv[i] = KVLoad<T, F8>::ld(vc + (size_t)blk * v_blk_stride + off);
+      rv[i] = KVLoad<T, F8>::ld(vc + (size_t)pv[i] * v_blk_stride + off);
     }
   };
   // XOR swizzle of the 16-byte pieces of a K row.  ds_read_b128 serves lanes {0-3,12-15,20-27},
@@ -723,7 +757,7 @@ __global__ __launch_bounds__(256, PREFILL_WGS_PER_CU) void paged_prefill_lds_ker
   // below) these masks put the sixteen lanes of every such group on sixteen different pieces, where the
   // earlier three-bit mask left them two-way (one extra LDS cycle per group on every K operand read).
   auto kswz = [](int key) { return KCH == 16 ? (key & 15) : (((key & 3) << 1) | ((key >> 3) & 1)); };
-  auto sstore = [&](int buf, const V8 (&rk)[KPT], const V8 (&rv)[VPT]) {
+  auto sstore = [&](int buf) {
 #pragma unroll
     for (int i = 0; i < KPT; ++i) {
       const int pi = tid + 256 * i;
@@ -837,48 +871,28 @@ __global__ __launch_bounds__(256, PREFILL_WGS_PER_CU) void paged_prefill_lds_ker
     }
   };
 
-#if PREFILL_REG_STAGES == 2
-  static_assert(!SPARSE, "the sparse form walks its step list with one register stage");
-  // prologue: tile 0 -> LDS buffer 0, tile 1 -> register stage A
-  if (step_lo < step_hi) {
-    gload(step_lo, rkA, rvA);
-    sstore(0, rkA, rvA);
-    if (step_lo + 1 < step_hi) gload(step_lo + 1, rkA, rvA);
-  }
-  __syncthreads();
-  for (int step = step_lo; step < step_hi; step += 2) {
-    // even half: consume buffer 0, stage A holds tile step+1, request tile step+2 into stage B
-    if (step + 2 < step_hi) gload(step + 2, rkB, rvB);
-    compute(step, 0);
-    if (step + 1 < step_hi) sstore(1, rkA, rvA);
-    __syncthreads();
-    if (step + 1 >= step_hi) break;
-    // odd half: consume buffer 1, stage B holds tile step+2, request tile step+3 into stage A
-    if (step + 3 < step_hi) gload(step + 3, rkA, rvA);
-    compute(step + 1, 1);
-    if (step + 2 < step_hi) sstore(0, rkB, rvB);
-    __syncthreads();
-  }
-#else
-  // One register stage (16 fewer registers: two workgroups fit a CU, so one wave's global-load and
-  // softmax latency is covered by the other wave of its SIMD rather than by a deeper software pipeline).
-  // Tile t+1 sits in registers while tile t is consumed, then moves to the other LDS buffer and tile t+2
-  // is requested.
+  // One register stage (two workgroups fit a CU, so one wave's global-load and softmax latency is covered by the other wave of
+  // its SIMD rather than by a deeper software pipeline).  Tile t+1 sits in registers while tile t is consumed, then moves to
+  // the other LDS buffer and tile t+2 is requested from the pages that were looked up an iteration before (looked up only then,
+  // two prompts of 500, 32 / 32 heads, take 74 us, so 67).
   int s0 = next_step(step_lo), s1 = next_step(s0 + 1), s2 = next_step(s1 + 1);
   if (s0 < step_hi) {
-    gload(s0, rkA, rvA);
-    sstore(0, rkA, rvA);
-    if (s1 < step_hi) gload(s1, rkA, rvA);
+    pages(s0);
+    gload(s0);
+    pages(s1);
+    sstore(0);
+    if (s1 < step_hi) gload(s1);
+    pages(s2);
   }
   __syncthreads();
   for (int buf = 0; s0 < step_hi; buf ^= 1) {
     compute(s0, buf);
-    if (s1 < step_hi) sstore(buf ^ 1, rkA, rvA);
-    if (s2 < step_hi) gload(s2, rkA, rvA);
-    __syncthreads();
+    if (s1 < step_hi) sstore(buf ^ 1);
+    if (s2 < step_hi) gload(s2);
     s0 = s1; s1 = s2; s2 = next_step(s2 + 1);
+    if (s2 < step_hi) pages(s2);
+    __syncthreads();
   }
-#endif
 
 #pragma unroll
   for (int ct = 0; ct < NCT; ++ct) {
@@ -891,6 +905,10 @@ __global__ __launch_bounds__(256, PREFILL_WGS_PER_CU) void paged_prefill_lds_ker
     const int c = wave * COLS + ct * 16 + r;
     const int head = head0 + c % G;
     const float inv = l[ct] > 0.f ? p.v_scale / l[ct] : 0.f;
+    if (p.nsplit > 1) {
+      store_part<D>(p, col_off[ct], head, g, acc[ct], inv, m[ct], l[ct]);
+      continue;
+    }
     T* op = (T*)p.out + col_off[ct] * p.out_stride + (long)head * D + 4 * g;
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
@@ -916,10 +934,13 @@ __global__ __launch_bounds__(256, PREFILL_WGS_PER_CU) void paged_prefill_lds_ker
 constexpr int REDUCE_ONE_WAVE = 8;                      // partitions
 template <typename T, int D, int W>
 __global__ __launch_bounds__(64 * W) void attn_reduce_kernel(T* out, const float* part_out, const float* part_lse,
-                                                             int Hq, int nsplit, long out_stride) {
+                                                             int Hq, int nsplit, long out_stride, const int* q_start_loc,
+                                                             int num_seqs) {
   constexpr int LANES = D / 4, ROWS = 64 * W / LANES, MAXP = W == 1 ? REDUCE_ONE_WAVE : 64, U = (MAXP + ROWS - 1) / ROWS;
   __shared__ __attribute__((aligned(16))) float sum[ROWS][D];
   const long th = blockIdx.x;          // token * Hq + head
+  // (prompts: rows that belong to no sequence have no parts and stay as they are)
+  if (q_start_loc && (th / Hq < q_start_loc[0] || th / Hq >= q_start_loc[num_seqs])) return;
   const int lane = threadIdx.x & 63, col = 4 * ((int)threadIdx.x % LANES), row = threadIdx.x / LANES;
   f32x4 v[U];
 #pragma unroll
@@ -1001,14 +1022,14 @@ static int launch_attn(const AttnParams& p, int form, int grid_x, hipStream_t st
       else hipLaunchKernelGGL((paged_decode_kernel<T, D, BS, 2, F8>), grid, block, 0, st, c);
     }
   } else if (form == 3) {
-    dim3 grid(grid_x, p.Hkv, 1);
+    dim3 grid(grid_x, p.Hkv, p.nsplit);
     if constexpr (D == 64 || D == 128) {          // the LDS tile layout is built for rows of 8 or 16 pieces
       hipLaunchKernelGGL((paged_prefill_lds_kernel<T, D, BS, F8>), grid, block, 0, st, p, SparseSel{});
     } else {
       hipLaunchKernelGGL((paged_attn_kernel<T, D, BS, 2, F8>), grid, block, 0, st, p);
     }
   } else {
-    dim3 grid(grid_x, p.Hkv, 1);
+    dim3 grid(grid_x, p.Hkv, p.nsplit);
     hipLaunchKernelGGL((paged_attn_kernel<T, D, BS, 2, F8>), grid, block, 0, st, p);
   }
   VDA_CHECK_LAUNCH();
@@ -1051,6 +1072,25 @@ static int dispatch_d(const AttnParams& p, int d, int bs, int form, int grid_x, 
   return dispatch_d8<T, false>(p, d, bs, form, grid_x, st);
 }
 
+static void launch_reduce(const AttnParams& p, int dtype, int D, int num_tokens, const int* q_start_loc, hipStream_t st) {
+  const long n = (long)num_tokens * p.Hq;
+#define RED(TT, DD) do {                                                                                              \
+    if (p.nsplit <= REDUCE_ONE_WAVE)                                                                                     \
+      hipLaunchKernelGGL((attn_reduce_kernel<TT, DD, 1>), dim3(n), dim3(64), 0, st, (TT*)p.out, p.part_out, p.part_lse, \
+                         p.Hq, p.nsplit, p.out_stride, q_start_loc, p.num_seqs);                                         \
+    else                                                                                                                 \
+      hipLaunchKernelGGL((attn_reduce_kernel<TT, DD, 4>), dim3(n), dim3(256), 0, st, (TT*)p.out, p.part_out, p.part_lse, \
+                         p.Hq, p.nsplit, p.out_stride, q_start_loc, p.num_seqs); } while (0)
+  if (dtype == VDA_BF16) {
+    if (D == 64) RED(bf16_t, 64); else if (D == 96) RED(bf16_t, 96); else if (D == 128) RED(bf16_t, 128);
+    else if (D == 192) RED(bf16_t, 192); else RED(bf16_t, 256);
+  } else {
+    if (D == 64) RED(f16_t, 64); else if (D == 96) RED(f16_t, 96); else if (D == 128) RED(f16_t, 128);
+    else if (D == 192) RED(f16_t, 192); else RED(f16_t, 256);
+  }
+#undef RED
+}
+
 // Decode / speculative-verify attention.  Every sequence contributes
 // q_len = q_start_loc[s+1]-q_start_loc[s] query tokens with q_len * (Hq/Hkv) <= 32.
 // num_tokens is only needed to size the split-KV reduce.
@@ -1075,20 +1115,7 @@ VDA_EXPORT int vda_paged_attention_decode(
                              : dispatch_d<f16_t>(p, D, block_size, form, num_seqs, st, kv_fp8);
   if (rc) return rc;
   if (nsplit > 1) {
-    const long n = (long)num_tokens * Hq;
-#define RED(TT, DD) do {                                                                                             \
-    if (nsplit <= REDUCE_ONE_WAVE) hipLaunchKernelGGL((attn_reduce_kernel<TT, DD, 1>), dim3(n), dim3(64), 0, st,        \
-                                                      (TT*)out, part_out, part_lse, Hq, nsplit, out_stride);            \
-    else hipLaunchKernelGGL((attn_reduce_kernel<TT, DD, 4>), dim3(n), dim3(256), 0, st, (TT*)out, part_out, part_lse,  \
-                            Hq, nsplit, out_stride); } while (0)
-    if (dtype == VDA_BF16) {
-      if (D == 64) RED(bf16_t, 64); else if (D == 96) RED(bf16_t, 96); else if (D == 128) RED(bf16_t, 128);
-      else if (D == 192) RED(bf16_t, 192); else RED(bf16_t, 256);
-    } else {
-      if (D == 64) RED(f16_t, 64); else if (D == 96) RED(f16_t, 96); else if (D == 128) RED(f16_t, 128);
-      else if (D == 192) RED(f16_t, 192); else RED(f16_t, 256);
-    }
-#undef RED
+    launch_reduce(p, dtype, D, num_tokens, nullptr, st);
     VDA_CHECK_LAUNCH();
   }
   return 0;
@@ -1102,6 +1129,24 @@ static long g_prefill_wide_min_wgs = 192;
 VDA_EXPORT int vda_set_prefill_variant(int v) { g_prefill_variant = v; return 0; }
 VDA_EXPORT int vda_set_prefill_wide_min_wgs(long n) { g_prefill_wide_min_wgs = n; return 0; }
 
+// Into how many parts the keys of each query tile are cut (1: not at all; what lse_out and the wide form take).  max_keys: an
+// upper bound of the sequences' lengths.  Without parts a few tiles walk a long prefix alone, 32 keys in some 1.2 us:
+// 100 new tokens on 2000 of each of two, 32 / 8 heads of 64 137 us in one part, 37 in seven; 16 / 8 heads of 256 386 -> 83, 24 / 8 of 96 255 -> 57;
+// of 128, on 3500, 300 -> 70; one prompt of 1000, 8 / 1 heads, 47 -> 30.
+// Two workgroups a CU are filled, with eight steps a part at least; a part's rows are written and read back once, so that
+// many query rows want few parts: their cost grows with the parts as the walk's falls.
+VDA_EXPORT int vda_prefill_parts(int num_seqs, int num_tokens, int Hq, int Hkv, int D, int max_q_len, long max_keys) {
+  if (Hkv < 1 || Hq % Hkv || Hq / Hkv > 128) return 1;
+  const int G = Hq / Hkv, q_tile = 128 / G;
+  if (D == 128 && 256 % G == 0 && (g_prefill_variant == 3 || (g_prefill_variant == 1 &&
+      (long)(num_tokens / (256 / G)) * Hkv >= g_prefill_wide_min_wgs))) return 1;
+  const long wgs = (long)(num_tokens / q_tile + min(num_seqs, num_tokens)) * Hkv, steps = (max_keys + 31) / 32;
+  if (wgs < 1 || wgs > 256 || steps < 16) return 1;
+  const double walk = 1.2 * steps, row_part = (double)num_tokens * Hq * D * 8 / 4e6;         // us
+  const long parts = max(1L, min(min(min(512 / wgs, steps / 8), (long)sqrt(walk / row_part) + 1), 64L));
+  return walk * (1 - 1.0 / parts) > 4 + row_part * parts ? (int)parts : 1;                    // (4: the launch that merges them)
+}
+
 // Varlen attention of new tokens against the paged cache (the new tokens' own K/V must already be in
 // the cache): causal, or bidirectional within each sequence (encoder models; the shared-prefix pass of
 // cascade attention, where one pseudo-sequence holds every query token of the batch).  lse_out, when
@@ -1112,13 +1157,15 @@ VDA_EXPORT int vda_paged_attention_prefill(
     const int* seq_lens, const int* q_start_loc, const float* alibi, int num_seqs, int num_tokens,
     int Hq, int Hkv, int D, int block_size, int max_blocks, long q_stride, long out_stride, float scale,
     float softcap, int window, int dtype, int kv_fp8, float k_scale, float v_scale, int causal, float* lse_out,
-    int max_q_len, const float* sink, int chunk, int v_shift, const float* dist_bias, int dist_far, hipStream_t st) {
+    int max_q_len, const float* sink, int chunk, int v_shift, const float* dist_bias, int dist_far, float* part_out,
+    float* part_lse, int nsplit, hipStream_t st) {
   if (Hq % Hkv) return -1;
   const int G = Hq / Hkv;
   if (G > 128) return -4;
   if (!causal && (window > 0 || chunk > 0)) return -5;
   if (chunk < 0 || v_shift < 0 || (Hkv >> v_shift) << v_shift != Hkv) return -7;
   if (dist_bias && dist_far < 0) return -7;
+  if (nsplit < 1 || nsplit > 64 || (nsplit > 1 && (!part_out || !part_lse || lse_out))) return -6;
   // not in the direct-to-register form
   const bool extras = sink != nullptr || chunk > 0 || v_shift > 0 || dist_bias != nullptr;
   const int q_tile = 128 / G;     // 4 waves x 32 columns
@@ -1128,7 +1175,7 @@ VDA_EXPORT int vda_paged_attention_prefill(
   p.sink = sink; p.chunk = chunk; p.v_shift = v_shift; p.dist_bias = dist_bias; p.dist_far = dist_far;
   // Wide form (8 waves, 256 columns, 64-key tiles): head size 128 and enough query tiles to occupy the
   // chip (one workgroup per CU); short chunks keep the 4-wave form, which cuts them into more workgroups.
-  if (D == 128 && 256 % G == 0 && (g_prefill_variant == 1 || g_prefill_variant == 3)) {
+  if (nsplit == 1 && D == 128 && 256 % G == 0 && (g_prefill_variant == 1 || g_prefill_variant == 3)) {
     const int wide_tile = 256 / G;
     const long wgs = (long)(num_tokens / wide_tile) * Hkv;
     if (g_prefill_variant == 3 || wgs >= g_prefill_wide_min_wgs) {
@@ -1138,8 +1185,13 @@ VDA_EXPORT int vda_paged_attention_prefill(
   }
   const int grid_x = num_tokens / q_tile + num_seqs;
   const int form = (g_prefill_variant == 0 && !extras) ? 2 : 3;
-  return dtype == VDA_BF16 ? dispatch_d<bf16_t>(p, D, block_size, form, grid_x, st, kv_fp8)
-                           : dispatch_d<f16_t>(p, D, block_size, form, grid_x, st, kv_fp8);
+  p.part_out = part_out; p.part_lse = part_lse; p.nsplit = nsplit;
+  const int rc = dtype == VDA_BF16 ? dispatch_d<bf16_t>(p, D, block_size, form, grid_x, st, kv_fp8)
+                                   : dispatch_d<f16_t>(p, D, block_size, form, grid_x, st, kv_fp8);
+  if (rc || nsplit == 1) return rc;
+  launch_reduce(p, dtype, D, num_tokens, q_start_loc, st);
+  VDA_CHECK_LAUNCH();
+  return 0;
 }
 
 // Sparse (vertical-slash) prefill: the 4-wave LDS form, one head per workgroup, visiting only the selected 32-key
