@@ -95,3 +95,18 @@ def test_tile_search(S, D):
     n_live = torch.tensor([0] + [new[s] for s in live]).cumsum(0).to(torch.int32).to(DEV)
     want = R.paged_attention(q.float(), kc.float(), vc.float(), table[live], sl[live], n_live, D ** -0.5)
     assert float((out.float() - want).abs().max()) <= (2 * 2.0 ** -9 + 1e-5) * float(vc.float().abs().max())
+
+
+@pytest.mark.parametrize("D", [96, 192, 256])
+@pytest.mark.parametrize("Hq,Hkv", [(6, 2), (64, 1), (80, 1)])           # a head group as wide as a workgroup's columns, and wider
+@pytest.mark.parametrize("kw", [dict(), dict(window=50), dict(causal=False)])
+def test_heads_that_are_no_power_of_two_or_wide(D, Hq, Hkv, kw):
+    """Tiles and key steps that end inside a workgroup, every page size's rows in LDS."""
+    for BS in (16, 32, 64):
+        b = _batch([3, 64, 130, 33], [0, 31, 5, 64], Hq, Hkv, D, BS, torch.float16)
+        q, kc, vc, table, sl, starts = b
+        out = torch.empty_like(q)
+        out, lse = ops.paged_attention_prefill(out, q, kc, vc, table, sl, starts, D ** -0.5, return_lse=True, **kw)
+        want, want_lse = R.paged_attention(q.float(), kc.float(), vc.float(), table, sl, starts, D ** -0.5, return_lse=True, **kw)
+        assert float((out.float() - want).abs().max()) <= (2 * 2.0 ** -12 + 1e-5) * float(vc.float().abs().max())
+        torch.testing.assert_close(lse, want_lse.float(), atol=1e-4, rtol=1e-5)

@@ -609,18 +609,24 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(AttnParams p) {
 // Inside a visited step every key is seen (subject to the causal limit), so the pattern is a superset of the exact
 // lines at 32-key granularity.
 constexpr int SPARSE_BM_WORDS = 4096;        // 4096 x 32 steps x 32 keys = 4 Mi keys per table
+// Query columns of a workgroup: 32 a wave, or 16 where the outputs and the queries of more would not fit the registers of two
+// workgroups a CU.  Heads of 96, 192 and 256 values took the direct form before: us, eight prompts of some 1000, 16 / 8 heads of 256 535 -> 308,
+// 24 / 8 of 96 255 -> 196; four of 300 78 -> 54 and 49 -> 41.
+template <int D> constexpr int PREFILL_COLS = D <= 128 ? 128 : 64;
 template <typename T, int D, int BS, bool F8, bool SPARSE = false>
 __global__ __launch_bounds__(256, PREFILL_WGS_PER_CU) void paged_prefill_lds_kernel(AttnParams p, SparseSel sp) {
   using V8 = typename Vec<T>::v8;
   using V4 = typename Vec<T>::v4;
   using CT = typename KVElem<T, F8>::type;
-  constexpr int KS = D / 32, NT = D / 16, DQ = D / 4, NCT = 2, COLS = 32;
+  constexpr int KS = D / 32, NT = D / 16, DQ = D / 4, NCT = PREFILL_COLS<D> / 64, COLS = 16 * NCT;
   constexpr int KCH = D / 8;          // 16-byte pieces per K row
+  constexpr bool XOR = (KCH & (KCH - 1)) == 0;
+  constexpr int KROW = XOR ? KCH : KCH + 1;     // pieces between two rows: swizzled ones, or an odd number
   constexpr int KP = 32 * KCH;        // K pieces per 32-key step
   constexpr int VP = D * 4;           // V pieces per step (D rows x 4 groups of 8 keys)
-  constexpr int KPT = KP / 256, VPT = VP / 256;
-  static_assert(KP % 256 == 0 && VP % 256 == 0, "head size must be a multiple of 64");
-  __shared__ V8 sK[2][KP];
+  constexpr int KPT = (KP + 255) / 256, VPT = (VP + 255) / 256;
+  static_assert(D % 32 == 0, "head sizes are multiples of an MFMA step");
+  __shared__ V8 sK[2][32 * KROW];
   __shared__ V8 sV[2][VP];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
@@ -733,11 +739,13 @@ __global__ __launch_bounds__(256, PREFILL_WGS_PER_CU) void paged_prefill_lds_ker
 #pragma unroll
     for (int i = 0; i < VPT; ++i) pv[i] = (unsigned)bt[max(min((tb + 8 * ((tid + 256 * i) & 3)) / BS, nblk_valid - 1), 0)];
   };
+  // (the last of a thread's pieces may be past a step's)
   auto gload = [&](int step) {
     const int tb = step * 32;
 #pragma unroll
     for (int i = 0; i < KPT; ++i) {
       const int pi = tid + 256 * i;
+      if (KP % 256 && pi >= KP) break;
       const int key = pi / KCH, ch = pi % KCH;
       const int tok = tb + key;
       const unsigned off = k_head + (unsigned)(tok % BS) * D + ch * 8;
@@ -746,6 +754,7 @@ __global__ __launch_bounds__(256, PREFILL_WGS_PER_CU) void paged_prefill_lds_ker
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
       const int pi = tid + 256 * i;
+      if (VP % 256 && pi >= VP) break;
       const int d = pi >> 2, c = pi & 3;
       const int tok = tb + 8 * c;
       const unsigned off = v_head + (unsigned)d * BS + (tok % BS);
@@ -756,17 +765,19 @@ __global__ __launch_bounds__(256, PREFILL_WGS_PER_CU) void paged_prefill_lds_ker
   // {4-11,16-19,28-31} (and the same in the upper half) together; with the key a lane reads (krow0 + 4u
   // below) these masks put the sixteen lanes of every such group on sixteen different pieces, where the
   // earlier three-bit mask left them two-way (one extra LDS cycle per group on every K operand read).
-  auto kswz = [](int key) { return KCH == 16 ? (key & 15) : (((key & 3) << 1) | ((key >> 3) & 1)); };
+  auto kswz = [](int key) { return !XOR ? 0 : KCH >= 16 ? (key & 15) : (((key & 3) << 1) | ((key >> 3) & 1)); };
   auto sstore = [&](int buf) {
 #pragma unroll
     for (int i = 0; i < KPT; ++i) {
       const int pi = tid + 256 * i;
+      if (KP % 256 && pi >= KP) break;
       const int key = pi / KCH, ch = pi % KCH;
-      sK[buf][key * KCH + (ch ^ kswz(key))] = rk[i];
+      sK[buf][key * KROW + (ch ^ kswz(key))] = rk[i];
     }
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
       const int pi = tid + 256 * i;
+      if (VP % 256 && pi >= VP) break;
       const int d = pi >> 2, c = pi & 3;
       sV[buf][d * 4 + (c ^ ((d >> 1) & 3))] = rv[i];
     }
@@ -792,17 +803,23 @@ __global__ __launch_bounds__(256, PREFILL_WGS_PER_CU) void paged_prefill_lds_ker
     if (!(tb0 < wave_hi && tb0 + 32 > wave_lo)) return;   // wave-uniform: tile outside this wave's causal range
     const bool far_tile = p.dist_bias != nullptr && tb0 + 32 <= full_hi - p.dist_far;
     const bool fast = plain && tb0 + 32 <= full_hi && tb0 >= full_lo && (p.dist_bias == nullptr || far_tile);
-    V8 kf[2][KS], vf[NT];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    // read once for all of a wave's column tiles, or where they are multiplied
+    auto k_piece = [&](int u, int s) {
       const int key = krow0 + 4 * u;
-#pragma unroll
-      for (int s = 0; s < KS; ++s) kf[u][s] = sK[buf][key * KCH + ((g * KS + s) ^ kswz(key))];
-    }
-#pragma unroll
-    for (int n = 0; n < NT; ++n) {
+      return sK[buf][key * KROW + ((g * KS + s) ^ kswz(key))];
+    };
+    auto v_piece = [&](int n) {
       const int d = 16 * n + r;
-      vf[n] = sV[buf][d * 4 + (g ^ ((d >> 1) & 3))];
+      return sV[buf][d * 4 + (g ^ ((d >> 1) & 3))];
+    };
+    V8 kf[2][KS], vf[NT];
+    if constexpr (NCT > 1) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int s = 0; s < KS; ++s) kf[u][s] = k_piece(u, s);
+#pragma unroll
+      for (int n = 0; n < NT; ++n) vf[n] = v_piece(n);
     }
     const int tb = tb0 + 8 * g;
 #pragma unroll
@@ -810,8 +827,8 @@ __global__ __launch_bounds__(256, PREFILL_WGS_PER_CU) void paged_prefill_lds_ker
       f32x4 s0 = {0, 0, 0, 0}, s1 = {0, 0, 0, 0};
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
-        s0 = mfma16(kf[0][s], qf[ct][s], s0);
-        s1 = mfma16(kf[1][s], qf[ct][s], s1);
+        s0 = mfma16(NCT > 1 ? kf[0][s] : k_piece(0, s), qf[ct][s], s0);
+        s1 = mfma16(NCT > 1 ? kf[1][s] : k_piece(1, s), qf[ct][s], s1);
       }
       float sv[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
       float mx = -INFINITY;
@@ -867,7 +884,7 @@ __global__ __launch_bounds__(256, PREFILL_WGS_PER_CU) void paged_prefill_lds_ker
         for (int n = 0; n < NT; ++n) acc[ct][n] *= alpha;
       }
 #pragma unroll
-      for (int n = 0; n < NT; ++n) acc[ct][n] = mfma16(vf[n], pb, acc[ct][n]);
+      for (int n = 0; n < NT; ++n) acc[ct][n] = mfma16(NCT > 1 ? vf[n] : v_piece(n), pb, acc[ct][n]);
     }
   };
 
@@ -1023,11 +1040,7 @@ static int launch_attn(const AttnParams& p, int form, int grid_x, hipStream_t st
     }
   } else if (form == 3) {
     dim3 grid(grid_x, p.Hkv, p.nsplit);
-    if constexpr (D == 64 || D == 128) {          // the LDS tile layout is built for rows of 8 or 16 pieces
-      hipLaunchKernelGGL((paged_prefill_lds_kernel<T, D, BS, F8>), grid, block, 0, st, p, SparseSel{});
-    } else {
-      hipLaunchKernelGGL((paged_attn_kernel<T, D, BS, 2, F8>), grid, block, 0, st, p);
-    }
+    hipLaunchKernelGGL((paged_prefill_lds_kernel<T, D, BS, F8>), grid, block, 0, st, p, SparseSel{});
   } else {
     dim3 grid(grid_x, p.Hkv, p.nsplit);
     hipLaunchKernelGGL((paged_attn_kernel<T, D, BS, 2, F8>), grid, block, 0, st, p);
@@ -1125,6 +1138,7 @@ VDA_EXPORT int vda_paged_attention_decode(
 // 0: direct-to-register form, 2: always the 4-wave LDS form, 3: the wide form whenever the shape allows
 // (0 / 2 / 3 are for A/B measurements and tests)
 static int g_prefill_variant = 1;
+static int prefill_cols(int D) { return D <= 128 ? PREFILL_COLS<128> : PREFILL_COLS<256>; }
 static long g_prefill_wide_min_wgs = 192;
 VDA_EXPORT int vda_set_prefill_variant(int v) { g_prefill_variant = v; return 0; }
 VDA_EXPORT int vda_set_prefill_wide_min_wgs(long n) { g_prefill_wide_min_wgs = n; return 0; }
@@ -1137,7 +1151,7 @@ VDA_EXPORT int vda_set_prefill_wide_min_wgs(long n) { g_prefill_wide_min_wgs = n
 // many query rows want few parts: their cost grows with the parts as the walk's falls.
 VDA_EXPORT int vda_prefill_parts(int num_seqs, int num_tokens, int Hq, int Hkv, int D, int max_q_len, long max_keys) {
   if (Hkv < 1 || Hq % Hkv || Hq / Hkv > 128) return 1;
-  const int G = Hq / Hkv, q_tile = 128 / G;
+  const int G = Hq / Hkv, q_tile = (G <= prefill_cols(D) ? prefill_cols(D) : 128) / G;
   if (D == 128 && 256 % G == 0 && (g_prefill_variant == 3 || (g_prefill_variant == 1 &&
       (long)(num_tokens / (256 / G)) * Hkv >= g_prefill_wide_min_wgs))) return 1;
   const long wgs = (long)(num_tokens / q_tile + min(num_seqs, num_tokens)) * Hkv, steps = (max_keys + 31) / 32;
@@ -1168,7 +1182,9 @@ VDA_EXPORT int vda_paged_attention_prefill(
   if (nsplit < 1 || nsplit > 64 || (nsplit > 1 && (!part_out || !part_lse || lse_out))) return -6;
   // not in the direct-to-register form
   const bool extras = sink != nullptr || chunk > 0 || v_shift > 0 || dist_bias != nullptr;
-  const int q_tile = 128 / G;     // 4 waves x 32 columns
+  // the form with K and V in LDS takes a head group's queries as columns of one workgroup
+  const bool lds = (g_prefill_variant != 0 || extras) && G <= prefill_cols(D);
+  const int q_tile = (lds ? prefill_cols(D) : 128) / G;
   AttnParams p{q, k_cache, v_cache, out, nullptr, nullptr, block_table, seq_lens, q_start_loc, alibi,
                num_seqs, Hq, Hkv, max_blocks, 1, q_stride, out_stride, scale * (kv_fp8 ? k_scale : 1.f), softcap,
                kv_fp8 ? v_scale : 1.f, window, q_tile, causal, num_tokens, lse_out, max_q_len};
@@ -1184,7 +1200,7 @@ VDA_EXPORT int vda_paged_attention_prefill(
     }
   }
   const int grid_x = num_tokens / q_tile + num_seqs;
-  const int form = (g_prefill_variant == 0 && !extras) ? 2 : 3;
+  const int form = lds ? 3 : 2;
   p.part_out = part_out; p.part_lse = part_lse; p.nsplit = nsplit;
   const int rc = dtype == VDA_BF16 ? dispatch_d<bf16_t>(p, D, block_size, form, grid_x, st, kv_fp8)
                                    : dispatch_d<f16_t>(p, D, block_size, form, grid_x, st, kv_fp8);
