@@ -45,19 +45,18 @@ __device__ __forceinline__ QueryTile query_tile(const AttnParams& p, int tile) {
   return t;
 }
 
-// Prompts whose query tiles do not fill the chip: part blockIdx.z of gridDim.z of a tile's 32-key steps (prefill_parts says
-// how many), whose results attn_reduce_kernel merges.
-__device__ __forceinline__ void key_part(const AttnParams& p, int& step_lo, int& step_hi) {
+// Prompts whose query tiles do not fill the chip: one part of a tile's 32-key steps (vda_prefill_parts says how many there are), whose results attn_reduce_kernel merges.
+__device__ __forceinline__ void key_part(const AttnParams& p, int part, int& step_lo, int& step_hi) {
   if (p.nsplit <= 1) return;
   const int per = (max(step_hi - step_lo, 0) + p.nsplit - 1) / p.nsplit;
-  step_lo += blockIdx.z * per;
+  step_lo += part * per;
   step_hi = min(step_hi, step_lo + per);
 }
 // a lane's values 16 n + 4 g of one (token, head), as that part's row and its log2-domain weight
 template <int D>
-__device__ __forceinline__ void store_part(const AttnParams& p, long tok, int head, int g, const f32x4 (&acc)[D / 16], float inv,
-                                           float m, float l) {
-  const long at = (tok * p.Hq + head) * p.nsplit + blockIdx.z;
+__device__ __forceinline__ void store_part(const AttnParams& p, int part, long tok, int head, int g, const f32x4 (&acc)[D / 16],
+                                           float inv, float m, float l) {
+  const long at = (tok * p.Hq + head) * p.nsplit + part;
   if (l > 0.f) {                                          // (a part without keys is left out by its weight)
     float* po = p.part_out + at * D + 4 * g;
 #pragma unroll
@@ -126,7 +125,7 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(AttnParams p) {
     wave_lo = min(wave_lo, __shfl_xor(wave_lo, o, 64));
   }
   int step_lo = wave_hi > 0 ? wave_lo / 32 : 0, step_hi = (wave_hi + 31) / 32;
-  key_part(p, step_lo, step_hi);
+  key_part(p, blockIdx.z, step_lo, step_hi);
 
   float m[NCT], l[NCT];
   f32x4 acc[NCT][NT];
@@ -244,7 +243,7 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(AttnParams p) {
     const int head = kvh * G + c % G;
     const float inv = l[ct] > 0.f ? p.v_scale / l[ct] : 0.f;
     if (p.nsplit > 1) {
-      store_part<D>(p, col_off[ct], head, g, acc[ct], inv, m[ct], l[ct]);
+      store_part<D>(p, blockIdx.z, col_off[ct], head, g, acc[ct], inv, m[ct], l[ct]);
       continue;
     }
     T* op = (T*)p.out + col_off[ct] * p.out_stride + (long)head * D + 4 * g;
@@ -632,10 +631,22 @@ __global__ __launch_bounds__(256, PREFILL_WGS_PER_CU) void paged_prefill_lds_ker
   const int lane = tid & 63, wave = tid >> 6;
   const int r = lane & 15, g = lane >> 4;
   const int G = SPARSE ? 1 : p.Hq / p.Hkv;
-  const int kvh = SPARSE ? blockIdx.y / (p.Hq / p.Hkv) : blockIdx.y;
+  // The tiles of one kv head's part read the same keys: neighbouring items of one XCD (workgroups are dealt to the eight in
+  // turn), whose L2 then serves them, the longest tiles of a prompt first (us, tiles over all XCDs -> this: eight prompts of some
+  // 1000, 16 / 8 heads of 256 308 -> 268, 24 / 8 of 96 196 -> 167, 32 / 8 of 64 141 -> 128; 25 new tokens on 3000 of two, 64 / 8 of
+  // 128, 70 -> 45).
+  int tile = blockIdx.x, part = 0, kvh = SPARSE ? blockIdx.y / (p.Hq / p.Hkv) : blockIdx.y;
+  if constexpr (!SPARSE) {
+    const int tiles = gridDim.x, n = tiles * gridDim.y * gridDim.z;
+    const int id = blockIdx.x + tiles * (blockIdx.y + gridDim.y * blockIdx.z), x = id & 7, more = n & 7;
+    const int item = x * (n >> 3) + min(x, more) + (id >> 3), group = item / tiles;
+    tile = tiles - 1 - (item - group * tiles);
+    kvh = group % (int)gridDim.y;
+    part = group / (int)gridDim.y;
+  }
   const int head0 = SPARSE ? blockIdx.y : kvh * G;        // first query head of this workgroup's columns
 
-  const QueryTile own = query_tile(p, blockIdx.x);
+  const QueryTile own = query_tile(p, tile);
   const int seq = own.seq, q0 = own.q0, qs = own.qs, q_len = own.q_len, seq_len = own.seq_len;
   if (q0 >= q_len) return;                  // uniform over the workgroup
   const int ctx = seq_len - q_len;
@@ -680,9 +691,9 @@ __global__ __launch_bounds__(256, PREFILL_WGS_PER_CU) void paged_prefill_lds_ker
   if (p.chunk > 0 && p.causal) wg_lo = max(wg_lo, (ctx + q0) / p.chunk * p.chunk);
   int step_lo = wg_lo / 32, step_hi = (wg_hi + 31) / 32;
   if constexpr (!SPARSE) {
-    key_part(p, step_lo, step_hi);
+    key_part(p, part, step_lo, step_hi);
 #pragma unroll
-    for (int ct = 0; ct < NCT; ++ct) sink_m[ct] = blockIdx.z > 0 ? -INFINITY : sink_m[ct];   // (a sink joins once)
+    for (int ct = 0; ct < NCT; ++ct) sink_m[ct] = part > 0 ? -INFINITY : sink_m[ct];   // (a sink joins once)
   }
 
   __shared__ unsigned bm[SPARSE ? SPARSE_BM_WORDS : 1];
@@ -923,7 +934,7 @@ __global__ __launch_bounds__(256, PREFILL_WGS_PER_CU) void paged_prefill_lds_ker
     const int head = head0 + c % G;
     const float inv = l[ct] > 0.f ? p.v_scale / l[ct] : 0.f;
     if (p.nsplit > 1) {
-      store_part<D>(p, col_off[ct], head, g, acc[ct], inv, m[ct], l[ct]);
+      store_part<D>(p, part, col_off[ct], head, g, acc[ct], inv, m[ct], l[ct]);
       continue;
     }
     T* op = (T*)p.out + col_off[ct] * p.out_stride + (long)head * D + 4 * g;
