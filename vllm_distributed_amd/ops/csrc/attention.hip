@@ -1150,7 +1150,9 @@ VDA_EXPORT int vda_paged_attention_decode(
 // (0 / 2 / 3 are for A/B measurements and tests)
 static int g_prefill_variant = 1;
 static int prefill_cols(int D) { return D <= 128 ? PREFILL_COLS<128> : PREFILL_COLS<256>; }
-static long g_prefill_wide_min_wgs = 192;
+// (from 128 on: us, 4-wave form with the keys in parts / wide form, 128 of them 67.8 / 49.4 and 88 / 61, 144 25.4 / 22.8, 184 140 / 119; 100 of long
+// prompts 97 / 113, of 1000 tokens 44.6 / 39.8)
+static long g_prefill_wide_min_wgs = 128;
 VDA_EXPORT int vda_set_prefill_variant(int v) { g_prefill_variant = v; return 0; }
 VDA_EXPORT int vda_set_prefill_wide_min_wgs(long n) { g_prefill_wide_min_wgs = n; return 0; }
 
