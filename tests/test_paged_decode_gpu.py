@@ -88,3 +88,16 @@ def test_order_of_large_batches(S, lens):
 @pytest.mark.parametrize("D", [64, 96, 128, 192, 256])
 def test_merge_of_parts(D, nsplit):
     _check([1, 40, 300, 2100, 0], [1] * 5, 6, 2, D, 16, torch.bfloat16, False, nsplit)
+
+
+# two parts of few sequences: eight waves of one workgroup (up to 256 of them), parts and a merge beyond and above 16 columns
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("D,Hq,Hkv,S", [(64, 4, 4, 17), (128, 16, 1, 17), (96, 6, 2, 17), (192, 4, 1, 17), (256, 4, 2, 17), (128, 8, 8, 32),
+                                        (128, 8, 8, 33), (128, 32, 1, 17)])
+def test_two_parts(D, Hq, Hkv, S, fp8):
+    if fp8 and D not in (64, 128):
+        pytest.skip("e4m3 caches: head sizes 64 and 128")
+    lens = ((EDGES + [0, 1025]) * 2)[:S]
+    _check(lens, [1] * S, Hq, Hkv, D, 16, torch.bfloat16, fp8, 2)
+    if Hq // Hkv <= 4:
+        _check([max(n, 4) for n in lens], [1 + i % 4 for i in range(S)], Hq, Hkv, D, 16, torch.float16, fp8, 2, window=300)

@@ -263,7 +263,12 @@ def paged_attention_decode(out, q, k_cache, v_cache, block_table, seq_lens, q_st
     S = seq_lens.shape[0]
     part_out = part_lse = None
     if num_splits > 1:
-        if workspace is not None:
+        # a few short sequences (512 workgroups of four waves at most): two parts as waves of one workgroup, which want no
+        # workspace and no launch that merges them
+        Hkv = k_cache.shape[1]
+        if num_splits == 2 and S * Hkv <= 256 and D <= 192 and max_q_len * (Hq // Hkv) <= 16:
+            pass
+        elif workspace is not None:
             part_out, part_lse = workspace[0].data_ptr(), workspace[1].data_ptr()
         else:                                            # the parts' rows, then their weights: an allocation is 1.5 us
             part = torch.empty(T * Hq * num_splits * (D + 1), dtype=torch.float32, device=q.device)
