@@ -213,3 +213,28 @@ def test_two_states_a_lane_without(left_out):
     # one bf16 rounding of y
     torch.testing.assert_close(y.float(), want.float(), atol=0.05, rtol=2 ** -7)
     torch.testing.assert_close(a["ssm_state"], b["ssm_state"], atol=1e-4, rtol=1e-4)
+
+
+@pytest.mark.parametrize("Ch,N,heads,groups", [(128, 64, 4, 1), (64, 128, 4, 1), (256, 128, 4, 2), (64, 256, 2, 2), (32, 128, 1, 1)])
+@pytest.mark.parametrize("new,ctx", [([100, 1, 8, 9, 0], [0, 4, 0, 1, 0]),           # eight tokens at a time, tiles of 16
+                                     ([15, 16, 17, 130], [2, 0, 1, 0]), ([64, 65, 97, 2], [0, 5, 0, 3])])
+@pytest.mark.parametrize("chunks", [False, True])
+def test_eight_states_a_lane(monkeypatch, new, ctx, Ch, N, heads, groups, chunks):
+    # heads of one workgroup's channels and of several workgroups', chunks of two tiles (the setting asks for them)
+    if chunks:
+        monkeypatch.setenv("VDA_SCAN_CHUNK_MIN_TOKENS", "96")
+    a = _scan_inputs(new, ctx, Ch, N, heads, groups, torch.float16, Ch + N + len(new))
+    a = {k: v.contiguous() if isinstance(v, torch.Tensor) else v for k, v in a.items()}
+    names = ("u", "delta", "A", "B", "C", "D", "z", "delta_bias", "ssm_state")
+    b = {k: v.clone() if isinstance(v, torch.Tensor) else v for k, v in a.items()}
+    called, call = [], ops.N.call
+    monkeypatch.setattr(ops.N, "call", lambda name, *args: (called.append((name, args[27], args[29])), call(name, *args))[1])
+    y = ops.selective_scan(**a, max_query_len=max(new))
+    (name, form, nchunks), = called
+    assert (name, form) == ("vda_selective_scan_pairs", 3) and (nchunks > 1) == chunks
+    f = {k: v.float() if isinstance(v, torch.Tensor) and v.dtype == torch.float16 else v for k, v in b.items()}
+    want = R.selective_scan(*(f[k] for k in names), b["query_start_loc"], b["seq_lens"], b["block_table"], num_groups=groups)
+    live = torch.cat([torch.full((n,), bool(n + c)) for n, c in zip(new, ctx)]).to(DEV)
+    # 32-bit sums of N states carried through up to 130 decays, one fp16 rounding of the result
+    torch.testing.assert_close(y.float()[live], want[live], atol=1e-3, rtol=2 ** -10)
+    torch.testing.assert_close(a["ssm_state"], f["ssm_state"], atol=1e-4, rtol=1e-4)

@@ -1504,18 +1504,28 @@ def selective_scan(u: torch.Tensor, delta: torch.Tensor, A: torch.Tensor, B: tor
     # x 8192 channels 89 / 125 us, of 34 x 4096 80 / 79, 100 of 43 x 4096 87 / 75, 64 of 51 69 / 56, three of 1558 x 8192 300 / 163.
     lanes = not step and Nst == 16 and A.dim() == 2 and rep == 1 and (num_groups == 1 or gch % 32 == 0) \
         and ssm_state.data_ptr() % 16 == 0 and A.data_ptr() % 16 == 0 and (not few_tokens or paired and max_query_len >= 40)
-    paired = paired or lanes
+    # Eight states a lane (Mamba-2 in 16 bits: 64 states and more, a decay rate per head), from 16 tokens on.  us, pairs / this, 4096
+    # channels x 128 states: one of 80 tokens 61 / 20, of 482 114 / 70, three of 1558 at most 598 / 254, 16 of 173 226 / 118, of 17
+    # 27.6 / 25.8, 64 of 34 123 / 121, of 8 49 / 70
+    own = 2048 // Nst                                                  # channels of a workgroup
+    groups = not step and Nst in (64, 128, 256) and A.dim() == 1 and eb == 2 and max_query_len >= 16 \
+        and Ch % own == 0 and rep % own == 0 and gch % own == 0 and ssm_state.data_ptr() % 16 == 0 \
+        and all(t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (B, C))
+    paired = paired or lanes or groups
     chunk, nchunks, ws_p, ws_h = 0, 1, None, None
     # unless the setting says otherwise, from 96 tokens on in pairs (seven prompts of 82 tokens on average, 4096 x 16: 140 us in
     # one pass, 82 in chunks of 32), from 256 on in the plain form, where more passes over more states pay later, and with
     # two states a lane, whose waves (eight channels each) are only cut where they leave SIMDs with less than two: us in one
     # pass / cut, 4096 channels: 241 tokens 32 / 32, 402 43 / 33, 1609 148 / 70; 8192: 322 tokens 31 / 37, 1609 155 / 119;
-    # 16384 channels and sequences: 1212 tokens 126 / 128; 24576: 1558 tokens 163 / 206
-    if max_query_len >= ((96 if paired and not lanes else 256) if set_min is None else set_min):
+    # 16384 channels and sequences: 1212 tokens 126 / 128; 24576: 1558 tokens 163 / 206.  Eight states a lane likewise, from 768 on: 4096
+    # channels: 482 tokens 69 / 70, 1609 248 / 192; 8192: 1212 tokens 196 / 193; 12288: 1558 254 / 339
+    if max_query_len >= ((768 if groups else 96 if paired and not lanes else 256) if set_min is None else set_min):
         # lanes per channel: N / 16, or as many for a pair of them
         least = 32 if paired else 64
         if lanes:
             want = -(-65536 // (S * Ch)) if S * Ch < 16384 else 1
+        elif groups:
+            want = -(-16384 // (S * Ch)) if S * Ch < 8192 else 1
         else:
             want = -(-524288 // (S * (Ch // (2 if paired else 1)) * (Nst // 16)))
         if want > 1:
@@ -1530,7 +1540,7 @@ def selective_scan(u: torch.Tensor, delta: torch.Tensor, A: torch.Tensor, B: tor
             u.stride(0), delta.stride(0), B.stride(0), C.stride(0), z.stride(0) if z is not None else 0, out.stride(0),
             rep, int(A.dim() == 1), gch, int(softplus))
     if paired:
-        N.call("vda_selective_scan_pairs", *args, 2 if lanes else int(step), chunk, nchunks, N.ptr(ws_p), N.ptr(ws_h), N.dt(u.dtype), N.stream())
+        N.call("vda_selective_scan_pairs", *args, 2 if lanes else 3 if groups else int(step), chunk, nchunks, N.ptr(ws_p), N.ptr(ws_h), N.dt(u.dtype), N.stream())
     else:
         N.call("vda_selective_scan", *args, chunk, nchunks, N.ptr(ws_p), N.ptr(ws_h), N.dt(u.dtype), N.stream())
     return out

@@ -308,7 +308,8 @@ __global__ __launch_bounds__(256) void scan_combine_kernel(float* __restrict__ w
 // the request's slot while the first one may not have begun, so the carry kernel puts the slot's state aside first.
 // Bound by vector issue: per state and token exp2 (4 slots), its argument, two for the state and one for y.
 // 3325 tokens of 8192 channels x 16 states, three sequences: both passes 637 -> 320 us;
-// 1100 tokens of 64 heads x 64 x 128 states: 990 -> 283 with the convolution.
+// 1100 tokens of 64 heads x 64 x 128 states: 990 -> 283 with the convolution.  (The two forms below take most of what this one
+// took: it keeps 32-bit inputs, rows off their boundaries, few tokens of many sequences.)
 struct ScanArgs {
   void* out;
   const void *u, *delta;
@@ -649,6 +650,183 @@ __global__ __launch_bounds__(256) void scan_lanes_kernel(ScanArgs p, int vec) {
   if (mine && (MODE == 1 || last)) *reinterpret_cast<f32x2*>(MODE == 1 ? p.ws_h + wc * N + 2 * q : hp) = h;
 }
 
+// ---- selective scan, one decay a head: eight states a lane --------------------------------------------------------------
+// Mamba-2: a step size and a decay rate per head, 64 states and more.  A workgroup takes 64 / Q channels of one head, its 4 Q lane
+// groups eight states each (Q lanes of every wave share a channel): three prompts of 64 heads x 64 are 3072 waves, which walk their
+// tokens in one pass.  Step size, decay and dt * u are worked out while a tile of 16 tokens is staged, and the gate and D join
+// when its sums come back, as above; the recurrence reads a pair and 16 values of B and C a token from LDS and does three
+// instructions a state.  A channel's sums go over its Q lanes transposed (Q tokens at a time) and over the waves through LDS.
+// Bound by the reads of B and C from LDS (32 cycles of a CU a wave and token beside 30 instructions).  us, pairs -> this, 4096 x 128
+// states: 3325 tokens of three 598 -> 254, one of 1609 337 -> 192, 16 of 173 at most 226 -> 118.
+constexpr int GR_TT = 16;
+template <typename T, int N, int MODE>
+__global__ __launch_bounds__(256) void scan_groups_kernel(ScanArgs p) {
+  typedef T v8_t __attribute__((ext_vector_type(8)));
+  constexpr int Q = N / 32, CH = 64 / Q;                // lanes of a wave per channel, channels of a workgroup
+  constexpr int PER = N / 4;                            // 16-byte pieces (8 values) of B and C of a tile
+  constexpr int STEPS = GR_TT * PER / 256 > 0 ? GR_TT * PER / 256 : 1;
+  __shared__ __attribute__((aligned(16))) float bc[GR_TT][2][N], dd[GR_TT][CH][2], ys[4][GR_TT][CH];
+  __shared__ float head_dt[GR_TT][2];
+  const int s = blockIdx.y;
+  const int sl = p.seq_lens[s];
+  if (sl <= 0) return;
+  const int t0 = p.qsl[s], L = p.qsl[s + 1] - t0;
+  const int nch = MODE == 0 ? 1 : min((L + p.chunk - 1) / p.chunk, (int)gridDim.z), kch = MODE == 0 ? 0 : blockIdx.z;
+  if (kch >= nch || (MODE == 1 && kch == nch - 1)) return;
+  const bool last = kch == nch - 1;
+  const int ta = MODE == 0 ? 0 : kch * p.chunk, tb = last ? L : ta + p.chunk;
+  if (ta >= tb) return;
+  const bool from_state = sl - L > 0 && kch == 0;
+  const int nb = gridDim.x, cb = nb % 8 ? (int)blockIdx.x : (int)(blockIdx.x % 8) * (nb / 8) + (int)(blockIdx.x / 8);
+  const int cw = cb * CH, e = cw / p.dt_div;            // (a workgroup's channels are one head's)
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane % Q, mych = lane / Q, c = cw + mych;
+  const int n0 = 8 * (wave * Q + q);
+  float* hp = p.state + ((long)p.block_table[s * p.bt_stride] * p.Ch + c) * N + n0;
+  const long wc = ((long)s * gridDim.z + kch) * p.Ch + c;
+  const float rate = p.A[e] * LOG2E, dbias = p.delta_bias ? p.delta_bias[e] : 0.f, dv = p.D ? p.D[e] : 0.f;
+  f32x4 h[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+  {
+    const float* from = MODE == 2 && kch > 0 ? p.ws_h + (wc - p.Ch) * N + n0
+                        : MODE == 2 && from_state && nch > 1 ? p.ws_h + (wc + (long)(nch - 1) * p.Ch) * N + n0
+                        : from_state ? hp : nullptr;
+    if (from) { h[0] = reinterpret_cast<const f32x4*>(from)[0]; h[1] = reinterpret_cast<const f32x4*>(from)[1]; }
+  }
+  const long g = (long)(cw / p.group_ch) * N;
+  const T* U = (const T*)p.u + (long)t0 * p.u_stride + cw;
+  const T* Dt = (const T*)p.delta + (long)t0 * p.d_stride + e;
+  const T* Z = p.z ? (const T*)p.z + (long)t0 * p.z_stride + cw : nullptr;
+  const T* B = (const T*)p.B + (long)t0 * p.b_stride + g;
+  const T* C = (const T*)p.C + (long)t0 * p.c_stride + g;
+  T* O = (T*)p.out + (long)t0 * p.o_stride + cw;
+  // staging: pieces of B and C, one value of u and z for each of GR_TT * CH / 256 tokens, a token's step size
+  constexpr int UV = (GR_TT * CH + 255) / 256;
+  v8_t nbc[STEPS];
+  float nu[UV], nz[UV], nd = 0.f;
+  auto fetch = [&](int tt) {                            // (past the end: the last token's again)
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) {
+      const int pi = tid + 256 * i, t = pi / PER, k = pi % PER;
+      const long at = min(tt + min(t, GR_TT - 1), tb - 1);
+      nbc[i] = k < PER / 2 ? *reinterpret_cast<const v8_t*>(B + at * p.b_stride + 8 * k)
+                           : *reinterpret_cast<const v8_t*>(C + at * p.c_stride + 8 * (k - PER / 2));
+    }
+#pragma unroll
+    for (int i = 0; i < UV; ++i) {
+      const int vi = tid + 256 * i, t = min(vi / CH, GR_TT - 1), ch = vi % CH;
+      const long at = min(tt + t, tb - 1);
+      nu[i] = (float)U[at * p.u_stride + ch];
+      nz[i] = MODE != 1 && Z ? (float)Z[at * p.z_stride + ch] : 0.f;
+    }
+    if (tid < GR_TT) nd = (float)Dt[(long)min(tt + tid, tb - 1) * p.d_stride];
+  };
+  fetch(ta);
+  float sdt = 0.f;
+  for (int tt = ta; tt < tb; tt += GR_TT) {
+    if (tid < GR_TT) {
+      float dt = nd + dbias;
+      if (p.softplus) dt = softplus_f(dt);
+      if (tt + tid >= tb) dt = 0.f;                     // no token: the state stays as it is
+      sdt += dt;
+      head_dt[tid][0] = __builtin_amdgcn_exp2f(dt * rate);
+      head_dt[tid][1] = dt;
+    }
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) {
+      const int pi = tid + 256 * i, t = pi / PER, k = pi % PER;
+      if (GR_TT * PER % 256 && t >= GR_TT) break;
+      float* to = &bc[t][0][0] + 8 * k;                 // (B's values, then C's)
+#pragma unroll
+      for (int v = 0; v < 2; ++v) {
+        f32x4 w;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] = tt + t < tb ? (float)nbc[i][4 * v + j] : 0.f;
+        reinterpret_cast<f32x4*>(to)[v] = w;
+      }
+    }
+    float cu[UV], cz[UV];
+#pragma unroll
+    for (int i = 0; i < UV; ++i) { cu[i] = nu[i]; cz[i] = nz[i]; }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < UV; ++i) {
+      const int vi = tid + 256 * i, t = vi / CH, ch = vi % CH;
+      if (GR_TT * CH % 256 && t >= GR_TT) break;
+      const float dt = head_dt[t][1];
+      *reinterpret_cast<f32x2*>(&dd[t][ch][0]) = f32x2{head_dt[t][0], tt + t < tb ? dt * cu[i] : 0.f};
+    }
+    __syncthreads();
+    if (tt + GR_TT < tb) fetch(tt + GR_TT);             // under this tile's arithmetic
+    const int nt = min(GR_TT, tb - tt);
+    for (int tk = 0; tk < nt; tk += 8) {
+      float y[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const f32x2 d = *reinterpret_cast<const f32x2*>(&dd[tk + k][mych][0]);
+        const f32x4* b = reinterpret_cast<const f32x4*>(&bc[tk + k][0][n0]);
+        const f32x4* cc = reinterpret_cast<const f32x4*>(&bc[tk + k][1][n0]);
+        y[k] = 0.f;
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+          const f32x4 bv = b[v], cv = MODE != 1 ? cc[v] : f32x4{0, 0, 0, 0};
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            h[v][j] = fmaf(d[0], h[v][j], d[1] * bv[j]);
+            if (MODE != 1) y[k] = fmaf(cv[j], h[v][j], y[k]);
+          }
+        }
+      }
+      if (MODE != 1) {                                  // lane q of a channel's Q ends with tokens q, q + Q, ...
+        auto meet = [](float keep, float send, auto ctrl) {
+          return keep + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(send), decltype(ctrl)::value, 0xf, 0xf, true));
+        };
+        if constexpr (Q == 8) {
+          const bool b2 = q & 4;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) y[k] = meet(b2 ? y[k + 4] : y[k], b2 ? y[k] : y[k + 4], std::integral_constant<int, 0x141>());
+        }
+        constexpr int K4 = Q == 8 ? 4 : 8;              // values left: of every four, two and one
+        if constexpr (Q >= 4) {
+          const bool b1 = q & 2;
+#pragma unroll
+          for (int j = 0; j < K4; j += 4)
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+              y[j / 2 + k] = meet(b1 ? y[j + k + 2] : y[j + k], b1 ? y[j + k] : y[j + k + 2], std::integral_constant<int, 0x1b>());
+        }
+        constexpr int K2 = Q == 8 ? 2 : Q == 4 ? 4 : 8;
+        if constexpr (Q >= 2) {
+          const bool b0 = q & 1;
+#pragma unroll
+          for (int j = 0; j < K2; j += 2) y[j / 2] = meet(b0 ? y[j + 1] : y[j], b0 ? y[j] : y[j + 1], std::integral_constant<int, 0xb1>());
+        }
+#pragma unroll
+        for (int j = 0; j < 8 / Q; ++j) ys[wave][tk + Q * j + q][mych] = y[j];
+      }
+    }
+    __syncthreads();
+    if (MODE != 1)
+#pragma unroll
+      for (int i = 0; i < UV; ++i) {
+        const int vi = tid + 256 * i, t = vi / CH, ch = vi % CH;
+        if (t >= nt) break;
+        float v = fmaf(dv, cu[i], (ys[0][t][ch] + ys[1][t][ch]) + (ys[2][t][ch] + ys[3][t][ch]));
+        if (Z) v *= silu_f(cz[i]);
+        O[(long)(tt + t) * p.o_stride + ch] = (T)v;
+      }
+  }
+  if (MODE == 1 && wave == 0) {                         // the sum of dt, for every channel of the workgroup
+    sdt = lane < GR_TT ? sdt : 0.f;
+    sdt = group_sum<16>(sdt);
+    sdt = __shfl(sdt, 0, 64);
+    if (lane < CH) p.ws_dt[((long)s * gridDim.z + kch) * p.Ch + cw + lane] = sdt;
+  }
+  if (MODE == 1 || last) {
+    float* to = MODE == 1 ? p.ws_h + wc * N + n0 : hp;
+    reinterpret_cast<f32x4*>(to)[0] = h[0];
+    reinterpret_cast<f32x4*>(to)[1] = h[1];
+  }
+}
+
 // One thread per (sequence, channel, four states): walk the chunks, leaving in chunk k's place its TRUE end state, which is
 // where chunk k + 1 starts.  (The first chunk's is true already.)  The last chunk's place, which has no end state yet, takes
 // the state that the sequence continues from.
@@ -771,7 +949,7 @@ __global__ __launch_bounds__(256) void scan_step_kernel(ScanArgs p) {
 constexpr long SCAN_FEW = 5L << 20;                     // states of a one-token step (20 MB)
 
 // form 1: the sequences have one new token each (none and several are right too); 2: two states a lane (16 of them, a rate each, a step size per
-// channel, 32 channels on a boundary of 32 share B and C); 0: channels in pairs (the caller checks that pairs share B, C and are aligned).  nchunks > 1: ws_dt [S, nchunks, C] and ws_h [S, nchunks, C, N].
+// channel, 32 channels on a boundary of 32 share B and C); 3: eight states a lane (64 of them and more, a rate per head); 0: channels in pairs (the caller checks that pairs share B, C and are aligned).  nchunks > 1: ws_dt [S, nchunks, C] and ws_h [S, nchunks, C, N].
 VDA_EXPORT int vda_selective_scan_pairs(void* out, const void* u, const void* delta, const float* A, const void* Bm,
                                         const void* Cm, const float* D, const void* z, const float* delta_bias,
                                         float* ssm_state, const int* qsl, const int* seq_lens, const int* block_table,
@@ -782,7 +960,10 @@ VDA_EXPORT int vda_selective_scan_pairs(void* out, const void* u, const void* de
   if (S <= 0 || C <= 0) return 0;
   if (N != 16 && N != 32 && N != 64 && N != 128 && N != 256) return -1;
   if (dt_div < 1 || group_ch < 1) return -2;
-  const bool step = form == 1, lanes = form == 2;
+  const bool step = form == 1, lanes = form == 2, groups = form == 3;
+  // (a workgroup's channels: of one head and one group, rows of B and C in pieces of 16 bytes)
+  if (groups && ((N != 64 && N != 128 && N != 256) || !a_scalar || C % (2048 / N) || dt_div % (2048 / N) || group_ch % (2048 / N) || b_stride % 8 ||
+                 c_stride % 8 || dtype == VDA_F32 || (uintptr_t)Bm % 16 || (uintptr_t)Cm % 16)) return -4;
   if (lanes && (N != 16 || a_scalar || dt_div != 1 || (group_ch < C && group_ch % LN_CH))) return -4;
   const int nl = N / 16, wgch = 512 / nl;
   const int span = min((wgch + group_ch - 1) / group_ch + 1, (C + group_ch - 1) / group_ch);
@@ -817,6 +998,23 @@ VDA_EXPORT int vda_selective_scan_pairs(void* out, const void* u, const void* de
       hipLaunchKernelGGL((scan_carry_kernel<AA>), grid_carry, block, 0, st, p, NN, nchunks);                               \
       hipLaunchKernelGGL((scan_pairs_kernel<TT, NN, 2, AA>), grid, block, 0, st, p);                                       \
     } } while (0)
+#define K3(TT, NN) do {                                                                                                    \
+    const dim3 grid_groups(C / (2048 / NN), S, nchunks > 1 ? nchunks : 1);                                                 \
+    if (nchunks <= 1) hipLaunchKernelGGL((scan_groups_kernel<TT, NN, 0>), grid_groups, block, 0, st, p);                  \
+    else {                                                                                                                 \
+      hipLaunchKernelGGL((scan_groups_kernel<TT, NN, 1>), grid_groups, block, 0, st, p);                                   \
+      hipLaunchKernelGGL((scan_carry_kernel<true>), grid_carry, block, 0, st, p, N, nchunks);                              \
+      hipLaunchKernelGGL((scan_groups_kernel<TT, NN, 2>), grid_groups, block, 0, st, p);                                   \
+    } } while (0)
+#define BYG(TT) do { if (N == 64) K3(TT, 64); else if (N == 128) K3(TT, 128); else K3(TT, 256); } while (0)
+  if (groups) {
+    if (dtype == VDA_BF16) BYG(bf16_t);
+    else BYG(f16_t);
+    VDA_CHECK_LAUNCH();
+    return 0;
+  }
+#undef BYG
+#undef K3
 #define BYA(TT, NN) do { if (a_scalar) K(TT, NN, true); else K(TT, NN, false); } while (0)
 #define RUN(TT) do { if (lanes) K2(TT); else if (N == 16) BYA(TT, 16); else if (N == 32) BYA(TT, 32); else if (N == 64) BYA(TT, 64); \
                      else if (N == 128) BYA(TT, 128); else BYA(TT, 256); } while (0)
