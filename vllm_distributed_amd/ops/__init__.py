@@ -1271,7 +1271,7 @@ def moe_tiled_ok(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, gated: bo
             and I % 64 == 0 and w2.shape[1] % 4 == 0 and w13.shape[0] <= 1024)
 
 
-def moe_rows_form(num_pairs: int, num_experts: int, rows: int, weight_bytes: int = 2) -> int:
+def moe_rows_form(num_pairs: int, num_experts: int, rows: int, weight_bytes: int = 2, depth: int = 0) -> int:
     """Grouped expert GEMM, which form (0 K-split, 1 row-split with 64 tokens per pass, 2 with 128): the
     row-split kernel (each wave 16 output rows over the whole K, activations shared through LDS) pays once
     an expert sees enough tokens for the shared tile to matter and the launch still fills the chip; below
@@ -1285,6 +1285,14 @@ def moe_rows_form(num_pairs: int, num_experts: int, rows: int, weight_bytes: int
         return 0
     avg = num_pairs / max(num_experts, 1)
     fills = (rows // 64) * num_experts >= 512
+    # 8-bit weights and at most a pair an expert: those without a pair have no workgroups, and the K-split form leads while the row-split one's 64
+    # rows a workgroup are too few, and past its first full wave where the depth gives the K-split form steps to ask ahead for.  us, K-split / 128-token
+    # row-split, workgroups of 64 rows in brackets: 4096 rows of depth 14336 39 / 128 (128), 71 / 131 (256), 109 / 135 (512); of depth 6400 23 / 61
+    # (128), 69 / 66 (512), 118 / 125 (1024); 14336 rows of depth 4096 64 / 58 (448), 90 / 110 (896), 165 / 176 (1792); 1024 and 1408 rows of depth
+    # 2048 17 / 31 (128), 24 / 31 (176), 40 / 36 (512); 2048 rows of depth 1024 22 / 17 (512)
+    groups = (rows // 64) * num_pairs
+    if weight_bytes == 1 and num_pairs <= num_experts and (groups < 384 or (depth >= 4096 and groups > 448)):
+        return 0
     # measured: with 8-bit weights the 128-token pass is ahead at every size once the launch fills the chip;
     # with 16-bit weights from ~40 tokens per expert; a launch that does not fill the chip (one or two
     # experts on the rank) wants it only when experts would otherwise need several passes
@@ -1330,11 +1338,11 @@ def _moe_grouped_ungated(x, w1, w2, topk_w, topk_ids, activation: str):
     out2 = torch.empty((T * k, H), dtype=x.dtype, device=dev)
     out = torch.empty((T, H), dtype=x.dtype, device=dev)
     N.call("vda_moe_up_act", inter.data_ptr(), x.data_ptr(), w1.data_ptr(), sorted_ids.data_ptr(), offsets.data_ptr(),
-           E, I, H, k, T, x.stride(0), N.dt(x.dtype), int(moe_rows_form(T * k, E, I, w1.element_size())),
+           E, I, H, k, T, x.stride(0), N.dt(x.dtype), int(moe_rows_form(T * k, E, I, w1.element_size(), H)),
            N.ACT[activation], st)
     N.call("vda_moe_down", out2.data_ptr(), inter.data_ptr(), w2.data_ptr(), None, tw.data_ptr(),
            sorted_ids.data_ptr(), offsets.data_ptr(), E, H, I, T, N.dt(x.dtype), N.dt(w2.dtype),
-           int(moe_rows_form(T * k, E, H, w2.element_size())), st)
+           int(moe_rows_form(T * k, E, H, w2.element_size(), I)), st)
     N.call("vda_moe_sum", out.data_ptr(), out2.data_ptr(), ids.data_ptr(), T, H, k, out.stride(0), N.dt(x.dtype), st)
     return out
 
@@ -1422,10 +1430,10 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, topk_w: torc
     max_pairs = T
     N.call("vda_moe_gate_up", inter, x.data_ptr(), w13.data_ptr(), N.ptr(w13_scale), sorted_ids,
            offsets, E, I, H, k, max_pairs, x.stride(0), N.dt(x.dtype), wd,
-           int(moe_rows_form(n, E, I, w13.element_size())), N.ACT[activation], float(act_limit), st)
+           int(moe_rows_form(n, E, I, w13.element_size(), H)), N.ACT[activation], float(act_limit), st)
     N.call("vda_moe_down", out2, inter, w2.data_ptr(), N.ptr(w2_scale), tw.data_ptr(),
            sorted_ids, offsets, E, H, I, max_pairs, N.dt(x.dtype), wd,
-           int(moe_rows_form(n, E, H, w2.element_size())), st)
+           int(moe_rows_form(n, E, H, w2.element_size(), I)), st)
     N.call("vda_moe_sum", out.data_ptr(), out2, ids.data_ptr(), T, H, k, out.stride(0), N.dt(x.dtype), st)
     return out
 

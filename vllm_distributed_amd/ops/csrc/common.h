@@ -108,8 +108,9 @@ template <typename T> struct WLoadFp8 {
   using V8 = typename Vec<T>::v8;
   static constexpr int kElemBytes = 1;
   static __device__ __forceinline__ V8 ld(const void* base, long elem_off) {
-    const u32x2 raw = __builtin_nontemporal_load(
-        reinterpret_cast<const u32x2*>(reinterpret_cast<const uint8_t*>(base) + elem_off));
+    return widen(__builtin_nontemporal_load(reinterpret_cast<const u32x2*>(reinterpret_cast<const uint8_t*>(base) + elem_off)));
+  }
+  static __device__ __forceinline__ V8 widen(u32x2 raw) {
     V8 o;
     const f32x2 a = __builtin_amdgcn_cvt_pk_f32_fp8(raw[0], false), b = __builtin_amdgcn_cvt_pk_f32_fp8(raw[0], true);
     const f32x2 c = __builtin_amdgcn_cvt_pk_f32_fp8(raw[1], false), d = __builtin_amdgcn_cvt_pk_f32_fp8(raw[1], true);
