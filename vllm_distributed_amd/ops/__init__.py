@@ -1288,7 +1288,7 @@ def moe_rows_form(num_pairs: int, num_experts: int, rows: int, weight_bytes: int
     # 8-bit weights and at most a pair an expert: those without a pair have no workgroups, and the K-split form leads while the row-split one's 64
     # rows a workgroup are too few, and past its first full wave where the depth gives the K-split form steps to ask ahead for.  us, K-split / 128-token
     # row-split, workgroups of 64 rows in brackets: 4096 rows of depth 14336 39 / 128 (128), 71 / 131 (256), 109 / 135 (512); of depth 6400 23 / 61
-    # (128), 69 / 66 (512), 118 / 125 (1024); 14336 rows of depth 4096 64 / 58 (448), 90 / 110 (896), 165 / 176 (1792); 1024 and 1408 rows of depth
+    # (128), 69 / 65 (512), 118 / 125 (1024); 14336 rows of depth 4096 65 / 61 (448), 90 / 109 (896), 164 / 164 (1792); 1024 and 1408 rows of depth
     # 2048 17 / 31 (128), 24 / 31 (176), 40 / 36 (512); 2048 rows of depth 1024 22 / 17 (512)
     groups = (rows // 64) * num_pairs
     if weight_bytes == 1 and num_pairs <= num_experts and (groups < 384 or (depth >= 4096 and groups > 448)):

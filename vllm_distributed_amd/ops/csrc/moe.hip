@@ -501,9 +501,14 @@ __global__ __launch_bounds__(256) void moe_grouped_rows_kernel(
       if (i < mt_n) *reinterpret_cast<V8*>(&sx[buf][(tid >> 4) + 16 * i][(piece ^ ((tid >> 4) & 15)) * 8]) = xr[i];
   };
 
-  const int nchunk = K >> 7;
-  loadx(0);
-  loadw(0, wa, wb);
+  // Gate halves: each workgroup starts at another step (see the K-split form: memory channels).  us, all from the first -> so: bf16,
+  // 8 experts of 14336 x 4096, 333 tokens 530 -> 482; 64 of 1024 x 2048, 128 tokens 129 -> 114; e4m3, 16 of 6400 x 4096, 48 tokens
+  // 238 -> 219.  The second product gains nothing, and loses where experts take several passes: they meet in the last-level cache
+  // (333 tokens, 262 -> 307).
+  const int nchunk = K >> 7, turn = GATE_UP ? (int)(blockIdx.x * 5u % (unsigned)nchunk) : 0;
+  auto at = [&](int c) { return c + turn < nchunk ? c + turn : c + turn - nchunk; };
+  loadx(at(0));
+  loadw(at(0), wa, wb);
   storex(0);
   __syncthreads();
   // one K step: request the next step's activations and weights, multiply this step out of LDS buffer
@@ -511,7 +516,7 @@ __global__ __launch_bounds__(256) void moe_grouped_rows_kernel(
   // weight register sets swap roles from step to step (no copies).
   auto step = [&](int c, V8 (&ca)[4], V8 (&cb)[4], V8 (&na)[4], V8 (&nb)[4]) {
     const bool more = c + 1 < nchunk;
-    if (more) { loadx(c + 1); loadw(c + 1, na, nb); }
+    if (more) { loadx(at(c + 1)); loadw(at(c + 1), na, nb); }
     const int buf = c & 1;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
