@@ -150,11 +150,16 @@ __global__ __launch_bounds__(512, 1) void tile_gemm_kernel(const TileGemmArgs a)
     }
     xsrc[j] = xbase + row * a.x_stride * EB + ((slot ^ swz(tau)) << 4);
   }
-  const int nk = (int)(kbytes >> 7);
+  // Experts: each weight panel starts at a K step of its own (the m-tiles that share it, at the same one), since rows are a power of two
+  // apart in most models, and panels all read at the same column fall on few memory channels.  Layers, us, all from the first -> so: bf16, 64
+  // experts of 1024 x 2048, 333 tokens 211 -> 184, 700 247 -> 226; 60 of 1408 x 2048, 700 tokens 265 -> 236; e4m3, 16 of 6400 x 4096, 128
+  // tokens 296 -> 277, 700 350 -> 332.  On the 256-row tiles below, bound by the matrix cores, it gave nothing (3088 / 3096).
+  const int nk = (int)(kbytes >> 7), turn = GROUPED ? (ni * 5 + e * 3) % nk : 0;
+  auto step_at = [&](int kt) { return kt + turn < nk ? kt + turn : kt + turn - nk; };
   auto stage = [&](int kt) {                  // ring slot kt % 3 <- K step min(kt, nk - 1) (a re-fill of the
     uint8_t* lw = lds + (kt % 3) * STAGE + wave * 1024;      // last step keeps the operation count uniform)
     uint8_t* lx = lw + WBYTES;
-    const long ko = (long)min(kt, nk - 1) * 128;
+    const long ko = (long)step_at(min(kt, nk - 1)) * 128;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       glds16(wsrc[j] + ko, lw + j * 8192);
@@ -217,9 +222,9 @@ __global__ __launch_bounds__(512, 1) void tile_gemm_kernel(const TileGemmArgs a)
     float sx[TN], sw[4];
     if (SC == SC_BLOCK) {
 #pragma unroll
-      for (int nt = 0; nt < TN; ++nt) sx[nt] = xs_row[nt][kt];
+      for (int nt = 0; nt < TN; ++nt) sx[nt] = xs_row[nt][step_at(kt)];
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt) sw[mt] = ws_row[mt][kt];
+      for (int mt = 0; mt < 4; ++mt) sw[mt] = ws_row[mt][step_at(kt)];
     }
     const uint8_t* base = lds + (kt % 3) * STAGE;
     i32x4 wa[4][2], xb[TN][2];
