@@ -56,3 +56,31 @@ def test_the_rule(monkeypatch):
     assert form(2, 8, 4096, 1, 14336) == 0 and form(2, 8, 14336, 1, 4096) != 0 and form(4, 8, 14336, 1, 4096) == 0
     assert form(16, 64, 1024, 1, 2048) == 0 and form(32, 64, 1024, 1, 2048) != 0 and form(10, 8, 4096, 1, 14336) != 0
     assert form(2, 8, 4096, 2, 14336) == 0
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,k", [(95, 2), (96, 2), (64, 3), (1023, 1), (700, 3)])
+def test_large_experts_from_tiles(monkeypatch, dt, T, k):
+    """Experts of 192 MiB on both sides of 192 pairs, some of another rank, rows of a wider tensor: as the grouped kernel has it,
+    within rounding; and replayed with other tokens."""
+    x, w13, w2, tw, ids, _, _ = experts(T, 8, k, 4096, 1024, False, dt)
+    x = torch.cat([x, x], 1)[:, :4096]
+    ids[::5, 0] = -1
+
+    def run():
+        return ops.fused_moe(x, w13, w2, tw, ids)
+    g = torch.cuda.CUDAGraph()
+    run()
+    with torch.cuda.graph(g):
+        held = run()
+    for _ in range(3):
+        x.copy_(torch.randn_like(x) * 0.5)
+        g.replay()
+        out = run()
+        monkeypatch.setenv("VDA_MOE_GROUPED_MAX_PAIRS_LARGE", "4096")
+        monkeypatch.setenv("VDA_MOE_GROUPED_MAX_PAIRS", "4096")
+        ref = run()
+        monkeypatch.undo()
+        atol = 6 * torch.finfo(dt).eps * float(ref.float().abs().max())      # (as above)
+        torch.testing.assert_close(out.float(), ref.float(), rtol=0, atol=atol)
+        torch.testing.assert_close(held.float(), ref.float(), rtol=0, atol=atol)
