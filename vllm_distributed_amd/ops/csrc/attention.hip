@@ -591,7 +591,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_kernel(AttnParams p) 
   }
 }
 
-// Prefill form with K/V staged through LDS.  The direct-to-register form above makes every wave of a
+// Prefill form with K/V staged through LDS.  The direct-to-register form above (head groups of more queries than a workgroup has columns here) makes every wave of a
 // workgroup fetch the same keys from L2 (4x the traffic) and is L2-bandwidth bound in prefill; here the
 // 256 threads copy each 32-key K tile and V tile once (fully coalesced 16-byte pieces, fp8 caches are
 // widened on the way in), double-buffered so that the next tile's global loads fly during the MFMAs, and
@@ -1189,8 +1189,8 @@ VDA_EXPORT int vda_prefill_parts(int num_seqs, int num_tokens, int Hq, int Hkv, 
 // Varlen attention of new tokens against the paged cache (the new tokens' own K/V must already be in
 // the cache): causal, or bidirectional within each sequence (encoder models; the shared-prefix pass of
 // cascade attention, where one pseudo-sequence holds every query token of the batch).  lse_out, when
-// given, receives the log-sum-exp of every (head, token) for merging with another pass.  q_tile = 128 / (Hq/Hkv) query tokens
-// per workgroup; the grid over-allocates one tile per sequence.
+// given, receives the log-sum-exp of every (head, token) for merging with another pass.  A workgroup has 128 / (Hq/Hkv) query tokens
+// (64 / where heads hold more than 128 values, 256 / in the wide form); the grid over-allocates one tile per sequence.
 VDA_EXPORT int vda_paged_attention_prefill(
     void* out, const void* q, const void* k_cache, const void* v_cache, const int* block_table,
     const int* seq_lens, const int* q_start_loc, const float* alibi, int num_seqs, int num_tokens,
