@@ -514,6 +514,14 @@ template <typename T> __device__ __forceinline__ void load_few(const T* p, float
     for (int i = 0; i < 4; ++i) v[i] = (float)p[min(i, last)];
   }
 }
+// The first of the four channels that a staging thread reads.  Threads past the last channel (their values are dropped) read the
+// last four again where four are read at once, which begin where theirs would: C is a multiple of four there.
+__host__ __device__ __forceinline__ int lane_channel(int at, int C, int vec) {
+  const int most = C - (vec ? 4 : 1);
+  return at < most ? at : most;
+}
+// (for the test of its bounds, which runs on the host)
+VDA_EXPORT int vda_scan_lane_channel(int at, int C, int vec) { return lane_channel(at, C, vec); }
 // a chunk's MODE, as in the pairs above; vec: rows of four channels may be read and written at once
 template <typename T, int MODE>
 __global__ __launch_bounds__(256) void scan_lanes_kernel(ScanArgs p, int vec) {
@@ -546,7 +554,7 @@ __global__ __launch_bounds__(256) void scan_lanes_kernel(ScanArgs p, int vec) {
   else if (from_state) h = *reinterpret_cast<const f32x2*>(hp);
 
   // staging: this thread's token of a tile, its four channels, and its two states' B and C
-  const int st = threadIdx.x >> 3, sc = 4 * (threadIdx.x & 7), c4 = min(cw + sc, p.Ch - 1), left = p.Ch - 1 - c4;
+  const int st = threadIdx.x >> 3, sc = 4 * (threadIdx.x & 7), c4 = lane_channel(cw + sc, p.Ch, vec), left = p.Ch - 1 - c4;
   const long g = (long)(cw / p.group_ch) * N + 2 * (threadIdx.x & 7);
   const T* U = (const T*)p.u + (long)t0 * p.u_stride + c4;
   const T* Dt = (const T*)p.delta + (long)t0 * p.d_stride + c4;
