@@ -10,15 +10,18 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
-def _noise(seed: int, V: int) -> np.ndarray:
+def _words(seed: int, V: int) -> np.ndarray:
     with np.errstate(over="ignore"):
         x = np.uint64(seed) * np.uint64(0x9E3779B97F4A7C15) + np.arange(V, dtype=np.uint64) + np.uint64(0x632BE59BD9B4E019)
         for mul in (0xff51afd7ed558ccd, 0xc4ceb9fe1a85ec53):
             x ^= x >> np.uint64(33)
             x *= np.uint64(mul)
         x ^= x >> np.uint64(33)
-    r = (x >> np.uint64(16)).astype(np.uint32)
-    return -np.log(-np.log(((r >> np.uint32(8)).astype(np.float64) + 0.5) / 16777216.0))
+    return (x >> np.uint64(16)).astype(np.uint32)
+
+
+def _noise(seed: int, V: int) -> np.ndarray:
+    return -np.log(-np.log(((_words(seed, V) >> np.uint32(8)).astype(np.float64) + 0.5) / 16777216.0))
 
 
 def _scores(row, temp, k, p, mp, seed):
@@ -161,3 +164,22 @@ def test_hash_whose_upper_word_changes_along_a_row():
         for s, seed in enumerate(seeds):
             sure, may = _scores(x[s], 1.0, 0, p, 0.0, seed % 2 ** 64)
             assert may[int(got[s])] >= sure.max() - 2.0 ** -14               # as above
+
+
+@pytest.mark.parametrize("V", [8191, 8192, 50257])                       # one workgroup a row, several
+def test_a_nan_logit_weighs_nothing(V):
+    """It is neither part of the weight that top-p takes a share of nor drawn: the row draws as if it were masked."""
+    g = torch.Generator().manual_seed(V)
+    S = 64
+    x = torch.randn(S, V, generator=g) * 2.0
+    x.scatter_add_(1, torch.randint(0, V, (S, 5), generator=g), torch.rand(S, 5, generator=g) * 10)
+    at = torch.randint(0, V, (S, 1), generator=g)
+    nan, masked = x.scatter(1, at, float("nan")), x.scatter(1, at, -float("inf"))
+    p = 0.2 + 0.6 * torch.rand(S, generator=g)
+    seeds = torch.randint(0, 2 ** 62, (S,), generator=g)
+    args = [None, None, p.to(DEV), None, seeds.to(DEV)]
+    assert torch.equal(ops.sample(nan.to(DEV), *args), ops.sample(masked.to(DEV), *args))
+    args[2] = None
+    assert torch.equal(ops.sample(nan.to(DEV), *args), ops.sample(masked.to(DEV), *args))
+    kept, want = ops.topk_topp_mask(nan.to(DEV), None, p.to(DEV)), ops.topk_topp_mask(masked.to(DEV), None, p.to(DEV))
+    assert torch.equal(torch.where(kept.isnan(), -float("inf"), kept), want)

@@ -123,11 +123,11 @@ __device__ __forceinline__ float opaque(float v) {
 }
 // 1 / temperature
 __device__ __forceinline__ float inverse(float t) { return opaque(__builtin_amdgcn_rcpf(t)); }
-// exp(z - zmax) as a 32.32 fixed-point number
-// (at most 1: a conversion to 32 bits, which saturates, and one more for the largest entry; to 64 bits it is ten instructions)
+// exp(z - zmax) as a 32.32 fixed-point number; 0 of a NaN, of which both comparisons are false
+// (at most 1: a conversion to 32 bits and a case for the largest entry; to 64 bits it is ten instructions)
 __device__ __forceinline__ unsigned long long fixed_weight(float z, float zmax) {
   const float w = __expf(opaque(opaque(z) - zmax)) * 4294967296.f;
-  const uint32_t low = (uint32_t)fminf(w, 4294967040.f);
+  const uint32_t low = w < 4294967296.f ? (uint32_t)w : 0u;
   return w >= 4294967296.f ? 1ull << 32 : (unsigned long long)low;
 }
 
