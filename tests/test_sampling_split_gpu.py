@@ -183,3 +183,17 @@ def test_a_nan_logit_weighs_nothing(V):
     assert torch.equal(ops.sample(nan.to(DEV), *args), ops.sample(masked.to(DEV), *args))
     kept, want = ops.topk_topp_mask(nan.to(DEV), None, p.to(DEV)), ops.topk_topp_mask(masked.to(DEV), None, p.to(DEV))
     assert torch.equal(torch.where(kept.isnan(), -float("inf"), kept), want)
+
+
+@pytest.mark.parametrize("V", [8191, 8192, 50257])
+def test_a_row_of_nothing_but_nan_gives_a_token(V):
+    """Nothing wins such a row; what comes out indexes the next step's embedding all the same."""
+    x = torch.full((4, V), float("nan"), device=DEV)
+    x[3, 5:] = -float("inf")
+    t = torch.tensor([0.0, 1.0, 0.7, 1.0], device=DEV)
+    for k, p in ((None, None), (torch.tensor([0, 5, 0, 5], dtype=torch.int32, device=DEV), torch.tensor([1.0, 1.0, 0.5, 0.5], device=DEV))):
+        got = ops.sample(x, t, k, p)
+        assert bool(((got >= 0) & (got < V)).all()), got
+    for dt in (torch.float32, torch.bfloat16, torch.float16):
+        got = ops.argmax(x[:3].to(dt))
+        assert bool(((got >= 0) & (got < V)).all()), got

@@ -45,6 +45,9 @@ __device__ __forceinline__ ArgMax block_argmax(ArgMax a, float* rv, int* ri) {
   return t;
 }
 
+// the token of a row's winner; of a row in which nothing wins (all NaN) the first one, which indexes the next embedding safely
+__device__ __forceinline__ long winner(ArgMax a) { return a.i == 0x7fffffff ? 0 : a.i; }
+
 template <typename T>
 __global__ __launch_bounds__(1024) void argmax_kernel(const T* __restrict__ logits, long* __restrict__ out, int V,
                                                       long stride) {
@@ -68,7 +71,7 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const T* __restrict__ logi
   }
   for (int i = i0 + threadIdx.x; i < V; i += 1024) a = amax2(a, ArgMax{(float)row[i], i});
   a = block_argmax(a, rv, ri);
-  if (threadIdx.x == 0) out[blockIdx.x] = a.i;
+  if (threadIdx.x == 0) out[blockIdx.x] = winner(a);
 }
 
 // The histogram bin (256 of them, the highest keys in bin 255) in which the running sum from the top reaches
@@ -222,7 +225,7 @@ __device__ void sample_row(const SampleArgs& p, int rowi, float zmax_known, bool
     ArgMax a{-INFINITY, 0x7fffffff};
     for (int i = threadIdx.x; i < V; i += 1024) a = amax2(a, ArgMax{row[i], i});
     a = block_argmax(a, rv, ri);
-    if (threadIdx.x == 0) p.out[rowi] = a.i;
+    if (threadIdx.x == 0) p.out[rowi] = winner(a);
     return;
   }
   const float inv_t = inverse(temp);
@@ -250,7 +253,7 @@ __device__ void sample_row(const SampleArgs& p, int rowi, float zmax_known, bool
     if (fkey(z) >= thr) a = amax2(a, ArgMax{noisy(z, seed, i), i});
   }
   a = block_argmax(a, rv, ri);
-  if (threadIdx.x == 0) p.out[rowi] = a.i;
+  if (threadIdx.x == 0) p.out[rowi] = winner(a);
 }
 
 __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs p) {
@@ -725,7 +728,7 @@ __global__ __launch_bounds__(1024) void split_finish_kernel(SampleArgs p, SplitR
     }
   }
   a = block_argmax(a, rv, ri);
-  if (threadIdx.x == 0) p.out[rowi] = a.i;
+  if (threadIdx.x == 0) p.out[rowi] = winner(a);
 }
 
 // In place: logits masked below the same thresholds the sampler would use (-inf),
