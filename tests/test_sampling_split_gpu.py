@@ -197,3 +197,18 @@ def test_a_row_of_nothing_but_nan_gives_a_token(V):
     for dt in (torch.float32, torch.bfloat16, torch.float16):
         got = ops.argmax(x[:3].to(dt))
         assert bool(((got >= 0) & (got < V)).all()), got
+
+
+# (length, seed, token) whose hash is the largest word: the noise of a u that rounds to 1 would be infinite
+@pytest.mark.parametrize("V,seed,token", [(8191, 764, 290), (8191, 2558, 5888), (128256, 137, 125767), (128256, 236, 25723)])
+@pytest.mark.parametrize("k", [0, 201])
+def test_the_largest_word_is_finite_noise(V, seed, token, k):
+    assert _words(seed, V)[token] >> np.uint32(8) == 0xffffff
+    g = torch.Generator().manual_seed(seed)
+    x = torch.full((1, V), -100.0)
+    high = torch.randperm(V, generator=g)[:201]
+    x[0, high[high != token][:200]] = torch.randn(200, generator=g)
+    x[0, token] = -40.0                        # finite noise is at most log(2^24) = 16.7 there and at least -log(log(2^25)) = -2.9 elsewhere
+    got = ops.sample(x.to(DEV), None, torch.tensor([k], dtype=torch.int32, device=DEV) if k else None, None, None,
+                     torch.tensor([seed], device=DEV))
+    assert int(got) != token and float(x[0, int(got)]) > -10.0

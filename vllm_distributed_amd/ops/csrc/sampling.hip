@@ -169,9 +169,10 @@ __device__ uint32_t radix_threshold(At at, int n, float zmax, float target, unsi
 }
 
 // z_i + Gumbel noise: the noise is a function of the row's seed and the token alone.  (The logarithms' arguments are at least
-// 2^-25 or zero, so the bare instruction does.)
+// 2^-25, so the bare instruction does.)  The largest word's u rounds to 1, whose noise would be infinite and win whatever the
+// logit: one draw in 131 over 128256 tokens was such a token.  It takes the number below 1.
 __device__ __forceinline__ float gumbel(float z, uint32_t rnd) {
-  const float u = ((float)(rnd >> 8) + 0.5f) * (1.f / 16777216.f);     // (0, 1]
+  const float u = fminf(((float)(rnd >> 8) + 0.5f) * (1.f / 16777216.f), 0x1.fffffep-1f);     // (0, 1)
   const float e = -(__builtin_amdgcn_logf(u) * 0.6931471805599453f);
   return opaque(z) - opaque(__builtin_amdgcn_logf(e) * 0.6931471805599453f);
 }
