@@ -110,3 +110,21 @@ def test_heads_that_are_no_power_of_two_or_wide(D, Hq, Hkv, kw):
         want, want_lse = R.paged_attention(q.float(), kc.float(), vc.float(), table, sl, starts, D ** -0.5, return_lse=True, **kw)
         assert float((out.float() - want).abs().max()) <= (2 * 2.0 ** -12 + 1e-5) * float(vc.float().abs().max())
         torch.testing.assert_close(lse, want_lse.float(), atol=1e-4, rtol=1e-5)
+
+
+@pytest.mark.parametrize("D,Hq,Hkv", [(64, 8, 2), (128, 8, 1), (192, 4, 2), (256, 80, 1)])      # (the last: heads past a workgroup's columns)
+@pytest.mark.parametrize("where", ["query", "key", "last key"])
+def test_nan_comes_out_of_parts(D, Hq, Hkv, where):
+    """A row that is NaN in one part (see test_options_in_parts) is NaN where its keys are cut."""
+    b = _batch([20, 70], [1000, 1300], Hq, Hkv, D, 16, torch.bfloat16)
+    q, kc, vc, table, sl, starts = b
+    assert _parts(b, Hq) > 1
+    if where == "query":
+        q[3, 1], q[50, 0] = float("nan"), float("nan")
+    else:
+        at = 600 if where == "key" else 1369                       # of the second sequence; the last one is the last row's alone
+        kc[int(table[1, at // 16]), Hkv - 1, at % 16, 5] = float("nan")
+    one, parts = torch.empty_like(q), torch.empty_like(q)
+    ops.paged_attention_prefill(one, q, kc, vc, table, sl, starts, D ** -0.5, return_lse=True)
+    ops.paged_attention_prefill(parts, q, kc, vc, table, sl, starts, D ** -0.5)
+    assert bool(one.isnan().any()) and torch.equal(one.isnan(), parts.isnan())

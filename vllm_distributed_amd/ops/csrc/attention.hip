@@ -57,12 +57,12 @@ template <int D>
 __device__ __forceinline__ void store_part(const AttnParams& p, int part, long tok, int head, int g, const f32x4 (&acc)[D / 16],
                                            float inv, float m, float l) {
   const long at = (tok * p.Hq + head) * p.nsplit + part;
-  if (l > 0.f) {                                          // (a part without keys is left out by its weight)
+  if (l != 0.f) {                                         // (a part without keys is left out by its weight; one that is NaN is not)
     float* po = p.part_out + at * D + 4 * g;
 #pragma unroll
     for (int n = 0; n < D / 16; ++n) *reinterpret_cast<f32x4*>(po + 16 * n) = acc[n] * inv;
   }
-  if (g == 0) p.part_lse[at] = l > 0.f ? m + log2f(l) : -INFINITY;
+  if (g == 0) p.part_lse[at] = l != 0.f ? m + log2f(l) : -INFINITY;
 }
 
 template <typename T, int D, int BS, int NCT, bool F8>
