@@ -38,6 +38,7 @@ class AttentionMetadata:
     prefill_query_start_loc: Optional[torch.Tensor] = None
     max_query_len: int = 1
     max_seq_len: int = 0
+    max_prefill_seq_len: int = 0        # of the prefill / chunked-prefill sequences alone
     max_decode_query_len: int = 1
     decode_num_splits: int = 1
     decode_workspace: Optional[tuple] = None

@@ -134,7 +134,7 @@ class Attention(nn.Module):
                                         md.seq_lens[nd:nd + n_pre], md.prefill_query_start_loc, self.scale,
                                         window=self.sliding_window, softcap=self.softcap, alibi=self.alibi_slopes,
                                         k_scale=ksc, v_scale=vsc, causal=self.causal, max_q_len=md.max_query_len,
-                                        max_kv_len=md.max_seq_len)
+                                        max_kv_len=md.max_prefill_seq_len)
         if n < T:
             out[n:].zero_()
         return out.view(T, Hq * D)
@@ -215,7 +215,7 @@ class Attention(nn.Module):
                                             sl[nd:nd + n_pre], pqsl, self.scale,
                                             window=self.sliding_window, softcap=self.softcap, alibi=self.alibi_slopes,
                                             k_scale=ksc, v_scale=vsc, causal=self.causal,
-                                            max_q_len=md.max_query_len, max_kv_len=md.max_seq_len)
+                                            max_q_len=md.max_query_len, max_kv_len=md.max_prefill_seq_len)
         if conn is not None:
             conn.save_kv_layer(self.layer_name, (self.k_cache, self.v_cache), md)
         return out.view(T, qs)
@@ -403,7 +403,7 @@ class DualChunkAttention(Attention):
                 ops.paged_attention_prefill(out[ndt:e], q[ndt:e], self.k_cache, self.v_cache,
                                             md.local_block_table[nd:nd + n_pre], md.local_seq_lens[nd:nd + n_pre],
                                             md.local_prefill_query_start_loc, self.scale, softcap=self.softcap,
-                                            k_scale=ksc, v_scale=vsc, causal=True)
+                                            k_scale=ksc, v_scale=vsc, causal=True, max_kv_len=md.max_prefill_seq_len)
         elif md.dca_passes != 1:
             ops.rotary_embedding((p_in + L).clamp_(max=self.chunk_size), q_succ, None, table, rd, D, neox)
             ops.rotary_embedding(torch.full_like(p_in, min(2 * L - 1, self.chunk_size)), q_inter, None, table, rd, D,

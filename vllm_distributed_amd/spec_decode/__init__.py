@@ -175,7 +175,7 @@ class EagleProposer:
         if not decode:
             runner._to_dev(runner.prefill_qsl, cu)
         nsplit = runner._decode_splits(nd, max_seq, False)
-        md = runner._build_attn_metadata(S, T, nd, ndt, max_seq, int(n_q.max()), nsplit)
+        md = runner._build_attn_metadata(S, T, nd, ndt, max_seq, int(n_q.max()), nsplit, 0 if decode else max_seq)
         with set_forward_context(md, num_tokens=0):
             return self.model(runner.input_ids[:T], runner.positions[:T], hidden)
 

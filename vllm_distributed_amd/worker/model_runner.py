@@ -680,7 +680,8 @@ class ModelRunner:
             if self.uses_mrope:
                 pos = self._mrope_positions(req_ids, rows, n_sched, cu, pos)
             nd, ndt = self._upload_attention_inputs(rows, n_sched, cu, pos, slot, seq_lens)
-            att = (S, T, nd, ndt, int(seq_lens.max()) if S else 0, int(n_sched.max()) if S else 0)
+            att = (S, T, nd, ndt, int(seq_lens.max()) if S else 0, int(n_sched.max()) if S else 0,
+                   int(seq_lens[nd:].max()) if nd < S else 0)
         logits_idx = (cu[1:] - 1).astype(np.int64)
         return req_ids, rows, n_sched, cu, S, T, logits_idx, att, tmd
 
@@ -753,7 +754,8 @@ class ModelRunner:
         perm_t = inv_t = None
         if is_root:
             self._to_dev(self.input_ids, ib.token_ids[tok_rows, pos])
-        att = (S_l, T_l, nd, ndt, int(seq_l.max()) if S_l else 0, int(n_l.max()) if S_l else 0)
+        att = (S_l, T_l, nd, ndt, int(seq_l.max()) if S_l else 0, int(n_l.max()) if S_l else 0,
+               int(seq_l[nd:].max()) if nd < S_l else 0)
         if self.tk_rx is not None:
             # peer-memory form: index lists and counts go into the persistent device buffers
             gbs = self._tknp_graph_bs(len(req_ids), n_sched)
@@ -857,7 +859,7 @@ class ModelRunner:
             self._ws = ws = (po, pl, need)
         return ws[0], ws[1]
 
-    def _build_attn_metadata(self, S, T, nd, ndt, max_seq, max_q, nsplit, decode_only=False) -> AttentionMetadata:
+    def _build_attn_metadata(self, S, T, nd, ndt, max_seq, max_q, nsplit, max_pre=0, decode_only=False) -> AttentionMetadata:
         local = {}
         if self.local_chunk:
             # decode_only (captured graphs, warm-up): the virtual sequences are the S sequences themselves
@@ -876,7 +878,7 @@ class ModelRunner:
             num_prefill_tokens=T - ndt, slot_mapping=self.slot_mapping, block_table=self.block_table[:S],
             seq_lens=self.seq_lens[:S], query_start_loc=self.query_start_loc[:S + 1],
             prefill_query_start_loc=self.prefill_qsl[:S - nd + 1] if nd < S else None,
-            max_query_len=max_q, max_seq_len=max_seq, max_decode_query_len=self.max_decode_q,
+            max_query_len=max_q, max_seq_len=max_seq, max_prefill_seq_len=max_pre, max_decode_query_len=self.max_decode_q,
             decode_num_splits=nsplit, decode_workspace=self._workspace(max(ndt, 1), nsplit),
             state_table=self.state_table[:S] if self.state_table is not None else None)
 
@@ -947,6 +949,7 @@ class ModelRunner:
                 slot_mapping=self.slot_mapping[t0:], block_table=self.block_table[a:b], seq_lens=self.seq_lens[a:b],
                 query_start_loc=qsl, prefill_query_start_loc=pqsl if nd_u < b - a else None,
                 max_query_len=int(n_sched[a:b].max()), max_seq_len=max_seq,
+                max_prefill_seq_len=int(seq_lens[a + nd_u:b].max()) if a + nd_u < b else 0,
                 max_decode_query_len=self.max_decode_q, decode_num_splits=nsplit,
                 decode_workspace=self._workspace(max(ndt_u, 1), nsplit))
             out.append(MicroBatch(t0, t1, md))
@@ -977,7 +980,7 @@ class ModelRunner:
                 mm_e, mm_mask = self._gather_mm_embeddings(req_ids, rows, n_sched, cu)
                 if mm_e is not None:
                     inputs_embeds = self.model.get_input_embeddings(self.input_ids[:T], mm_e, mm_mask)
-        S_a, T_a, nd, ndt, max_seq, max_q = att        # what THIS rank attends for (== the batch without TKNP)
+        S_a, T_a, nd, ndt, max_seq, max_q, max_pre = att        # what THIS rank attends for (== the batch without TKNP)
         ib = self.input_batch
         pure_decode = nd == S and max_q == 1
         pp = get_pp_group()
@@ -1026,7 +1029,7 @@ class ModelRunner:
             hidden = hidden_buf
         else:
             nsplit = self._decode_splits(nd, max_seq, False)
-            md = self._build_attn_metadata(S_a, T_a, nd, ndt, max_seq, max_q, nsplit)
+            md = self._build_attn_metadata(S_a, T_a, nd, ndt, max_seq, max_q, nsplit, max_pre)
             P = self._cascade_prefix_len(so, rows, n_sched, S) if tmd is None else 0
             if P:
                 self._to_dev(self.cascade_seq_len, np.array([P], dtype=np.int32))
