@@ -1,8 +1,9 @@
 """Which 16-bit expert layers take 256-row tiles (ops._moe_wide_pays): where single experts past a tile's rows open another round over
 the CUs, they do not.  Layers by experts, hidden and intermediate width, and rows an expert; times in the rule's comment."""
 import pytest
+import torch
 
-from vllm_distributed_amd import ops
+from vllm_distributed_amd import envs, ops
 
 
 @pytest.mark.parametrize("E,H,I,rows,pays", [(64, 2048, 1024, 219, True), (64, 2048, 1024, 225, False), (64, 2048, 1024, 231, False),
@@ -11,3 +12,17 @@ from vllm_distributed_amd import ops
                                              (8, 4096, 14336, 200, False), (8, 1024, 512, 360, False)])
 def test_rounds_opened_by_few_experts_count(E, H, I, rows, pays):
     assert ops._moe_wide_pays(E * rows, E, -(-I // 128), H, -(-H // 256), I) is pays
+
+
+@pytest.mark.parametrize("pairs,large,limit", [(None, None, 191), ("4096", None, 4096), ("64", None, 64), (None, "500", 500),
+                                               ("4096", "500", 500), ("300", "500", 300)])
+def test_a_limit_that_is_set_holds_for_large_experts(monkeypatch, pairs, large, limit):
+    for name, value in (("VDA_MOE_GROUPED_MAX_PAIRS", pairs), ("VDA_MOE_GROUPED_MAX_PAIRS_LARGE", large)):
+        monkeypatch.delenv(name, raising=False)
+        if value is not None:
+            monkeypatch.setenv(name, value)
+        assert envs.is_set(name) == (value is not None)
+    x, w13, w2 = (torch.empty(s, dtype=torch.bfloat16, device="meta") for s in ((1, 4096), (8, 28672, 4096), (8, 4096, 14336)))
+    assert ops.moe_grouped_limit(x, w13, w2) == limit
+    small = [torch.empty(s, dtype=torch.bfloat16, device="meta") for s in ((8, 1024, 1024), (8, 1024, 512))]
+    assert ops.moe_grouped_limit(x, *small) == int(pairs or 2048)

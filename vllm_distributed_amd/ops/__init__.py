@@ -1351,6 +1351,23 @@ def _moe_grouped_ungated(x, w1, w2, topk_w, topk_ids, activation: str):
 MOE_ACTIVATIONS = ("silu", "gelu", "gelu_tanh", "gelu_pytorch_tanh", "relu", "relu2", "clamped_swiglu")
 
 
+def moe_grouped_limit(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor) -> int:
+    """Up to how many (token, slot) pairs ``fused_moe`` takes the grouped kernels; matrix tiles beyond."""
+    limit = envs.VDA_MOE_GROUPED_MAX_PAIRS
+    if w13.dtype == torch.float8_e4m3fn:
+        return min(limit, envs.VDA_MOE_GROUPED_MAX_PAIRS_FP8)
+    # 16-bit experts of 192 MiB and more: 64-row tiles stream them as fast and read an expert's weights once, where the grouped kernel's
+    # passes of 64 or 128 tokens read them again.  Layers, us, grouped / tiles at 96, 192, 512 and 1024 pairs: 8 experts of 4096 x 14336
+    # 541 / 532, 572 / 543, 687 / 632, 1090 / 735; 64 of 2048 x 1024 159 / 148, 176 / 164, 170 / 167, 182 / 170; 60 of 2048 x 1408 181 / 189,
+    # 215 / 204, 229 / 210, 246 / 215; 8 of 4096 x 1792 95 / 100, 115 / 105, 143 / 112, 228 / 135.  Smaller experts are bound by the launches,
+    # of which tiles have more: 32 of 1024 x 512 (96 MiB) 42 / 64, 43 / 64, 46 / 64, 54 / 64.
+    # A limit that is set and this one left alone: the one that is set holds for them too.
+    if (w13.numel() + w2.numel()) * w13.element_size() >= 192 << 20 and moe_tiled_ok(x, w13, w2) \
+            and (envs.is_set("VDA_MOE_GROUPED_MAX_PAIRS_LARGE") or not envs.is_set("VDA_MOE_GROUPED_MAX_PAIRS")):
+        limit = min(limit, envs.VDA_MOE_GROUPED_MAX_PAIRS_LARGE)
+    return limit
+
+
 def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, topk_w: torch.Tensor, topk_ids: torch.Tensor,
               w13_scale: Optional[torch.Tensor] = None, w2_scale: Optional[torch.Tensor] = None,
               block_scales: bool = False, activation: str = "silu", x_scale: Optional[torch.Tensor] = None,
@@ -1407,16 +1424,7 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, topk_w: torc
     I = I2 // 2
     # e4m3 experts: from a few hundred pairs on, quantised activations through the fp8 MFMA tiles beat
     # widening the weights for 16-bit MFMAs (Mixtral-8x7B layer, 256 pairs: 396 us against 420; 2048: 684 / 1367)
-    limit = envs.VDA_MOE_GROUPED_MAX_PAIRS
-    if w13.dtype == torch.float8_e4m3fn:
-        limit = min(limit, envs.VDA_MOE_GROUPED_MAX_PAIRS_FP8)
-    # 16-bit experts of 192 MiB and more: 64-row tiles stream them as fast and read an expert's weights once, where the grouped kernel's
-    # passes of 64 or 128 tokens read them again.  Layers, us, grouped / tiles at 96, 192, 512 and 1024 pairs: 8 experts of 4096 x 14336
-    # 541 / 532, 572 / 543, 687 / 632, 1090 / 735; 64 of 2048 x 1024 159 / 148, 176 / 164, 170 / 167, 182 / 170; 60 of 2048 x 1408 181 / 189,
-    # 215 / 204, 229 / 210, 246 / 215; 8 of 4096 x 1792 95 / 100, 115 / 105, 143 / 112, 228 / 135.  Smaller experts are bound by the launches,
-    # of which tiles have more: 32 of 1024 x 512 (96 MiB) 42 / 64, 43 / 64, 46 / 64, 54 / 64
-    elif (w13.numel() + w2.numel()) * w13.element_size() >= 192 << 20 and moe_tiled_ok(x, w13, w2):
-        limit = min(limit, envs.VDA_MOE_GROUPED_MAX_PAIRS_LARGE)
+    limit = moe_grouped_limit(x, w13, w2)
     if T * k > limit or block_scales:
         return _moe_tiled(_contig_last(x), w13, w2, topk_w, topk_ids, w13_scale, w2_scale, block_scales, activation,
                           act_limit=act_limit)
