@@ -61,9 +61,10 @@ def test_the_rule(monkeypatch):
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("T,k", [(95, 2), (96, 2), (64, 3), (1023, 1), (700, 3)])
 def test_large_experts_from_tiles(monkeypatch, dt, T, k):
-    """Experts of 192 MiB on both sides of 192 pairs, some of another rank, rows of a wider tensor: as the grouped kernel has it,
+    """Experts of 264 MiB on both sides of 192 pairs, some of another rank, rows of a wider tensor: as the grouped kernel has it,
     within rounding; and replayed with other tokens."""
-    x, w13, w2, tw, ids, _, _ = experts(T, 8, k, 4096, 1024, False, dt)
+    x, w13, w2, tw, ids, _, _ = experts(T, 8, k, 4096, 1408, False, dt)
+    assert ops.moe_grouped_limit(x, w13, w2) == 191
     x = torch.cat([x, x], 1)[:, :4096]
     ids[::5, 0] = -1
 

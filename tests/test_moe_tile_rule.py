@@ -26,3 +26,13 @@ def test_a_limit_that_is_set_holds_for_large_experts(monkeypatch, pairs, large, 
     assert ops.moe_grouped_limit(x, w13, w2) == limit
     small = [torch.empty(s, dtype=torch.bfloat16, device="meta") for s in ((8, 1024, 1024), (8, 1024, 512))]
     assert ops.moe_grouped_limit(x, *small) == int(pairs or 2048)
+
+
+@pytest.mark.parametrize("E,H,I,limit", [(8, 4096, 1408, 191), (8, 4096, 1280, 383), (8, 4096, 1024, 383), (7, 4096, 1024, 2048), (16, 2048, 1024, 383),
+                                         (64, 1536, 512, 191), (32, 1024, 1408, 2048), (8, 1024, 5632, 2048), (64, 1024, 1024, 191)])
+def test_which_experts_are_large(monkeypatch, E, H, I, limit):
+    """Where tiles lead, by the measurements beside the rule: at either side of its lines in bytes and in width."""
+    for name in ("VDA_MOE_GROUPED_MAX_PAIRS", "VDA_MOE_GROUPED_MAX_PAIRS_LARGE"):
+        monkeypatch.delenv(name, raising=False)
+    x, w13, w2 = (torch.empty(s, dtype=torch.bfloat16, device="meta") for s in ((1, H), (E, 2 * I, H), (E, H, I)))
+    assert ops.moe_grouped_limit(x, w13, w2) == limit

@@ -1356,15 +1356,21 @@ def moe_grouped_limit(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor) -> i
     limit = envs.VDA_MOE_GROUPED_MAX_PAIRS
     if w13.dtype == torch.float8_e4m3fn:
         return min(limit, envs.VDA_MOE_GROUPED_MAX_PAIRS_FP8)
-    # 16-bit experts of 192 MiB and more: 64-row tiles stream them as fast and read an expert's weights once, where the grouped kernel's
-    # passes of 64 or 128 tokens read them again.  Layers, us, grouped / tiles at 96, 192, 512 and 1024 pairs: 8 experts of 4096 x 14336
-    # 541 / 532, 572 / 543, 687 / 632, 1090 / 735; 64 of 2048 x 1024 159 / 148, 176 / 164, 170 / 167, 182 / 170; 60 of 2048 x 1408 181 / 189,
-    # 215 / 204, 229 / 210, 246 / 215; 8 of 4096 x 1792 95 / 100, 115 / 105, 143 / 112, 228 / 135.  Smaller experts are bound by the launches,
-    # of which tiles have more: 32 of 1024 x 512 (96 MiB) 42 / 64, 43 / 64, 46 / 64, 54 / 64.
+    # Large 16-bit experts: 64-row tiles stream them as fast and read an expert's weights once, where the grouped kernel's passes of 64 or
+    # 128 tokens read them again.  Layers, us, grouped / tiles at 192, 512 and 1024 pairs: 8 experts of 4096 x 14336 572 / 543, 687 / 632,
+    # 1090 / 735; 64 of 2048 x 1024 176 / 164, 170 / 167, 182 / 170; 60 of 2048 x 1408 215 / 204, 229 / 210, 246 / 215; 264 MiB, 8 of
+    # 4096 x 1408 92 / 92, 131 / 98, 208 / 118, 16 of 2048 x 1408 77 / 75, 96 / 75, 118 / 80.  Smaller ones are bound by the launches, of
+    # which tiles have more, and by tiles too few to fill the chip: of 192 MiB, at 192, 384 and 1024 pairs, 8 of 4096 x 1024 68 / 82,
+    # 84 / 85, 142 / 106, 16 of 2048 x 1024 55 / 59, 70 / 61, 84 / 66; 32 of 1024 x 512 (96 MiB) 43 / 64, 46 / 64, 54 / 64.  Narrow
+    # models' second product has the fewest tiles: 8 of 1024 x 5632 (264 MiB) 91 / 124, 128 / 130, 167 / 181, 32 of 1024 x 1408 (264 MiB)
+    # 76 / 80, 70 / 78, 80 / 83; 64 of 1024 x 1024 (384 MiB) 99 / 93, 104 / 95, 106 / 101; 64 of 1536 x 512 (288 MiB) 81 / 75, 86 / 76, 85 / 80.
     # A limit that is set and this one left alone: the one that is set holds for them too.
-    if (w13.numel() + w2.numel()) * w13.element_size() >= 192 << 20 and moe_tiled_ok(x, w13, w2) \
-            and (envs.is_set("VDA_MOE_GROUPED_MAX_PAIRS_LARGE") or not envs.is_set("VDA_MOE_GROUPED_MAX_PAIRS")):
-        limit = min(limit, envs.VDA_MOE_GROUPED_MAX_PAIRS_LARGE)
+    mib = (w13.numel() + w2.numel()) * w13.element_size() >> 20
+    if mib >= (192 if w13.shape[2] >= 1536 else 384) and moe_tiled_ok(x, w13, w2):
+        if envs.is_set("VDA_MOE_GROUPED_MAX_PAIRS_LARGE"):
+            limit = min(limit, envs.VDA_MOE_GROUPED_MAX_PAIRS_LARGE)
+        elif not envs.is_set("VDA_MOE_GROUPED_MAX_PAIRS"):
+            limit = envs.VDA_MOE_GROUPED_MAX_PAIRS_LARGE if mib >= 256 else 383
     return limit
 
 
