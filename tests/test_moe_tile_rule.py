@@ -36,3 +36,12 @@ def test_which_experts_are_large(monkeypatch, E, H, I, limit):
         monkeypatch.delenv(name, raising=False)
     x, w13, w2 = (torch.empty(s, dtype=torch.bfloat16, device="meta") for s in ((1, H), (E, 2 * I, H), (E, H, I)))
     assert ops.moe_grouped_limit(x, w13, w2) == limit
+
+
+@pytest.mark.parametrize("pairs,E,rows,depth,split", [(6, 8, 4096, 14336, True), (4, 8, 7168, 4096, True), (8, 32, 4096, 4096, False), (9, 32, 4096, 4096, True),
+                                                      (8, 16, 4096, 6400, True), (32, 128, 768, 2048, True), (12, 60, 2048, 1408, False),
+                                                      (8, 60, 2048, 1408, True), (2, 8, 14336, 4096, False), (8, 256, 2048, 7168, True)])
+def test_few_pairs_of_8_bit_experts(monkeypatch, pairs, E, rows, depth, split):
+    """The K-split form where the workgroups of the experts that are chosen are too few for the other, or more than its first wave."""
+    monkeypatch.delenv("VDA_MOE_ROWS_FORM", raising=False)
+    assert (ops.moe_rows_form(pairs, E, rows, 1, depth) == 0) is split

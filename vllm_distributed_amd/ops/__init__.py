@@ -1286,13 +1286,16 @@ def moe_rows_form(num_pairs: int, num_experts: int, rows: int, weight_bytes: int
         return 0
     avg = num_pairs / max(num_experts, 1)
     fills = (rows // 64) * num_experts >= 512
-    # 8-bit weights and at most a pair an expert: those without a pair have no workgroups, and the K-split form leads while the row-split one's 64
-    # rows a workgroup are too few, and past its first full wave where the depth gives the K-split form steps to ask ahead for.  us, K-split / 128-token
-    # row-split, workgroups of 64 rows in brackets: 4096 rows of depth 14336 39 / 128 (128), 71 / 131 (256), 109 / 135 (512); of depth 6400 23 / 61
-    # (128), 69 / 65 (512), 118 / 125 (1024); 14336 rows of depth 4096 65 / 61 (448), 90 / 109 (896), 164 / 164 (1792); 1024 and 1408 rows of depth
-    # 2048 17 / 31 (128), 24 / 31 (176), 40 / 36 (512); 2048 rows of depth 1024 22 / 17 (512)
-    groups = (rows // 64) * num_pairs
-    if weight_bytes == 1 and num_pairs <= num_experts and (groups < 384 or (depth >= 4096 and groups > 448)):
+    # 8-bit weights and at most a pair an expert: only experts with a pair have workgroups, so many on average of 64 rows each.  The K-split form
+    # leads while these are too few for the row-split one, and again past its first full wave of 512 where the depth gives the K-split
+    # form steps to ask ahead for; random choices fall on either side of an average near it.  us, K-split / 128-token row-split,
+    # workgroups in brackets: depth 14336 39 / 127 (120), 107 / 133 (336), 141 / 136 (512, each expert another); of 6400 50 / 61 (329),
+    # 57 / 62 (413), 80 / 98 (552); of 4096 32 / 41 (329), 58 / 59 (413), 64 / 61 (420), 63 / 59 (448), 69 / 60 (512, each another), 67 / 81
+    # (494), 99 / 105 (742); of 2048 32 / 34 (341), 36 / 34 (405), 46 / 54 (543), 66 / 62 (813); of 1408 14 / 16 (242), 19 / 17 (351); of
+    # 1024 20 / 14 (456)
+    groups = (rows // 64) * num_experts * (1.0 - (1.0 - 1.0 / max(num_experts, 1)) ** num_pairs)
+    if weight_bytes == 1 and num_pairs <= num_experts and (
+            groups < (416 if depth >= 4096 else 400 if depth >= 2048 else 300) or (depth >= 4096 and groups > 464)):
         return 0
     # measured: with 8-bit weights the 128-token pass is ahead at every size once the launch fills the chip;
     # with 16-bit weights from ~40 tokens per expert; a launch that does not fill the chip (one or two
