@@ -97,7 +97,8 @@ def test_merge_of_parts(D, nsplit):
 def test_two_parts(D, Hq, Hkv, S, fp8):
     if fp8 and D not in (64, 128):
         pytest.skip("e4m3 caches: head sizes 64 and 128")
-    lens = ((EDGES + [0, 1025]) * 2)[:S]
-    _check(lens, [1] * S, Hq, Hkv, D, 16, torch.bfloat16, fp8, 2)
-    if Hq // Hkv <= 4:
-        _check([max(n, 4) for n in lens], [1 + i % 4 for i in range(S)], Hq, Hkv, D, 16, torch.float16, fp8, 2, window=300)
+    for longest in (768, 1025):                                     # (eight waves up to 768 keys; parts and a merge beyond them too)
+        lens = [min(n, longest) for n in ((EDGES + [0, 1025]) * 2)[:S]]
+        _check(lens, [1] * S, Hq, Hkv, D, 16, torch.bfloat16, fp8, 2)
+        if Hq // Hkv <= 4:
+            _check([max(n, 4) for n in lens], [1 + i % 4 for i in range(S)], Hq, Hkv, D, 16, torch.float16, fp8, 2, window=300)

@@ -127,7 +127,7 @@ class Attention(nn.Module):
                                        md.seq_lens[:nd], md.query_start_loc[:nd + 1], self.scale,
                                        num_splits=md.decode_num_splits, max_q_len=md.max_decode_query_len,
                                        window=self.sliding_window, softcap=self.softcap, alibi=self.alibi_slopes,
-                                       workspace=md.decode_workspace, k_scale=ksc, v_scale=vsc)
+                                       workspace=md.decode_workspace, k_scale=ksc, v_scale=vsc, max_kv_len=md.max_seq_len)
         if n_pre > 0:
             e = ndt + md.num_prefill_tokens
             ops.paged_attention_prefill(out[ndt:e], q[ndt:e], src.k_cache, src.v_cache, md.block_table[nd:nd + n_pre],
@@ -208,7 +208,8 @@ class Attention(nn.Module):
                                            sl[:nd], qsl[:nd + 1], self.scale,
                                            num_splits=md.decode_num_splits, max_q_len=md.max_decode_query_len,
                                            window=self.sliding_window, softcap=self.softcap, alibi=self.alibi_slopes,
-                                           workspace=md.decode_workspace, k_scale=ksc, v_scale=vsc)
+                                           workspace=md.decode_workspace, k_scale=ksc, v_scale=vsc,
+                                           max_kv_len=md.max_seq_len)
             if n_pre > 0:
                 e = ndt + md.num_prefill_tokens
                 ops.paged_attention_prefill(out[ndt:e], q[ndt:e], self.k_cache, self.v_cache, bt[nd:nd + n_pre],
@@ -397,7 +398,7 @@ class DualChunkAttention(Attention):
                                            md.local_seq_lens[:nd], qsl[:nd + 1], self.scale,
                                            num_splits=md.decode_num_splits, max_q_len=md.max_decode_query_len,
                                            softcap=self.softcap, workspace=md.decode_workspace, k_scale=ksc,
-                                           v_scale=vsc)
+                                           v_scale=vsc, max_kv_len=md.max_seq_len)
             if n_pre > 0:
                 e = ndt + md.num_prefill_tokens
                 ops.paged_attention_prefill(out[ndt:e], q[ndt:e], self.k_cache, self.v_cache,

@@ -243,12 +243,22 @@ def decode_num_splits(num_seqs: int, num_kv_heads: int, max_seq_len: int) -> int
     return max(1, min(target // wgs, by_len, 64))
 
 
+def decode_parts_as_waves(num_splits: int, num_seqs: int, num_heads: int, num_kv_heads: int, head_size: int, max_q_len: int, keys: int) -> bool:
+    """Two parts of a few short sequences (512 workgroups of four waves at most): eight waves of one workgroup, which want no
+    workspace and no launch that merges them.  ``keys``: an upper bound of a sequence's.  Up to 768 of them (whole pages below that), where
+    ``decode_num_splits`` asks for two parts: longer sequences want the loads of two CUs (one of 2000, 8 kv heads of 128, in a
+    graph, us, two parts / eight waves 19 / 25, of 8000 54 / 100; eight 25 / 33, 75 / 113; eight of 700 14.1 / 14.8, 32 of 700 26 / 23)."""
+    return (num_splits == 2 and num_seqs * num_kv_heads <= 256 and head_size <= 192
+            and max_q_len * (num_heads // num_kv_heads) <= 16 and keys <= 768)
+
+
 def paged_attention_decode(out, q, k_cache, v_cache, block_table, seq_lens, q_start_loc, scale: float,
                            num_splits: int = 1, max_q_len: int = 1, window: int = 0, softcap: float = 0.0,
                            alibi: Optional[torch.Tensor] = None, workspace=None, k_scale: float = 1.0,
                            v_scale: float = 1.0, sink: Optional[torch.Tensor] = None, chunk: int = 0,
-                           v_shift: int = 0, dist_bias: Optional[torch.Tensor] = None):
+                           v_shift: int = 0, dist_bias: Optional[torch.Tensor] = None, max_kv_len: int = 0):
     """q, out: [T, Hq, D].  Each sequence has <= max_q_len query tokens (1 for plain decode).
+    ``max_kv_len``: the most keys of a sequence when the caller knows it on the host (0: what the block table can hold).
     ``sink`` fp32 [Hq]: exp(sink[h]) joins head h's softmax denominator; ``chunk`` > 0: keys of the query's own chunk
     of that many positions only; ``v_shift``: K head k reads V head k >> v_shift (v_cache holds that many fewer heads);
     ``dist_bias`` (rows of ``padded_distance_rows``): the value of min(query position - key position, far) joins head
@@ -263,10 +273,8 @@ def paged_attention_decode(out, q, k_cache, v_cache, block_table, seq_lens, q_st
     S = seq_lens.shape[0]
     part_out = part_lse = None
     if num_splits > 1:
-        # a few short sequences (512 workgroups of four waves at most): two parts as waves of one workgroup, which want no
-        # workspace and no launch that merges them
-        Hkv = k_cache.shape[1]
-        if num_splits == 2 and S * Hkv <= 256 and D <= 192 and max_q_len * (Hq // Hkv) <= 16:
+        keys = block_table.shape[1] * k_cache.shape[2]
+        if decode_parts_as_waves(num_splits, S, Hq, k_cache.shape[1], D, max_q_len, min(keys, max_kv_len) if max_kv_len > 0 else keys):
             pass
         elif workspace is not None:
             part_out, part_lse = workspace[0].data_ptr(), workspace[1].data_ptr()
