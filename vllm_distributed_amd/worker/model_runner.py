@@ -1116,7 +1116,7 @@ class ModelRunner:
             sample_hidden = hidden[self.logits_indices[:S]]
             logits = self._compute_logits(sample_hidden, logits_idx[:S])
             if so.logit_taps:                # on their way to the host before anything changes them
-                taps = self._start_taps(so, hidden, req_ids, n_sched, cu, logits, logits_idx[:S])
+                taps = self._start_taps(so, req_ids, n_sched, cu, logits, logits_idx[:S])
             if envs.VLLM_COMPUTE_NANS_IN_LOGITS:
                 self._last_nans = {r: int(x) for r, x in zip(req_ids, logits.isnan().sum(-1).tolist())}
             if so.grammar_bitmask is not None:
@@ -1166,7 +1166,7 @@ class ModelRunner:
             failed_recving=failed_recving,
             num_nans_in_logits=getattr(self, "_last_nans", None))
         if so.logit_taps:
-            result.tapped_logits = self._collect_taps(taps or self._start_taps(so, hidden, req_ids, n_sched, cu))
+            result.tapped_logits = self._tap_logits(so, hidden, req_ids, n_sched, cu, taps)
         if tmd is not None and not tk_plain:
             get_tknp_group().broadcast_object(result, src=0)
         return result
@@ -1360,9 +1360,8 @@ class ModelRunner:
             out[rid] = LogprobsLists(ids.tolist(), lps.tolist(), ranks.tolist())
         return out
 
-    def _start_taps(self, so, hidden, req_ids, n_sched, cu, logits=None, logits_idx=None):
-        """Queue the full-vocabulary fp32 logits at the positions ``so.logit_taps`` names for the host.  ``logits``: those of the
-        rows ``logits_idx``, which are not worked out a second time where they are the ones that are asked for."""
+    def _tapped_rows(self, so, req_ids, n_sched, cu) -> tuple[list, dict]:
+        """The step's rows whose logits ``so.logit_taps`` asks for, and which of them are each request's."""
         idx, spans = [], {}
         for i, rid in enumerate(req_ids):
             taps = so.logit_taps.get(rid)
@@ -1372,11 +1371,14 @@ class ModelRunner:
                 raise ValueError(f"logit taps {taps} of request {rid} lie outside its {int(n_sched[i])} tokens")
             spans[rid] = (len(idx), len(idx) + len(taps))
             idx.extend(int(cu[i]) + int(t) for t in taps)
-        if not idx:
-            return None, spans, None
-        if logits is None or idx != logits_idx.tolist():
-            sel = torch.tensor(idx, dtype=torch.int64, device=self.device)
-            logits = self._compute_logits(hidden[sel], np.asarray(idx))
+        return idx, spans
+
+    def _start_taps(self, so, req_ids, n_sched, cu, logits, logits_idx):
+        """Queue the step's own logits (fp32, of rows ``logits_idx``) for the host where they are the ones that are asked for, at most
+        a row per request of pinned memory; None where others are."""
+        idx, spans = self._tapped_rows(so, req_ids, n_sched, cu)
+        if not idx or idx != logits_idx.tolist():
+            return None
         rows = torch.empty(logits.shape, dtype=torch.float32, pin_memory=self.pin)
         rows.copy_(logits.float() if self.is_gpu else logits, non_blocking=True)
         done = None
@@ -1385,12 +1387,18 @@ class ModelRunner:
             done.record()
         return rows, spans, done
 
-    @staticmethod
-    def _collect_taps(started) -> dict:
-        """Per request, on the host."""
-        rows, spans, done = started
-        if done is not None:
-            done.synchronize()
+    def _tap_logits(self, so, hidden, req_ids, n_sched, cu, started) -> dict:
+        """Full-vocabulary fp32 logits at the positions ``so.logit_taps`` names, per request, on the host."""
+        if started is not None:
+            rows, spans, done = started
+            if done is not None:
+                done.synchronize()
+        else:
+            idx, spans = self._tapped_rows(so, req_ids, n_sched, cu)
+            if not idx:
+                return {}
+            sel = torch.tensor(idx, dtype=torch.int64, device=self.device)
+            rows = self._compute_logits(hidden[sel], np.asarray(idx)).float().cpu()
         return {rid: rows[a:b].numpy() for rid, (a, b) in spans.items()}
 
     def _compute_logits(self, hidden_rows: torch.Tensor, index: np.ndarray) -> torch.Tensor:
