@@ -361,3 +361,18 @@ def test_wq_slices_of_many_rows():
     for rows in (4, 3):
         got = ops.wq_gemm(x[:rows], qw, sz, G, 8).float()
         assert (got - ref[:rows]).abs().max().item() <= 2 ** -7 * ref.abs().max().item() + 2 ** -6
+
+
+@pytest.mark.parametrize("bits,last", [(4, 10), (8, 12)])
+def test_wq_slices_of_long_rows(bits, last):
+    """More than 8192 elements, up to the last row count of the rule and one beyond."""
+    from vllm_distributed_amd import ops
+    torch.manual_seed(6)
+    N, K, G = 5132, 9216, 128
+    x = (torch.rand(last + 1, K, device="cuda") * 2 - 1).to(torch.bfloat16)
+    qw, scales, zeros, sz, deq = _quantised(N, K, G, bits, torch.bfloat16)
+    ref = x.float() @ deq.to(torch.bfloat16).float().t()
+    for rows in (1, last, last + 1):
+        assert ops.N.lib().vda_wq_slices_pay(rows, N, K, bits, G, 0) == (rows <= last)
+        got = ops.wq_gemm(x[:rows], qw, sz, G, bits).float()
+        assert (got - ref[:rows]).abs().max().item() <= 2 ** -7 * ref.abs().max().item() + 2 ** -6      # as in test_wq_slices

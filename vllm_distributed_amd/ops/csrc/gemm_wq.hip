@@ -4,7 +4,7 @@
 // in LDS; they are widened to the activation type only on their way into the MFMA operand registers.
 //
 // Two kernels.  Up to 128 activation rows (decode): the weight stream is the whole cost, so wq_stream_kernel keeps
-// it out of LDS altogether: packed words go global -> registers eight (4 bit) or four (8 bit) K steps ahead, are
+// it out of LDS altogether: packed words go global -> registers four K steps ahead, are
 // widened in registers and fed to the MFMAs as the A operand, while the activations of a K step are shared by the
 // waves through an LDS ring (the scheme of gemm_decode.hip with a quarter / half of its HBM bytes).  More rows:
 // wq_gemm_kernel, the two-group schedule of gemm_dense.hip (one wave group issues 32 MFMAs from registers while the other issues
@@ -451,18 +451,52 @@ __global__ __launch_bounds__(256 * WM, WM == 1 ? 2 : 1) void wq_stream_kernel(co
 // arithmetic its registers take the activations two steps ahead and the weights four ahead (plain loads, which the
 // compiler counts: were they inline assembly, a build that has to spill would spill what has not arrived).
 // Bound by the memory system's latency and by activations from the L2, of which a wave of 32 weight rows reads M / 8 (4 bits) bytes
-// a byte of weights.  us, K over workgroups -> this: 8192 x 8192 in 4 bits, 2 rows 21.0 -> 12.9, 16 rows 21.9 -> 17.3, in 8 bits, 9
-// rows 25.4 -> 17.8; 28672 x 4096, 9 rows 32.3 -> 27.4, in 8 bits 43.6 -> 35.3; 6144 x 4096 16 -> 10.6.  Twice the steps in
-// flight 34.8 and 19.7 for the second and the fourth of these, eight waves 20.8 for the second.
+// a byte of weights.  Twice the steps in flight, or eight waves, are slower.
 constexpr int WQ_KS = 4;
-// Longer rows of many activations lose: 8192 x 28672 in 4 bits, 1 / 10 / 13 / 16 rows 40.4 -> 34.4 / 41.4 -> 41.5 / 41.9 -> 45.0 / 42.1
-// -> 48.8; 4096 x 14336, 9 / 13 / 16 rows 22.6 -> 20.7 / 23.2 -> 23.5 / 22.6 -> 25.6; in 8 bits 9 / 16 rows 27.1 -> 25.2 / 27.2 -> 30.0.
-// Where workgroups of 128 weight rows fill the chip, the kernel above has no parts to sum (57344 x 8192 in 4 bits, 1 / 13
-// rows 61.8 / 61.9 there, 65.6 / 90.2 here), but for 8 bits and very few rows: 98.7 there, 88.6 here.
-static bool wq_slices_pay(int M, int N, int K, int bits) {
-  const bool fills = (N + 127) / 128 * 4 >= 512 * 3;
-  return M <= 16 && (fills ? bits == 8 && M <= 4 : K <= 8192 || M <= (bits == 4 ? 10 : 12));
+// Up to how many activation rows (of 16) this kernel leads, by what the kernel above would launch.  A step of 128 elements takes a
+// wave here 0.4 (one row) to 0.7 us (16), in 8 bits 0.55 to 0.9, and it walks a quarter of them; the kernel above cuts K into
+// up to 32 parts for 5 us of a launch that sums them.  us, kernel above / this, weights cold, 1, 8 and 16 rows:
+//   one workgroup a CU there: 4 bits 2048 x 4096 10.1 / 7.0, 10.2 / 8.4, 10.5 / 9.9; x 6144 10.6 / 8.8, 11.1 / 10.7, 11.4 / 12.8; x 8192 11.2 / 10.5,
+//     11.7 / 12.8, 11.7 / 15.7; 8 bits x 4096 12.4 / 8.8, 12.7 / 10.3, 13.0 / 11.8; x 8192 13.8 / 13.8, 14.7 / 16.3, 15.2 / 19.1
+//   more: 4 bits 8192 x 8192 18.9 / 15.5, 19.5 / 15.2, 19.8 / 17.9; x 14336 25.9 / 23.2, 26.7 / 24.8, (10 rows) 26.9 / 25.5; x 28672 38.9 / 40.5,
+//     40.0 / 44.0; 4096 x 14336 19.9 / 18.8, 20.3 / 21.1; 8 bits 8192 x 28672 67 / 52, 70 / 57, (12 rows) 67 / 59; 4096 x 28672 45.7 / 43.9,
+//     46.0 / 47.4; 3072 x 14336 25.7 / 22.1, 26.4 / 25.6, x 28672 38.1 / 40.5, 38.6 / 46.8
+//   wide layers in 4 bits, by how many workgroups a CU has to take here: 10240 x 8192 22.1 / 21.5, 23.5 / 25.9, 24.3 / 31.2; 14336 x 8192 29.5 / 23.3,
+//     30.3 / 27.0, 31.6 / 31.8; 28672 x 4096 25.5 / 23.9, 26.2 / 28.5, 27.6 / 34.5
+//   scaled in registers (groups of 64), which costs both more arithmetic: 2048 x 8192 13.0 / 13.0, 13.3 / 13.2, 13.6 / 14.9; 8192 x 14336 30.7 / 24.7,
+//     30.8 / 25.8; 8192 x 28672 48.5 / 44.3, 49.0 / 46.0; 4096 x 28672 33.3 / 38.7; 10240 x 8192 25.2 / 24.3, 25.9 / 25.2, 26.4 / 29.8; 14336 x 8192
+//     36.1 / 26.0, 35.9 / 27.6, 36.8 / 31.0; 28672 x 8192 52.8 / 46.4, 52.1 / 50.0, 52.7 / 58.9
+//   workgroups of 128 weight rows that fill the chip, nothing to sum: 57344 x 8192 4 bits 61.8 / 65.6, 8 bits 111 / 96 (one row), 107 / 107 (10)
+static int wq_slices_rows(int N, int K, int bits, bool scaled) {
+  const int nk = K >> 7, groups = (N + 127) / 128, wgs = groups * max(1, min(min((512 + groups - 1) / groups, nk / 8), 32));
+  if (groups * 4 >= 512 * 3) return bits == 8 ? 4 : 0;
+  if (wgs <= 256) {
+    if (nk <= 32) return 16;
+    if (bits == 4) return scaled ? (nk <= 48 ? 16 : nk <= 64 ? 10 : 0) : nk <= 48 ? 8 : nk <= 64 ? 2 : 0;
+    return nk <= 40 ? 12 : nk <= 48 ? 10 : nk <= 64 && groups >= 24 ? 4 : 0;
+  }
+  if (bits == 8) {
+    if (nk <= 64) return groups <= 128 || nk <= 32 ? 16 : 12;
+    return groups >= 40 ? 12 : groups >= 32 ? (nk <= 160 ? 12 : 4) : nk <= 128 ? 10 : 0;
+  }
+  if (scaled) {
+    if (groups > 128) return nk <= 32 ? 12 : 8;
+    if (groups > 96) return nk <= 64 ? 16 : 10;
+    if (groups > 64) return nk <= 32 ? 16 : nk <= 128 ? 8 : 1;
+    return nk <= 64 ? 16 : nk <= 128 ? 10 : groups >= (nk <= 160 ? 32 : 48) ? 8 : 0;
+  }
+  if (groups > 128) return nk <= 32 ? 2 : nk <= 64 ? 1 : 0;
+  if (groups > 96) return nk <= 32 ? 10 : nk <= 64 ? 16 : nk <= 128 ? 8 : 0;
+  if (groups > 64) return nk <= 32 ? 8 : nk <= 64 ? 1 : 0;
+  return nk <= 64 ? 16 : nk <= 128 ? (groups >= 40 ? 10 : 4) : nk <= 176 ? (groups >= 40 ? 4 : 0) : groups >= 48 ? 1 : 0;
 }
+static bool wq_unscaled(int N, int bits, int group) { return bits == 4 && group % 128 == 0 && N % 4 == 0; }
+static bool wq_slices_pay(int M, int N, int K, int bits, int group, bool no_split) {
+  if (no_split && (N + 127) / 128 * 4 < 512 * 3) return M <= 16 && (K <= 8192 || M <= (bits == 4 ? 10 : 12));   // K in one part there
+  return M <= wq_slices_rows(N, K, bits, !wq_unscaled(N, bits, group));
+}
+// (for the test of the rule, which runs on the host)
+VDA_EXPORT int vda_wq_slices_pay(int M, int N, int K, int bits, int group, int no_split) { return wq_slices_pay(M, N, K, bits, group, no_split); }
 template <typename T, int BITS, bool POST>
 __global__ __launch_bounds__(64 * WQ_KS, 2) void wq_slices_kernel(const WqGemmArgs wa) {
   using V8 = typename Vec<T>::v8;
@@ -608,7 +642,7 @@ static int launch_wq_slices(const WqGemmArgs& wa, hipStream_t st) {
   const DenseGemmArgs& a = wa.d;
   const dim3 grid((unsigned)((a.N + 31) / 32));
   if constexpr (BITS == 4) {
-    if (!wa.per_element && wa.group % 128 == 0 && a.N % 4 == 0) {
+    if (!wa.per_element && wq_unscaled(a.N, 4, wa.group)) {
       hipLaunchKernelGGL((wq_slices_kernel<T, 4, true>), grid, dim3(64 * WQ_KS), 0, st, wa);
       return 0;
     }
@@ -690,7 +724,7 @@ VDA_EXPORT int vda_wq_gemm(void* out, const void* x, const void* qw, const void*
     const int nk = K >> 7;
     const int groups = (N + 127) / 128;
     const int slots = M <= 64 ? 512 : 256;
-    if (variant == 0 && splits < 1 && wq_slices_pay(M, N, K, bits)) {
+    if (variant == 0 && splits < 1 && wq_slices_pay(M, N, K, bits, group, no_split)) {
       rc = dtype == VDA_BF16 ? (bits == 4 ? launch_wq_slices<bf16_t, 4>(wa, st) : launch_wq_slices<bf16_t, 8>(wa, st))
                              : (bits == 4 ? launch_wq_slices<f16_t, 4>(wa, st) : launch_wq_slices<f16_t, 8>(wa, st));
       VDA_CHECK_LAUNCH();
