@@ -128,3 +128,24 @@ def test_nan_comes_out_of_parts(D, Hq, Hkv, where):
     ops.paged_attention_prefill(one, q, kc, vc, table, sl, starts, D ** -0.5, return_lse=True)
     ops.paged_attention_prefill(parts, q, kc, vc, table, sl, starts, D ** -0.5)
     assert bool(one.isnan().any()) and torch.equal(one.isnan(), parts.isnan())
+
+
+@pytest.mark.parametrize("keys", [1, 31, 96, 97, 200])
+@pytest.mark.parametrize("kw", [dict(), dict(causal=False), dict(softcap=5.0), "sink"])
+def test_short_prompts_of_96_values(keys, kw):
+    """The direct form up to 96 keys, by the table or by the bound; options that it does not have, and longer prompts, in the other."""
+    if kw == "sink":
+        kw = dict(sink=torch.linspace(-1, 4, 6, device=DEV))
+    b = _batch([min(keys, 40), 1, keys], [keys - min(keys, 40), keys - 1, 0], 6, 2, 96, 16, torch.float16)
+    q, kc, vc, table, sl, starts = b
+    tall = torch.cat([table, table.new_zeros(3, 40)], 1)
+    one, two, three = torch.empty_like(q), torch.empty_like(q), torch.empty_like(q)
+    ops.paged_attention_prefill(one, q, kc, vc, table, sl, starts, 96 ** -0.5, **kw)
+    ops.paged_attention_prefill(two, q, kc, vc, tall, sl, starts, 96 ** -0.5, max_kv_len=keys, **kw)
+    assert torch.equal(one, two) or keys > 80                       # (tables are whole pages: 96 keys are six)
+    ops.paged_attention_prefill(three, q, kc, vc, tall, sl, starts, 96 ** -0.5, max_kv_len=640, return_lse=True, **kw)
+    bound = (4 * 2.0 ** -12 + 2e-5) * float(vc.float().abs().max())
+    assert float((one.float() - three.float()).abs().max()) <= bound and float((two.float() - three.float()).abs().max()) <= bound
+    if "sink" not in kw:
+        want = R.paged_attention(q.float(), kc.float(), vc.float(), table, sl, starts, 96 ** -0.5, **kw)
+        assert float((one.float() - want).abs().max()) <= (2 * 2.0 ** -12 + 1e-5) * float(vc.float().abs().max())

@@ -336,10 +336,10 @@ def paged_attention_prefill(out, q, k_cache, v_cache, block_table, seq_lens, q_s
     lse = torch.full((Hq, T), float("-inf"), dtype=torch.float32, device=q.device) if return_lse else None
     Hkv, page = k_cache.shape[1], k_cache.shape[2]
     part_out, part_lse, parts = None, None, 1
+    keys = block_table.shape[1] * page                     # that a tile of 128 rows at most can see
+    for bound in (max_kv_len, window + 128 if window > 0 else 0, chunk + 128 if chunk > 0 else 0):
+        keys = min(keys, bound) if bound > 0 else keys
     if not return_lse:
-        keys = block_table.shape[1] * page                 # that a tile of 128 rows at most can see
-        for bound in (max_kv_len, window + 128 if window > 0 else 0, chunk + 128 if chunk > 0 else 0):
-            keys = min(keys, bound) if bound > 0 else keys
         parts = N.lib().vda_prefill_parts(seq_lens.shape[0], T, Hq, Hkv, D, int(max_q_len), keys)
         if parts > 1:
             part = torch.empty(T * Hq * parts * (D + 1), dtype=torch.float32, device=q.device)
@@ -350,7 +350,7 @@ def paged_attention_prefill(out, q, k_cache, v_cache, block_table, seq_lens, q_s
            Hq, Hkv, D, page, block_table.stride(0), q.stride(0), out.stride(0), scale,
            softcap, window, N.dt(q.dtype), _kv_fp8(k_cache), k_scale, v_scale, int(bool(causal)), N.ptr(lse),
            int(max_q_len), N.ptr(sink), int(chunk), int(v_shift), *_dist_bias_args(dist_bias, Hq), part_out, part_lse, parts,
-           N.stream())
+           keys, N.stream())
     return (out, lse) if return_lse else out
 
 

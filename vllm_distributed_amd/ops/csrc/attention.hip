@@ -1198,13 +1198,14 @@ VDA_EXPORT int vda_prefill_parts(int num_seqs, int num_tokens, int Hq, int Hkv, 
 // cascade attention, where one pseudo-sequence holds every query token of the batch).  lse_out, when
 // given, receives the log-sum-exp of every (head, token) for merging with another pass.  A workgroup has 128 / (Hq/Hkv) query tokens
 // (64 / where heads hold more than 128 values, 256 / in the wide form); the grid over-allocates one tile per sequence.
+// max_keys: an upper bound of what a tile sees of a sequence.
 VDA_EXPORT int vda_paged_attention_prefill(
     void* out, const void* q, const void* k_cache, const void* v_cache, const int* block_table,
     const int* seq_lens, const int* q_start_loc, const float* alibi, int num_seqs, int num_tokens,
     int Hq, int Hkv, int D, int block_size, int max_blocks, long q_stride, long out_stride, float scale,
     float softcap, int window, int dtype, int kv_fp8, float k_scale, float v_scale, int causal, float* lse_out,
     int max_q_len, const float* sink, int chunk, int v_shift, const float* dist_bias, int dist_far, float* part_out,
-    float* part_lse, int nsplit, hipStream_t st) {
+    float* part_lse, int nsplit, long max_keys, hipStream_t st) {
   if (Hq % Hkv) return -1;
   const int G = Hq / Hkv;
   if (G > 128) return -4;
@@ -1214,8 +1215,10 @@ VDA_EXPORT int vda_paged_attention_prefill(
   if (nsplit < 1 || nsplit > 64 || (nsplit > 1 && (!part_out || !part_lse || lse_out))) return -6;
   // not in the direct-to-register form
   const bool extras = sink != nullptr || chunk > 0 || v_shift > 0 || dist_bias != nullptr;
-  // the form with K and V in LDS takes a head group's queries as columns of one workgroup
-  const bool lds = (g_prefill_variant != 0 || extras) && G <= prefill_cols(D);
+  // The form with K and V in LDS takes a head group's queries as columns of one workgroup.  Heads of 96 values, whose rows are no
+  // whole number of pieces a thread, do not pay for it over three steps of keys: us, direct / LDS, 24 / 8 heads, 17 tokens 5.3 / 6.3, 64 7.6 / 8.7,
+  // 16 x 60 9.4 / 10.4, 100 10.2 / 10.3, 128 11.4 / 11.2, 300 21.8 / 19.3; of 192 17 tokens 7.5 / 6.3.
+  const bool lds = (g_prefill_variant != 0 || extras) && G <= prefill_cols(D) && (D != 96 || extras || max_keys > 96);
   const int q_tile = (lds ? prefill_cols(D) : 128) / G;
   AttnParams p{q, k_cache, v_cache, out, nullptr, nullptr, block_table, seq_lens, q_start_loc, alibi,
                num_seqs, Hq, Hkv, max_blocks, 1, q_stride, out_stride, scale * (kv_fp8 ? k_scale : 1.f), softcap,
