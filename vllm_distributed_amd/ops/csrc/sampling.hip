@@ -273,15 +273,15 @@ __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs p) {
 // workgroups and four launches, 51 us and 17 us (of the 51: 8 + 12 + 21 + 10; 256 rows of 151936 136: 26 + 33 + 66 + 12):
 //   stats    the row's maximum and smallest finite value (argmax of a greedy row)
 //   bins     counts (top-k) or fixed-point weights (top-p) in SPLIT_BINS bins that are LINEAR between the maximum and the
-//            smallest value: neighbouring lanes hit different bins, and a bin holds a few hundred entries; rows without a
-//            filter draw among half of their entries
+//            smallest value: neighbouring lanes hit different bins, and a bin holds a few hundred entries
 //   collect  draws among the entries above the bin in which the running sum reaches the target, and collects
 //            that bin's entries (top-k and top-p together: all entries down to it)
 //   finish   the exact threshold key among the collected entries, the draw among them, and the row's winner
 // Bound by the noise's 64-bit hash (45 issue slots an entry) where many entries are drawn from, by trips to memory of a
 // microsecond each elsewhere.  A fifth less than a form (62 us; 203 for 256 rows of 151936) that let the entries beyond the span meet in one bin's
-// atomic (92 us of the 203), hashed the upper word anew for every entry, left the filterless rows' draws to the collecting launch,
-// listed entries with a memory atomic each and always took the radix descent at the end.  One launch for collect and
+// atomic (92 us of the 203), hashed the upper word anew for every entry,
+// listed entries with a memory atomic each and always took the radix descent at the end.  Rows without a filter draw in the collecting launch
+// alone: half of their entries in the one before gave nothing (61 rows 52.8 / 52.8 us) and cost a single row 2.5 us.  One launch for collect and
 // finish, the row's last workgroup finishing it, is no way: the fences it needs took it from 20 to 155 us.
 // A row whose bin overflows the list (thousands of equal logits) is done by its finish workgroup alone, the way of the
 // short rows.  The result is that of the one-workgroup form: the bins are monotone in the key, sums are integers, and each
@@ -453,17 +453,11 @@ __device__ __forceinline__ ArgMax split_draw(const SampleArgs& p, const SplitFil
   const Noise n = noise_of((uint64_t)(p.seeds ? p.seeds[rowi] : 0), c.a, c.b);
   return n.same ? split_draw_as<true>(f.inv_t, floor_key, row, c, ahead, n) : split_draw_as<false>(f.inv_t, floor_key, row, c, ahead, n);
 }
-// A row without top-k and top-p has no bins to fill, but noise for every entry, which costs more than all that a filtered row
-// asks for: it draws among the first half of each share here and among the second in the next launch.
-__device__ __forceinline__ int split_half(SplitChunk c) { return c.a + (((c.b - c.a) / 2) & ~3); }
-
 // Sums in two 32-bit words, each of which 65535 entries cannot overflow: 16 bits of a weight each (the upper one up to 65536,
 // and mostly zero).  A 64-bit LDS atomic of a wave costs three times a 32-bit one.
 constexpr int SPLIT_SUMMED = 65532;
 __global__ __launch_bounds__(1024) void split_bins_kernel(SampleArgs p, SplitRow* ws_rows, int row0) {
   __shared__ uint32_t low[SPLIT_BINS], high[SPLIT_BINS];
-  __shared__ float rv[16];
-  __shared__ int ri[16];
   const int rowi = row0 + blockIdx.y;
   SplitRow* ws = ws_rows + blockIdx.y;
   const float* row = p.logits + (long)rowi * p.stride;
@@ -471,15 +465,8 @@ __global__ __launch_bounds__(1024) void split_bins_kernel(SampleArgs p, SplitRow
   SplitAhead ahead = split_ahead(row, c, c.a);
   const f32x2 parts = split_parts(ws, gridDim.x);
   const SplitFilter f = split_filter(p, rowi);
-  if (f.greedy) return;
+  if (f.greedy || f.mode == MODE_NONE) return;
   const SplitScale sc = split_scale(parts);
-  if (f.mode == MODE_NONE) {
-    c.b = split_half(c);
-    ArgMax a = split_draw(p, f, sc, rowi, row, c, ahead);
-    a = block_argmax(a, rv, ri);
-    if (threadIdx.x == 0) { ws->part_v[blockIdx.x] = a.v; ws->part_i[blockIdx.x] = a.i; }
-    return;
-  }
   const int end = c.b;
   for (;;) {
 #pragma unroll
@@ -606,7 +593,7 @@ __device__ uint32_t ranked_threshold(const uint2* list, const unsigned long long
   return found == 0xffffffffu ? 0u : found;
 }
 
-__global__ __launch_bounds__(1024) void split_collect_kernel(SampleArgs p, SplitRow* ws_rows, int row0, int half_drawn) {
+__global__ __launch_bounds__(1024) void split_collect_kernel(SampleArgs p, SplitRow* ws_rows, int row0) {
   __shared__ float rv[16];
   __shared__ int ri[16];
   __shared__ unsigned long long s_wave[16];
@@ -616,8 +603,7 @@ __global__ __launch_bounds__(1024) void split_collect_kernel(SampleArgs p, Split
   const int rowi = row0 + blockIdx.y;
   SplitRow* ws = ws_rows + blockIdx.y;
   const float* row = p.logits + (long)rowi * p.stride;
-  SplitChunk c = split_chunk(row, p.V, gridDim.x);
-  const int half = split_half(c);
+  const SplitChunk c = split_chunk(row, p.V, gridDim.x);
   const SplitAhead ahead = split_ahead(row, c, c.a);
   const f32x2 parts = split_parts(ws, gridDim.x);
   const u64x2 bin_sum = reinterpret_cast<const u64x2*>(ws->hist)[threadIdx.x];
@@ -626,9 +612,7 @@ __global__ __launch_bounds__(1024) void split_collect_kernel(SampleArgs p, Split
   const SplitScale sc = split_scale(parts);
   ArgMax a{-INFINITY, 0x7fffffff};
   if (f.mode == MODE_NONE) {
-    if (half_drawn) c.a = half;
-    a = split_draw(p, f, sc, rowi, row, c, half_drawn ? split_ahead(row, c, c.a) : ahead);
-    if (half_drawn && threadIdx.x == 0) a = amax2(a, ArgMax{ws->part_v[blockIdx.x], ws->part_i[blockIdx.x]});
+    a = split_draw(p, f, sc, rowi, row, c, ahead);
   } else {
     if (threadIdx.x == 0) s_count = 0u;
     const SplitCut cut = split_cut(bin_sum, f, s_wave, &s_cut);
@@ -818,7 +802,7 @@ VDA_EXPORT int vda_sample(const float* logits, long* out, const float* temperatu
     const int G = max(1, min(min(512 / rows, (V + 4095) / 4096), SPLIT_MAX_G));
     hipLaunchKernelGGL(split_stats_kernel, dim3(G, rows), dim3(1024), 0, st, p, ws, row0);
     if (filtered) hipLaunchKernelGGL(split_bins_kernel, dim3(G, rows), dim3(1024), 0, st, p, ws, row0);
-    hipLaunchKernelGGL(split_collect_kernel, dim3(G, rows), dim3(1024), 0, st, p, ws, row0, (int)filtered);
+    hipLaunchKernelGGL(split_collect_kernel, dim3(G, rows), dim3(1024), 0, st, p, ws, row0);
     hipLaunchKernelGGL(split_finish_kernel, dim3(rows), dim3(1024), 0, st, p, ws, row0, G);
   }
   VDA_CHECK_LAUNCH();
