@@ -270,7 +270,7 @@ __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs p) {
 // ---- rows over several workgroups --------------------------------------------------------------------------------
 // One workgroup per row spends up to ten passes over 0.5 MB (V = 128256) on one CU, most of the time in LDS atomics that
 // all hit the few leading bytes real logits share: 447 us for 61 rows of V = 128256, 73 us for one.  Here a row takes G
-// workgroups and four launches, 51 us and 17 us (of the 51: 8 + 12 + 21 + 10; 256 rows of 151936 136: 26 + 33 + 66 + 12):
+// workgroups and four launches, 47 us and 15 us (256 rows of 151936 120):
 //   stats    the row's maximum and smallest finite value (argmax of a greedy row)
 //   bins     counts (top-k) or fixed-point weights (top-p) in SPLIT_BINS bins that are LINEAR between the maximum and the
 //            smallest value: neighbouring lanes hit different bins, and a bin holds a few hundred entries
@@ -339,9 +339,10 @@ __device__ __forceinline__ SplitChunk split_chunk(const float* row, int V, int G
   c.vec = (reinterpret_cast<uintptr_t>(row) & 15) == 0;
   return c;
 }
-// Sixteen entries a thread are on their way at once; the first of them (``ahead``) since before anything else is known of
-// the row: every trip to what another kernel has just written costs about a microsecond.
-constexpr int SPLIT_AHEAD = 4;
+// Eight entries a thread are on their way at once; the first of them (``ahead``) since before anything else is known of
+// the row: every trip to what another kernel has just written costs about a microsecond.  (Sixteen took the collecting kernel to 86
+// registers, which leaves a CU one workgroup of the two that the launch is cut for: 64 rows of 151936 58.5 us, so 50.2; 256 136 / 120.)
+constexpr int SPLIT_AHEAD = 2;
 struct SplitAhead { f32x4 v[SPLIT_AHEAD]; };
 __device__ __forceinline__ SplitAhead split_ahead(const float* row, SplitChunk c, int from) {
   SplitAhead h;
@@ -376,6 +377,7 @@ __device__ __forceinline__ void split_walk(const float* row, SplitChunk c, Split
 
 // the row's maximum and the width of its bins, from the workgroups' partial results; every thread returns the same
 struct SplitScale { float zmax, per; };
+__device__ __forceinline__ float uniform(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
 // (split_parts asks for them)
 __device__ __forceinline__ f32x2 split_parts(const SplitRow* ws, int G) {
   const int lane = threadIdx.x & 63;
@@ -609,13 +611,15 @@ __global__ __launch_bounds__(1024) void split_collect_kernel(SampleArgs p, Split
   const u64x2 bin_sum = reinterpret_cast<const u64x2*>(ws->hist)[threadIdx.x];
   const SplitFilter f = split_filter(p, rowi);
   if (f.greedy) return;
-  const SplitScale sc = split_scale(parts);
+  SplitScale sc = split_scale(parts);                     // (64 registers, two workgroups a CU: what is the row's own is in scalar ones)
+  sc = SplitScale{uniform(sc.zmax), uniform(sc.per)};
   ArgMax a{-INFINITY, 0x7fffffff};
   if (f.mode == MODE_NONE) {
     a = split_draw(p, f, sc, rowi, row, c, ahead);
   } else {
     if (threadIdx.x == 0) s_count = 0u;
-    const SplitCut cut = split_cut(bin_sum, f, s_wave, &s_cut);
+    SplitCut cut = split_cut(bin_sum, f, s_wave, &s_cut);
+    cut.bin = __builtin_amdgcn_readfirstlane(cut.bin);
     const bool all = f.mode == MODE_ALL;
     // a count that reaches the -inf entries keeps every other one: none of them needs to be listed
     const bool keeps_all = cut.bin < 0 || cut.bin == SPLIT_BINS - 1;
