@@ -32,7 +32,7 @@ def _batch(new, prefix, Hq, Hkv, D, BS, dt, fp8=False, spare=0):
 
 def _parts(b, Hq, keys=0):
     q, kc, _, table, sl, _ = b
-    return ops.N.lib().vda_prefill_parts(sl.shape[0], q.shape[0], Hq, kc.shape[1], q.shape[2], 0, keys or table.shape[1] * kc.shape[2])
+    return ops.N.lib().vda_prefill_parts(sl.shape[0], q.shape[0], Hq, kc.shape[1], q.shape[2], keys or table.shape[1] * kc.shape[2])
 
 
 @pytest.mark.parametrize("D,Hq,Hkv,BS,fp8", [(64, 8, 2, 16, False), (64, 4, 4, 64, True), (96, 6, 2, 16, False), (128, 8, 1, 16, False),

@@ -1190,17 +1190,20 @@ VDA_EXPORT int vda_set_prefill_wide_min_wgs(long n) { g_prefill_wide_min_wgs = n
 // 100 new tokens on 2000 of each of two, 32 / 8 heads of 64 137 us in one part, 37 in seven; 16 / 8 heads of 256 386 -> 83, 24 / 8 of 96 255 -> 57;
 // of 128, on 3500, 300 -> 70; one prompt of 1000, 8 / 1 heads, 47 -> 30.
 // Two workgroups a CU are filled, with eight steps a part at least; a part's rows are written and read back once, so that
-// many query rows want few parts: their cost grows with the parts as the walk's falls.
-VDA_EXPORT int vda_prefill_parts(int num_seqs, int num_tokens, int Hq, int Hkv, int D, int max_q_len, long max_keys) {
+// many query rows want few parts: their cost grows with the parts as the walk's falls.  The merge is a workgroup a (token, head), of which some
+// 3500 a us start: 32 / 8 heads of 64, prompts of 520, 700 and 1000 tokens, one part / two 20.7 / 22.9, 26.0 / 28.2, 34.4 / 39.8; 14 / 2 heads, three of 500
+// 22.0 / 25.3; 32 / 8 of 128, 300 on 300 30.1 / 27.5, 100 on 450 of each of four 28.6 / 29.5; 16 / 8 of 256, these 35.8 / 31.9.
+VDA_EXPORT int vda_prefill_parts(int num_seqs, int num_tokens, int Hq, int Hkv, int D, long max_keys) {
   if (Hkv < 1 || Hq % Hkv || Hq / Hkv > 128) return 1;
   const int G = Hq / Hkv, q_tile = (G <= prefill_cols(D) ? prefill_cols(D) : 128) / G;
   if (D == 128 && 256 % G == 0 && (g_prefill_variant == 3 || (g_prefill_variant == 1 &&
       (long)(num_tokens / (256 / G)) * Hkv >= g_prefill_wide_min_wgs))) return 1;
   const long wgs = (long)(num_tokens / q_tile + min(num_seqs, num_tokens)) * Hkv, steps = (max_keys + 31) / 32;
   if (wgs < 1 || wgs > 256 || steps < 16) return 1;
-  const double walk = 1.2 * steps, row_part = (double)num_tokens * Hq * D * 8 / 4e6;         // us
-  const long parts = max(1L, min(min(min(512 / wgs, steps / 8), (long)sqrt(walk / row_part) + 1), 64L));
-  return walk * (1 - 1.0 / parts) > 4 + row_part * parts ? (int)parts : 1;                    // (4: the launch that merges them)
+  const double rows = (double)num_tokens * Hq, row_part = rows * D * 8 / 4e6;                 // us
+  const long parts = max(1L, min(min(min(512 / wgs, steps / 8), (long)sqrt(1.2 * steps / row_part) + 1), 64L));
+  const double walk = (0.7 + 0.0055 * D) * steps, merge = 4 + rows / 3500 + row_part * parts;
+  return walk * (1 - 1.0 / parts) > merge ? (int)parts : 1;
 }
 
 // Varlen attention of new tokens against the paged cache (the new tokens' own K/V must already be in
