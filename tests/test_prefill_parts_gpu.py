@@ -149,3 +149,29 @@ def test_short_prompts_of_96_values(keys, kw):
     if "sink" not in kw:
         want = R.paged_attention(q.float(), kc.float(), vc.float(), table, sl, starts, 96 ** -0.5, **kw)
         assert float((one.float() - want).abs().max()) <= (2 * 2.0 ** -12 + 1e-5) * float(vc.float().abs().max())
+
+
+@pytest.mark.parametrize("kw", [dict(chunk=96), dict(v_shift=1), "sink", "bias", "alibi", dict(window=70, softcap=5.0)])
+@pytest.mark.parametrize("D", [96, 192])
+@pytest.mark.parametrize("prefix", [0, 700])                            # one part, and (the last five tokens) several
+def test_options_of_heads_of_96_and_192_values(D, kw, prefix):
+    """Against the decode kernel, where every new token is a sequence of its own."""
+    Hq, Hkv = 8, 2
+    new = [150, 5] if not prefix else [5]
+    b = _batch(new, [prefix] * len(new), Hq, Hkv, D, 16, torch.float16)
+    q, kc, vc, table, sl, starts = b
+    if kw == "sink":
+        kw = dict(sink=torch.linspace(-1, 4, Hq, device=DEV))
+    elif kw == "alibi":
+        kw = dict(alibi=torch.linspace(0.001, 0.1, Hq, device=DEV))
+    elif kw == "bias":
+        kw = dict(dist_bias=ops.padded_distance_rows(torch.linspace(1, -1, 90 * Hq, device=DEV).view(90, Hq)))
+    if kw.get("v_shift"):
+        vc = vc[:, :1].contiguous()
+    out, rows = torch.empty_like(q), torch.empty_like(q)
+    ops.paged_attention_prefill(out, q, kc, vc, table, sl, starts, D ** -0.5, **kw)
+    own = torch.cat([torch.full((n,), s) for s, n in enumerate(new)]).to(DEV)
+    lens = torch.cat([prefix + 1 + torch.arange(n) for n in new]).to(torch.int32).to(DEV)
+    each = torch.arange(len(own) + 1, dtype=torch.int32, device=DEV)
+    ops.paged_attention_decode(rows, q, kc, vc, table[own].contiguous(), lens, each, D ** -0.5, **kw)
+    assert float((out.float() - rows.float()).abs().max()) <= (4 * 2.0 ** -12 + 2e-5) * float(vc.float().abs().max())   # as above

@@ -278,8 +278,8 @@ __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs p) {
 //            that bin's entries (top-k and top-p together: all entries down to it)
 //   finish   the exact threshold key among the collected entries, the draw among them, and the row's winner
 // Bound by the noise's 64-bit hash (45 issue slots an entry) where many entries are drawn from, by trips to memory of a
-// microsecond each elsewhere.  A fifth less than a form (62 us; 203 for 256 rows of 151936) that let the entries beyond the span meet in one bin's
-// atomic (92 us of the 203), hashed the upper word anew for every entry,
+// microsecond each elsewhere.  A fifth and a third less than a form (59 us; 185 for 256 rows of 151936) that let the entries beyond the span meet in
+// one bin's atomic (half of the 185), hashed the upper word anew for every entry,
 // listed entries with a memory atomic each and always took the radix descent at the end.  Rows without a filter draw in the collecting launch
 // alone: half of their entries in the one before gave nothing (61 rows 52.8 / 52.8 us) and cost a single row 2.5 us.  One launch for collect and
 // finish, the row's last workgroup finishing it, is no way: the fences it needs took it from 20 to 155 us.
