@@ -238,3 +238,24 @@ def test_eight_states_a_lane(monkeypatch, new, ctx, Ch, N, heads, groups, chunks
     # 32-bit sums of N states carried through up to 130 decays, one fp16 rounding of the result
     torch.testing.assert_close(y.float()[live], want[live], atol=1e-3, rtol=2 ** -10)
     torch.testing.assert_close(a["ssm_state"], f["ssm_state"], atol=1e-4, rtol=1e-4)
+
+
+@pytest.mark.parametrize("S,tokens,Ch,N,cut", [(1, 160, 2048, 64, True), (1, 150, 2048, 64, False), (1, 160, 2048, 128, True), (1, 150, 2048, 128, False),
+                                               (3, 256, 1024, 128, True), (3, 200, 1024, 128, False), (1, 600, 4096, 128, True), (1, 500, 4096, 128, False),
+                                               (1, 160, 2048, 256, True), (3, 767, 2048, 128, False), (3, 768, 2048, 128, True), (4, 700, 2048, 64, True), (8, 700, 2048, 64, False)])
+def test_prompts_are_cut_where_the_chip_has_room(monkeypatch, S, tokens, Ch, N, cut):
+    """Eight states a lane: the rule by states and tokens, and the same result either way."""
+    monkeypatch.delenv("VDA_SCAN_CHUNK_MIN_TOKENS", raising=False)
+    a = _scan_inputs([tokens] * S, [i % 2 for i in range(S)], Ch, N, Ch // 64, 1, torch.float16, Ch + N)
+    a = {k: v.contiguous() if isinstance(v, torch.Tensor) else v for k, v in a.items()}
+    b = {k: v.clone() if isinstance(v, torch.Tensor) else v for k, v in a.items()}
+    called, call = [], ops.N.call
+    monkeypatch.setattr(ops.N, "call", lambda name, *args: (called.append((name, args[27], args[29])), call(name, *args))[1])
+    y = ops.selective_scan(**a, max_query_len=tokens)
+    (name, form, nchunks), = called
+    assert (name, form) == ("vda_selective_scan_pairs", 3) and (nchunks > 1) is cut
+    monkeypatch.setenv("VDA_SCAN_CHUNK_MIN_TOKENS", "100000" if cut else "32")
+    other = ops.selective_scan(**b, max_query_len=tokens)
+    # sums of N states in another order over some hundred decays below one, and one fp16 rounding each
+    torch.testing.assert_close(y.float(), other.float(), atol=2e-3, rtol=2 ** -9)
+    torch.testing.assert_close(a["ssm_state"], b["ssm_state"], atol=2e-4, rtol=2e-4)

@@ -1558,23 +1558,28 @@ def selective_scan(u: torch.Tensor, delta: torch.Tensor, A: torch.Tensor, B: tor
     # one pass, 82 in chunks of 32), from 256 on in the plain form, where more passes over more states pay later, and with
     # two states a lane, whose waves (eight channels each) are only cut where they leave SIMDs with less than two: us in one
     # pass / cut, 4096 channels: 241 tokens 32 / 32, 402 43 / 33, 1609 148 / 70; 8192: 322 tokens 31 / 37, 1609 155 / 119;
-    # 16384 channels and sequences: 1212 tokens 126 / 128; 24576: 1558 tokens 163 / 206.  Eight states a lane likewise, from 768 on: 4096
-    # channels: 482 tokens 69 / 70, 1609 248 / 192; 8192: 1212 tokens 196 / 193; 12288: 1558 254 / 339
-    if max_query_len >= ((768 if groups else 96 if paired and not lanes else 256) if set_min is None else set_min):
-        # lanes per channel: N / 16, or as many for a pair of them
-        least = 32 if paired else 64
+    # 16384 channels and sequences: 1212 tokens 126 / 128; 24576: 1558 tokens 163 / 206.
+    # Eight states a lane: four waves a SIMD are 2^21 states (two in rows of 256), which that many pieces of the tokens make; the fewer a
+    # batch has, the earlier it is cut.  us, one pass / cut, 150, 250, 500 and 1000 tokens: 16 pieces (2048 x 64 states) 26 / 19, 40 / 23, 74 / 36,
+    # 143 / 53; 8 (4096 x 64) 26 / 24, 41 / 34, 74 / 51, 143 / 83; 6 (three of 1024 x 128) 26 / 30, 39 / 38, 72 / 65, 150 / 112; 4 (4096 x 128) 25 / 31,
+    # 39 / 45, 72 / 72, 139 / 129; 3 (three of 2048 x 128) 30 / 41, 45 / 57, 84 / 99, 170 / 178, but of 1266 tokens at most 219 / 210
+    least, want = 32 if paired else 64, 1
+    if groups:
+        pieces = -(-(1 << 21) // (S * Ch * min(Nst, 128)))
+        start = 160 if pieces >= 8 else 256 if pieces >= 6 else 600 if pieces >= 4 and Nst < 256 else 768
+        if pieces >= 3 and max_query_len >= (start if set_min is None else set_min):
+            want = pieces
+    elif max_query_len >= ((96 if paired and not lanes else 256) if set_min is None else set_min):
         if lanes:
             want = -(-65536 // (S * Ch)) if S * Ch < 16384 else 1
-        elif groups:
-            want = -(-16384 // (S * Ch)) if S * Ch < 8192 else 1
-        else:
+        else:                                    # lanes per channel: N / 16, or as many for a pair of them
             want = -(-524288 // (S * (Ch // (2 if paired else 1)) * (Nst // 16)))
-        if want > 1:
-            chunk = max(least, -(-(-(-max_query_len // want)) // least) * least)
-            nchunks = -(-max_query_len // chunk)
-        if nchunks > 1:
-            ws_p = torch.empty((S, nchunks, Ch) if paired else (S, nchunks, Ch, Nst), dtype=torch.float32, device=u.device)
-            ws_h = torch.empty((S, nchunks, Ch, Nst), dtype=torch.float32, device=u.device)
+    if want > 1:
+        chunk = max(least, -(-(-(-max_query_len // want)) // least) * least)
+        nchunks = -(-max_query_len // chunk)
+    if nchunks > 1:
+        ws_p = torch.empty((S, nchunks, Ch) if paired else (S, nchunks, Ch, Nst), dtype=torch.float32, device=u.device)
+        ws_h = torch.empty((S, nchunks, Ch, Nst), dtype=torch.float32, device=u.device)
     args = (out.data_ptr(), u.data_ptr(), delta.data_ptr(), A.data_ptr(), B.data_ptr(),
             C.data_ptr(), N.ptr(D), N.ptr(z), N.ptr(delta_bias), ssm_state.data_ptr(), query_start_loc.data_ptr(),
             seq_lens.data_ptr(), block_table.data_ptr(), block_table.stride(0), S, Ch, Nst,
