@@ -175,3 +175,14 @@ def test_options_of_heads_of_96_and_192_values(D, kw, prefix):
     each = torch.arange(len(own) + 1, dtype=torch.int32, device=DEV)
     ops.paged_attention_decode(rows, q, kc, vc, table[own].contiguous(), lens, each, D ** -0.5, **kw)
     assert float((out.float() - rows.float()).abs().max()) <= (4 * 2.0 ** -12 + 2e-5) * float(vc.float().abs().max())   # as above
+
+
+@pytest.mark.parametrize("new", [[845], [846], [864], [430, 400], [500, 1, 700], [300] * 4])           # 47, 48, 49 tiles, and more of several prompts
+def test_four_groups_of_tiles(new):
+    """Four kv heads, whose tiles go to the XCDs in turn from 48 on and for up to three prompts, in runs otherwise: all of them, once each."""
+    b = _batch(new, [5] * len(new), 28, 4, 128, 16, torch.bfloat16)
+    q, kc, vc, table, sl, starts = b
+    out = torch.full_like(q, float("nan"))
+    ops.paged_attention_prefill(out, q, kc, vc, table, sl, starts, 128 ** -0.5, max_kv_len=32 * 15)      # (one part)
+    want = R.paged_attention(q.float(), kc.float(), vc.float(), table, sl, starts, 128 ** -0.5)
+    assert float((out.float() - want).abs().max()) <= (2 * 2.0 ** -9 + 1e-5) * float(vc.float().abs().max())

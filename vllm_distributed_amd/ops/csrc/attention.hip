@@ -644,14 +644,14 @@ __global__ __launch_bounds__(256, PREFILL_WGS_PER_CU) void paged_prefill_lds_ker
   // turn), whose L2 then serves them, the longest tiles of a prompt first (us, tiles over all XCDs -> this: eight prompts of some
   // 1000, 16 / 8 heads of 256 308 -> 268, 24 / 8 of 96 196 -> 167, 32 / 8 of 64 141 -> 128; 25 new tokens on 3000 of two, 64 / 8 of
   // 128, 70 -> 45).  Four groups of few prompts share their two XCDs tile by tile (28 / 4 heads of 128, one of 4000 275 -> 186, three of 1500
-  // 127 -> 108, 16 / 4 of 192 293 -> 180); many prompts, and fewer groups, are even enough in runs, and stay in their L2 (eight of
-  // 1000, dealt by tiles 118 -> 131, two groups 85 -> 116).
+  // 127 -> 108, 16 / 4 of 192 293 -> 180); many prompts, few tiles and fewer groups are even enough in runs, and stay in their L2 (eight of
+  // 1000, dealt by tiles 118 -> 131, two groups 85 -> 116; one of 300, 17 tiles, 21.9 -> 22.6).
   int tile = blockIdx.x, part = 0, kvh = SPARSE ? blockIdx.y / (p.Hq / p.Hkv) : blockIdx.y;
   if constexpr (!SPARSE) {
     const int tiles = gridDim.x, groups = gridDim.y * gridDim.z, n = tiles * groups;
     const int id = blockIdx.x + tiles * (blockIdx.y + gridDim.y * blockIdx.z), x = id & 7;
     int group, at;
-    if (groups == 4 && p.num_seqs <= 3) {                 // two XCDs a group: its tiles in turn, or one of them has all of the longest
+    if (groups == 4 && p.num_seqs <= 3 && tiles >= 48) {  // two XCDs a group: its tiles in turn, or one of them has all of the longest
       group = x & 3;
       at = (id >> 3) * 2 + (x >> 2);
     } else {
