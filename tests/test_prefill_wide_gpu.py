@@ -121,3 +121,55 @@ def test_wide_prefill_fp8_cache(bs):
     ops.paged_attention_prefill(out, q, kc8, vc8, bt, sl, qsl, scale, k_scale=ks, v_scale=vs)
     ref = R.paged_attention(q, kc8, vc8, bt, sl, qsl, scale, k_scale=ks, v_scale=vs)
     torch.testing.assert_close(out.float(), ref.float(), **tol(dt))
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_wide_prefill_lagging_maximum(dt):
+    """Scores that climb key by key: by less than the lag of the running maximum (a factor of 2^8) for long stretches,
+    beyond it in between, at tile edges and inside, and a row that its last key carries alone."""
+    Hq, Hkv, bs, n = 8, 2, 16, 700
+    q, kc, vc, bt, sl, qsl = _paged_problem([n], [n], Hq, Hkv, 128, bs, dt)
+    q[:] = 0.3
+    for pos in range(n):
+        kc[int(bt[0, pos // bs]), :, pos % bs, :] = 0.01 * pos + (1.5 if pos in (63, 64, 200, 411, 699) else 0.0)
+    scale = 1.0 / math.sqrt(128)                     # scores 0 .. 24, steps of 0.034 and of 5.1
+    out = torch.full_like(q, float("nan"))
+    _, lse = ops.paged_attention_prefill(out, q, kc, vc, bt, sl, qsl, scale, return_lse=True)
+    ref, lref = R.paged_attention(q, kc, vc, bt, sl, qsl, scale, return_lse=True)
+    torch.testing.assert_close(out.float(), ref.float(), **tol(dt))
+    # the sum of weights rounded to 8 bits and more: 2^-9 relative at most, and fp32 sums
+    torch.testing.assert_close(lse, lref, atol=3e-3, rtol=1e-4)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_wide_prefill_more_tiles_than_lanes(fp8):
+    """Page numbers are held for 64 tiles at a time: prefixes that end just before, at and behind the 64th and 128th tile."""
+    dt, Hq, Hkv, D, bs = torch.bfloat16, 8, 2, 128, 16
+    seq_lens, q_lens = [4095, 4096, 4097, 4161, 8300, 3970], [40, 64, 65, 1, 130, 3970]
+    q, kc, vc, bt, sl, qsl = _paged_problem(seq_lens, q_lens, Hq, Hkv, D, bs, dt)
+    if fp8:
+        kc, vc = (c.float().clamp(-448, 448).to(torch.float8_e4m3fn) for c in (kc, vc))
+    scale = 1.0 / math.sqrt(D)
+    out = torch.full_like(q, float("nan"))
+    ops.paged_attention_prefill(out, q, kc, vc, bt, sl, qsl, scale)
+    ref = R.paged_attention(q, kc, vc, bt, sl, qsl, scale)
+    torch.testing.assert_close(out.float(), ref.float(), **tol(dt))
+
+
+def test_unaligned_caches_take_the_four_wave_form():
+    """The wide form copies 16-byte pieces to LDS; caches that start elsewhere give the 4-wave form's result."""
+    dt, Hq, Hkv, bs = torch.bfloat16, 16, 4, 16
+    q, kc, vc, bt, sl, qsl = _paged_problem([300, 90], [300, 30], Hq, Hkv, 128, bs, dt)
+    scale = 1.0 / math.sqrt(128)
+    N.call("vda_set_prefill_variant", 2)
+    want = torch.empty_like(q)
+    ops.paged_attention_prefill(want, q, kc, vc, bt, sl, qsl, scale)
+    N.call("vda_set_prefill_variant", 3)
+    moved = []
+    for c in (kc, vc):
+        room = torch.empty(c.numel() + 4, dtype=dt, device=DEV)
+        moved.append(room[4:].view(c.shape).copy_(c))
+        assert moved[-1].data_ptr() % 16 == 8
+    got = torch.empty_like(q)
+    ops.paged_attention_prefill(got, q, *moved, bt, sl, qsl, scale)
+    assert torch.equal(got, want)

@@ -1239,7 +1239,9 @@ VDA_EXPORT int vda_paged_attention_prefill(
   p.sink = sink; p.chunk = chunk; p.v_shift = v_shift; p.dist_bias = dist_bias; p.dist_far = dist_far;
   // Wide form (8 waves, 256 columns, 64-key tiles): head size 128 and enough query tiles to occupy the
   // chip (one workgroup per CU); short chunks keep the 4-wave form, which cuts them into more workgroups.
-  if (nsplit == 1 && D == 128 && 256 % G == 0 && (g_prefill_variant == 1 || g_prefill_variant == 3)) {
+  // Its copies to LDS ask for caches aligned to 16 bytes.
+  const bool aligned = (((uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0;
+  if (nsplit == 1 && D == 128 && 256 % G == 0 && aligned && (g_prefill_variant == 1 || g_prefill_variant == 3)) {
     const int wide_tile = 256 / G;
     const long wgs = (long)(num_tokens / wide_tile) * Hkv;
     if (g_prefill_variant == 3 || wgs >= g_prefill_wide_min_wgs) {

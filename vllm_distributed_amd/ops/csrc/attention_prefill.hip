@@ -1,5 +1,5 @@
 // Wide prefill attention for gfx950, head size 128: 8 waves per workgroup, 32 query columns per wave,
-// 64-key tiles, 32x32x16 MFMA.
+// 64-key tiles, 32x32x16 MFMA, products and softmax of neighbouring tiles interleaved.
 //
 // Same role as the prefill side of the reference's Triton unified attention
 // (vllm/attention/ops/triton_unified_attention.py) and its ROCm flash-attention backend
@@ -9,26 +9,49 @@
 // columns of 16x16x32 tiles and a 32-key step, which costs ~230 vector-ALU instructions per 32 MFMAs
 // (per-lane block-table lookups, address arithmetic for a copy step of only 32 keys, two cross-lane
 // maximum exchanges per 16-column tile) -- the VALU, not the matrix pipe, sets its speed.  Here
-//   * a column's 32 scores of a 32-key block sit in ONE lane pair (l, l+32) (swapped product
+//   * a column's scores of a 32-key block sit in ONE lane pair (l, l+32) (swapped product
 //     S^T = K.Q^T on the 32x32 tile), so the running maximum needs one half-swap per 64 keys;
 //   * P never moves between lanes: registers 8t..8t+7 of a score block are, after conversion, the
-//     B operand of the P.V product for k-step t; the matching permutation of the key order is applied
-//     to V when it is copied into LDS (4-key granules regrouped), which costs nothing;
-//   * one barrier and one copy step per 64 keys, block numbers fetched one tile ahead of the loads
-//     that need them, loads for tile t+1 in flight during the products of tile t;
+//     B operand of the P.V product for k-step t.  The K rows are handed to the first product in an order (key_of_row) that makes
+//     those eight registers eight consecutive keys, so V needs no regrouping;
+//   * so 16-bit K and V go global -> LDS without passing registers, one page number (scalar) for all that a wave copies of a tile,
+//     into rings of four tiles;
 //   * workgroup id -> (kv head = id mod Hkv, query tile descending): with 8 kv heads every XCD
 //     keeps one head's keys in its L2, and the longest causal tiles start first.
 //
+// Schedule.  Scores, softmax and P.V of one key depend on each other, so a half step works on three blocks of 32 keys at once:
+//   half step h: scores of block h + 1 and P.V of block h - 1 (16 MFMAs), and between them, in slices, the softmax of block h.
+// (An MFMA of this size takes the matrix pipe for 32 cycles and the issue for 8; a vector instruction takes 4, an exponential 8.)
+// A step is two of them, a tile of 64 keys, with one barrier.  Step t reads blocks of K tiles t and t + 1 and of V tiles t - 1 and
+// t, which live in rings of four: it issues batch t + 2 (V of tile t + 2, K of tile t + 3) into the places that step t - 1 read
+// last, and waits, before its barrier, for the batch that step t - 1 issued, which is read from step t + 1 on.  LDS reads run
+// eight products ahead, across half steps and barriers.
+//
+// The maximum that weights are relative to may lag behind by a factor of 2^8 (a column's own decision), so that scaling the
+// 64 sums of a lane is rare; with a maximum kept exact, some column of 32 moved in most steps of sequences of a few
+// thousand keys, and the products of the scaling were a third of all vector instructions.  Weights are then not at most one, and the
+// largest one is no longer exact in 16 bits; the denominator adds the rounded weights (one v_dot2 for two of them), so that a row which
+// one key carries still is that key's value.  Error against 64 bits as before (0.0027 over ragged prompts of some 1100 tokens, cache and output
+// in bf16).
+//
+// Measured (MI355X, bf16, 32 / 8 heads, attention alone; before: one barrier a tile, products and softmax of a tile one after the other, K
+// and V through registers): 2048 tokens on 8192 keys 361 -> 313 us, 2 x 4096 331 -> 291, 2048 82 -> 65, 8 x 1024 118 -> 107, 16 x 256 32.5 -> 33.9;
+// seven portions of some 1100 tokens with rotary embedding and cache write 260 -> 221; e4m3 cache, 2 x 1512 on 368: 267 -> 214.
+// What bounds long prompts now is power: 3650 cycles a step (2112 of them MFMA) at 1.9 GHz, before 5000 at 2.4; the products alone,
+// without any softmax, take 241 us of the 313 at 1.8 GHz.  The two waves of a SIMD taking turns at products and softmax of whole tiles
+// (two barriers a tile) were at 304 on the long prompt, 289 and 66 on the next two, and slower on short ones (16 x 256 33.8, 9 x 138 with 64 heads 22.6
+// where this form takes 21.3).
+//
 // Lane maps (l = lane, c = l & 31, h = l >> 5), 32x32x16:
 //   A: row c, k = 8h + j        B: k = 8h + j, column c        C: row (r&3) + 8(r>>2) + 4h, column c
-// Scores:  S[kb][r] = key 32kb + (r&3) + 8(r>>2) + 4h  of query column c.
-// P.V:     k-step t of a tile (16 keys) takes registers 8(t&1)..+7 of block t>>1; element j of lane
-//          half h is key 16t + 8(j>>2) + 4h + (j&3): two 4-key granules, numbers 4t + h and 4t + 2 + h.
+// Scores:  row i of a block is key_of_row(i) (bits 2 and 3 of i change places), so register r of block kb is
+//          key 32kb + 16(r>>3) + 8h + (r&7) of query column c.
+// P.V:     k-step t of a tile (16 keys) takes registers 8(t&1)..+7 of block t>>1: keys 16t + 8h + j.
 // LDS:     K image  [key][16 pieces of 16 B], piece p of key k stored at p ^ (k & 15);
-//          V image  [d][8 slots of 16 B]: slot 2t + h holds granules 4t + h and 4t + 2 + h (one
-//          ds_read_b128 = one P.V operand), stored at slot ^ ((d >> 1) & 7); the two halves of a
-//          16-byte piece of the cache row (granules 2p, 2p + 1) go to slots 2(p>>1) and 2(p>>1) + 1.
+//          V image  [16-key part][d][2 pieces of 16 B], piece p of row d stored at p ^ ((d >> 4) & 1).
+//          Any 16 lanes that a 16-byte read serves together (rows 0-3, 12-15, 20-27 or the others) touch all 64 banks.
 #include "attention.h"
+#include <climits>
 #include <type_traits>
 
 namespace {
@@ -57,27 +80,61 @@ __device__ __forceinline__ float pair_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-#ifndef PW_GLOAD_LATE
-#define PW_GLOAD_LATE 1
-#endif
 constexpr int WD = 128;              // head size
 constexpr int KT = 64;               // keys per tile
 constexpr int K_BYTES = KT * 256;    // one K image
 constexpr int V_BYTES = WD * 128;    // one V image
+constexpr int RING = 4;              // tiles of either in LDS
+constexpr float LAG = 8.f;           // powers of two that a column's maximum may stay behind
+
+__device__ __forceinline__ int key_of_row(int i) { return (i & 19) | ((i & 4) << 1) | ((i & 8) >> 1); }
+
+// the sum of two 16-bit weights and c, in fp32
+__device__ __forceinline__ float dot_one(bf16_t a, bf16_t b, float c) {
+  typedef bf16_t v2 __attribute__((ext_vector_type(2)));
+  return __builtin_amdgcn_fdot2_f32_bf16(v2{a, b}, v2{(bf16_t)1.f, (bf16_t)1.f}, c, false);
+}
+__device__ __forceinline__ float dot_one(f16_t a, f16_t b, float c) {
+  typedef f16_t v2 __attribute__((ext_vector_type(2)));
+  return __builtin_amdgcn_fdot2(v2{a, b}, v2{(f16_t)1.f, (f16_t)1.f}, c, false);
+}
+
+// c += a b, in place: with the builtin, whose result may lie elsewhere, the compiler keeps two copies of the 64 sums across the branches
+// of a step and spills the queries (300 bytes).  It does not look into the statement, so the wait between an operand's last vector
+// instruction and the MFMA stands here, and settle() stands between these and what reads or scales the sums.
+__device__ __forceinline__ void mfma_to(f32x16& c, bf16x8 a, bf16x8 b) {
+  asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void mfma_to(f32x16& c, f16x8 a, f16x8 b) {
+  asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void settle(f32x16 (&c)[4]) {
+  asm volatile("s_nop 15\n\ts_nop 15" : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3]));
+}
+
+// Twice 16 bytes a lane from a buffer to LDS, at dst + 16 * lane.  A statement of its own: told of the copy, the compiler would wait for
+// all of them before the next LDS read, although they fill another tile of the ring.  Counted in the kernel's loop.
+typedef int buf_t __attribute__((ext_vector_type(4)));
+// (m0, then two copies: the second reads `step` bytes and 1024 more of voff1 and lands 1024 bytes further on)
+__device__ __forceinline__ void copy16x2(buf_t buf, unsigned voff0, unsigned voff1, unsigned step, unsigned dst) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 1\n\tbuffer_load_dwordx4 %1, %3, 0 offen lds\n\tbuffer_load_dwordx4 %2, %3, %4 offen offset:1024 lds"
+               ::"s"(dst), "v"(voff0), "v"(voff1), "s"(buf), "s"(step) : "memory", "m0");
+}
+// `bytes` from a page's head on; loads past them bring zeros
+__device__ __forceinline__ buf_t page_buffer(uint64_t head, unsigned page, unsigned page_bytes, unsigned bytes) {
+  const uint64_t a = head + (uint64_t)page * page_bytes;
+  return buf_t{(int)a, (int)(a >> 32) & 0xffff, (int)bytes, 0x00027000};
+}
 
 template <typename T, int BS, bool F8, bool GENERAL>
-__global__ __launch_bounds__(512) void paged_prefill_wide_kernel(AttnParams p, int ntiles, int levels) {
+__global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p, int ntiles, int levels) {
   using V8 = typename Vec<T>::v8;
   using V4 = typename Vec<T>::v4;
   using CT = typename KVElem<T, F8>::type;
   constexpr int D = WD;
-  constexpr int PPB = BS / 8;          // 16-byte V pieces per d-row of one cache block
-  __shared__ __attribute__((aligned(16))) unsigned char smem[2 * K_BYTES + 2 * V_BYTES];
-  unsigned char* const sKb = smem;
-  unsigned char* const sVb = smem + 2 * K_BYTES;
+  __shared__ __attribute__((aligned(16))) unsigned char smem[RING * (K_BYTES + V_BYTES)];
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c32 = lane & 31, hi = lane >> 5;
   const int G = p.Hq / p.Hkv;
   const int kvh = blockIdx.x % p.Hkv;
@@ -144,6 +201,10 @@ __global__ __launch_bounds__(512) void paged_prefill_wide_kernel(AttnParams p, i
     full_hi = min(full_hi, __shfl_xor(full_hi, o, 64));
     full_lo = max(full_lo, __shfl_xor(full_lo, o, 64));
   }
+  wave_hi = __builtin_amdgcn_readfirstlane(wave_hi);
+  wave_lo = __builtin_amdgcn_readfirstlane(wave_lo);
+  full_hi = __builtin_amdgcn_readfirstlane(full_hi);
+  full_lo = __builtin_amdgcn_readfirstlane(full_lo);
   // workgroup-uniform key range (all waves take part in every tile copy)
   const int wg_hi = p.causal ? ctx + qt_end : seq_len;
   int wg_lo = p.window > 0 ? max(0, ctx + q0 + 1 - p.window) : 0;
@@ -156,61 +217,77 @@ __global__ __launch_bounds__(512) void paged_prefill_wide_kernel(AttnParams p, i
   const unsigned v_blk_stride = (unsigned)(p.Hkv >> p.v_shift) * D * BS;     // per V cache block (fewer heads when shared)
   const unsigned k_head = (unsigned)kvh * BS * D, v_head = (unsigned)(kvh >> p.v_shift) * D * BS;
 
-  // ---- copy step: 1024 K pieces and 1024 V pieces of 16 bytes per tile, two of each per thread ----
-  // K piece pi: key = pi >> 4, piece = pi & 15.   V piece pi: cache block j = pi / (128 * PPB) of the tile,
-  // d = (pi / PPB) & 127, piece inside the block row = pi % PPB (consecutive threads read consecutive memory).
-  int k_key[2], k_dst[2], v_tok[2], v_dst[2], v_dst2[2];
-  unsigned k_src[2], v_src[2];
+  // ---- copies: wave w takes keys 8 w .. 8 w + 7 of a tile's K and half of the value rows of its 16-key part w / 2, so one page ----
+  const int part = wave >> 1, in_page = 16 * part % BS;
+  // (in two pieces of 1 KB; the second's rows lie 4 and 32 further on, and a K row's pieces change with bit 2 of the key)
+  const int key0 = 8 * (wave & 1) + (lane >> 4), d0 = 64 * (wave & 1) + (lane >> 1);
+  const unsigned k_off = (unsigned)(in_page + key0) * D + (((lane & 15) ^ key0) << 3);         // elements, from the page's head
+  const unsigned v_off = (unsigned)d0 * BS + in_page + (((lane & 1) ^ ((d0 >> 4) & 1)) << 3);
+  constexpr int K_STEP = 4 * D, V_STEP = 32 * BS;
+  const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
+  // page numbers of this wave's part, of 64 tiles at a time
+  const int n = max(kt_hi - kt_lo, 0);               // tiles of this workgroup
+  int pages = 0;
+  auto fetch_pages = [&](int t) {
+    pages = bt[max(min(((kt_lo + t + lane) * KT + 16 * part) / BS, nblk_valid - 1), 0)];
+    __builtin_amdgcn_s_waitcnt(0x0f70);              // vmcnt(0), here and not behind the branch, where it would be waited for in every step
+  };
+  auto page_of = [&](int t) { return __builtin_amdgcn_readlane(pages, t & 63); };
+  auto pages_for = [&](int t) {                      // before page_of(t), for every t in turn
+    if ((t & 63) == 0) fetch_pages(t);
+  };
+  int page = 0;                                      // of the K tile that was copied last: V's turn is a batch later
+  const uint64_t k_base = (uint64_t)(kc + k_head), v_base = (uint64_t)(vc + v_head);      // of this kv head in page 0
+  const unsigned k_page = blk_stride * sizeof(CT), v_page = v_blk_stride * sizeof(CT);
+  // an e4m3 cache is widened on its way: a batch waits in registers for a step and is written by commit()
+  u32x2 rk[F8 ? 2 : 1], rv[F8 ? 2 : 1];
+  auto copy_k = [&](int page, int slot, bool exists) {
+    if constexpr (F8) {
+      if (exists)
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int pi = tid + 512 * i;
-    const int key = pi >> 4, pc = pi & 15;
-    k_key[i] = key;
-    k_src[i] = k_head + (unsigned)(key % BS) * D + pc * 8;
-    k_dst[i] = key * 256 + 16 * (pc ^ (key & 15));
-    const int pin = pi % PPB, d = (pi / PPB) & 127, j = pi / (128 * PPB);
-    v_tok[i] = j * BS + pin * 8;
-    v_src[i] = v_head + (unsigned)d * BS + pin * 8;
-    const int piece = v_tok[i] >> 3;                  // 16-byte piece of the 64-key row
-    const int sl = 2 * (piece >> 1), f = (d >> 1) & 7;
-    v_dst[i] = d * 128 + 16 * (sl ^ f) + 8 * (piece & 1);
-    v_dst2[i] = d * 128 + 16 * ((sl + 1) ^ f) + 8 * (piece & 1);
-  }
-  int kblk[2], vblk[2];
-  auto bload = [&](int kt) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      kblk[i] = bt[max(min((kt * KT + k_key[i]) / BS, nblk_valid - 1), 0)];
-      vblk[i] = bt[max(min((kt * KT + v_tok[i]) / BS, nblk_valid - 1), 0)];
+        for (int i = 0; i < 2; ++i)
+          rk[i] = *reinterpret_cast<const u32x2*>(k_base + (uint64_t)(unsigned)page * k_page + i * K_STEP + (k_off ^ (32 * i)));
+    } else {
+      copy16x2(page_buffer(k_base, page, k_page, exists ? BS * D * 2 : 0), k_off * 2, (k_off ^ 32) * 2, K_STEP * 2 - 1024,
+               lds0 + slot * K_BYTES + wave * 2048);
     }
   };
-  V8 rk[2], rv[2];
-  auto gload = [&]() {
+  auto copy_v = [&](int page, int slot, bool exists) {
+    if constexpr (F8) {
+      if (exists)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      rk[i] = KVLoad<T, F8>::ld(kc + (size_t)(unsigned)kblk[i] * blk_stride + k_src[i]);
-      rv[i] = KVLoad<T, F8>::ld(vc + (size_t)(unsigned)vblk[i] * v_blk_stride + v_src[i]);
+        for (int i = 0; i < 2; ++i)
+          rv[i] = *reinterpret_cast<const u32x2*>(v_base + (uint64_t)(unsigned)page * v_page + i * V_STEP + v_off);
+    } else {
+      copy16x2(page_buffer(v_base, page, v_page, exists ? BS * D * 2 : 0), v_off * 2, v_off * 2, V_STEP * 2 - 1024,
+               lds0 + RING * K_BYTES + slot * V_BYTES + wave * 2048);
     }
   };
-  auto sstore = [&](int buf) {
+  auto commit_k = [&](int slot) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      *reinterpret_cast<V8*>(sKb + buf * K_BYTES + k_dst[i]) = rk[i];
-      V4 a, b;
+    for (int i = 0; i < 2; ++i)
+      *reinterpret_cast<V8*>(smem + slot * K_BYTES + wave * 2048 + i * 1024 + lane * 16) = KVLoad<T, true>::widen(rk[F8 ? i : 0]);
+  };
+  auto commit_v = [&](int slot) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) { a[e] = rv[i][e]; b[e] = rv[i][4 + e]; }
-      *reinterpret_cast<V4*>(sVb + buf * V_BYTES + v_dst[i]) = a;
-      *reinterpret_cast<V4*>(sVb + buf * V_BYTES + v_dst2[i]) = b;
-    }
+    for (int i = 0; i < 2; ++i)
+      *reinterpret_cast<V8*>(smem + RING * K_BYTES + slot * V_BYTES + wave * 2048 + i * 1024 + lane * 16) = KVLoad<T, true>::widen(rv[F8 ? i : 0]);
+  };
+  // batch u: V of tile u and K of tile u + 1.  A tile that does not exist is copied from an empty buffer, so that all batches count alike.
+  auto batch_v = [&](int u) { copy_v(page, u & (RING - 1), u < n); };
+  auto batch_k = [&](int u) {
+    page = page_of(u + 1);
+    copy_k(page, (u + 1) & (RING - 1), u + 1 < n);
+  };
+  auto commit = [&](int u) {
+    if (u < n) commit_v(u & (RING - 1));
+    if (u + 1 < n) commit_k((u + 1) & (RING - 1));
   };
 
-  // ---- operand read addresses (bytes, buffer 0) ----
-  int k_rd[8];       // K operand of k-step s: key c32 (+32 for the second block), piece 2s + hi
-#pragma unroll
-  for (int s = 0; s < 8; ++s) k_rd[s] = c32 * 256 + 16 * ((2 * s + hi) ^ (c32 & 15));
-  int v_rd[4];       // V operand of k-step t: row d = c32 (+32 per d block: +4096 bytes), slot 2t + hi
-#pragma unroll
-  for (int t = 0; t < 4; ++t) v_rd[t] = c32 * 128 + 16 * ((2 * t + hi) ^ ((c32 >> 1) & 7));
+  // ---- operand read addresses (bytes, slot 0) ----
+  // K operand of k-step s: row c32 (+32 for the second block), piece 2s + hi, which is k_rd ^ 32 s
+  const int k_rd = key_of_row(c32) * 256 + 16 * (hi ^ (key_of_row(c32) & 15));
+  const int v_rd = RING * K_BYTES + c32 * 32 + 16 * (hi ^ (c32 >> 4));    // V operand: + 4096 a k-step, + 1024 a block of 32 rows
 
   float m = -INFINITY, l = 0.f;       // l: this lane's half of the column's sum
   if (p.sink && valid) {               // a sink: the maximum starts there, the sum with its weight of one (in one half)
@@ -226,178 +303,221 @@ __global__ __launch_bounds__(512) void paged_prefill_wide_kernel(AttnParams p, i
   const float sl2 = p.scale * 1.4426950408889634f;
   const bool far_plain = p.dist_bias != nullptr && !(p.softcap > 0.f) && p.alibi == nullptr;
 
-  // A tile is worked in two halves of 32 keys, each with its own online-softmax update, ordered so that the
-  // vector ALU and the matrix pipe have independent work inside one wave:
-  //     scores(0) . scores(1) || softmax(0) . rescale . P.V(0) || softmax(1) . rescale . P.V(1)
-  // (a || b: same basic block, no dependence).  MODE 0: no masking, scale folded into the exponent's fma;
-  // 1: causal / window masking only; 2: soft-cap, ALiBi and a distance-bias table as well (its own kernel instance, GENERAL, so
-  // that the common instance does not pay for its registers).
-  f32x16 S[2];
-  auto qk_half = [&](int buf, int kb) {
-    const unsigned char* kb_ = sKb + buf * K_BYTES + kb * 8192;
+  f32x16 S[2];                                       // scores and weights of a tile's two blocks
+  V8 pb[2][2];
+  // ---- products of a half step, with the operands read AHEAD of them: scores of block kb of the tile in K slot ks (bit 0 of `what`), P.V
+  // of block vb of the tile in V slot vs (bit 1).  Where both are there they alternate, so that no MFMA waits for the one before it. ----
+  constexpr int AHEAD = 8;                           // (a divisor of 16)
+  V8 fr[AHEAD];
+  auto read = [&](int i, int what, int ks, int kb, int vs, int vb) {
+    const int j = what == 3 ? i >> 1 : i;
+    if (what == 1 || (what == 3 && (i & 1) == 0))
+      fr[i % AHEAD] = *reinterpret_cast<const V8*>(smem + ((ks * K_BYTES + k_rd) ^ (32 * j)) + kb * 8192);
+    else
+      fr[i % AHEAD] = *reinterpret_cast<const V8*>(smem + vs * V_BYTES + v_rd + (2 * vb + (j >> 2)) * 4096 + (j & 3) * 1024);
+  };
+  auto product = [&](int i, int what, int kb, int vb) {
+    const int j = what == 3 ? i >> 1 : i;
+    if (what == 1 || (what == 3 && (i & 1) == 0)) {
+      if (j == 0)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) S[kb][r] = 0.f;
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      const V8 a = *reinterpret_cast<const V8*>(kb_ + k_rd[s]);
-      S[kb] = Mfma32<V8>::run(a, qf[s], S[kb]);
+        for (int r = 0; r < 16; ++r) S[kb][r] = 0.f;
+      S[kb] = Mfma32<V8>::run(fr[i % AHEAD], qf[j], S[kb]);
+    } else {
+      mfma_to(acc[j & 3], fr[i % AHEAD], pb[vb][j >> 2]);
     }
   };
-  auto softmax_half = [&](int tb, int kb, V8 (&pb)[2], auto mode) -> float {
-    constexpr int MODE = decltype(mode)::value;
-    float mx = -INFINITY;
-    f32x4 bq[4];                                   // MODE 2: the biases of this lane's four runs of four keys
-    if constexpr (MODE == 2) {
+  // blocks of this wave's range, and those of them that need no mask (wave-uniform)
+  const int key_lo = kt_lo * KT, blocks = 2 * n;
+  const int a_lo = wave_hi > wave_lo ? max((wave_lo - key_lo) >> 5, 0) : blocks, a_hi = min((wave_hi + 31 - key_lo) >> 5, blocks);
+  const int w_lo = (full_lo + 31 - key_lo) >> 5, w_hi = (full_hi - key_lo) >> 5;
+  const int f_hi = GENERAL ? (far_plain ? (full_hi - p.dist_far - key_lo) >> 5 : INT_MIN) : 0;
+  auto active = [&](int h) { return h >= a_lo && h < a_hi; };
+  // ---- softmax of a block in slices.  Before it, sm_mask: what a block needs beside the scale, which is otherwise folded into the
+  // exponent's fma: causal and window masks; in the GENERAL instance (of its own, so that the common one does not pay for its
+  // registers) soft cap, ALiBi and a distance-bias table as well, of which only the last value remains, as a constant of that
+  // fma, for blocks at least dist_far behind every column. ----
+  float mx, alpha, off, ps[2], mul = sl2, add = 0.f;
+  bool move;
+  auto sm_mask = [&](int h, int kb) {
+    const bool whole = h >= w_lo && h < w_hi;
+    if (GENERAL) {
+      const bool far = whole && h < f_hi;
+      mul = far ? sl2 : 1.f;
+      add = far ? bfar2 : 0.f;
+      if (far) return;
+    } else if (whole) return;
+    const int tb = key_lo + 32 * h, left = limit - (tb + 8 * hi), skip = lower - (tb + 8 * hi);      // key k of this lane's: skip <= k < left
 #pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        bq[q4] = f32x4{0, 0, 0, 0};
-        // keys tb + 8 q4 + 4 hi + (0 .. 3) sit limit - 1 - key behind the query: ascending distances from the last
-        if (bias_col) bq[q4] = dist_bias4(bias_col, limit - 1 - (tb + 8 * q4 + 4 * hi + 3), p.dist_far);
-      }
-    }
+    for (int q = 0; q < 4; ++q) {
+      const int key0 = 16 * (q >> 1) + 4 * (q & 1);
+      f32x4 bq = {0, 0, 0, 0};                       // the biases of this run of four keys
+      // keys k .. k + 3 sit limit - 1 - key behind the query: ascending distances from the last
+      if (GENERAL && bias_col) bq = dist_bias4(bias_col, left - 1 - (key0 + 3), p.dist_far);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      float x = S[kb][r];
-      if constexpr (MODE == 1 || MODE == 2) {
-        const int tok = tb + (r & 3) + 8 * (r >> 2) + 4 * hi;
-        if constexpr (MODE == 2) {
+      for (int r = 4 * q; r < 4 * q + 4; ++r) {
+        const int key = key0 + (r & 3);
+        float x = S[kb][r];
+        if constexpr (GENERAL) {
           x *= p.scale;
           if (p.softcap > 0.f) x = p.softcap * fast_tanh(x / p.softcap);
-          x += slope * (float)(tok - (limit - 1));
-          x += bq[r >> 2][3 - (r & 3)];
+          x += slope * (float)(key - (left - 1));
+          x += bq[3 - (r & 3)];
           x *= 1.4426950408889634f;
         }
-        x = (tok < limit && tok >= lower) ? x : -INFINITY;
-        S[kb][r] = x;
+        S[kb][r] = (key < left && key >= skip) ? x : -INFINITY;
       }
-      mx = fmaxf(mx, x);
     }
-    // MODE 3: an unmasked tile at least dist_far behind every column, no soft cap, no ALiBi: the table's last value
-    // joins the exponent's fma as a constant
-    const float mul = MODE == 2 ? 1.f : sl2;
-    float off = -INFINITY;
-    if constexpr (MODE == 3) mx = fmaf(mx, sl2, bfar2);
-    else if constexpr (MODE != 2) mx *= sl2;          // the scale is positive
-    mx = pair_max(mx);
-    const float m_new = fmaxf(m, mx);
-    const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-    const float alpha = fexp2(m - m_use);
-    m = m_new;
-    off = MODE == 3 ? bfar2 - m_use : -m_use;
-    float ps = 0.f;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float e = fexp2(fmaf(S[kb][8 * t + j], mul, off));
-        ps += e;
-        pb[t][j] = (T)e;
-      }
-    l = l * alpha + ps;
-    return alpha;
   };
-  auto rescale = [&](float alpha) {
-    if (__any(alpha != 1.f)) {          // the running maximum settles early: most tiles need no rescale
+  auto sm_max = [&](int kb, int q) {                  // quarter q of the maximum: four keys
+    if (q == 0) mx = -INFINITY;
+#pragma unroll
+    for (int r = 4 * q; r < 4 * q + 4; ++r) mx = fmaxf(mx, S[kb][r]);
+  };
+  auto sm_move = [&] {
+    mx = pair_max(GENERAL ? fmaf(mx, mul, add) : mx * mul);       // the scale is positive
+    move = mx > m + LAG;
+    alpha = move ? fexp2(m - mx) : 1.f;
+    m = move ? mx : m;
+    off = (GENERAL ? add : 0.f) - (m == -INFINITY ? 0.f : m);
+    ps[0] = ps[1] = 0.f;
+  };
+  auto sm_exp = [&](int kb, int k) {                  // weights 2 k and 2 k + 1 of the lane's 16
+    const int t = k >> 2, j = 2 * (k & 3);
+    pb[kb][t][j] = (T)fexp2(fmaf(S[kb][2 * k], mul, off));
+    pb[kb][t][j + 1] = (T)fexp2(fmaf(S[kb][2 * k + 1], mul, off));
+    ps[k & 1] = dot_one(pb[kb][t][j], pb[kb][t][j + 1], ps[k & 1]);
+  };
+  auto sm_end = [&] {                                 // (the sums hold the blocks before this one)
+    if (__any(move)) {
+      l *= alpha;
+      settle(acc);
 #pragma unroll
       for (int db = 0; db < 4; ++db)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
+      settle(acc);
     }
+    l += ps[0] + ps[1];
   };
-  auto pv_half = [&](int buf, int kb, const V8 (&pb)[2]) {
-    const unsigned char* vb_ = sVb + buf * V_BYTES;
-#pragma unroll
-    for (int db = 0; db < 4; ++db) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const V8 a = *reinterpret_cast<const V8*>(vb_ + db * 4096 + v_rd[2 * kb + t]);
-        acc[db] = Mfma32<V8>::run(a, pb[t], acc[db]);
-      }
-    }
+
+  auto step_end = [&] {
+    if (F8) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");       // all but the last batch have landed
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
   };
-  // request for tile t+2 (and the block numbers of tile t+3)
-  auto issue_next = [&](int kt) {
-    if (kt + 2 < kt_hi) gload();
-    if (kt + 3 < kt_hi) bload(kt + 3);
-  };
-  auto tile_compute = [&](int kt, int buf, auto mode) {
-    constexpr int MODE = decltype(mode)::value;
-    const int tb0 = kt * KT;
-    V8 p0[2], p1[2];
-    // second half wholly above every column's causal limit (diagonal tiles): nothing to do for it
-    const bool second = MODE != 1 || tb0 + 32 < wave_hi;
-    // The probabilities are pinned before each rescale branch (otherwise their exponentials sink behind
-    // it, out of the block that holds the products they should overlap), and in the unmasked mode the
-    // scheduler is told the interleave: one MFMA, then a slice of the softmax.
-    auto pin = [](V8 (&pb)[2]) { asm volatile("" : "+v"(pb[0]), "+v"(pb[1])); };
-    auto interleave = [] {
-      if constexpr (MODE == 0 || MODE == 3) {
+  // half step h, whose block is number b of tile t: block h + 1 lies in K slot ks, block h - 1 in V slot vs
+  auto half_full = [&](int h, auto b_, int ks, int vs, int ks_next, int vs_next, auto extra) {       // all three parts, interleaved
+    constexpr int b = decltype(b_)::value;
+    sm_mask(h, b);
+    // (empty statements keep a slice's results in its place: otherwise the exponentials sink behind the branch of sm_end)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);     // MFMA
-          __builtin_amdgcn_sched_group_barrier(0x002, 11, 0);    // VALU
+    for (int i = 0; i < 16; ++i) {
+      product(i, 3, 1 - b, 1 - b);
+      // the first operands of the next half step as well
+      if (i + AHEAD < 16) read(i + AHEAD, 3, ks, 1 - b, vs, 1 - b);
+      else read(i + AHEAD - 16, 3, ks_next, b, vs_next, b);
+      if (i == 1 || i == 2) {                          // (the last scores left the matrix pipe a while ago)
+        sm_max(b, 2 * (i - 1));
+        sm_max(b, 2 * (i - 1) + 1);
+        asm volatile("" : "+v"(mx));
+      } else if (i == 3) {
+        sm_move();
+        asm volatile("" : "+v"(off), "+v"(alpha));
+      } else if (i > 3) {
+#pragma unroll
+        for (int k = (i - 4) * 8 / 12; k < (i - 3) * 8 / 12; ++k) {
+          sm_exp(b, k);
+          asm volatile("" : "+v"(ps[k & 1]));
         }
       }
+      extra(i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    sm_end();
+  };
+  auto half_parts = [&](int h, auto b_, int ks, int vs) {       // the parts that exist, one after another
+    constexpr int b = decltype(b_)::value;
+    auto products = [&](auto what_) {
+      constexpr int what = decltype(what_)::value;
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i) read(i, what, ks, 1 - b, vs, 1 - b);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        product(i, what, 1 - b, 1 - b);
+        if (i + AHEAD < 8) read(i + AHEAD, what, ks, 1 - b, vs, 1 - b);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     };
-    qk_half(buf, 0);
-    if constexpr (MODE == 0 || MODE == 3) __builtin_amdgcn_sched_barrier(0);
-    if (second) qk_half(buf, 1);
-#if PW_GLOAD_LATE
-    issue_next(kt);
-#endif
-    const float a0 = softmax_half(tb0, 0, p0, mode);
-    pin(p0);
-    interleave();
-    rescale(a0);
-    pv_half(buf, 0, p0);
-    if (second) {
-      const float a1 = softmax_half(tb0 + 32, 1, p1, mode);
-      pin(p1);
-      interleave();
-      rescale(a1);
-      pv_half(buf, 1, p1);
+    if (active(h + 1)) products(std::integral_constant<int, 1>{});
+    if (active(h - 1)) products(std::integral_constant<int, 2>{});
+    if (active(h)) {
+      sm_mask(h, b);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) sm_max(b, q);
+      sm_move();
+#pragma unroll
+      for (int k = 0; k < 8; ++k) sm_exp(b, k);
+      sm_end();
     }
   };
+  constexpr std::integral_constant<int, 0> first{};
+  constexpr std::integral_constant<int, 1> second{};
+  auto step_copies = [&](int t) {                    // batch t + 2 (t + 3 into registers)
+    const int u = F8 ? t + 3 : t + 2;
+    if (F8) commit(t + 2);
+    pages_for(u + 1);
+    batch_v(u);
+    batch_k(u);
+  };
+  const int full_first = (a_lo + 2) >> 1, full_end = (a_hi - 1) >> 1;       // tiles whose three parts exist in both half steps
 
-  // Tile t is consumed from LDS buffer t & 1.  Tile t+1 was requested from memory one iteration earlier and
-  // sits in registers: it moves into the other buffer at the START of iteration t (nobody reads that
-  // buffer: every wave passed the barrier that ended iteration t-1), which frees the registers for the
-  // request of tile t+2 -- every load has a whole iteration to land before anything waits for it.
-  if (kt_lo < kt_hi) {
-    bload(kt_lo);
-    gload();
-    if (kt_lo + 1 < kt_hi) bload(kt_lo + 1);
-    sstore(0);
-    if (kt_lo + 1 < kt_hi) gload();
-    if (kt_lo + 2 < kt_hi) bload(kt_lo + 2);
-  }
-  __syncthreads();
-  for (int kt = kt_lo, buf = 0; kt < kt_hi; ++kt, buf ^= 1) {
-    const int tb0 = kt * KT;
-    const bool active = tb0 < wave_hi && tb0 + KT > wave_lo;   // wave-uniform: tile inside this wave's key range
-    if (kt + 1 < kt_hi) sstore(buf ^ 1);
-#if !PW_GLOAD_LATE
-    issue_next(kt);
-#endif
-    __builtin_amdgcn_sched_barrier(0);
-    if (!active) {
-#if PW_GLOAD_LATE
-      issue_next(kt);
-#endif
-    } else {
-      if constexpr (GENERAL) {
-        if (far_plain && tb0 + KT <= full_hi - p.dist_far && tb0 >= full_lo)
-          tile_compute(kt, buf, std::integral_constant<int, 3>{});
-        else
-          tile_compute(kt, buf, std::integral_constant<int, 2>{});
-      } else {
-        if (tb0 + KT <= full_hi && tb0 >= full_lo) tile_compute(kt, buf, std::integral_constant<int, 0>{});
-        else tile_compute(kt, buf, std::integral_constant<int, 1>{});
-      }
+  if (n > 0) {
+    // K tile 0, batches 0 and 1; an e4m3 cache: and the batch that step 0 commits
+    pages_for(0);
+    page = page_of(0);
+    copy_k(page, 0, true);
+    if (F8) commit_k(0);
+    for (int u = 0; u < (F8 ? 3 : 2); ++u) {
+      batch_v(u);
+      batch_k(u);
+      if (F8 && u < 2) commit(u);
     }
-    __syncthreads();
+    step_end();                                      // all but batch 1 have landed
+    if (active(0)) half_parts(-1, second, 0, 0);
+    for (int t = 0; t < n; ++t) {
+      if (t >= full_first && t < full_end) {
+        // K tiles t and t + 1 and V tiles t - 1 and t are there throughout step t, and the next step's first operands with them
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+          read(i, 3, t & (RING - 1), 1, (t - 1) & (RING - 1), 1);
+          __builtin_amdgcn_sched_barrier(0);         // in the loop's own order: the loop's first wait is for the oldest alone
+        }
+        for (; t < full_end; ++t) {
+          const int s0 = t & (RING - 1), s1 = (t + 1) & (RING - 1);
+          if (F8) step_copies(t);
+          else pages_for(t + 3);
+          half_full(2 * t, first, s0, (t - 1) & (RING - 1), s1, s0, [&](int i) {
+            if (!F8 && i == 6) batch_v(t + 2);
+            if (!F8 && i == 11) batch_k(t + 2);
+          });
+          half_full(2 * t + 1, second, s1, s0, s1, s0, [](int) {});
+          step_end();
+        }
+      }
+      step_copies(t);
+      half_parts(2 * t, first, t & (RING - 1), (t - 1) & (RING - 1));
+      half_parts(2 * t + 1, second, (t + 1) & (RING - 1), t & (RING - 1));
+      step_end();
+    }
+    if (active(2 * n - 1)) half_parts(2 * n, first, 0, (n - 1) & (RING - 1));
   }
 
+  settle(acc);
   l = pair_sum(l);
   if (col_off < 0) return;
   const float inv = l > 0.f ? p.v_scale / l : 0.f;
