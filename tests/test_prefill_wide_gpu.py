@@ -173,3 +173,14 @@ def test_unaligned_caches_take_the_four_wave_form():
     got = torch.empty_like(q)
     ops.paged_attention_prefill(got, q, *moved, bt, sl, qsl, scale)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("lens", [[300], [64] * 16, [70, 500, 70, 500, 1, 129], [90, 31, 200] * 5 + [7], [90, 31, 200] * 6, [1000] + [1] * 20])
+@pytest.mark.parametrize("bound", [0, 1])
+def test_wide_prefill_order_of_the_tiles(lens, bound):
+    """Sequences of about one length, up to 16 of unlike lengths (sorted; with equal ones among them), more than 16; with and
+    without the longest query run from the host: every tile of every sequence once."""
+    q, kc, vc, bt, sl, qsl = _paged_problem([n + 40 * (i % 3) for i, n in enumerate(lens)], lens, 16, 2, 128, 16, torch.bfloat16)
+    out = torch.full_like(q, float("nan"))
+    ops.paged_attention_prefill(out, q, kc, vc, bt, sl, qsl, 0.09, max_q_len=bound * max(lens))
+    torch.testing.assert_close(out.float(), R.paged_attention(q, kc, vc, bt, sl, qsl, 0.09).float(), **tol(torch.bfloat16))

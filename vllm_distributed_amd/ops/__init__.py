@@ -320,7 +320,7 @@ def paged_attention_prefill(out, q, k_cache, v_cache, block_table, seq_lens, q_s
     all ``seq_lens[s]`` keys of its sequence (encoder models, the shared-prefix pass of cascade
     attention).  ``return_lse``: also return the log-sum-exp [Hq, T] (natural log) of every row.
     ``max_q_len``: the longest query run of the batch when the caller knows it on the host (0 = unknown);
-    the wide kernel then starts the longest causal tiles of all sequences first.  ``max_kv_len``: the most keys of a
+    the wide kernel then knows how many tiles a sequence has at most.  ``max_kv_len``: the most keys of a
     sequence when the caller knows it on the host (0: what the block table can hold); few query rows over long
     sequences are cut along their keys by it.  A caller whose table is much wider than its sequences names it: two prompts of
     100 tokens, 32 / 8 heads of 128, take 10 us with it and 20 under a table of 512 pages without."""

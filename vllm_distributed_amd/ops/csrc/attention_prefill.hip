@@ -16,8 +16,7 @@
 //     those eight registers eight consecutive keys, so V needs no regrouping;
 //   * so 16-bit K and V go global -> LDS without passing registers, one page number (scalar) for all that a wave copies of a tile,
 //     into rings of four tiles;
-//   * workgroup id -> (kv head = id mod Hkv, query tile descending): with 8 kv heads every XCD
-//     keeps one head's keys in its L2, and the longest causal tiles start first.
+//   * workgroup id -> (kv head = id mod Hkv, query tile): with 8 kv heads every XCD keeps one head's keys in its L2.
 //
 // Schedule.  Scores, softmax and P.V of one key depend on each other, so a half step works on three blocks of 32 keys at once:
 //   half step h: scores of block h + 1 and P.V of block h - 1 (16 MFMAs), and between them, in slices, the softmax of block h.
@@ -36,7 +35,7 @@
 //
 // Measured (MI355X, bf16, 32 / 8 heads, attention alone; before: one barrier a tile, products and softmax of a tile one after the other, K
 // and V through registers): 2048 tokens on 8192 keys 361 -> 313 us, 2 x 4096 331 -> 291, 2048 82 -> 65, 8 x 1024 118 -> 107, 16 x 256 32.5 -> 33.9;
-// seven portions of some 1100 tokens with rotary embedding and cache write 260 -> 221; e4m3 cache, 2 x 1512 on 368: 267 -> 214.
+// seven portions of some 1100 tokens with rotary embedding and cache write 260 -> 221 (208 in the order of tiles of launch_bs); e4m3 cache, 2 x 1512 on 368: 267 -> 214.
 // What bounds long prompts now is power: 3650 cycles a step (2112 of them MFMA) at 1.9 GHz, before 5000 at 2.4; the products alone,
 // without any softmax, take 241 us of the 313 at 1.8 GHz.  The two waves of a SIMD taking turns at products and softmax of whole tiles
 // (two barriers a tile) were at 304 on the long prompt, 289 and 66 on the next two, and slower on short ones (16 x 256 33.8, 9 x 138 with 64 heads 22.6
@@ -85,6 +84,7 @@ constexpr int KT = 64;               // keys per tile
 constexpr int K_BYTES = KT * 256;    // one K image
 constexpr int V_BYTES = WD * 128;    // one V image
 constexpr int RING = 4;              // tiles of either in LDS
+constexpr int SORTED = 16;           // sequences that workgroups sort by length
 constexpr float LAG = 8.f;           // powers of two that a column's maximum may stay behind
 
 __device__ __forceinline__ int key_of_row(int i) { return (i & 19) | ((i & 4) << 1) | ((i & 8) >> 1); }
@@ -137,19 +137,34 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c32 = lane & 31, hi = lane >> 5;
   const int G = p.Hq / p.Hkv;
-  const int kvh = blockIdx.x % p.Hkv;
-  int seq, q0;
-  if (levels > 0) {
-    // Host knows the longest query run: workgroup rank r -> (level j = r / S counted from the END of every
-    // sequence, sequence r % S).  The longest causal tiles of all sequences start first, and no search.
-    const int r = blockIdx.x / p.Hkv;
-    seq = r % p.num_seqs;
-    const int n_s = (p.q_start_loc[seq + 1] - p.q_start_loc[seq] + p.q_tile - 1) / p.q_tile;
-    const int j = r / p.num_seqs;
-    if (j >= n_s) return;                   // uniform over the workgroup
-    q0 = (n_s - 1 - j) * p.q_tile;
+  const int kvh = blockIdx.x % p.Hkv, rank = blockIdx.x / p.Hkv;
+  int seq, q0, qs, q_len, seq_len;
+  if (levels > 0) {                                  // tile j from the end of every sequence, with another sequence first for each j
+    const int j = rank / p.num_seqs;
+    seq = (rank - j * p.num_seqs + j) % p.num_seqs;
+    qs = p.q_start_loc[seq];
+    q_len = p.q_start_loc[seq + 1] - qs;
+    seq_len = p.seq_lens[seq];
+    const int tiles = (q_len + p.q_tile - 1) / p.q_tile;
+    if (j >= tiles) return;                          // uniform over the workgroup
+    q0 = (tiles - 1 - j) * p.q_tile;
+  } else if (p.num_seqs <= SORTED) {                 // sequence after sequence, the one with the most keys first, each from its end
+    const int s = min(lane, p.num_seqs - 1), start = p.q_start_loc[s], end = p.q_start_loc[s + 1], len = p.seq_lens[s];
+    const int tiles = lane < p.num_seqs ? (end - start + p.q_tile - 1) / p.q_tile : 0;
+    const int place = (min(len, (1 << 26) - 1) << 4) + SORTED - 1 - s;                  // unique
+    int first = 0;                                   // rank of this lane's sequence's first tile
+#pragma unroll
+    for (int i = 0; i < SORTED; ++i)
+      first += __builtin_amdgcn_readlane(place, i) > place ? __builtin_amdgcn_readlane(tiles, i) : 0;
+    const unsigned long long hit = __ballot(lane < SORTED && rank >= first && rank < first + tiles);
+    if (hit == 0) return;                            // uniform over the workgroup
+    seq = __builtin_ctzll(hit);
+    q0 = (__builtin_amdgcn_readlane(tiles - 1 + first, seq) - rank) * p.q_tile;
+    qs = __builtin_amdgcn_readlane(start, seq);
+    q_len = __builtin_amdgcn_readlane(end, seq) - qs;
+    seq_len = __builtin_amdgcn_readlane(len, seq);
   } else {
-    const int tile = ntiles - 1 - (int)(blockIdx.x / p.Hkv);
+    const int tile = ntiles - 1 - rank;
     // tile -> sequence: the largest s whose first tile, q_start_loc[s] / q_tile + s (increasing in s), is not
     // behind this one; 64 candidates per load instead of one dependent load per bisection step
     seq = 0;
@@ -162,12 +177,12 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
       if (mask != ~0ull) break;
     }
     seq = __builtin_amdgcn_readfirstlane(seq);
-    q0 = (tile - (p.q_start_loc[seq] / p.q_tile + seq)) * p.q_tile;
+    qs = p.q_start_loc[seq];
+    q0 = (tile - (qs / p.q_tile + seq)) * p.q_tile;
+    q_len = p.q_start_loc[seq + 1] - qs;
+    seq_len = p.seq_lens[seq];
+    if (q0 >= q_len) return;                         // uniform over the workgroup
   }
-  const int qs = p.q_start_loc[seq];
-  const int q_len = p.q_start_loc[seq + 1] - qs;
-  const int seq_len = p.seq_lens[seq];
-  if (q0 >= q_len) return;                  // uniform over the workgroup
   const int ctx = seq_len - q_len;
   const int* bt = p.block_table + (long)seq * p.max_blocks;
   const int nblk_valid = (seq_len + BS - 1) / BS;
@@ -467,25 +482,37 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
   };
   constexpr std::integral_constant<int, 0> first{};
   constexpr std::integral_constant<int, 1> second{};
-  auto step_copies = [&](int t) {                    // batch t + 2 (t + 3 into registers)
-    const int u = F8 ? t + 3 : t + 2;
-    if (F8) commit(t + 2);
-    pages_for(u + 1);
-    batch_v(u);
-    batch_k(u);
+  auto step_copies = [&](int t) {                    // batch t + 2 (into registers, and t + 1 from there)
+    if (F8) commit(t + 1);
+    pages_for(t + 3);
+    batch_v(t + 2);
+    batch_k(t + 2);
   };
   const int full_first = (a_lo + 2) >> 1, full_end = (a_hi - 1) >> 1;       // tiles whose three parts exist in both half steps
 
   if (n > 0) {
-    // K tile 0, batches 0 and 1; an e4m3 cache: and the batch that step 0 commits
     pages_for(0);
-    page = page_of(0);
-    copy_k(page, 0, true);
-    if (F8) commit_k(0);
-    for (int u = 0; u < (F8 ? 3 : 2); ++u) {
-      batch_v(u);
-      batch_k(u);
-      if (F8 && u < 2) commit(u);
+    if constexpr (F8) {                              // K tile 0 and batch 0 in one trip; batch 1, which step 0 commits
+      u32x2 k0[2];
+      page = page_of(0);
+      copy_k(page, 0, true);
+      k0[0] = rk[0];
+      k0[1] = rk[1];
+      batch_v(0);
+      batch_k(0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        *reinterpret_cast<V8*>(smem + wave * 2048 + i * 1024 + lane * 16) = KVLoad<T, true>::widen(k0[i]);
+      commit(0);
+      batch_v(1);
+      batch_k(1);
+    } else {                                         // K tile 0, batches 0 and 1
+      page = page_of(0);
+      copy_k(page, 0, true);
+      for (int u = 0; u < 2; ++u) {
+        batch_v(u);
+        batch_k(u);
+      }
     }
     step_end();                                      // all but batch 1 have landed
     if (active(0)) half_parts(-1, second, 0, 0);
@@ -548,11 +575,19 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
 
 template <typename T, bool F8, bool GENERAL>
 int launch_bs(const AttnParams& p, int bs, int ntiles, hipStream_t st) {
-  // level order when the host passed the longest query run and the (level, sequence) grid is not much
-  // larger than the number of real tiles (a batch of one long and many short prompts keeps the linear order)
-  int levels = p.max_q_len > 0 ? (p.max_q_len + p.q_tile - 1) / p.q_tile : 0;
-  if ((long)levels * p.num_seqs > 2L * ntiles) levels = 0;
-  const dim3 grid((unsigned)(levels > 0 ? levels * p.num_seqs : ntiles) * p.Hkv), block(512);
+  // The order of the tiles.  The longest query run, when the host passed it, bounds the tiles of a sequence, so that a tile of every
+  // sequence in turn, the longest (causal) ones first, is a count without a search: for sequences of about one length, and for many.  Where
+  // up to 16 are of unlike lengths, that gives neighbours in time no keys to share and ties sequences to shader engines (a
+  // workgroup's number decides on its engine): these go one after another, the one with the most keys first.
+  // us, tile of every sequence / in the batch's order / sorted, 32 / 8 heads: 8 ragged of some 1000 tokens on 500 237 / 162 / 157, 4 of 2000
+  // 335 / 209 / 196, 15 of 240 on 3700 229 / 212 / 177, 7 of 1100 on 900 203 / 183 / 178; 8 equal ones of 1024 107 / - / 118, 32 of 64 14.4 / 20.7 / -.
+  const int bound = p.max_q_len > 0 ? (p.max_q_len + p.q_tile - 1) / p.q_tile : 0;
+  const long by_level = (long)bound * p.num_seqs;
+  const bool alike = (long)p.max_q_len * p.num_seqs * 15 <= (long)p.num_tokens * 16;
+  // (nor does the order matter where all tiles run at once)
+  const int levels = bound > 0 && by_level <= 2L * ntiles && (p.num_seqs > SORTED || alike || by_level * p.Hkv <= 256) ? bound : 0;
+  const long ranks = levels > 0 || (bound > 0 && by_level < ntiles) ? by_level : ntiles;
+  const dim3 grid((unsigned)(ranks * p.Hkv)), block(512);
   switch (bs) {
     case 16: hipLaunchKernelGGL((paged_prefill_wide_kernel<T, 16, F8, GENERAL>), grid, block, 0, st, p, ntiles, levels); break;
     case 32: hipLaunchKernelGGL((paged_prefill_wide_kernel<T, 32, F8, GENERAL>), grid, block, 0, st, p, ntiles, levels); break;
