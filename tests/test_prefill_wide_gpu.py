@@ -175,6 +175,21 @@ def test_unaligned_caches_take_the_four_wave_form():
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("Hq,Hkv", [(28, 4), (3, 1), (11, 1), (15, 1)])
+def test_wide_prefill_groups_that_do_not_divide_the_columns(Hq, Hkv):
+    """Columns left over belong to no token: 36 tokens of 7 heads are 252 of 256; tiles that end in the middle of a sequence."""
+    tile = 256 // (Hq // Hkv)
+    q_lens = [4 * tile, 4 * tile + 1, 2 * tile - 1, 3 * tile, 5 * tile + 7]
+    seq_lens = [n + c for n, c in zip(q_lens, [0, 100, 0, 63, 64])]
+    q, kc, vc, bt, sl, qsl = _paged_problem(seq_lens, q_lens, Hq, Hkv, 128, 16, torch.bfloat16)
+    scale = 1.0 / math.sqrt(128)
+    out = torch.full_like(q, float("nan"))
+    _, lse = ops.paged_attention_prefill(out, q, kc, vc, bt, sl, qsl, scale, return_lse=True)
+    ref, lref = R.paged_attention(q, kc, vc, bt, sl, qsl, scale, return_lse=True)
+    torch.testing.assert_close(out.float(), ref.float(), **tol(torch.bfloat16))
+    torch.testing.assert_close(lse, lref, atol=3e-3, rtol=1e-4)
+
+
 @pytest.mark.parametrize("lens", [[300], [64] * 16, [70, 500, 70, 500, 1, 129], [90, 31, 200] * 5 + [7], [90, 31, 200] * 6, [1000] + [1] * 20])
 @pytest.mark.parametrize("bound", [0, 1])
 def test_wide_prefill_order_of_the_tiles(lens, bound):

@@ -1185,6 +1185,16 @@ static long g_prefill_wide_min_wgs = 128;
 VDA_EXPORT int vda_set_prefill_variant(int v) { g_prefill_variant = v; return 0; }
 VDA_EXPORT int vda_set_prefill_wide_min_wgs(long n) { g_prefill_wide_min_wgs = n; return 0; }
 
+// Query tokens of a wide workgroup (0: the wide form does not apply to this batch).  A group that does not divide the 256 columns leaves at
+// most a sixteenth of them idle, or the 4-wave form takes it; and it has prompts of three of its tiles on average: us, 4-wave / wide,
+// 28 / 4 heads, 2 x 2161 tokens 244 / 143, 8 x 200 37.7 / 33, 24 x 150 50.6 / 48.8, 24 / 8 heads 43.3 / 34.1 (one of 1000), 226 / 160, but 40 / 8, 24 x 40 27.7 / 30.2,
+// 48 / 8 27.9 / 30.0, 28 / 4 25 x 81 on 740 75.8 / 79.2.
+static int wide_tokens(int G, int num_tokens, int num_seqs) {
+  const int tokens = 256 / G;
+  if (256 % G && (tokens * G < 240 || (long)num_tokens < 3L * tokens * num_seqs)) return 0;
+  return tokens;
+}
+
 // Into how many parts the keys of each query tile are cut (1: not at all; what lse_out and the wide form take).  max_keys: an
 // upper bound of the sequences' lengths.  Without parts a few tiles walk a long prefix alone, 32 keys in some 1.2 us:
 // 100 new tokens on 2000 of each of two, 32 / 8 heads of 64 137 us in one part, 37 in seven; 16 / 8 heads of 256 386 -> 83, 24 / 8 of 96 255 -> 57;
@@ -1196,8 +1206,8 @@ VDA_EXPORT int vda_set_prefill_wide_min_wgs(long n) { g_prefill_wide_min_wgs = n
 VDA_EXPORT int vda_prefill_parts(int num_seqs, int num_tokens, int Hq, int Hkv, int D, long max_keys) {
   if (Hkv < 1 || Hq % Hkv || Hq / Hkv > 128) return 1;
   const int G = Hq / Hkv, q_tile = (G <= prefill_cols(D) ? prefill_cols(D) : 128) / G;
-  if (D == 128 && 256 % G == 0 && (g_prefill_variant == 3 || (g_prefill_variant == 1 &&
-      (long)(num_tokens / (256 / G)) * Hkv >= g_prefill_wide_min_wgs))) return 1;
+  const int wide = D == 128 ? wide_tokens(G, num_tokens, num_seqs) : 0;
+  if (wide && (g_prefill_variant == 3 || (g_prefill_variant == 1 && (long)(num_tokens / wide) * Hkv >= g_prefill_wide_min_wgs))) return 1;
   const long wgs = (long)(num_tokens / q_tile + min(num_seqs, num_tokens)) * Hkv, steps = (max_keys + 31) / 32;
   if (wgs < 1 || wgs > 256 || steps < 16) return 1;
   const double rows = (double)num_tokens * Hq, row_part = rows * D * 8 / 4e6;                 // us
@@ -1241,8 +1251,8 @@ VDA_EXPORT int vda_paged_attention_prefill(
   // chip (one workgroup per CU); short chunks keep the 4-wave form, which cuts them into more workgroups.
   // Its copies to LDS ask for caches aligned to 16 bytes.
   const bool aligned = (((uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0;
-  if (nsplit == 1 && D == 128 && 256 % G == 0 && aligned && (g_prefill_variant == 1 || g_prefill_variant == 3)) {
-    const int wide_tile = 256 / G;
+  if (nsplit == 1 && D == 128 && wide_tokens(G, num_tokens, num_seqs) && aligned && (g_prefill_variant == 1 || g_prefill_variant == 3)) {
+    const int wide_tile = wide_tokens(G, num_tokens, num_seqs);
     const long wgs = (long)(num_tokens / wide_tile) * Hkv;
     if (g_prefill_variant == 3 || wgs >= g_prefill_wide_min_wgs) {
       p.q_tile = wide_tile;

@@ -606,7 +606,7 @@ int launch_mode(const AttnParams& p, int bs, int ntiles, hipStream_t st) {
 
 }  // namespace
 
-// p.q_tile must be 256 / (Hq / Hkv); the caller has checked D == 128 and that the group size divides 256.
+// p.q_tile must be 256 / (Hq / Hkv) (columns left over belong to no token); the caller has checked D == 128.
 int vda_launch_prefill_wide(const AttnParams& p, int block_size, int dtype, int kv_fp8, hipStream_t st) {
   const int ntiles = p.num_tokens / p.q_tile + p.num_seqs;
   if (dtype == VDA_BF16)
