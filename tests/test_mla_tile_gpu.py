@@ -172,3 +172,26 @@ def test_what_the_tiles_do_not_take(page, scale, new, total, H, fp8):
         ops.mla_attention(out, q, kc, vt, table, lens, starts, scale, max(new), splits)
         want = R.mla_attention(q, kc, vt, table, lens, starts, scale)
         torch.testing.assert_close(out.float(), want.float(), atol=12 * 2.0 ** -9, rtol=2.0 ** -8)
+
+
+def _ragged(n, mean):
+    return [max(1, int(mean * (0.25 + 1.5 * ((0.618 * i + 0.37) % 1)))) for i in range(n)]
+
+
+@pytest.mark.parametrize("S,new,prefix,H,window", [
+    (16, 1, 900, 16, 0), (17, 1, 300, 16, 0), (64, 1, 200, 128, 0), (65, 1, 200, 40, 90), (190, 1, 120, 32, 0), (260, 1, 60, 128, 0),       # decoding
+    (2, 150, 0, 128, 0), (8, 90, 200, 32, 0), (16, 30, 100, 16, 50), (17, 40, 60, 128, 0), (70, 9, 30, 128, 0), (260, 3, 20, 64, 0),      # prompts
+    (3, 5, 1500, 16, 700), (5, 12, 2000, 16, 0), (6, 3, 700, 128, 100)])                                            # blocks and pieces
+def test_every_column_block_and_piece_has_its_workgroup(S, new, prefix, H, window):
+    """Workgroups are numbered over the work that the lengths give: sorted (up to 16 sequences), two halves (up to 256), by column
+    block (sequences alike, or more); among them sequences without a new token."""
+    news = [1] * S if new == 1 else _ragged(S, new)
+    if S > 4:
+        news[1] = news[S - 2] = 0
+    total = [n + p for n, p in zip(news, _ragged(S, prefix)[::-1])] if prefix else list(news)
+    kc, vt, table, lens, starts = _batch(news, total, 16, torch.bfloat16, S)
+    q = torch.randn(sum(news), H, DK, device=DEV).to(torch.bfloat16)
+    out = torch.full((sum(news), H, DV), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ops.mla_attention(out, q, kc, vt, table, lens, starts, 192 ** -0.5, max(news), 8, window=window)
+    want = R.mla_attention(q, kc, vt, table, lens, starts, 192 ** -0.5, 1.0, window)
+    torch.testing.assert_close(out.float(), want.float(), atol=12 * 2.0 ** -9, rtol=2.0 ** -8)
