@@ -39,6 +39,8 @@ def _routing(counts, k, g):
     ([513, 0, 1, 272, 1400, 31], 2, 192, 320, False),
     ([200] * 9, 4, 576, 1088, True),                  # 9 x 9 and 9 x 3 tiles: eighths that do not come out even
     ([700, 705] * 20, 3, 128, 1152, True),            # whole rounds of 512 tiles and a rest
+    ([287, 288, 289, 320, 321, 576, 577, 865, 33, 64, 65, 96, 1153], 1, 64, 192, True),      # either side of 288 rows, and of 32 of them
+    ([224, 193, 160, 225, 97, 320], 1, 192, 320, False),      # each number of fragments
 ])
 def test_wide_tiles(monkeypatch, dt, counts, k, H, I, gated):
     monkeypatch.setenv("VDA_MOE_GROUPED_MAX_PAIRS", "0")

@@ -58,7 +58,7 @@ struct TileGemmArgs {
   const int* sorted;         // grouped: pair ids sorted by expert
   const int* tile_expert;    // grouped: expert of m-tile i
   const int* tile_beg;       // grouped: first sorted position of m-tile i
-  const int* tile_end;       // grouped: end of that expert's sorted range
+  const int* tile_end;       // grouped: end of that expert's sorted range; wide tiles: of the m-tile
   const int* num_tiles;      // grouped: number of valid m-tiles (device)
   int M;                     // dense: activation rows
   int N;                     // output columns (EPI_GATE_UP: I, the weight has 2 I rows)
@@ -313,166 +313,269 @@ __global__ __launch_bounds__(512, 1) void tile_gemm_kernel(const TileGemmArgs a)
 }
 
 // ---------------------------------------------------------------------------------------------
-// Grouped 16-bit GEMM on 256 x 256 tiles, for experts that see more than 128 rows each.  The kernel above reads 6 KB of LDS
-// operands per 16 MFMAs of a wave, from an LDS that the fill of the next steps writes meanwhile, and reaches 0.85 PFLOP/s; here a
-// wave holds 4 x 8 accumulator tiles (12 KB per 32 MFMAs) and the two waves of a SIMD take turns, one at its MFMAs while the
-// other reads fragments and issues copies.  K is walked in units of 64 elements (whole 128-byte lines per row) with two
-// LDS slots of 64 KB, a unit in two halves of K = 32:
+// Grouped 16-bit GEMM on tiles of 256 weight rows x up to 288 activation rows, for experts that see more than 128 rows each.
+// Four waves, one a SIMD, as 2 (weight rows) x 2 (activation rows): a wave holds 8 x NF accumulator tiles of 16 x 16 and reads
+// 17 KB of LDS operands per 72 MFMAs (eight waves of 4 x 8 tiles read 12 per 32, which with the fill is all that an LDS
+// delivers in that time).  K is walked in steps of 32 elements through a ring of four LDS slots:
 //
-//   R0(u): read the fragments of half 0, issue the copies of unit u + 1      C0(u): 32 MFMAs
-//   R1(u): read the fragments of half 1, wait for the copies of unit u + 1   C1(u): 32 MFMAs
+//   step k: wait for the own copies of step k + 1 and the own reads of step k; barrier; then, dealt out between the MFMAs
+//   of step k: the reads of the fragments of step k + 1 (second register set) and the copies of step k + 4
 //
-// waves 4-7 (the upper 128 activation rows) run one slot behind waves 0-3.  Write-after-read: unit u + 1 overwrites the slot
-// of unit u - 1, last read by waves 4-7 in R1(u - 1), which drains its LDS reads before the barrier that precedes
-// R0(u) of waves 0-3.  Read-after-write: every thread waits for its own copies at the end of its R1(u), before a barrier
-// that every reader of unit u + 1 passes first.  LDS image as above but with f(r) = (r >> 1) & 7: a lane reads
-// one chunk, 4 h + g, per row and half.  What bounds it is the chip's power at this density: dense products of this K run
-// at 1.1 (kernels here) to 1.4 PFLOP/s (library).
-// 8 experts 4096 x 14336, top 2, whole layer: 4099 tokens 3290 -> 2940 us (0.98 PFLOP/s with rows that exist), 3200 tokens
-// 2741 -> 2234; 16 experts 4096 x 6400, 5600 tokens 2076 -> 1746.
-template <typename T, int EPI>
-__global__ __launch_bounds__(512, 1) void moe_wide_gemm_kernel(const TileGemmArgs a) {
+// Write-after-read: the slot of step k is written after the barrier of step k, which every wave reaches with its reads of it
+// done.  Read-after-write: slot k + 1 is read after that barrier, which every wave reaches with its copies to it landed (those of
+// steps k + 2 and k + 3 may be in flight: up to three steps, 3000 cycles of MFMAs, for a copy).  K is a multiple of 64, so the steps are even.
+//
+// An expert's rows are cut into the fewest tiles of at most 288 rows, of like sizes (moe_tile_map_kernel): batches of 2048 or
+// 4096 tokens over eight experts are 256-row tiles but for a few rows, which opened tiles of their own in half of the experts.
+// NF, the 16-row fragments of a wave, is a template argument: tiles of few rows do few MFMAs.
+//
+// LDS image of a slot: [row][4 chunks of 16 bytes], chunk c of row r at c ^ wide_swz(r), on the source side of the copy.  Of a fragment read
+// the lanes of rows {0-3, 12-15} at chunk q are served with those of {4-11} at q ^ 1: with 0, 2, 3, 1 for the four rows of four they
+// touch the sixteen 16-byte columns of a 256-byte bank row once each.
+// WIDE_FIGURES
+constexpr int WIDE_ROWS = 288, WIDE_SLOT = (256 + WIDE_ROWS) * 64;
+
+// 16 bytes a lane from a buffer to LDS, at dst + 16 * lane.  As a statement of its own: told of the copy, the compiler waits for
+// all of them before the next LDS read, although they fill another slot of the ring.  Waited for by the counts in the loop.
+__device__ __forceinline__ void wide_copy(i32x4 buf, unsigned voff, int soff, unsigned dst) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               ::"s"(dst), "v"(voff), "s"(buf), "s"(soff) : "memory", "m0");
+}
+__device__ __forceinline__ i32x4 wide_buffer(const void* p) {
+  const uint64_t at = reinterpret_cast<uint64_t>(p);
+  return i32x4{__builtin_amdgcn_readfirstlane((int)(uint32_t)at), __builtin_amdgcn_readfirstlane((int)((at >> 32) & 0xffff)), -1, 0x00020000};
+}
+
+// c += a b as a statement, with the sums in accumulator registers (ACC) or, the 32 that are more than 256, in ordinary ones: left to
+// itself the compiler moves hundreds of them to and fro in each step.  It does not look into these: operands come from LDS
+// reads that the loop waits for, sums are touched again sixteen MFMAs later at the earliest, and the loop is followed by enough
+// wait states for a reader.
+template <bool ACC> __device__ __forceinline__ void wide_mfma(f32x4& c, bf16x8 a, bf16x8 b) {
+  if (ACC) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+  else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+}
+template <bool ACC> __device__ __forceinline__ void wide_mfma(f32x4& c, f16x8 a, f16x8 b) {
+  if (ACC) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+  else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+}
+
+// gate_act and gated_pair with the choice made once for four values
+__device__ __forceinline__ f32x4 gate_four(f32x4 g, int kind) {
+  auto all = [&](int k) { return f32x4{gate_act(g[0], k), gate_act(g[1], k), gate_act(g[2], k), gate_act(g[3], k)}; };
+  switch (kind) {
+    case 1: return all(1);
+    case 2: return all(2);
+    case 3: return all(3);
+    case 8: return all(8);
+    default: return all(0);
+  }
+}
+__device__ __forceinline__ f32x4 gated_four(f32x4 g, f32x4 u, int kind, float limit) {
+  if (kind == 9) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) g[i] = gated_pair(g[i], u[i], 9, limit);
+    return g;
+  }
+  return gate_four(g, kind) * u;
+}
+
+__device__ __forceinline__ int wide_swz(int r) { return (r >> 1 & 2) ^ (r & 8 ? 3 : 0); }
+
+// one tile: acc[mt][nt] = the sum over K of W fragment mt . X fragment nt, then the epilogue.  pair, tw: the pair of each row
+// of the tile and its routing weight, in LDS
+template <typename T, int EPI, int NF>
+__device__ __forceinline__ void wide_walk(const TileGemmArgs& a, uint8_t* lds, const int* pair, const float* tw, int e, int beg, int cnt,
+                                          int n0) {
   using V8 = typename Vec<T>::v8;
   using V4 = typename Vec<T>::v4;
-  constexpr int WT = 4, XT = 8, WR = 256, XR = 256;
-  constexpr int WB = WR * 128, UNIT = WB + XR * 128;
-  __shared__ __attribute__((aligned(16))) uint8_t lds[2 * UNIT];
-  int mi, ni;
-  if (!tile_of_block(min(*a.num_tiles, a.m_tiles), a.n_tiles, mi, ni)) return;
-  const int e = a.tile_expert[mi], beg = a.tile_beg[mi], cnt = min(a.tile_end[mi] - beg, XR);
+  constexpr int WT = 8, XP = 2 * NF, XC = (XP + 3) / 4, CP = 4 + XC;     // 1 KB pieces of X, and what a wave copies in a step
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
-  const int grp = wave >> 2, wn = wave & 3;
-  const int n0 = ni * (EPI == EPI_GATE_UP ? WR / 2 : WR);
+  const int wi = wave & 1, xi = wave >> 1;
   const int w_rows = EPI == EPI_GATE_UP ? 2 * a.N : a.N;
   const unsigned kbytes = (unsigned)a.K * 2u;
-  const uint8_t* wbase = reinterpret_cast<const uint8_t*>(a.w) + (long)e * a.w_expert_stride * 2;
-  const uint8_t* xbase = reinterpret_cast<const uint8_t*>(a.x);
+  const i32x4 wbuf = wide_buffer(reinterpret_cast<const uint8_t*>(a.w) + (long)e * a.w_expert_stride * 2), xbuf = wide_buffer(a.x);
+  const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
 
-  // staging roles: in round j, lane L of wave w fills LDS row 64 j + 8 w + (L >> 3), position L & 7
-  unsigned voff_w[4], voff_x[4];             // (host: both operands of an expert below 4 GiB)
+  // copies: lane L of a 1 KB piece fills row L >> 2 of its sixteen, position L & 3.  Wave w takes pieces w, w + 4, ...; where the
+  // pieces of X do not divide, the last is copied by two waves
+  unsigned voff[CP];                         // (host: both operands of an expert below 4 GiB)
+  int at[XC];
   {
-    const int lrow = 8 * wave + (lane >> 3), pos = lane & 7;
+    const int lrow = lane >> 2, chunk = ((lane & 3) ^ wide_swz(lrow)) << 4;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int rho = 64 * j + lrow;
-      int row = EPI == EPI_GATE_UP ? (rho < WR / 2 ? n0 + rho : a.N + n0 + rho - WR / 2) : n0 + rho;
-      row = min(row, w_rows - 1);
-      voff_w[j] = (unsigned)row * kbytes + ((pos ^ ((rho >> 1) & 7)) << 4);
-      const int p = a.sorted[beg + min(rho, cnt - 1)];
+      const int rho = 16 * (wave + 4 * j) + lrow;
+      const int row = EPI == EPI_GATE_UP ? (rho < 128 ? n0 + rho : a.N + n0 + rho - 128) : n0 + rho;
+      voff[j] = (unsigned)min(row, w_rows - 1) * kbytes + chunk;
+    }
+#pragma unroll
+    for (int j = 0; j < XC; ++j) {
+      const int piece = min(wave + 4 * j, XP - 1);
+      const int p = pair[min(16 * piece + lrow, cnt - 1)];
       const int xrow = EPI == EPI_DOWN ? p : p / a.top_k;
-      voff_x[j] = (unsigned)xrow * (unsigned)(a.x_stride * 2) + ((pos ^ ((rho >> 1) & 7)) << 4);
+      voff[4 + j] = (unsigned)xrow * (unsigned)(a.x_stride * 2) + chunk;
+      at[j] = 256 * 64 + piece * 1024;
     }
   }
-  const int nun = a.K >> 6;
-  auto issue = [&](int u, int slot) {
-    const long ko = (long)min(u, nun - 1) * 128;
-    uint8_t* lw = lds + slot * UNIT + wave * 1024;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) glds16(wbase + ko + voff_w[j], lw + j * 8192);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) glds16(xbase + ko + voff_x[j], lw + WB + j * 8192);
+  const int steps = a.K >> 5;
+  auto copy = [&](int k, int j) {            // piece j of step k (the last step's again beyond the end: into a slot that is free)
+    const int ko = min(k, steps - 1) * 64;
+    const unsigned slot = lds0 + (k & 3) * WIDE_SLOT;
+    if (j < 4) wide_copy(wbuf, voff[j], ko, slot + (wave + 4 * j) * 1024);
+    else wide_copy(xbuf, voff[j], ko, slot + at[j - 4]);
   };
-
-  // weight fragment mt of wave wn starts at tile row wrow(mt); with a gate half two are gate rows and two the up rows of
+  // weight fragment mt of wave column wi starts at tile row wrow(mt); with a gate half four are gate rows and four the up rows of
   // the same columns
-  auto wrow = [&](int mt) { return EPI == EPI_GATE_UP ? (mt < 2 ? 32 * wn + 16 * mt : 128 + 32 * wn + 16 * (mt - 2))
-                                                      : 64 * wn + 16 * mt; };
-  const int cpos = (g ^ ((r >> 1) & 7)) << 4;          // K half 0; half 1 is cpos ^ 64
-  const int wl = wrow(0) * 128 + r * 128, xl = WB + (128 * grp + r) * 128;
-  f32x4 acc[WT][XT];
+  auto wrow = [&](int mt) { return EPI == EPI_GATE_UP ? (mt < 4 ? 64 * wi + 16 * mt : 128 + 64 * wi + 16 * (mt - 4))
+                                                      : 128 * wi + 16 * mt; };
+  const int cpos = r * 64 + ((g ^ wide_swz(r)) << 4);
+  const int wl = wrow(0) * 64 + cpos, xl = (256 + 16 * NF * xi) * 64 + cpos;
+  f32x4 acc[WT][NF];
 #pragma unroll
   for (int mt = 0; mt < WT; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < XT; ++nt) acc[mt][nt] = f32x4{0, 0, 0, 0};
+    for (int nt = 0; nt < NF; ++nt) acc[mt][nt] = f32x4{0, 0, 0, 0};
+  V8 wf[2][WT], xf[2][NF];
+  auto read = [&](const uint8_t* slot, int i, V8 (&w)[WT], V8 (&x)[NF]) {      // fragment i of a step: the first weight rows' first
+    if (i < 4) w[i] = *reinterpret_cast<const V8*>(slot + wl + (wrow(i) - wrow(0)) * 64);
+    else if (i < 4 + NF) x[i - 4] = *reinterpret_cast<const V8*>(slot + xl + (i - 4) * 1024);
+    else w[i - NF] = *reinterpret_cast<const V8*>(slot + wl + (wrow(i - NF) - wrow(0)) * 64);
+  };
 
-  issue(0, 0);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+#pragma unroll
+    for (int j = 0; j < CP; ++j) copy(k, j);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(3 * CP) : "memory");
   __builtin_amdgcn_s_barrier();
-  if (grp == 1) __builtin_amdgcn_s_barrier();
-  // 16-row fragments of this wave's half that hold rows: an expert's last tile is cut off there (at 1025 rows an expert
-  // it holds one row in half of the experts)
-  const int frags = max(0, min(XT, (cnt - 128 * grp + 15) >> 4));
-  auto walk = [&](auto full) {
-    constexpr bool FULL = decltype(full)::value;
-    for (int u = 0; u < nun; ++u) {
-      const uint8_t* base = lds + (u & 1) * UNIT;
-      V8 wf[WT], xf[XT];
+  asm volatile("" ::: "memory");
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int cp = h ? cpos ^ 64 : cpos;
+  for (int i = 0; i < WT + NF; ++i) read(lds, i, wf[0], xf[0]);
+  for (int k0 = 0; k0 < steps; k0 += 2) {
 #pragma unroll
-        for (int nt = 0; nt < XT; ++nt)
-          if (FULL || nt < frags) xf[nt] = *reinterpret_cast<const V8*>(base + xl + cp + nt * 2048);
+    for (int h = 0; h < 2; ++h) {
+      const int k = k0 + h;
+      constexpr int OPS = WT + NF + CP, ALL = WT * NF;
+      static_assert(8 * OPS <= 14 * ALL, "two operations behind an MFMA at most");
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(2 * CP) : "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      const uint8_t* next = lds + ((k + 1) & 3) * WIDE_SLOT;
 #pragma unroll
-        for (int mt = 0; mt < WT; ++mt)
-          if (FULL || frags > 0) wf[mt] = *reinterpret_cast<const V8*>(base + wl + cp + (wrow(mt) - wrow(0)) * 128);
-        __builtin_amdgcn_sched_barrier(0);             // fragment reads first: their latency runs under the copy issue
-        if (h == 0) issue(u + 1, (u + 1) & 1);
-        if (h == 0) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_setprio(1);
+      for (int m = 0; m < ALL; ++m) {
+        const int nt = m / WT, mt = m % WT;
+        if (nt < 8) wide_mfma<true>(acc[mt][nt], wf[h][mt], xf[h][nt]);
+        else wide_mfma<false>(acc[mt][nt], wf[h][mt], xf[h][nt]);
+        // the OPS reads and copies behind the first seven eighths of the MFMAs, two at most behind one
+        auto upto = [](int m) { return (m * 8 * OPS + 7 * ALL - 1) / (7 * ALL); };
 #pragma unroll
-        for (int nt = 0; nt < XT; ++nt)
-          if (FULL || nt < frags) {
-#pragma unroll
-            for (int mt = 0; mt < WT; ++mt) acc[mt][nt] = mfma16(wf[mt], xf[nt], acc[mt][nt]);
+        for (int z = 0; z < 2; ++z) {
+          const int o = upto(m) + z;
+          if (o < upto(m + 1) && o < OPS) {
+            const int before = o * (WT + NF) / OPS;
+            if ((o + 1) * (WT + NF) / OPS > before) read(next, before, wf[1 - h], xf[1 - h]);
+            else copy(k + 4, o - before);
           }
-        __builtin_amdgcn_s_setprio(0);
+        }
         __builtin_amdgcn_sched_barrier(0);
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
       }
     }
-  };
-  if (frags == XT) walk(std::true_type{});
-  else walk(std::false_type{});
-  if (grp == 0) __builtin_amdgcn_s_barrier();
-
-  // ---- lane holds out[token 16 (8 grp + nt) + r][column of fragment mt, + 4 g + i]; loads first, then only stores ----
-  int pair[XT];
-  float tw[XT];
-#pragma unroll
-  for (int nt = 0; nt < XT; ++nt) {
-    pair[nt] = a.sorted[beg + min(16 * (XT * grp + nt) + r, cnt - 1)];
-    tw[nt] = EPI == EPI_DOWN ? a.topk_w[pair[nt]] : 1.f;
   }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 7" ::: "memory");
+
+  // ---- a lane holds rows 16 (NF xi + nt) + r, columns 4 g + i of fragment mt.  Four nt at a time through this wave's quarter of the
+  // ring, so that a row is stored in 128 bytes or more at once ----
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  constexpr int CG = EPI == EPI_GATE_UP ? 16 : 32;     // lanes of a row, four columns each
+  constexpr int ROW = 4 * 16 * WT + 16;                // bytes between rows: 16-byte columns of a bank row in turn
+  uint8_t* mine = lds + wave * WIDE_SLOT;
+  static_assert(64 * ROW <= WIDE_SLOT, "four fragments of rows fit a quarter");
 #pragma unroll
-  for (int nt = 0; nt < XT; ++nt) {
-    if (16 * (XT * grp + nt) + r >= cnt) continue;
-    T* op = reinterpret_cast<T*>(a.out) + (long)pair[nt] * a.out_stride;
+  for (int q = 0; q < NF; q += 4) {
+    constexpr int Q = 4;
+    const int rows = 16 * (NF - q < Q ? NF - q : Q);
 #pragma unroll
-    for (int mt = 0; mt < (EPI == EPI_GATE_UP ? 2 : WT); ++mt) {
-      const int n = n0 + wrow(mt) + 4 * g;
+    for (int nt = q; nt < NF && nt < q + Q; ++nt)
+#pragma unroll
+      for (int mt = 0; mt < WT; ++mt)
+        *reinterpret_cast<f32x4*>(mine + (16 * (nt - q) + r) * ROW + 64 * mt + 16 * g) = acc[mt][nt];
+    asm volatile("" ::: "memory");
+#pragma unroll 1
+    for (int i0 = 0; i0 < rows; i0 += 64 / CG) {
+      const int row = i0 + lane / CG, token = 16 * (NF * xi + q) + row, cl = 4 * (lane % CG);
+      const int n = n0 + (EPI == EPI_GATE_UP ? 64 : 128) * wi + cl;
+      f32x4 v = *reinterpret_cast<const f32x4*>(mine + row * ROW + 4 * cl);
+      if (token >= cnt) continue;
+      if (EPI == EPI_GATE_UP) {
+        const f32x4 u = *reinterpret_cast<const f32x4*>(mine + row * ROW + 256 + 4 * cl);
+        v = gated_four(v, u, a.act, a.act_limit);
+      } else if (EPI == EPI_UP_ACT) v = gate_four(v, a.act);
+      else
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] *= tw[token];
+      T* op = reinterpret_cast<T*>(a.out) + (long)pair[token] * a.out_stride + n;
       V4 o;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float v = acc[mt][nt][i];
-        if (EPI == EPI_GATE_UP) v = gated_pair(v, acc[mt + 2][nt][i], a.act, a.act_limit);
-        else if (EPI == EPI_UP_ACT) v = gate_act(v, a.act);
-        else v *= tw[nt];
-        o[i] = (T)v;
-      }
-      if (n + 3 < a.N) *reinterpret_cast<V4*>(op + n) = o;
+      for (int i = 0; i < 4; ++i) o[i] = (T)v[i];
+      if (n + 3 < a.N) *reinterpret_cast<V4*>(op) = o;
       else
-        for (int i = 0; i < 4; ++i) if (n + i < a.N) op[n + i] = o[i];
+        for (int i = 0; i < 4; ++i) if (n + i < a.N) op[i] = o[i];
     }
+    asm volatile("" ::: "memory");
+  }
+}
+
+template <typename T, int EPI>
+__global__ __launch_bounds__(256, 1) void moe_wide_gemm_kernel(const TileGemmArgs a) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[4 * WIDE_SLOT];
+  __shared__ int pair[WIDE_ROWS];
+  __shared__ float tw[EPI == EPI_DOWN ? WIDE_ROWS : 1];
+  int mi, ni;
+  if (!tile_of_block(min(*a.num_tiles, a.m_tiles), a.n_tiles, mi, ni)) return;
+  const int e = a.tile_expert[mi], beg = a.tile_beg[mi], cnt = min(a.tile_end[mi] - beg, WIDE_ROWS);
+  const int n0 = ni * (EPI == EPI_GATE_UP ? 128 : 256);
+  for (int i = threadIdx.x; i < cnt; i += 256) {
+    const int p = a.sorted[beg + i];
+    pair[i] = p;
+    if (EPI == EPI_DOWN) tw[i] = a.topk_w[p];
+  }
+  __syncthreads();
+  const auto walk = [&](auto nf) { wide_walk<T, EPI, decltype(nf)::value>(a, lds, pair, tw, e, beg, cnt, n0); };
+  switch ((cnt + 31) >> 5) {
+    case 9: return walk(std::integral_constant<int, 9>());
+    case 8: return walk(std::integral_constant<int, 8>());
+    case 7: return walk(std::integral_constant<int, 7>());
+    case 6: return walk(std::integral_constant<int, 6>());
+    case 5: return walk(std::integral_constant<int, 5>());
+    case 4: case 3: return walk(std::integral_constant<int, 4>());
+    default: return walk(std::integral_constant<int, 2>());
   }
 }
 
 // ---------------------------------------------------------------------------------------------
-// m-tile table: for expert e with c tokens, ceil(c / rows) tiles.  One workgroup, E <= 1024.
+// m-tile table: for expert e with c tokens, ceil(c / rows) tiles; with rows == 256 (the wide tiles) the fewest of at most WIDE_ROWS,
+// of like sizes in 32 rows.  One workgroup, E <= 1024.
 __global__ __launch_bounds__(1024) void moe_tile_map_kernel(int* __restrict__ tile_expert, int* __restrict__ tile_beg,
                                                             int* __restrict__ tile_end, int* __restrict__ num_tiles,
                                                             const int* __restrict__ offsets, int E, int rows,
                                                             int max_tiles) {
   __shared__ int pre[1025];
   const int tid = threadIdx.x;
+  const bool wide = rows == 256;
   int nt = 0, b = 0, en = 0;
-  if (tid < E) { b = offsets[tid]; en = offsets[tid + 1]; nt = (en - b + rows - 1) / rows; }
+  if (tid < E) {
+    b = offsets[tid];
+    en = offsets[tid + 1];
+    if (wide) {
+      nt = (en - b + WIDE_ROWS - 1) / WIDE_ROWS;
+      rows = nt ? ((en - b + nt - 1) / nt + 31) & ~31 : rows;
+      nt = (en - b + rows - 1) / rows;
+    } else nt = (en - b + rows - 1) / rows;
+  }
   pre[tid + 1] = nt;
   if (tid == 0) pre[0] = 0;
   __syncthreads();
@@ -487,7 +590,7 @@ __global__ __launch_bounds__(1024) void moe_tile_map_kernel(int* __restrict__ ti
     const int first = pre[tid];
     for (int i = 0; i < nt; ++i) {
       const int t = first + i;
-      if (t < max_tiles) { tile_expert[t] = tid; tile_beg[t] = b + i * rows; tile_end[t] = en; }
+      if (t < max_tiles) { tile_expert[t] = tid; tile_beg[t] = b + i * rows; tile_end[t] = wide ? min(en, b + (i + 1) * rows) : en; }
     }
   }
   if (tid == 0) *num_tiles = min(pre[E], max_tiles);
@@ -575,7 +678,7 @@ VDA_EXPORT int vda_moe_align_large(int* sorted, int* offsets, int* counts, int* 
 // ---------------------------------------------------------------------------------------------
 template <typename T>
 static int launch_wide_gemm(const TileGemmArgs& a, int epi, hipStream_t st) {
-  const dim3 grid(tile_blocks(a.m_tiles, a.n_tiles)), block(512);
+  const dim3 grid(tile_blocks(a.m_tiles, a.n_tiles)), block(256);
   if (epi == EPI_GATE_UP) hipLaunchKernelGGL((moe_wide_gemm_kernel<T, EPI_GATE_UP>), grid, block, 0, st, a);
   else if (epi == EPI_DOWN) hipLaunchKernelGGL((moe_wide_gemm_kernel<T, EPI_DOWN>), grid, block, 0, st, a);
   else if (epi == EPI_UP_ACT) hipLaunchKernelGGL((moe_wide_gemm_kernel<T, EPI_UP_ACT>), grid, block, 0, st, a);
