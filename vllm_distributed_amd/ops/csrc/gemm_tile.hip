@@ -316,24 +316,26 @@ __global__ __launch_bounds__(512, 1) void tile_gemm_kernel(const TileGemmArgs a)
 // Grouped 16-bit GEMM on tiles of 256 weight rows x up to 288 activation rows, for experts that see more than 128 rows each.
 // Four waves, one a SIMD, as 2 (weight rows) x 2 (activation rows): a wave holds 8 x NF accumulator tiles of 16 x 16 and reads
 // 17 KB of LDS operands per 72 MFMAs (eight waves of 4 x 8 tiles read 12 per 32, which with the fill is all that an LDS
-// delivers in that time).  K is walked in steps of 32 elements through a ring of four LDS slots:
+// delivers in that time).  K is walked in units of 64 elements, whole 128-byte lines of a row (half lines, in steps of 32, kept the L2
+// busy with twice the requests), through two LDS slots, a unit in two halves.  Dealt out between the MFMAs of unit u:
 //
-//   step k: wait for the own copies of step k + 1 and the own reads of step k; barrier; then, dealt out between the MFMAs
-//   of step k: the reads of the fragments of step k + 1 (second register set) and the copies of step k + 4
+//   half 0: to three quarters, the reads of half 1 (second register set); barrier: the slot of unit u is free
+//   from there to three quarters of half 1: the copies of unit u + 2 into it
+//   half 1: at a quarter, wait for the own copies of unit u + 1; barrier; then the reads of its half 0
 //
-// Write-after-read: the slot of step k is written after the barrier of step k, which every wave reaches with its reads of it
-// done.  Read-after-write: slot k + 1 is read after that barrier, which every wave reaches with its copies to it landed (those of
-// steps k + 2 and k + 3 may be in flight: up to three steps, 3000 cycles of MFMAs, for a copy).  K is a multiple of 64, so the steps are even.
+// so a copy has one and a half to two and a half halves of MFMAs to arrive.  Write-after-read: copies of unit u + 2 follow a barrier that every
+// wave reaches with its reads of unit u done.  Read-after-write: the reads of unit u + 1 follow one that every wave reaches
+// with its copies of it landed (the AHEAD younger ones may be in flight).
 //
 // An expert's rows are cut into the fewest tiles of at most 288 rows, of like sizes (moe_tile_map_kernel): batches of 2048 or
 // 4096 tokens over eight experts are 256-row tiles but for a few rows, which opened tiles of their own in half of the experts.
 // NF, the 16-row fragments of a wave, is a template argument: tiles of few rows do few MFMAs.
 //
-// LDS image of a slot: [row][4 chunks of 16 bytes], chunk c of row r at c ^ wide_swz(r), on the source side of the copy.  Of a fragment read
-// the lanes of rows {0-3, 12-15} at chunk q are served with those of {4-11} at q ^ 1: with 0, 2, 3, 1 for the four rows of four they
-// touch the sixteen 16-byte columns of a 256-byte bank row once each.
+// LDS image of a slot: [row][8 chunks of 16 bytes], chunk c of row r at c ^ ((r >> 1) & 7), on the source side of the copy.  Of a fragment read
+// the lanes of rows {0-3, 12-15} at chunk q are served with those of {4-11} at q ^ 1: they touch the sixteen 16-byte columns of
+// a 256-byte bank row once each.
 // WIDE_FIGURES
-constexpr int WIDE_ROWS = 288, WIDE_SLOT = (256 + WIDE_ROWS) * 64;
+constexpr int WIDE_ROWS = 288, WIDE_UNIT = (256 + WIDE_ROWS) * 128;
 
 // 16 bytes a lane from a buffer to LDS, at dst + 16 * lane.  As a statement of its own: told of the copy, the compiler waits for
 // all of them before the next LDS read, although they fill another slot of the ring.  Waited for by the counts in the loop.
@@ -379,8 +381,6 @@ __device__ __forceinline__ f32x4 gated_four(f32x4 g, f32x4 u, int kind, float li
   return gate_four(g, kind) * u;
 }
 
-__device__ __forceinline__ int wide_swz(int r) { return (r >> 1 & 2) ^ (r & 8 ? 3 : 0); }
-
 // one tile: acc[mt][nt] = the sum over K of W fragment mt . X fragment nt, then the epilogue.  pair, tw: the pair of each row
 // of the tile and its routing weight, in LDS
 template <typename T, int EPI, int NF>
@@ -388,7 +388,7 @@ __device__ __forceinline__ void wide_walk(const TileGemmArgs& a, uint8_t* lds, c
                                           int n0) {
   using V8 = typename Vec<T>::v8;
   using V4 = typename Vec<T>::v4;
-  constexpr int WT = 8, XP = 2 * NF, XC = (XP + 3) / 4, CP = 4 + XC;     // 1 KB pieces of X, and what a wave copies in a step
+  constexpr int WT = 8, CP = 8 + NF, READS = WT + NF;  // copies of 1 KB of a wave in a unit, and its fragment reads in half of one
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
@@ -398,88 +398,73 @@ __device__ __forceinline__ void wide_walk(const TileGemmArgs& a, uint8_t* lds, c
   const i32x4 wbuf = wide_buffer(reinterpret_cast<const uint8_t*>(a.w) + (long)e * a.w_expert_stride * 2), xbuf = wide_buffer(a.x);
   const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
 
-  // copies: lane L of a 1 KB piece fills row L >> 2 of its sixteen, position L & 3.  Wave w takes pieces w, w + 4, ...; where the
-  // pieces of X do not divide, the last is copied by two waves
+  // copies: lane L of a 1 KB piece fills row L >> 3 of its eight, position L & 7.  Wave w takes pieces w, w + 4, ...
   unsigned voff[CP];                         // (host: both operands of an expert below 4 GiB)
-  int at[XC];
   {
-    const int lrow = lane >> 2, chunk = ((lane & 3) ^ wide_swz(lrow)) << 4;
+    const int lrow = lane >> 3, chunk = ((lane & 7) ^ ((4 * wave + (lrow >> 1)) & 7)) << 4;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int rho = 16 * (wave + 4 * j) + lrow;
+    for (int j = 0; j < 8; ++j) {
+      const int rho = 8 * (wave + 4 * j) + lrow;
       const int row = EPI == EPI_GATE_UP ? (rho < 128 ? n0 + rho : a.N + n0 + rho - 128) : n0 + rho;
       voff[j] = (unsigned)min(row, w_rows - 1) * kbytes + chunk;
     }
 #pragma unroll
-    for (int j = 0; j < XC; ++j) {
-      const int piece = min(wave + 4 * j, XP - 1);
-      const int p = pair[min(16 * piece + lrow, cnt - 1)];
+    for (int j = 0; j < NF; ++j) {
+      const int p = pair[min(8 * (wave + 4 * j) + lrow, cnt - 1)];
       const int xrow = EPI == EPI_DOWN ? p : p / a.top_k;
-      voff[4 + j] = (unsigned)xrow * (unsigned)(a.x_stride * 2) + chunk;
-      at[j] = 256 * 64 + piece * 1024;
+      voff[8 + j] = (unsigned)xrow * (unsigned)(a.x_stride * 2) + chunk;
     }
   }
-  const int steps = a.K >> 5;
-  auto copy = [&](int k, int j) {            // piece j of step k (the last step's again beyond the end: into a slot that is free)
-    const int ko = min(k, steps - 1) * 64;
-    const unsigned slot = lds0 + (k & 3) * WIDE_SLOT;
-    if (j < 4) wide_copy(wbuf, voff[j], ko, slot + (wave + 4 * j) * 1024);
-    else wide_copy(xbuf, voff[j], ko, slot + at[j - 4]);
+  const int units = a.K >> 6;
+  auto copy = [&](int u, int j) {            // piece j of unit u (the last unit's again beyond the end: into a slot that is free)
+    wide_copy(j < 8 ? wbuf : xbuf, voff[j], min(u, units - 1) * 128,
+              lds0 + (u & 1) * WIDE_UNIT + (j < 8 ? 0 : 256 * 128) + (wave + 4 * (j < 8 ? j : j - 8)) * 1024);
   };
   // weight fragment mt of wave column wi starts at tile row wrow(mt); with a gate half four are gate rows and four the up rows of
   // the same columns
   auto wrow = [&](int mt) { return EPI == EPI_GATE_UP ? (mt < 4 ? 64 * wi + 16 * mt : 128 + 64 * wi + 16 * (mt - 4))
                                                       : 128 * wi + 16 * mt; };
-  const int cpos = r * 64 + ((g ^ wide_swz(r)) << 4);
-  const int wl = wrow(0) * 64 + cpos, xl = (256 + 16 * NF * xi) * 64 + cpos;
+  const int cpos = r * 128 + ((g ^ (r >> 1)) << 4);    // half 0 of a unit; half 1 is at cpos ^ 64
   f32x4 acc[WT][NF];
 #pragma unroll
   for (int mt = 0; mt < WT; ++mt)
 #pragma unroll
     for (int nt = 0; nt < NF; ++nt) acc[mt][nt] = f32x4{0, 0, 0, 0};
   V8 wf[2][WT], xf[2][NF];
-  auto read = [&](const uint8_t* slot, int i, V8 (&w)[WT], V8 (&x)[NF]) {      // fragment i of a step: the first weight rows' first
-    if (i < 4) w[i] = *reinterpret_cast<const V8*>(slot + wl + (wrow(i) - wrow(0)) * 64);
-    else if (i < 4 + NF) x[i - 4] = *reinterpret_cast<const V8*>(slot + xl + (i - 4) * 1024);
-    else w[i - NF] = *reinterpret_cast<const V8*>(slot + wl + (wrow(i - NF) - wrow(0)) * 64);
+  auto read = [&](int u, int h, int i) {     // fragment i of half h, in the order in which they are needed
+    const uint8_t* slot = lds + (u & 1) * WIDE_UNIT + (h ? cpos ^ 64 : cpos);
+    if (i < WT) wf[h][i] = *reinterpret_cast<const V8*>(slot + wrow(0) * 128 + (wrow(i) - wrow(0)) * 128);
+    else xf[h][i - WT] = *reinterpret_cast<const V8*>(slot + (256 + 16 * NF * xi) * 128 + (i - WT) * 2048);
   };
 
 #pragma unroll
-  for (int k = 0; k < 4; ++k)
+  for (int u = 0; u < 2; ++u)
 #pragma unroll
-    for (int j = 0; j < CP; ++j) copy(k, j);
-  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(3 * CP) : "memory");
+    for (int j = 0; j < CP; ++j) copy(u, j);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(CP) : "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 #pragma unroll
-  for (int i = 0; i < WT + NF; ++i) read(lds, i, wf[0], xf[0]);
-  for (int k0 = 0; k0 < steps; k0 += 2) {
+  for (int i = 0; i < READS; ++i) read(0, 0, i);
+  constexpr int ALL = WT * NF, FREE = ALL * 3 / 4, LAND = ALL / 4;
+  // n operations over w places: how many stand before place i
+  auto upto = [](int i, int n, int w) constexpr { return (i * n + w - 1) / w; };
+  constexpr int AHEAD = ((ALL + LAND - FREE) * CP + ALL - 1) / ALL;      // copies of unit u + 2 before unit u + 1 is waited for
+  static_assert(READS <= FREE && CP <= ALL, "one read and one copy behind an MFMA at most");
+  for (int u = 0; u < units; ++u) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int k = k0 + h;
-      constexpr int OPS = WT + NF + CP, ALL = WT * NF;
-      static_assert(8 * OPS <= 14 * ALL, "two operations behind an MFMA at most");
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(2 * CP) : "memory");
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-      const uint8_t* next = lds + ((k + 1) & 3) * WIDE_SLOT;
 #pragma unroll
       for (int m = 0; m < ALL; ++m) {
+        if (h == 0 && m == FREE) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (h == 1 && m == LAND) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(AHEAD) : "memory");
         const int nt = m / WT, mt = m % WT;
         if (nt < 8) wide_mfma<true>(acc[mt][nt], wf[h][mt], xf[h][nt]);
         else wide_mfma<false>(acc[mt][nt], wf[h][mt], xf[h][nt]);
-        // the OPS reads and copies behind the first seven eighths of the MFMAs, two at most behind one
-        auto upto = [](int m) { return (m * 8 * OPS + 7 * ALL - 1) / (7 * ALL); };
-#pragma unroll
-        for (int z = 0; z < 2; ++z) {
-          const int o = upto(m) + z;
-          if (o < upto(m + 1) && o < OPS) {
-            const int before = o * (WT + NF) / OPS;
-            if ((o + 1) * (WT + NF) / OPS > before) read(next, before, wf[1 - h], xf[1 - h]);
-            else copy(k + 4, o - before);
-          }
-        }
+        const int i = h ? m - LAND : m, before = upto(i, READS, FREE);
+        if (i >= 0 && i < FREE && upto(i + 1, READS, FREE) > before) read(u + h, 1 - h, before);
+        const int c = h * ALL + m - FREE, done = upto(c, CP, ALL);
+        if (c >= 0 && c < ALL && upto(c + 1, CP, ALL) > done) copy(u + 2, done);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -492,8 +477,8 @@ __device__ __forceinline__ void wide_walk(const TileGemmArgs& a, uint8_t* lds, c
   asm volatile("" ::: "memory");
   constexpr int CG = EPI == EPI_GATE_UP ? 16 : 32;     // lanes of a row, four columns each
   constexpr int ROW = 4 * 16 * WT + 16;                // bytes between rows: 16-byte columns of a bank row in turn
-  uint8_t* mine = lds + wave * WIDE_SLOT;
-  static_assert(64 * ROW <= WIDE_SLOT, "four fragments of rows fit a quarter");
+  uint8_t* mine = lds + wave * (WIDE_UNIT / 2);
+  static_assert(64 * ROW <= WIDE_UNIT / 2, "four fragments of rows fit a quarter");
 #pragma unroll
   for (int q = 0; q < NF; q += 4) {
     constexpr int Q = 4;
@@ -531,7 +516,7 @@ __device__ __forceinline__ void wide_walk(const TileGemmArgs& a, uint8_t* lds, c
 
 template <typename T, int EPI>
 __global__ __launch_bounds__(256, 1) void moe_wide_gemm_kernel(const TileGemmArgs a) {
-  __shared__ __attribute__((aligned(16))) uint8_t lds[4 * WIDE_SLOT];
+  __shared__ __attribute__((aligned(16))) uint8_t lds[2 * WIDE_UNIT];
   __shared__ int pair[WIDE_ROWS];
   __shared__ float tw[EPI == EPI_DOWN ? WIDE_ROWS : 1];
   int mi, ni;
