@@ -489,27 +489,28 @@ __device__ __forceinline__ void wide_walk(const TileGemmArgs& a, uint8_t* lds, c
       for (int mt = 0; mt < WT; ++mt)
         *reinterpret_cast<f32x4*>(mine + (16 * (nt - q) + r) * ROW + 64 * mt + 16 * g) = acc[mt][nt];
     asm volatile("" ::: "memory");
-#pragma unroll 1
-    for (int i0 = 0; i0 < rows; i0 += 64 / CG) {
-      const int row = i0 + lane / CG, token = 16 * (NF * xi + q) + row, cl = 4 * (lane % CG);
-      const int n = n0 + (EPI == EPI_GATE_UP ? 64 : 128) * wi + cl;
-      f32x4 v = *reinterpret_cast<const f32x4*>(mine + row * ROW + 4 * cl);
-      if (token >= cnt) continue;
-      if (EPI == EPI_GATE_UP) {
-        const f32x4 u = *reinterpret_cast<const f32x4*>(mine + row * ROW + 256 + 4 * cl);
-        v = gated_four(v, u, a.act, a.act_limit);
-      } else if (EPI == EPI_UP_ACT) v = gate_four(v, a.act);
-      else
+    auto store = [&](auto finish) {
+#pragma unroll 4                                       // several rows in flight: a wave is alone on its SIMD
+      for (int i0 = 0; i0 < rows; i0 += 64 / CG) {
+        const int row = i0 + lane / CG, token = 16 * (NF * xi + q) + row, cl = 4 * (lane % CG);
+        const int n = n0 + (EPI == EPI_GATE_UP ? 64 : 128) * wi + cl;
+        f32x4 v = *reinterpret_cast<const f32x4*>(mine + row * ROW + 4 * cl), u = v;
+        if (EPI == EPI_GATE_UP) u = *reinterpret_cast<const f32x4*>(mine + row * ROW + 256 + 4 * cl);
+        v = finish(v, u, token);
+        T* op = reinterpret_cast<T*>(a.out) + (long)pair[token] * a.out_stride + n;
+        V4 o;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] *= tw[token];
-      T* op = reinterpret_cast<T*>(a.out) + (long)pair[token] * a.out_stride + n;
-      V4 o;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = (T)v[i];
-      if (n + 3 < a.N) *reinterpret_cast<V4*>(op) = o;
-      else
-        for (int i = 0; i < 4; ++i) if (n + i < a.N) op[i] = o[i];
-    }
+        for (int i = 0; i < 4; ++i) o[i] = (T)v[i];
+        if (token < cnt) {
+          if (n + 3 < a.N) *reinterpret_cast<V4*>(op) = o;
+          else
+            for (int i = 0; i < 4; ++i) if (n + i < a.N) op[i] = o[i];
+        }
+      }
+    };
+    if (EPI == EPI_DOWN) store([&](f32x4 v, f32x4, int token) { return v * tw[token]; });
+    else if (a.act == 0) store([&](f32x4 v, f32x4 u, int) { v = gate_four(v, 0); return EPI == EPI_GATE_UP ? v * u : v; });
+    else store([&](f32x4 v, f32x4 u, int) { return EPI == EPI_GATE_UP ? gated_four(v, u, a.act, a.act_limit) : gate_four(v, a.act); });
     asm volatile("" ::: "memory");
   }
 }
