@@ -45,3 +45,13 @@ def test_few_pairs_of_8_bit_experts(monkeypatch, pairs, E, rows, depth, split):
     """The K-split form where the workgroups of the experts that are chosen are too few for the other, or more than its first wave."""
     monkeypatch.delenv("VDA_MOE_ROWS_FORM", raising=False)
     assert (ops.moe_rows_form(pairs, E, rows, 1, depth) == 0) is split
+
+
+@pytest.mark.parametrize("E,H,I,rows,wide", [(64, 2048, 1024, 128, False), (64, 2048, 1024, 129, True), (64, 2048, 1024, 300, True),     # 512 and 512 tiles
+                                             (8, 4096, 14336, 256, True), (8, 3840, 14336, 256, False),       # 128 and 120 in the second product
+                                             (8, 4096, 8192, 256, True), (8, 4096, 8064, 256, False),         # 512 and 504 in the first
+                                             (16, 1024, 4096, 300, False), (32, 1024, 512, 450, True)])
+def test_layers_of_many_tiles_take_the_wide_ones_at_any_rows(E, H, I, rows, wide):
+    x, w13, w2 = (torch.empty(s, dtype=torch.bfloat16, device="meta") for s in ((E * rows, H), (E, 2 * I, H), (E, H, I)))
+    assert ops._moe_wide(x, w13, w2, E * rows, -(-I // 128), H, -(-H // 256), I) is wide
+    assert not ops._moe_wide(x, w13.to(torch.float8_e4m3fn), w2, E * rows, -(-I // 128), H, -(-H // 256), I)

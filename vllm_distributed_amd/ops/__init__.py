@@ -1170,29 +1170,44 @@ def moe_align_tiles(topk_ids: torch.Tensor, E: int, rows_per_tile: int):
     return sorted_ids, offsets, tiles, max_tiles
 
 
-def _moe_wide_ok(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, pairs: int) -> bool:
-    """Can 16-bit experts gain by 256 x 256 tiles?  From 129 rows an expert on, except between 233 and 351, where most experts
-    are cut into one whole tile and one that is nearly empty (60 experts 2048 x 1408 with 300 rows: 541 us on 128-row tiles, 620
-    on these; 64 experts 2048 x 1024 436 / 460; eight experts 4096 x 14336, whose rounds come out even, 1292 / 1161).  The
-    kernel's offsets inside an operand are 32-bit."""
-    rows = pairs / w13.shape[0]
-    return (w13.dtype != torch.float8_e4m3fn and rows > 128 and not 232 < rows < 352
+def _moe_wide_fits(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, pairs: int) -> bool:
+    """Can 16-bit experts run on the wide tiles (256 columns x up to 288 rows), and do they see more rows than a 128-row tile holds?
+    The kernel's offsets inside an operand are 32-bit.  (With 80 rows an expert 64 experts 2048 x 1024 take 204 us on 128-row tiles
+    and 238 on these, 32 experts 2048 x 2048 183 / 232; with 115 rows 259 / 249 and 250 / 240.)"""
+    return (w13.dtype != torch.float8_e4m3fn and pairs > 128 * w13.shape[0]
             and max(max(x.stride(0), x.shape[1]) * x.shape[0], w2.shape[2] * pairs, w13.shape[1] * w13.shape[2],
                     w2.shape[1] * w2.shape[2]) < 1 << 31)
 
 
+def _moe_wide_ok(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, pairs: int) -> bool:
+    """Can layers of few tiles gain by the wide ones?  Not between 233 and 351 rows an expert, where they leave CUs idle (8
+    experts 1024 x 512, 300 rows: 53 us on 128-row tiles, 68 on these)."""
+    return _moe_wide_fits(x, w13, w2, pairs) and not 232 < pairs / w13.shape[0] < 352
+
+
+def _moe_wide(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, pairs: int, n1: int, k1: int, n2: int, k2: int) -> bool:
+    """Wide tiles or 128-row ones, for products of n1 and n2 tiles of columns, k1 and k2 deep?  Layers in which one tile an expert makes two
+    rounds over the CUs in the first product and half a round in the second take the wide ones at any number of rows: 128-row tiles / these,
+    in us: 8 experts 4096 x 14336 with 140, 256, 300 and 512 rows each 798 / 656, 1108 / 836, 1259 / 947, 1805 / 1188; 64 experts
+    2048 x 1024 301 / 257, 367 / 303, 430 / 404, 653 / 466; 512 experts 2048 x 512 1158 / 1011, 1564 / 1404, 1833 / 1510, 2717 / 2168;
+    nine such layers at eleven sizes gain 3 to 52 %.  Below that single tiles decide: 16 experts 1024 x 4096, whose second product has
+    64 tiles, with 300 rows 241 / 262; 32 experts 1024 x 512 with 210 rows 72 / 80."""
+    E = w13.shape[0]
+    if E * n1 >= 512 and E * n2 >= 128:
+        return _moe_wide_fits(x, w13, w2, pairs)
+    return _moe_wide_ok(x, w13, w2, pairs) and _moe_wide_pays(pairs, E, n1, k1, n2, k2)
+
+
 @functools.lru_cache(maxsize=1024)
 def _moe_wide_pays(pairs: int, E: int, n1: int, k1: int, n2: int, k2: int) -> bool:
-    """Do 256 x 256 tiles cost less than 128 x 256 ones, for ``pairs`` rows over E experts in products [rows, k] x [k, n tiles]?
-    A CU holds one tile at a time: a product takes rounds of 256 tiles (whole ones while they are few; later their ends overlap)
-    of K steps each, and a round of wide tiles costs 1.65 of the others (1.6 .. 1.9 where both fill their rounds).  Both
+    """Do wide tiles cost less than 128 x 256 ones in a layer of few tiles, for ``pairs`` rows over E experts in products [rows, k] x
+    [k, n tiles]?  A CU holds one tile at a time: a product takes rounds of 256 tiles (whole ones while they are few; later their ends
+    overlap) of K steps each, and a round of wide tiles costs at most 1.65 of the others.  Both
     estimates of the tiles have to say so: every expert takes its share of rows and a standard deviation, and the number to be
-    expected, where one expert in 64 that exceeds 256 rows opens a round (64 experts 2048 x 1024 with 219 rows each 341 us on
-    128-row tiles, 328 on these; with 225 378 / 414).  Layer times in us, 128-row tiles / 256-row tiles: 64 experts 2048 x 1024 with 160 rows
-    each 322 / 305, 440 rows 561 / 492, 500 rows 618 / 575; 8 experts
-    4096 x 14336 with 440 rows 1522 / 1260, 200 rows 834 / 917; 8 experts 1024 x 512, whose tiles leave CUs idle, with 360
-    rows 52 / 72; 16 experts 2048 x 1408 with 620 rows 282 / 312.  Of 200 such points in the range above (9 layers, 135 .. 1025
-    rows) this takes 107; three of them lose more than 2 %, the worst 4.3 %."""
+    expected, where one expert in 64 that exceeds 256 rows opens a round.  The estimates cut experts at 256 rows, the kernel at
+    288: they err to the side of 128-row tiles.  128-row tiles / wide ones, in us: 32 experts 1024 x 512 with 210 rows 72 / 80,
+    with 450 113 / 91, with 512, which this leaves to the former, 144 / 99; 8 experts 1024 x 512, whose tiles leave CUs idle, with
+    360 rows 53 / 57; 16 experts 1024 x 4096 with 512 rows 358 / 276."""
     rows = pairs / E
     sd = math.sqrt(rows)
 
@@ -1223,7 +1238,7 @@ def _moe_tiled(x, w13, w2, topk_w, topk_ids, w13_scale, w2_scale, block_scales: 
     I = I2 // 2 if gated else I2
     P_ = T * k
     dev = x.device
-    wide = _moe_wide_ok(x, w13, w2, P_) and _moe_wide_pays(P_, E, -(-I // (128 if gated else 256)), H, -(-H // 256), I)
+    wide = _moe_wide(x, w13, w2, P_, -(-I // (128 if gated else 256)), H, -(-H // 256), I)
     rows = 256 if wide else _tile_rows(P_ / E)
     sorted_ids, _, tiles, max_tiles = moe_align_tiles(topk_ids, E, rows)
     te, tb, tend, ntl = (tiles[:max_tiles], tiles[max_tiles:2 * max_tiles], tiles[2 * max_tiles:3 * max_tiles],

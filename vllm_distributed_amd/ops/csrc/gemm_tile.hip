@@ -334,7 +334,11 @@ __global__ __launch_bounds__(512, 1) void tile_gemm_kernel(const TileGemmArgs a)
 // LDS image of a slot: [row][8 chunks of 16 bytes], chunk c of row r at c ^ ((r >> 1) & 7), on the source side of the copy.  Of a fragment read
 // the lanes of rows {0-3, 12-15} at chunk q are served with those of {4-11} at q ^ 1: they touch the sixteen 16-byte columns of
 // a 256-byte bank row once each.
-// WIDE_FIGURES
+// What bounds it: the MFMAs run 70 % of the cycles, at a clock that the chip's power takes down to 1.7 GHz of 2.4; without copies the
+// second product of 8 experts 4096 x 14336 over 8198 rows takes 617 us (1.56 PFLOP/s, a large library product reaches 1.60), with them 760;
+// the results of the first, which leave in bursts with the MFMAs idle, are a tenth of it.  Asking the L2 ahead for a share of each line made it 3 % slower.
+// us, eight waves of 64 x 128 sums -> this, whole layer: 4099 tokens of 8 experts 4096 x 14336, top 2, 2940 -> 2260 (1.28 PFLOP/s with rows that
+// exist); 4096 of 64 experts 2048 x 1024, top 8, 576 -> 469; 4096 of 16 experts 4096 x 6400 1453 -> 1151.
 constexpr int WIDE_ROWS = 288, WIDE_UNIT = (256 + WIDE_ROWS) * 128;
 
 // 16 bytes a lane from a buffer to LDS, at dst + 16 * lane.  As a statement of its own: told of the copy, the compiler waits for
