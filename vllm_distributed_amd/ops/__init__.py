@@ -605,6 +605,25 @@ def skinny_gemm_ok(M: int, N_: int, K: int, dtype: torch.dtype, max_m: Optional[
             and dtype in (torch.bfloat16, torch.float16) and not envs.VDA_DISABLE_SKINNY_GEMM)
 
 
+def skinny_gemm_wanted(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> bool:
+    """Does a 16-bit linear of a few rows and a small weight matrix take the skinny kernel?  Its workgroups of 16 columns split K over eight
+    waves with everything in flight at once: ahead of the library where one round of them is on the chip (256 of them, two of short
+    K) and K is short.  Library / this, in us, one and 16 rows (graphs of calls on changing weights): 4096 x 4096 15.5 / 10.5 and 15.5 / 11.8, 3072 x
+    2048 11.2 / 5.6 and 11.2 / 6.7, 256 x 512 7.5 / 2.4 and 7.7 / 2.8, 8192 x 2048 14.3 / 9.7 and 13.0 / 11.5; beyond: 6144 x 4096 14.3 / 20.1 with 16
+    rows, 2048 x 5632 10.4 / 14.0 with 12.  Of 17 .. 32 rows: 2048 x 2048 with 32 11.1 / 8.1, 8192 x 1024 11.5 / 8.9, but 2048 x 3072
+    10.1 / 11.9, 6144 x 2048 12.4 / 14.9, 256 x 2048 7.6 / 7.9."""
+    M, K = x.shape
+    N_ = w.shape[0]
+    if not _dev(x) or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):
+        return False
+    few = M <= 16 and ((N_ <= 4096 and K <= 4096) or (N_ <= 8192 and K <= 2048))
+    more = M <= 32 and ((512 <= N_ <= 4096 and K <= 2048) or (N_ <= 8192 and K <= 1024))
+    return ((few or more) and M >= 1 and N_ >= 256 and N_ % 16 == 0 and K >= 512 and K % 128 == 0 and w.shape[1] == K
+            and x.dtype in (torch.bfloat16, torch.float16) and w.dtype == x.dtype and w.is_contiguous() and x.stride(0) % 8 == 0
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and not envs.VDA_DISABLE_SKINNY_GEMM
+            and (bias is None or (bias.dtype == x.dtype and bias.is_contiguous() and bias.data_ptr() % 8 == 0)))
+
+
 def skinny_gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
                 w_scale: Optional[torch.Tensor] = None) -> torch.Tensor:
     """y = x @ w.T (+ bias) for x [M<=64, K], w [N, K]; w may be e4m3 with a per-tensor ``w_scale``
@@ -719,7 +738,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     their switches are set), hipBLASLt otherwise."""
     if x.is_cuda and x.dim() == 2 and x.stride(-1) == 1 and w.stride(-1) == 1:
         M, K = x.shape
-        if skinny_gemm_ok(M, w.shape[0], K, x.dtype):
+        if skinny_gemm_ok(M, w.shape[0], K, x.dtype) or skinny_gemm_wanted(x, w, bias):
             return skinny_gemm(x, w, bias)
         if decode_gemm_ok(M, w.shape[0], K, x.dtype) and w.dtype == x.dtype and w.is_contiguous() \
                 and x.stride(0) % 8 == 0 and (bias is None or bias.dtype == x.dtype):

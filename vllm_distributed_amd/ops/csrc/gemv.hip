@@ -2,13 +2,19 @@
 // The weight matrix is streamed exactly once straight from HBM into MFMA A
 // operands (16 weight rows per workgroup, 64 contiguous bytes per lane per
 // 128-wide K chunk); the few activation rows ride on the MFMA column dimension,
-// so one kernel covers M = 1 .. 64 without a GEMV special case.  The 4 waves of
-// a workgroup split K and are summed through LDS.
+// so one kernel covers M = 1 .. 64 without a GEMV special case.  The waves of
+// a workgroup split K and are summed through LDS: eight up to 32 rows (of 8-bit weights where N is at most 8192), which puts a K of
+// 2048 into flight at once, and four beyond, whose activation loads leave no room (us, bf16,
+// 12 rows, four -> eight waves: 3072 x 2048 7.0 -> 6.3, 4096 x 4096 13.5 -> 11.3, 11264 x 2048 16.9 -> 14.9,
+// 10240 x 8192 57.5 -> 53.5; sixteen waves 6.5, 11.9, 17.2, 55.4; two weight tiles a workgroup 8.6, 15.9, 16.1, 60.3).
+// Bound by one trip to memory and a launch while weights are small; beyond some 16 million of them by the activations, which
+// every workgroup reads again.
 // Role of the reference's csrc/rocm/skinny_gemms.cu (LLMM1 / wvSplitK).
 #include "common.h"
 
-template <typename T, int MT, typename WL>   // MT = number of 16-row activation tiles, WL = weight loader
-__global__ __launch_bounds__(256) void skinny_gemm_kernel(T* __restrict__ y, const T* __restrict__ x,
+// MT = number of 16-row activation tiles, WL = weight loader, W = waves of a workgroup
+template <typename T, int MT, typename WL, int W>
+__global__ __launch_bounds__(64 * W) void skinny_gemm_kernel(T* __restrict__ y, const T* __restrict__ x,
                                                           const void* __restrict__ w, const T* __restrict__ bias,
                                                           const float* __restrict__ w_scale,
                                                           int M, int N, int K, long x_stride, long w_stride,
@@ -39,25 +45,25 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(T* __restrict__ y, con
   const int nchunk = K >> 7;
   // two chunks per iteration keep 8 weight loads per lane in flight
   int c = wave;
-  for (; c + 4 < nchunk; c += 8) {
+  for (; c + W < nchunk; c += 2 * W) {
     V8 wa[4], wb[4];
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       wa[s] = WL::ld(w, wp + (long)c * 128 + koff(s));
-      wb[s] = WL::ld(w, wp + (long)(c + 4) * 128 + koff(s));
+      wb[s] = WL::ld(w, wp + (long)(c + W) * 128 + koff(s));
     }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const V8 xa = xv[mt] ? ld16<V8>(xp[mt] + (long)c * 128 + koff(s)) : V8{};
-        const V8 xb = xv[mt] ? ld16<V8>(xp[mt] + (long)(c + 4) * 128 + koff(s)) : V8{};
+        const V8 xb = xv[mt] ? ld16<V8>(xp[mt] + (long)(c + W) * 128 + koff(s)) : V8{};
         acc[mt] = mfma16(wa[s], xa, acc[mt]);
         acc[mt] = mfma16(wb[s], xb, acc[mt]);
       }
     }
   }
-  for (; c < nchunk; c += 4) {
+  for (; c < nchunk; c += W) {
     V8 wa[4];
 #pragma unroll
     for (int s = 0; s < 4; ++s)
@@ -72,7 +78,7 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(T* __restrict__ y, con
     }
   }
 
-  __shared__ f32x4 red[3][MT][64];
+  __shared__ f32x4 red[W - 1][MT][64];
   if (wave > 0) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) red[wave - 1][mt][lane] = acc[mt];
@@ -85,7 +91,9 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(T* __restrict__ y, con
   if (bias) bv = *reinterpret_cast<const V4*>(bias + n0 + 4 * g);
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
-    const f32x4 s = acc[mt] + red[0][mt][lane] + red[1][mt][lane] + red[2][mt][lane];
+    f32x4 s = acc[mt];
+#pragma unroll
+    for (int k = 0; k < W - 1; ++k) s += red[k][mt][lane];
     if (xv[mt]) {
       V4 o;
 #pragma unroll
@@ -100,12 +108,15 @@ VDA_EXPORT int vda_skinny_gemm(void* y, const void* x, const void* w, const void
                                int N, int K, long x_stride, long w_stride, long y_stride, int dtype, int wdtype,
                                hipStream_t st) {
   if (M < 1 || M > 64 || N % 16 || K % 128) return -1;
-  dim3 grid(N / 16), block(256);
+  const dim3 grid(N / 16);
   const int mt = (M + 15) / 16;
-#define L(TT, MM, WL) hipLaunchKernelGGL((skinny_gemm_kernel<TT, MM, WL>), grid, block, 0, st, (TT*)y, (const TT*)x, \
-                                         w, (const TT*)bias, w_scale, M, N, K, x_stride, w_stride, y_stride)
-#define BY(TT, WL) do { if (mt == 1) L(TT, 1, WL); else if (mt == 2) L(TT, 2, WL); else if (mt == 3) L(TT, 3, WL); \
-                        else L(TT, 4, WL); } while (0)
+  // 8-bit weights, us, four -> eight waves: 4096 x 14336, one row 32.5 -> 23.6; 28672 x 4096 32.1 -> 34.6
+  const bool eight = wdtype != VDA_FP8 || N <= 8192;
+#define L(TT, MM, WL, WW) hipLaunchKernelGGL((skinny_gemm_kernel<TT, MM, WL, WW>), grid, dim3(64 * WW), 0, st, (TT*)y, (const TT*)x, \
+                                             w, (const TT*)bias, w_scale, M, N, K, x_stride, w_stride, y_stride)
+#define BY(TT, WL) do { if (mt == 1) { if (eight) L(TT, 1, WL, 8); else L(TT, 1, WL, 4); } \
+                        else if (mt == 2) { if (eight) L(TT, 2, WL, 8); else L(TT, 2, WL, 4); } \
+                        else if (mt == 3) L(TT, 3, WL, 4); else L(TT, 4, WL, 4); } while (0)
   const bool f8 = wdtype == VDA_FP8;
   if (dtype == VDA_BF16) { if (f8) BY(bf16_t, WLoadFp8<bf16_t>); else BY(bf16_t, WLoad<bf16_t>); }
   else if (dtype == VDA_F16) { if (f8) BY(f16_t, WLoadFp8<f16_t>); else BY(f16_t, WLoad<f16_t>); }
