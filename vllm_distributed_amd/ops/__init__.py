@@ -8,6 +8,7 @@ KV cache layout used throughout:
 """
 from __future__ import annotations
 
+import ctypes
 import functools
 import math
 from typing import Optional
@@ -59,6 +60,25 @@ def _contig_last(x: torch.Tensor) -> torch.Tensor:
 
 
 # ---- normalisation -----------------------------------------------------------
+UPLOAD_MAX = 16                                      # blocks of one ``upload``
+
+
+def mapped_host(pinned: torch.Tensor) -> Optional[int]:
+    """The address by which kernels read a pinned host tensor, or None where it is not mapped."""
+    at = ctypes.c_void_p()
+    return at.value if pinned.is_pinned() and N.lib().vda_mapped_host(ctypes.byref(at), pinned.data_ptr()) == 0 else None
+
+
+def upload(blocks: list) -> None:
+    """Blocks of mapped host memory into device memory, in order of the current stream and ``UPLOAD_MAX`` to a launch: rows of
+    (mapped address, device address, 4-byte words of a row, rows, words between rows on the device).  The caller keeps the host
+    side as it is until the stream has passed."""
+    for i in range(0, len(blocks), UPLOAD_MAX):
+        part = blocks[i:i + UPLOAD_MAX]
+        table = (ctypes.c_long * (5 * len(part)))(*(v for b in part for v in b))
+        N.call("vda_upload", ctypes.addressof(table), len(part), N.stream())
+
+
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float, residual: Optional[torch.Tensor] = None,
              weight_bias: float = 0.0, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """y = rmsnorm(x [+ residual]) * (weight + weight_bias); residual is updated in place."""

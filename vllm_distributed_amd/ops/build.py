@@ -87,7 +87,8 @@ def _compile_one(src: str, obj: str, flags: list[str], force: bool, cc: str | No
 
 # kernels every generation path launches (linear layers, gated activations, norms, sampling); a model class adds its
 # own in ``native_sources``
-COMMON_OPS_SOURCES = ("activation.hip", "norm.hip", "sampling.hip", "gemm_dense.hip", "gemv.hip", "gemm_decode.hip")
+COMMON_OPS_SOURCES = ("activation.hip", "norm.hip", "sampling.hip", "gemm_dense.hip", "gemv.hip", "gemm_decode.hip",
+                      "upload.hip")
 
 
 def ensure_built_for(model_dir: str | None, log=None) -> None:

@@ -27,6 +27,8 @@ ACT = {"silu": 0, "gelu": 1, "gelu_tanh": 2, "gelu_pytorch_tanh": 2, "relu": 3, 
 
 P, I, L, F = c_void_p, c_int, c_long, c_float
 _SIGS = {
+    "vda_upload": [P, I, P],
+    "vda_mapped_host": [P, P],
     "vda_rms_norm": [P, P, P, P, F, I, I, L, L, L, F, I, P, P, P, I, P],
     "vda_layer_norm": [P, P, P, P, F, I, I, L, L, I, P],
     "vda_act_and_mul": [P, P, L, I, L, L, I, I, F, P, I, P],

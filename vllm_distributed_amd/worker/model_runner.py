@@ -37,6 +37,8 @@ from ..sched.output import EMPTY_MODEL_RUNNER_OUTPUT, ModelRunnerOutput, Schedul
 from .input_batch import InputBatch
 
 logger = init_logger(__name__)
+_UPLOAD_TYPES = {torch.int32: np.int32, torch.int64: np.int64, torch.float32: np.float32}
+_UPLOAD_BYTES = 1 << 18           # of one array; a kernel reads the host at some 30 GB/s, a copy engine at 50
 _CAPTURE_STATE_ANCHOR = None      # see ModelRunner.capture_model
 
 
@@ -162,6 +164,8 @@ class ModelRunner:
         self.cascade_suffix_lens = torch.zeros(Spad, dtype=torch.int32, device=dev)
         self.pin = self.is_gpu
         self._stage_bufs, self._stage_idx, self._stage_off = None, 0, 0
+        self._stage_np, self._stage_at = [], []      # the arenas as numpy arrays, and where kernels see them
+        self._uploads: Optional[list] = None         # blocks that one launch will carry (see _start_uploads)
         # one step uploads ~24 bytes per token plus one block-table row per sequence
         self._stage_bytes = int(Tpad * 40 + Spad * (self.max_blocks * 4 + 64) + (1 << 20))
         self.intermediate: Optional[IntermediateTensors] = None
@@ -186,8 +190,7 @@ class ModelRunner:
         if not self.pin:
             return torch.from_numpy(src)
         nb = src.nbytes
-        if self._stage_bufs is None:
-            self._stage_bufs = [torch.empty(self._stage_bytes, dtype=torch.uint8).pin_memory() for _ in range(3)]
+        self._make_stages()
         off = (self._stage_off + 15) // 16 * 16
         if off + nb > self._stage_bytes:
             return torch.from_numpy(src).pin_memory()          # oversize upload: rare, pay the pin
@@ -200,9 +203,59 @@ class ModelRunner:
         self._stage_idx = (self._stage_idx + 1) % 3
         self._stage_off = 0
 
+    def _make_stages(self) -> None:
+        if self._stage_bufs is None:
+            self._stage_bufs = [torch.empty(self._stage_bytes, dtype=torch.uint8).pin_memory() for _ in range(3)]
+            self._stage_np = [b.numpy() for b in self._stage_bufs]
+            self._stage_at = [None if envs.VDA_FORCE_TORCH_OPS else ops.mapped_host(b) for b in self._stage_bufs]
+
     def _to_dev(self, dst: torch.Tensor, src: np.ndarray) -> None:
+        if self._uploads is not None and self._queue_upload(dst, src):
+            return
         t = self._stage(src)
         dst[: t.shape[0]].copy_(t, non_blocking=True)
+
+    def _start_uploads(self) -> None:
+        """Until ``_flush_uploads`` what ``_to_dev`` and ``_table_to_dev`` are given goes to the device in one launch.  Nothing may read
+        these buffers on the device in between."""
+        if self.is_gpu and self.pin:
+            self._make_stages()
+            if None not in self._stage_at:
+                self._uploads = []
+
+    def _flush_uploads(self) -> None:
+        blocks, self._uploads = self._uploads, None
+        if blocks:
+            ops.upload(blocks)
+
+    def _queue_upload(self, dst: torch.Tensor, src: np.ndarray) -> bool:
+        """``src`` (one row, or rows of a table) into the first columns of ``dst``.  Large arrays, for which a copy engine is the better
+        one, and those that the arena has no room for are left to the caller."""
+        want = _UPLOAD_TYPES.get(dst.dtype)
+        if want is None or dst.stride(-1) != 1 or src.nbytes > _UPLOAD_BYTES:
+            return False
+        if not src.size:
+            return True
+        off = (self._stage_off + 15) // 16 * 16
+        size = dst.element_size()
+        end = off + src.size * size
+        if end > self._stage_bytes:
+            return False
+        rows = src.shape[0] if src.ndim == 2 else 1
+        if src.shape[-1] > dst.shape[-1] or (src.ndim == 2 and rows > dst.shape[0]) or src.ndim != dst.dim():
+            return False
+        self._stage_off = end
+        self._stage_np[self._stage_idx][off:end].view(want).reshape(src.shape)[...] = src
+        words = size // 4
+        self._uploads.append((self._stage_at[self._stage_idx] + off, dst.data_ptr(), src.shape[-1] * words, rows,
+                              dst.stride(0) * words if rows > 1 else 0))
+        return True
+
+    def _table_to_dev(self, dst: torch.Tensor, src: np.ndarray) -> None:
+        """The first rows and columns of a table."""
+        if self._uploads is not None and self._queue_upload(dst, src):
+            return
+        dst[: src.shape[0], : src.shape[1]].copy_(self._stage(src), non_blocking=True)
 
     # ------------------------------------------------------------------
     def _sleep_pool(self, tag: str):
@@ -648,12 +701,13 @@ class ModelRunner:
         self._to_dev(self.seq_lens, seq_lens)
         self._to_dev(self.query_start_loc, cu)
         if S:
-            self.block_table[:S, :W].copy_(self._stage(ib.block_tables[0][rows, :W]), non_blocking=True)
+            self._table_to_dev(self.block_table, ib.block_tables[0][rows, :W])
         if nd < S:
             self._to_dev(self.prefill_qsl, (cu[nd:] - cu[nd]).astype(np.int32))
         if self.state_table is not None and S:
             self._to_dev(self.state_table.view(-1), (rows + 1).astype(np.int32))
         if self.local_chunk:
+            self._flush_uploads()            # (it reads the block table on the device)
             self._upload_local_attention(rows, n_sched, cu, seq_lens, nd)
         return nd, ndt
 
@@ -674,20 +728,27 @@ class ModelRunner:
         if self.tknp_size > 1:
             tmd, att = self._prepare_token_parallel(so, req_ids, rows, n_sched, req_idx, tok_rows, pos)
         else:
-            self._to_dev(self.input_ids, ib.token_ids[tok_rows, pos])
-            if self._pend_of:
-                self._feed_pending_tokens(req_ids, rows, cu)
-            if self.uses_mrope:
-                pos = self._mrope_positions(req_ids, rows, n_sched, cu, pos)
-            nd, ndt = self._upload_attention_inputs(rows, n_sched, cu, pos, slot, seq_lens)
+            self._start_uploads()
+            try:
+                self._to_dev(self.input_ids, ib.token_ids[tok_rows, pos])
+                pending = self._pending_tokens(req_ids, rows, cu) if self._pend_of else 0
+                if self.uses_mrope:
+                    pos = self._mrope_positions(req_ids, rows, n_sched, cu, pos)
+                nd, ndt = self._upload_attention_inputs(rows, n_sched, cu, pos, slot, seq_lens)
+            finally:
+                self._flush_uploads()
+            if pending:
+                vals = self._pend_ids.index_select(0, self._pend_src[:pending]).to(self.input_ids.dtype)
+                self.input_ids.index_copy_(0, self._pend_dst[:pending], vals)
             att = (S, T, nd, ndt, int(seq_lens.max()) if S else 0, int(n_sched.max()) if S else 0,
                    int(seq_lens[nd:].max()) if nd < S else 0)
         logits_idx = (cu[1:] - 1).astype(np.int64)
         return req_ids, rows, n_sched, cu, S, T, logits_idx, att, tmd
 
-    def _feed_pending_tokens(self, req_ids, rows, cu) -> None:
+    def _pending_tokens(self, req_ids, rows, cu) -> int:
         """Run-ahead scheduling: requests whose newest token was sampled by the step still in flight read it
-        from that step's device result (the host copy of the token arrives later)."""
+        from that step's device result (the host copy of the token arrives later).  Uploads which of its tokens go where,
+        and returns how many."""
         ib = self.input_batch
         dst, src = [], []
         for i, rid in enumerate(req_ids):
@@ -695,13 +756,10 @@ class ModelRunner:
             if j is not None and ib.num_computed[rows[i]] == ib.num_tokens[rows[i]]:
                 dst.append(int(cu[i]))
                 src.append(j)
-        if not dst:
-            return
-        n = len(dst)
-        self._to_dev(self._pend_dst, np.asarray(dst, dtype=np.int64))
-        self._to_dev(self._pend_src, np.asarray(src, dtype=np.int64))
-        vals = self._pend_ids.index_select(0, self._pend_src[:n]).to(self.input_ids.dtype)
-        self.input_ids.index_copy_(0, self._pend_dst[:n], vals)
+        if dst:
+            self._to_dev(self._pend_dst, np.asarray(dst, dtype=np.int64))
+            self._to_dev(self._pend_src, np.asarray(src, dtype=np.int64))
+        return len(dst)
 
     def _mrope_positions(self, req_ids, rows, n_sched, cu, pos: np.ndarray) -> np.ndarray:
         """Multimodal rotary positions.  Requests with images carry three position rows for their prompt
@@ -1112,10 +1170,14 @@ class ModelRunner:
         if spec_sched and self.rejection_sampler is not None:
             out = self._sample_with_spec(so, hidden, req_ids, rows, n_sched, cu, S)
         else:
-            self._to_dev(self.logits_indices, logits_idx)
-            sample_hidden = hidden[self.logits_indices[:S]]
+            if T == S:                       # a token of every request: its row is the request's own
+                sample_hidden = hidden[:S]
+            else:
+                self._to_dev(self.logits_indices, logits_idx)
+                sample_hidden = hidden[self.logits_indices[:S]]
             logits = self._compute_logits(sample_hidden, logits_idx[:S])
             if so.logit_taps:                # on their way to the host before anything changes them
+                logits = logits.float()      # (the sampler's form: converted once)
                 taps = self._start_taps(so, req_ids, n_sched, cu, logits, logits_idx[:S])
             if envs.VLLM_COMPUTE_NANS_IN_LOGITS:
                 self._last_nans = {r: int(x) for r, x in zip(req_ids, logits.isnan().sum(-1).tolist())}
@@ -1380,7 +1442,7 @@ class ModelRunner:
         if not idx or idx != logits_idx.tolist():
             return None
         rows = torch.empty(logits.shape, dtype=torch.float32, pin_memory=self.pin)
-        rows.copy_(logits.float() if self.is_gpu else logits, non_blocking=True)
+        rows.copy_(logits, non_blocking=True)
         done = None
         if self.is_gpu:
             done = torch.cuda.Event()
