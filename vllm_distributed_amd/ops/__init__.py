@@ -64,9 +64,9 @@ UPLOAD_MAX = 16                                      # blocks of one ``upload``
 
 
 def mapped_host(pinned: torch.Tensor) -> Optional[int]:
-    """The address by which kernels read a pinned host tensor, or None where it is not mapped."""
-    at = ctypes.c_void_p()
-    return at.value if pinned.is_pinned() and N.lib().vda_mapped_host(ctypes.byref(at), pinned.data_ptr()) == 0 else None
+    """The address by which kernels read a pinned host tensor, or None where it is not mapped (or the library has no ``upload``)."""
+    fn, at = getattr(N.lib(), "vda_mapped_host", None), ctypes.c_void_p()
+    return at.value if fn is not None and pinned.is_pinned() and fn(ctypes.byref(at), pinned.data_ptr()) == 0 else None
 
 
 def upload(blocks: list) -> None:
