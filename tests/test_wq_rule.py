@@ -25,3 +25,11 @@ def test_where_the_other_kernel_cannot_cut_k():
                                         (8, 10240, 8192, True), (16, 14336, 8192, True), (8, 28672, 8192, True), (16, 28672, 8192, False)])
 def test_rule_of_groups_of_64(M, n, k, pays):
     assert N.lib().vda_wq_slices_pay(M, n, k, 4, 64, 0) == pays
+
+
+@pytest.mark.parametrize("M,n,k,bits,parts", [(13, 10240, 8192, 4, 6), (64, 10240, 8192, 8, 6), (65, 10240, 8192, 4, 3), (13, 5120, 5120, 4, 5), (65, 5120, 13824, 4, 6),
+                                              (13, 21760, 4096, 8, 3), (13, 21888, 4096, 8, 1), (32, 28672, 4096, 4, 1), (33, 28672, 4096, 4, 2),
+                                              (32, 28672, 5248, 4, 2), (64, 32768, 4096, 8, 1), (13, 32896, 4096, 8, 2), (13, 49024, 4096, 4, 2),
+                                              (13, 49152, 4096, 4, 1), (128, 24448, 4096, 4, 1), (128, 24576, 4096, 4, 1), (16, 256, 512, 4, 1)])
+def test_parts_of_one_round(M, n, k, bits, parts):
+    assert N.lib().vda_wq_parts(M, n, k, bits) == parts

@@ -491,6 +491,7 @@ static int wq_slices_rows(int N, int K, int bits, bool scaled) {
   return nk <= 64 ? 16 : nk <= 128 ? (groups >= 40 ? 10 : 4) : nk <= 176 ? (groups >= 40 ? 4 : 0) : groups >= 48 ? 1 : 0;
 }
 static bool wq_unscaled(int N, int bits, int group) { return bits == 4 && group % 128 == 0 && N % 4 == 0; }
+static bool wq_unscaled_or_8(int N, int bits, int group) { return bits == 8 || wq_unscaled(N, bits, group); }
 static bool wq_slices_pay(int M, int N, int K, int bits, int group, bool no_split) {
   if (no_split && (N + 127) / 128 * 4 < 512 * 3) return M <= 16 && (K <= 8192 || M <= (bits == 4 ? 10 : 12));   // K in one part there
   return M <= wq_slices_rows(N, K, bits, !wq_unscaled(N, bits, group));
@@ -696,6 +697,23 @@ static int launch_wq_gemm(const WqGemmArgs& wa, int xt, hipStream_t st) {
 // out [M, N].  K % 32 == 0, group % 32 == 0 and K % group == 0, N % 4 == 0 for split K.  variant: 0 picks by shape,
 // 1 the tiled kernel, 2 the streaming kernel (M <= 128, K % 128 == 0, group a power of two or K), 3 the streaming
 // kernel in its per-element form.  Returns 0 or a negative code for shapes it does not take.
+// Into how many parts the kernel of up to 128 rows cuts K, for N / 128 workgroups each, of which the chip holds 512 (256 beyond 64 rows).
+// As many as one round holds: a few workgroups more make a second one.  us, weights cold, parts that just exceed a round -> those that fit:
+// 13 rows of 10240 x 8192 21.9 -> 19.5, 64 rows 36.1 -> 31.5 (8 bits 50.3 -> 41.8); 64 of 28672 x 8192 72.6 -> 63.9; 65 rows of 10240 x 8192 63.4 ->
+// 45.2, of 5120 x 13824 58.4 -> 40.0, of 14336 x 4096 47.8 -> 34.0, of 22016 x 4096 62.2 -> 53.9.  Where two parts fit and one already
+// gives two thirds of the CUs a workgroup, one saves the launch that sums: 8 bits 28672 x 4096, 13 rows, two 36.0, one 31.0, x 8192 60.6 -> 53.0; 4 bits
+// 21.8 -> 20.5, 25600 x 5120 28.1 -> 25.0, but 64 rows 45.4 / 51.0 and 28672 x 8192, four rows, 34.8 / 36.9.  From 257 workgroups on one part leaves more idle
+// than a second round costs: 304 of them, 13 rows, 44.5 with one, 39.8 with two.
+static int wq_parts(int M, int N, int K, int bits) {
+  const int groups = (N + 127) / 128, nk = K >> 7, slots = M <= 64 ? 512 : 256;
+  if (groups * 4 >= slots * 3) return 1;
+  if (M <= 64 && groups > 170 && groups <= 256 && (bits == 8 || (M <= 32 && nk <= 40))) return 1;
+  const int parts = slots == 512 && groups > 256 ? 2 : slots / groups;
+  return max(1, min(min(parts, nk / 8), 32));
+}
+// (for the test of the rule, which runs on the host)
+VDA_EXPORT int vda_wq_parts(int M, int N, int K, int bits) { return wq_parts(M, N, K, bits); }
+
 VDA_EXPORT int vda_wq_gemm(void* out, const void* x, const void* qw, const void* sz, const void* bias, float* ws,
                            size_t ws_bytes, int M, int N, int K, int group, int bits, long x_stride, long out_stride,
                            int dtype, int splits, int variant, hipStream_t st) {
@@ -723,19 +741,18 @@ VDA_EXPORT int vda_wq_gemm(void* out, const void* x, const void* qw, const void*
   if (variant == 2 || (variant == 0 && can_stream && (M <= 64 || bits == 4))) {   // 8 bit, 65..128 rows: tiled is faster
     const int nk = K >> 7;
     const int groups = (N + 127) / 128;
-    const int slots = M <= 64 ? 512 : 256;
-    if (variant == 0 && splits < 1 && wq_slices_pay(M, N, K, bits, group, no_split)) {
+    const int parts = wq_parts(M, N, K, bits);
+    // (layers that the kernel below takes in one part with a workgroup on most CUs lead there at any number of rows: 28672 x 4096 in 8 bits, 4, 8
+    // and 13 rows, slices 31.9, 35.0 and 38.1 us, this 30.1, 30.6 and 31.2; with 172 of them, 22016 x 4096, slices 24.9, 26.9 and 29.3, this
+    // 29.0, 29.4 and 29.9)
+    const bool whole = parts == 1 && groups >= 224 && groups <= 256 && wq_unscaled_or_8(N, bits, group);
+    if (variant == 0 && splits < 1 && !whole && wq_slices_pay(M, N, K, bits, group, no_split)) {
       rc = dtype == VDA_BF16 ? (bits == 4 ? launch_wq_slices<bf16_t, 4>(wa, st) : launch_wq_slices<bf16_t, 8>(wa, st))
                              : (bits == 4 ? launch_wq_slices<f16_t, 4>(wa, st) : launch_wq_slices<f16_t, 8>(wa, st));
       VDA_CHECK_LAUNCH();
       return rc;
     }
-    if (splits < 1) {
-      splits = 1;
-      if (groups * 4 < slots * 3) splits = (slots + groups - 1) / groups;
-      splits = min(splits, max(nk / 8, 1));
-      splits = min(splits, 32);
-    }
+    if (splits < 1) splits = parts;
     splits = min(splits, nk);
     if (no_split) splits = 1;
     while (splits > 1 && (size_t)splits * M * N * sizeof(float) > ws_bytes) --splits;

@@ -126,6 +126,7 @@ _SIGS = {
     "vda_scaled_softcap": [P, P, L, L, I, F, F, I, P],
     "vda_selective_scan_pairs": [P, P, P, P, P, P, P, P, P, P, P, P, P, L, I, I, I, L, L, L, L, L, L, I, I, I, I, I, I, I, P, P, I, P],
     "vda_scan_lane_channel": [I, I, I],
+    "vda_wq_parts": [I, I, I, I],
     "vda_wq_slices_pay": [I, I, I, I, I, I],
     "vda_selective_scan": [P, P, P, P, P, P, P, P, P, P, P, P, P, L, I, I, I, L, L, L, L, L, L, I, I, I, I, I, I, P, P,
                            I, P],
