@@ -54,6 +54,11 @@ _VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 EXTRA_FLAGS = {f: _VGPR_FORM for f in ("attention.hip", "attention_prefill.hip", "mla.hip", "mla_tile.hip", "delta_rule.hip",
                                        "linear_attention.hip")}
 
+DEVICE_FLAGS = [f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-ffast-math", "-fno-finite-math-only",
+                "-fvisibility=hidden", "-Wno-unused-value", "-DNDEBUG",
+                # no packed fp32 arithmetic: the compiler forms v_pk_*_f32 from plain float code by itself
+                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+
 
 def _hipcc() -> str:
     exe = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
@@ -120,10 +125,7 @@ def build(force: bool = False, jobs: int | None = None, verbose: bool = True, on
           skip: tuple = ()) -> list[str]:
     """``only``: file names of ops/csrc to put into libvda_ops.so (None: all of them)."""
     jobs = jobs or min(16, os.cpu_count() or 1)
-    flags = [f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-ffast-math", "-fno-finite-math-only",
-             "-fvisibility=hidden", "-Wno-unused-value", "-DNDEBUG",
-             # no packed fp32 arithmetic: the compiler forms v_pk_*_f32 from plain float code by itself
-             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+    flags = DEVICE_FLAGS
     built = []
     for name, spec in LIBS.items():
         srcdir = spec["dir"]
