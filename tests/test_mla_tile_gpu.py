@@ -195,3 +195,16 @@ def test_every_column_block_and_piece_has_its_workgroup(S, new, prefix, H, windo
     ops.mla_attention(out, q, kc, vt, table, lens, starts, 192 ** -0.5, max(news), 8, window=window)
     want = R.mla_attention(q, kc, vt, table, lens, starts, 192 ** -0.5, 1.0, window)
     torch.testing.assert_close(out.float(), want.float(), atol=12 * 2.0 ** -9, rtol=2.0 ** -8)
+
+
+@pytest.mark.parametrize("new,total,H,window", [([264], [534], 1, 2), ([264, 1, 0, 40], [534, 90, 7, 41], 1, 2), ([659] + [3] * 23, [3583] + [3] * 23, 1, 1),
+                                                ([300], [900], 2, 33), ([200], [700], 3, 1)])
+def test_windows_of_blocks_of_many_tokens(new, total, H, window):
+    """With one head a column block is 128 tokens: under a window it has up to five key steps more than a last block of one token, and
+    as many more pieces."""
+    kc, vt, table, lens, starts = _batch(new, total, 16, torch.bfloat16, H)
+    q = torch.randn(sum(new), H, DK, device=DEV).to(torch.bfloat16)
+    out = torch.full((sum(new), H, DV), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ops.mla_attention(out, q, kc, vt, table, lens, starts, 192 ** -0.5, max(new), 8, window=window)
+    want = R.mla_attention(q, kc, vt, table, lens, starts, 192 ** -0.5, 1.0, window)
+    torch.testing.assert_close(out.float(), want.float(), atol=12 * 2.0 ** -9, rtol=2.0 ** -8)
