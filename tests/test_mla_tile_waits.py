@@ -86,3 +86,19 @@ def test_copies_have_landed_before_rows_take_their_place(kernels):
                     state[k] = now
                     todo.append(k)
         assert rows >= 16, which
+
+
+def test_key_loop_fetches_nothing_from_scratch(kernels):
+    """A register that comes back from scratch inside the key loop is waited for together with every copy issued before it."""
+    for which, body in kernels.items():
+        blocks, after = _blocks(body)
+        for i, b in enumerate(blocks):
+            if not any(t.startswith("v_mfma") for t in b):
+                continue
+            seen, todo = set(), list(after[i])
+            while todo:
+                k = todo.pop()
+                if k not in seen:
+                    seen.add(k)
+                    todo += after[k]
+            assert i not in seen or not any(t.startswith("scratch_") for t in b), which
