@@ -124,9 +124,9 @@ def test_wide_prefill_fp8_cache(bs):
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
-def test_wide_prefill_lagging_maximum(dt):
-    """Scores that climb key by key: by less than the lag of the running maximum (a factor of 2^8) for long stretches,
-    beyond it in between, at tile edges and inside, and a row that its last key carries alone."""
+def test_wide_prefill_climbing_maximum(dt):
+    """Scores that climb key by key, a little for long stretches and by far more in between, at tile edges and inside, and a
+    row that its last key carries alone: the sums are scaled in every block."""
     Hq, Hkv, bs, n = 8, 2, 16, 700
     q, kc, vc, bt, sl, qsl = _paged_problem([n], [n], Hq, Hkv, 128, bs, dt)
     q[:] = 0.3
@@ -137,8 +137,8 @@ def test_wide_prefill_lagging_maximum(dt):
     _, lse = ops.paged_attention_prefill(out, q, kc, vc, bt, sl, qsl, scale, return_lse=True)
     ref, lref = R.paged_attention(q, kc, vc, bt, sl, qsl, scale, return_lse=True)
     torch.testing.assert_close(out.float(), ref.float(), **tol(dt))
-    # the sum of weights rounded to 8 bits and more: 2^-9 relative at most, and fp32 sums
-    torch.testing.assert_close(lse, lref, atol=3e-3, rtol=1e-4)
+    # the denominator is a sum of fp32 weights: some 100 roundings of 2^-24, and scores of up to 24 rounded to 2^-24 of them a few times
+    torch.testing.assert_close(lse, lref, atol=5e-5, rtol=2e-6)
 
 
 @pytest.mark.parametrize("fp8", [False, True])
@@ -187,7 +187,7 @@ def test_wide_prefill_groups_that_do_not_divide_the_columns(Hq, Hkv):
     _, lse = ops.paged_attention_prefill(out, q, kc, vc, bt, sl, qsl, scale, return_lse=True)
     ref, lref = R.paged_attention(q, kc, vc, bt, sl, qsl, scale, return_lse=True)
     torch.testing.assert_close(out.float(), ref.float(), **tol(torch.bfloat16))
-    torch.testing.assert_close(lse, lref, atol=3e-3, rtol=1e-4)
+    torch.testing.assert_close(lse, lref, atol=5e-5, rtol=2e-6)           # (as above)
 
 
 @pytest.mark.parametrize("lens", [[300], [64] * 16, [70, 500, 70, 500, 1, 129], [90, 31, 200] * 5 + [7], [90, 31, 200] * 6, [1000] + [1] * 20])

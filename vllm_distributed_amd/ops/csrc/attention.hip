@@ -1186,9 +1186,9 @@ VDA_EXPORT int vda_set_prefill_variant(int v) { g_prefill_variant = v; return 0;
 VDA_EXPORT int vda_set_prefill_wide_min_wgs(long n) { g_prefill_wide_min_wgs = n; return 0; }
 
 // Query tokens of a wide workgroup (0: the wide form does not apply to this batch).  A group that does not divide the 256 columns leaves at
-// most a sixteenth of them idle, or the 4-wave form takes it; and it has prompts of three of its tiles on average: us, 4-wave / wide,
-// 28 / 4 heads, 2 x 2161 tokens 244 / 143, 8 x 200 37.7 / 33, 24 x 150 50.6 / 48.8, 24 / 8 heads 43.3 / 34.1 (one of 1000), 226 / 160, but 40 / 8, 24 x 40 27.7 / 30.2,
-// 48 / 8 27.9 / 30.0, 28 / 4 25 x 81 on 740 75.8 / 79.2.
+// most a sixteenth of them idle, or the 4-wave form takes it; and it has prompts of three of its tiles on average: us, 4-wave / wide, attention alone,
+// 28 / 4 heads, 2 x 2161 tokens 135 / 93, 8 ragged of some 200 25.0 / 20.7, 24 of 150 34.4 / 28.4, 24 / 8 heads, one of 1000 45 / 37, 2 of 2161 189 / 145; but ragged
+// ones of less, 40 / 8, 24 of 40 13.8 / 15.1, 48 / 8 14.5 / 16.6, 28 / 4 25 of 81 on 740 77 / 86.
 static int wide_tokens(int G, int num_tokens, int num_seqs) {
   const int tokens = 256 / G;
   if (256 % G && (tokens * G < 240 || (long)num_tokens < 3L * tokens * num_seqs)) return 0;

@@ -26,20 +26,19 @@
 // last, and waits, before its barrier, for the batch that step t - 1 issued, which is read from step t + 1 on.  LDS reads run
 // eight products ahead, across half steps and barriers.
 //
-// The maximum that weights are relative to may lag behind by a factor of 2^8 (a column's own decision), so that scaling the
-// 64 sums of a lane is rare; with a maximum kept exact, some column of 32 moved in most steps of sequences of a few
-// thousand keys, and the products of the scaling were a third of all vector instructions.  Weights are then not at most one, and the
-// largest one is no longer exact in 16 bits; the denominator adds the rounded weights (one v_dot2 for two of them), so that a row which
-// one key carries still is that key's value.  Error against 64 bits as before (0.0027 over ragged prompts of some 1100 tokens, cache and output
-// in bf16).
+// The maximum that weights are relative to is exact after every block: the largest weight, which often carries the row, is one and so exact in
+// 16 bits, and the denominator adds the weights in fp32.  One that may lag by 2^8 spares most of the scaling of the 64 sums of a lane (in
+// sequences of a few thousand keys some column of 32 moves in most steps) and was 10 % faster, but its largest weight is rounded, so that the
+// denominator had to add rounded weights: 0.00272 against 64 bits over ragged prompts of some 1100 tokens where this is at 0.00267 (cache and output in
+// bf16), and a log-sum-exp that was off by up to 0.0013.
 //
 // Measured (MI355X, bf16, 32 / 8 heads, attention alone; before: one barrier a tile, products and softmax of a tile one after the other, K
-// and V through registers): 2048 tokens on 8192 keys 361 -> 313 us, 2 x 4096 331 -> 291, 2048 82 -> 65, 8 x 1024 118 -> 107, 16 x 256 32.5 -> 33.9;
-// seven portions of some 1100 tokens with rotary embedding and cache write 260 -> 221 (208 in the order of tiles of launch_bs); e4m3 cache, 2 x 1512 on 368: 267 -> 214.
-// What bounds long prompts now is power: 3650 cycles a step (2112 of them MFMA) at 1.9 GHz, before 5000 at 2.4; the products alone,
-// without any softmax, take 241 us of the 313 at 1.8 GHz.  The two waves of a SIMD taking turns at products and softmax of whole tiles
-// (two barriers a tile) were at 304 on the long prompt, 289 and 66 on the next two, and slower on short ones (16 x 256 33.8, 9 x 138 with 64 heads 22.6
-// where this form takes 21.3).
+// and V through registers): 2048 tokens on 8192 keys 348 -> 317 us, 2 x 4096 323 -> 304, 2048 74 -> 69, 8 x 1024 115 -> 113, 16 x 256 36.1 -> 35.3;
+// with rotary embedding and cache write: seven portions of some 1100 tokens 261 -> 232, 64 / 8 heads, nine of some 138 39.4 -> 36.3; e4m3 cache, 2 of some
+// 1512, one on 368, 261 -> 148 (the order of tiles of launch_bs has its part in the ragged ones).
+// What bounds long prompts is power and the scaling: without the latter (a lagging maximum) a step took 3650 cycles (2112 of them MFMA) at 1.9 GHz,
+// before 5000 at 2.4.  The two waves of a SIMD taking turns at products and softmax of whole tiles (two barriers a tile) were no faster on long prompts
+// and slower on short ones.
 //
 // Lane maps (l = lane, c = l & 31, h = l >> 5), 32x32x16:
 //   A: row c, k = 8h + j        B: k = 8h + j, column c        C: row (r&3) + 8(r>>2) + 4h, column c
@@ -85,19 +84,8 @@ constexpr int K_BYTES = KT * 256;    // one K image
 constexpr int V_BYTES = WD * 128;    // one V image
 constexpr int RING = 4;              // tiles of either in LDS
 constexpr int SORTED = 16;           // sequences that workgroups sort by length
-constexpr float LAG = 8.f;           // powers of two that a column's maximum may stay behind
 
 __device__ __forceinline__ int key_of_row(int i) { return (i & 19) | ((i & 4) << 1) | ((i & 8) >> 1); }
-
-// the sum of two 16-bit weights and c, in fp32
-__device__ __forceinline__ float dot_one(bf16_t a, bf16_t b, float c) {
-  typedef bf16_t v2 __attribute__((ext_vector_type(2)));
-  return __builtin_amdgcn_fdot2_f32_bf16(v2{a, b}, v2{(bf16_t)1.f, (bf16_t)1.f}, c, false);
-}
-__device__ __forceinline__ float dot_one(f16_t a, f16_t b, float c) {
-  typedef f16_t v2 __attribute__((ext_vector_type(2)));
-  return __builtin_amdgcn_fdot2(v2{a, b}, v2{(f16_t)1.f, (f16_t)1.f}, c, false);
-}
 
 // c += a b, in place: with the builtin, whose result may lie elsewhere, the compiler keeps two copies of the 64 sums across the branches
 // of a step and spills the queries (300 bytes).  It does not look into the statement, so the wait between an operand's last vector
@@ -353,7 +341,6 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
   // registers) soft cap, ALiBi and a distance-bias table as well, of which only the last value remains, as a constant of that
   // fma, for blocks at least dist_far behind every column. ----
   float mx, alpha, off, ps[2], mul = sl2, add = 0.f;
-  bool move;
   auto sm_mask = [&](int h, int kb) {
     const bool whole = h >= w_lo && h < w_hi;
     if (GENERAL) {
@@ -391,29 +378,36 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
   };
   auto sm_move = [&] {
     mx = pair_max(GENERAL ? fmaf(mx, mul, add) : mx * mul);       // the scale is positive
-    move = mx > m + LAG;
-    alpha = move ? fexp2(m - mx) : 1.f;
-    m = move ? mx : m;
-    off = (GENERAL ? add : 0.f) - (m == -INFINITY ? 0.f : m);
+    const float m_new = fmaxf(m, mx), m_use = m_new == -INFINITY ? 0.f : m_new;
+    alpha = fexp2(m - m_use);
+    m = m_new;
+    off = (GENERAL ? add : 0.f) - m_use;
     ps[0] = ps[1] = 0.f;
   };
   auto sm_exp = [&](int kb, int k) {                  // weights 2 k and 2 k + 1 of the lane's 16
     const int t = k >> 2, j = 2 * (k & 3);
-    pb[kb][t][j] = (T)fexp2(fmaf(S[kb][2 * k], mul, off));
-    pb[kb][t][j + 1] = (T)fexp2(fmaf(S[kb][2 * k + 1], mul, off));
-    ps[k & 1] = dot_one(pb[kb][t][j], pb[kb][t][j + 1], ps[k & 1]);
+    const float a = fexp2(fmaf(S[kb][2 * k], mul, off)), b = fexp2(fmaf(S[kb][2 * k + 1], mul, off));
+    pb[kb][t][j] = (T)a;
+    pb[kb][t][j + 1] = (T)b;
+    ps[0] += a;
+    ps[1] += b;
   };
-  auto sm_end = [&] {                                 // (the sums hold the blocks before this one)
-    if (__any(move)) {
-      l *= alpha;
-      settle(acc);
+  // What a block's new maximum scales the sums by is due before that block's P.V, in the next half step: there a quarter of the sums is
+  // scaled in front of its first product, beside the scores' MFMAs.
+  float due = 1.f;
+  bool any_due = false;
+  auto sm_end = [&](bool first_block) {                // (whose sums are still zero)
+    l = l * alpha + (ps[0] + ps[1]);
+    due = alpha;
+    any_due = !first_block && __any(alpha != 1.f);
+  };
+  auto scale_due = [&](int j) {
+    if (any_due) {
+      asm volatile("s_nop 11" : "+v"(acc[j]));         // (the quarter's last product)
 #pragma unroll
-      for (int db = 0; db < 4; ++db)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
-      settle(acc);
+      for (int r = 0; r < 16; ++r) acc[j][r] *= due;
+      asm volatile("" : "+v"(acc[j]));
     }
-    l += ps[0] + ps[1];
   };
 
   auto step_end = [&] {
@@ -432,6 +426,7 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
     // (empty statements keep a slice's results in its place: otherwise the exponentials sink behind the branch of sm_end)
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
+      if (i < 8 && (i & 1)) scale_due(i >> 1);
       product(i, 3, 1 - b, 1 - b);
       // the first operands of the next half step as well
       if (i + AHEAD < 16) read(i + AHEAD, 3, ks, 1 - b, vs, 1 - b);
@@ -447,13 +442,13 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
 #pragma unroll
         for (int k = (i - 4) * 8 / 12; k < (i - 3) * 8 / 12; ++k) {
           sm_exp(b, k);
-          asm volatile("" : "+v"(ps[k & 1]));
+          asm volatile("" : "+v"(ps[0]), "+v"(ps[1]));
         }
       }
       extra(i);
       __builtin_amdgcn_sched_barrier(0);
     }
-    sm_end();
+    sm_end(false);
   };
   auto half_parts = [&](int h, auto b_, int ks, int vs) {       // the parts that exist, one after another
     constexpr int b = decltype(b_)::value;
@@ -463,6 +458,7 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
       for (int i = 0; i < AHEAD; ++i) read(i, what, ks, 1 - b, vs, 1 - b);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
+        if (what == 2 && i < 4) scale_due(i);
         product(i, what, 1 - b, 1 - b);
         if (i + AHEAD < 8) read(i + AHEAD, what, ks, 1 - b, vs, 1 - b);
         __builtin_amdgcn_sched_barrier(0);
@@ -477,7 +473,7 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
       sm_move();
 #pragma unroll
       for (int k = 0; k < 8; ++k) sm_exp(b, k);
-      sm_end();
+      sm_end(h == a_lo);
     }
   };
   constexpr std::integral_constant<int, 0> first{};
@@ -579,8 +575,8 @@ int launch_bs(const AttnParams& p, int bs, int ntiles, hipStream_t st) {
   // sequence in turn, the longest (causal) ones first, is a count without a search: for sequences of about one length, and for many.  Where
   // up to 16 are of unlike lengths, that gives neighbours in time no keys to share and ties sequences to shader engines (a
   // workgroup's number decides on its engine): these go one after another, the one with the most keys first.
-  // us, tile of every sequence / in the batch's order / sorted, 32 / 8 heads: 8 ragged of some 1000 tokens on 500 237 / 162 / 157, 4 of 2000
-  // 335 / 209 / 196, 15 of 240 on 3700 229 / 212 / 177, 7 of 1100 on 900 203 / 183 / 178; 8 equal ones of 1024 107 / - / 118, 32 of 64 14.4 / 20.7 / -.
+  // us, tile of every sequence / in the batch's order / sorted, 32 / 8 heads, ragged: 8 of some 1000 tokens on 500 250 / 233 / 227, 15 of 240 on 3700
+  // 386 / 378 / 319, 7 of 1100, half of them on 900, 232 / 202 / 203, 4 of 2000 226 / 229 / 227; equal ones: 8 of 1024 113 / 120 / 126, 32 of 64 14.0 / 19.1 / -.
   const int bound = p.max_q_len > 0 ? (p.max_q_len + p.q_tile - 1) / p.q_tile : 0;
   const long by_level = (long)bound * p.num_seqs;
   const bool alike = (long)p.max_q_len * p.num_seqs * 15 <= (long)p.num_tokens * 16;
