@@ -632,16 +632,29 @@ def skinny_gemm_wanted(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Te
     2048 11.2 / 5.6 and 11.2 / 6.7, 256 x 512 7.5 / 2.4 and 7.7 / 2.8, 8192 x 2048 14.3 / 9.7 and 13.0 / 11.5; beyond: 6144 x 4096 14.3 / 20.1 with 16
     rows, 2048 x 5632 10.4 / 14.0 with 12.  Of 17 .. 32 rows: 2048 x 2048 with 32 11.1 / 8.1, 8192 x 1024 11.5 / 8.9, but 2048 x 3072
     10.1 / 11.9, 6144 x 2048 12.4 / 14.9, 256 x 2048 7.6 / 7.9."""
-    M, K = x.shape
-    N_ = w.shape[0]
-    if not _dev(x) or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):
+    if not _dev(x) or x.dim() != 2 or w.dim() != 2:
         return False
+    (M, K), N_ = x.shape, w.shape[0]
     few = M <= 16 and ((N_ <= 4096 and K <= 4096) or (N_ <= 8192 and K <= 2048))
     more = M <= 32 and ((512 <= N_ <= 4096 and K <= 2048) or (N_ <= 8192 and K <= 1024))
     return ((few or more) and M >= 1 and N_ >= 256 and N_ % 16 == 0 and K >= 512 and K % 128 == 0 and w.shape[1] == K
-            and x.dtype in (torch.bfloat16, torch.float16) and w.dtype == x.dtype and w.is_contiguous() and x.stride(0) % 8 == 0
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and not envs.VDA_DISABLE_SKINNY_GEMM
-            and (bias is None or (bias.dtype == x.dtype and bias.is_contiguous() and bias.data_ptr() % 8 == 0)))
+            and x.dtype in (torch.bfloat16, torch.float16) and w.dtype == x.dtype and not envs.VDA_DISABLE_SKINNY_GEMM
+            and (bias is None or (bias.shape == (N_,) and bias.dtype == x.dtype)) and _launches_as_is(x, w, bias)
+            and w.is_contiguous() and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and (bias is None or (bias.is_contiguous() and bias.data_ptr() % 8 == 0)))
+
+
+def _launches_as_is(x: torch.Tensor, *others: Optional[torch.Tensor]) -> bool:
+    """May a call that a library operation took become a launch on the operands' memory?  All of them plain tensors of one device, and
+    nobody who would act on the operation itself: reverse- and forward-mode gradients, vmap and its like, tracing, dispatch modes, autocast.
+    (About 1 us.)"""
+    grad = torch.is_grad_enabled()
+    for t in (x, *others):
+        if t is not None and (type(t) not in (torch.Tensor, torch.nn.Parameter) or t.device != x.device or (grad and t.requires_grad)):
+            return False
+    return (torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._get_tracing_state() is None
+            and not torch.is_autocast_enabled(x.device.type) and not torch.compiler.is_compiling())
 
 
 def skinny_gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
