@@ -693,15 +693,12 @@ static int launch_wq_gemm(const WqGemmArgs& wa, int xt, hipStream_t st) {
   return 0;
 }
 
-// x [M, K] 16-bit (row stride x_stride elements), qw packed [N, K] (bits 4 or 8), sz [K / group, N, 2] of x's type,
-// out [M, N].  K % 32 == 0, group % 32 == 0 and K % group == 0, N % 4 == 0 for split K.  variant: 0 picks by shape,
-// 1 the tiled kernel, 2 the streaming kernel (M <= 128, K % 128 == 0, group a power of two or K), 3 the streaming
-// kernel in its per-element form.  Returns 0 or a negative code for shapes it does not take.
 // Into how many parts the kernel of up to 128 rows cuts K, for N / 128 workgroups each, of which the chip holds 512 (256 beyond 64 rows).
 // As many as one round holds: a few workgroups more make a second one.  us, weights cold, parts that just exceed a round -> those that fit:
 // 13 rows of 10240 x 8192 21.9 -> 19.5, 64 rows 36.1 -> 31.5 (8 bits 50.3 -> 41.8); 64 of 28672 x 8192 72.6 -> 63.9; 65 rows of 10240 x 8192 63.4 ->
 // 45.2, of 5120 x 13824 58.4 -> 40.0, of 14336 x 4096 47.8 -> 34.0, of 22016 x 4096 62.2 -> 53.9.  Where two parts fit and one already
-// gives two thirds of the CUs a workgroup, one saves the launch that sums: 8 bits 28672 x 4096, 13 rows, two 36.0, one 31.0, x 8192 60.6 -> 53.0; 4 bits
+// gives two thirds of the CUs a workgroup, one saves the launch that sums: 8 bits 28672 x 4096, 13 rows, two 36.0, one 31.0, x 8192 60.6 -> 53.0; 171 blocks,
+// the fewest, 17, 32 and 64 rows, x 4096 36.4 -> 32.8, 38.6 -> 33.9, 47.1 -> 41.1, x 8192 62.7 -> 57.3, 65.9 -> 59.1, 78.0 -> 71.7; 4 bits
 // 21.8 -> 20.5, 25600 x 5120 28.1 -> 25.0, but 64 rows 45.4 / 51.0 and 28672 x 8192, four rows, 34.8 / 36.9.  From 257 workgroups on one part leaves more idle
 // than a second round costs: 304 of them, 13 rows, 44.5 with one, 39.8 with two.
 static int wq_parts(int M, int N, int K, int bits) {
@@ -714,6 +711,10 @@ static int wq_parts(int M, int N, int K, int bits) {
 // (for the test of the rule, which runs on the host)
 VDA_EXPORT int vda_wq_parts(int M, int N, int K, int bits) { return wq_parts(M, N, K, bits); }
 
+// x [M, K] 16-bit (row stride x_stride elements), qw packed [N, K] (bits 4 or 8), sz [K / group, N, 2] of x's type,
+// out [M, N].  K % 32 == 0, group % 32 == 0 and K % group == 0, N % 4 == 0 for split K.  variant: 0 picks by shape,
+// 1 the tiled kernel, 2 the streaming kernel (M <= 128, K % 128 == 0, group a power of two or K), 3 the streaming
+// kernel in its per-element form.  Returns 0 or a negative code for shapes it does not take.
 VDA_EXPORT int vda_wq_gemm(void* out, const void* x, const void* qw, const void* sz, const void* bias, float* ws,
                            size_t ws_bytes, int M, int N, int K, int group, int bits, long x_stride, long out_stride,
                            int dtype, int splits, int variant, hipStream_t st) {
