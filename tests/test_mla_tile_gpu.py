@@ -208,3 +208,21 @@ def test_windows_of_blocks_of_many_tokens(new, total, H, window):
     ops.mla_attention(out, q, kc, vt, table, lens, starts, 192 ** -0.5, max(new), 8, window=window)
     want = R.mla_attention(q, kc, vt, table, lens, starts, 192 ** -0.5, 1.0, window)
     torch.testing.assert_close(out.float(), want.float(), atol=12 * 2.0 ** -9, rtol=2.0 ** -8)
+
+
+@pytest.mark.parametrize("S,H,new", [(1, 16, 1), (7, 16, 1), (12, 16, 1), (13, 16, 1), (6, 16, 2), (3, 5, 6), (1, 128, 1), (6, 128, 1), (7, 128, 1), (6, 40, 3)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_few_sequences_piece_by_piece(S, H, new, fp8):
+    """Sequences of one column block, either side of where workgroups look through the lengths: pieces of unlike numbers, one sequence without
+    a new token, and rows that an unused piece must leave to the others."""
+    news = [new] * S
+    if S > 3:
+        news[2] = 0
+    total = [n + p for n, p in zip(news, _ragged(S, 1300))]
+    kc, vt, table, lens, starts = _batch(news, total, 16, torch.float8_e4m3fn if fp8 else torch.bfloat16, S + H)
+    q = torch.randn(sum(news), H, DK, device=DEV).to(torch.bfloat16)
+    for window in (0, 70):
+        out = torch.full((sum(news), H, DV), float("nan"), device=DEV, dtype=torch.bfloat16)
+        ops.mla_attention(out, q, kc, vt, table, lens, starts, 192 ** -0.5, new, 8, window=window)
+        want = R.mla_attention(q, kc, vt, table, lens, starts, 192 ** -0.5, 1.0, window)
+        torch.testing.assert_close(out.float(), want.float(), atol=12 * 2.0 ** -9, rtol=2.0 ** -8)

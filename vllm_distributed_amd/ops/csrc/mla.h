@@ -20,7 +20,7 @@ struct MlaParams {
   const float* sink;        // [H] or null: exp(sink[h]) joins head h's softmax denominator, with no key and no value
   int cuts;                 // key pieces of each column block that fill the chip, if all are alike (mla_tile.hip)
   int num_seqs;             // (mla_tile.hip)
-  int levels;               // 1: workgroups are numbered by column block, then sequence (mla_tile.hip)
+  int levels;               // workgroups are numbered by column block (1) or piece (2), then sequence (mla_tile.hip)
   int wave_cols;            // 1: every wave takes 16 columns of its own over all keys (prompts: neighbouring tokens
                             //    walk the same keys at the same time, so the rows come from the cache near the CU);
                             // 0: the 4 waves share 16 columns and split the keys (few query tokens)
@@ -33,7 +33,7 @@ struct MlaTilePlan {
   int nsplit;               // pieces that a column block's keys can be cut into
   int cuts;                 // pieces of each that fill the chip, if all are alike
   long items;               // column blocks of the whole batch, at most
-  int levels;               // 1: sequences of about one length, several column blocks each
+  int levels;               // 1: sequences of about one length, several column blocks each; 2: a few of one block each; 0: by their lengths
 };
 MlaTilePlan mla_tile_plan(int S, int T_tokens, int H, int BS, int max_blocks, int max_q);
 int mla_tile_launch(const MlaParams& p, const MlaTilePlan& plan, int S, int dtype, bool f8, hipStream_t st);
