@@ -226,3 +226,17 @@ def test_few_sequences_piece_by_piece(S, H, new, fp8):
         ops.mla_attention(out, q, kc, vt, table, lens, starts, 192 ** -0.5, new, 8, window=window)
         want = R.mla_attention(q, kc, vt, table, lens, starts, 192 ** -0.5, 1.0, window)
         torch.testing.assert_close(out.float(), want.float(), atol=12 * 2.0 ** -9, rtol=2.0 ** -8)
+
+
+@pytest.mark.parametrize("S,H,new", [(3, 16, 51), (7, 16, 60), (2, 128, 45), (5, 1, 800)])
+def test_ragged_prompts_that_run_at_once(S, H, new):
+    """As many column blocks as CUs at most: by block, then sequence, whatever the lengths; a sequence without a new token among them."""
+    news = _ragged(S, new)
+    if S > 3:
+        news[1] = 0
+    kc, vt, table, lens, starts = _batch(news, news, 16, torch.bfloat16, S + H)
+    q = torch.randn(sum(news), H, DK, device=DEV).to(torch.bfloat16)
+    out = torch.full((sum(news), H, DV), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ops.mla_attention(out, q, kc, vt, table, lens, starts, 192 ** -0.5, max(news), 1)
+    want = R.mla_attention(q, kc, vt, table, lens, starts, 192 ** -0.5)
+    torch.testing.assert_close(out.float(), want.float(), atol=12 * 2.0 ** -9, rtol=2.0 ** -8)
