@@ -88,17 +88,32 @@ def test_copies_have_landed_before_rows_take_their_place(kernels):
         assert rows >= 16, which
 
 
+def _in_the_key_loop(body):
+    """Blocks with products that lead back to themselves."""
+    blocks, after = _blocks(body)
+    for i, b in enumerate(blocks):
+        if not any(t.startswith("v_mfma") for t in b):
+            continue
+        seen, todo = set(), list(after[i])
+        while todo:
+            k = todo.pop()
+            if k not in seen:
+                seen.add(k)
+                todo += after[k]
+        if i in seen:
+            yield b
+
+
 def test_key_loop_fetches_nothing_from_scratch(kernels):
     """A register that comes back from scratch inside the key loop is waited for together with every copy issued before it."""
     for which, body in kernels.items():
-        blocks, after = _blocks(body)
-        for i, b in enumerate(blocks):
-            if not any(t.startswith("v_mfma") for t in b):
-                continue
-            seen, todo = set(), list(after[i])
-            while todo:
-                k = todo.pop()
-                if k not in seen:
-                    seen.add(k)
-                    todo += after[k]
-            assert i not in seen or not any(t.startswith("scratch_") for t in b), which
+        for b in _in_the_key_loop(body):
+            assert not any(t.startswith("scratch_") for t in b), which
+
+
+def test_key_loop_moves_no_sums(kernels):
+    """The products that add to the sums are opaque statements: a sum that the compiler copied just before or after one would lack the waits that
+    it places around its own products."""
+    for which, body in kernels.items():
+        for b in _in_the_key_loop(body):
+            assert not any(t.startswith("v_accvgpr_") for t in b), which
