@@ -212,3 +212,34 @@ def test_the_largest_word_is_finite_noise(V, seed, token, k):
     got = ops.sample(x.to(DEV), None, torch.tensor([k], dtype=torch.int32, device=DEV) if k else None, None, None,
                      torch.tensor([seed], device=DEV))
     assert int(got) != token and float(x[0, int(got)]) > -10.0
+
+
+# logits on the bins' edges, far from zero (2^23 bins of 1 / 128 are 65536), in steps wider than the bins that are kept, and a single one far above the
+# others; fractions close to one, and lists around the number that is ranked at once
+@pytest.mark.parametrize("shape", ["edges", "far", "beyond", "steep", "peak", "hot"])
+def test_bins_cut_where_the_one_workgroup_form_does(shape):
+    g = torch.Generator().manual_seed(len(shape))
+    S, V = 48, 8191
+    x = torch.randn(S, V, generator=g) * 2.0
+    temp = 0.4 + torch.rand(S, generator=g)
+    if shape == "edges":
+        x, temp = (x * 128).round() / 128, torch.ones(S)
+    elif shape == "far":
+        x = x + torch.where(torch.arange(S) % 2 == 0, 65000.0, -2.0e5)[:, None]
+    elif shape == "beyond":
+        x = x * 60
+    elif shape == "steep":
+        temp = torch.full((S,), 2e-4)
+    elif shape == "peak":
+        x[:, 77] = 90.0
+    else:
+        temp = torch.full((S,), 30.0)
+    r = torch.arange(S)
+    k = torch.where(r % 3 == 1, torch.randint(1, 1200, (S,), generator=g), 0).to(torch.int32)
+    p = torch.where(r % 3 == 1, torch.where(r % 2 == 0, 1.0, 0.9), torch.where(r % 2 == 0, 1.0 - torch.rand(S, generator=g) * 1e-4,
+                                                                                torch.rand(S, generator=g)))
+    mp = torch.where(r % 5 == 4, 0.02, 0.0)
+    seeds = torch.randint(0, 2 ** 62, (S,), generator=g)
+    args = [t.to(DEV) for t in (temp, k, p, mp, seeds)]
+    wide = torch.cat([x, torch.full((S, 1), -float("inf"))], 1)
+    assert torch.equal(ops.sample(wide.to(DEV), *args), ops.sample(x.to(DEV), *args))

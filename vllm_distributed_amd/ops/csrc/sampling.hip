@@ -8,6 +8,8 @@
 // on); shorter rows are walked by one workgroup each.
 // Reference behaviour: vllm/v1/sample/sampler.py, ops/topk_topp_sampler.py,
 // csrc/sampler.cu (apply_repetition_penalties_).
+#include <cfloat>
+
 #include "common.h"
 
 __device__ __forceinline__ uint32_t fkey(float f) {
@@ -127,11 +129,19 @@ __device__ __forceinline__ float opaque(float v) {
 // 1 / temperature
 __device__ __forceinline__ float inverse(float t) { return opaque(__builtin_amdgcn_rcpf(t)); }
 // exp(z - zmax) as a 32.32 fixed-point number; 0 of a NaN, of which both comparisons are false
-// (at most 1: a conversion to 32 bits and a case for the largest entry; to 64 bits it is ten instructions)
-__device__ __forceinline__ unsigned long long fixed_weight(float z, float zmax) {
+// (at most 1: a conversion to 32 bits, which ends at their largest and makes 0 of a NaN, and the one that the largest entry lacks
+// then; a conversion to 64 bits is ten instructions)
+struct FixedWeight { uint32_t low, largest; };           // their sum
+__device__ __forceinline__ FixedWeight weight_parts(float z, float zmax) {
   const float w = __expf(opaque(opaque(z) - zmax)) * 4294967296.f;
-  const uint32_t low = w < 4294967296.f ? (uint32_t)w : 0u;
-  return w >= 4294967296.f ? 1ull << 32 : (unsigned long long)low;
+  FixedWeight f;
+  asm("v_cvt_u32_f32 %0, %1" : "=v"(f.low) : "v"(w));
+  f.largest = w >= 4294967296.f ? 1u : 0u;
+  return f;
+}
+__device__ __forceinline__ unsigned long long fixed_weight(float z, float zmax) {
+  const FixedWeight f = weight_parts(z, zmax);
+  return (unsigned long long)f.low + f.largest;
 }
 
 // One radix descent by 1024 threads over n entries; at(i) is entry i's scaled logit.  weight(i) = 1 (COUNT) or exp(z_i - zmax) for
@@ -214,6 +224,7 @@ struct SampleArgs {
   const long* seeds;
   int V;
   long stride;
+  bool late;                   // (several workgroups a row) rows without a filter draw in the second launch
 };
 
 // One row by one workgroup of 1024.
@@ -270,43 +281,59 @@ __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs p) {
 // ---- rows over several workgroups --------------------------------------------------------------------------------
 // One workgroup per row spends up to ten passes over 0.5 MB (V = 128256) on one CU, most of the time in LDS atomics that
 // all hit the few leading bytes real logits share: 447 us for 61 rows of V = 128256, 73 us for one.  Here a row takes G
-// workgroups and four launches, 47 us and 15 us (256 rows of 151936 120):
-//   stats    the row's maximum and smallest finite value (argmax of a greedy row)
-//   bins     counts (top-k) or fixed-point weights (top-p) in SPLIT_BINS bins that are LINEAR between the maximum and the
-//            smallest value: neighbouring lanes hit different bins, and a bin holds a few hundred entries
-//   collect  draws among the entries above the bin in which the running sum reaches the target, and collects
-//            that bin's entries (top-k and top-p together: all entries down to it)
+// workgroups and three launches:
+//   survey   the maximum of a workgroup's share and, from its registers, counts (top-k) or weights (top-p) of what lies below that
+//            maximum.  The bins lie on a grid that does not depend on the row, so that the shares' sums can meet in the next launch.
+//            Rows without a filter draw here at once, greedy ones take their argmax
+//   collect  the bin in which the running sum over the row's bins reaches the target; draws among the entries above it, collects
+//            that bin's entries (top-k and top-p together: all entries down to it), and sums the exact weights
 //   finish   the exact threshold key among the collected entries, the draw among them, and the row's winner
-// Bound by the noise's 64-bit hash (45 issue slots an entry) where many entries are drawn from, by trips to memory of a
-// microsecond each elsewhere.  A fifth and a third less than a form (59 us; 185 for 256 rows of 151936) that let the entries beyond the span meet in
-// one bin's atomic (half of the 185), hashed the upper word anew for every entry,
-// listed entries with a memory atomic each and always took the radix descent at the end.  Rows without a filter draw in the collecting launch
-// alone: half of their entries in the one before gave nothing (61 rows 52.8 / 52.8 us) and cost a single row 2.5 us.  One launch for collect and
-// finish, the row's last workgroup finishing it, is no way: the fences it needs took it from 20 to 155 us.
-// A row whose bin overflows the list (thousands of equal logits) is done by its finish workgroup alone, the way of the
-// short rows.  The result is that of the one-workgroup form: the bins are monotone in the key, sums are integers, and each
-// number is rounded alike in every kernel (opaque).
-constexpr int SPLIT_BINS = 2048;      // bin 0: the maximum; the last: -inf; the last but one: beyond the span (two per thread)
+// The survey's weights are estimates, relative to the top of their bin (the row's maximum is not known yet) and of 2^-16 each.  Where the target
+// comes that close to a bin's edge, both bins are collected; and the finish, which has the exact sums, hands a row whose collected bins do not
+// hold its threshold to the one-workgroup form, so the result never hangs on the estimate.  A row whose bins overflow a list (thousands of equal
+// logits), with NaN under a top-k, or with a maximum beyond the grid goes the same way.
+// The result is that of the one-workgroup form: the bins are monotone in the key, sums are integers, and each number is rounded alike
+// in every kernel (opaque).
+// Bound by issue and by trips to memory of a microsecond each: 61 rows, kernel times: 14 where rows without a filter draw (the noise's 64-bit hash
+// is 45 issue slots an entry) and 12 where bins are counted, of 8.6 for a read; 19 in the collecting launch for rows of top-p (exact weights 12 slots
+// an entry; what is drawn from is brought together 64 entries at a time), 9 in the last.  us a call, with a launch more, in which statistics came
+// ahead of bins between the row's extremes -> this: 61 rows of 128256 48 -> 38, one 19 -> 16.5, 256 of 151936 128 -> 104, 148 of 32000 60 -> 35, five
+// 26 -> 20.  All bins of a row in every workgroup instead of groups first: 42 instead of 38.  One launch for collect and finish, the row's last
+// workgroup finishing it, is no way: the fences it needs took it from 20 to 155 us.
+constexpr int SPLIT_BINS = 4096;      // a ring in groups of 64: bin b of the grid is at b mod SPLIT_BINS; the row's top SPLIT_GROUPS groups count
+constexpr int SPLIT_GROUPS = SPLIT_BINS / 64;          // a lane each
+constexpr float SPLIT_PER = 128.f;    // bins a unit of logit (counts) or of scaled logit (weights, whose 2^-32 is 22.2 units down)
 constexpr int SPLIT_LIST = 4096;      // collected entries of a row
 constexpr int SPLIT_MAX_G = 64;
 constexpr int SPLIT_MIN_V = 8192;     // shorter rows: the launches cost more than the one-workgroup form's passes
+constexpr int SPLIT_HOLDS = 16;       // entries of a thread that the survey holds at once
+constexpr float SPLIT_FAR = 0x1p23f;  // bins; a maximum further from zero than this is not binned (bins are whole 32-bit numbers)
 // Without top-k and top-p the one-workgroup form walks a row twice, not ten times, and many rows fill the chip by themselves:
-// the launches pay from longer rows on.  Kernel times in us, one workgroup a row / several, draws (greedy rows): 8 x 16384
-// 11.9 / 13.0 (5.5 / 8.1), 8 x 32000 19.4 / 13.2 (7.9 / 8.1), 64 x 32000 19.9 / 17.7 (8.1 / 10.2), 256 x 50257 44.7 / 41.9, 600 x 50257
-// 82.9 / 99.7 (39.5 / 45.6), 600 x 65536 107 / 106.
+// the launches pay from longer rows on.  Kernel times in us, one workgroup a row / several, draws: 8 x 16384 11.3 / 9.2, 8 x 32000 17.7 / 9.5,
+// 64 x 24576 14.8 / 11.3, 256 x 32000 27.7 / 17.4, 600 x 24576 41 / 34, 600 x 50257 95 / 50; with min-p, which takes a launch more: 8 x 16384
+// 11.4 / 14, 64 x 32000 21.7 / 20, 256 x 50257 42 / 33, 600 x 32000 51 / 57.  Filtered: 8 x 8192 24.9 / 20, 256 x 8192 26 / 27, 600 x 8192 55 / 54.
 static int split_min_v(int S, bool filtered) {
   return filtered ? SPLIT_MIN_V : S <= 32 ? 24576 : S <= 256 ? 40960 : 65536;
 }
 constexpr int SPLIT_ROWS = 512;       // rows of one set of launches (bounds the workspace)
 
-struct SplitRow {                     // workspace of one row
-  unsigned long long hist[SPLIT_BINS];
-  uint2 list[SPLIT_LIST];             // (key, token)
-  float part_max[SPLIT_MAX_G], part_min[SPLIT_MAX_G], part_v[SPLIT_MAX_G];
+struct SplitRow {                     // workspace of one row: a word of each of its workgroups
+  unsigned long long total[SPLIT_MAX_G], above[SPLIT_MAX_G];      // exact weights: of everything, of what lies above the collected bins
+  float part_max[SPLIT_MAX_G];        // in logits (counts) or scaled logits
+  float part_v[SPLIT_MAX_G];
   int part_i[SPLIT_MAX_G];
-  uint32_t count;                     // of list, also past its end
-  uint32_t pad[3];
+  uint32_t part_n[SPLIT_MAX_G];       // collected entries, also past the list's end
+  uint32_t finite[SPLIT_MAX_G];       // entries above -inf (counts); SPLIT_NAN
+  uint32_t rem, counts, pad[2];       // what is left of a count in the collected bins, where one is left
 };
+struct SplitPart {                    // workspace of one workgroup
+  uint32_t hist[SPLIT_BINS], group[SPLIT_GROUPS];      // and the groups' sums: counts, or weights relative to the group's top as a float
+  uint2 list[SPLIT_LIST];             // (key, token)
+};
+constexpr uint32_t SPLIT_NAN = 0x80000000u, SPLIT_ALONE = 0xffffffffu;
+constexpr int SPLIT_RANKED = 256;     // entries that can be ranked at once
+constexpr int SPLIT_DIRECT = 96;      // and that are: n of them are n^2 / 8 cycles of LDS reads
+struct KeyWeight { uint32_t key; unsigned long long weight; };
 
 enum SplitMode { MODE_NONE, MODE_BOUNDARY, MODE_ALL };
 // what a row asks for: a count (k > 0) and / or a weight fraction (tp < 1)
@@ -329,249 +356,440 @@ __device__ __forceinline__ SplitFilter split_filter(const SampleArgs& p, int row
   return f;
 }
 
-// a workgroup's share of the row, walked four entries at a time where the row is aligned
+// a workgroup's share of the row, read four entries at a time where the row is aligned
 struct SplitChunk { int a, b; bool vec; };
+__host__ __device__ __forceinline__ int split_share(int V, int G) { return ((V + G - 1) / G + 3) & ~3; }
 __device__ __forceinline__ SplitChunk split_chunk(const float* row, int V, int G) {
-  const int per = ((V + G - 1) / G + 3) & ~3;
+  const int per = split_share(V, G);
   SplitChunk c;
   c.a = min((int)blockIdx.x * per, V);
   c.b = min(c.a + per, V);
   c.vec = (reinterpret_cast<uintptr_t>(row) & 15) == 0;
   return c;
 }
-// Eight entries a thread are on their way at once; the first of them (``ahead``) since before anything else is known of
-// the row: every trip to what another kernel has just written costs about a microsecond.  (Sixteen took the collecting kernel to 86
-// registers, which leaves a CU one workgroup of the two that the launch is cut for: 64 rows of 151936 58.5 us, so 50.2; 256 136 / 120.)
-constexpr int SPLIT_AHEAD = 2;
-struct SplitAhead { f32x4 v[SPLIT_AHEAD]; };
-__device__ __forceinline__ SplitAhead split_ahead(const float* row, SplitChunk c, int from) {
-  SplitAhead h;
-  const int nv = c.a + ((c.b - c.a) & ~3);
-#pragma unroll
-  for (int u = 0; u < SPLIT_AHEAD; ++u) {
-    const int i = from + 4 * (int)threadIdx.x + 4096 * u;
-    h.v[u] = c.vec && i < nv ? *reinterpret_cast<const f32x4*>(row + i) : f32x4{0, 0, 0, 0};
-  }
-  return h;
+// E entries a thread from ``at`` on, all asked for at once, in rising order; -inf past the share's end
+template <bool VEC> __device__ __forceinline__ int split_index(int at, int e) {
+  return VEC ? at + 4 * (int)threadIdx.x + 4096 * (e >> 2) + (e & 3) : at + (int)threadIdx.x + 1024 * e;
 }
-template <typename F>
-__device__ __forceinline__ void split_walk(const float* row, SplitChunk c, SplitAhead h, F f) {
-  if (c.vec) {
-    const int nv = c.a + ((c.b - c.a) & ~3);
-    for (int from = c.a; from < nv;) {
+// whether any of the workgroup's entries e is in the share (the same for every thread)
+template <bool VEC> __device__ __forceinline__ bool split_any(int at, int e, int end) {
+  return (VEC ? at + 4096 * (e >> 2) : at + 1024 * e) < end;
+}
+template <bool VEC, int E> __device__ __forceinline__ void split_load(const float* row, int at, int end, float (&v)[E]) {
+  if (VEC) {
 #pragma unroll
-      for (int u = 0; u < SPLIT_AHEAD; ++u) {
-        const int i = from + 4 * (int)threadIdx.x + 4096 * u;
-        if (i >= nv) break;
+    for (int u = 0; u < E / 4; ++u) {
+      const int i = split_index<true>(at, 4 * u);
+      f32x4 q = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      if (!split_any<true>(at, 4 * u, end)) {}
+      else if (i + 4 <= end) q = *reinterpret_cast<const f32x4*>(row + i);
+      else
 #pragma unroll
-        for (int j = 0; j < 4; ++j) f(h.v[u][j], i + j);
-      }
-      from += 4096 * SPLIT_AHEAD;
-      if (from < nv) h = split_ahead(row, c, from);
+        for (int j = 0; j < 3; ++j)
+          if (i + j < end) q[j] = row[i + j];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[4 * u + j] = q[j];
     }
-    for (int i = nv + threadIdx.x; i < c.b; i += 1024) f(row[i], i);
   } else {
-    for (int i = c.a + threadIdx.x; i < c.b; i += 1024) f(row[i], i);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int i = split_index<false>(at, e);
+      v[e] = -INFINITY;
+      if (split_any<false>(at, e, end) && i < end) v[e] = row[i];
+    }
   }
 }
+// the bin of x on the grid, a whole number; NaN and infinities stay what they are
+__device__ __forceinline__ float split_bin(float x) { return floorf(opaque(x) * SPLIT_PER); }
 
-// the row's maximum and the width of its bins, from the workgroups' partial results; every thread returns the same
-struct SplitScale { float zmax, per; };
-__device__ __forceinline__ float uniform(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
-// (split_parts asks for them)
-__device__ __forceinline__ f32x2 split_parts(const SplitRow* ws, int G) {
-  const int lane = threadIdx.x & 63;
-  return lane < G ? f32x2{ws->part_max[lane], ws->part_min[lane]} : f32x2{-INFINITY, INFINITY};
+// An inclusive scan over the wave in six instructions (steps inside rows of 16 lanes, then the rows' ends); ``none``: what joins nothing
+template <typename T, typename F> __device__ __forceinline__ T wave_scan(T x, T none, F join) {
+  const auto from = [&](auto ctrl, auto rows) {
+    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, none), __builtin_bit_cast(int, x), decltype(ctrl)::value,
+                                                             decltype(rows)::value, 0xf, false));
+  };
+  using std::integral_constant;
+  x = join(x, from(integral_constant<int, 0x111>(), integral_constant<int, 0xf>()));
+  x = join(x, from(integral_constant<int, 0x112>(), integral_constant<int, 0xf>()));
+  x = join(x, from(integral_constant<int, 0x114>(), integral_constant<int, 0xf>()));
+  x = join(x, from(integral_constant<int, 0x118>(), integral_constant<int, 0xf>()));
+  x = join(x, from(integral_constant<int, 0x142>(), integral_constant<int, 0xa>()));
+  x = join(x, from(integral_constant<int, 0x143>(), integral_constant<int, 0xc>()));
+  return x;
 }
-__device__ __forceinline__ SplitScale split_scale(f32x2 parts) {
-  float mx = parts[0], mn = parts[1];
-  mx = wave_max(mx);
-  mn = -wave_max(-mn);
-  // weights below 2^-32 of the largest are zero: 22.2; a k-th largest entry further down lands in the last bins
-  const float span = fminf(fmaxf(mx - mn, 1e-3f), 24.f);
-  return {mx, opaque((float)(SPLIT_BINS - 2) * opaque(__builtin_amdgcn_rcpf(span)))};
+template <typename T> __device__ __forceinline__ T scan_add(T x) { return wave_scan(x, T(0), [](T a, T b) { return a + b; }); }
+// the sum over a row of 16 lanes, in its last one
+template <typename T> __device__ __forceinline__ T row_sum(T v) {
+  const auto from = [&](auto ctrl) {
+    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value, 0xf, 0xf, false));
+  };
+  using std::integral_constant;
+  v += from(integral_constant<int, 0x111>());
+  v += from(integral_constant<int, 0x112>());
+  v += from(integral_constant<int, 0x114>());
+  v += from(integral_constant<int, 0x118>());
+  return v;
 }
-// functions of the scaled logit that never decrease as it falls
-__device__ __forceinline__ float split_place(float z, SplitScale sc) {
-  return fmaxf(opaque(opaque(sc.zmax - opaque(z)) * sc.per), 0.f);
+template <typename T> __device__ __forceinline__ T last_lane(T x) {
+  return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), 63));
 }
-__device__ __forceinline__ int split_bin(float z, SplitScale sc) {
-  if (z == -INFINITY) return SPLIT_BINS - 1;
-  return (int)fminf(split_place(z, sc), (float)(SPLIT_BINS - 2));
+__device__ __forceinline__ float all_max(float x) { return last_lane(wave_scan(x, -INFINITY, [](float a, float b) { return fmaxf(a, b); })); }
+// a thread's sum of weights (below 2^45) added over the wave, in its last lane: 20 bits and the rest
+__device__ __forceinline__ unsigned long long wave_weight(unsigned long long w) {
+  return ((unsigned long long)scan_add((uint32_t)(w >> 20)) << 20) + scan_add((uint32_t)w & 0xfffffu);
 }
 
-__global__ __launch_bounds__(1024) void split_stats_kernel(SampleArgs p, SplitRow* ws_rows, int row0) {
-  __shared__ float red[16];
-  __shared__ float rv[16];
-  __shared__ int ri[16];
-  const int rowi = row0 + blockIdx.y, G = gridDim.x;
-  SplitRow* ws = ws_rows + blockIdx.y;
-  const float* row = p.logits + (long)rowi * p.stride;
-  for (int b = blockIdx.x * 1024 + threadIdx.x; b < SPLIT_BINS; b += G * 1024) ws->hist[b] = 0ull;
-  if (blockIdx.x == 0 && threadIdx.x == 0) ws->count = 0u;
-  const SplitChunk c = split_chunk(row, p.V, G);
-  const SplitAhead ahead = split_ahead(row, c, c.a);
-  const SplitFilter f = split_filter(p, rowi);
-  if (f.greedy) {
-    ArgMax a{-INFINITY, 0x7fffffff};
-    split_walk(row, c, ahead, [&](float v, int i) { a = amax2(a, ArgMax{v, i}); });
-    a = block_argmax(a, rv, ri);
-    if (threadIdx.x == 0) { ws->part_v[blockIdx.x] = a.v; ws->part_i[blockIdx.x] = a.i; }
-    return;
-  }
-  float mx = -INFINITY, mn = INFINITY;
-  split_walk(row, c, ahead, [&](float v, int) {
-    const float z = v * f.inv_t;
-    mx = fmaxf(mx, z);
-    if (z > -INFINITY) mn = fminf(mn, z);
-  });
-  mx = block_max(mx, red);
-  mn = -block_max(-mn, red);
-  if (threadIdx.x == 0) { ws->part_max[blockIdx.x] = mx; ws->part_min[blockIdx.x] = mn; }
-}
+constexpr float SPLIT_UNIT = 1.4426950408889634f / SPLIT_PER;        // log2 of the weight between two bins
+// of bin f of a group relative to its highest bin
+__device__ __forceinline__ float group_weight(int f) { return __builtin_amdgcn_exp2f((float)(f - 63) * SPLIT_UNIT); }
 
 // a thread walks its share in order: the first of equals stays
 __device__ __forceinline__ void later(ArgMax& a, float v, int i) {
   if (v > a.v) { a.v = v; a.i = i; }
 }
-// the best of a share's entries that are drawn from without a filter
-template <bool SAME>
-__device__ __forceinline__ ArgMax split_draw_as(float inv_t, uint32_t floor_key, const float* row, SplitChunk c, const SplitAhead& ahead,
-                                                const Noise& n) {
+
+struct SurveyLds {
+  float red[16], rv[16];
+  int ri[16];
+  uint32_t finite;
+  uint4 hist[SPLIT_BINS / 2];         // two copies of each word: lanes that meet in one wait for each other
+};
+// best entry of a share: the largest (no noise), or with its noise
+template <bool VEC, typename F>
+__device__ __forceinline__ ArgMax split_best(const float* row, const SplitChunk& c, F value) {
   ArgMax a{-INFINITY, 0x7fffffff};
-  if (floor_key) {
-    split_walk(row, c, ahead, [&](float v, int i) {
-      const float z = v * inv_t;
-      if (fkey(z) >= floor_key) later(a, noisy<SAME>(z, n, i), i);
-    });
-  } else {
-    split_walk(row, c, ahead, [&](float v, int i) { later(a, noisy<SAME>(v * inv_t, n, i), i); });
+  float v[SPLIT_HOLDS];
+  for (int at = c.a; at < c.b; at += 1024 * SPLIT_HOLDS) {
+    split_load<VEC>(row, at, c.b, v);
+#pragma unroll
+    for (int e = 0; e < SPLIT_HOLDS; ++e) {
+      if (!split_any<VEC>(at, e, c.b)) break;
+      const int i = split_index<VEC>(at, e);
+      later(a, value(v[e], i), i);
+    }
   }
   return a;
 }
-__device__ __forceinline__ ArgMax split_draw(const SampleArgs& p, const SplitFilter& f, const SplitScale& sc, int rowi, const float* row,
-                                             SplitChunk c, const SplitAhead& ahead) {
-  const uint32_t floor_key = f.mp > 0.f ? fkey(sc.zmax + __logf(f.mp)) : 0u;
-  const Noise n = noise_of((uint64_t)(p.seeds ? p.seeds[rowi] : 0), c.a, c.b);
-  return n.same ? split_draw_as<true>(f.inv_t, floor_key, row, c, ahead, n) : split_draw_as<false>(f.inv_t, floor_key, row, c, ahead, n);
+template <bool VEC>
+__device__ __forceinline__ void split_survey(const SampleArgs& p, const SplitFilter& f, int rowi, const float* row, const SplitChunk& c,
+                                             SplitRow* ws, SplitPart* part, float unit, SurveyLds& s) {
+  if (f.greedy || f.mode == MODE_NONE) {
+    ArgMax a;
+    if (f.greedy || f.mp > 0.f || p.late) a = split_best<VEC>(row, c, [&](float v, int) { return v * f.inv_t; });      // (the maximum, for the floor)
+    else {
+      const Noise n = noise_of((uint64_t)(p.seeds ? p.seeds[rowi] : 0), c.a, c.b);
+      a = n.same ? split_best<VEC>(row, c, [&](float v, int i) { return noisy<true>(v * f.inv_t, n, i); })
+                 : split_best<VEC>(row, c, [&](float v, int i) { return noisy<false>(v * f.inv_t, n, i); });
+    }
+    a = block_argmax(a, s.rv, s.ri);
+    if (threadIdx.x == 0) { ws->part_max[blockIdx.x] = a.v; ws->part_v[blockIdx.x] = a.v; ws->part_i[blockIdx.x] = a.i; ws->part_n[blockIdx.x] = 0u; }
+    return;
+  }
+  s.hist[threadIdx.x] = s.hist[threadIdx.x + 1024] = uint4{0u, 0u, 0u, 0u};
+  if (threadIdx.x == 0) s.finite = 0u;
+  const float scale = f.k ? 1.f : f.inv_t;
+  float v[SPLIT_HOLDS], mx = -INFINITY;
+  uint32_t finite = 0u;
+  bool nan = false;
+  int at = c.a;
+  for (;;) {
+    split_load<VEC>(row, at, c.b, v);
+#pragma unroll
+    for (int e = 0; e < SPLIT_HOLDS; ++e) {
+      if (!split_any<VEC>(at, e, c.b)) break;
+      mx = fmaxf(mx, v[e] * scale);
+      if (f.k) {
+        finite += v[e] > -INFINITY;
+        nan |= v[e] != v[e];
+      }
+    }
+    if (at + 1024 * SPLIT_HOLDS >= c.b) break;
+    at += 1024 * SPLIT_HOLDS;
+  }
+  mx = block_max(mx, s.red);
+  if (f.k) {
+    finite = scan_add(finite);
+    const bool any = __any(nan);
+    if ((threadIdx.x & 63) == 63) atomicAdd(&s.finite, finite);
+    if (any && (threadIdx.x & 63) == 0) atomicOr(&s.finite, SPLIT_NAN);
+  }
+  const float top_group = floorf(split_bin(mx) * (1.f / 64.f));
+  uint32_t* hist = reinterpret_cast<uint32_t*>(s.hist) + (threadIdx.x & 1);
+  for (;;) {                                            // from the entries that are still held backwards
+#pragma unroll
+    for (int e = 0; e < SPLIT_HOLDS; ++e) {
+      if (!split_any<VEC>(at, e, c.b)) break;
+      const float x = v[e] * scale, b = split_bin(x);
+      if (top_group - floorf(b * (1.f / 64.f)) < (float)SPLIT_GROUPS) {
+        uint32_t w = 1u;
+        if (!f.k) w = (uint32_t)fmaf(__builtin_amdgcn_exp2f((x * SPLIT_PER - (b + 1.f)) * SPLIT_UNIT), unit, 0.5f);
+        atomicAdd(hist + 2 * ((int)b & (SPLIT_BINS - 1)), w);
+      }
+    }
+    if (at == c.a) break;
+    at -= 1024 * SPLIT_HOLDS;
+    split_load<VEC>(row, at, c.b, v);
+  }
+  __syncthreads();
+  const uint4 q0 = s.hist[2 * threadIdx.x], q1 = s.hist[2 * threadIdx.x + 1];
+  const uint4 h = {q0.x + q0.y, q0.z + q0.w, q1.x + q1.y, q1.z + q1.w};
+  *reinterpret_cast<uint4*>(part->hist + 4 * threadIdx.x) = h;
+  const int b0 = 4 * (threadIdx.x & 15);                // 16 threads a group
+  const uint32_t group = f.k ? row_sum(h.x + h.y + h.z + h.w)
+                             : __float_as_uint(row_sum((float)h.x * group_weight(b0) + (float)h.y * group_weight(b0 + 1) +
+                                                       (float)h.z * group_weight(b0 + 2) + (float)h.w * group_weight(b0 + 3)));
+  if ((threadIdx.x & 15) == 15) part->group[threadIdx.x >> 4] = group;
+  if (threadIdx.x == 0) { ws->part_max[blockIdx.x] = mx; ws->finite[blockIdx.x] = s.finite; }
 }
-// Sums in two 32-bit words, each of which 65535 entries cannot overflow: 16 bits of a weight each (the upper one up to 65536,
-// and mostly zero).  A 64-bit LDS atomic of a wave costs three times a 32-bit one.
-constexpr int SPLIT_SUMMED = 65532;
-__global__ __launch_bounds__(1024) void split_bins_kernel(SampleArgs p, SplitRow* ws_rows, int row0) {
-  __shared__ uint32_t low[SPLIT_BINS], high[SPLIT_BINS];
+__global__ __launch_bounds__(1024, 8) void split_survey_kernel(SampleArgs p, SplitRow* ws_rows, SplitPart* ws_parts, int row0, float unit) {
+  __shared__ SurveyLds s;
   const int rowi = row0 + blockIdx.y;
+  const float* row = p.logits + (long)rowi * p.stride;
+  const SplitChunk c = split_chunk(row, p.V, gridDim.x);
+  const SplitFilter f = split_filter(p, rowi);
+  SplitPart* part = ws_parts + (long)blockIdx.y * gridDim.x + blockIdx.x;
+  if (c.vec) split_survey<true>(p, f, rowi, row, c, ws_rows + blockIdx.y, part, unit, s);
+  else split_survey<false>(p, f, rowi, row, c, ws_rows + blockIdx.y, part, unit, s);
+}
+
+// Where a row is cut: entries of ``draw_from`` and more are drawn from at once, others of ``list_from`` and more (and above -inf) are
+// collected.  In logits (counts) or scaled logits: a bin's edges are multiples of 1 / SPLIT_PER.
+struct SplitCut {
+  float draw_from, list_from;
+  uint32_t rem, n;                    // counts: what is left of k in the collected bins, the entries that these hold
+  bool counts;                        // whether a count cuts among them
+};
+struct CollectLds {
+  float rv[16];
+  int ri[16];
+  uint32_t n;
+  unsigned long long sum[2];
+  uint2 queue[16][128];
+};
+
+// Where a row's bins reach the target, the same in all of its workgroups and waves: the group by the groups' sums, a lane each, then the bin among
+// the group's 64.  (All bins of all shares at once are G^2 histograms a row: as much to read as the logits, 4 us of 61 rows.)
+constexpr int SPLIT_ASKED = 8;        // workgroups whose sums are asked for at once
+struct SplitSums { uint32_t h[SPLIT_ASKED]; };
+__device__ __forceinline__ SplitSums split_sums(const SplitPart* parts, int w0, int G, int word) {
+  SplitSums r;
+#pragma unroll
+  for (int j = 0; j < SPLIT_ASKED; ++j) r.h[j] = (&parts[min(w0 + j, G - 1)].hist[0])[word];
+  return r;
+}
+// a lane's word over the workgroups.  A ring's word stands for one of the row's groups if that is not above the workgroup's own highest group
+// (``highest``, of the workgroup that is this lane's number).
+template <typename F>
+__device__ __forceinline__ void split_join(const SplitPart* parts, SplitSums sums, int G, int word, int group, int highest, F add) {
+  for (int w = 0;;) {
+#pragma unroll
+    for (int j = 0; j < SPLIT_ASKED; ++j) {
+      const int own = __builtin_amdgcn_readlane(highest, min(w + j, SPLIT_MAX_G - 1));
+      add(w + j < G && group <= own ? sums.h[j] : 0u);
+    }
+    w += SPLIT_ASKED;
+    if (w >= G) return;
+    sums = split_sums(parts, w, G, word);
+  }
+}
+__device__ __forceinline__ SplitCut split_cut(const SplitFilter& f, const SplitPart* parts, const SplitSums& sums, int G, int highest, int row_top,
+                                              uint32_t finite, float margin) {
+  const int lane = threadIdx.x & 63, row_group = row_top >> 6;
+  // sums came by word of the ring; from the row's highest group down: lane l takes the word of group row_group - l
+  const int word = lane, mine = row_group - ((row_group - word) & (SPLIT_GROUPS - 1));
+  const int from = 4 * ((row_group - lane) & (SPLIT_GROUPS - 1));
+  const auto edge = [&](int bin) { return (float)bin * (1.f / SPLIT_PER); };
+  SplitCut cut{-FLT_MAX, INFINITY, 0u, 0u, false};
+  if (f.k) {
+    const uint32_t k = (uint32_t)f.k;
+    uint32_t count = 0u;
+    split_join(parts, sums, G, SPLIT_BINS + word, mine, highest, [&](uint32_t h) { count += h; });
+    count = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)count);
+    const uint32_t cum = scan_add(count), all = last_lane(cum);
+    if (k <= all) {
+      const int l = __ffsll(__ballot(cum >= k)) - 1, group = row_group - l, at = 64 * (group & (SPLIT_GROUPS - 1)) + 63 - lane;
+      const uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)(cum - count), l);
+      uint32_t bin = 0u;
+      split_join(parts, split_sums(parts, 0, G, at), G, at, group, highest, [&](uint32_t h) { bin += h; });
+      const uint32_t upto = before + scan_add(bin);
+      const int b = __ffsll(__ballot(upto >= k)) - 1;
+      const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)bin, b), above = (uint32_t)__builtin_amdgcn_readlane((int)upto, b) - n;
+      cut = SplitCut{edge(64 * group + 64 - b), edge(64 * group + 63 - b), k - above, n, true};
+    } else if (k <= finite) {
+      cut = SplitCut{edge(64 * (row_group - SPLIT_GROUPS + 1)), -INFINITY, k - all, finite - all, true};
+    }
+    if (f.mode == MODE_ALL) {          // (a count that keeps every finite entry: the fraction is one of all of them)
+      cut.n = !cut.counts ? finite : cut.n + f.k - cut.rem;
+      cut.rem = (uint32_t)f.k;
+      if (!cut.counts) cut.list_from = -INFINITY;
+      cut.draw_from = INFINITY;
+    }
+  } else {
+    float weight = 0.f;
+    split_join(parts, sums, G, SPLIT_BINS + word, mine, highest, [&](uint32_t h) { weight += __uint_as_float(h); });
+    weight = __int_as_float(__builtin_amdgcn_ds_bpermute(from, __float_as_int(weight)));
+    // (relative to the maximum's group's top)
+    weight *= __builtin_amdgcn_exp2f((float)(-64 * lane) * SPLIT_UNIT);
+    const float cum = scan_add(weight), all = last_lane(cum), target = f.tp * all, off = margin * all;
+    const unsigned long long reached = __ballot(cum + off >= target);
+    const int l = reached ? __ffsll(reached) - 1 : 0, group = row_group - l, at = 64 * (group & (SPLIT_GROUPS - 1)) + 63 - lane;
+    const float before = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cum - weight), l));
+    float bin = 0.f;
+    split_join(parts, split_sums(parts, 0, G, at), G, at, group, highest, [&](uint32_t h) { bin += (float)h; });
+    const float upto = before + scan_add(bin * __builtin_amdgcn_exp2f((float)(-64 * l - lane) * SPLIT_UNIT));
+    const unsigned long long lo = __ballot(upto + off >= target), hi = __ballot(upto - off >= target);
+    // (the target at the group's end: the next group's first bin joins, and the finish has the last word)
+    const int b = lo ? __ffsll(lo) - 1 : 63, e = hi ? __ffsll(hi) - 1 : 64;
+    cut.draw_from = edge(64 * group + 64 - b);
+    cut.list_from = edge(64 * group + 63 - e);
+  }
+  return cut;
+}
+
+// COUNTS, WEIGHS: which of them cuts the row; neither: every entry is drawn from
+template <bool VEC, bool SAME, bool COUNTS, bool WEIGHS>
+__device__ __forceinline__ ArgMax split_collect(const SplitFilter& f, const float* row, const SplitChunk& c, float (&v)[8], const Noise& noise,
+                                                float zmax, SplitCut cut, SplitPart* part, CollectLds& s) {
+  const int lane = threadIdx.x & 63;
+  const float floor_z = f.mp > 0.f ? zmax + __logf(f.mp) : -INFINITY;
+  const uint32_t floor_key = f.mp > 0.f ? fkey(floor_z) : 0u;
+  const float list_from = fmaxf(cut.list_from, -FLT_MAX);
+  uint2* queue = s.queue[threadIdx.x >> 6];
+  // (the total is one of the weights' lower parts here; their ``largest`` lies among what is drawn from or collected)
+  unsigned long long total = 0ull, above = 0ull;
+  ArgMax a{-INFINITY, 0x7fffffff};
+  int held = 0;                                         // of the wave's queue, below 64 between two entries
+  auto draw = [&](int from, int n) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (lane < n) {
+      const uint2 q = queue[from + lane];
+      const float z = __uint_as_float(q.x);
+      if (WEIGHS) {
+        const FixedWeight w = weight_parts(z, zmax);
+        above += (unsigned long long)w.low + w.largest;
+        total += w.largest;
+      }
+      if (fkey(z) >= floor_key) a = amax2(a, ArgMax{noisy<SAME>(z, noise, (int)q.y), (int)q.y});
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  };
+  for (int at = c.a; at < c.b;) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      if (!split_any<VEC>(at, e, c.b)) break;
+      const int i = split_index<VEC>(at, e);
+      const float z = v[e] * f.inv_t, x = WEIGHS ? z : v[e];
+      if (!COUNTS && !WEIGHS) {
+        if (fkey(z) >= floor_key) later(a, noisy<SAME>(z, noise, i), i);
+        continue;
+      }
+      if (WEIGHS) total += weight_parts(z, zmax).low;
+      const bool drawn = x >= cut.draw_from && (WEIGHS || z >= floor_z);
+      const unsigned long long mask = __ballot(drawn);
+      if (mask) {
+        if (drawn) queue[held + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u))] =
+            make_uint2(__float_as_uint(z), (uint32_t)i);
+        held += __popcll(mask);
+        if (held >= 64) {
+          held -= 64;
+          draw(held, 64);
+        }
+      }
+      if (x >= list_from && x < cut.draw_from) {
+        if (WEIGHS) total += weight_parts(z, zmax).largest;
+        const uint32_t to = atomicAdd(&s.n, 1u);
+        if (to < (uint32_t)SPLIT_LIST) part->list[to] = make_uint2(fkey(z), (uint32_t)i);
+      }
+    }
+    at += 8192;
+    if (at < c.b) split_load<VEC>(row, at, c.b, v);
+  }
+  draw(0, held);
+  if (WEIGHS) {
+    total = wave_weight(total);
+    above = wave_weight(above);
+    if (lane == 63) {
+      atomicAdd(&s.sum[0], total);
+      atomicAdd(&s.sum[1], above);
+    }
+  }
+  return a;
+}
+
+// (64 registers, and fewer scalar ones than the 106 that it took by itself, leave a CU its second workgroup)
+__global__ __launch_bounds__(1024, 8) void split_collect_kernel(SampleArgs p, SplitRow* ws_rows, SplitPart* ws_parts, int row0, float margin) {
+  __shared__ CollectLds s;
+  const int rowi = row0 + blockIdx.y, G = gridDim.x, lane = threadIdx.x & 63;
   SplitRow* ws = ws_rows + blockIdx.y;
   const float* row = p.logits + (long)rowi * p.stride;
-  SplitChunk c = split_chunk(row, p.V, gridDim.x);
-  SplitAhead ahead = split_ahead(row, c, c.a);
-  const f32x2 parts = split_parts(ws, gridDim.x);
+  const SplitChunk c = split_chunk(row, p.V, G);
+  // everything that is wanted first is on its way before anything is known of the row
+  float v[8];
+  if (c.vec) split_load<true>(row, c.a, c.b, v);
+  else split_load<false>(row, c.a, c.b, v);
+  const float part_max = lane < G ? ws->part_max[lane] : -INFINITY;
+  const uint32_t part_finite = lane < G ? ws->finite[lane] : 0u;
+  const SplitPart* parts = ws_parts + (long)blockIdx.y * G;
+  SplitSums sums;
+  if (p.top_k || p.top_p) sums = split_sums(parts, 0, G, SPLIT_BINS + lane);
   const SplitFilter f = split_filter(p, rowi);
-  if (f.greedy || f.mode == MODE_NONE) return;
-  const SplitScale sc = split_scale(parts);
-  const int end = c.b;
-  for (;;) {
-#pragma unroll
-    for (int b = threadIdx.x; b < SPLIT_BINS; b += 1024) { low[b] = 0u; high[b] = 0u; }
-    __syncthreads();
-    c.b = min(c.a + SPLIT_SUMMED, end);
-    if (f.k) {
-      // most of a row far below its maximum, or masked, is one bin: lanes that meet there wait for each other
-      uint32_t beyond = 0u, masked = 0u;
-      split_walk(row, c, ahead, [&](float v, int) {
-        const int b = split_bin(v * f.inv_t, sc);
-        beyond += b == SPLIT_BINS - 2;
-        masked += b == SPLIT_BINS - 1;
-        if (b < SPLIT_BINS - 2) atomicAdd(&low[b], 1u);
-      });
-      if (beyond) atomicAdd(&low[SPLIT_BINS - 2], beyond);
-      if (masked) atomicAdd(&low[SPLIT_BINS - 1], masked);
-    } else {
-      split_walk(row, c, ahead, [&](float v, int) {
-        const float z = v * f.inv_t;
-        const unsigned long long w = fixed_weight(z, sc.zmax);
-        const int b = split_bin(z, sc);
-        const uint32_t lo = (uint32_t)w & 0xffffu, hi = (uint32_t)(w >> 16);
-        if (lo) atomicAdd(&low[b], lo);
-        if (hi) atomicAdd(&high[b], hi);
-      });
+  if (f.greedy || (f.mode == MODE_NONE && !(f.mp > 0.f) && !p.late)) return;
+  if (threadIdx.x == 0) { s.n = 0u; s.sum[0] = s.sum[1] = 0ull; }
+  const float mx = all_max(part_max), zmax = f.k ? mx * f.inv_t : mx, top = split_bin(mx);
+  SplitCut cut{-FLT_MAX, INFINITY, 0u, 0u, false};
+  bool alone = false;
+  if (f.mode != MODE_NONE) {
+    alone = !(fabsf(top) < SPLIT_FAR) || (f.k && __any((part_finite & SPLIT_NAN) != 0u));
+    if (!alone) {
+      const uint32_t finite = last_lane(scan_add(part_finite));
+      cut = split_cut(f, parts, sums, G, (int)fmaxf(split_bin(part_max), -SPLIT_FAR) >> 6, (int)top, finite, margin);
+      alone = cut.n > (uint32_t)SPLIT_LIST;
     }
-    __syncthreads();
-#pragma unroll
-    for (int b = threadIdx.x; b < SPLIT_BINS; b += 1024) {
-      const unsigned long long sum = ((unsigned long long)high[b] << 16) + low[b];
-      if (sum) atomicAdd(&ws->hist[b], sum);
-    }
-    c.a = c.b;
-    if (c.a >= end) return;
-    ahead = split_ahead(row, SplitChunk{c.a, min(c.a + SPLIT_SUMMED, end), c.vec}, c.a);
-    __syncthreads();
+  }
+  ArgMax a{-INFINITY, 0x7fffffff};
+  if (!alone) {
+    __syncthreads();                                     // (what thread 0 cleared)
+    SplitPart* part = ws_parts + (long)blockIdx.y * G + blockIdx.x;
+    const Noise n = noise_of((uint64_t)(p.seeds ? p.seeds[rowi] : 0), c.a, c.b);
+#define COLLECT(VEC, SAME)                                                                                       \
+    a = f.mode == MODE_NONE ? split_collect<VEC, SAME, false, false>(f, row, c, v, n, zmax, cut, part, s)        \
+        : f.k ? split_collect<VEC, SAME, true, false>(f, row, c, v, n, zmax, cut, part, s)                       \
+              : split_collect<VEC, SAME, false, true>(f, row, c, v, n, zmax, cut, part, s)
+    if (c.vec && n.same) COLLECT(true, true);
+    else if (c.vec) COLLECT(true, false);
+    else if (n.same) COLLECT(false, true);
+    else COLLECT(false, false);
+#undef COLLECT
+  }
+  a = block_argmax(a, s.rv, s.ri);
+  if (threadIdx.x == 0) {
+    const int w = blockIdx.x;
+    ws->part_v[w] = a.v;
+    ws->part_i[w] = a.i;
+    ws->part_n[w] = alone ? SPLIT_ALONE : s.n;
+    ws->total[w] = s.sum[0];
+    ws->above[w] = s.sum[1];
+    if (w == 0) { ws->rem = cut.rem; ws->counts = cut.counts; }
   }
 }
 
-// Where the running sum over the bins reaches the target: the bin, what is left of the target there, and (counts)
-// how many entries it and all before it hold.  bin -1: no weight at all, nothing is filtered.
-struct SplitCut { int bin; unsigned long long rem, upto; };
-// w: the sums of the two bins that are this thread's.
-typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ SplitCut split_cut(u64x2 w, const SplitFilter& f, unsigned long long* s_wave /*[16]*/,
-                                              SplitCut* s_cut) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  unsigned long long cum = w[0] + w[1];
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const unsigned long long up = __shfl_up(cum, o, 64);
-    if (lane >= o) cum += up;
-  }
-  if (lane == 63) s_wave[wid] = cum;
-  if (threadIdx.x == 0) *s_cut = SplitCut{-1, 0ull, 0ull};
-  __syncthreads();
-  unsigned long long total = 0ull;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    if (i < wid) cum += s_wave[i];
-    total += s_wave[i];
-  }
-  unsigned long long remaining;
-  if (f.k) remaining = (unsigned long long)f.k;
-  else {
-    remaining = (unsigned long long)((double)f.tp * (double)total);
-    if (remaining < 1ull) remaining = 1ull;
-  }
-  const unsigned long long before = cum - w[0] - w[1];
-  if (w[0] > 0ull && before < remaining && before + w[0] >= remaining)
-    *s_cut = SplitCut{2 * (int)threadIdx.x, remaining - before, before + w[0]};
-  else if (w[1] > 0ull && before + w[0] < remaining && cum >= remaining)
-    *s_cut = SplitCut{2 * (int)threadIdx.x + 1, remaining - before - w[0], cum};
-  __syncthreads();
-  return *s_cut;
-}
-
-// Rows that one workgroup finishes by itself: counts that say before collecting that the list is too short
-// (top-k and top-p together list everything down to the cut, without the -inf entries), and rows of nothing but -inf.
-__device__ __forceinline__ bool split_alone(const SplitFilter& f, const SplitCut& cut, const SplitScale& sc) {
-  if (sc.zmax == -INFINITY) return true;
-  if (f.mode != MODE_ALL) return false;
-  const unsigned long long n = cut.bin == SPLIT_BINS - 1 ? (unsigned long long)f.k - cut.rem : cut.upto;
-  return n > (unsigned long long)SPLIT_LIST;
-}
-
-// The same threshold as radix_threshold over a list of 256 at most, in one go: four threads an entry sum what lies above it.
-// The key is the lowest of those above which less than the target lies (0 where there is no weight at all).
-template <bool COUNT>
-__device__ uint32_t ranked_threshold(const uint2* list, const unsigned long long* weight, int n, unsigned long long target,
-                                     float fraction, uint32_t floor_key, uint32_t* s_key) {
+// The same threshold as radix_threshold over a list of SPLIT_RANKED entries at most, in one go: four threads an entry sum what lies
+// above it.  The key is the lowest of those above which less than the target lies (0 where there is no weight at all; SPLIT_NOT where
+// the list holds less than the target).  at(i): entry i's key and its weight.
+constexpr uint32_t SPLIT_NOT = 0xffffffffu;
+template <bool COUNT, typename At>
+__device__ uint32_t ranked_threshold(At at, int n, unsigned long long target, float fraction, uint32_t floor_key, uint32_t* s_key) {
   const int i = threadIdx.x >> 2;
-  if (threadIdx.x == 0) *s_key = 0xffffffffu;
-  const uint32_t key = i < n ? list[i].x : 0u;
+  if (threadIdx.x == 0) s_key[0] = SPLIT_NOT;
+  const KeyWeight mine = i < n ? at(i) : KeyWeight{0u, 0ull};
   unsigned long long above = 0ull, total = 0ull;
   if (i < n) {
 #pragma unroll 4
     for (int j = threadIdx.x & 3; j < n; j += 4) {
-      const uint32_t k = list[j].x;
-      const unsigned long long w = COUNT ? 1ull : weight[j];
-      above += k > key ? w : 0ull;
-      if (!COUNT) total += k >= floor_key ? w : 0ull;
+      const KeyWeight other = at(j);
+      const unsigned long long w = COUNT ? 1ull : other.weight;
+      above += other.key > mine.key ? w : 0ull;
+      if (!COUNT) total += other.key >= floor_key ? w : 0ull;
     }
   }
 #pragma unroll
@@ -583,137 +801,184 @@ __device__ uint32_t ranked_threshold(const uint2* list, const unsigned long long
     target = (unsigned long long)((double)fraction * (double)total);
     if (target < 1ull) target = 1ull;
   }
-  const bool in = i < n && key >= floor_key && above < target && (COUNT || weight[i] > 0ull);
-  uint32_t lowest = in ? key : 0xffffffffu;
+  if (threadIdx.x == 0) s_key[1] = !COUNT && target > total;
+  const bool in = i < n && mine.key >= floor_key && above < target && (COUNT || mine.weight > 0ull);
+  uint32_t lowest = in ? mine.key : SPLIT_NOT;
 #pragma unroll
   for (int o = 4; o < 64; o <<= 1) lowest = min(lowest, (uint32_t)__shfl_xor((int)lowest, o, 64));
   __syncthreads();
-  if ((threadIdx.x & 63) == 0 && lowest != 0xffffffffu) atomicMin(s_key, lowest);
+  if ((threadIdx.x & 63) == 0 && lowest != SPLIT_NOT) atomicMin(s_key, lowest);
   __syncthreads();
-  const uint32_t found = *s_key;
+  const uint32_t found = s_key[0], lacks = s_key[1];
   __syncthreads();
-  return found == 0xffffffffu ? 0u : found;
+  if (!COUNT && fraction < 0.f && lacks) return SPLIT_NOT;
+  return found == SPLIT_NOT ? 0u : found;
 }
 
-__global__ __launch_bounds__(1024) void split_collect_kernel(SampleArgs p, SplitRow* ws_rows, int row0) {
-  __shared__ float rv[16];
-  __shared__ int ri[16];
-  __shared__ unsigned long long s_wave[16];
-  __shared__ SplitCut s_cut;
-  __shared__ uint32_t s_count, s_base;
-  __shared__ uint2 list[SPLIT_LIST];
-  const int rowi = row0 + blockIdx.y;
-  SplitRow* ws = ws_rows + blockIdx.y;
-  const float* row = p.logits + (long)rowi * p.stride;
-  const SplitChunk c = split_chunk(row, p.V, gridDim.x);
-  const SplitAhead ahead = split_ahead(row, c, c.a);
-  const f32x2 parts = split_parts(ws, gridDim.x);
-  const u64x2 bin_sum = reinterpret_cast<const u64x2*>(ws->hist)[threadIdx.x];
-  const SplitFilter f = split_filter(p, rowi);
-  if (f.greedy) return;
-  SplitScale sc = split_scale(parts);                     // (64 registers, two workgroups a CU: what is the row's own is in scalar ones)
-  sc = SplitScale{uniform(sc.zmax), uniform(sc.per)};
-  ArgMax a{-INFINITY, 0x7fffffff};
-  if (f.mode == MODE_NONE) {
-    a = split_draw(p, f, sc, rowi, row, c, ahead);
-  } else {
-    if (threadIdx.x == 0) s_count = 0u;
-    SplitCut cut = split_cut(bin_sum, f, s_wave, &s_cut);
-    cut.bin = __builtin_amdgcn_readfirstlane(cut.bin);
-    const bool all = f.mode == MODE_ALL;
-    // a count that reaches the -inf entries keeps every other one: none of them needs to be listed
-    const bool keeps_all = cut.bin < 0 || cut.bin == SPLIT_BINS - 1;
-    // Bins below draw_to are drawn from here, bins list_from .. list_to are collected: in places between bins, as split_bin has
-    // them ahead of its rounding down (-inf entries and those beyond the span share the place at infinity)
-    const float draw_to = all ? 0.f : keeps_all ? INFINITY : (float)cut.bin;
-    const float list_from = all ? 0.f : keeps_all ? NAN : (float)cut.bin;
-    const bool beyond = cut.bin >= SPLIT_BINS - 2;
-    const float list_end = beyond ? INFINITY : (float)(cut.bin + 1);
-    const uint32_t floor_key = f.mp > 0.f ? fkey(sc.zmax + __logf(f.mp)) : 0u;
-    const Noise noise = noise_of((uint64_t)(p.seeds ? p.seeds[rowi] : 0), c.a, c.b);
-    auto walk = [&](auto same) {
-      split_walk(row, c, ahead, [&](float v, int i) {
-        const float z = v * f.inv_t, at = split_place(z, sc);
-        if (at < draw_to) {
-          if (!floor_key || fkey(z) >= floor_key) later(a, noisy<decltype(same)::value>(z, noise, i), i);
-        } else if (at >= list_from && (at < list_end || (beyond && z != -INFINITY))) {
-          const uint32_t to = atomicAdd(&s_count, 1u);
-          if (to < (uint32_t)SPLIT_LIST) list[to] = make_uint2(fkey(z), (uint32_t)i);
-        }
-      });
-    };
-    if (!split_alone(f, cut, sc)) {
-      if (noise.same) walk(std::true_type());
-      else walk(std::false_type());
-      // this share's entries behind those of others: one atomic on the row's count
-      __syncthreads();
-      const uint32_t n = s_count;
-      if (n > 0u) {
-        if (threadIdx.x == 0) s_base = atomicAdd(&ws->count, n);
-        __syncthreads();
-        const uint32_t base = s_base;
-        for (uint32_t i = threadIdx.x; i < n && base + i < (uint32_t)SPLIT_LIST; i += 1024) ws->list[base + i] = list[i];
-      }
+// The same for more entries: a histogram of 1024 bins between the lowest and the highest key, and the one that holds the threshold ranked.
+// (The radix descent's four passes of five barriers each: 11.6 us of the launch where this takes 9.)  SPLIT_MANY: that bin holds more than SPLIT_RANKED.
+constexpr uint32_t SPLIT_MANY = 0xfffffffeu;
+struct RefineLds {
+  unsigned long long hist[1024], wave[16], rem;
+  KeyWeight few[SPLIT_RANKED];
+  uint32_t low, high, bin, n, key[2];
+};
+template <bool COUNT, typename At>
+__device__ uint32_t refined_threshold(At at, int n, unsigned long long target, float fraction, uint32_t floor_key, RefineLds& s) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  s.hist[threadIdx.x] = 0ull;
+  if (threadIdx.x == 0) { s.low = 0xffffffffu; s.high = 0u; s.bin = 0xffffffffu; s.n = 0u; }
+  __syncthreads();
+  uint32_t low = 0xffffffffu, high = 0u;
+  for (int i = threadIdx.x; i < n; i += 1024) {
+    const uint32_t key = at(i).key;
+    if (key < floor_key) continue;
+    low = min(low, key);
+    high = max(high, key);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    low = min(low, (uint32_t)__shfl_xor((int)low, o, 64));
+    high = max(high, (uint32_t)__shfl_xor((int)high, o, 64));
+  }
+  if (lane == 0) { atomicMin(&s.low, low); atomicMax(&s.high, high); }
+  __syncthreads();
+  low = s.low;
+  high = s.high;
+  if (low > high) return 0u;
+  const int shift = max(0, 22 - __clz((high - low) | 1u));
+  for (int i = threadIdx.x; i < n; i += 1024) {
+    const KeyWeight e = at(i);
+    if (e.key >= floor_key) atomicAdd(&s.hist[(high - e.key) >> shift], COUNT ? 1ull : e.weight);
+  }
+  __syncthreads();
+  const unsigned long long mine = s.hist[threadIdx.x];
+  unsigned long long cum = wave_weight(mine);            // (a bin's sum is below 2^45)
+  if (lane == 63) s.wave[wid] = cum;
+  __syncthreads();
+  unsigned long long total = 0ull;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    if (i < wid) cum += s.wave[i];
+    total += s.wave[i];
+  }
+  if (!COUNT && fraction >= 0.f) {
+    target = (unsigned long long)((double)fraction * (double)total);
+    if (target < 1ull) target = 1ull;
+  }
+  if (mine && cum >= target && cum - mine < target) { s.bin = threadIdx.x; s.rem = target - (cum - mine); }
+  __syncthreads();
+  const uint32_t bin = s.bin;
+  if (bin == 0xffffffffu) return !COUNT && fraction < 0.f ? SPLIT_NOT : 0u;
+  if (shift == 0) return high - bin;
+  for (int i = threadIdx.x; i < n; i += 1024) {
+    const KeyWeight e = at(i);
+    if (e.key >= floor_key && (high - e.key) >> shift == bin) {
+      const uint32_t to = atomicAdd(&s.n, 1u);
+      if (to < (uint32_t)SPLIT_RANKED) s.few[to] = e;
     }
   }
-  a = block_argmax(a, rv, ri);
-  if (threadIdx.x == 0) { ws->part_v[blockIdx.x] = a.v; ws->part_i[blockIdx.x] = a.i; }
+  __syncthreads();
+  if (s.n > (uint32_t)SPLIT_RANKED) return SPLIT_MANY;
+  return ranked_threshold<COUNT>([&](int i) { return s.few[i]; }, (int)s.n, s.rem, -1.f, 0u, s.key);
 }
 
-constexpr int SPLIT_RANKED = 256;     // entries; more take the radix descent (its LDS histogram holds the weights of these)
-__global__ __launch_bounds__(1024) void split_finish_kernel(SampleArgs p, SplitRow* ws_rows, int row0, int G) {
+__global__ __launch_bounds__(1024) void split_finish_kernel(SampleArgs p, const SplitRow* ws_rows, const SplitPart* ws_parts, int row0, int G) {
   __shared__ float red[16];
   __shared__ float rv[16];
   __shared__ int ri[16];
-  __shared__ unsigned long long hist[256];
+  __shared__ RefineLds s;
   __shared__ uint32_t s_sel;
-  __shared__ unsigned long long s_rem, s_wave[16];
-  __shared__ SplitCut s_cut;
+  __shared__ unsigned long long s_rem;
   __shared__ uint2 list[SPLIT_LIST];
-  const int rowi = row0 + blockIdx.x;
-  SplitRow* ws = ws_rows + blockIdx.x;
-  // everything that may be wanted in one trip (list entries past the count: nobody's)
-  const f32x2 parts = split_parts(ws, G);
-  const u64x2 bin_sum = reinterpret_cast<const u64x2*>(ws->hist)[threadIdx.x];
-  const uint2 entry = ws->list[threadIdx.x];
-  const uint32_t n = ws->count;
+  const int rowi = row0 + blockIdx.x, lane = threadIdx.x & 63;
+  const SplitRow* ws = ws_rows + blockIdx.x;
+  const SplitPart* parts = ws_parts + (long)blockIdx.x * G;
+  // everything that may be wanted in one trip (list entries past the counts: nobody's)
+  const int each = 1024 / G, from = threadIdx.x / each, slot = threadIdx.x % each;      // of workgroup from's list
+  const uint2 entry = parts[min(from, G - 1)].list[slot];
+  const bool there = lane < G;
+  const float part_max = there ? ws->part_max[lane] : -INFINITY;
+  const uint32_t part_n = there ? ws->part_n[lane] : 0u;
+  unsigned long long total = there ? ws->total[lane] : 0ull, above = there ? ws->above[lane] : 0ull;
+  const uint32_t count_rem = ws->rem;
+  const bool counts = ws->counts != 0u;
   ArgMax a{-INFINITY, 0x7fffffff};
   if ((int)threadIdx.x < G) a = ArgMax{ws->part_v[threadIdx.x], ws->part_i[threadIdx.x]};
   const SplitFilter f = split_filter(p, rowi);
-  if (!f.greedy) {
-    const SplitScale sc = split_scale(parts);
-    SplitCut cut{-1, 0ull, 0ull};
-    if (f.mode != MODE_NONE) cut = split_cut(bin_sum, f, s_wave, &s_cut);
-    const bool all = f.mode == MODE_ALL;
-    if (n > (uint32_t)SPLIT_LIST || split_alone(f, cut, sc)) {
-      sample_row(p, rowi, sc.zmax, true, red, rv, ri, hist, &s_sel, &s_rem);
-      return;
+  if (!f.greedy && f.mode != MODE_NONE) {
+    const float mx = all_max(part_max), zmax = f.k ? mx * f.inv_t : mx;
+    const bool all = f.mode == MODE_ALL, weighs = f.tp < 1.f;
+    bool alone = __any(part_n > (uint32_t)SPLIT_LIST);
+    const uint32_t end = alone ? 0u : scan_add(part_n), n = last_lane(end);
+    alone |= n > (uint32_t)SPLIT_LIST;
+    unsigned long long target = 1ull;
+    if (weighs && !all) {                                // the exact sums say whether the collected bins hold the threshold
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        total += __shfl_xor(total, o, 64);
+        above += __shfl_xor(above, o, 64);
+      }
+      target = (unsigned long long)((double)f.tp * (double)total);
+      if (target < 1ull) target = 1ull;
+      alone |= !(above < target) || n == 0u;             // (the threshold is among what is drawn from, or nowhere)
+      target -= above;
     }
-    if (n > 0u) {
-      list[threadIdx.x] = entry;
-      for (uint32_t i = threadIdx.x + 1024; i < n; i += 1024) list[i] = ws->list[i];
+    if (!alone && n > 0u) {
+      if (!__any(part_n > (uint32_t)each)) {
+        const uint32_t of_n = (uint32_t)__shfl((int)part_n, min(from, 63), 64), of_end = (uint32_t)__shfl((int)end, min(from, 63), 64);
+        if (from < G && (uint32_t)slot < of_n) list[of_end - of_n + slot] = entry;
+      } else {                                           // longer lists: another trip
+        for (uint32_t i = threadIdx.x; i < n; i += 1024) {
+          int w = 0;
+          uint32_t start = 0u;
+          for (int k = 0; k < G; ++k) {
+            const uint32_t k_end = (uint32_t)__builtin_amdgcn_readlane((int)end, k);
+            if (i >= k_end) { w = k + 1; start = k_end; }
+          }
+          list[i] = parts[w].list[i - start];
+        }
+      }
       __syncthreads();
       auto at = [&](int i) {
         const uint32_t key = list[i].x;
         return __uint_as_float((key & 0x80000000u) ? key ^ 0x80000000u : ~key);
       };
-      uint32_t thr = 0;
+      auto counted = [&](int i) { return KeyWeight{list[i].x, 1ull}; };
+      auto weighed = [&](int i) { return KeyWeight{list[i].x, fixed_weight(at(i), zmax)}; };
+      uint32_t thr = 0u;
       // the list starts with what lies above the cut bin (all) or with that bin
-      const bool counts = f.k && cut.bin != SPLIT_BINS - 1, weighs = f.tp < 1.f;
-      if (n <= (uint32_t)SPLIT_RANKED) {
-        if (weighs && threadIdx.x < n) hist[threadIdx.x] = fixed_weight(at(threadIdx.x), sc.zmax);
-        __syncthreads();
-        if (counts) thr = ranked_threshold<true>(list, hist, (int)n, all ? (unsigned long long)f.k : cut.rem, -1.f, 0u, &s_sel);
-        if (weighs) thr = max(thr, ranked_threshold<false>(list, hist, (int)n, cut.rem, all ? f.tp : -1.f, thr, &s_sel));
+      const float fraction = all ? f.tp : -1.f;
+      if (n <= (uint32_t)SPLIT_DIRECT) {
+        if (counts) thr = ranked_threshold<true>(counted, (int)n, count_rem, -1.f, 0u, s.key);
+        if (weighs) {
+          if (threadIdx.x < n) s.few[threadIdx.x] = weighed(threadIdx.x);
+          __syncthreads();
+          const uint32_t by_weight = ranked_threshold<false>([&](int i) { return s.few[i]; }, (int)n, target, fraction, thr, s.key);
+          alone = by_weight == SPLIT_NOT;
+          thr = max(thr, by_weight);
+        }
       } else {
-        if (counts) thr = radix_threshold<true>(at, (int)n, sc.zmax, all ? (float)f.k : (float)cut.rem, 0ull, 0u, hist, &s_sel, &s_rem);
-        if (weighs)
-          thr = max(thr, radix_threshold<false>(at, (int)n, sc.zmax, f.tp, all ? 0ull : cut.rem, thr, hist, &s_sel, &s_rem));
+        if (counts) thr = refined_threshold<true>(counted, (int)n, count_rem, -1.f, 0u, s);
+        __syncthreads();
+        alone = thr == SPLIT_MANY;
+        if (weighs && !alone) {
+          const uint32_t by_weight = refined_threshold<false>(weighed, (int)n, target, fraction, thr, s);
+          __syncthreads();
+          alone = by_weight >= SPLIT_MANY;
+          thr = max(thr, by_weight);
+        }
       }
-      if (f.mp > 0.f) thr = max(thr, fkey(sc.zmax + __logf(f.mp)));
-      const uint64_t seed = (uint64_t)(p.seeds ? p.seeds[rowi] : 0);
-      for (uint32_t i = threadIdx.x; i < n; i += 1024)
-        if (list[i].x >= thr) a = amax2(a, ArgMax{noisy(at((int)i), seed, (int)list[i].y), (int)list[i].y});
+      if (!alone) {
+        if (f.mp > 0.f) thr = max(thr, fkey(zmax + __logf(f.mp)));
+        const uint64_t seed = (uint64_t)(p.seeds ? p.seeds[rowi] : 0);
+        for (uint32_t i = threadIdx.x; i < n; i += 1024)
+          if (list[i].x >= thr) a = amax2(a, ArgMax{noisy(at((int)i), seed, (int)list[i].y), (int)list[i].y});
+      }
+    }
+    if (alone) {
+      sample_row(p, rowi, zmax, true, red, rv, ri, s.hist, &s_sel, &s_rem);
+      return;
     }
   }
   a = block_argmax(a, rv, ri);
@@ -781,16 +1046,24 @@ VDA_EXPORT int vda_argmax(const void* logits, long* out, int S, int V, long stri
   return 0;
 }
 
+// Workgroups of a row: two of 1024 threads per CU and no more (61 rows in nine parts are 549, and the last 37 cost as much as all the
+// others), at least a float4 for every thread
+static int split_groups(int rows, int V) { return max(1, min(min(SPLIT_ROWS / rows, (V + 4095) / 4096), SPLIT_MAX_G)); }
+
 // bytes of workspace that vda_sample wants for rows of V entries, with top_k or top_p (filtered) or without (0: none)
 VDA_EXPORT long vda_sample_workspace(int S, int V, int filtered) {
-  return V < split_min_v(S, filtered) ? 0 : (long)sizeof(SplitRow) * (S < SPLIT_ROWS ? S : SPLIT_ROWS);
+  if (V < split_min_v(S, filtered)) return 0;
+  long parts = 0;
+  for (int rows : {min(S, SPLIT_ROWS), S % SPLIT_ROWS})
+    if (rows > 0) parts = max(parts, (long)rows * split_groups(rows, V));
+  return (long)sizeof(SplitRow) * min(S, SPLIT_ROWS) + (long)sizeof(SplitPart) * parts;
 }
 
 VDA_EXPORT int vda_sample(const float* logits, long* out, const float* temperature, const int* top_k,
                           const float* top_p, const float* min_p, const long* seeds, int S, int V, long stride,
                           void* workspace, long workspace_bytes, hipStream_t st) {
   if (S == 0) return 0;
-  const SampleArgs p{logits, out, temperature, top_k, top_p, min_p, seeds, V, stride};
+  SampleArgs p{logits, out, temperature, top_k, top_p, min_p, seeds, V, stride, false};
   const bool filtered = top_k || top_p;
   if (V < split_min_v(S, filtered)) {
     hipLaunchKernelGGL(sample_kernel, dim3(S), dim3(1024), 0, st, p);
@@ -799,15 +1072,20 @@ VDA_EXPORT int vda_sample(const float* logits, long* out, const float* temperatu
   }
   if (!workspace || workspace_bytes < vda_sample_workspace(S, V, filtered)) return -1;
   SplitRow* ws = (SplitRow*)workspace;
+  SplitPart* parts = (SplitPart*)(ws + min(S, SPLIT_ROWS));
   for (int row0 = 0; row0 < S; row0 += SPLIT_ROWS) {
-    const int rows = min(S - row0, SPLIT_ROWS);
-    // two workgroups of 1024 threads per CU and no more (61 rows in nine parts are 549, and the last 37 cost as much as all the
-    // others), at least a float4 for every thread
-    const int G = max(1, min(min(512 / rows, (V + 4095) / 4096), SPLIT_MAX_G));
-    hipLaunchKernelGGL(split_stats_kernel, dim3(G, rows), dim3(1024), 0, st, p, ws, row0);
-    if (filtered) hipLaunchKernelGGL(split_bins_kernel, dim3(G, rows), dim3(1024), 0, st, p, ws, row0);
-    hipLaunchKernelGGL(split_collect_kernel, dim3(G, rows), dim3(1024), 0, st, p, ws, row0);
-    hipLaunchKernelGGL(split_finish_kernel, dim3(rows), dim3(1024), 0, st, p, ws, row0, G);
+    const int rows = min(S - row0, SPLIT_ROWS), G = split_groups(rows, V);
+    int bits = 16;                                       // of a weight: a share's sum fits 32
+    while (bits > 0 && (long)split_share(V, G) >> (32 - bits)) --bits;
+    const float unit = (float)(1 << bits);
+    // With min-p alone its rows need the second launch, and the others join there while the first is a matter of trips only (8 x 32000, all three
+    // launches, us: there 14.1, in the first 15.3)
+    p.late = !filtered && min_p && split_share(V, G) <= 1024 * SPLIT_HOLDS;
+    hipLaunchKernelGGL(split_survey_kernel, dim3(G, rows), dim3(1024), 0, st, p, ws, parts, row0, unit);
+    // (the estimate's rounding is half a unit a weight; 2^-32 of every entry and the sums' own are 1e-5 of the total)
+    if (filtered || min_p)
+      hipLaunchKernelGGL(split_collect_kernel, dim3(G, rows), dim3(1024), 0, st, p, ws, parts, row0, 1.f / unit + 1e-5f);
+    hipLaunchKernelGGL(split_finish_kernel, dim3(rows), dim3(1024), 0, st, p, ws, parts, row0, G);
   }
   VDA_CHECK_LAUNCH();
   return 0;
