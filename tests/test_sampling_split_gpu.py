@@ -229,7 +229,7 @@ def test_bins_cut_where_the_one_workgroup_form_does(shape):
     elif shape == "beyond":
         x = x * 60
     elif shape == "steep":
-        temp = torch.full((S,), 2e-4)
+        temp = torch.where(torch.arange(S) % 2 == 0, 2e-4, 2e-5)         # scaled logits on either side of 2^23 bins
     elif shape == "peak":
         x[:, 77] = 90.0
     else:

@@ -307,7 +307,9 @@ constexpr int SPLIT_LIST = 4096;      // collected entries of a row
 constexpr int SPLIT_MAX_G = 64;
 constexpr int SPLIT_MIN_V = 8192;     // shorter rows: the launches cost more than the one-workgroup form's passes
 constexpr int SPLIT_HOLDS = 16;       // entries of a thread that the survey holds at once
-constexpr float SPLIT_FAR = 0x1p23f;  // bins; a maximum further from zero than this is not binned (bins are whole 32-bit numbers)
+// A maximum further from zero than this many bins is not binned.  Counts have to be exact, so bins are whole 32-bit numbers there; weights
+// are summed exactly later (a temperature of 1e-4 takes logits of 20 beyond 2^24 bins).
+constexpr float SPLIT_FAR = 0x1p30f, SPLIT_FAR_COUNTS = 0x1p23f;
 // Without top-k and top-p the one-workgroup form walks a row twice, not ten times, and many rows fill the chip by themselves:
 // the launches pay from longer rows on.  Kernel times in us, one workgroup a row / several, draws: 8 x 16384 11.3 / 9.2, 8 x 32000 17.7 / 9.5,
 // 64 x 24576 14.8 / 11.3, 256 x 32000 27.7 / 17.4, 600 x 24576 41 / 34, 600 x 50257 95 / 50; with min-p, which takes a launch more: 8 x 16384
@@ -640,7 +642,10 @@ __device__ __forceinline__ SplitCut split_cut(const SplitFilter& f, const SplitP
     const unsigned long long lo = __ballot(upto + off >= target), hi = __ballot(upto - off >= target);
     // (the target at the group's end: the next group's first bin joins, and the finish has the last word)
     const int b = lo ? __ffsll(lo) - 1 : 63, e = hi ? __ffsll(hi) - 1 : 64;
-    cut.draw_from = edge(64 * group + 64 - b);
+    // (from 2^23 bins on the next bin is the next number)
+    const float at_b = edge(64 * group + 63 - b);
+    cut.draw_from = abs(64 * group) < 0x7fffc0 ? edge(64 * group + 64 - b)
+                                               : __int_as_float(__float_as_int(at_b) + (at_b > 0.f ? 1 : -1));
     cut.list_from = edge(64 * group + 63 - e);
   }
   return cut;
@@ -739,7 +744,7 @@ __global__ __launch_bounds__(1024, 8) void split_collect_kernel(SampleArgs p, Sp
   SplitCut cut{-FLT_MAX, INFINITY, 0u, 0u, false};
   bool alone = false;
   if (f.mode != MODE_NONE) {
-    alone = !(fabsf(top) < SPLIT_FAR) || (f.k && __any((part_finite & SPLIT_NAN) != 0u));
+    alone = !(fabsf(top) < (f.k ? SPLIT_FAR_COUNTS : SPLIT_FAR)) || (f.k && __any((part_finite & SPLIT_NAN) != 0u));
     if (!alone) {
       const uint32_t finite = last_lane(scan_add(part_finite));
       cut = split_cut(f, parts, sums, G, (int)fmaxf(split_bin(part_max), -SPLIT_FAR) >> 6, (int)top, finite, margin);
