@@ -1,0 +1,52 @@
+"""Calls of the kernel library's functions through the extension module: the same values arrive as through ctypes (no GPU: functions
+that answer from sizes, and argument checks that come ahead of a launch)."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from vllm_distributed_amd.ops import native as N
+
+pytestmark = pytest.mark.skipif(not N.is_available(), reason="libvda_ops.so is not built")
+
+
+def test_values_are_those_of_ctypes():
+    for args in ((1, 10, 32, 8, 128, 4000), (7, 2000, 28, 4, 128, 1 << 33)):
+        assert N.value("vda_prefill_parts", *args) == N.lib().vda_prefill_parts(*args)
+    for scale in (0.3, 0, 1, -1.0):                      # a float among integers; whole numbers in its place
+        args = (43, 43, 128, 576, 16, 300, 1, scale, 4)
+        assert N.value("vda_mla_splits", *args) == N.lib().vda_mla_splits(*args)
+
+
+def _decode(**change):
+    names = ("out q k v table lens starts alibi part lse S T Hq Hkv D block cols nsplit maxq qs os scale softcap window dtype fp8 ks vs "
+             "sink chunk v_shift bias far").split()
+    ok = dict(zip(names, [None] * 10 + [1, 1, 32, 8, 128, 16, 4, 1, 1, 4096, 4096, 0.1, 0.0, 0, 0, 0, 1.0, 1.0, None, 0, 0, None, 0]))
+    n = len(N._SIGS["vda_paged_attention_decode"])
+    return list(dict(ok, **change).values()) + [0] * (n - len(ok))
+
+
+# the codes of checks on arguments that go into registers, onto the stack, and lie behind four floats
+@pytest.mark.parametrize("change,code", [(dict(Hkv=5), -1), (dict(nsplit=0), -6), (dict(chunk=-1), -7), (dict(v_shift=4), -7),
+                                         (dict(maxq=9), -4), (dict(bias=64, far=-1), -7)])
+def test_a_status_names_the_function(change, code):
+    args = _decode(**change)
+    assert N.lib().vda_paged_attention_decode(*args) == code
+    assert N.value("vda_paged_attention_decode", *args) == code
+    with pytest.raises(RuntimeError, match=f"vda_paged_attention_decode failed with code {code}"):
+        N.call("vda_paged_attention_decode", *args)
+
+
+def test_other_kinds_of_arguments_go_through_ctypes():
+    assert N.value("vda_scan_lane_channel", ctypes.c_int(30), 32, True) == N.lib().vda_scan_lane_channel(30, 32, 1)
+    for bad in ("8", 2.5, np.float32(2)):
+        with pytest.raises(ctypes.ArgumentError):
+            N.value("vda_scan_lane_channel", bad, 32, 1)
+    with pytest.raises(TypeError):
+        N.value("vda_scan_lane_channel", 30)
+
+
+def test_a_function_that_is_not_there():
+    N.lib()
+    with pytest.raises(RuntimeError, match="has no kernel vda_nothing"):
+        N.call("vda_nothing", 1)

@@ -52,7 +52,7 @@ R = _ReferenceOps(_reference)
 
 
 def _dev(x: torch.Tensor) -> bool:
-    return x.is_cuda and not envs.VDA_FORCE_TORCH_OPS
+    return x.is_cuda and not (envs.is_set("VDA_FORCE_TORCH_OPS") and envs.VDA_FORCE_TORCH_OPS)
 
 
 def _contig_last(x: torch.Tensor) -> torch.Tensor:
@@ -302,11 +302,12 @@ def paged_attention_decode(out, q, k_cache, v_cache, block_table, seq_lens, q_st
             part = torch.empty(T * Hq * num_splits * (D + 1), dtype=torch.float32, device=q.device)
             part_out = part.data_ptr()
             part_lse = part_out + 4 * T * Hq * num_splits * D
+    bias, far = (None, 0) if dist_bias is None else _dist_bias_args(dist_bias, Hq)
     N.call("vda_paged_attention_decode", out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
            block_table.data_ptr(), seq_lens.data_ptr(), q_start_loc.data_ptr(), N.ptr(alibi), part_out,
            part_lse, S, T, Hq, k_cache.shape[1], D, k_cache.shape[2], block_table.stride(0), num_splits,
            max_q_len, q.stride(0), out.stride(0), scale, softcap, window, N.dt(q.dtype), _kv_fp8(k_cache), k_scale,
-           v_scale, N.ptr(sink), int(chunk), int(v_shift), *_dist_bias_args(dist_bias, Hq), N.stream())
+           v_scale, N.ptr(sink), int(chunk), int(v_shift), bias, far, N.stream())
     return out
 
 
@@ -360,16 +361,17 @@ def paged_attention_prefill(out, q, k_cache, v_cache, block_table, seq_lens, q_s
     for bound in (max_kv_len, window + 128 if window > 0 else 0, chunk + 128 if chunk > 0 else 0):
         keys = min(keys, bound) if bound > 0 else keys
     if not return_lse:
-        parts = N.lib().vda_prefill_parts(seq_lens.shape[0], T, Hq, Hkv, D, keys)
+        parts = N.value("vda_prefill_parts", seq_lens.shape[0], T, Hq, Hkv, D, keys)
         if parts > 1:
             part = torch.empty(T * Hq * parts * (D + 1), dtype=torch.float32, device=q.device)
             part_out = part.data_ptr()
             part_lse = part_out + 4 * T * Hq * parts * D
+    bias, far = (None, 0) if dist_bias is None else _dist_bias_args(dist_bias, Hq)
     N.call("vda_paged_attention_prefill", out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
            block_table.data_ptr(), seq_lens.data_ptr(), q_start_loc.data_ptr(), N.ptr(alibi), seq_lens.shape[0], T,
            Hq, Hkv, D, page, block_table.stride(0), q.stride(0), out.stride(0), scale,
            softcap, window, N.dt(q.dtype), _kv_fp8(k_cache), k_scale, v_scale, int(bool(causal)), N.ptr(lse),
-           int(max_q_len), N.ptr(sink), int(chunk), int(v_shift), *_dist_bias_args(dist_bias, Hq), part_out, part_lse, parts,
+           int(max_q_len), N.ptr(sink), int(chunk), int(v_shift), bias, far, part_out, part_lse, parts,
            keys, N.stream())
     return (out, lse) if return_lse else out
 
@@ -444,7 +446,7 @@ def mla_cache_write(kv_c: torch.Tensor, k_pe: torch.Tensor, kc: torch.Tensor, vt
 def _mla_splits(S: int, T: int, H: int, DK: int, page: int, width: int, max_q: int, scale: float, num_splits: int) -> int:
     """Parts that a sequence's keys can be cut into: the kernels of some sizes cut by a sequence's real length and say themselves
     how many there are at most, from the sizes alone (so the answer is kept: asking is 1 us of a 22 us call)."""
-    return N.lib().vda_mla_splits(S, T, H, DK, page, width, max_q, scale, num_splits)
+    return N.value("vda_mla_splits", S, T, H, DK, page, width, max_q, scale, num_splits)
 
 
 def mla_attention(out: torch.Tensor, q: torch.Tensor, kc: torch.Tensor, vt: torch.Tensor, block_table: torch.Tensor,
@@ -1486,20 +1488,22 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, topk_w: torc
             return _moe_tiled(x, w13, w2, topk_w, topk_ids, w13_scale, w2_scale, False, activation, x_scale, odt,
                               act_limit)
         x = (x.float() * x_scale.float().reshape(-1, 1)).to(odt)
-    if _dev(x) and block_scales and not moe_tiled_ok(x, w13, w2):
+    on_device = _dev(x)
+    grouped_ok = moe_grouped_ok(x, w13, w2)
+    if on_device and block_scales and not moe_tiled_ok(x, w13, w2):
         raise RuntimeError(f"block-scaled expert shapes {tuple(w13.shape)} / {tuple(w2.shape)} are outside the tiled "
                            "fp8 GEMM (hidden and expert width must be multiples of 128)")
-    if _dev(x) and not moe_grouped_ok(x, w13, w2) and not moe_tiled_ok(x, w13, w2) and moe_pairs_ok(x, w13, w2) \
+    if on_device and not grouped_ok and not moe_tiled_ok(x, w13, w2) and moe_pairs_ok(x, w13, w2) \
             and w13_scale is None and w2_scale is None:
         return _moe_pairs(_contig_last(x), w13, w2, topk_w, topk_ids, activation, act_limit)
-    if not _dev(x) or (not moe_grouped_ok(x, w13, w2) and not moe_tiled_ok(x, w13, w2)):
-        if _dev(x) and torch.cuda.is_current_stream_capturing():
+    if not on_device or (not grouped_ok and not moe_tiled_ok(x, w13, w2)):
+        if on_device and torch.cuda.is_current_stream_capturing():
             raise RuntimeError(
                 f"expert shapes {tuple(w13.shape)} / {tuple(w2.shape)} are outside the grouped MoE kernel (hidden and "
                 "expert width must be multiples of 128); the PyTorch fallback synchronises and cannot be captured "
                 "into a hipGraph: run with enforce_eager=True")
         return R.fused_moe(x, w13, w2, topk_w, topk_ids, w13_scale, w2_scale, block_scales, activation, act_limit)
-    if not moe_grouped_ok(x, w13, w2):
+    if not grouped_ok:
         return _moe_tiled(_contig_last(x), w13, w2, topk_w, topk_ids, w13_scale, w2_scale, block_scales, activation,
                           act_limit=act_limit)
     T, H = x.shape
@@ -1592,11 +1596,17 @@ def selective_scan(u: torch.Tensor, delta: torch.Tensor, A: torch.Tensor, B: tor
     # (a batch of two rows a sequence and more is one of prompts, whatever the hint says)
     step = max_query_len <= 1 and T < 2 * S
     wgch = 512 * 16 // Nst
-    paired = ssm_state.data_ptr() % 16 == 0 and A.data_ptr() % (16 if A.dim() == 2 else 4) == 0 and (step or (
+    u_at, d_at, b_at, c_at, out_at, a_at, state_at = (u.data_ptr(), delta.data_ptr(), B.data_ptr(), C.data_ptr(), out.data_ptr(),
+                                                      A.data_ptr(), ssm_state.data_ptr())
+    u_row, d_row, b_row, c_row, out_row = u.stride(0), delta.stride(0), B.stride(0), C.stride(0), out.stride(0)
+    z_at, z_row = (None, 0) if z is None else (z.data_ptr(), z.stride(0))
+    per_state = A.dim() == 2
+    # (a power of two divides several numbers where it divides what their bits are together)
+    paired = state_at % 16 == 0 and a_at % (16 if per_state else 4) == 0 and (step or (
         Ch % 2 == 0 and gch % 2 == 0 and (rep == 1 or rep % 2 == 0)
         and 2 * Nst * min(-(-wgch // gch) + 1, -(-Ch // gch)) <= 8192
-        and all(t.stride(0) % 2 == 0 and t.data_ptr() % (2 * eb) == 0
-                for t in (u, out) + ((delta,) if rep == 1 else ()) + ((z,) if z is not None else ()))))
+        and (u_row | out_row | z_row | (d_row if rep == 1 else 0)) % 2 == 0
+        and (u_at | out_at | (z_at or 0) | (d_at if rep == 1 else 0)) % (2 * eb) == 0))
     # In one pass (below 96 tokens) pairs leave half as many lanes, each with twice the work: with few of them the plain form is
     # ahead, whose lanes of 16 states are counted here.  Scan times in us, plain / pairs: 16 states a channel, one sequence of 40 tokens
     # before its inputs came a token ahead 31 / 41, 24 of 43 tokens at most with 4096 channels (98 304 lanes) 41 / 47 since, 64
@@ -1610,15 +1620,15 @@ def selective_scan(u: torch.Tensor, delta: torch.Tensor, A: torch.Tensor, B: tor
     # Two states a lane (Mamba: 16 of them, a decay rate each, a step size per channel): one pass where pairs take two.  A
     # workgroup's setup and its tile of 32 tokens want some tokens to work on: pairs / this, 128 sequences of 20 tokens at most
     # x 8192 channels 89 / 125 us, of 34 x 4096 80 / 79, 100 of 43 x 4096 87 / 75, 64 of 51 69 / 56, three of 1558 x 8192 300 / 163.
-    lanes = not step and Nst == 16 and A.dim() == 2 and rep == 1 and (num_groups == 1 or gch % 32 == 0) \
-        and ssm_state.data_ptr() % 16 == 0 and A.data_ptr() % 16 == 0 and (not few_tokens or paired and max_query_len >= 40)
+    lanes = not step and Nst == 16 and per_state and rep == 1 and (num_groups == 1 or gch % 32 == 0) \
+        and state_at % 16 == 0 and a_at % 16 == 0 and (not few_tokens or paired and max_query_len >= 40)
     # Eight states a lane (Mamba-2 in 16 bits: 64 states and more, a decay rate per head), from 16 tokens on.  us, pairs / this, 4096
     # channels x 128 states: one of 80 tokens 61 / 20, of 482 114 / 70, three of 1558 at most 598 / 254, 16 of 173 226 / 118, of 17
     # 27.6 / 25.8, 64 of 34 123 / 121, of 8 49 / 70
     own = 2048 // Nst                                                  # channels of a workgroup
-    groups = not step and Nst in (64, 128, 256) and A.dim() == 1 and eb == 2 and max_query_len >= 16 \
-        and Ch % own == 0 and rep % own == 0 and gch % own == 0 and ssm_state.data_ptr() % 16 == 0 \
-        and all(t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (B, C))
+    groups = not step and Nst in (64, 128, 256) and not per_state and eb == 2 and max_query_len >= 16 \
+        and Ch % own == 0 and rep % own == 0 and gch % own == 0 and state_at % 16 == 0 \
+        and (b_row | c_row) % 8 == 0 and (b_at | c_at) % 16 == 0
     paired = paired or lanes or groups
     chunk, nchunks, ws_p, ws_h = 0, 1, None, None
     # unless the setting says otherwise, from 96 tokens on in pairs (seven prompts of 82 tokens on average, 4096 x 16: 140 us in
@@ -1647,11 +1657,9 @@ def selective_scan(u: torch.Tensor, delta: torch.Tensor, A: torch.Tensor, B: tor
     if nchunks > 1:
         ws_p = torch.empty((S, nchunks, Ch) if paired else (S, nchunks, Ch, Nst), dtype=torch.float32, device=u.device)
         ws_h = torch.empty((S, nchunks, Ch, Nst), dtype=torch.float32, device=u.device)
-    args = (out.data_ptr(), u.data_ptr(), delta.data_ptr(), A.data_ptr(), B.data_ptr(),
-            C.data_ptr(), N.ptr(D), N.ptr(z), N.ptr(delta_bias), ssm_state.data_ptr(), query_start_loc.data_ptr(),
-            seq_lens.data_ptr(), block_table.data_ptr(), block_table.stride(0), S, Ch, Nst,
-            u.stride(0), delta.stride(0), B.stride(0), C.stride(0), z.stride(0) if z is not None else 0, out.stride(0),
-            rep, int(A.dim() == 1), gch, int(softplus))
+    args = (out_at, u_at, d_at, a_at, b_at, c_at, N.ptr(D), z_at, N.ptr(delta_bias), state_at, query_start_loc.data_ptr(),
+            seq_lens.data_ptr(), block_table.data_ptr(), block_table.stride(0), S, Ch, Nst, u_row, d_row, b_row, c_row, z_row, out_row,
+            rep, int(not per_state), gch, int(softplus))
     if paired:
         N.call("vda_selective_scan_pairs", *args, 2 if lanes else 3 if groups else int(step), chunk, nchunks, N.ptr(ws_p), N.ptr(ws_h), N.dt(u.dtype), N.stream())
     else:

@@ -7,6 +7,7 @@ Produces, next to this file:
     libvda_ops.so    HIP kernels of ops/csrc/*.hip (C ABI, loaded with ctypes)
     libvda_comm.so   peer-memory collectives of parallel/csrc
     libvda_host.so   host-only runtime of runtime/csrc (g++): shared-memory RPC ring
+    _vda_call.so     calls of libvda_ops.so's functions from Python (binding/call.cpp, g++)
 Object files and content hashes live in ops/build/ so unchanged sources are
 not recompiled.
 """
@@ -18,6 +19,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -40,6 +42,14 @@ LIBS = {
         "dir": os.path.join(PKG, "runtime", "csrc"),
         "out": os.path.join(PKG, "runtime", "libvda_host.so"),
         "ldflags": ["-lpthread", "-lrt"],
+        "host": True,
+    },
+    # Python's way to the C functions of libvda_ops.so (g++, an extension module)
+    "_vda_call.so": {
+        "dir": os.path.join(HERE, "binding"),
+        "out": os.path.join(HERE, "_vda_call.so"),
+        "ldflags": [],
+        "cflags": ["-I" + sysconfig.get_paths()["include"]],
         "host": True,
     },
 }
@@ -142,7 +152,7 @@ def build(force: bool = False, jobs: int | None = None, verbose: bool = True, on
         changed = False
         host = spec.get("host", False)
         cc = (shutil.which("g++") or "g++") if host else None
-        fl = ["-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-DNDEBUG"] if host else flags
+        fl = ["-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-DNDEBUG", *spec.get("cflags", [])] if host else flags
         with ThreadPoolExecutor(jobs) as ex:
             for src, did in ex.map(lambda a: _compile_one(a[0], a[1], fl + ([] if host else EXTRA_FLAGS.get(
                     os.path.basename(a[0]), [])), force, cc), zip(srcs, objs)):

@@ -1,4 +1,5 @@
-"""ctypes binding of libvda_ops.so (HIP kernels with a C ABI).
+"""Binding of libvda_ops.so (HIP kernels with a C ABI): loaded with ctypes, called through the extension module
+``_vda_call`` (``call``: status functions, ``value``: functions that answer with a number).
 
 Kernels are launched on PyTorch's current HIP stream, so they order with
 PyTorch work and are captured by ``torch.cuda.graph`` like any other launch.
@@ -144,21 +145,42 @@ def is_available() -> bool:
     return os.path.exists(library_path())
 
 
+_KINDS = {c_void_p: "P", c_int: "I", c_long: "L", c_float: "F"}
+
+
+def _bind(name: str, fn) -> None:
+    from . import _vda_call
+    _vda_call.bind(name, ctypes.cast(fn, c_void_p).value, "".join(_KINDS[a] for a in fn.argtypes), fn)
+
+
+def _missing(name: str) -> None:
+    raise RuntimeError(f"{library_path()} has no kernel {name}: it was built from a subset of the sources; "
+                       "run `python -m vllm_distributed_amd.ops.build` to complete it")
+
+
 def lib() -> ctypes.CDLL:
-    global _LIB
+    global _LIB, call, value
     if _LIB is None:
         path = library_path()
         if not os.path.exists(path):
             raise RuntimeError(
                 f"{path} is missing: build it with `python -m vllm_distributed_amd.ops.build` "
                 "(the HIP kernels are mandatory on the GPU path)")
-        _LIB = ctypes.CDLL(path)
+        try:
+            from . import _vda_call
+        except ImportError as e:
+            raise RuntimeError("ops/_vda_call.so is missing: build it with `python -m vllm_distributed_amd.ops.build`") from e
+        loaded = ctypes.CDLL(path)
         for name, sig in _SIGS.items():
-            fn = getattr(_LIB, name, None)
+            fn = getattr(loaded, name, None)
             if fn is None:
                 continue       # optional symbol (e.g. MoE kernels are registered by their module)
             fn.argtypes = sig
             fn.restype = c_long if name in _LONG_RESULTS else c_int
+            if name not in _LONG_RESULTS:
+                _bind(name, fn)
+        _vda_call.on_missing(_missing)
+        _LIB, call, value = loaded, _vda_call.call, _vda_call.value
     return _LIB
 
 
@@ -168,6 +190,7 @@ def register(name: str, sig: list) -> None:
         fn = getattr(_LIB, name)
         fn.argtypes = sig
         fn.restype = c_int
+        _bind(name, fn)
 
 
 def stream() -> int:
@@ -187,11 +210,14 @@ def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
+# Until the library is loaded; then these are the extension module's own functions
 def call(name: str, *args) -> None:
-    fn = getattr(lib(), name, None)
-    if fn is None:
-        raise RuntimeError(f"{library_path()} has no kernel {name}: it was built from a subset of the sources; "
-                           "run `python -m vllm_distributed_amd.ops.build` to complete it")
-    rc = fn(*args)
-    if rc != 0:
-        raise RuntimeError(f"{name} failed with code {rc}")
+    """Run the C function ``name``; RuntimeError unless it answers 0."""
+    lib()
+    return call(name, *args)
+
+
+def value(name: str, *args) -> int:
+    """What the C function ``name`` answers (an int)."""
+    lib()
+    return value(name, *args)
