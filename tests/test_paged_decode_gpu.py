@@ -102,3 +102,36 @@ def test_two_parts(D, Hq, Hkv, S, fp8):
         _check(lens, [1] * S, Hq, Hkv, D, 16, torch.bfloat16, fp8, 2)
         if Hq // Hkv <= 4:
             _check([max(n, 4) for n in lens], [1 + i % 4 for i in range(S)], Hq, Hkv, D, 16, torch.float16, fp8, 2, window=300)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("D,BS,Hq,Hkv,nsplit", [(128, 16, 32, 8, 2), (128, 64, 8, 8, 1), (64, 32, 8, 2, 2), (256, 16, 4, 2, 1), (128, 16, 32, 8, 3)])
+def test_tables_hold_anything_past_a_sequence(D, BS, Hq, Hkv, nsplit, fp8):
+    """The first pages are asked for ahead of a sequence's length: what lies behind its last page (here the number of a page of NaN, in a
+    row that is longer than the table) is read and not used."""
+    if fp8 and D not in (64, 128):
+        pytest.skip("e4m3 caches: head sizes 64 and 128")
+    g = torch.Generator().manual_seed(D + BS)
+    lens = [1, 15, 16, 17, 33, 64, 65, 250, 300, 513, 700]
+    S, width = len(lens), 704 // BS
+    need = [-(-n // BS) for n in lens]
+    pages = torch.randperm(sum(need), generator=g).to(torch.int32)
+    nan = sum(need)
+    wide = torch.full((S, width + 9), nan, dtype=torch.int32)
+    at = 0
+    for s, n in enumerate(need):
+        wide[s, :n] = pages[at:at + n]
+        at += n
+    dt = FP8 if fp8 else torch.bfloat16
+    k, v = torch.randn(nan + 1, Hkv, BS, D, generator=g), torch.randn(nan + 1, Hkv, D, BS, generator=g)
+    k[nan], v[nan] = float("nan"), float("nan")
+    q = torch.randn(S, Hq, D, generator=g).to(torch.bfloat16).to(DEV)
+    starts = torch.arange(S + 1, dtype=torch.int32, device=DEV)
+    sl = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    kc, vc = k.to(dt).to(DEV), v.to(dt).to(DEV)
+    got = []
+    for rows in (wide.to(DEV)[:, :width], torch.where(wide == nan, 0, wide).to(DEV)):
+        out = torch.empty(S, Hq, D, dtype=torch.bfloat16, device=DEV)
+        ops.paged_attention_decode(out, q, kc, vc, rows, sl, starts, D ** -0.5, num_splits=nsplit, max_kv_len=700)
+        got.append(out)
+    assert not got[0].isnan().any() and torch.equal(got[0], got[1])

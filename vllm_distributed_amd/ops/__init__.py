@@ -307,7 +307,7 @@ def paged_attention_decode(out, q, k_cache, v_cache, block_table, seq_lens, q_st
            block_table.data_ptr(), seq_lens.data_ptr(), q_start_loc.data_ptr(), N.ptr(alibi), part_out,
            part_lse, S, T, Hq, k_cache.shape[1], D, k_cache.shape[2], block_table.stride(0), num_splits,
            max_q_len, q.stride(0), out.stride(0), scale, softcap, window, N.dt(q.dtype), _kv_fp8(k_cache), k_scale,
-           v_scale, N.ptr(sink), int(chunk), int(v_shift), bias, far, N.stream())
+           v_scale, N.ptr(sink), int(chunk), int(v_shift), bias, far, block_table.shape[1], N.stream())
     return out
 
 

@@ -38,6 +38,7 @@ struct AttnParams {
   // more, so that a lane reads the biases of consecutive keys with one clamped 16-byte load
   const float* dist_bias;
   int dist_far;
+  int table_cols;           // entries of a block table row that may be read whatever a sequence's length is (0: none); decode
 };
 
 constexpr int DIST_PAD = 32;

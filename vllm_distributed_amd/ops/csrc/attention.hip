@@ -273,18 +273,23 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(AttnParams p) {
 // keys as give every lane 16 bytes of a value row: 32 of a 16-bit cache, 64 of an e4m3 one (RUN keys in a row per lane group;
 // the 16-key MFMA tiles take keys RUN g + 4 u + i, so that the products' operands are what the lane loaded).  Rows stay raw in
 // registers until the product takes them: the next step's keys are requested as soon as the scores have used this step's, its
-// values as soon as the outputs have, and page numbers a step before that, so that no load waits for another.
+// values as soon as the outputs have, and page numbers a step before that, so that no load waits for another.  Few short sequences are a
+// chain of trips instead: in one part and without a window the first steps' pages are asked for together with the lengths, and eight
+// waves hold two steps each.
 //
 // What it measured (us, before -> after): 183 sequences of 525 .. 3675 keys, 64 / 8 heads of 128, e4m3 cache 257 -> 148 (5.3 TB/s),
 // 16-bit 310 -> 271; 256 of 1100, 64 / 8 heads, e4m3 160 -> 113, 16-bit 206 -> 200 (5.8 TB/s), of 300 keys 70 -> 64; 64 of
-// 500 .. 3500, 16 / 8 heads of 256 308 -> 203; 5 of some 390 keys 13.0 -> 11.7.  Of the first, 203 without the order of sequences below; held to the 168 registers of three
+// 500 .. 3500, 16 / 8 heads of 256 308 -> 203 (198 since four lanes' pieces of a key row lie one behind another).  Short ones, before the pages came
+// ahead and the waves' sums met in one step -> since, with rotation and cache write: 5 of some 390 keys 13.9 -> 13.4 in a graph, ten of 46, 16 / 8
+// heads of 256, 10.8 -> 9.6; as calls 64 of 600, 32 / 8 heads, 45.2 -> 44.2, 256 of 300, e4m3, 58.3 -> 55.9.  A CU takes in 31 bytes a cycle at
+// most: 675 keys of one head are 11000 cycles of the launch's 24000.  Of the first, 203 without the order of sequences below; held to the 168 registers of three
 // waves per SIMD it spills 15 and takes 177.  Non-temporal loads: e4m3 rows 6 % faster, 16-bit ones, of which a lane's pieces share
 // lines, up to 60 % slower.
 constexpr unsigned DECODE_RANKED = 512;    // two workgroups per CU are resident
 constexpr int DECODE_APART = 256;          // keys
 // WAVES: four, or eight where few sequences of few keys are asked for in two parts of four waves: the waves of one workgroup
 // do what the parts would, and their sums meet in LDS instead of in memory and another launch.  Five of some 390 keys, 32 / 8 heads of
-// 128, with rotation and cache write: 14.2 us in a graph as before, 20.0 -> 16.5 as single calls; of 96 values 12.5 -> 10.8, e4m3 14.4 -> 12.2.  Three
+// 128, with rotation and cache write: 20.0 -> 16.5 us as single calls when it came; of 96 values 12.5 -> 10.8 in a graph, e4m3 14.4 -> 12.2.  Three
 // and four parts in eight waves: 15.2 -> 17.0 and 14.8 -> 18.8 in a graph.
 template <typename T, int D, int BS, int NCT, bool F8, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void paged_decode_kernel(AttnParams p) {
@@ -293,11 +298,12 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_kernel(AttnParams p) 
   using V4 = typename Vec<T>::v4;
   constexpr int KS = D / 32;       // MFMA k-steps over the head dimension
   constexpr int NT = D / 16;       // 16-wide d tiles of the output
-  constexpr int DQ = D / 4;        // d elements owned by one lane group in QK^T
+  constexpr int PIECE = 16 / (int)sizeof(CT);        // d elements of 16 bytes: four lanes' pieces of a row lie one behind another
   constexpr int HS = F8 ? 2 : 1;   // 32-key halves of a step
   constexpr int RUN = 8 * HS, KEYS = 32 * HS;
-  constexpr int KB = DQ * (int)sizeof(CT) / 16;      // 16-byte pieces of a key row per lane
+  constexpr int KB = D / (4 * PIECE);                // pieces of a key row per lane
   constexpr int COLS = 16 * NCT;   // query columns
+  constexpr int DEPTH = WAVES == 8 && D <= 128 ? 2 : 1;      // steps whose rows a wave holds (registers of two waves a SIMD)
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, g = lane >> 4;
   // Workgroup -> (sequence, part, kv head), heads fastest.  A grid larger than the chip holds takes its sequences longest
@@ -308,7 +314,20 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_kernel(AttnParams p) 
   // batch's; e4m3 33.4 / 30.2).
   const int kvh = blockIdx.x, part = blockIdx.y;
   int seq = blockIdx.z;
+  // (the pages of the first steps, in the same trip: read(), below)
+  int page_k[DEPTH], page_v[DEPTH];
+  auto pages_ahead = [&] {
+    if (p.table_cols <= 0) return;
+    const int* row = p.block_table + (long)seq * p.max_blocks;
+#pragma unroll
+    for (int i = 0; i < DEPTH; ++i) {
+      const int st = wave + i * WAVES;
+      page_k[i] = row[min((st * KEYS + RUN * (r >> 2)) / BS, p.table_cols - 1)];
+      page_v[i] = row[min((st * KEYS + RUN * g) / BS, p.table_cols - 1)];
+    }
+  };
   int qs = p.q_start_loc[seq], q_end = p.q_start_loc[seq + 1], seq_len = p.seq_lens[seq];
+  pages_ahead();
   if (gridDim.x * gridDim.y * gridDim.z > DECODE_RANKED && p.num_seqs <= 256) {
     const int base = p.seq_lens[0], bits = min(32 - __clz(p.max_blocks * BS), 22);
     int key[4];                                         // length, then the first of the batch; no two alike
@@ -330,6 +349,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_kernel(AttnParams p) 
       }
       seq = 255 - (found & 255);
       qs = p.q_start_loc[seq]; q_end = p.q_start_loc[seq + 1]; seq_len = p.seq_lens[seq];
+      pages_ahead();
     }
   }
   const int G = p.Hq / p.Hkv;
@@ -358,21 +378,23 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_kernel(AttnParams p) 
     // a sink is a score without key or value: the running maximum starts there and the sum with its weight of one, once
     // per column: in one lane group of one wave of one part
     sink_m[ct] = (p.sink && valid && wave == 0 && part == 0) ? p.sink[head] * 1.4426950408889634f : -INFINITY;
-    const T* qp = (const T*)p.q + (long)(qs + (valid ? ti : 0)) * p.q_stride + (long)head * D + g * DQ;
+    const T* qp = (const T*)p.q + (long)(qs + (valid ? ti : 0)) * p.q_stride + (long)head * D + g * PIECE;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) qf[ct][s] = valid ? ld16<V8>(qp + 8 * s) : V8{};
+    for (int s = 0; s < KS; ++s) qf[ct][s] = valid ? ld16<V8>(qp + s / HS * 4 * PIECE + s % HS * 8) : V8{};
     col_off[ct] = valid ? (long)(qs + ti) : -1;
     if (valid) {
       wave_hi = max(wave_hi, limit[ct]); wave_lo = min(wave_lo, lower[ct]);
       full_hi = min(full_hi, limit[ct]); full_lo = max(full_lo, lower[ct]);
     }
   }
+  if (q_len > 1) {                                      // (the columns of one token see the same keys)
 #pragma unroll
-  for (int o = 8; o > 0; o >>= 1) {
-    wave_hi = max(wave_hi, __shfl_xor(wave_hi, o, 64));
-    wave_lo = min(wave_lo, __shfl_xor(wave_lo, o, 64));
-    full_hi = min(full_hi, __shfl_xor(full_hi, o, 64));
-    full_lo = max(full_lo, __shfl_xor(full_lo, o, 64));
+    for (int o = 8; o > 0; o >>= 1) {
+      wave_hi = max(wave_hi, __shfl_xor(wave_hi, o, 64));
+      wave_lo = min(wave_lo, __shfl_xor(wave_lo, o, 64));
+      full_hi = min(full_hi, __shfl_xor(full_hi, o, 64));
+      full_lo = max(full_lo, __shfl_xor(full_lo, o, 64));
+    }
   }
   wave_hi = __builtin_amdgcn_readfirstlane(wave_hi);
   wave_lo = __builtin_amdgcn_readfirstlane(wave_lo);
@@ -400,25 +422,25 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_kernel(AttnParams p) 
   const CT* vc = (const CT*)p.v_cache;
   const int hkv_v = p.Hkv >> p.v_shift, kvh_v = kvh >> p.v_shift;      // the value head behind this key head
   const int page_lo = wave_lo / BS, page_hi = max((seq_len + BS - 1) / BS - 1, 0);
-  u32x4 kr[HS][2][KB], vr[NT];
-  int kpage, vpage, vpage_next;
+  u32x4 kr[DEPTH][HS][2][KB], vr[DEPTH][NT];
+  int knext, vnext;                                     // pages of the step that is asked for next
   auto page_at = [&](int tok) { return bt[max(min(tok / BS, page_hi), page_lo)]; };
-  auto load_k = [&](int st) {          // half h, tile u, row r: key RUN (r / 4) + 8 h + 4 u + r % 4 of the step
+  auto load_k = [&](int i, int st, int page) {          // half h, tile u, row r: key RUN (r / 4) + 8 h + 4 u + r % 4 of the step
     const int tok = st * KEYS + RUN * (r >> 2) + (r & 3);
-    const CT* kp = kc + (((long)kpage * p.Hkv + kvh) * BS + tok % BS) * (long)D + g * DQ;
+    const CT* kp = kc + (((long)page * p.Hkv + kvh) * BS + tok % BS) * (long)D + g * PIECE;
 #pragma unroll
     for (int h = 0; h < HS; ++h)
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int b = 0; b < KB; ++b)
-          kr[h][u][b] = *reinterpret_cast<const u32x4*>(kp + (8 * h + 4 * u) * D + b * (16 / (int)sizeof(CT)));
+          kr[i][h][u][b] = *reinterpret_cast<const u32x4*>(kp + (8 * h + 4 * u) * D + b * 4 * PIECE);
   };
-  auto load_v = [&](int st) {
+  auto load_v = [&](int i, int st, int page) {
     const int tok = st * KEYS + RUN * g;
-    const CT* vp = vc + (((long)vpage * hkv_v + kvh_v) * (long)D + r) * BS + tok % BS;
+    const CT* vp = vc + (((long)page * hkv_v + kvh_v) * (long)D + r) * BS + tok % BS;
 #pragma unroll
-    for (int n = 0; n < NT; ++n) vr[n] = *reinterpret_cast<const u32x4*>(vp + n * 16 * BS);
+    for (int n = 0; n < NT; ++n) vr[i][n] = *reinterpret_cast<const u32x4*>(vp + n * 16 * BS);
   };
   auto operand = [](const u32x4& raw, int half) {      // 8 values: all of a 16-bit piece, one half of an e4m3 piece
     if constexpr (F8) return KVLoad<T, true>::widen(u32x2{raw[2 * half], raw[2 * half + 1]});
@@ -427,16 +449,27 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_kernel(AttnParams p) 
 
   const bool plain = !(p.softcap > 0.f) && p.alibi == nullptr && p.dist_bias == nullptr;
   const float sl2 = p.scale * 1.4426950408889634f;
-  if (step < step_hi) {
-    kpage = page_at(step * KEYS + RUN * (r >> 2));
-    vpage = page_at(step * KEYS + RUN * g);
-    load_k(step);
-    kpage = page_at((step + WAVES) * KEYS + RUN * (r >> 2));
-    vpage_next = page_at((step + WAVES) * KEYS + RUN * g);
-    load_v(step);
-    vpage = vpage_next;
+  auto pages = [&](int st) {
+    knext = page_at(st * KEYS + RUN * (r >> 2));
+    vnext = page_at(st * KEYS + RUN * g);
+  };
+#pragma unroll
+  for (int i = 0; i < DEPTH; ++i) {
+    const int st = step + i * WAVES;
+    if (st >= step_hi) break;
+    if (p.table_cols > 0) {
+      // What was read past the sequence's last page is nobody's: those keys, which are masked, are read in the step's first page
+      const int k0 = __builtin_amdgcn_readlane(page_k[i], 0), v0 = __builtin_amdgcn_readlane(page_v[i], 0);
+      knext = (st * KEYS + RUN * (r >> 2)) / BS <= page_hi ? page_k[i] : k0;
+      vnext = (st * KEYS + RUN * g) / BS <= page_hi ? page_v[i] : v0;
+    } else {
+      pages(st);
+    }
+    load_k(i, st, knext);
+    load_v(i, st, vnext);
   }
-  for (; step < step_hi; step += WAVES) {
+  if (step + DEPTH * WAVES < step_hi) pages(step + DEPTH * WAVES);
+  auto work = [&](int i, int step) {
     f32x4 s[NCT][HS][2];
 #pragma unroll
     for (int h = 0; h < HS; ++h)
@@ -446,16 +479,16 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_kernel(AttnParams p) 
         for (int ct = 0; ct < NCT; ++ct) s[ct][h][u] = f32x4{0, 0, 0, 0};
 #pragma unroll
         for (int k = 0; k < KS; ++k) {
-          const V8 a = operand(kr[h][u][k / HS], k % HS);
+          const V8 a = operand(kr[i][h][u][k / HS], k % HS);
 #pragma unroll
           for (int ct = 0; ct < NCT; ++ct) s[ct][h][u] = mfma16(a, qf[ct][k], s[ct][h][u]);
         }
       }
-    const bool more = step + WAVES < step_hi;
-    if (more) {
-      load_k(step + WAVES);
-      kpage = page_at((step + 2 * WAVES) * KEYS + RUN * (r >> 2));
-      vpage_next = page_at((step + 2 * WAVES) * KEYS + RUN * g);
+    const int ahead = step + DEPTH * WAVES;             // takes this step's place
+    int vpage = vnext;
+    if (ahead < step_hi) {
+      load_k(i, ahead, knext);
+      if (ahead + WAVES < step_hi) pages(ahead + WAVES);
     }
     __builtin_amdgcn_sched_barrier(0);
     const int tb = step * KEYS + RUN * g;               // first key of this lane's
@@ -518,15 +551,17 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_kernel(AttnParams p) 
     for (int n = 0; n < NT; ++n)
 #pragma unroll
       for (int h = 0; h < HS; ++h) {
-        const V8 a = operand(vr[n], h);
+        const V8 a = operand(vr[i][n], h);
 #pragma unroll
         for (int ct = 0; ct < NCT; ++ct) acc[ct][n] = mfma16(a, pb[ct][h], acc[ct][n]);
       }
     __builtin_amdgcn_sched_barrier(0);
-    if (more) {
-      load_v(step + WAVES);
-      vpage = vpage_next;
-    }
+    if (ahead < step_hi) load_v(i, ahead, vpage);
+  };
+  for (; step < step_hi; step += DEPTH * WAVES) {
+    work(0, step);
+    if constexpr (DEPTH == 2)
+      if (step + WAVES < step_hi) work(1, step + WAVES);
   }
 
   // lane-partial row sums -> full sums
@@ -535,65 +570,46 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_kernel(AttnParams p) 
     l[ct] += __shfl_xor(l[ct], 16, 64);
     l[ct] += __shfl_xor(l[ct], 32, 64);
   }
-  // ---- merge the waves: tree over LDS, lane-linear slots ---------------------
-  // Partner waves use the same lane -> element map, so a lane reads back exactly
-  // the slot positions its partner lane wrote: no layout change, no conflicts.
-  __shared__ f32x4 s_acc[WAVES / 2][NCT * NT][64];
-  __shared__ float s_ml[WAVES / 2][NCT][2][64];
-#pragma unroll
-  for (int cnt = WAVES / 2; cnt > 0; cnt >>= 1) {         // waves cnt .. 2 cnt - 1 send
-    if (wave >= cnt && wave < 2 * cnt) {
-      const int slot = wave - cnt;
-#pragma unroll
-      for (int ct = 0; ct < NCT; ++ct) {
-        s_ml[slot][ct][0][lane] = m[ct];
-        s_ml[slot][ct][1][lane] = l[ct];
-#pragma unroll
-        for (int n = 0; n < NT; ++n) s_acc[slot][ct * NT + n][lane] = acc[ct][n];
-      }
-    }
-    __syncthreads();
-    if (wave < cnt) {
-#pragma unroll
-      for (int ct = 0; ct < NCT; ++ct) {
-        const float m2 = s_ml[wave][ct][0][lane], l2 = s_ml[wave][ct][1][lane];
-        const float M = fmaxf(m[ct], m2);
-        const float Mu = (M == -INFINITY) ? 0.f : M;
-        const float f1 = fexp2(m[ct] - Mu), f2 = fexp2(m2 - Mu);
-        l[ct] = l[ct] * f1 + l2 * f2;
-        m[ct] = M;
-#pragma unroll
-        for (int n = 0; n < NT; ++n) acc[ct][n] = acc[ct][n] * f1 + s_acc[wave][ct * NT + n][lane] * f2;
-      }
-    }
-    __syncthreads();
-  }
-  if (wave != 0) return;
+  // ---- merge the waves: their sums meet in LDS, and every thread joins four values of a column over the waves --------
+  // (rows of D + 4: a lane's 16 bytes lie a bank group beside its neighbours'.  A tree over halves of the waves was two barriers a level)
+  constexpr int ROW = D + 4;
+  __shared__ __attribute__((aligned(16))) float s_acc[WAVES][COLS][ROW];
+  __shared__ float s_m[COLS][WAVES], s_l[COLS][WAVES];
 #pragma unroll
   for (int ct = 0; ct < NCT; ++ct) {
     if (col_off[ct] < 0) continue;
     const int c = ct * 16 + r;
+#pragma unroll
+    for (int n = 0; n < NT; ++n) *reinterpret_cast<f32x4*>(&s_acc[wave][c][16 * n + 4 * g]) = acc[ct][n];
+    if (g == 0) { s_m[c][wave] = m[ct]; s_l[c][wave] = l[ct]; }
+  }
+  __syncthreads();
+  const int columns = min(q_len * G, COLS);
+  for (int item = threadIdx.x; item < columns * (D / 4); item += 64 * WAVES) {
+    const int c = item / (D / 4), d = 4 * (item % (D / 4));
+    float M = -INFINITY, L = 0.f, f[WAVES];
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) M = fmaxf(M, s_m[c][w]);
+    const float Mu = (M == -INFINITY) ? 0.f : M;
+    f32x4 o = {0, 0, 0, 0};
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      f[w] = fexp2(s_m[c][w] - Mu);
+      L += s_l[c][w] * f[w];
+      o += *reinterpret_cast<const f32x4*>(&s_acc[w][c][d]) * f[w];
+    }
+    o *= L > 0.f ? p.v_scale / L : 0.f;
     const int head = kvh * G + c % G;
-    const float L = l[ct];
-    const float inv = L > 0.f ? p.v_scale / L : 0.f;
+    const long token = qs + c / G;
     if (p.nsplit == 1) {
-      T* op = (T*)p.out + col_off[ct] * p.out_stride + (long)head * D + 4 * g;
+      V4 to;
 #pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        V4 o;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = (T)(acc[ct][n][i] * inv);
-        *reinterpret_cast<V4*>(op + 16 * n) = o;
-      }
+      for (int i = 0; i < 4; ++i) to[i] = (T)o[i];
+      *reinterpret_cast<V4*>((T*)p.out + token * p.out_stride + (long)head * D + d) = to;
     } else {
-      const long pi = (col_off[ct] * p.Hq + head) * p.nsplit + part;
-      float* po = p.part_out + pi * D + 4 * g;
-#pragma unroll
-      for (int n = 0; n < NT; ++n) *reinterpret_cast<f32x4*>(po + 16 * n) = acc[ct][n] * inv;
-      if (g == 0) {
-        const float Mu = (m[ct] == -INFINITY) ? 0.f : m[ct];
-        p.part_lse[pi] = L > 0.f ? Mu + log2f(L) : -INFINITY;
-      }
+      const long pi = (token * p.Hq + head) * p.nsplit + part;
+      *reinterpret_cast<f32x4*>(p.part_out + pi * D + d) = o;
+      if (d == 0) p.part_lse[pi] = L > 0.f ? Mu + log2f(L) : -INFINITY;
     }
   }
 }
@@ -1147,7 +1163,7 @@ VDA_EXPORT int vda_paged_attention_decode(
     int num_seqs, int num_tokens, int Hq, int Hkv, int D, int block_size, int max_blocks, int nsplit,
     int max_q_len, long q_stride, long out_stride, float scale, float softcap, int window, int dtype,
     int kv_fp8, float k_scale, float v_scale, const float* sink, int chunk, int v_shift, const float* dist_bias,
-    int dist_far, hipStream_t st) {
+    int dist_far, int table_cols, hipStream_t st) {
   if (Hq % Hkv) return -1;
   if (chunk < 0 || v_shift < 0 || (Hkv >> v_shift) << v_shift != Hkv || (dist_bias && dist_far < 0)) return -7;
   if (nsplit < 1 || nsplit > 64) return -6;      // the reduce kernel keeps one partition per lane
@@ -1164,6 +1180,8 @@ VDA_EXPORT int vda_paged_attention_decode(
     waves = 8;
     p.nsplit = nsplit = 1;
   }
+  // the first steps are the sequence's first keys: their pages need not wait for its length
+  if (nsplit == 1 && window <= 0 && chunk == 0) p.table_cols = table_cols;
   int rc = dtype == VDA_BF16 ? dispatch_d<bf16_t>(p, D, block_size, form, num_seqs, st, kv_fp8, waves)
                              : dispatch_d<f16_t>(p, D, block_size, form, num_seqs, st, kv_fp8, waves);
   if (rc) return rc;

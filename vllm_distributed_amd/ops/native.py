@@ -42,7 +42,7 @@ _SIGS = {
     "vda_transfer_blocks_ex": [P, P, P, P, I, L, L, L, L, L, P],
     "vda_gather_cache": [P, P, P, P, P, I, I, I, I, I, P],
     "vda_paged_attention_decode": [P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, I, L, L, F, F, I, I, I, F, F, P, I,
-                                   I, P, I, P],
+                                   I, P, I, I, P],
     "vda_paged_attention_prefill": [P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, L, L, F, F, I, I, I, F, F, I, P,
                                     I, P, I, I, P, I, P, P, I, L, P],
     "vda_prefill_parts": [I, I, I, I, I, L],
