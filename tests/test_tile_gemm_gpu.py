@@ -176,3 +176,57 @@ def test_fused_moe_tiled_in_graph(monkeypatch):
     torch.cuda.synchronize()
     ref = R.fused_moe(x, w13, w2, tw2, ids2)
     assert _rel(out, ref) < 1.5e-2
+
+
+# one workgroup of 1, 4 and 16 ids a thread and their edges, several of them, more than 64 chunks; all pairs with one expert, all elsewhere; and the
+# wide tiles' table
+@pytest.mark.parametrize("n", [0, 1, 1023, 1024, 1025, 4096, 4097, 16384, 16385, 131073, 140000])
+@pytest.mark.parametrize("E,ids_of", [(1, "random"), (8, "random"), (60, "one"), (64, "elsewhere"), (1024, "random")])
+def test_pairs_are_sorted_and_cut_into_tiles(n, E, ids_of):
+    g = torch.Generator().manual_seed(n + E)
+    ids = torch.randint(-1, E, (n,), generator=g, dtype=torch.int32) if ids_of == "random" else \
+        torch.full((n,), E - 1 if ids_of == "one" else -1, dtype=torch.int32)
+    cnt = torch.bincount(ids[ids >= 0].long(), minlength=E).tolist()
+    order, off = ops.sort_by_key(ids.to(DEV), E)
+    assert off.cpu().tolist() == [0] + torch.tensor(cnt).cumsum(0).tolist()
+    for rows in (64, 128, 256):
+        sorted_ids, offsets, tiles, most = ops.moe_align_tiles(ids.view(-1, 1).to(DEV), E, rows)
+        assert torch.equal(offsets, off)
+        for got in (order, sorted_ids):
+            got = got[:sum(cnt)].cpu().long()
+            assert torch.equal(ids[got], torch.repeat_interleave(torch.arange(E, dtype=torch.int32), torch.tensor(cnt)))
+            assert got.unique().numel() == got.numel()
+        want, at = [], 0
+        for e, c in enumerate(cnt):
+            step = rows
+            if rows == 256 and c:
+                step = (-(-c // -(-c // 288)) + 31) & ~31
+            want += [(e, at + b, min(at + c, at + b + step) if rows == 256 else at + c) for b in range(0, c, step)]
+            at += c
+        assert int(tiles[3 * most]) == len(want) <= most
+        assert list(zip(*(tiles[i * most:i * most + len(want)].cpu().tolist() for i in range(3)))) == want
+
+
+@pytest.mark.parametrize("E", [8, 64, 65, 128, 160, 256, 512])
+@pytest.mark.parametrize("renorm", [True, False])
+def test_router_choice(E, renorm):
+    """Ties go to the lowest expert, NaN is never chosen, and what is left over has weight 0."""
+    g = torch.Generator().manual_seed(E)
+    x = torch.randn(70, E, generator=g)
+    x[1] = 0.0
+    x[2] = (x[2] * 2).round() / 2
+    x[3, ::2] = float("nan")
+    x[4] = -float("inf")
+    x[4, E - 1] = 1.0
+    k = min(E, 8)
+    w, ids = ops.moe_topk_softmax(x.to(DEV), k, renorm)
+    p = torch.softmax(torch.where(x.isnan(), -float("inf"), x).double(), -1)
+    order = torch.argsort(p, dim=-1, descending=True, stable=True)[:, :k]
+    want = p.gather(1, order)
+    assert bool((ids.cpu() == order)[[0, 1, 2] + list(range(5, 70))].all())
+    chosen = ids.cpu()[3][w.cpu()[3] > 0].long()
+    assert not x[3, chosen].isnan().any() and int(ids[4, 0]) == E - 1
+    if renorm:
+        want = want / want.sum(-1, keepdim=True)
+    rows = [0, 1, 2] + list(range(5, 70))
+    torch.testing.assert_close(w.cpu().double()[rows], want[rows], rtol=1e-5, atol=1e-7)      # 32-bit exponentials and sums

@@ -1152,14 +1152,10 @@ def sort_by_key(keys: torch.Tensor, num_keys: int):
         return order, off
     keys = keys.to(torch.int32)
     sorted_ids = torch.zeros(n, dtype=torch.int32, device=keys.device)
-    meta = torch.empty(3 * num_keys + 2, dtype=torch.int32, device=keys.device)
-    offsets = meta[:num_keys + 1]
-    if n > 4096:
-        N.call("vda_moe_align_large", sorted_ids.data_ptr(), offsets.data_ptr(), meta[num_keys + 1:].data_ptr(),
-               meta[2 * num_keys + 1:].data_ptr(), keys.data_ptr(), n, num_keys, N.stream())
-    else:
-        N.call("vda_moe_align", sorted_ids.data_ptr(), offsets.data_ptr(), keys.data_ptr(), n, num_keys, N.stream())
-    return sorted_ids, offsets
+    meta = torch.empty(num_keys + 1 + N.value("vda_moe_align_counts", n, num_keys), dtype=torch.int32, device=keys.device)
+    at = meta.data_ptr()
+    N.call("vda_moe_align", sorted_ids.data_ptr(), at, None, at + 4 * (num_keys + 1), keys.data_ptr(), n, num_keys, 0, 0, N.stream())
+    return sorted_ids, meta[:num_keys + 1]
 
 
 def ep_prep(topk_ids: torch.Tensor, world: int, experts_per_rank: int):
@@ -1207,20 +1203,14 @@ def moe_align_tiles(topk_ids: torch.Tensor, E: int, rows_per_tile: int):
     ids = topk_ids.contiguous().view(-1)
     n = ids.numel()
     dev = ids.device
-    sorted_ids = torch.empty(n, dtype=torch.int32, device=dev)
-    meta = torch.empty(3 * E + 2, dtype=torch.int32, device=dev)
-    offsets, counts, cursor = meta[:E + 1], meta[E + 1:2 * E + 1], meta[2 * E + 1:3 * E + 1]
-    st = N.stream()
-    if n > 4096:
-        N.call("vda_moe_align_large", sorted_ids.data_ptr(), offsets.data_ptr(), counts.data_ptr(), cursor.data_ptr(),
-               ids.data_ptr(), n, E, st)
-    else:
-        N.call("vda_moe_align", sorted_ids.data_ptr(), offsets.data_ptr(), ids.data_ptr(), n, E, st)
     max_tiles = min(n, n // rows_per_tile + E)
-    tiles = torch.empty(3 * max_tiles + 1, dtype=torch.int32, device=dev)
-    N.call("vda_moe_tile_map", tiles[:max_tiles].data_ptr(), tiles[max_tiles:2 * max_tiles].data_ptr(),
-           tiles[2 * max_tiles:3 * max_tiles].data_ptr(), tiles[3 * max_tiles:].data_ptr(), offsets.data_ptr(), E,
-           rows_per_tile, max_tiles, st)
+    # sorted pairs, tiles, offsets and what counts between the launches, in one allocation
+    meta = torch.empty(n + 3 * max_tiles + E + 2 + N.value("vda_moe_align_counts", n, E), dtype=torch.int32, device=dev)
+    sorted_ids, tiles, offsets = meta[:n], meta[n:n + 3 * max_tiles + 1], meta[n + 3 * max_tiles + 1:n + 3 * max_tiles + E + 2]
+    at = meta.data_ptr()
+    tiles_at = at + 4 * n
+    offsets_at = tiles_at + 4 * (3 * max_tiles + 1)
+    N.call("vda_moe_align", at, offsets_at, tiles_at, offsets_at + 4 * (E + 1), ids.data_ptr(), n, E, rows_per_tile, max_tiles, N.stream())
     return sorted_ids, offsets, tiles, max_tiles
 
 
@@ -1414,7 +1404,7 @@ def _moe_grouped_ungated(x, w1, w2, topk_w, topk_ids, activation: str):
     sorted_ids = torch.empty(T * k, dtype=torch.int32, device=dev)
     offsets = torch.empty(E + 1, dtype=torch.int32, device=dev)
     st = N.stream()
-    N.call("vda_moe_align", sorted_ids.data_ptr(), offsets.data_ptr(), ids.data_ptr(), T * k, E, st)
+    N.call("vda_moe_align", sorted_ids.data_ptr(), offsets.data_ptr(), None, None, ids.data_ptr(), T * k, E, 0, 0, st)
     inter = torch.empty((T * k, I), dtype=x.dtype, device=dev)
     out2 = torch.empty((T * k, H), dtype=x.dtype, device=dev)
     out = torch.empty((T, H), dtype=x.dtype, device=dev)
@@ -1527,7 +1517,7 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, topk_w: torc
     out2 = inter + n * I * eb
     sorted_ids = out2 + n * H * eb
     offsets = sorted_ids + 4 * n
-    N.call("vda_moe_align", sorted_ids, offsets, ids.data_ptr(), n, E, st)
+    N.call("vda_moe_align", sorted_ids, offsets, None, None, ids.data_ptr(), n, E, 0, 0, st)
     out = torch.empty((T, H), dtype=x.dtype, device=dev)
     wd = N.dt(w13.dtype)
     # one expert can receive at most one slot of every token

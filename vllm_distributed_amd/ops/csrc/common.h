@@ -1,6 +1,7 @@
 // Shared device helpers for the gfx950 op library.
 // Wave size is 64 everywhere; 16-bit activations are bf16 or fp16.
 #pragma once
+#include <type_traits>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -56,6 +57,27 @@ __device__ __forceinline__ float wave_max(float v) {
   for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
   return v;
 }
+
+// An inclusive scan over the wave in six instructions (steps inside rows of 16 lanes, then the rows' ends); ``none``: what joins nothing
+template <typename T, typename F> __device__ __forceinline__ T wave_scan(T x, T none, F join) {
+  const auto from = [&](auto ctrl, auto rows) {
+    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, none), __builtin_bit_cast(int, x), decltype(ctrl)::value,
+                                                             decltype(rows)::value, 0xf, false));
+  };
+  using std::integral_constant;
+  x = join(x, from(integral_constant<int, 0x111>(), integral_constant<int, 0xf>()));
+  x = join(x, from(integral_constant<int, 0x112>(), integral_constant<int, 0xf>()));
+  x = join(x, from(integral_constant<int, 0x114>(), integral_constant<int, 0xf>()));
+  x = join(x, from(integral_constant<int, 0x118>(), integral_constant<int, 0xf>()));
+  x = join(x, from(integral_constant<int, 0x142>(), integral_constant<int, 0xa>()));
+  x = join(x, from(integral_constant<int, 0x143>(), integral_constant<int, 0xc>()));
+  return x;
+}
+template <typename T> __device__ __forceinline__ T scan_add(T x) { return wave_scan(x, T(0), [](T a, T b) { return a + b; }); }
+template <typename T> __device__ __forceinline__ T last_lane(T x) {
+  return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), 63));
+}
+__device__ __forceinline__ float all_max(float x) { return last_lane(wave_scan(x, -INFINITY, [](float a, float b) { return fmaxf(a, b); })); }
 
 // Block-wide reductions for blocks of up to 1024 threads (16 waves). `red` is
 // an LDS scratch of at least 16 floats; the result is returned to every thread.

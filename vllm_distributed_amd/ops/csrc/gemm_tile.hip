@@ -1,7 +1,5 @@
 // LDS-tiled MFMA GEMM family for gfx950: the compute-bound regime (many rows per weight matrix).
 //
-//   vda_moe_tile_map      m-tile table (expert, first sorted position) from the expert offsets
-//   vda_moe_align_large   counting sort of (token, slot) pairs by expert over many workgroups
 //   vda_tile_gemm         out = epilogue(X . W^T) for one dense weight matrix or for the experts of a
 //                         routed MoE layer over expert-sorted (token, slot) pairs
 //
@@ -327,7 +325,7 @@ __global__ __launch_bounds__(512, 1) void tile_gemm_kernel(const TileGemmArgs a)
 // wave reaches with its reads of unit u done.  Read-after-write: the reads of unit u + 1 follow one that every wave reaches
 // with its copies of it landed (the AHEAD younger ones may be in flight).
 //
-// An expert's rows are cut into the fewest tiles of at most 288 rows, of like sizes (moe_tile_map_kernel): batches of 2048 or
+// An expert's rows are cut into the fewest tiles of at most 288 rows, of like sizes (align_tiles in moe.hip): batches of 2048 or
 // 4096 tokens over eight experts are 256-row tiles but for a few rows, which opened tiles of their own in half of the experts.
 // NF, the 16-row fragments of a wave, is a template argument: tiles of few rows do few MFMAs.
 //
@@ -339,7 +337,7 @@ __global__ __launch_bounds__(512, 1) void tile_gemm_kernel(const TileGemmArgs a)
 // the results of the first, which leave in bursts with the MFMAs idle, are a tenth of it.  Asking the L2 ahead for a share of each line made it 3 % slower.
 // us, eight waves of 64 x 128 sums -> this, whole layer: 4099 tokens of 8 experts 4096 x 14336, top 2, 2940 -> 2260 (1.28 PFLOP/s with rows that
 // exist); 4096 of 64 experts 2048 x 1024, top 8, 576 -> 469; 4096 of 16 experts 4096 x 6400 1453 -> 1151.
-constexpr int WIDE_ROWS = 288, WIDE_UNIT = (256 + WIDE_ROWS) * 128;
+constexpr int WIDE_UNIT = (256 + WIDE_ROWS) * 128;
 
 // 16 bytes a lane from a buffer to LDS, at dst + 16 * lane.  As a statement of its own: told of the copy, the compiler waits for
 // all of them before the next LDS read, although they fill another slot of the ring.  Waited for by the counts in the loop.
@@ -544,125 +542,6 @@ __global__ __launch_bounds__(256, 1) void moe_wide_gemm_kernel(const TileGemmArg
     case 4: case 3: return walk(std::integral_constant<int, 4>());
     default: return walk(std::integral_constant<int, 2>());
   }
-}
-
-// ---------------------------------------------------------------------------------------------
-// m-tile table: for expert e with c tokens, ceil(c / rows) tiles; with rows == 256 (the wide tiles) the fewest of at most WIDE_ROWS,
-// of like sizes in 32 rows.  One workgroup, E <= 1024.
-__global__ __launch_bounds__(1024) void moe_tile_map_kernel(int* __restrict__ tile_expert, int* __restrict__ tile_beg,
-                                                            int* __restrict__ tile_end, int* __restrict__ num_tiles,
-                                                            const int* __restrict__ offsets, int E, int rows,
-                                                            int max_tiles) {
-  __shared__ int pre[1025];
-  const int tid = threadIdx.x;
-  const bool wide = rows == 256;
-  int nt = 0, b = 0, en = 0;
-  if (tid < E) {
-    b = offsets[tid];
-    en = offsets[tid + 1];
-    if (wide) {
-      nt = (en - b + WIDE_ROWS - 1) / WIDE_ROWS;
-      rows = nt ? ((en - b + nt - 1) / nt + 31) & ~31 : rows;
-      nt = (en - b + rows - 1) / rows;
-    } else nt = (en - b + rows - 1) / rows;
-  }
-  pre[tid + 1] = nt;
-  if (tid == 0) pre[0] = 0;
-  __syncthreads();
-  // inclusive scan over 1024 entries (Hillis-Steele, 10 rounds)
-  for (int d = 1; d < 1024; d <<= 1) {
-    const int v = tid + 1 > d ? pre[tid + 1 - d] : 0;
-    __syncthreads();
-    pre[tid + 1] += v;
-    __syncthreads();
-  }
-  if (tid < E) {
-    const int first = pre[tid];
-    for (int i = 0; i < nt; ++i) {
-      const int t = first + i;
-      if (t < max_tiles) { tile_expert[t] = tid; tile_beg[t] = b + i * rows; tile_end[t] = wide ? min(en, b + (i + 1) * rows) : en; }
-    }
-  }
-  if (tid == 0) *num_tiles = min(pre[E], max_tiles);
-}
-
-VDA_EXPORT int vda_moe_tile_map(int* tile_expert, int* tile_beg, int* tile_end, int* num_tiles, const int* offsets,
-                                int E, int rows, int max_tiles, hipStream_t st) {
-  if (E < 1 || E > 1024 || rows < 1 || max_tiles < 1) return -1;
-  hipLaunchKernelGGL(moe_tile_map_kernel, dim3(1), dim3(1024), 0, st, tile_expert, tile_beg, tile_end, num_tiles,
-                     offsets, E, rows, max_tiles);
-  VDA_CHECK_LAUNCH();
-  return 0;
-}
-
-// ---------------------------------------------------------------------------------------------
-// Counting sort over many workgroups.  counts[E] must be zero on entry (the caller's memset node);
-// pass 1 histograms, pass 2 (one workgroup) turns counts into offsets and cursors, pass 3 reserves one
-// range per (workgroup, expert) with a single global atomic and scatters.  Order inside an expert is
-// not fixed between runs; every output row is computed independently of its position, so results are.
-constexpr int ALIGN_CHUNK = 2048;       // pairs per workgroup
-
-__global__ __launch_bounds__(256) void moe_hist_kernel(int* __restrict__ counts, const int* __restrict__ ids, int n, int E) {
-  __shared__ int h[1024];
-  for (int i = threadIdx.x; i < E; i += 256) h[i] = 0;
-  __syncthreads();
-  const int base = blockIdx.x * ALIGN_CHUNK;
-  for (int p = base + threadIdx.x; p < min(base + ALIGN_CHUNK, n); p += 256) {
-    const int e = ids[p];
-    if (e >= 0 && e < E) atomicAdd(&h[e], 1);
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < E; i += 256) if (h[i]) atomicAdd(&counts[i], h[i]);
-}
-
-__global__ __launch_bounds__(1024) void moe_scan_kernel(int* __restrict__ offsets, int* __restrict__ cursor,
-                                                        const int* __restrict__ counts, int E) {
-  __shared__ int pre[1025];
-  const int tid = threadIdx.x;
-  pre[tid + 1] = tid < E ? counts[tid] : 0;
-  if (tid == 0) pre[0] = 0;
-  __syncthreads();
-  for (int d = 1; d < 1024; d <<= 1) {
-    const int v = tid + 1 > d ? pre[tid + 1 - d] : 0;
-    __syncthreads();
-    pre[tid + 1] += v;
-    __syncthreads();
-  }
-  if (tid < E) { offsets[tid] = pre[tid]; cursor[tid] = pre[tid]; }
-  if (tid == 0) offsets[E] = pre[E];
-}
-
-__global__ __launch_bounds__(256) void moe_scatter_kernel(int* __restrict__ sorted, int* __restrict__ cursor,
-                                                          const int* __restrict__ ids, int n, int E) {
-  __shared__ int h[1024];
-  __shared__ int start[1024];
-  for (int i = threadIdx.x; i < E; i += 256) h[i] = 0;
-  __syncthreads();
-  const int base = blockIdx.x * ALIGN_CHUNK, lim = min(base + ALIGN_CHUNK, n);
-  for (int p = base + threadIdx.x; p < lim; p += 256) {
-    const int e = ids[p];
-    if (e >= 0 && e < E) atomicAdd(&h[e], 1);
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < E; i += 256) { start[i] = h[i] ? atomicAdd(&cursor[i], h[i]) : 0; h[i] = 0; }
-  __syncthreads();
-  for (int p = base + threadIdx.x; p < lim; p += 256) {
-    const int e = ids[p];
-    if (e >= 0 && e < E) sorted[start[e] + atomicAdd(&h[e], 1)] = p;
-  }
-}
-
-VDA_EXPORT int vda_moe_align_large(int* sorted, int* offsets, int* counts, int* cursor, const int* ids, int n, int E,
-                                   hipStream_t st) {
-  if (E < 1 || E > 1024 || n < 0) return -1;
-  hipError_t err = hipMemsetAsync(counts, 0, sizeof(int) * E, st);
-  if (err != hipSuccess) return (int)err;
-  const int blocks = (n + ALIGN_CHUNK - 1) / ALIGN_CHUNK;
-  if (blocks > 0) hipLaunchKernelGGL(moe_hist_kernel, dim3(blocks), dim3(256), 0, st, counts, ids, n, E);
-  hipLaunchKernelGGL(moe_scan_kernel, dim3(1), dim3(1024), 0, st, offsets, cursor, counts, E);
-  if (blocks > 0) hipLaunchKernelGGL(moe_scatter_kernel, dim3(blocks), dim3(256), 0, st, sorted, cursor, ids, n, E);
-  VDA_CHECK_LAUNCH();
-  return 0;
 }
 
 // ---------------------------------------------------------------------------------------------

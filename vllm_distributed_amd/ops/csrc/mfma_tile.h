@@ -3,6 +3,8 @@
 #pragma once
 #include "common.h"
 
+constexpr int WIDE_ROWS = 288;         // most rows of an expert in one of the wide tiles
+
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 

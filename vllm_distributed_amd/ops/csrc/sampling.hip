@@ -404,22 +404,6 @@ template <bool VEC, int E> __device__ __forceinline__ void split_load(const floa
 // the bin of x on the grid, a whole number; NaN and infinities stay what they are
 __device__ __forceinline__ float split_bin(float x) { return floorf(opaque(x) * SPLIT_PER); }
 
-// An inclusive scan over the wave in six instructions (steps inside rows of 16 lanes, then the rows' ends); ``none``: what joins nothing
-template <typename T, typename F> __device__ __forceinline__ T wave_scan(T x, T none, F join) {
-  const auto from = [&](auto ctrl, auto rows) {
-    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, none), __builtin_bit_cast(int, x), decltype(ctrl)::value,
-                                                             decltype(rows)::value, 0xf, false));
-  };
-  using std::integral_constant;
-  x = join(x, from(integral_constant<int, 0x111>(), integral_constant<int, 0xf>()));
-  x = join(x, from(integral_constant<int, 0x112>(), integral_constant<int, 0xf>()));
-  x = join(x, from(integral_constant<int, 0x114>(), integral_constant<int, 0xf>()));
-  x = join(x, from(integral_constant<int, 0x118>(), integral_constant<int, 0xf>()));
-  x = join(x, from(integral_constant<int, 0x142>(), integral_constant<int, 0xa>()));
-  x = join(x, from(integral_constant<int, 0x143>(), integral_constant<int, 0xc>()));
-  return x;
-}
-template <typename T> __device__ __forceinline__ T scan_add(T x) { return wave_scan(x, T(0), [](T a, T b) { return a + b; }); }
 // the sum over a row of 16 lanes, in its last one
 template <typename T> __device__ __forceinline__ T row_sum(T v) {
   const auto from = [&](auto ctrl) {
@@ -432,10 +416,6 @@ template <typename T> __device__ __forceinline__ T row_sum(T v) {
   v += from(integral_constant<int, 0x118>());
   return v;
 }
-template <typename T> __device__ __forceinline__ T last_lane(T x) {
-  return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), 63));
-}
-__device__ __forceinline__ float all_max(float x) { return last_lane(wave_scan(x, -INFINITY, [](float a, float b) { return fmaxf(a, b); })); }
 // a thread's sum of weights (below 2^45) added over the wave, in its last lane: 20 bits and the rest
 __device__ __forceinline__ unsigned long long wave_weight(unsigned long long w) {
   return ((unsigned long long)scan_add((uint32_t)(w >> 20)) << 20) + scan_add((uint32_t)w & 0xfffffu);

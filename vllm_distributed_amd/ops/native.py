@@ -63,7 +63,8 @@ _SIGS = {
     "vda_fp8_dequant": [P, P, P, L, I, P],
     "vda_skinny_gemm": [P, P, P, P, P, I, I, I, L, L, L, I, I, P],
     "vda_moe_topk_softmax": [P, P, P, I, I, I, I, L, I, P],
-    "vda_moe_align": [P, P, P, I, I, P],
+    "vda_moe_align": [P, P, P, P, P, I, I, I, I, P],
+    "vda_moe_align_counts": [I, I],
     "vda_residual_norms": [P, P, L, P, P, P, L, F, F, I, I, I, P],
     "vda_latent_norm_rope_cache": [P, L, P, L, P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, I, I, P],
     "vda_head_gate_rows": [P, P, L, L, P, L, I, I, I, I, P],
@@ -85,8 +86,6 @@ _SIGS = {
     "vda_moe_up_act": [P, P, P, P, P, I, I, I, I, I, L, I, I, I, P],
     "vda_moe_sum": [P, P, P, I, I, I, L, I, P],
     "vda_ep_prep": [P, I, I, I, P, P, P, P, P, P],
-    "vda_moe_tile_map": [P, P, P, P, P, I, I, I, P],
-    "vda_moe_align_large": [P, P, P, P, P, I, I, P],
     "vda_tile_gemm": [P, P, P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, L, L, L, I, I, I, I, I, I, F, P],
     "vda_decode_gemm": [P, P, P, P, P, L, I, I, I, L, L, I, P],
     "vda_wq_gemm": [P, P, P, P, P, P, L, I, I, I, I, I, L, L, I, I, I, P],
