@@ -199,3 +199,27 @@ def test_wide_prefill_order_of_the_tiles(lens, bound):
     out = torch.full_like(q, float("nan"))
     ops.paged_attention_prefill(out, q, kc, vc, bt, sl, qsl, 0.09, max_q_len=bound * max(lens))
     torch.testing.assert_close(out.float(), R.paged_attention(q, kc, vc, bt, sl, qsl, 0.09).float(), **tol(torch.bfloat16))
+
+
+# heads of 64 and 96 values lie in images of 128-value rows: every page size, group and option that the form takes
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Hq,Hkv", [(32, 8), (8, 1), (4, 4), (6, 2)])
+@pytest.mark.parametrize("D,bs,fp8", [(64, 16, False), (64, 32, False), (64, 64, False), (64, 16, True), (64, 64, True), (96, 16, False),
+                                      (96, 32, False), (96, 64, False)])
+def test_narrower_heads(dt, Hq, Hkv, D, bs, fp8):
+    q_lens = [5, 130, 44, 77, 1, 100, 64, 129, 300]
+    seq_lens = [5, 130, 300, 77, 1, 257, 64, 640, 300]
+    if 256 % (Hq // Hkv):
+        q_lens, seq_lens = [n + 300 for n in q_lens], [n + 300 for n in seq_lens]
+    q, kc, vc, bt, sl, qsl = _paged_problem(seq_lens, q_lens, Hq, Hkv, D, bs, dt)
+    if fp8:
+        kc, vc = (c.float().clamp(-448, 448).to(torch.float8_e4m3fn) for c in (kc, vc))
+    scale = 1.0 / math.sqrt(D)
+    out = torch.full_like(q, float("nan"))
+    _, lse = ops.paged_attention_prefill(out, q, kc, vc, bt, sl, qsl, scale, return_lse=True)
+    ref, ref_lse = R.paged_attention(q, kc, vc, bt, sl, qsl, scale, return_lse=True)
+    torch.testing.assert_close(out.float(), ref.float(), **tol(dt))
+    torch.testing.assert_close(lse, ref_lse, rtol=1e-4, atol=1e-4)           # fp32 scores and sums
+    for kw in (dict(window=64), dict(window=300), dict(softcap=30.0)):
+        ops.paged_attention_prefill(out, q, kc, vc, bt, sl, qsl, scale, **kw)
+        torch.testing.assert_close(out.float(), R.paged_attention(q, kc, vc, bt, sl, qsl, scale, **kw).float(), **tol(dt))

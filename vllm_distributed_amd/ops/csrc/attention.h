@@ -73,6 +73,6 @@ struct SparseSel {
   int NV, NS;
 };
 
-// Wide prefill form (attention_prefill.hip): 512 threads, 256 query columns per workgroup, head size 128.
+// Wide prefill form (attention_prefill.hip): 512 threads, 256 query columns per workgroup, heads of 64, 96 (16-bit caches) and 128 values.
 // Returns -100 when the shape is outside what that kernel serves (the caller then takes the 4-wave form).
-int vda_launch_prefill_wide(const AttnParams& p, int block_size, int dtype, int kv_fp8, hipStream_t st);
+int vda_launch_prefill_wide(const AttnParams& p, int D, int block_size, int dtype, int kv_fp8, hipStream_t st);

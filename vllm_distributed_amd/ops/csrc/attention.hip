@@ -1198,7 +1198,8 @@ VDA_EXPORT int vda_paged_attention_decode(
 static int g_prefill_variant = 1;
 static int prefill_cols(int D) { return D <= 128 ? PREFILL_COLS<128> : PREFILL_COLS<256>; }
 // (from 128 on: us, 4-wave form with the keys in parts / wide form, 128 of them 67.8 / 49.4 and 88 / 61, 144 25.4 / 22.8, 184 140 / 119; 100 of long
-// prompts 97 / 113, of 1000 tokens 44.6 / 39.8)
+// prompts 97 / 113, of 1000 tokens 44.6 / 39.8; heads of 64, 128 of them, 32 / 8 heads 37 / 29 and, with 2000 keys before, 125 / 89, 8 / 1 heads 74.3 / 75.4; 96,
+// 16 / 16 heads of 64 38.9 / 29.5 and on 2000 keys 52 / 80: fewer than 128 depend on the keys)
 static long g_prefill_wide_min_wgs = 128;
 VDA_EXPORT int vda_set_prefill_variant(int v) { g_prefill_variant = v; return 0; }
 VDA_EXPORT int vda_set_prefill_wide_min_wgs(long n) { g_prefill_wide_min_wgs = n; return 0; }
@@ -1207,10 +1208,25 @@ VDA_EXPORT int vda_set_prefill_wide_min_wgs(long n) { g_prefill_wide_min_wgs = n
 // most a sixteenth of them idle, or the 4-wave form takes it; and it has prompts of three of its tiles on average: us, 4-wave / wide, attention alone,
 // 28 / 4 heads, 2 x 2161 tokens 135 / 93, 8 ragged of some 200 25.0 / 20.7, 24 of 150 34.4 / 28.4, 24 / 8 heads, one of 1000 45 / 37, 2 of 2161 189 / 145; but ragged
 // ones of less, 40 / 8, 24 of 40 13.8 / 15.1, 48 / 8 14.5 / 16.6, 28 / 4 25 of 81 on 740 77 / 86.
-static int wide_tokens(int G, int num_tokens, int num_seqs) {
+static int wide_tokens(int G, int D, int num_tokens, int num_seqs) {
   const int tokens = 256 / G;
+  if (D != 64 && D != 96 && D != 128) return 0;
   if (256 % G && (tokens * G < 240 || (long)num_tokens < 3L * tokens * num_seqs)) return 0;
   return tokens;
+}
+// Whether it is taken: workgroups for half of the CUs, and prompts that fill its tiles.  Where they don't, the 4-wave form's smaller tiles do
+// less for nobody, the more so where a row of keys is short and the products little: us, 4-wave / wide, with rotary embedding and cache
+// write, n x tokens + tokens in the cache: 32 / 8 heads of 128, 160 x 20 + 300 87 / 100, 80 x 40 + 300 82 / 85, 46 x 70 + 300 80 / 72; 8 / 4, 104 x 40 + 300 48 / 52, 60 x 70
+// + 300 46 / 42; 64 / 8, 200 x 8 + 300 87 / 106, 80 x 20 76 / 79; 8 / 1, 352 x 20 + 300 59 / 50.
+// Of 96, 16 / 8 heads, 104 x 20 27 / 31, 52 x 40 25.2 / 24.6, 51 x 70 38 / 32; 16 / 16, 52 x 40 32 / 34, 51 x 70 + 300 85 / 70, 12 x 300 67 / 48.
+// Of 64, in one wave of workgroups, 32 / 8, 26 x 40 17.7 / 18.8, 15 x 70 18.1 / 16.0, 11 x 100 + 300 39 / 28, 8 / 4, 60 x 70 21 / 18; in more, 32 / 32, 32 x 100 51 / 54, 16 / 4,
+// 43 x 150 + 300 53 / 59, 12 / 12, 57 x 150 51 / 56, and 32 / 32, 16 x 200 57 / 53, 32 / 8 35 / 30, 8 / 1, 64 x 200 + 300 55 / 50.
+static bool wide_pays(int wide, int Hkv, int D, int num_tokens, int num_seqs) {
+  if (g_prefill_variant == 3) return true;
+  if (g_prefill_variant != 1 || (long)(num_tokens / wide) * Hkv < g_prefill_wide_min_wgs) return false;
+  const int mean = num_tokens / max(num_seqs, 1);
+  if (D == 128) return mean >= min(40, wide / 2);
+  return mean >= 64 && (D == 96 || mean >= 192 || (long)((mean + wide - 1) / wide) * num_seqs * Hkv <= 256);
 }
 
 // Into how many parts the keys of each query tile are cut (1: not at all; what lse_out and the wide form take).  max_keys: an
@@ -1224,8 +1240,8 @@ static int wide_tokens(int G, int num_tokens, int num_seqs) {
 VDA_EXPORT int vda_prefill_parts(int num_seqs, int num_tokens, int Hq, int Hkv, int D, long max_keys) {
   if (Hkv < 1 || Hq % Hkv || Hq / Hkv > 128) return 1;
   const int G = Hq / Hkv, q_tile = (G <= prefill_cols(D) ? prefill_cols(D) : 128) / G;
-  const int wide = D == 128 ? wide_tokens(G, num_tokens, num_seqs) : 0;
-  if (wide && (g_prefill_variant == 3 || (g_prefill_variant == 1 && (long)(num_tokens / wide) * Hkv >= g_prefill_wide_min_wgs))) return 1;
+  const int wide = wide_tokens(G, D, num_tokens, num_seqs);
+  if (wide && wide_pays(wide, Hkv, D, num_tokens, num_seqs)) return 1;
   const long wgs = (long)(num_tokens / q_tile + min(num_seqs, num_tokens)) * Hkv, steps = (max_keys + 31) / 32;
   if (wgs < 1 || wgs > 256 || steps < 16) return 1;
   const double rows = (double)num_tokens * Hq, row_part = rows * D * 8 / 4e6;                 // us
@@ -1265,17 +1281,14 @@ VDA_EXPORT int vda_paged_attention_prefill(
                num_seqs, Hq, Hkv, max_blocks, 1, q_stride, out_stride, scale * (kv_fp8 ? k_scale : 1.f), softcap,
                kv_fp8 ? v_scale : 1.f, window, q_tile, causal, num_tokens, lse_out, max_q_len};
   p.sink = sink; p.chunk = chunk; p.v_shift = v_shift; p.dist_bias = dist_bias; p.dist_far = dist_far;
-  // Wide form (8 waves, 256 columns, 64-key tiles): head size 128 and enough query tiles to occupy the
+  // Wide form (8 waves, 256 columns, 64-key tiles): heads of 64, 96 and 128 values and enough query tiles to occupy the
   // chip (one workgroup per CU); short chunks keep the 4-wave form, which cuts them into more workgroups.
   // Its copies to LDS ask for caches aligned to 16 bytes.
   const bool aligned = (((uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0;
-  if (nsplit == 1 && D == 128 && wide_tokens(G, num_tokens, num_seqs) && aligned && (g_prefill_variant == 1 || g_prefill_variant == 3)) {
-    const int wide_tile = wide_tokens(G, num_tokens, num_seqs);
-    const long wgs = (long)(num_tokens / wide_tile) * Hkv;
-    if (g_prefill_variant == 3 || wgs >= g_prefill_wide_min_wgs) {
-      p.q_tile = wide_tile;
-      return vda_launch_prefill_wide(p, block_size, dtype, kv_fp8, st);
-    }
+  const int wide = wide_tokens(G, D, num_tokens, num_seqs);
+  if (nsplit == 1 && wide && aligned && wide_pays(wide, Hkv, D, num_tokens, num_seqs)) {
+    p.q_tile = wide;
+    return vda_launch_prefill_wide(p, D, block_size, dtype, kv_fp8, st);
   }
   const int grid_x = num_tokens / q_tile + num_seqs;
   const int form = lds ? 3 : 2;

@@ -1,4 +1,4 @@
-// Wide prefill attention for gfx950, head size 128: 8 waves per workgroup, 32 query columns per wave,
+// Wide prefill attention for gfx950, heads of 64, 96 and 128 values: 8 waves per workgroup, 32 query columns per wave,
 // 64-key tiles, 32x32x16 MFMA, products and softmax of neighbouring tiles interleaved.
 //
 // Same role as the prefill side of the reference's Triton unified attention
@@ -40,6 +40,11 @@
 // before 5000 at 2.4.  The two waves of a SIMD taking turns at products and softmax of whole tiles (two barriers a tile) were no faster on long prompts
 // and slower on short ones.
 //
+// Heads of 64 and 96 values keep the images of 128 (their rows' last pieces are zeros that nobody reads: a copy goes to LDS by lane, in whole
+// kilobytes, and the ring has room) and have 8 and 12 products a half step for the same softmax, which is then what bounds them.  With rotary
+// embedding and cache write, against the 4-wave form, us: 32 / 8 heads of 64, six of some 493 tokens on 2928 212 -> 130, 2 x 3000 265 -> 225, e4m3 cache,
+// 15 of some 405 79 -> 63; 24 / 8 of 96, 277 -> 157, 376 -> 239 and, in bf16, 92 -> 62.
+//
 // Lane maps (l = lane, c = l & 31, h = l >> 5), 32x32x16:
 //   A: row c, k = 8h + j        B: k = 8h + j, column c        C: row (r&3) + 8(r>>2) + 4h, column c
 // Scores:  row i of a block is key_of_row(i) (bits 2 and 3 of i change places), so register r of block kb is
@@ -78,10 +83,9 @@ __device__ __forceinline__ float pair_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-constexpr int WD = 128;              // head size
 constexpr int KT = 64;               // keys per tile
-constexpr int K_BYTES = KT * 256;    // one K image
-constexpr int V_BYTES = WD * 128;    // one V image
+constexpr int K_BYTES = KT * 256;    // one K image, rows of 128 values
+constexpr int V_BYTES = 128 * 128;   // one V image
 constexpr int RING = 4;              // tiles of either in LDS
 constexpr int SORTED = 16;           // sequences that workgroups sort by length
 
@@ -96,8 +100,10 @@ __device__ __forceinline__ void mfma_to(f32x16& c, bf16x8 a, bf16x8 b) {
 __device__ __forceinline__ void mfma_to(f32x16& c, f16x8 a, f16x8 b) {
   asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
 }
-__device__ __forceinline__ void settle(f32x16 (&c)[4]) {
-  asm volatile("s_nop 15\n\ts_nop 15" : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3]));
+template <int N> __device__ __forceinline__ void settle(f32x16 (&c)[N]) {
+  asm volatile("s_nop 15\n\ts_nop 15" : "+v"(c[0]));
+#pragma unroll
+  for (int i = 1; i < N; ++i) asm volatile("" : "+v"(c[i]));
 }
 
 // Twice 16 bytes a lane from a buffer to LDS, at dst + 16 * lane.  A statement of its own: told of the copy, the compiler would wait for
@@ -108,18 +114,26 @@ __device__ __forceinline__ void copy16x2(buf_t buf, unsigned voff0, unsigned vof
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 1\n\tbuffer_load_dwordx4 %1, %3, 0 offen lds\n\tbuffer_load_dwordx4 %2, %3, %4 offen offset:1024 lds"
                ::"s"(dst), "v"(voff0), "v"(voff1), "s"(buf), "s"(step) : "memory", "m0");
 }
+// The same with both sources named in full
+__device__ __forceinline__ void copy16_two(buf_t buf, unsigned voff0, unsigned voff1, unsigned dst) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 1\n\tbuffer_load_dwordx4 %1, %3, 0 offen lds\n\t"
+               "s_add_u32 m0, %0, 0x400\n\ts_nop 1\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds"
+               ::"s"(dst), "v"(voff0), "v"(voff1), "s"(buf) : "memory", "m0", "scc");
+}
+constexpr unsigned NOWHERE = 0x40000000;               // past any page
 // `bytes` from a page's head on; loads past them bring zeros
 __device__ __forceinline__ buf_t page_buffer(uint64_t head, unsigned page, unsigned page_bytes, unsigned bytes) {
   const uint64_t a = head + (uint64_t)page * page_bytes;
   return buf_t{(int)a, (int)(a >> 32) & 0xffff, (int)bytes, 0x00027000};
 }
 
-template <typename T, int BS, bool F8, bool GENERAL>
+template <typename T, int D, int BS, bool F8, bool GENERAL>
 __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p, int ntiles, int levels) {
   using V8 = typename Vec<T>::v8;
   using V4 = typename Vec<T>::v4;
   using CT = typename KVElem<T, F8>::type;
-  constexpr int D = WD;
+  static_assert(D == 64 || D == 96 || D == 128, "rows of up to 128 values, in blocks of 32");
+  constexpr int PART = D / 16, FULL = 2 * PART, DB = D / 32;       // products of the scores, as many of P.V, both; blocks of value rows
   __shared__ __attribute__((aligned(16))) unsigned char smem[RING * (K_BYTES + V_BYTES)];
 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -189,11 +203,11 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
   const float* bias_col = p.dist_bias ? dist_row(p, head) : nullptr;       // this column's distance biases
   const float bfar2 = (p.dist_bias && valid) ? bias_col[p.dist_far] * 1.4426950408889634f : 0.f;
   const long col_off = valid ? (long)(qs + qt) : -1;
-  V8 qf[8];
+  V8 qf[PART];
   {
     const T* qp = (const T*)p.q + (long)(qs + (valid ? qt : q0)) * p.q_stride + (long)head * D + 8 * hi;
 #pragma unroll
-    for (int s = 0; s < 8; ++s) qf[s] = valid ? ld16<V8>(qp + 16 * s) : V8{};
+    for (int s = 0; s < PART; ++s) qf[s] = valid ? ld16<V8>(qp + 16 * s) : V8{};
   }
   int wave_hi = valid ? limit : 0, wave_lo = valid ? lower : 0x7fffffff;
   int full_hi = valid ? limit : 0x7fffffff, full_lo = valid ? lower : 0;
@@ -224,9 +238,13 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
   const int part = wave >> 1, in_page = 16 * part % BS;
   // (in two pieces of 1 KB; the second's rows lie 4 and 32 further on, and a K row's pieces change with bit 2 of the key)
   const int key0 = 8 * (wave & 1) + (lane >> 4), d0 = 64 * (wave & 1) + (lane >> 1);
-  const unsigned k_off = (unsigned)(in_page + key0) * D + (((lane & 15) ^ key0) << 3);         // elements, from the page's head
+  // elements, from the page's head; heads of fewer than 128 values leave pieces of the images that nobody reads
+  const int piece = (lane & 15) ^ key0;
+  const unsigned k_off = (unsigned)(in_page + key0) * D + (piece << 3);
+  const unsigned k_off1 = D == 128 ? k_off ^ 32 : (unsigned)(in_page + key0) * D + ((piece ^ 4) << 3);
   const unsigned v_off = (unsigned)d0 * BS + in_page + (((lane & 1) ^ ((d0 >> 4) & 1)) << 3);
   constexpr int K_STEP = 4 * D, V_STEP = 32 * BS;
+  const bool k_there = piece < D / 8, k_there1 = (piece ^ 4) < D / 8, v_there = d0 < D, v_there1 = d0 + 32 < D;
   const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
   // page numbers of this wave's part, of 64 tiles at a time
   const int n = max(kt_hi - kt_lo, 0);               // tiles of this workgroup
@@ -249,10 +267,14 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
       if (exists)
 #pragma unroll
         for (int i = 0; i < 2; ++i)
-          rk[i] = *reinterpret_cast<const u32x2*>(k_base + (uint64_t)(unsigned)page * k_page + i * K_STEP + (k_off ^ (32 * i)));
-    } else {
-      copy16x2(page_buffer(k_base, page, k_page, exists ? BS * D * 2 : 0), k_off * 2, (k_off ^ 32) * 2, K_STEP * 2 - 1024,
+          rk[i] = *reinterpret_cast<const u32x2*>(k_base + (uint64_t)(unsigned)page * k_page +
+                                                  (i == 0 ? k_there ? k_off : 0 : k_there1 ? K_STEP + k_off1 : 0));
+    } else if constexpr (D == 128) {
+      copy16x2(page_buffer(k_base, page, k_page, exists ? BS * D * 2 : 0), k_off * 2, k_off1 * 2, K_STEP * 2 - 1024,
                lds0 + slot * K_BYTES + wave * 2048);
+    } else {
+      copy16_two(page_buffer(k_base, page, k_page, exists ? BS * D * 2 : 0), k_there ? k_off * 2 : NOWHERE,
+                 k_there1 ? (K_STEP + k_off1) * 2 : NOWHERE, lds0 + slot * K_BYTES + wave * 2048);
     }
   };
   auto copy_v = [&](int page, int slot, bool exists) {
@@ -260,10 +282,13 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
       if (exists)
 #pragma unroll
         for (int i = 0; i < 2; ++i)
-          rv[i] = *reinterpret_cast<const u32x2*>(v_base + (uint64_t)(unsigned)page * v_page + i * V_STEP + v_off);
-    } else {
+          rv[i] = *reinterpret_cast<const u32x2*>(v_base + (uint64_t)(unsigned)page * v_page + ((i == 0 ? v_there : v_there1) ? i * V_STEP + v_off : 0));
+    } else if constexpr (D == 128) {
       copy16x2(page_buffer(v_base, page, v_page, exists ? BS * D * 2 : 0), v_off * 2, v_off * 2, V_STEP * 2 - 1024,
                lds0 + RING * K_BYTES + slot * V_BYTES + wave * 2048);
+    } else {
+      copy16_two(page_buffer(v_base, page, v_page, exists ? BS * D * 2 : 0), v_there ? v_off * 2 : NOWHERE,
+                 v_there1 ? (V_STEP + v_off) * 2 : NOWHERE, lds0 + RING * K_BYTES + slot * V_BYTES + wave * 2048);
     }
   };
   auto commit_k = [&](int slot) {
@@ -297,9 +322,9 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
     m = p.sink[head] * 1.4426950408889634f;
     l = hi == 0 ? 1.f : 0.f;
   }
-  f32x16 acc[4];
+  f32x16 acc[DB];
 #pragma unroll
-  for (int db = 0; db < 4; ++db)
+  for (int db = 0; db < DB; ++db)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
 
@@ -310,14 +335,14 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
   V8 pb[2][2];
   // ---- products of a half step, with the operands read AHEAD of them: scores of block kb of the tile in K slot ks (bit 0 of `what`), P.V
   // of block vb of the tile in V slot vs (bit 1).  Where both are there they alternate, so that no MFMA waits for the one before it. ----
-  constexpr int AHEAD = 8;                           // (a divisor of 16)
+  constexpr int AHEAD = D == 96 ? 6 : 8;             // (a divisor of FULL)
   V8 fr[AHEAD];
   auto read = [&](int i, int what, int ks, int kb, int vs, int vb) {
     const int j = what == 3 ? i >> 1 : i;
     if (what == 1 || (what == 3 && (i & 1) == 0))
       fr[i % AHEAD] = *reinterpret_cast<const V8*>(smem + ((ks * K_BYTES + k_rd) ^ (32 * j)) + kb * 8192);
     else
-      fr[i % AHEAD] = *reinterpret_cast<const V8*>(smem + vs * V_BYTES + v_rd + (2 * vb + (j >> 2)) * 4096 + (j & 3) * 1024);
+      fr[i % AHEAD] = *reinterpret_cast<const V8*>(smem + vs * V_BYTES + v_rd + (2 * vb + j / DB) * 4096 + j % DB * 1024);
   };
   auto product = [&](int i, int what, int kb, int vb) {
     const int j = what == 3 ? i >> 1 : i;
@@ -327,7 +352,7 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
         for (int r = 0; r < 16; ++r) S[kb][r] = 0.f;
       S[kb] = Mfma32<V8>::run(fr[i % AHEAD], qf[j], S[kb]);
     } else {
-      mfma_to(acc[j & 3], fr[i % AHEAD], pb[vb][j >> 2]);
+      mfma_to(acc[j % DB], fr[i % AHEAD], pb[vb][j / DB]);
     }
   };
   // blocks of this wave's range, and those of them that need no mask (wave-uniform)
@@ -425,12 +450,12 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
     sm_mask(h, b);
     // (empty statements keep a slice's results in its place: otherwise the exponentials sink behind the branch of sm_end)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      if (i < 8 && (i & 1)) scale_due(i >> 1);
+    for (int i = 0; i < FULL; ++i) {
+      if (i < 2 * DB && (i & 1)) scale_due(i >> 1);
       product(i, 3, 1 - b, 1 - b);
       // the first operands of the next half step as well
-      if (i + AHEAD < 16) read(i + AHEAD, 3, ks, 1 - b, vs, 1 - b);
-      else read(i + AHEAD - 16, 3, ks_next, b, vs_next, b);
+      if (i + AHEAD < FULL) read(i + AHEAD, 3, ks, 1 - b, vs, 1 - b);
+      else read(i + AHEAD - FULL, 3, ks_next, b, vs_next, b);
       if (i == 1 || i == 2) {                          // (the last scores left the matrix pipe a while ago)
         sm_max(b, 2 * (i - 1));
         sm_max(b, 2 * (i - 1) + 1);
@@ -440,7 +465,7 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
         asm volatile("" : "+v"(off), "+v"(alpha));
       } else if (i > 3) {
 #pragma unroll
-        for (int k = (i - 4) * 8 / 12; k < (i - 3) * 8 / 12; ++k) {
+        for (int k = (i - 4) * 8 / (FULL - 4); k < (i - 3) * 8 / (FULL - 4); ++k) {
           sm_exp(b, k);
           asm volatile("" : "+v"(ps[0]), "+v"(ps[1]));
         }
@@ -455,12 +480,12 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
     auto products = [&](auto what_) {
       constexpr int what = decltype(what_)::value;
 #pragma unroll
-      for (int i = 0; i < AHEAD; ++i) read(i, what, ks, 1 - b, vs, 1 - b);
+      for (int i = 0; i < min(AHEAD, PART); ++i) read(i, what, ks, 1 - b, vs, 1 - b);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        if (what == 2 && i < 4) scale_due(i);
+      for (int i = 0; i < PART; ++i) {
+        if (what == 2 && i < DB) scale_due(i);
         product(i, what, 1 - b, 1 - b);
-        if (i + AHEAD < 8) read(i + AHEAD, what, ks, 1 - b, vs, 1 - b);
+        if (i + AHEAD < PART) read(i + AHEAD, what, ks, 1 - b, vs, 1 - b);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
@@ -525,8 +550,8 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
           if (F8) step_copies(t);
           else pages_for(t + 3);
           half_full(2 * t, first, s0, (t - 1) & (RING - 1), s1, s0, [&](int i) {
-            if (!F8 && i == 6) batch_v(t + 2);
-            if (!F8 && i == 11) batch_k(t + 2);
+            if (!F8 && i == FULL * 6 / 16) batch_v(t + 2);
+            if (!F8 && i == FULL * 11 / 16) batch_k(t + 2);
           });
           half_full(2 * t + 1, second, s1, s0, s1, s0, [](int) {});
           step_end();
@@ -548,7 +573,7 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
   // groups gives every lane 16 contiguous bytes, so the row leaves in 8 stores of 16 bytes, not 16 of 8.
   T* op = (T*)p.out + col_off * p.out_stride + (long)head * D + 8 * hi;
 #pragma unroll
-  for (int db = 0; db < 4; ++db)
+  for (int db = 0; db < DB; ++db)
 #pragma unroll
     for (int rr = 0; rr < 4; rr += 2) {
       V4 oa, ob;
@@ -569,7 +594,7 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_wide_kernel(AttnParams p
         l > 0.f ? (m + log2f(l)) * 0.6931471805599453f : -INFINITY;
 }
 
-template <typename T, bool F8, bool GENERAL>
+template <typename T, int D, bool F8, bool GENERAL>
 int launch_bs(const AttnParams& p, int bs, int ntiles, hipStream_t st) {
   // The order of the tiles.  The longest query run, when the host passed it, bounds the tiles of a sequence, so that a tile of every
   // sequence in turn, the longest (causal) ones first, is a count without a search: for sequences of about one length, and for many.  Where
@@ -585,27 +610,34 @@ int launch_bs(const AttnParams& p, int bs, int ntiles, hipStream_t st) {
   const long ranks = levels > 0 || (bound > 0 && by_level < ntiles) ? by_level : ntiles;
   const dim3 grid((unsigned)(ranks * p.Hkv)), block(512);
   switch (bs) {
-    case 16: hipLaunchKernelGGL((paged_prefill_wide_kernel<T, 16, F8, GENERAL>), grid, block, 0, st, p, ntiles, levels); break;
-    case 32: hipLaunchKernelGGL((paged_prefill_wide_kernel<T, 32, F8, GENERAL>), grid, block, 0, st, p, ntiles, levels); break;
-    case 64: hipLaunchKernelGGL((paged_prefill_wide_kernel<T, 64, F8, GENERAL>), grid, block, 0, st, p, ntiles, levels); break;
+    case 16: hipLaunchKernelGGL((paged_prefill_wide_kernel<T, D, 16, F8, GENERAL>), grid, block, 0, st, p, ntiles, levels); break;
+    case 32: hipLaunchKernelGGL((paged_prefill_wide_kernel<T, D, 32, F8, GENERAL>), grid, block, 0, st, p, ntiles, levels); break;
+    case 64: hipLaunchKernelGGL((paged_prefill_wide_kernel<T, D, 64, F8, GENERAL>), grid, block, 0, st, p, ntiles, levels); break;
     default: return -2;
   }
   VDA_CHECK_LAUNCH();
   return 0;
 }
 
-template <typename T, bool F8>
+template <typename T, int D, bool F8>
 int launch_mode(const AttnParams& p, int bs, int ntiles, hipStream_t st) {
   const bool general = p.softcap > 0.f || p.alibi != nullptr || p.dist_bias != nullptr;
-  return general ? launch_bs<T, F8, true>(p, bs, ntiles, st) : launch_bs<T, F8, false>(p, bs, ntiles, st);
+  return general ? launch_bs<T, D, F8, true>(p, bs, ntiles, st) : launch_bs<T, D, F8, false>(p, bs, ntiles, st);
+}
+template <typename T>
+int launch_dim(const AttnParams& p, int D, int bs, bool f8, int ntiles, hipStream_t st) {
+  switch (D) {
+    case 64: return f8 ? launch_mode<T, 64, true>(p, bs, ntiles, st) : launch_mode<T, 64, false>(p, bs, ntiles, st);
+    case 96: return f8 ? -3 : launch_mode<T, 96, false>(p, bs, ntiles, st);
+    case 128: return f8 ? launch_mode<T, 128, true>(p, bs, ntiles, st) : launch_mode<T, 128, false>(p, bs, ntiles, st);
+  }
+  return -3;
 }
 
 }  // namespace
 
-// p.q_tile must be 256 / (Hq / Hkv) (columns left over belong to no token); the caller has checked D == 128.
-int vda_launch_prefill_wide(const AttnParams& p, int block_size, int dtype, int kv_fp8, hipStream_t st) {
+// p.q_tile must be 256 / (Hq / Hkv) (columns left over belong to no token)
+int vda_launch_prefill_wide(const AttnParams& p, int D, int block_size, int dtype, int kv_fp8, hipStream_t st) {
   const int ntiles = p.num_tokens / p.q_tile + p.num_seqs;
-  if (dtype == VDA_BF16)
-    return kv_fp8 ? launch_mode<bf16_t, true>(p, block_size, ntiles, st) : launch_mode<bf16_t, false>(p, block_size, ntiles, st);
-  return kv_fp8 ? launch_mode<f16_t, true>(p, block_size, ntiles, st) : launch_mode<f16_t, false>(p, block_size, ntiles, st);
+  return dtype == VDA_BF16 ? launch_dim<bf16_t>(p, D, block_size, kv_fp8, ntiles, st) : launch_dim<f16_t>(p, D, block_size, kv_fp8, ntiles, st);
 }
