@@ -1207,11 +1207,12 @@ VDA_EXPORT int vda_set_prefill_wide_min_wgs(long n) { g_prefill_wide_min_wgs = n
 // Query tokens of a wide workgroup (0: the wide form does not apply to this batch).  A group that does not divide the 256 columns leaves at
 // most a sixteenth of them idle, or the 4-wave form takes it; and it has prompts of three of its tiles on average: us, 4-wave / wide, attention alone,
 // 28 / 4 heads, 2 x 2161 tokens 135 / 93, 8 ragged of some 200 25.0 / 20.7, 24 of 150 34.4 / 28.4, 24 / 8 heads, one of 1000 45 / 37, 2 of 2161 189 / 145; but ragged
-// ones of less, 40 / 8, 24 of 40 13.8 / 15.1, 48 / 8 14.5 / 16.6, 28 / 4 25 of 81 on 740 77 / 86.
+// ones of less, 40 / 8, 24 of 40 13.8 / 15.1, 48 / 8 14.5 / 16.6, 28 / 4 25 of 81 on 740 77 / 86.  Heads of 96 gain enough to do without: 24 / 8 heads, with rotary
+// embedding and cache write, 37 x 64 34 / 28, 16 x 90 + 300 48 / 34, 22 x 200 57 / 46.
 static int wide_tokens(int G, int D, int num_tokens, int num_seqs) {
   const int tokens = 256 / G;
   if (D != 64 && D != 96 && D != 128) return 0;
-  if (256 % G && (tokens * G < 240 || (long)num_tokens < 3L * tokens * num_seqs)) return 0;
+  if (256 % G && (tokens * G < 240 || (D != 96 && (long)num_tokens < 3L * tokens * num_seqs))) return 0;
   return tokens;
 }
 // Whether it is taken: workgroups for half of the CUs, and prompts that fill its tiles.  Where they don't, the 4-wave form's smaller tiles do
@@ -1226,7 +1227,8 @@ static bool wide_pays(int wide, int Hkv, int D, int num_tokens, int num_seqs) {
   if (g_prefill_variant != 1 || (long)(num_tokens / wide) * Hkv < g_prefill_wide_min_wgs) return false;
   const int mean = num_tokens / max(num_seqs, 1);
   if (D == 128) return mean >= min(40, wide / 2);
-  return mean >= 64 && (D == 96 || mean >= 192 || (long)((mean + wide - 1) / wide) * num_seqs * Hkv <= 256);
+  if (D == 96) return mean >= min(64, wide / 2);
+  return mean >= 64 && (mean >= 192 || (long)((mean + wide - 1) / wide) * num_seqs * Hkv <= 256);
 }
 
 // Into how many parts the keys of each query tile are cut (1: not at all; what lse_out and the wide form take).  max_keys: an
