@@ -42,6 +42,24 @@ def test_wq_gemm_matches_fp32(dtype, bits, M, N, K, G):
 
 
 @pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M", [1, 65, 96, 97, 130, 160, 161, 192, 193, 224, 225, 257, 511, 513])
+@pytest.mark.parametrize("N,K,G", [(260, 32, 32), (516, 96, 96), (1024, 480, 96), (300, 1056, 32), (252, 1152, 64), (512, 4160, 4160)])
+def test_tiles_and_their_ends(bits, M, N, K, G):
+    """Every number of row tiles, weight rows past a tile, K that ends in half a unit or is shorter than the rings, groups of any multiple
+    of 32; the weights are rounded to 16 bits, the products' sums are fp32: what is left is the order of K sums, and the rounding of the output."""
+    from vllm_distributed_amd import ops
+    torch.manual_seed(M + N + K)
+    x = torch.randn(M, K, device="cuda").to(torch.bfloat16)
+    qw, scales, zeros, sz, deq = _quantised(N, K, G, bits, torch.bfloat16)
+    ref = x.double() @ deq.to(torch.bfloat16).double().t()
+    worst = x.double().abs() @ deq.to(torch.bfloat16).double().abs().t()
+    for splits in (0, 1, 2, 5):
+        got = ops.wq_gemm(x, qw, sz, G, bits, splits=splits, variant=1).double()
+        # (s q - s z in fp32 may fall on the other side of a rounding boundary: one step of a weight, 2^-8 of it, now and then)
+        assert ((got - ref).abs() <= 2.0 ** -8 * ref.abs() + 2.0 ** -8 * worst / max(1.0, K ** 0.5) + K * 2.0 ** -24 * worst).all(), splits
+
+
+@pytest.mark.parametrize("bits", [4, 8])
 def test_wq_gemm_exact_layout(bits):
     """Identity activations return the dequantised rows exactly: a misplaced nibble, byte, scale or zero cannot pass."""
     from vllm_distributed_amd import ops

@@ -961,8 +961,8 @@ def wq_gemm_ok(x: torch.Tensor, qw: torch.Tensor, group: int, bits: int) -> bool
 def wq_gemm(x: torch.Tensor, qw: torch.Tensor, sz: torch.Tensor, group: int, bits: int,
             bias: Optional[torch.Tensor] = None, splits: int = 0, variant: int = 0) -> torch.Tensor:
     """y = x @ dequant(qw).T (+ bias) for any number of rows with the weights kept packed: they are widened inside
-    the kernel (ops/csrc/gemm_wq.hip): up to 128 rows a weight-streaming kernel (packed words global -> registers),
-    more rows a tiled ping-pong kernel.  ``qw``: int32 [N, K/8] (4 bit, nibble order of ``w4_pack``) or uint8 [N, K];
+    the kernel (ops/csrc/gemm_wq.hip): few rows (up to 128) in a weight-streaming kernel (packed words global -> registers),
+    more in a tiled one.  ``qw``: int32 [N, K/8] (4 bit, nibble order of ``w4_pack``) or uint8 [N, K];
     ``sz``: [K/group, N, 2] (scale, zero) pairs in x's dtype.  ``variant`` 1 / 2 force the tiled / streaming kernel."""
     M, K = x.shape
     N_ = qw.shape[0]
@@ -980,7 +980,7 @@ def wq_gemm(x: torch.Tensor, qw: torch.Tensor, sz: torch.Tensor, group: int, bit
 def wq_linear(x: torch.Tensor, qw: torch.Tensor, scales: torch.Tensor, zeros: torch.Tensor, sz: torch.Tensor,
               group: int, bits: int, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Weight-only quantised linear over weights that stay packed in device memory.  Up to ``VDA_WQ_GEMM_MAX_M``
-    rows the packed-weight kernels run (weight-streaming up to 128 rows, tiled ping-pong above: both read a quarter /
+    rows the packed-weight kernels run (weight-streaming for few rows, tiled for more: both read a quarter /
     half of the bytes of 16-bit weights).  Larger prefill batches are compute bound: a transient 16-bit copy made by
     the dequantisation kernel plus the library GEMM is faster there and is freed right after.  CPU: PyTorch."""
     M = x.shape[0]

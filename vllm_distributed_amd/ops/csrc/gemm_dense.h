@@ -1,5 +1,5 @@
-// Shared by the ping-pong MFMA GEMM kernels (gemm_dense.hip: 16-bit weights; gemm_wq.hip: packed 4- / 8-bit
-// weights widened on the way into the MFMAs): launch arguments, the epilogue and the split-K reduction.
+// Shared by the MFMA GEMM kernels (gemm_dense.hip: 16-bit weights; gemm_wq.hip: packed 4- / 8-bit weights widened
+// on the way into the MFMAs): launch arguments, the epilogue and the split-K reduction.
 #pragma once
 #include "mfma_tile.h"
 

@@ -3,15 +3,12 @@
 // activations: GPTQ / AWQ W4A16, 8-bit GPTQ, GGUF Q4_0 / Q8_0 after repacking.  The weights stay packed in HBM and
 // in LDS; they are widened to the activation type only on their way into the MFMA operand registers.
 //
-// Two kernels.  Up to 128 activation rows (decode): the weight stream is the whole cost, so wq_stream_kernel keeps
+// Two kernels.  Few activation rows (decode): the weight stream is the whole cost, so wq_stream_kernel keeps
 // it out of LDS altogether: packed words go global -> registers four K steps ahead, are
 // widened in registers and fed to the MFMAs as the A operand, while the activations of a K step are shared by the
 // waves through an LDS ring (the scheme of gemm_decode.hip with a quarter / half of its HBM bytes).  More rows:
-// wq_gemm_kernel, the two-group schedule of gemm_dense.hip (one wave group issues 32 MFMAs from registers while the other issues
-// the LDS-DMA copies of a later K unit, reads its next fragments AND widens them: the nibble extraction and the
-// scale / zero arithmetic run on the vector ALU of the group that is not using the matrix pipe).  A K unit is 32
-// elements: per tile 256 weight rows x 16 bytes (4 bit) or 32 bytes (8 bit), 256 (scale, zero) pairs and the
-// activation rows x 64 bytes.
+// wq_tile_kernel, tiles of 256 weight rows by up to 256 activation rows, one wave a SIMD, whose vector instructions widen the next
+// product's weights behind the MFMAs of this one.
 //
 // Layouts (made by ops.wq_pack_* at load time):
 //   qweight 4 bit  uint32 [N, K / 8]: word j of row n holds K elements 8 j .. 8 j + 7, element e in nibble
@@ -29,6 +26,7 @@ struct WqGemmArgs {
   const void* sz;         // [K / G, N, 2]
   int group;              // G
   int gshift;             // log2(G / 32) when G is a power of two (30 when one group spans K), else -1
+  unsigned group_magic;   // see wq_group_of
   int per_element;        // streaming kernel: scale every weight element even where the unscaled form applies
 };
 
@@ -56,149 +54,6 @@ __device__ __forceinline__ typename Vec<T>::v8 wq_expand(const uint32_t* q, floa
   }
   return o;
 }
-
-__device__ __forceinline__ void glds4(const uint8_t* src, uint8_t* lds_wave_base) {
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                   (__attribute__((address_space(3))) void*)lds_wave_base, 4, 0, 0);
-}
-
-template <typename T, int BITS, int XT>
-__global__ __launch_bounds__(512, 1) void wq_gemm_kernel(const WqGemmArgs wa) {
-  using V8 = typename Vec<T>::v8;
-  const DenseGemmArgs& a = wa.d;
-  constexpr int WT = 4, WR = 256, XR = 32 * XT;
-  constexpr int ROWB = 4 * BITS;                   // packed bytes of one weight row in a unit
-  constexpr int WB = WR * ROWB;                    // 4 KiB or 8 KiB
-  constexpr int SB = WR * 4;                       // (scale, zero) pairs
-  constexpr int XROUNDS = XR / 128 > 0 ? XR / 128 : 1, XB = XROUNDS * 8192;
-  constexpr int UNIT = WB + SB + XB;
-  constexpr int NG = 2 + XROUNDS;
-  constexpr int D = UNIT <= 16384 ? 8 : 6;         // ring slots (XT = 8 with 8-bit weights: 25 KiB x 6)
-  constexpr int AHEAD = NG * (D - 2);
-  static_assert(AHEAD < 64, "vmcnt is a 6-bit counter");
-  __shared__ __attribute__((aligned(16))) uint8_t lds[D * UNIT];
-
-  int mi, ni, sp;
-  if (a.m_tiles == 1) {
-    mi = 0; ni = blockIdx.x % a.n_tiles; sp = blockIdx.x / a.n_tiles;
-  } else {
-    // workgroup -> tile: each XCD (blockIdx.x % 8) takes a contiguous run of the tile list, and the list walks the
-    // output in columns of eight weight tiles, row by row: the 32 workgroups an XCD runs at a time cover about
-    // 4 x 8 tiles, so its L2 serves every weight tile four times and every activation tile eight times
-    const int label = blockIdx.x & 7, seq = blockIdx.x >> 3;
-    const int tiles = a.m_tiles * a.n_tiles;
-    const int t = label * ((tiles + 7) >> 3) + seq;
-    if (seq >= ((tiles + 7) >> 3) || t >= tiles) return;
-    const int col = t / (8 * a.m_tiles), rem = t - col * 8 * a.m_tiles;
-    const int width = min(8, a.n_tiles - 8 * col);
-    mi = rem / width; ni = 8 * col + rem % width; sp = blockIdx.y;
-  }
-  if (ni >= a.n_tiles || mi >= a.m_tiles || sp >= a.splits) return;
-  const int nu_all = a.K >> 5;
-  const int u0 = sp * a.units_per_split;
-  const int nun = min(a.units_per_split, nu_all - u0);
-  if (nun <= 0) return;
-  const int beg = mi * XR, cnt = min(a.M - beg, XR);
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r = lane & 15, g = lane >> 4;
-  const int grp = wave >> 2, wn = wave & 3;
-  const int n0 = ni * WR;
-  const uint8_t* wbase = reinterpret_cast<const uint8_t*>(a.w) + (long)u0 * ROWB;
-  const uint8_t* xbase = reinterpret_cast<const uint8_t*>(a.x) + (long)u0 * 64;
-  const uint8_t* szbase = reinterpret_cast<const uint8_t*>(wa.sz);
-  const int units_per_group = wa.group >> 5;
-
-  // ---- staging roles ------------------------------------------------------------------------------------
-  // weights: 4 bit: lane L of wave w copies the 16 bytes of row 64 (w & 3) + L (waves 4-7 write the same bytes
-  // again, which keeps the copy count per wave uniform); 8 bit: thread t copies half t & 1 of row t >> 1.
-  // pairs: lane L of wave w copies the 4 bytes of row 64 (w & 3) + L.
-  unsigned voff_w, voff_s, voff_x[XROUNDS];
-  uint8_t* lds_w;
-  {
-    const int srow = 64 * wn + lane;
-    if (BITS == 4) {
-      voff_w = (unsigned)min(n0 + srow, a.N - 1) * (unsigned)(a.K >> 1);
-      lds_w = lds + wn * 1024;
-    } else {
-      voff_w = (unsigned)min(n0 + (tid >> 1), a.N - 1) * (unsigned)a.K + ((tid & 1) << 4);
-      lds_w = lds + wave * 1024;
-    }
-    voff_s = (unsigned)min(n0 + srow, a.N - 1) * 4u;
-    const int lrow = 16 * wave + (lane >> 2), pos = lane & 3;
-#pragma unroll
-    for (int j = 0; j < XROUNDS; ++j) {
-      const int tau = 128 * j + lrow;
-      voff_x[j] = (unsigned)(beg + min(tau, cnt - 1)) * (unsigned)(a.x_stride * 2) + ((pos ^ swz64(tau & 15)) << 4);
-    }
-  }
-  auto issue = [&](int u, int slot) {
-    const int uu = min(u, nun - 1);
-    uint8_t* base = lds + slot * UNIT;
-    glds16(wbase + (long)uu * ROWB + voff_w, lds_w + slot * UNIT);
-    const long gi = (u0 + uu) / units_per_group;
-    glds4(szbase + gi * a.N * 4 + voff_s, base + WB + wn * 256);
-    const uint8_t* xb = xbase + (long)uu * 64;
-#pragma unroll
-    for (int j = 0; j < XROUNDS; ++j) glds16(xb + voff_x[j], base + WB + SB + wave * 1024 + j * 8192);
-  };
-
-  // ---- compute roles: wave (grp, wn) owns weight rows [64 wn, 64 wn + 64) and activation rows of half grp ----
-  const int wl = (64 * wn + r) * ROWB + g * (ROWB / 4);
-  const int sl = WB + (64 * wn + r) * 4;
-  const int xl = WB + SB + (16 * XT * grp + r) * 64 + ((g ^ swz64(r)) << 4);
-
-  f32x4 acc[WT][XT];
-#pragma unroll
-  for (int mt = 0; mt < WT; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < XT; ++nt) acc[mt][nt] = f32x4{0, 0, 0, 0};
-
-#pragma unroll
-  for (int u = 0; u < D - 1; ++u) issue(u, u);
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AHEAD) : "memory");
-  __builtin_amdgcn_s_barrier();
-  if (grp == 1) __builtin_amdgcn_s_barrier();
-  int rs = 0, wsl = D - 1;
-  for (int u = 0; u < nun; ++u) {
-    issue(u + D - 1, wsl);
-    const uint8_t* base = lds + rs * UNIT;
-    V8 wf[WT], xf[XT];
-#pragma unroll
-    for (int nt = 0; nt < XT; ++nt) xf[nt] = *reinterpret_cast<const V8*>(base + xl + nt * 1024);
-    uint32_t q[WT][2], pr[WT];
-#pragma unroll
-    for (int mt = 0; mt < WT; ++mt) {
-      const uint8_t* wp = base + wl + mt * 16 * ROWB;
-      q[mt][0] = *reinterpret_cast<const uint32_t*>(wp);
-      q[mt][1] = BITS == 8 ? *reinterpret_cast<const uint32_t*>(wp + 4) : 0u;
-      pr[mt] = *reinterpret_cast<const uint32_t*>(base + sl + mt * 64);
-    }
-#pragma unroll
-    for (int mt = 0; mt < WT; ++mt) {
-      const typename Vec<T>::v4 pv = __builtin_bit_cast(typename Vec<T>::v4, u32x2{pr[mt], 0u});
-      const float s = (float)pv[0];
-      wf[mt] = wq_expand<T, BITS>(q[mt], s, -(float)pv[1] * s);
-    }
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(AHEAD) : "memory");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int nt = 0; nt < XT; ++nt)
-#pragma unroll
-      for (int mt = 0; mt < WT; ++mt) acc[mt][nt] = mfma16(wf[mt], xf[nt], acc[mt][nt]);
-    __builtin_amdgcn_s_setprio(0);
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    rs = rs + 1 == D ? 0 : rs + 1;
-    wsl = wsl + 1 == D ? 0 : wsl + 1;
-  }
-  if (grp == 0) __builtin_amdgcn_s_barrier();
-  dense_epilogue<T, DG_PLAIN, WT, XT>(a, acc, sp, beg, cnt, n0, r, g, grp, wn);
-}
-
 
 // ---- decode: weights global -> registers, activations through an LDS ring -----------------------------------
 // A K step is 128 elements.  Lane (r, g) of a wave holds, for each of the wave's two 16-row weight fragments, the
@@ -443,6 +298,324 @@ __global__ __launch_bounds__(256 * WM, WM == 1 ? 2 : 1) void wq_stream_kernel(co
   }
 }
 
+// ---- many rows: one wave a SIMD, all operands through LDS ---------------------------------------------------
+// A workgroup of four waves has 256 weight rows and 32 NT activation rows; wave w widens the weights of its 64 rows, once for all
+// activation rows, and holds 64 x 32 NT sums (up to 256 accumulation registers, so one wave a SIMD).  A K unit is 64 elements: four
+// products of 16, of which lane (r, h) has elements 32 h + 8 j .. + 7 of row r, as the packed words and a row's pieces of 16 bytes have them.
+//   Copies to LDS run DX - 1 units ahead for activations, DW - 1 for weights, one behind each fragment's products; a unit's last third begins with
+//   the wait for the next one and the only barrier, from which on fragments of the next unit are read, four ahead.
+//   The widening of product j + 1 (some 3 instructions an element) is cut into 16 slices, spread evenly over the MFMAs of product j: a wave issues an
+//   instruction in 4 cycles, an MFMA of 32x32x16 takes 32, and what lies between two of them beyond 7 instructions leaves the matrix pipe idle.
+// LDS images: activations [row][8 pieces of 16 B], piece p of row t at p ^ ((t >> 1) & 7); weights [row][2 or 4 pieces], piece p of row t at p ^ ((t >> 3) & 1)
+// (4 bits) or p ^ ((t >> 2) & 3): the 16 lanes that a read serves together (rows 0-3, 12-15, 20-27 or the others) touch all banks.
+//
+// us, before (tiles of 256 x 32 XT, two groups of waves that took turns at widening and products, of 64 x 16 XT sums a wave and two barriers per 32
+// elements; weights were widened twice) / now, groups of 128: 4 bits, 160, 256 and 512 rows, 57344 x 8192 305 / 155, 312 / 218, 610 / 430;
+// 8192 x 28672 151 / 87, 159 / 117, 290 / 207; 10240 x 8192 71 / 45, 78 / 61, 129 / 93; 6144 x 4096 39 / 31, 44 / 37, 59 / 46; 8 bits, 57344 x 8192 286 / 173, 292 / 237, 558 / 449;
+// 8192 x 28672 147 / 88, 160 / 127, 272 / 216.  512 x 57344 x 8192 is 1.12 PFLOP/s, of 256 rows the matrix pipe works 69 % of the cycles, at 1.93 GHz: what bounds the large ones is
+// power; of 64 rows 28 %: widening.
+typedef int wq_buf_t __attribute__((ext_vector_type(4)));
+constexpr unsigned WQ_RECORDS = 0xffffffc0u, WQ_NOWHERE = 0xfffffff0u;      // a copy from past the records brings zeros
+// 16 or 4 bytes a lane to LDS, at dst + AT + 16 (4) * lane.  Statements of their own: told of the copies, the compiler would wait for them before
+// every LDS read.
+template <int AT> __device__ __forceinline__ void wq_copy16(wq_buf_t buf, unsigned voff, unsigned soff, unsigned dst) {
+  asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               ::"s"(dst), "v"(voff), "s"(buf), "s"(soff), "n"(AT) : "memory", "m0", "scc");
+}
+template <int AT> __device__ __forceinline__ void wq_copy4(wq_buf_t buf, unsigned voff, unsigned soff, unsigned dst) {
+  asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+               ::"s"(dst), "v"(voff), "s"(buf), "s"(soff), "n"(AT) : "memory", "m0", "scc");
+}
+// the group of 32 elements number k32 (magic: 2^32 over a group's number of those, rounded up; 0: one)
+__device__ __forceinline__ unsigned wq_group_of(unsigned k32, unsigned magic) { return magic ? __umulhi(k32, magic) : k32; }
+__device__ __forceinline__ wq_buf_t wq_buffer(const void* p) {
+  const uint64_t at = reinterpret_cast<uint64_t>(p);
+  return wq_buf_t{__builtin_amdgcn_readfirstlane((int)at), __builtin_amdgcn_readfirstlane((int)(at >> 32) & 0xffff), (int)WQ_RECORDS, 0x00027000};
+}
+template <typename V8> __device__ __forceinline__ f32x16 wq_mfma32(V8 a, V8 b, f32x16 c) {
+  if constexpr (std::is_same<V8, bf16x8>::value) return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+  else return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+template <int LO, int HI, typename F> __device__ __forceinline__ void wq_each(F&& fn) {
+  if constexpr (LO < HI) {
+    fn(std::integral_constant<int, LO>{});
+    wq_each<LO + 1, HI>(fn);
+  }
+}
+template <int BITS, int NT> struct WqTile {
+  static constexpr int XB = 32 * NT * 128;             // a unit's activations
+  static constexpr int ROWB = 8 * BITS, WB = 256 * ROWB, SB = 2 * 1024, PB = WB + SB;   // weights, (scale, zero) pairs of both halves
+  static constexpr int DX = NT > 5 ? 3 : 4;            // ring slots
+  static constexpr int ROOM = (160 * 1024 - DX * XB) / PB;
+  static constexpr int DW = ROOM < 8 ? ROOM : 8;
+  static constexpr int LX = NT, LW = 2 * (BITS / 4) + 2;                                // copies of a wave and unit
+  static constexpr int YOUNGER = (DX - 3) * (LX + LW) + (DW > DX ? LW : 0);
+  static_assert(DW >= DX && YOUNGER < 64, "");
+};
+
+template <typename T, int BITS, int NT>
+__global__ __launch_bounds__(256, 1) void wq_tile_kernel(const WqGemmArgs wa) {
+  using V8 = typename Vec<T>::v8;
+  using V4 = typename Vec<T>::v4;
+  using C = WqTile<BITS, NT>;
+  const DenseGemmArgs& a = wa.d;
+  constexpr int XR = 32 * NT, NQ = BITS / 4, DX = C::DX, DW = C::DW, AHEAD = 4, FLAT = 4 * NT;
+  constexpr int COPIES = C::LX + C::LW, EACH = NT < 4 ? 2 : 1;      // copies behind a fragment's products
+  constexpr int LATEST = FLAT - (COPIES + EACH - 1) / EACH, MEET = 3 * NT - 2 < LATEST ? 3 * NT - 2 : LATEST;
+  static_assert(MEET >= 4, "");
+  __shared__ __attribute__((aligned(16))) uint8_t lds[DX * C::XB + DW * C::PB];
+
+  // workgroup -> tile: each XCD (blockIdx.x % 8) takes a contiguous run of tiles, the row tiles of one weight tile next to each other
+  const int tiles = a.m_tiles * a.n_tiles, per = (tiles * a.splits + 7) >> 3;
+  const int t = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || t >= tiles * a.splits) return;
+  const int sp = t / tiles, mi = t % tiles % a.m_tiles, ni = t % tiles / a.m_tiles;
+  const int nu_all = (a.K + 63) >> 6;
+  const int u0 = sp * a.units_per_split;
+  const int nun = min(a.units_per_split, nu_all - u0);
+  if (nun <= 0) return;
+  const int beg = mi * XR, cnt = min(a.M - beg, XR), n0 = ni * 256;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 31, h = lane >> 5;
+  const int turn = a.splits == 1 ? (int)((unsigned)ni * 5u % (unsigned)nun) : 0;
+  auto unit_at = [&](int u) {
+    const int v = min(u, nun - 1) + turn;
+    return u0 + (v < nun ? v : v - nun);
+  };
+
+  // ---- copies: the wave's own 64 weight rows and their pairs, eight activation rows of every 32 ----
+  const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds;
+  const wq_buf_t xbuf = wq_buffer(reinterpret_cast<const uint8_t*>(a.x) + (long)beg * a.x_stride * 2);
+  const wq_buf_t wbuf = wq_buffer(reinterpret_cast<const uint8_t*>(a.w) + (long)n0 * ((long)a.K * BITS / 8));
+  const wq_buf_t sbuf = wq_buffer(wa.sz);
+  unsigned voff_x[NT], voff_w[C::LW - 2], voff_s;
+  bool late_w[C::LW - 2];                              // a piece of a unit's second half
+  const int xchunk = (lane & 7) ^ ((lane >> 4) | (wave & 1) << 2);           // rows 32 i + 8 wave + lane / 8: (row >> 1) & 7
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    const int row = min(32 * i + 8 * wave + (lane >> 3), cnt - 1);
+    voff_x[i] = (unsigned)row * (unsigned)(a.x_stride * 2) + (xchunk << 4);
+  }
+#pragma unroll
+  for (int i = 0; i < C::LW - 2; ++i) {
+    // 4 bits: 32 rows a copy, two pieces of 16 bytes; 8 bits: 16 rows, four
+    const int row = BITS == 4 ? 32 * i + (lane >> 1) : 16 * i + (lane >> 2);
+    const int piece = BITS == 4 ? (lane & 1) ^ ((row >> 3) & 1) : (lane & 3) ^ ((row >> 2) & 3);
+    voff_w[i] = (unsigned)min(64 * wave + row, a.N - 1 - n0) * (unsigned)(a.K * BITS / 8) + (piece << 4);
+    late_w[i] = piece >= BITS / 4;
+  }
+  voff_s = (unsigned)min(n0 + 64 * wave + lane, a.N - 1) * 4u;
+  // a batch: the activations of unit ux, the weights of unit uw, behind each other in the rings
+  unsigned xdst = lds0 + wave * 1024, wdst = lds0 + DX * C::XB + wave * (64 * C::ROWB), sdst = lds0 + DX * C::XB + C::WB + wave * 256;
+  const unsigned plane = (unsigned)a.N * 4u;
+  unsigned xoff = 0, woff = 0, soff[2] = {0, 0};
+  bool xhalf = false, whalf = false;                   // a unit of 32 elements, at the end of K
+  // (in four stages, for the loop; the values of the last batch are in use until stage 3)
+  int kx = 0, kw = 0;
+  unsigned group0 = 0, group1 = 0;
+  auto batch = [&](int ux, int uw, int stage) {
+    if (stage == 0) {
+      kx = unit_at(ux) << 6;
+    } else if (stage == 1) {
+      kw = unit_at(uw) << 6;
+    } else if (stage == 2) {
+      group0 = wq_group_of((unsigned)(kw >> 5), wa.group_magic) * plane;
+      group1 = kw + 32 >= a.K ? group0 : wq_group_of((unsigned)(kw >> 5) + 1, wa.group_magic) * plane;
+    } else {
+      xoff = (unsigned)kx * 2;
+      xhalf = kx + 32 >= a.K;
+      woff = (unsigned)kw * BITS / 8;
+      whalf = kw + 32 >= a.K;
+      soff[0] = group0;
+      soff[1] = group1;
+    }
+  };
+  // copy i of a batch (i a constant): activations, weights, pairs
+  auto copy = [&](auto i_) {
+    constexpr int i = decltype(i_)::value;
+    if constexpr (i < NT) {
+      wq_copy16<i * 4096>(xbuf, xhalf && xchunk >= 4 ? WQ_NOWHERE : voff_x[i], xoff, xdst);
+      if constexpr (i == NT - 1) xdst = xdst + C::XB == lds0 + wave * 1024 + DX * C::XB ? lds0 + wave * 1024 : xdst + C::XB;
+    } else if constexpr (i < NT + C::LW - 2) {
+      wq_copy16<(i - NT) * 1024>(wbuf, whalf && late_w[i - NT] ? WQ_NOWHERE : voff_w[i - NT], woff, wdst);
+    } else if constexpr (i < COPIES) {
+      constexpr int p = i - (COPIES - 2);
+      wq_copy4<p * 1024>(sbuf, voff_s, soff[p], sdst);
+      if constexpr (p == 1) {
+        const bool last = sdst + C::PB == lds0 + DX * C::XB + C::WB + wave * 256 + DW * C::PB;
+        wdst = last ? wdst - (DW - 1) * C::PB : wdst + C::PB;
+        sdst = last ? sdst - (DW - 1) * C::PB : sdst + C::PB;
+      }
+    }
+  };
+
+  // ---- operands: lane (r, h) has elements 32 h .. 32 h + 31 of a unit, eight to each of its four products of 16 ----
+  const int x_rd = r * 128, x_sw = (r >> 1) & 7;
+  int xr = 0, wr = 0;                                  // slots that are read
+  i32x4 wq[2][NQ], wn[2][NQ];
+  uint32_t pr[2];
+  auto read_w = [&] {
+    const uint8_t* base = lds + DX * C::XB + wr * C::PB;
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
+      const uint8_t* p = base + wave * (64 * C::ROWB) + (32 * mt + r) * C::ROWB;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+        wn[mt][q] = *reinterpret_cast<const i32x4*>(p + ((BITS == 4 ? h ^ ((r >> 3) & 1) : (2 * h + q) ^ ((r >> 2) & 3)) << 4));
+      pr[mt] = *reinterpret_cast<const uint32_t*>(base + C::WB + h * 1024 + wave * 256 + (32 * mt + r) * 4);
+    }
+    wr = wr + 1 == DW ? 0 : wr + 1;
+  };
+  V8 xf[AHEAD];
+  u32x4 wf[2][2];                                      // [which of two products][row tile]
+  float sc[2], nz[2];
+  auto take_w = [&] {
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) wq[mt][q] = wn[mt][q];
+      const V4 pv = __builtin_bit_cast(V4, u32x2{pr[mt], 0u});
+      sc[mt] = (float)pv[0];
+      nz[mt] = -(float)pv[1] * sc[mt];
+    }
+  };
+  // Widening in 16 slices: slice 2 k spreads the words that elements 2 i and 2 i + 1 (i = k & 3) of product j's operand of row tile k >> 2 are
+  // in, slice 2 k + 1 scales and packs them.
+  uint32_t nib[2];
+  float raw[2];
+  auto widen = [&](int j, int slice) {
+    typedef T T2 __attribute__((ext_vector_type(2)));
+    const int mt = slice >> 3, i = (slice >> 1) & 3;
+    if ((slice & 1) == 0) {
+      if constexpr (BITS == 4) {
+        if (i == 0) {                                  // (kept apart: bytes convert in one instruction, nibbles in two)
+          nib[0] = (uint32_t)wq[mt][0][j] & 0x0F0F0F0Fu;
+          nib[1] = ((uint32_t)wq[mt][0][j] >> 4) & 0x0F0F0F0Fu;
+          asm volatile("" : "+v"(nib[0]), "+v"(nib[1]));
+        }
+        const uint32_t m = nib[i & 1];
+        raw[0] = (float)(i < 2 ? m & 0xff : (m >> 8) & 0xff);
+        raw[1] = (float)(i < 2 ? (m >> 16) & 0xff : m >> 24);
+      } else {
+        const uint32_t q = (uint32_t)wq[mt][j >> 1][2 * (j & 1) + (i >> 1)];
+        raw[0] = (float)(i & 1 ? (q >> 16) & 0xff : q & 0xff);
+        raw[1] = (float)(i & 1 ? q >> 24 : (q >> 8) & 0xff);
+      }
+      asm volatile("" : "+v"(raw[0]), "+v"(raw[1]));
+    } else {
+      const T2 o = {(T)fmaf(raw[0], sc[mt], nz[mt]), (T)fmaf(raw[1], sc[mt], nz[mt])};
+      wf[j & 1][mt][i] = __builtin_bit_cast(uint32_t, o);
+    }
+  };
+  // fragment f of the unit in slot `slot`: product f / NT, rows 32 (f % NT) ..
+  auto read_x = [&](int f, int slot) {
+    xf[f % AHEAD] = *reinterpret_cast<const V8*>(lds + slot * C::XB + x_rd + f % NT * 4096 + (((4 * h + f / NT) ^ x_sw) << 4));
+  };
+
+  f32x16 acc[2][NT];
+#pragma unroll
+  for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[mt][nt][i] = 0.f;
+
+  for (int v = 1 - DW; v < 0; ++v) {
+    if (v == -1) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C::YOUNGER) : "memory");
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    for (int stage = 0; stage < 4; ++stage) batch(max(v + DX - 1, 0), v + DW - 1, stage);
+    if (v + DX - 1 >= 0) wq_each<0, NT>(copy);
+    wq_each<NT, COPIES>(copy);
+  }
+  read_w();
+#pragma unroll
+  for (int f = 0; f < AHEAD; ++f) read_x(f, 0);
+  take_w();
+#pragma unroll
+  for (int k = 0; k < 16; ++k) widen(0, k);
+
+  for (int u = 0; u < nun; ++u) {
+    const int next = xr + 1 == DX ? 0 : xr + 1;
+    wq_each<0, FLAT>([&](auto f_) {
+      constexpr int f = decltype(f_)::value, j = f / NT, nt = f % NT;
+      if (f == MEET) {                                 // the next unit is there, for all waves
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C::YOUNGER) : "memory");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        batch(u + DX - 1, u + DW - 1, 3);
+        read_w();
+      }
+      wq_each<0, 2>([&](auto mt_) {
+        constexpr int mt = decltype(mt_)::value, s = 2 * nt + mt;
+        acc[mt][nt] = wq_mfma32(__builtin_bit_cast(V8, wf[j & 1][mt]), xf[f % AHEAD], acc[mt][nt]);
+        if (mt == 1) {
+          if (f + AHEAD < FLAT) read_x(f + AHEAD, xr);
+          else read_x(f + AHEAD - FLAT, next);
+        }
+        // a share of the next product's widening behind each product, and a copy
+#pragma unroll
+        for (int k = s * 8 / NT; k < (s + 1) * 8 / NT; ++k) {
+          if (j == 3 && k == 0) take_w();              // (this unit's words are widened)
+          widen((j + 1) & 3, k);
+        }
+        if constexpr (f >= MEET && (EACH == 2 || mt == 0)) copy(std::integral_constant<int, EACH * (f - MEET) + (EACH == 2 ? mt : 0)>{});
+        if constexpr (mt == 1 && f >= MEET - 4 && f < MEET - 1) batch(u + DX - 1, u + DW - 1, f - (MEET - 4));
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    });
+    xr = next;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // nothing in flight into LDS
+
+  // ---- out[token beg + 32 nt + r][n0 + 64 wave + 32 mt + 8 q + 4 h + i] = acc[mt][nt][4 q + i] ----
+  const int nb = n0 + 64 * wave + 4 * h;
+  V4 bias[2][4];
+#pragma unroll
+  for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int n = nb + 32 * mt + 8 * q + i;
+        bias[mt][q][i] = a.splits == 1 && a.bias && n < a.N ? reinterpret_cast<const T*>(a.bias)[n] : (T)0.f;
+      }
+  const bool wide = a.out_stride % 4 == 0;
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    const int tok = 32 * nt + r;
+    if (tok >= cnt) continue;
+    // (in their places until here: read out of them all at once, the sums would not fit)
+    asm volatile("" : "+a"(acc[0][nt]), "+a"(acc[1][nt]));
+    float* wsp = a.ws + ((long)sp * a.M + beg + tok) * a.N;
+    T* op = reinterpret_cast<T*>(a.out) + (long)(beg + tok) * a.out_stride;
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int n = nb + 32 * mt + 8 * q;
+        if (n >= a.N) continue;
+        f32x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = acc[mt][nt][4 * q + i];
+        if (a.splits > 1) {                            // (N is a multiple of 4)
+          *reinterpret_cast<f32x4*>(wsp + n) = v;
+        } else {
+          V4 o;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[i] = (T)(v[i] + (float)bias[mt][q][i]);
+          if (wide && n + 3 < a.N) *reinterpret_cast<V4*>(op + n) = o;
+          else
+            for (int i = 0; i < 4; ++i) if (n + i < a.N) op[n + i] = o[i];
+        }
+      }
+  }
+}
+
 // ---- decode, fewer weight rows than fill the chip: K over the waves of a workgroup --------------------------
 // Up to 16 activation rows.  The kernel above splits K over workgroups there, and the sum of the parts is a launch of its own
 // (5 us and a gap of 2, of 20 in all).  Here a workgroup owns 32 weight rows and its KS waves a slice of K each: nothing is shared until
@@ -678,14 +851,18 @@ static int launch_wq_stream(const WqGemmArgs& wa, hipStream_t st) {
 }
 
 template <typename T, int BITS>
-static int launch_wq_gemm(const WqGemmArgs& wa, int xt, hipStream_t st) {
+static int launch_wq_tile(const WqGemmArgs& wa, int nt, hipStream_t st) {
   const DenseGemmArgs& a = wa.d;
-  dim3 grid;
-  if (a.m_tiles == 1) grid = dim3((unsigned)(a.n_tiles * a.splits));
-  else grid = dim3((unsigned)((a.m_tiles * a.n_tiles + 7) / 8 * 8), (unsigned)a.splits);
-#define LAUNCH(XT) hipLaunchKernelGGL((wq_gemm_kernel<T, BITS, XT>), grid, dim3(512), 0, st, wa)
-  if (xt == 8) LAUNCH(8); else if (xt == 4) LAUNCH(4); else if (xt == 2) LAUNCH(2); else LAUNCH(1);
-#undef LAUNCH
+  const dim3 grid((unsigned)(((long)a.m_tiles * a.n_tiles * a.splits + 7) / 8 * 8));
+  switch (nt) {
+    case 1: case 2: hipLaunchKernelGGL((wq_tile_kernel<T, BITS, 2>), grid, dim3(256), 0, st, wa); break;
+    case 3: hipLaunchKernelGGL((wq_tile_kernel<T, BITS, 3>), grid, dim3(256), 0, st, wa); break;
+    case 4: hipLaunchKernelGGL((wq_tile_kernel<T, BITS, 4>), grid, dim3(256), 0, st, wa); break;
+    case 5: hipLaunchKernelGGL((wq_tile_kernel<T, BITS, 5>), grid, dim3(256), 0, st, wa); break;
+    case 6: hipLaunchKernelGGL((wq_tile_kernel<T, BITS, 6>), grid, dim3(256), 0, st, wa); break;
+    case 7: hipLaunchKernelGGL((wq_tile_kernel<T, BITS, 7>), grid, dim3(256), 0, st, wa); break;
+    default: hipLaunchKernelGGL((wq_tile_kernel<T, BITS, 8>), grid, dim3(256), 0, st, wa); break;
+  }
   if (a.splits > 1) {
     const long quads = (long)a.M * (a.N >> 2);
     hipLaunchKernelGGL((dense_gemm_reduce_kernel<T, DG_PLAIN>), dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, a);
@@ -711,6 +888,18 @@ static int wq_parts(int M, int N, int K, int bits) {
 // (for the test of the rule, which runs on the host)
 VDA_EXPORT int vda_wq_parts(int M, int N, int K, int bits) { return wq_parts(M, N, K, bits); }
 
+// From how many of up to 128 rows the tiled kernel leads.  us, kernel above / tiled:
+//   8 bits, 17, 33, 64, 96 and 128 rows: 57344 x 8192 114 / 112, 131 / 112, 138 / 118, 207 / 133 (here the tiled kernel before, as at 128), 207 / 149;
+//     8192 x 28672 69 / 54, 79 / 53, 83 / 58, 98 / 67, 103 / 77; 8192 x 8192 26 / 23, 33 / 25, 36 / 28, 40 / 31, 42 / 35; 5120 x 13824 35 / 26, 41 / 27, 45 / 29;
+//     but of short rows 28672 x 4096 34 / 32, 40 / 35, 41 / 38, 6144 x 4096 15.4 / 15.9, 17.7 / 17.8, 21 / 21, 27 / 23
+//   4 bits scaled in registers (groups of 64), 48, 64, 96: 57344 x 8192 106 / 100, 107 / 100, 214 / 117; 10240 x 8192 29 / 29, 30 / 31, 47 / 36; 28672 x 4096
+//     37 / 36, 38 / 37, 56 / 44; 6144 x 4096 17 / 20, 18 / 22, 26 / 26
+//   4 bits unscaled: the kernel above has exact operands, whose sums are nearer to the product than those of weights rounded to 16 bits
+static bool wq_tiles_pay(int M, int N, int K, int bits, int group, bool no_split) {
+  if (M <= 64) return bits == 8 && !no_split && M > (K >= 8192 ? 16 : 32);
+  return !wq_unscaled(N, bits, group);
+}
+
 // x [M, K] 16-bit (row stride x_stride elements), qw packed [N, K] (bits 4 or 8), sz [K / group, N, 2] of x's type,
 // out [M, N].  K % 32 == 0, group % 32 == 0 and K % group == 0, N % 4 == 0 for split K.  variant: 0 picks by shape,
 // 1 the tiled kernel, 2 the streaming kernel (M <= 128, K % 128 == 0, group a power of two or K), 3 the streaming
@@ -733,13 +922,14 @@ VDA_EXPORT int vda_wq_gemm(void* out, const void* x, const void* qw, const void*
   if (group == K) wa.gshift = 30;
   else
     for (int sh = 0; sh < 16; ++sh) if (group == (32 << sh)) wa.gshift = sh;
+  wa.group_magic = group == 32 ? 0u : (unsigned)(((1ull << 32) + group / 32 - 1) / (group / 32));
   const bool can_stream = M <= 128 && K % 128 == 0 && wa.gshift >= 0;
   wa.per_element = variant == 3;
   if (variant == 3) variant = 2;
   if (variant == 2 && !can_stream) return -1;
   const bool no_split = N % 4 || out_stride % 4 || !ws;
   int rc;
-  if (variant == 2 || (variant == 0 && can_stream && (M <= 64 || bits == 4))) {   // 8 bit, 65..128 rows: tiled is faster
+  if (variant == 2 || (variant == 0 && can_stream && !wq_tiles_pay(M, N, K, bits, group, no_split))) {
     const int nk = K >> 7;
     const int groups = (N + 127) / 128;
     const int parts = wq_parts(M, N, K, bits);
@@ -763,24 +953,26 @@ VDA_EXPORT int vda_wq_gemm(void* out, const void* x, const void* qw, const void*
     if (dtype == VDA_BF16) rc = bits == 4 ? launch_wq_stream<bf16_t, 4>(wa, st) : launch_wq_stream<bf16_t, 8>(wa, st);
     else rc = bits == 4 ? launch_wq_stream<f16_t, 4>(wa, st) : launch_wq_stream<f16_t, 8>(wa, st);
   } else {
-    const int xt = M > 128 ? 8 : M > 64 ? 4 : M > 32 ? 2 : 1;
-    a.m_tiles = (M + 32 * xt - 1) / (32 * xt);
+    a.m_tiles = (M + 255) / 256;
+    const int nt = ((M + a.m_tiles - 1) / a.m_tiles + 31) / 32;
     a.n_tiles = (N + 255) / 256;
-    const int nu = K >> 5;
+    const int nu = (K + 63) >> 6;
     if (splits < 1) {
-      splits = 1;
       const long tiles = (long)a.m_tiles * a.n_tiles;
-      if (tiles * 4 < 256 * 3) splits = (int)(256 / tiles);
-      splits = min(splits, max(nu / 16, 1));
-      splits = min(splits, 16);
+      const double unit = 0.4 + 0.16 * nt;
+      double best = 1e30;
+      for (int s = 1; s <= min(16, max(nu / 4, 1)); ++s) {
+        const double t = (double)((tiles * s + 255) / 256) * ((nu + s - 1) / s * unit + 2) + (s > 1 ? 5 + s * (double)M * N * 8 / 4e6 : 0);
+        if (t < best) { best = t; splits = s; }
+      }
     }
     splits = min(splits, nu);
     if (no_split) splits = 1;
     while (splits > 1 && (size_t)splits * M * N * sizeof(float) > ws_bytes) --splits;
     a.units_per_split = (nu + splits - 1) / splits;
     a.splits = (nu + a.units_per_split - 1) / a.units_per_split;
-    if (dtype == VDA_BF16) rc = bits == 4 ? launch_wq_gemm<bf16_t, 4>(wa, xt, st) : launch_wq_gemm<bf16_t, 8>(wa, xt, st);
-    else rc = bits == 4 ? launch_wq_gemm<f16_t, 4>(wa, xt, st) : launch_wq_gemm<f16_t, 8>(wa, xt, st);
+    if (dtype == VDA_BF16) rc = bits == 4 ? launch_wq_tile<bf16_t, 4>(wa, nt, st) : launch_wq_tile<bf16_t, 8>(wa, nt, st);
+    else rc = bits == 4 ? launch_wq_tile<f16_t, 4>(wa, nt, st) : launch_wq_tile<f16_t, 8>(wa, nt, st);
   }
   if (rc) return rc;
   VDA_CHECK_LAUNCH();
