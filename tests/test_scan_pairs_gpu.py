@@ -200,6 +200,24 @@ def test_two_states_a_lane(monkeypatch, new, ctx, Ch, groups, offset, chunks):
     torch.testing.assert_close(a["ssm_state"], b["ssm_state"], atol=1e-4, rtol=1e-4)
 
 
+@pytest.mark.parametrize("N,heads", [(16, 0), (128, 1)])
+@pytest.mark.parametrize("S", [2, 63, 64, 65])
+def test_sequences_are_taken_by_length(S, N, heads):
+    # lengths that repeat, rise and fall, an absent one; more of them than are put in order
+    new = [(37 * i) % 50 + 1 for i in range(S)]
+    new[S // 2] = 0
+    new[-1] = 90
+    a = _scan_inputs(new, [i % 3 if n else 0 for i, n in enumerate(new)], 128, N, heads and 2, 1, torch.float16, S + N)
+    a = {k: v.contiguous() if isinstance(v, torch.Tensor) else v for k, v in a.items()}
+    names = ("u", "delta", "A", "B", "C", "D", "z", "delta_bias", "ssm_state")
+    f = {k: v.float() if isinstance(v, torch.Tensor) and v.dtype == torch.float16 else v.clone() if isinstance(v, torch.Tensor) else v for k, v in a.items()}
+    y = ops.selective_scan(**a, max_query_len=90)
+    want = R.selective_scan(*(f[k] for k in names), f["query_start_loc"], f["seq_lens"], f["block_table"])
+    # 32-bit sums of N states carried through up to 90 decays, one fp16 rounding of the result
+    torch.testing.assert_close(y.float(), want, atol=1e-3, rtol=2 ** -10)
+    torch.testing.assert_close(a["ssm_state"], f["ssm_state"], atol=1e-4, rtol=1e-4)
+
+
 @pytest.mark.parametrize("left_out", ["z", "D", "delta_bias"])
 def test_two_states_a_lane_without(left_out):
     a = _scan_inputs([100, 3], [0, 2], 64, 16, 0, 1, torch.bfloat16, 9)

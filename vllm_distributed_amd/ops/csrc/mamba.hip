@@ -489,6 +489,22 @@ __global__ __launch_bounds__(256) void scan_pairs_kernel(ScanArgs p) {
   }
 }
 
+// The sequence of workgroups blockIdx.y == at of a pass over whole sequences: the longest ones' start first (up to 64 of them).  What waits for a place
+// on the chip at its end is short then, and of the waves of a SIMD the first to start is the first to issue, so the longest one does not
+// walk its last tokens alone, when only every eighth cycle issues.  us, convolution and scan, in the batch's order -> this: 16 states, 8192 channels, three of
+// 1558, 1043 and 724 tokens 215 -> 207, 16 of some 180 162 -> 156, two of some 1400 305 -> 294; 128 states, 4096 channels, these three 276 -> 261, 16 of some
+// 180 231 -> 224.  (With s_setprio by length as well: 209, 159, 296, 263, 227.)  Called by whole waves.
+__device__ __forceinline__ int by_length(const int* qsl, int S, int at) {
+  if (S > 64) return at;
+  const int lane = threadIdx.x & 63;
+  const int len = lane < S ? qsl[lane + 1] - qsl[lane] : -1;
+  int before = 0;
+  for (int i = 0; i < S; ++i) {
+    const int other = __builtin_amdgcn_readlane(len, i);
+    before += other > len || (other == len && i < lane);
+  }
+  return __builtin_amdgcn_readfirstlane((int)__builtin_ctzll(__ballot(before == at && lane < S)));
+}
 // ---- selective scan, two states a lane ---------------------------------------------------------------------------------
 // 16 states with decay rates of their own (Mamba): eight lanes share a channel, two states each, so that three prompts of 8192
 // channels are 3072 waves and walk their tokens in one pass where the pairs above took two.  A SIMD issues at its full rate from
@@ -528,7 +544,7 @@ __global__ __launch_bounds__(256) void scan_lanes_kernel(ScanArgs p, int vec) {
   constexpr int N = 16;
   typedef T v4_t __attribute__((ext_vector_type(4)));
   __shared__ __attribute__((aligned(16))) float dd[LN_TT][LN_CH][2], bc[LN_TT][8][4], ys[LN_TT][LN_YS];
-  const int s = blockIdx.y;
+  const int s = MODE == 0 ? by_length(p.qsl, gridDim.y, blockIdx.y) : blockIdx.y;
   const int sl = p.seq_lens[s];
   if (sl <= 0) return;
   const int t0 = p.qsl[s], L = p.qsl[s + 1] - t0;
@@ -675,7 +691,7 @@ __global__ __launch_bounds__(256) void scan_groups_kernel(ScanArgs p) {
   constexpr int STEPS = GR_TT * PER / 256 > 0 ? GR_TT * PER / 256 : 1;
   __shared__ __attribute__((aligned(16))) float bc[GR_TT][2][N], dd[GR_TT][CH][2], ys[4][GR_TT][CH];
   __shared__ float head_dt[GR_TT][2];
-  const int s = blockIdx.y;
+  const int s = MODE == 0 ? by_length(p.qsl, gridDim.y, blockIdx.y) : blockIdx.y;
   const int sl = p.seq_lens[s];
   if (sl <= 0) return;
   const int t0 = p.qsl[s], L = p.qsl[s + 1] - t0;
