@@ -230,3 +230,17 @@ def test_router_choice(E, renorm):
         want = want / want.sum(-1, keepdim=True)
     rows = [0, 1, 2] + list(range(5, 70))
     torch.testing.assert_close(w.cpu().double()[rows], want[rows], rtol=1e-5, atol=1e-7)      # 32-bit exponentials and sums
+
+
+@pytest.mark.parametrize("gated", [True, False])
+def test_more_pairs_than_one_workgroup_sorts_in_the_grouped_kernels(monkeypatch, gated):
+    """A limit set this high sends them there; the sort then counts in memory."""
+    monkeypatch.setenv("VDA_MOE_GROUPED_MAX_PAIRS", "65536")
+    T, E, k, H, I = 5500, 8, 3, 128, 128
+    x = torch.randn(T, H, device=DEV, dtype=torch.bfloat16) * 0.5
+    w13 = torch.randn(E, (2 if gated else 1) * I, H, device=DEV, dtype=torch.bfloat16) * 0.05
+    w2 = torch.randn(E, H, I, device=DEV, dtype=torch.bfloat16) * 0.05
+    tw, ids = R.moe_topk_softmax(torch.randn(T, E, device=DEV), k, True)
+    out = ops.fused_moe(x, w13, w2, tw, ids, gated=gated)
+    ref = R.fused_moe(x, w13, w2, tw, ids, gated=gated)
+    assert _rel(out, ref) < 1.5e-2, _rel(out, ref)

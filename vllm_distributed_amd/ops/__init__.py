@@ -1402,9 +1402,9 @@ def _moe_grouped_ungated(x, w1, w2, topk_w, topk_ids, activation: str):
     dev = x.device
     ids, tw = topk_ids.contiguous(), topk_w.contiguous()
     sorted_ids = torch.empty(T * k, dtype=torch.int32, device=dev)
-    offsets = torch.empty(E + 1, dtype=torch.int32, device=dev)
+    offsets = torch.empty(E + 1 + N.value("vda_moe_align_counts", T * k, E), dtype=torch.int32, device=dev)   # (and counts)
     st = N.stream()
-    N.call("vda_moe_align", sorted_ids.data_ptr(), offsets.data_ptr(), None, None, ids.data_ptr(), T * k, E, 0, 0, st)
+    N.call("vda_moe_align", sorted_ids.data_ptr(), offsets.data_ptr(), None, offsets.data_ptr() + 4 * (E + 1), ids.data_ptr(), T * k, E, 0, 0, st)
     inter = torch.empty((T * k, I), dtype=x.dtype, device=dev)
     out2 = torch.empty((T * k, H), dtype=x.dtype, device=dev)
     out = torch.empty((T, H), dtype=x.dtype, device=dev)
@@ -1510,14 +1510,15 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, topk_w: torc
     dev = x.device
     ids = topk_ids.contiguous()
     tw = topk_w.contiguous()
-    # what passes between the launches, in one allocation (1.5 us each): both products' rows, the sorted pairs, the experts' offsets
+    # what passes between the launches, in one allocation (1.5 us each): both products' rows, the sorted pairs, the experts' offsets, and
+    # the sort's counts (of more pairs than the limits above let through by themselves)
     st, eb, n = N.stream(), x.element_size(), T * k
-    scratch = torch.empty(n * (I + H) * eb + 4 * (n + E + 1), dtype=torch.uint8, device=dev)
+    scratch = torch.empty(n * (I + H) * eb + 4 * (n + E + 1 + N.value("vda_moe_align_counts", n, E)), dtype=torch.uint8, device=dev)
     inter = scratch.data_ptr()
     out2 = inter + n * I * eb
     sorted_ids = out2 + n * H * eb
     offsets = sorted_ids + 4 * n
-    N.call("vda_moe_align", sorted_ids, offsets, None, None, ids.data_ptr(), n, E, 0, 0, st)
+    N.call("vda_moe_align", sorted_ids, offsets, None, offsets + 4 * (E + 1), ids.data_ptr(), n, E, 0, 0, st)
     out = torch.empty((T, H), dtype=x.dtype, device=dev)
     wd = N.dt(w13.dtype)
     # one expert can receive at most one slot of every token
