@@ -1,6 +1,8 @@
 """Calls of the kernel library's functions through the extension module: the same values arrive as through ctypes (no GPU: functions
 that answer from sizes, and argument checks that come ahead of a launch)."""
 import ctypes
+import gc
+import weakref
 
 import numpy as np
 import pytest
@@ -50,3 +52,27 @@ def test_a_function_that_is_not_there():
     N.lib()
     with pytest.raises(RuntimeError, match="has no kernel vda_nothing"):
         N.call("vda_nothing", 1)
+
+
+@pytest.mark.parametrize("argument", [7, ctypes.c_int(7)])          # straight from the object; through ctypes
+def test_a_name_is_bound_again_while_its_function_runs(argument):
+    """What a call uses lives until it has answered."""
+    from vllm_distributed_amd.ops import _vda_call
+    alive = []
+
+    def body(x):
+        _vda_call.bind("vda_test_again", target, "I", other)
+        gc.collect()
+        alive.append(bound() is not None)
+        return x + 1
+
+    kind = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_int)
+    code = kind(body)                                              # (holds the code that is called; what is bound holds none)
+    target = ctypes.cast(code, ctypes.c_void_p).value
+    other, function = kind(target), kind(target)
+    bound = weakref.ref(function)
+    _vda_call.bind("vda_test_again", target, "I", function)
+    del function
+    assert _vda_call.value("vda_test_again", argument) == 8
+    gc.collect()
+    assert alive == [True] and bound() is None

@@ -51,21 +51,9 @@ bool through_ctypes(const Function& fn, PyObject* const* args, Py_ssize_t n, lon
   return result != -1 || !PyErr_Occurred();
 }
 
-// args: the name, then the function's own
-bool run(PyObject* const* args, Py_ssize_t n, long& result) {
-  if (n < 1) {
-    PyErr_SetString(PyExc_TypeError, "the first argument is a function's name");
-    return false;
-  }
-  PyObject* capsule = PyDict_GetItemWithError(functions, args[0]);
-  if (!capsule) {
-    if (!PyErr_Occurred()) Py_XDECREF(PyObject_CallOneArg(missing, args[0]));
-    if (!PyErr_Occurred()) PyErr_SetObject(PyExc_KeyError, args[0]);
-    return false;
-  }
-  const Function& fn = *static_cast<Function*>(PyCapsule_GetPointer(capsule, nullptr));
-  ++args;
-  if (--n != fn.n || !fn.address) return through_ctypes(fn, args, n, result);
+// args: the function's own
+bool run_bound(const Function& fn, PyObject* const* args, Py_ssize_t n, long& result) {
+  if (n != fn.n || !fn.address) return through_ctypes(fn, args, n, result);
   long v[MOST_INTS];
   float f[MOST_FLOATS] = {};
   int nv = 0, nf = 0;
@@ -90,6 +78,25 @@ bool run(PyObject* const* args, Py_ssize_t n, long& result) {
   result = INVOKES[fn.ints](fn.address, v, f);
   Py_END_ALLOW_THREADS
   return true;
+}
+
+// args: the name, then the function's own
+bool run(PyObject* const* args, Py_ssize_t n, long& result) {
+  if (n < 1) {
+    PyErr_SetString(PyExc_TypeError, "the first argument is a function's name");
+    return false;
+  }
+  PyObject* capsule = PyDict_GetItemWithError(functions, args[0]);
+  if (!capsule) {
+    if (!PyErr_Occurred()) Py_XDECREF(PyObject_CallOneArg(missing, args[0]));
+    if (!PyErr_Occurred()) PyErr_SetObject(PyExc_KeyError, args[0]);
+    return false;
+  }
+  // (another thread, which runs while this one has given up the interpreter's lock, can bind the name anew)
+  Py_INCREF(capsule);
+  const bool answered = run_bound(*static_cast<Function*>(PyCapsule_GetPointer(capsule, nullptr)), args + 1, n - 1, result);
+  Py_DECREF(capsule);
+  return answered;
 }
 
 // call(name, *args): raises unless the function answers 0
