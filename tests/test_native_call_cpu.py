@@ -2,6 +2,8 @@
 that answer from sizes, and argument checks that come ahead of a launch)."""
 import ctypes
 import gc
+import threading
+import time
 import weakref
 
 import numpy as np
@@ -76,3 +78,29 @@ def test_a_name_is_bound_again_while_its_function_runs(argument):
     assert _vda_call.value("vda_test_again", argument) == 8
     gc.collect()
     assert alive == [True] and bound() is None
+
+
+def test_the_library_is_loaded_once(monkeypatch):
+    """Threads whose first calls come together wait for one of them to load it and to bind its functions."""
+    N.lib()
+    loads, real, started = [], ctypes.CDLL, threading.Barrier(3)
+
+    def load(path):
+        loads.append(path)
+        time.sleep(0.2)
+        return real(path)
+
+    monkeypatch.setattr(N.ctypes, "CDLL", load)
+    monkeypatch.setattr(N, "_LIB", None)
+    got = []
+
+    def first():
+        started.wait()
+        got.append(N.lib())
+
+    threads = [threading.Thread(target=first) for _ in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(loads) == 1 and len(got) == 3 and all(x is got[0] for x in got)

@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import threading
 from ctypes import c_float, c_int, c_long, c_void_p
 from typing import Optional
 
@@ -19,6 +20,7 @@ from .. import envs
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB: Optional[ctypes.CDLL] = None
+_LOAD = threading.Lock()
 
 BF16, F16, F32, FP8 = 0, 1, 2, 3
 _DT = {torch.bfloat16: BF16, torch.float16: F16, torch.float32: F32, torch.float8_e4m3fn: FP8}
@@ -159,7 +161,11 @@ def _missing(name: str) -> None:
 
 def lib() -> ctypes.CDLL:
     global _LIB, call, value
-    if _LIB is None:
+    if _LIB is not None:
+        return _LIB
+    with _LOAD:                # (threads whose first calls come together: one of them loads)
+        if _LIB is not None:
+            return _LIB
         path = library_path()
         if not os.path.exists(path):
             raise RuntimeError(
@@ -179,17 +185,18 @@ def lib() -> ctypes.CDLL:
             if name not in _LONG_RESULTS:
                 _bind(name, fn)
         _vda_call.on_missing(_missing)
-        _LIB, call, value = loaded, _vda_call.call, _vda_call.value
+        call, value, _LIB = _vda_call.call, _vda_call.value, loaded      # (in this order: whoever sees the library finds the functions)
     return _LIB
 
 
 def register(name: str, sig: list) -> None:
-    _SIGS[name] = sig
-    if _LIB is not None:
-        fn = getattr(_LIB, name)
-        fn.argtypes = sig
-        fn.restype = c_int
-        _bind(name, fn)
+    with _LOAD:
+        _SIGS[name] = sig
+        if _LIB is not None:
+            fn = getattr(_LIB, name)
+            fn.argtypes = sig
+            fn.restype = c_int
+            _bind(name, fn)
 
 
 def stream() -> int:
