@@ -5,6 +5,9 @@ lengths, the most sequences that it ranks, one more).
 
 Tolerance: a weight is rounded to 16 bits (unit u) under a sum that is not, the output once more: with weights that add up to
 one an element moves by at most 2 u max|v|; fp32 sums and the bare exponential add a few 1e-6 of it (1e-5 here)."""
+import zlib
+
+import numpy as np
 import pytest
 import torch
 
@@ -135,3 +138,35 @@ def test_tables_hold_anything_past_a_sequence(D, BS, Hq, Hkv, nsplit, fp8):
         ops.paged_attention_decode(out, q, kc, vc, rows, sl, starts, D ** -0.5, num_splits=nsplit, max_kv_len=700)
         got.append(out)
     assert not got[0].isnan().any() and torch.equal(got[0], got[1])
+
+
+# (heads, key/value heads, values, page, e4m3, parts, sequences, most keys, tokens a sequence) and the checksum of the result's bytes
+BITS = [((32, 8, 128, 16, False, 2, 25, 600, 1), 0xc6e13883),       # parts as waves of one workgroup
+        ((32, 8, 128, 16, False, 1, 40, 1300, 1), 0x12719c80),
+        ((32, 8, 128, 32, True, 1, 40, 1300, 1), 0x12dd8b1),
+        ((16, 8, 64, 16, False, 7, 20, 3000, 1), 0xc8746bd1),
+        ((16, 16, 64, 64, True, 2, 12, 500, 1), 0x9b88ecac),
+        ((24, 8, 96, 16, False, 2, 30, 500, 4), 0x5dbefaa7),
+        ((16, 8, 256, 16, False, 1, 30, 2000, 1), 0x102e32cf)]
+
+
+@pytest.mark.parametrize("case,want", BITS)
+def test_results_keep_their_bits(case, want):
+    """The order in which products and the waves' sums are added is part of the result: a recorded run, replayed, gives its logits again.
+    (Inputs are whole numbers over 64, the same wherever they are made.)"""
+    Hq, Hkv, D, BS, fp8, parts, S, most, new = case
+    lens = [max(new, 389 * (i + 1) % most) for i in range(S)]
+    rng = np.random.RandomState(D + S)
+    width = -(-max(lens) // BS)
+    pages = len(lens) * width
+
+    def some(*shape):
+        return torch.from_numpy(rng.randint(-128, 129, shape).astype(np.float32) / 64).to(torch.bfloat16).to(DEV)
+
+    q, k, v = some(len(lens) * new, Hq, D), some(pages, Hkv, BS, D), some(pages, Hkv, D, BS)
+    table = torch.from_numpy(rng.permutation(pages).astype(np.int32)).view(len(lens), width).to(DEV)
+    starts = torch.arange(len(lens) + 1, dtype=torch.int32, device=DEV) * new
+    out = torch.empty_like(q)
+    ops.paged_attention_decode(out, q, k.to(FP8) if fp8 else k, v.to(FP8) if fp8 else v, table, torch.tensor(lens, dtype=torch.int32, device=DEV),
+                               starts, D ** -0.5, num_splits=parts, max_q_len=new)
+    assert zlib.crc32(out.cpu().view(torch.uint8).numpy().tobytes()) == want

@@ -267,6 +267,12 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(AttnParams p) {
   }
 }
 
+// a product that is rounded by itself
+__device__ __forceinline__ float rounded(float v) {
+  asm("" : "+v"(v));
+  return v;
+}
+
 // Decode: a workgroup per (sequence, kv head, part of the keys); its waves share the query columns and split the keys.
 //
 // Memory is all there is to do: each key and value byte is read once, so what counts is bytes in flight.  A step is as many
@@ -279,9 +285,10 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(AttnParams p) {
 //
 // What it measured (us, before -> after): 183 sequences of 525 .. 3675 keys, 64 / 8 heads of 128, e4m3 cache 257 -> 148 (5.3 TB/s),
 // 16-bit 310 -> 271; 256 of 1100, 64 / 8 heads, e4m3 160 -> 113, 16-bit 206 -> 200 (5.8 TB/s), of 300 keys 70 -> 64; 64 of
-// 500 .. 3500, 16 / 8 heads of 256 308 -> 203 (198 since four lanes' pieces of a key row lie one behind another).  Short ones, before the pages came
-// ahead and the waves' sums met in one step -> since, with rotation and cache write: 5 of some 390 keys 13.9 -> 13.4 in a graph, ten of 46, 16 / 8
-// heads of 256, 10.8 -> 9.6; as calls 64 of 600, 32 / 8 heads, 45.2 -> 44.2, 256 of 300, e4m3, 58.3 -> 55.9.  A CU takes in 31 bytes a cycle at
+// 500 .. 3500, 16 / 8 heads of 256 308 -> 203.  Before the pages came ahead and the waves' sums met in one step -> since, attention alone in
+// a graph: 256 of some 40 keys, 32 / 8 heads, 22.4 -> 16.4, of 300 64.7 -> 58.8, 40 of 900 32.5 -> 31.6, four tokens each of 16 on 1000 24.4 -> 22.6; ten of 46, 16 / 8
+// heads of 256, 7.6 -> 6.4, 64 of 2000 198.5 -> 195.6 (193 with four lanes' pieces of a key row one behind another, whose products add in
+// another order: results keep their bits instead).  A CU takes in 31 bytes a cycle at
 // most: 675 keys of one head are 11000 cycles of the launch's 24000.  Of the first, 203 without the order of sequences below; held to the 168 registers of three
 // waves per SIMD it spills 15 and takes 177.  Non-temporal loads: e4m3 rows 6 % faster, 16-bit ones, of which a lane's pieces share
 // lines, up to 60 % slower.
@@ -298,9 +305,10 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_kernel(AttnParams p) 
   using V4 = typename Vec<T>::v4;
   constexpr int KS = D / 32;       // MFMA k-steps over the head dimension
   constexpr int NT = D / 16;       // 16-wide d tiles of the output
-  constexpr int PIECE = 16 / (int)sizeof(CT);        // d elements of 16 bytes: four lanes' pieces of a row lie one behind another
+  constexpr int PIECE = 16 / (int)sizeof(CT);        // d elements of 16 bytes
   constexpr int HS = F8 ? 2 : 1;   // 32-key halves of a step
   constexpr int RUN = 8 * HS, KEYS = 32 * HS;
+  constexpr int DQ = D / 4;        // d elements owned by one lane group in QK^T
   constexpr int KB = D / (4 * PIECE);                // pieces of a key row per lane
   constexpr int COLS = 16 * NCT;   // query columns
   constexpr int DEPTH = WAVES == 8 && D <= 128 ? 2 : 1;      // steps whose rows a wave holds (registers of two waves a SIMD)
@@ -378,9 +386,9 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_kernel(AttnParams p) 
     // a sink is a score without key or value: the running maximum starts there and the sum with its weight of one, once
     // per column: in one lane group of one wave of one part
     sink_m[ct] = (p.sink && valid && wave == 0 && part == 0) ? p.sink[head] * 1.4426950408889634f : -INFINITY;
-    const T* qp = (const T*)p.q + (long)(qs + (valid ? ti : 0)) * p.q_stride + (long)head * D + g * PIECE;
+    const T* qp = (const T*)p.q + (long)(qs + (valid ? ti : 0)) * p.q_stride + (long)head * D + g * DQ;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) qf[ct][s] = valid ? ld16<V8>(qp + s / HS * 4 * PIECE + s % HS * 8) : V8{};
+    for (int s = 0; s < KS; ++s) qf[ct][s] = valid ? ld16<V8>(qp + 8 * s) : V8{};
     col_off[ct] = valid ? (long)(qs + ti) : -1;
     if (valid) {
       wave_hi = max(wave_hi, limit[ct]); wave_lo = min(wave_lo, lower[ct]);
@@ -427,14 +435,14 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_kernel(AttnParams p) 
   auto page_at = [&](int tok) { return bt[max(min(tok / BS, page_hi), page_lo)]; };
   auto load_k = [&](int i, int st, int page) {          // half h, tile u, row r: key RUN (r / 4) + 8 h + 4 u + r % 4 of the step
     const int tok = st * KEYS + RUN * (r >> 2) + (r & 3);
-    const CT* kp = kc + (((long)page * p.Hkv + kvh) * BS + tok % BS) * (long)D + g * PIECE;
+    const CT* kp = kc + (((long)page * p.Hkv + kvh) * BS + tok % BS) * (long)D + g * DQ;
 #pragma unroll
     for (int h = 0; h < HS; ++h)
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int b = 0; b < KB; ++b)
-          kr[i][h][u][b] = *reinterpret_cast<const u32x4*>(kp + (8 * h + 4 * u) * D + b * 4 * PIECE);
+          kr[i][h][u][b] = *reinterpret_cast<const u32x4*>(kp + (8 * h + 4 * u) * D + b * PIECE);
   };
   auto load_v = [&](int i, int st, int page) {
     const int tok = st * KEYS + RUN * g;
@@ -571,7 +579,8 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_kernel(AttnParams p) 
     l[ct] += __shfl_xor(l[ct], 32, 64);
   }
   // ---- merge the waves: their sums meet in LDS, and every thread joins four values of a column over the waves --------
-  // (rows of D + 4: a lane's 16 bytes lie a bank group beside its neighbours'.  A tree over halves of the waves was two barriers a level)
+  // (rows of D + 4: a lane's 16 bytes lie a bank group beside its neighbours'.  They add as a tree over halves of the waves, each level of
+  // which was two barriers; which product is rounded and which joins the sum unrounded is part of the result's bits)
   constexpr int ROW = D + 4;
   __shared__ __attribute__((aligned(16))) float s_acc[WAVES][COLS][ROW];
   __shared__ float s_m[COLS][WAVES], s_l[COLS][WAVES];
@@ -587,17 +596,23 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_kernel(AttnParams p) 
   const int columns = min(q_len * G, COLS);
   for (int item = threadIdx.x; item < columns * (D / 4); item += 64 * WAVES) {
     const int c = item / (D / 4), d = 4 * (item % (D / 4));
-    float M = -INFINITY, L = 0.f, f[WAVES];
+    float ms[WAVES], ls[WAVES];
+    f32x4 os[WAVES];
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) M = fmaxf(M, s_m[c][w]);
-    const float Mu = (M == -INFINITY) ? 0.f : M;
-    f32x4 o = {0, 0, 0, 0};
+    for (int w = 0; w < WAVES; ++w) { ms[w] = s_m[c][w]; ls[w] = s_l[c][w]; os[w] = *reinterpret_cast<const f32x4*>(&s_acc[w][c][d]); }
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
-      f[w] = fexp2(s_m[c][w] - Mu);
-      L += s_l[c][w] * f[w];
-      o += *reinterpret_cast<const f32x4*>(&s_acc[w][c][d]) * f[w];
-    }
+    for (int cnt = WAVES / 2; cnt > 0; cnt >>= 1)
+#pragma unroll
+      for (int w = 0; w < cnt; ++w) {
+        const float M = fmaxf(ms[w], ms[w + cnt]), Mu = (M == -INFINITY) ? 0.f : M;
+        const float f1 = fexp2(ms[w] - Mu), f2 = fexp2(ms[w + cnt] - Mu);
+        ls[w] = fmaf(ls[w], f1, rounded(ls[w + cnt] * f2));
+        ms[w] = M;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) os[w][j] = fmaf(os[w + cnt][j], f2, rounded(os[w][j] * f1));
+      }
+    const float L = ls[0], Mu = ms[0] == -INFINITY ? 0.f : ms[0];
+    f32x4 o = os[0];
     o *= L > 0.f ? p.v_scale / L : 0.f;
     const int head = kvh * G + c % G;
     const long token = qs + c / G;
