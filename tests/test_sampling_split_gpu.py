@@ -24,7 +24,13 @@ def _noise(seed: int, V: int) -> np.ndarray:
     return -np.log(-np.log(((_words(seed, V) >> np.uint32(8)).astype(np.float64) + 0.5) / 16777216.0))
 
 
-def _scores(row, temp, k, p, mp, seed):
+def _noise32(seed: int, V: int) -> np.ndarray:
+    """The same of the 32-bit u that the kernels have: close to 1, where the largest noise comes from, its steps are up to 1 % of that noise's exponential."""
+    u = ((_words(seed, V) >> np.uint32(8)).astype(np.float32) + np.float32(0.5)) * np.float32(2.0 ** -24)
+    return -np.log(-np.log(np.minimum(u, np.float32(1 - 2.0 ** -24)).astype(np.float64)))
+
+
+def _scores(row, temp, k, p, mp, seed, noise=_noise):
     """Noisy logits of the kept tokens, -inf elsewhere, and the same with one more token kept at the top-p edge (its
     weight may fall on either side: weights are rounded to 2^-32 and come from a 32-bit exponential)."""
     z = row.double().numpy() / temp
@@ -44,7 +50,7 @@ def _scores(row, temp, k, p, mp, seed):
             keep = z == z.max()
     if mp > 0:
         keep, edge = keep & (z >= z.max() + np.log(mp) + 1e-5), edge & (z >= z.max() + np.log(mp) - 1e-5)
-    g = z + _noise(seed, len(z))
+    g = z + noise(seed, len(z))
     return np.where(keep, g, -np.inf), np.where(edge, g, -np.inf)
 
 
@@ -243,3 +249,73 @@ def test_bins_cut_where_the_one_workgroup_form_does(shape):
     args = [t.to(DEV) for t in (temp, k, p, mp, seeds)]
     wide = torch.cat([x, torch.full((S, 1), -float("inf"))], 1)
     assert torch.equal(ops.sample(wide.to(DEV), *args), ops.sample(x.to(DEV), *args))
+
+
+# rows of nearly equal logits are cut on finer grids: each of them, its ends, shares on different ones, shares further apart than a grid's ring, masked
+# and NaN entries among them
+@pytest.mark.parametrize("V", [8191, 20000])
+@pytest.mark.parametrize("shape", [4.0, 1.0, 0.2, 0.05, 0.01, 0.002, 1e-4, 1e-6, "offset", "edges", "apart", "ramp", "peak", "masked", "nan"])
+def test_flat_rows_are_cut_where_the_sorted_form_does(V, shape):
+    g = torch.Generator().manual_seed(V + len(str(shape)))
+    S = 24
+    x = torch.randn(S, V, generator=g) * (shape if isinstance(shape, float) else 0.01)
+    if shape == "offset":
+        x = x + torch.tensor([1000.0, -300.0, 40000.0, 15.9])[torch.arange(S) % 4, None]
+    elif shape == "edges":
+        x = (x * 2 ** 17).round() / 2 ** 17
+    elif shape == "apart":
+        x[:, V // 2:] -= torch.tensor([0.3, 1.0, 5.0, 40.0])[torch.arange(S) % 4, None]
+    elif shape == "ramp":
+        x = x.sort(dim=1).values
+        x[::2] *= 30.0
+    elif shape == "peak":
+        x[:, 77] = 9.0
+    elif shape == "masked":
+        x[:, V // 3:] = torch.where(torch.rand(S, V - V // 3, generator=g) < 0.7, -float("inf"), x[:, V // 3:])
+        x[:4, 4096:] = -float("inf")
+    elif shape == "nan":
+        x.scatter_(1, torch.randint(0, V, (S, 3), generator=g), float("nan"))
+    r = torch.arange(S)
+    k = torch.where(r % 3 == 1, torch.randint(1, 3000, (S,), generator=g), 0).to(torch.int32)
+    p = torch.where(r % 3 == 1, torch.where(r % 2 == 0, 1.0, 0.9), 0.02 + 0.97 * torch.rand(S, generator=g))
+    temp = 0.4 + torch.rand(S, generator=g)
+    seeds = torch.randint(0, 2 ** 62, (S,), generator=g)
+    args = [t.to(DEV) for t in (temp, k, p, None, seeds) if t is not None]
+    args.insert(3, None)
+    got = ops.sample(x.to(DEV), *args)
+    if V == 8191:                              # one workgroup a row, several with a masked entry more
+        assert torch.equal(ops.sample(torch.cat([x, torch.full((S, 1), -float("inf"))], 1).to(DEV), *args), got)
+    if shape == "nan":
+        return
+    for s in range(S):
+        sure, may = _scores(x[s], float(temp[s]), int(k[s]), float(p[s]), 0.0, int(seeds[s]), _noise32)
+        # as above; offsets to 1e5 after the temperature: 2^-7 of rounding
+        assert may[int(got[s])] >= sure.max() - (2.0 ** -6 if shape == "offset" else 2.0 ** -14), s
+
+
+@pytest.mark.parametrize("std", [2.0, 0.3, 0.04, 0.02, 0.005, 5e-4])
+@pytest.mark.parametrize("V", [128256, 151936])
+def test_flat_rows_collect_short_lists(V, std):
+    """Rows of nearly equal logits stay with the workgroups that share them: what is collected at the cut fits the list (4096 entries), else one
+    workgroup does the row's ten passes alone.  A grid has 400 entries a bin on average or some 190 bins between a row's ends, whichever are more
+    entries; between a normal distribution's, some 9 std, the densest point has 0.4 * 9 times the average: 2900 entries a bin of 151936."""
+    g = torch.Generator().manual_seed(V)
+    S, per_row, at = 8, 2320, 1792 // 4        # bytes of a row's workspace (SplitRow), words before its counts of collected entries, one a workgroup
+    x = torch.randn(S, V, generator=g) * std
+    x[0, 5] = -float("inf")
+    temp = torch.where(torch.arange(S) % 4 == 3, 50.0, 1.0)
+    k = torch.where(torch.arange(S) % 2 == 1, torch.tensor([50, 20000, 64000, V - 9])[torch.arange(S) // 2], 0).to(torch.int32)
+    p = torch.where(torch.arange(S) % 2 == 0, torch.tensor([0.9, 0.5, 0.98, 0.1])[torch.arange(S) // 2], 1.0)
+    seeds = torch.randint(0, 2 ** 62, (S,), generator=g)
+    xd, td, kd, pd, sd = (t.to(DEV) for t in (x, temp, k, p, seeds))
+    n = ops.N.lib().vda_sample_workspace(S, V, 1)
+    ws = torch.zeros(n, dtype=torch.uint8, device=DEV)
+    out = torch.empty(S, dtype=torch.long, device=DEV)
+    ops.N.call("vda_sample", xd.data_ptr(), out.data_ptr(), td.data_ptr(), kd.data_ptr(), pd.data_ptr(), None, sd.data_ptr(), S, V, V, ws.data_ptr(),
+               n, ops.N.stream())
+    collected = ws[:per_row * S].view(torch.int32).view(S, -1)[:, at:at + 64].long() & 0xffffffff
+    assert int(collected.sum(1).max()) <= 4096, collected.sum(1)
+    assert torch.equal(out, ops.sample(xd, td, kd, pd, None, sd))
+    for s in range(S):
+        sure, may = _scores(x[s], float(temp[s]), int(k[s]), float(p[s]), 0.0, int(seeds[s]), _noise32)
+        assert may[int(out[s])] >= sure.max() - 2.0 ** -14, s

@@ -283,7 +283,8 @@ __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs p) {
 // all hit the few leading bytes real logits share: 447 us for 61 rows of V = 128256, 73 us for one.  Here a row takes G
 // workgroups and three launches:
 //   survey   the maximum of a workgroup's share and, from its registers, counts (top-k) or weights (top-p) of what lies below that
-//            maximum.  The bins lie on a grid that does not depend on the row, so that the shares' sums can meet in the next launch.
+//            maximum.  The bins lie on a grid that does not depend on the row, so that the shares' sums can meet in the next launch; shares
+//            whose entries lie close together (flat heads, high temperatures) fill a finer grid and from it the coarser ones.
 //            Rows without a filter draw here at once, greedy ones take their argmax
 //   collect  the bin in which the running sum over the row's bins reaches the target; draws among the entries above it, collects
 //            that bin's entries (top-k and top-p together: all entries down to it), and sums the exact weights
@@ -291,18 +292,24 @@ __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs p) {
 // The survey's weights are estimates, relative to the top of their bin (the row's maximum is not known yet) and of 2^-16 each.  Where the target
 // comes that close to a bin's edge, both bins are collected; and the finish, which has the exact sums, hands a row whose collected bins do not
 // hold its threshold to the one-workgroup form, so the result never hangs on the estimate.  A row whose bins overflow a list (thousands of equal
-// logits), with NaN under a top-k, or with a maximum beyond the grid goes the same way.
+// logits, or of logits within 1 / 128 beside others that are further apart than a finer grid reaches), with NaN under a top-k, or with a maximum
+// beyond the grid goes the same way.
 // The result is that of the one-workgroup form: the bins are monotone in the key, sums are integers, and each number is rounded alike
 // in every kernel (opaque).
 // Bound by issue and by trips to memory of a microsecond each: 61 rows, kernel times: 14 where rows without a filter draw (the noise's 64-bit hash
 // is 45 issue slots an entry) and 12 where bins are counted, of 8.6 for a read; 19 in the collecting launch for rows of top-p (exact weights 12 slots
 // an entry; what is drawn from is brought together 64 entries at a time), 9 in the last.  us a call, with a launch more, in which statistics came
 // ahead of bins between the row's extremes -> this: 61 rows of 128256 48 -> 38, one 19 -> 16.5, 256 of 151936 128 -> 104, 148 of 32000 60 -> 35, five
-// 26 -> 20.  All bins of a row in every workgroup instead of groups first: 42 instead of 38.  One launch for collect and finish, the row's last
-// workgroup finishing it, is no way: the fences it needs took it from 20 to 155 us.
+// 26 -> 20.  Normally distributed logits of a standard deviation of 2, 0.3, 0.04 and 0.005, 61 rows of 128256 under a top-p of 0.9: 37, 45, 48.6 and 49.4
+// (most entries of the last ones are drawn from), with one grid alone 37, 44, 265 and 262; 256 of 151936 98, 131, 134 and 136.  All bins of a row
+// in every workgroup instead of groups first: 42 instead of 38.  One launch for collect and finish, the row's last workgroup finishing it, is no
+// way: the fences it needs took it from 20 to 155 us.
 constexpr int SPLIT_BINS = 4096;      // a ring in groups of 64: bin b of the grid is at b mod SPLIT_BINS; the row's top SPLIT_GROUPS groups count
 constexpr int SPLIT_GROUPS = SPLIT_BINS / 64;          // a lane each
-constexpr float SPLIT_PER = 128.f;    // bins a unit of logit (counts) or of scaled logit (weights, whose 2^-32 is 22.2 units down)
+constexpr int SPLIT_LEVELS = 4;       // grids: 128 bins a unit of logit (counts) or of scaled logit (weights, whose 2^-32 is 22.2 units down), then eight for one
+// A finer grid is for rows of more than SPLIT_CROWD entries a bin between their ends, and has at most SPLIT_SPREAD bins between them, so that
+// the shares' entries lie in the row's ring though the ends are those of a few of the entries.
+constexpr float SPLIT_CROWD = 400.f, SPLIT_SPREAD = 1500.f;
 constexpr int SPLIT_LIST = 4096;      // collected entries of a row
 constexpr int SPLIT_MAX_G = 64;
 constexpr int SPLIT_MIN_V = 8192;     // shorter rows: the launches cost more than the one-workgroup form's passes
@@ -325,14 +332,20 @@ struct SplitRow {                     // workspace of one row: a word of each of
   float part_v[SPLIT_MAX_G];
   int part_i[SPLIT_MAX_G];
   uint32_t part_n[SPLIT_MAX_G];       // collected entries, also past the list's end
-  uint32_t finite[SPLIT_MAX_G];       // entries above -inf (counts); SPLIT_NAN
+  uint32_t finite[SPLIT_MAX_G];       // entries above -inf (counts), SPLIT_LEVEL times the share's finest grid, SPLIT_NAN
   uint32_t rem, counts, pad[2];       // what is left of a count in the collected bins, where one is left
 };
+constexpr int SPLIT_GRID = SPLIT_BINS + SPLIT_GROUPS;
 struct SplitPart {                    // workspace of one workgroup
-  uint32_t hist[SPLIT_BINS], group[SPLIT_GROUPS];      // and the groups' sums: counts, or weights relative to the group's top as a float
-  uint2 list[SPLIT_LIST];             // (key, token)
+  union {
+    struct {
+      uint32_t grid[SPLIT_GRID];      // bins, and the groups' sums: counts, or weights relative to the group's top as a float
+      uint2 list[SPLIT_LIST];         // (key, token)
+    };
+    uint32_t finer[SPLIT_LEVELS - 1][SPLIT_GRID];      // (in a second one, where its entries lie close together)
+  };
 };
-constexpr uint32_t SPLIT_NAN = 0x80000000u, SPLIT_ALONE = 0xffffffffu;
+constexpr uint32_t SPLIT_NAN = 0x80000000u, SPLIT_LEVEL = 0x08000000u, SPLIT_ALONE = 0xffffffffu;
 constexpr int SPLIT_RANKED = 256;     // entries that can be ranked at once
 constexpr int SPLIT_DIRECT = 96;      // and that are: n of them are n^2 / 8 cycles of LDS reads
 struct KeyWeight { uint32_t key; unsigned long long weight; };
@@ -401,29 +414,43 @@ template <bool VEC, int E> __device__ __forceinline__ void split_load(const floa
     }
   }
 }
-// the bin of x on the grid, a whole number; NaN and infinities stay what they are
-__device__ __forceinline__ float split_bin(float x) { return floorf(opaque(x) * SPLIT_PER); }
+// a grid's bins a unit and the width of one: powers of two
+__device__ __forceinline__ float split_per(int level) { return __int_as_float((127 + 7 + 3 * level) << 23); }
+__device__ __forceinline__ float split_width(int level) { return __int_as_float((127 - 7 - 3 * level) << 23); }
+// the bin of x on a grid, a whole number; NaN and infinities stay what they are
+__device__ __forceinline__ float split_bin(float x, float per) { return floorf(opaque(x) * per); }
+// The finest grid for a share of a row of V, with entries (above -inf) from some mn to mx
+__device__ __forceinline__ int split_level(float mx, float mn, int V) {
+  const float spread = mx - mn, far = fmaxf(fabsf(mx), fabsf(mn));
+  int level = 0;
+  while (level < SPLIT_LEVELS - 1 && SPLIT_CROWD * (spread * split_per(level)) < (float)V && spread * split_per(level + 1) <= SPLIT_SPREAD &&
+         far * split_per(level + 1) < SPLIT_FAR_COUNTS) ++level;
+  return mx == -INFINITY ? SPLIT_LEVELS - 1 : level;     // (no entry)
+}
 
-// the sum over a row of 16 lanes, in its last one
-template <typename T> __device__ __forceinline__ T row_sum(T v) {
+// an inclusive scan over a row of 16 lanes; ``none``: what joins nothing
+template <typename T, typename F> __device__ __forceinline__ T row_scan(T v, T none, F join) {
   const auto from = [&](auto ctrl) {
-    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value, 0xf, 0xf, false));
+    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, none), __builtin_bit_cast(int, v), decltype(ctrl)::value, 0xf, 0xf,
+                                                             false));
   };
   using std::integral_constant;
-  v += from(integral_constant<int, 0x111>());
-  v += from(integral_constant<int, 0x112>());
-  v += from(integral_constant<int, 0x114>());
-  v += from(integral_constant<int, 0x118>());
+  v = join(v, from(integral_constant<int, 0x111>()));
+  v = join(v, from(integral_constant<int, 0x112>()));
+  v = join(v, from(integral_constant<int, 0x114>()));
+  v = join(v, from(integral_constant<int, 0x118>()));
   return v;
 }
+// the sum over it, in its last lane
+template <typename T> __device__ __forceinline__ T row_sum(T v) { return row_scan(v, T(0), [](T a, T b) { return a + b; }); }
 // a thread's sum of weights (below 2^45) added over the wave, in its last lane: 20 bits and the rest
 __device__ __forceinline__ unsigned long long wave_weight(unsigned long long w) {
   return ((unsigned long long)scan_add((uint32_t)(w >> 20)) << 20) + scan_add((uint32_t)w & 0xfffffu);
 }
 
-constexpr float SPLIT_UNIT = 1.4426950408889634f / SPLIT_PER;        // log2 of the weight between two bins
-// of bin f of a group relative to its highest bin
-__device__ __forceinline__ float group_weight(int f) { return __builtin_amdgcn_exp2f((float)(f - 63) * SPLIT_UNIT); }
+// log2 of the weight between two bins, and the weight of a bin ``down`` bins below another
+__device__ __forceinline__ float split_unit(int level) { return 1.4426950408889634f * split_width(level); }
+__device__ __forceinline__ float split_weight(int down, float unit) { return __builtin_amdgcn_exp2f((float)-down * unit); }
 
 // a thread walks its share in order: the first of equals stays
 __device__ __forceinline__ void later(ArgMax& a, float v, int i) {
@@ -431,7 +458,7 @@ __device__ __forceinline__ void later(ArgMax& a, float v, int i) {
 }
 
 struct SurveyLds {
-  float red[16], rv[16];
+  float red[16], low[16], rv[16];
   int ri[16];
   uint32_t finite;
   uint4 hist[SPLIT_BINS / 2];         // two copies of each word: lanes that meet in one wait for each other
@@ -470,7 +497,7 @@ __device__ __forceinline__ void split_survey(const SampleArgs& p, const SplitFil
   s.hist[threadIdx.x] = s.hist[threadIdx.x + 1024] = uint4{0u, 0u, 0u, 0u};
   if (threadIdx.x == 0) s.finite = 0u;
   const float scale = f.k ? 1.f : f.inv_t;
-  float v[SPLIT_HOLDS], mx = -INFINITY;
+  float v[SPLIT_HOLDS], mx = -INFINITY, first = 0.f;
   uint32_t finite = 0u;
   bool nan = false;
   int at = c.a;
@@ -485,26 +512,40 @@ __device__ __forceinline__ void split_survey(const SampleArgs& p, const SplitFil
         nan |= v[e] != v[e];
       }
     }
+    if (at == c.a) first = v[0];
     if (at + 1024 * SPLIT_HOLDS >= c.b) break;
     at += 1024 * SPLIT_HOLDS;
   }
-  mx = block_max(mx, s.red);
+  const int lane = threadIdx.x & 63;
+  mx = all_max(mx);
+  // Whether the entries lie close together, as far as one a thread says: a guess is enough, what a ring does not hold lies below what it holds
+  first = first > -INFINITY ? first * scale : INFINITY;
+  float mn = -INFINITY;
+  if (!__any(first < mx - SPLIT_SPREAD * split_width(1))) mn = -all_max(-first);
+  if (lane == 0) { s.red[threadIdx.x >> 6] = mx; s.low[threadIdx.x >> 6] = -mn; }
+  __syncthreads();
+  {
+    const float both = row_scan(lane < 16 ? s.red[lane] : s.low[lane & 15], -INFINITY, [](float a, float b) { return fmaxf(a, b); });
+    mx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(both), 15));
+    mn = -__int_as_float(__builtin_amdgcn_readlane(__float_as_int(both), 31));
+  }
   if (f.k) {
     finite = scan_add(finite);
     const bool any = __any(nan);
-    if ((threadIdx.x & 63) == 63) atomicAdd(&s.finite, finite);
-    if (any && (threadIdx.x & 63) == 0) atomicOr(&s.finite, SPLIT_NAN);
+    if (lane == 63) atomicAdd(&s.finite, finite);
+    if (any && lane == 0) atomicOr(&s.finite, SPLIT_NAN);
   }
-  const float top_group = floorf(split_bin(mx) * (1.f / 64.f));
+  const int finest = split_level(mx, mn, p.V);
+  const float per = split_per(finest), top_group = floorf(split_bin(mx, per) * (1.f / 64.f)), width_log = split_unit(finest);
   uint32_t* hist = reinterpret_cast<uint32_t*>(s.hist) + (threadIdx.x & 1);
   for (;;) {                                            // from the entries that are still held backwards
 #pragma unroll
     for (int e = 0; e < SPLIT_HOLDS; ++e) {
       if (!split_any<VEC>(at, e, c.b)) break;
-      const float x = v[e] * scale, b = split_bin(x);
+      const float x = v[e] * scale, b = split_bin(x, per);
       if (top_group - floorf(b * (1.f / 64.f)) < (float)SPLIT_GROUPS) {
         uint32_t w = 1u;
-        if (!f.k) w = (uint32_t)fmaf(__builtin_amdgcn_exp2f((x * SPLIT_PER - (b + 1.f)) * SPLIT_UNIT), unit, 0.5f);
+        if (!f.k) w = (uint32_t)fmaf(__builtin_amdgcn_exp2f((x * per - (b + 1.f)) * width_log), unit, 0.5f);
         atomicAdd(hist + 2 * ((int)b & (SPLIT_BINS - 1)), w);
       }
     }
@@ -512,16 +553,32 @@ __device__ __forceinline__ void split_survey(const SampleArgs& p, const SplitFil
     at -= 1024 * SPLIT_HOLDS;
     split_load<VEC>(row, at, c.b, v);
   }
-  __syncthreads();
-  const uint4 q0 = s.hist[2 * threadIdx.x], q1 = s.hist[2 * threadIdx.x + 1];
-  const uint4 h = {q0.x + q0.y, q0.z + q0.w, q1.x + q1.y, q1.z + q1.w};
-  *reinterpret_cast<uint4*>(part->hist + 4 * threadIdx.x) = h;
-  const int b0 = 4 * (threadIdx.x & 15);                // 16 threads a group
-  const uint32_t group = f.k ? row_sum(h.x + h.y + h.z + h.w)
-                             : __float_as_uint(row_sum((float)h.x * group_weight(b0) + (float)h.y * group_weight(b0 + 1) +
-                                                       (float)h.z * group_weight(b0 + 2) + (float)h.w * group_weight(b0 + 3)));
-  if ((threadIdx.x & 15) == 15) part->group[threadIdx.x >> 4] = group;
-  if (threadIdx.x == 0) { ws->part_max[blockIdx.x] = mx; ws->finite[blockIdx.x] = s.finite; }
+  // this grid and, eight bins to one, those before it: the row takes the finest that all its shares have
+  int top = mx > -INFINITY ? (int)top_group : 0;
+  for (int level = finest;; --level) {
+    __syncthreads();
+    const uint4 q0 = s.hist[2 * threadIdx.x], q1 = s.hist[2 * threadIdx.x + 1];
+    const uint4 h = {q0.x + q0.y, q0.z + q0.w, q1.x + q1.y, q1.z + q1.w};
+    uint32_t* grid = level == 0 ? part->grid : part[gridDim.x * gridDim.y].finer[level - 1];
+    *reinterpret_cast<uint4*>(grid + 4 * threadIdx.x) = h;
+    const int down = 63 - 4 * (threadIdx.x & 15);       // 16 threads a group
+    const float u = split_unit(level);
+    const uint32_t group = f.k ? row_sum(h.x + h.y + h.z + h.w)
+                               : __float_as_uint(row_sum((float)h.x * split_weight(down, u) + (float)h.y * split_weight(down - 1, u) +
+                                                         (float)h.z * split_weight(down - 2, u) + (float)h.w * split_weight(down - 3, u)));
+    if ((threadIdx.x & 15) == 15) grid[SPLIT_BINS + (threadIdx.x >> 4)] = group;
+    if (level == 0) break;
+    __syncthreads();
+    s.hist[threadIdx.x] = s.hist[threadIdx.x + 1024] = uint4{0u, 0u, 0u, 0u};
+    __syncthreads();
+    const int bin = 64 * (top - ((top - (int)(threadIdx.x >> 4)) & (SPLIT_GROUPS - 1))) + 4 * (threadIdx.x & 15), to = 7 - (bin & 7);
+    const uint32_t sum = f.k ? h.x + h.y + h.z + h.w
+                             : (uint32_t)((float)h.x * split_weight(to, u) + (float)h.y * split_weight(to - 1, u) +
+                                          (float)h.z * split_weight(to - 2, u) + (float)h.w * split_weight(to - 3, u) + 0.5f);
+    if (sum) atomicAdd(hist + 2 * ((bin >> 3) & (SPLIT_BINS - 1)), sum);
+    top >>= 3;
+  }
+  if (threadIdx.x == 0) { ws->part_max[blockIdx.x] = mx; ws->finite[blockIdx.x] = s.finite | (uint32_t)finest * SPLIT_LEVEL; }
 }
 __global__ __launch_bounds__(1024, 8) void split_survey_kernel(SampleArgs p, SplitRow* ws_rows, SplitPart* ws_parts, int row0, float unit) {
   __shared__ SurveyLds s;
@@ -535,7 +592,7 @@ __global__ __launch_bounds__(1024, 8) void split_survey_kernel(SampleArgs p, Spl
 }
 
 // Where a row is cut: entries of ``draw_from`` and more are drawn from at once, others of ``list_from`` and more (and above -inf) are
-// collected.  In logits (counts) or scaled logits: a bin's edges are multiples of 1 / SPLIT_PER.
+// collected.  In logits (counts) or scaled logits: a bin's edges are multiples of its grid's width.
 struct SplitCut {
   float draw_from, list_from;
   uint32_t rem, n;                    // counts: what is left of k in the collected bins, the entries that these hold
@@ -556,7 +613,7 @@ struct SplitSums { uint32_t h[SPLIT_ASKED]; };
 __device__ __forceinline__ SplitSums split_sums(const SplitPart* parts, int w0, int G, int word) {
   SplitSums r;
 #pragma unroll
-  for (int j = 0; j < SPLIT_ASKED; ++j) r.h[j] = (&parts[min(w0 + j, G - 1)].hist[0])[word];
+  for (int j = 0; j < SPLIT_ASKED; ++j) r.h[j] = (&parts[min(w0 + j, G - 1)].finer[0][0])[word];
   return r;
 }
 // a lane's word over the workgroups.  A ring's word stands for one of the row's groups if that is not above the workgroup's own highest group
@@ -575,21 +632,22 @@ __device__ __forceinline__ void split_join(const SplitPart* parts, SplitSums sum
   }
 }
 __device__ __forceinline__ SplitCut split_cut(const SplitFilter& f, const SplitPart* parts, const SplitSums& sums, int G, int highest, int row_top,
-                                              uint32_t finite, float margin) {
-  const int lane = threadIdx.x & 63, row_group = row_top >> 6;
+                                              uint32_t finite, float margin, int level) {
+  const int lane = threadIdx.x & 63, row_group = row_top >> 6, grid = level > 0 ? (level - 1) * SPLIT_GRID : 0;
+  const float width = split_width(level), unit = split_unit(level);
   // sums came by word of the ring; from the row's highest group down: lane l takes the word of group row_group - l
   const int word = lane, mine = row_group - ((row_group - word) & (SPLIT_GROUPS - 1));
   const int from = 4 * ((row_group - lane) & (SPLIT_GROUPS - 1));
-  const auto edge = [&](int bin) { return (float)bin * (1.f / SPLIT_PER); };
+  const auto edge = [&](int bin) { return (float)bin * width; };
   SplitCut cut{-FLT_MAX, INFINITY, 0u, 0u, false};
   if (f.k) {
     const uint32_t k = (uint32_t)f.k;
     uint32_t count = 0u;
-    split_join(parts, sums, G, SPLIT_BINS + word, mine, highest, [&](uint32_t h) { count += h; });
+    split_join(parts, sums, G, grid + SPLIT_BINS + word, mine, highest, [&](uint32_t h) { count += h; });
     count = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)count);
     const uint32_t cum = scan_add(count), all = last_lane(cum);
     if (k <= all) {
-      const int l = __ffsll(__ballot(cum >= k)) - 1, group = row_group - l, at = 64 * (group & (SPLIT_GROUPS - 1)) + 63 - lane;
+      const int l = __ffsll(__ballot(cum >= k)) - 1, group = row_group - l, at = grid + 64 * (group & (SPLIT_GROUPS - 1)) + 63 - lane;
       const uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)(cum - count), l);
       uint32_t bin = 0u;
       split_join(parts, split_sums(parts, 0, G, at), G, at, group, highest, [&](uint32_t h) { bin += h; });
@@ -608,17 +666,17 @@ __device__ __forceinline__ SplitCut split_cut(const SplitFilter& f, const SplitP
     }
   } else {
     float weight = 0.f;
-    split_join(parts, sums, G, SPLIT_BINS + word, mine, highest, [&](uint32_t h) { weight += __uint_as_float(h); });
+    split_join(parts, sums, G, grid + SPLIT_BINS + word, mine, highest, [&](uint32_t h) { weight += __uint_as_float(h); });
     weight = __int_as_float(__builtin_amdgcn_ds_bpermute(from, __float_as_int(weight)));
     // (relative to the maximum's group's top)
-    weight *= __builtin_amdgcn_exp2f((float)(-64 * lane) * SPLIT_UNIT);
-    const float cum = scan_add(weight), all = last_lane(cum), target = f.tp * all, off = margin * all;
+    weight *= split_weight(64 * lane, unit);
+    const float cum = scan_add(weight), all = last_lane(cum), target = f.tp * all, off = margin * (float)(1 + level) * all;
     const unsigned long long reached = __ballot(cum + off >= target);
-    const int l = reached ? __ffsll(reached) - 1 : 0, group = row_group - l, at = 64 * (group & (SPLIT_GROUPS - 1)) + 63 - lane;
+    const int l = reached ? __ffsll(reached) - 1 : 0, group = row_group - l, at = grid + 64 * (group & (SPLIT_GROUPS - 1)) + 63 - lane;
     const float before = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cum - weight), l));
     float bin = 0.f;
     split_join(parts, split_sums(parts, 0, G, at), G, at, group, highest, [&](uint32_t h) { bin += (float)h; });
-    const float upto = before + scan_add(bin * __builtin_amdgcn_exp2f((float)(-64 * l - lane) * SPLIT_UNIT));
+    const float upto = before + scan_add(bin * split_weight(64 * l + lane, unit));
     const unsigned long long lo = __ballot(upto + off >= target), hi = __ballot(upto - off >= target);
     // (the target at the group's end: the next group's first bin joins, and the finish has the last word)
     const int b = lo ? __ffsll(lo) - 1 : 63, e = hi ? __ffsll(hi) - 1 : 64;
@@ -720,14 +778,26 @@ __global__ __launch_bounds__(1024, 8) void split_collect_kernel(SampleArgs p, Sp
   const SplitFilter f = split_filter(p, rowi);
   if (f.greedy || (f.mode == MODE_NONE && !(f.mp > 0.f) && !p.late)) return;
   if (threadIdx.x == 0) { s.n = 0u; s.sum[0] = s.sum[1] = 0ull; }
-  const float mx = all_max(part_max), zmax = f.k ? mx * f.inv_t : mx, top = split_bin(mx);
+  const float mx = all_max(part_max), zmax = f.k ? mx * f.inv_t : mx;
   SplitCut cut{-FLT_MAX, INFINITY, 0u, 0u, false};
   bool alone = false;
   if (f.mode != MODE_NONE) {
+    const int finest = (int)(part_finite / SPLIT_LEVEL) & 15;
+    int level = 0;
+    if (!__any(lane < G && finest == 0)) {              // entries close together: the finest grid that all have, and whose ring holds all of them
+      level = last_lane(wave_scan(lane < G ? finest : SPLIT_LEVELS - 1, SPLIT_LEVELS - 1, [](int a, int b) { return min(a, b); }));
+      const float lowest = -all_max(part_max > -INFINITY ? -part_max : -INFINITY);
+      while (level > 0 && (mx - lowest) * split_per(level) > SPLIT_SPREAD) --level;
+      if (level > 0) {
+        parts += G * gridDim.y;
+        sums = split_sums(parts, 0, G, (level - 1) * SPLIT_GRID + SPLIT_BINS + lane);
+      }
+    }
+    const float per = split_per(level), top = split_bin(mx, per);
     alone = !(fabsf(top) < (f.k ? SPLIT_FAR_COUNTS : SPLIT_FAR)) || (f.k && __any((part_finite & SPLIT_NAN) != 0u));
     if (!alone) {
-      const uint32_t finite = last_lane(scan_add(part_finite));
-      cut = split_cut(f, parts, sums, G, (int)fmaxf(split_bin(part_max), -SPLIT_FAR) >> 6, (int)top, finite, margin);
+      const uint32_t finite = last_lane(scan_add(part_finite & (SPLIT_LEVEL - 1u)));
+      cut = split_cut(f, parts, sums, G, (int)fmaxf(split_bin(part_max, per), -SPLIT_FAR) >> 6, (int)top, finite, margin, level);
       alone = cut.n > (uint32_t)SPLIT_LIST;
     }
   }
@@ -1041,7 +1111,7 @@ VDA_EXPORT long vda_sample_workspace(int S, int V, int filtered) {
   long parts = 0;
   for (int rows : {min(S, SPLIT_ROWS), S % SPLIT_ROWS})
     if (rows > 0) parts = max(parts, (long)rows * split_groups(rows, V));
-  return (long)sizeof(SplitRow) * min(S, SPLIT_ROWS) + (long)sizeof(SplitPart) * parts;
+  return (long)sizeof(SplitRow) * min(S, SPLIT_ROWS) + (long)sizeof(SplitPart) * (filtered ? 2 : 1) * parts;
 }
 
 VDA_EXPORT int vda_sample(const float* logits, long* out, const float* temperature, const int* top_k,
