@@ -361,7 +361,7 @@ def paged_attention_prefill(out, q, k_cache, v_cache, block_table, seq_lens, q_s
     for bound in (max_kv_len, window + 128 if window > 0 else 0, chunk + 128 if chunk > 0 else 0):
         keys = min(keys, bound) if bound > 0 else keys
     if not return_lse:
-        parts = N.value("vda_prefill_parts", seq_lens.shape[0], T, Hq, Hkv, D, keys)
+        parts = max(N.value("vda_prefill_form", seq_lens.shape[0], T, Hq, Hkv, D, keys, int(max_q_len)), 1)
         if parts > 1:
             part = torch.empty(T * Hq * parts * (D + 1), dtype=torch.float32, device=q.device)
             part_out = part.data_ptr()

@@ -1237,11 +1237,17 @@ static int wide_tokens(int G, int D, int num_tokens, int num_seqs) {
 // Of 96, 16 / 8 heads, 104 x 20 27 / 31, 52 x 40 25.2 / 24.6, 51 x 70 38 / 32; 16 / 16, 52 x 40 32 / 34, 51 x 70 + 300 85 / 70, 12 x 300 67 / 48.
 // Of 64, in one wave of workgroups, 32 / 8, 26 x 40 17.7 / 18.8, 15 x 70 18.1 / 16.0, 11 x 100 + 300 39 / 28, 8 / 4, 60 x 70 21 / 18; in more, 32 / 32, 32 x 100 51 / 54, 16 / 4,
 // 43 x 150 + 300 53 / 59, 12 / 12, 57 x 150 51 / 56, and 32 / 32, 16 x 200 57 / 53, 32 / 8 35 / 30, 8 / 1, 64 x 200 + 300 55 / 50.
-static bool wide_pays(int wide, int Hkv, int D, int num_tokens, int num_seqs) {
+// The mean says nothing of a batch of a long prompt among short ones.  Heads of 128, one wide tile of which costs a short prompt some 0.07 us more and a long one
+// saves some 6 us in 1000 tokens, 24 in 2000: us, 4-wave / wide, 32 / 8 heads, a prompt of 2000 with 100 of 10 98 / 85, with 250 of 15 125 / 115, with 500 of 10 217 / 217, with
+// 1000 253 / 293, 1000 with 100 of 8 54.0 / 51.2, with 200 65 / 68, 500 with 100 of 8 54 / 61, 3000 with 400 of 2 184 / 165; 64 / 8, 2000 with 500 of 10 266 / 276, 1000 with 100 of 8
+// 61 / 56; 32 / 32, 1000 with 100 of 8 on 500 279 / 253, with 200 131 / 151, 2000 with 500 of 10 536 / 601, 1500 with 130 136 / 124; 16 / 8, the last 76 / 69.
+// (max_q_len: the longest run where the caller knows it, else 0)
+static bool wide_pays(int wide, int Hkv, int D, int num_tokens, int num_seqs, long max_q_len) {
   if (g_prefill_variant == 3) return true;
   if (g_prefill_variant != 1 || (long)(num_tokens / wide) * Hkv < g_prefill_wide_min_wgs) return false;
   const int mean = num_tokens / max(num_seqs, 1);
-  if (D == 128) return mean >= min(40, wide / 2);
+  const long longest = max_q_len < num_tokens ? max_q_len : num_tokens;
+  if (D == 128) return mean >= min(40, wide / 2) || longest * longest >= 9000L * num_seqs;
   if (D == 96) return mean >= min(64, wide / 2);
   return mean >= 64 && (mean >= 192 || (long)((mean + wide - 1) / wide) * num_seqs * Hkv <= 256);
 }
@@ -1254,17 +1260,21 @@ static bool wide_pays(int wide, int Hkv, int D, int num_tokens, int num_seqs) {
 // many query rows want few parts: their cost grows with the parts as the walk's falls.  The merge is a workgroup a (token, head), of which some
 // 3500 a us start: 32 / 8 heads of 64, prompts of 520, 700 and 1000 tokens, one part / two 20.7 / 22.9, 26.0 / 28.2, 34.4 / 39.8; 14 / 2 heads, three of 500
 // 22.0 / 25.3; 32 / 8 of 128, 300 on 300 30.1 / 27.5, 100 on 450 of each of four 28.6 / 29.5; 16 / 8 of 256, these 35.8 / 31.9.
-VDA_EXPORT int vda_prefill_parts(int num_seqs, int num_tokens, int Hq, int Hkv, int D, long max_keys) {
+// max_q_len: the longest query run where it is known (0: not).  0 parts: the wide form takes the batch.
+VDA_EXPORT int vda_prefill_form(int num_seqs, int num_tokens, int Hq, int Hkv, int D, long max_keys, long max_q_len) {
   if (Hkv < 1 || Hq % Hkv || Hq / Hkv > 128) return 1;
   const int G = Hq / Hkv, q_tile = (G <= prefill_cols(D) ? prefill_cols(D) : 128) / G;
   const int wide = wide_tokens(G, D, num_tokens, num_seqs);
-  if (wide && wide_pays(wide, Hkv, D, num_tokens, num_seqs)) return 1;
+  if (wide && wide_pays(wide, Hkv, D, num_tokens, num_seqs, max_q_len)) return 0;
   const long wgs = (long)(num_tokens / q_tile + min(num_seqs, num_tokens)) * Hkv, steps = (max_keys + 31) / 32;
   if (wgs < 1 || wgs > 256 || steps < 16) return 1;
   const double rows = (double)num_tokens * Hq, row_part = rows * D * 8 / 4e6;                 // us
   const long parts = max(1L, min(min(min(512 / wgs, steps / 8), (long)sqrt(1.2 * steps / row_part) + 1), 64L));
   const double walk = (0.7 + 0.0055 * D) * steps, merge = 4 + rows / 3500 + row_part * parts;
   return walk * (1 - 1.0 / parts) > merge ? (int)parts : 1;
+}
+VDA_EXPORT int vda_prefill_parts(int num_seqs, int num_tokens, int Hq, int Hkv, int D, long max_keys) {
+  return max(vda_prefill_form(num_seqs, num_tokens, Hq, Hkv, D, max_keys, 0), 1);
 }
 
 // Varlen attention of new tokens against the paged cache (the new tokens' own K/V must already be in
@@ -1303,7 +1313,7 @@ VDA_EXPORT int vda_paged_attention_prefill(
   // Its copies to LDS ask for caches aligned to 16 bytes.
   const bool aligned = (((uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0;
   const int wide = wide_tokens(G, D, num_tokens, num_seqs);
-  if (nsplit == 1 && wide && aligned && wide_pays(wide, Hkv, D, num_tokens, num_seqs)) {
+  if (nsplit == 1 && wide && aligned && wide_pays(wide, Hkv, D, num_tokens, num_seqs, max_q_len)) {
     p.q_tile = wide;
     return vda_launch_prefill_wide(p, D, block_size, dtype, kv_fp8, st);
   }

@@ -48,6 +48,7 @@ _SIGS = {
     "vda_paged_attention_prefill": [P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, L, L, F, F, I, I, I, F, F, I, P,
                                     I, P, I, I, P, I, P, P, I, L, P],
     "vda_prefill_parts": [I, I, I, I, I, L],
+    "vda_prefill_form": [I, I, I, I, I, L, L],
     "vda_paged_attention_prefill_sparse": [P] * 13 + [I] * 9 + [L, L, F, F, I, I, F, F, I, P, L, P],
     "vda_set_prefill_variant": [I],
     "vda_int8_quant_azp": [P, P, P, P, P, P, I, I, L, L, I, P],
