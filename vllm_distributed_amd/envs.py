@@ -79,7 +79,7 @@ _REGISTRY: dict[str, tuple[Callable[[str], Any], Any]] = {
     # 16-bit dense layers with this many rows run the weight-streaming split-K MFMA kernel (ops/csrc/gemm_decode.hip)
     "VDA_DECODE_GEMM_MIN_M": (int, 33),
     "VDA_DECODE_GEMM_MAX_M": (int, 0),           # 0 = never (default: the tuned library GEMMs are faster, see docs/kernels.md)
-    "VDA_DECODE_GEMM_WS_MB": (int, 128),         # fp32 split-K workspace per device
+    "VDA_DECODE_GEMM_WS_MB": (int, 128),         # most fp32 sums of one product's K parts
     "VDA_DENSE_GEMM_MAX_M": (int, 192),          # rows up to which 16-bit linears run the in-tree ping-pong MFMA GEMM (0 = never;
                                                  # at 256 rows the library's selected algorithms win inside the engine)
     "VDA_SIGMOID_ATTN_FORM": (str, "auto"),      # sigmoid head-mixing attention: auto | mfma | plain (fp32 arithmetic)

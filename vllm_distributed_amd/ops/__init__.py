@@ -673,15 +673,20 @@ def skinny_gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] =
     return y
 
 
-_DECODE_WS: dict = {}
+_SPLIT_BYTES: Optional[int] = None
 
 
-def _gemm_workspace(device) -> torch.Tensor:
-    """Split-K partial sums; one arena per device, reused by every call (stream order)."""
-    ws = _DECODE_WS.get(device)
-    if ws is None:
-        ws = _DECODE_WS[device] = torch.empty(envs.VDA_DECODE_GEMM_WS_MB << 18, dtype=torch.float32, device=device)
-    return ws
+def _split_bytes() -> int:
+    """The most that the fp32 sums of one product's K parts may take (``VDA_DECODE_GEMM_WS_MB``, read once).  Each call has sums of its own:
+    with those of another stream's or thread's call in the same place, its second launch would add up both."""
+    global _SPLIT_BYTES
+    if _SPLIT_BYTES is None:
+        _SPLIT_BYTES = envs.VDA_DECODE_GEMM_WS_MB << 20
+    return _SPLIT_BYTES
+
+
+def _split_sums(slabs: int, floats: int, device) -> Optional[torch.Tensor]:
+    return torch.empty(slabs * floats, dtype=torch.float32, device=device) if slabs else None
 
 
 def decode_gemm_ok(M: int, N_: int, K: int, dtype: torch.dtype) -> bool:
@@ -706,9 +711,10 @@ def decode_gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] =
         raise ValueError("decode_gemm: x must be [M, K] with unit column stride and w [N, K] contiguous")
     if out is None:
         out = torch.empty((M, N_), dtype=x.dtype, device=x.device)
-    ws = _gemm_workspace(x.device)
-    N.call("vda_decode_gemm", out.data_ptr(), x.data_ptr(), w.data_ptr(), N.ptr(bias), ws.data_ptr(),
-           ws.numel() * 4, M, N_, K, x.stride(0), out.stride(0), N.dt(x.dtype), N.stream())
+    most = _split_bytes()
+    ws = _split_sums(N.value("vda_decode_gemm_slabs", M, N_, K, out.stride(0), most), M * N_, x.device)
+    N.call("vda_decode_gemm", out.data_ptr(), x.data_ptr(), w.data_ptr(), N.ptr(bias), N.ptr(ws),
+           most, M, N_, K, x.stride(0), out.stride(0), N.dt(x.dtype), N.stream())
     return out
 
 
@@ -748,9 +754,10 @@ def dense_gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = 
         raise ValueError("dense_gemm: x must be 16-bit [M, K] (K % 32 == 0), w [N, K] contiguous of the same dtype")
     if out is None:
         out = torch.empty((M, n_out), dtype=x.dtype, device=x.device)
-    ws = _gemm_workspace(x.device)
-    N.call("vda_dense_gemm", out.data_ptr(), x.data_ptr(), w.data_ptr(), N.ptr(bias), N.ptr(residual), ws.data_ptr(),
-           ws.numel() * 4, M, n_out, K, x.stride(0), out.stride(0), residual.stride(0) if residual is not None else 0,
+    most = _split_bytes()
+    ws = _split_sums(N.value("vda_dense_gemm_slabs", M, n_out, K, out.stride(0), epi, wt, splits, variant, 1, most), M * w.shape[0], x.device)
+    N.call("vda_dense_gemm", out.data_ptr(), x.data_ptr(), w.data_ptr(), N.ptr(bias), N.ptr(residual), N.ptr(ws),
+           most, M, n_out, K, x.stride(0), out.stride(0), residual.stride(0) if residual is not None else 0,
            epi, N.dt(x.dtype), wt, splits, variant, 1, 0, 0, 0, N.stream())
     return out
 
@@ -791,8 +798,9 @@ def grouped_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     y = torch.empty((G, M, n_out), dtype=x.dtype, device=x.device)
     if x.is_cuda and M <= min(envs.VDA_DENSE_GEMM_MAX_M, 256) and n_out % 4 == 0 and x.is_contiguous() and w.is_contiguous() \
             and dense_gemm_ok(x[0], w[0]) and w.shape == (G, n_out, K):
-        ws = _gemm_workspace(x.device)
-        N.call("vda_dense_gemm", y.data_ptr(), x.data_ptr(), w.data_ptr(), None, None, ws.data_ptr(), ws.numel() * 4, M, n_out,
+        most = _split_bytes()
+        ws = _split_sums(N.value("vda_dense_gemm_slabs", M, n_out, K, n_out, 0, 0, 0, 0, G, most), G * M * n_out, x.device)
+        N.call("vda_dense_gemm", y.data_ptr(), x.data_ptr(), w.data_ptr(), None, None, N.ptr(ws), most, M, n_out,
                K, K, n_out, 0, 0, N.dt(x.dtype), 0, 0, 0, G, M * K, n_out * K, M * n_out, N.stream())
         return y
     for g in range(G):
@@ -859,7 +867,7 @@ def w4_linear(x: torch.Tensor, qw: torch.Tensor, scales: torch.Tensor, zeros: to
 
 
 # ---- 4-bit code-book weights (bitsandbytes NF4 / FP4, NVFP4) -------------------------------------
-_CB4_WS: dict = {}
+_CB4_FLOATS = 1 << 23                                  # the most of a product's sums of K parts
 
 
 def cb4_chunk_layout_ok(K: int, group: int) -> bool:
@@ -922,12 +930,10 @@ def cb4_linear(x: torch.Tensor, codes: torch.Tensor, scales: torch.Tensor, table
         y = torch.empty((M, N_), dtype=x.dtype, device=x.device)
         if chunked:
             # K splits write slabs of fp32 partial sums that a second small kernel adds (fewer splits if they do not fit)
-            ws = _CB4_WS.get(x.device)
-            if ws is None:
-                ws = _CB4_WS[x.device] = torch.empty(1 << 23, dtype=torch.float32, device=x.device)
+            ws = _split_sums(N.value("vda_cb4_slabs", M, N_, K, _CB4_FLOATS, splits), M * N_, x.device)
             N.call("vda_cb4_skinny_gemm_post", y.data_ptr(), x.data_ptr(), codes.data_ptr(), scales.data_ptr(),
                    table.data_ptr(), N.ptr(bias), M, N_, K, group, int(hi_first), x.stride(0), y.stride(0),
-                   N.dt(x.dtype), ws.data_ptr(), ws.numel(), splits, N.stream())
+                   N.dt(x.dtype), N.ptr(ws), _CB4_FLOATS, splits, N.stream())
         else:
             N.call("vda_cb4_skinny_gemm", y.data_ptr(), x.data_ptr(), codes.data_ptr(), scales.data_ptr(),
                    table.data_ptr(), N.ptr(bias), M, N_, K, group, int(hi_first), x.stride(0), y.stride(0),
@@ -969,11 +975,10 @@ def wq_gemm(x: torch.Tensor, qw: torch.Tensor, sz: torch.Tensor, group: int, bit
     if sz.shape != (K // group, N_, 2) or sz.dtype != x.dtype or not sz.is_contiguous():
         raise ValueError(f"wq_gemm: sz must be contiguous [K/group, N, 2] of {x.dtype}, got {tuple(sz.shape)} {sz.dtype}")
     y = torch.empty((M, N_), dtype=x.dtype, device=x.device)
-    ws = _DECODE_WS.get(x.device)
-    if ws is None:
-        ws = _DECODE_WS[x.device] = torch.empty(envs.VDA_DECODE_GEMM_WS_MB << 18, dtype=torch.float32, device=x.device)
-    N.call("vda_wq_gemm", y.data_ptr(), x.data_ptr(), qw.data_ptr(), sz.data_ptr(), N.ptr(bias), ws.data_ptr(),
-           ws.numel() * 4, M, N_, K, group, bits, x.stride(0), y.stride(0), N.dt(x.dtype), splits, variant, N.stream())
+    most = _split_bytes()
+    ws = _split_sums(N.value("vda_wq_gemm_slabs", M, N_, K, group, bits, N_, most, splits, variant), M * N_, x.device)
+    N.call("vda_wq_gemm", y.data_ptr(), x.data_ptr(), qw.data_ptr(), sz.data_ptr(), N.ptr(bias), N.ptr(ws),
+           most, M, N_, K, group, bits, x.stride(0), y.stride(0), N.dt(x.dtype), splits, variant, N.stream())
     return y
 
 

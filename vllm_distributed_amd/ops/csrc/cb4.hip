@@ -371,22 +371,16 @@ __global__ __launch_bounds__(256) void cb4_finish_kernel(T* __restrict__ y, cons
   *reinterpret_cast<V4*>(y + (long)m * y_stride + n) = o;
 }
 
-// codes in the transposed-chunk layout, scales_t [K / G, N]
-VDA_EXPORT int vda_cb4_skinny_gemm_post(void* y, const void* x, const void* codes, const void* scales_t,
-                                        const void* table, const void* bias, int M, int N, int K, int G, int hi_first,
-                                        long x_stride, long y_stride, int dtype, void* ws, size_t ws_floats,
-                                        int splits, hipStream_t st) {
-  if (M < 1 || M > 64 || N < 16 || N % 16 || K < 128 || K % 128 || K % G) return -1;
-  if (!(G == 32 || G == 64 || (G >= 128 && G % 128 == 0))) return -1;
-  const int mt = (M + 15) / 16;
-  const int gq = G == 32 ? 1 : G == 64 ? 2 : 4;
+// Rows of a workgroup (16 rw) and the parts of K.  ws_floats: the most that the parts' fp32 sums may take (0: one part).
+struct Cb4Plan { int rw, blocks, sk; };
+static Cb4Plan cb4_plan(int M, int N, int K, size_t ws_floats, int splits) {
   // rows per workgroup: as many as keep two workgroups per CU busy (512 of them) and the accumulators in registers
   // (from 8 rows on the activations every workgroup re-reads from L2 outweigh its codes unless it owns 64 rows:
   // narrow layers then take 64-row workgroups too and fill the chip with K splits instead)
   int rw = 1;
   // (layers under 16 MiB of codes finish in about ten microseconds either way: the second launch would cost them more
   // than the wider workgroups gain)
-  const bool wide_rows = N % 32 == 0 && splits == 0 && ws && (size_t)N * K / 2 >= ((size_t)16 << 20);
+  const bool wide_rows = N % 32 == 0 && splits == 0 && ws_floats > 0 && (size_t)N * K / 2 >= ((size_t)16 << 20);
   if (N % 64 == 0 && (N / 64 >= 512 || wide_rows)) rw = 4;
   else if (N % 32 == 0 && (N / 32 >= 512 || wide_rows)) rw = 2;
   // K splits (splits = 0: chosen here): enough workgroups for four per CU, at least 16 chunks each; every split writes
@@ -400,8 +394,29 @@ VDA_EXPORT int vda_cb4_skinny_gemm_post(void* y, const void* x, const void* code
       while (sk < 8 && blocks * sk < 512 && nchunk / (sk * 2) >= 8) sk *= 2;
   }
   if (sk > nchunk) sk = nchunk;
-  while (sk > 1 && (!ws || ws_floats < (size_t)sk * M * N)) --sk;
-  dim3 grid(blocks, sk), block(256);
+  while (sk > 1 && ws_floats < (size_t)sk * M * N) --sk;
+  return {rw, blocks, sk};
+}
+// fp32 slabs of [M, N] that such a product wants as its workspace (0: none)
+VDA_EXPORT int vda_cb4_slabs(int M, int N, int K, size_t ws_floats, int splits) {
+  if (M < 1 || N < 16 || K < 128) return 0;
+  const int n = cb4_plan(M, N, K, ws_floats, splits).sk;
+  return n > 1 ? n : 0;
+}
+
+// codes in the transposed-chunk layout, scales_t [K / G, N].  ws: the sums of K's parts (vda_cb4_slabs says how many, of the same sizes and ws_floats)
+VDA_EXPORT int vda_cb4_skinny_gemm_post(void* y, const void* x, const void* codes, const void* scales_t,
+                                        const void* table, const void* bias, int M, int N, int K, int G, int hi_first,
+                                        long x_stride, long y_stride, int dtype, void* ws, size_t ws_floats,
+                                        int splits, hipStream_t st) {
+  if (M < 1 || M > 64 || N < 16 || N % 16 || K < 128 || K % 128 || K % G) return -1;
+  if (!(G == 32 || G == 64 || (G >= 128 && G % 128 == 0))) return -1;
+  const int mt = (M + 15) / 16;
+  const int gq = G == 32 ? 1 : G == 64 ? 2 : 4;
+  const Cb4Plan plan = cb4_plan(M, N, K, ws_floats, splits);
+  const int rw = plan.rw, sk = plan.sk;
+  if (sk > 1 && !ws) return -1;
+  dim3 grid(plan.blocks, sk), block(256);
 #define L(TT, MM, GG, RR) hipLaunchKernelGGL((cb4_skinny_post_kernel<TT, MM, GG, RR>), grid, block, 0, st, (TT*)y,      \
                                              (const TT*)x, (const uint8_t*)codes, (const float*)scales_t,             \
                                              (const float*)table, (const TT*)bias, M, N, K, G, hi_first, x_stride,    \

@@ -231,9 +231,17 @@ static int launch_decode_gemm(const DecodeGemmArgs& a, int wm, hipStream_t st) {
   return 0;
 }
 
+// fp32 slabs of [M, N] that such a product wants as its workspace (0: none)
+VDA_EXPORT int vda_decode_gemm_slabs(int M, int N, int K, long out_stride, size_t ws_bytes) {
+  if (M < 1 || M > 256 || N < 1 || K < 256 || out_stride % 4) return 0;
+  int steps;
+  const int n = decode_gemm_splits(M, N, K, M > 128 ? 2 : 1, ws_bytes, &steps);
+  return n > 1 ? n : 0;
+}
+
 // x [M, K] (row stride x_stride elements), w [N, K] contiguous, out [M, N] (row stride out_stride);
-// 1 <= M <= 256, K % 256 == 0, strides multiples of 8 elements.  ws: fp32 scratch of ws_bytes (may be null:
-// K is then not split).  dtype VDA_BF16 / VDA_F16.  Returns 0, or a negative code for shapes it does not take.
+// 1 <= M <= 256, K % 256 == 0, strides multiples of 8 elements.  ws: the sums of K's parts (vda_decode_gemm_slabs says how many, of the same
+// sizes and ws_bytes; 0 bytes: K is not split).  dtype VDA_BF16 / VDA_F16.  Returns 0, or a negative code for shapes it does not take.
 VDA_EXPORT int vda_decode_gemm(void* out, const void* x, const void* w, const void* bias, float* ws, size_t ws_bytes,
                                int M, int N, int K, long x_stride, long out_stride, int dtype, hipStream_t st) {
   if (M < 1 || M > 256 || N < 1 || K < 256 || K % 256) return -1;
@@ -243,8 +251,9 @@ VDA_EXPORT int vda_decode_gemm(void* out, const void* x, const void* w, const vo
   DecodeGemmArgs a;
   a.x = x; a.w = w; a.out = out; a.ws = ws; a.bias = bias; a.M = M; a.N = N; a.K = K;
   a.x_stride = x_stride; a.out_stride = out_stride;
-  a.splits = decode_gemm_splits(M, N, K, wm, ws ? ws_bytes : 0, &a.steps_per_split);
+  a.splits = decode_gemm_splits(M, N, K, wm, ws_bytes, &a.steps_per_split);
   if (a.splits > 1 && out_stride % 4) { a.splits = 1; a.steps_per_split = K >> 6; }
+  if (a.splits > 1 && !ws) return -1;
   const int rc = dtype == VDA_BF16 ? launch_decode_gemm<bf16_t>(a, wm, st) : launch_decode_gemm<f16_t>(a, wm, st);
   if (rc) return rc;
   VDA_CHECK_LAUNCH();

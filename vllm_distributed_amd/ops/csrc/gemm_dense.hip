@@ -376,29 +376,14 @@ static int launch_dense_gemm(const DenseGemmArgs& a, int wt, int xt, bool k64, i
   return 0;
 }
 
-// x [M, K] (row stride x_stride elements), w [N or 2 N, K] contiguous, out [M, N] (row stride out_stride), optional
-// bias [N] and residual [M, N] (PLAIN only).  K % 32 == 0; strides multiples of 8 elements; the byte size of x and
-// of w below 4 GiB (32-bit offsets in the copy addresses).  wt / splits: 0 = chosen here (wt 2 or 4: 128 or 256
-// weight rows per tile).  batch > 1 (M <= 256, no bias or residual): so many products of this size, x_batch / w_batch /
-// out_batch elements apart.  ws: fp32 scratch of ws_bytes for split K (may be null: K is then not split).
-// Returns 0, or a negative code for shapes it does not take.
-VDA_EXPORT int vda_dense_gemm(void* out, const void* x, const void* w, const void* bias, const void* residual,
-                              float* ws, size_t ws_bytes, int M, int N, int K, long x_stride, long out_stride,
-                              long res_stride, int epi, int dtype, int wt, int splits, int variant, int batch,
-                              long x_batch, long w_batch, long out_batch, hipStream_t st) {
-  if (M < 1) return M == 0 ? 0 : -1;
-  if (N < 1 || K < 32 || K % 32) return -1;
-  if (x_stride % 8 || (N % 4 && out_stride % 4)) return -1;
-  if (epi != DG_PLAIN && epi != DG_GATE_UP) return -4;
-  if (epi == DG_GATE_UP && (bias || residual || N % 4)) return -4;
-  if (dtype != VDA_BF16 && dtype != VDA_F16) return -3;
-  if (batch < 1 || (batch > 1 && (bias || residual || M > 256 || x_batch % 8 || w_batch % 8 || out_batch % 4))) return -1;
+// How a product is cut.  wt / splits: 0 = chosen here.  ws_bytes: the most that the parts' fp32 sums may take (0: K is not split).
+struct DensePlan { int xt, m_tiles, wt, n_tiles, splits, units_per_split; bool k64; };
+static DensePlan dense_plan(int M, int N, int K, long out_stride, int epi, int wt, int splits, int variant, int batch, size_t ws_bytes) {
   const long w_rows = epi == DG_GATE_UP ? 2L * N : N;
-  if (w_rows * K * 2 >= (1LL << 32) || (long)M * x_stride * 2 >= (1LL << 32)) return -2;
-  int xt = M > 128 ? 8 : M > 64 ? 4 : M > 32 ? 2 : 1;
+  const int xt = M > 128 ? 8 : M > 64 ? 4 : M > 32 ? 2 : 1;
   const int nu = K >> 5;
   const int m_tiles = (M + 32 * xt - 1) / (32 * xt);
-  const bool can_split = !(N % 4 || out_stride % 4 || !ws);
+  const bool can_split = !(N % 4 || out_stride % 4 || ws_bytes == 0);
   // Tile height and K split, when the caller leaves them open: the pair with the smaller estimated time.  A
   // workgroup streams (64 wt weight rows + 32 xt activation rows) x 64 bytes per unit; weight rows come from HBM at
   // about 24 GB/s per CU, activation rows from L2 (a sixteenth of that per row); a split adds the reduction
@@ -429,23 +414,51 @@ VDA_EXPORT int vda_dense_gemm(void* out, const void* x, const void* w, const voi
   double unused;
   splits = plan(wt, splits, &unused);
   const int ncol = epi == DG_GATE_UP ? 32 * wt : 64 * wt;
+  // variant: 0 = chosen here, 1 = ring of 32-element units, 2 = 64-element units (256 x 256 tiles, K % 64 == 0)
+  const bool k64 = (variant == 2 || (variant == 0 && m_tiles > 1)) && xt == 8 && wt == 4 && K % 64 == 0;
+  int units = (nu + splits - 1) / splits;
+  if (k64) units = (units + 1) & ~1;                   // whole 64-element units per split
+  return {xt, m_tiles, wt, (N + ncol - 1) / ncol, (nu + units - 1) / units, units, k64};
+}
+// fp32 slabs of [batch, M, rows of w] that such a product wants as its workspace (0: none)
+VDA_EXPORT int vda_dense_gemm_slabs(int M, int N, int K, long out_stride, int epi, int wt, int splits, int variant, int batch, size_t ws_bytes) {
+  if (M < 1 || N < 1 || K < 32 || batch < 1) return 0;
+  const int n = dense_plan(M, N, K, out_stride, epi, wt, splits, variant, batch, ws_bytes).splits;
+  return n > 1 ? n : 0;
+}
+
+// x [M, K] (row stride x_stride elements), w [N or 2 N, K] contiguous, out [M, N] (row stride out_stride), optional
+// bias [N] and residual [M, N] (PLAIN only).  K % 32 == 0; strides multiples of 8 elements; the byte size of x and
+// of w below 4 GiB (32-bit offsets in the copy addresses).  wt / splits: 0 = chosen here (wt 2 or 4: 128 or 256
+// weight rows per tile).  batch > 1 (M <= 256, no bias or residual): so many products of this size, x_batch / w_batch /
+// out_batch elements apart.  ws: the sums of K's parts (vda_dense_gemm_slabs says how many, of
+// the same sizes and ws_bytes; 0 bytes: K is not split).
+// Returns 0, or a negative code for shapes it does not take.
+VDA_EXPORT int vda_dense_gemm(void* out, const void* x, const void* w, const void* bias, const void* residual,
+                              float* ws, size_t ws_bytes, int M, int N, int K, long x_stride, long out_stride,
+                              long res_stride, int epi, int dtype, int wt, int splits, int variant, int batch,
+                              long x_batch, long w_batch, long out_batch, hipStream_t st) {
+  if (M < 1) return M == 0 ? 0 : -1;
+  if (N < 1 || K < 32 || K % 32) return -1;
+  if (x_stride % 8 || (N % 4 && out_stride % 4)) return -1;
+  if (epi != DG_PLAIN && epi != DG_GATE_UP) return -4;
+  if (epi == DG_GATE_UP && (bias || residual || N % 4)) return -4;
+  if (dtype != VDA_BF16 && dtype != VDA_F16) return -3;
+  if (batch < 1 || (batch > 1 && (bias || residual || M > 256 || x_batch % 8 || w_batch % 8 || out_batch % 4))) return -1;
+  const long w_rows = epi == DG_GATE_UP ? 2L * N : N;
+  if (w_rows * K * 2 >= (1LL << 32) || (long)M * x_stride * 2 >= (1LL << 32)) return -2;
+  const DensePlan plan = dense_plan(M, N, K, out_stride, epi, wt, splits, variant, batch, ws_bytes);
+  if (plan.splits > 1 && !ws) return -1;
   DenseGemmArgs a;
   a.out = out; a.x = x; a.w = w; a.bias = bias; a.residual = residual; a.ws = ws;
   a.M = M; a.N = N; a.K = K; a.x_stride = x_stride; a.out_stride = out_stride; a.res_stride = res_stride;
   a.x_batch = x_batch; a.w_batch = w_batch; a.out_batch = out_batch;
-  a.m_tiles = m_tiles;
-  a.n_tiles = (N + ncol - 1) / ncol;
-  // variant: 0 = chosen here, 1 = ring of 32-element units, 2 = 64-element units (256 x 256 tiles, K % 64 == 0)
-  const bool k64 = variant == 2 || (variant == 0 && a.m_tiles > 1);
-  const bool use_k64 = k64 && xt == 8 && wt == 4 && K % 64 == 0;
-  a.units_per_split = (nu + splits - 1) / splits;
-  if (use_k64) a.units_per_split = (a.units_per_split + 1) & ~1;       // whole 64-element units per split
-  a.splits = (nu + a.units_per_split - 1) / a.units_per_split;
+  a.m_tiles = plan.m_tiles; a.n_tiles = plan.n_tiles; a.splits = plan.splits; a.units_per_split = plan.units_per_split;
   int rc;
-  if (dtype == VDA_BF16) rc = epi == DG_GATE_UP ? launch_dense_gemm<bf16_t, DG_GATE_UP>(a, wt, xt, use_k64, batch, st)
-                                                : launch_dense_gemm<bf16_t, DG_PLAIN>(a, wt, xt, use_k64, batch, st);
-  else rc = epi == DG_GATE_UP ? launch_dense_gemm<f16_t, DG_GATE_UP>(a, wt, xt, use_k64, batch, st)
-                              : launch_dense_gemm<f16_t, DG_PLAIN>(a, wt, xt, use_k64, batch, st);
+  if (dtype == VDA_BF16) rc = epi == DG_GATE_UP ? launch_dense_gemm<bf16_t, DG_GATE_UP>(a, plan.wt, plan.xt, plan.k64, batch, st)
+                                                : launch_dense_gemm<bf16_t, DG_PLAIN>(a, plan.wt, plan.xt, plan.k64, batch, st);
+  else rc = epi == DG_GATE_UP ? launch_dense_gemm<f16_t, DG_GATE_UP>(a, plan.wt, plan.xt, plan.k64, batch, st)
+                              : launch_dense_gemm<f16_t, DG_PLAIN>(a, plan.wt, plan.xt, plan.k64, batch, st);
   if (rc) return rc;
   VDA_CHECK_LAUNCH();
   return 0;

@@ -900,10 +900,76 @@ static bool wq_tiles_pay(int M, int N, int K, int bits, int group, bool no_split
   return !wq_unscaled(N, bits, group);
 }
 
+// Which kernel takes a product, and in how many parts of K.  ws_bytes: the most that the parts' fp32 sums may take (0: one part).
+struct WqPlan {
+  enum { SLICES, STREAM, TILES } kernel;
+  int nt, m_tiles, n_tiles, splits, units_per_split;
+};
+// log2(group / 32) of a power of two, 30 of one group, else -1
+static int wq_group_shift(int K, int group) {
+  if (group == K) return 30;
+  for (int sh = 0; sh < 16; ++sh)
+    if (group == (32 << sh)) return sh;
+  return -1;
+}
+// Returns 0, or a negative code for shapes that are not taken.
+static int wq_plan(WqPlan& p, int M, int N, int K, int group, int bits, long out_stride, size_t ws_bytes, int splits, int variant) {
+  if (M < 1 || N < 1 || K < 32 || K % 32 || group < 32 || group % 32 || K % group || (bits != 4 && bits != 8)) return -1;
+  const bool can_stream = M <= 128 && K % 128 == 0 && wq_group_shift(K, group) >= 0;
+  const bool streams = variant == 2 || variant == 3;
+  if (streams && !can_stream) return -1;
+  const bool no_split = N % 4 || out_stride % 4 || ws_bytes == 0;
+  int units;
+  p.nt = 0;
+  if (streams || (variant == 0 && can_stream && !wq_tiles_pay(M, N, K, bits, group, no_split))) {
+    const int groups = (N + 127) / 128, parts = wq_parts(M, N, K, bits);
+    p.kernel = WqPlan::STREAM;
+    p.m_tiles = 1;
+    p.n_tiles = groups;
+    units = K >> 7;
+    // (layers that the kernel below takes in one part with a workgroup on most CUs lead there at any number of rows: 28672 x 4096 in 8 bits, 4, 8
+    // and 13 rows, slices 31.9, 35.0 and 38.1 us, this 30.1, 30.6 and 31.2; with 172 of them, 22016 x 4096, slices 24.9, 26.9 and 29.3, this
+    // 29.0, 29.4 and 29.9)
+    const bool whole = parts == 1 && groups >= 224 && groups <= 256 && wq_unscaled_or_8(N, bits, group);
+    if (variant == 0 && splits < 1 && !whole && wq_slices_pay(M, N, K, bits, group, no_split)) {
+      p.kernel = WqPlan::SLICES;
+      splits = 1;
+    }
+    if (splits < 1) splits = parts;
+  } else {
+    p.kernel = WqPlan::TILES;
+    p.m_tiles = (M + 255) / 256;
+    p.nt = ((M + p.m_tiles - 1) / p.m_tiles + 31) / 32;
+    p.n_tiles = (N + 255) / 256;
+    units = (K + 63) >> 6;
+    if (splits < 1) {
+      const long tiles = (long)p.m_tiles * p.n_tiles;
+      const double unit = 0.4 + 0.16 * p.nt;
+      double best = 1e30;
+      for (int s = 1; s <= min(16, max(units / 4, 1)); ++s) {
+        const double t = (double)((tiles * s + 255) / 256) * ((units + s - 1) / s * unit + 2) + (s > 1 ? 5 + s * (double)M * N * 8 / 4e6 : 0);
+        if (t < best) { best = t; splits = s; }
+      }
+    }
+  }
+  splits = min(splits, units);
+  if (no_split) splits = 1;
+  while (splits > 1 && (size_t)splits * M * N * sizeof(float) > ws_bytes) --splits;
+  p.units_per_split = (units + splits - 1) / splits;
+  p.splits = (units + p.units_per_split - 1) / p.units_per_split;
+  return 0;
+}
+// fp32 slabs of [M, N] that such a product wants as its workspace (0: none)
+VDA_EXPORT int vda_wq_gemm_slabs(int M, int N, int K, int group, int bits, long out_stride, size_t ws_bytes, int splits, int variant) {
+  WqPlan p;
+  return wq_plan(p, M, N, K, group, bits, out_stride, ws_bytes, splits, variant) == 0 && p.splits > 1 ? p.splits : 0;
+}
+
 // x [M, K] 16-bit (row stride x_stride elements), qw packed [N, K] (bits 4 or 8), sz [K / group, N, 2] of x's type,
 // out [M, N].  K % 32 == 0, group % 32 == 0 and K % group == 0, N % 4 == 0 for split K.  variant: 0 picks by shape,
 // 1 the tiled kernel, 2 the streaming kernel (M <= 128, K % 128 == 0, group a power of two or K), 3 the streaming
-// kernel in its per-element form.  Returns 0 or a negative code for shapes it does not take.
+// kernel in its per-element form.  ws: the sums of K's parts (vda_wq_gemm_slabs says how many, of the same sizes and ws_bytes).  Returns 0
+// or a negative code for shapes it does not take.
 VDA_EXPORT int vda_wq_gemm(void* out, const void* x, const void* qw, const void* sz, const void* bias, float* ws,
                            size_t ws_bytes, int M, int N, int K, int group, int bits, long x_stride, long out_stride,
                            int dtype, int splits, int variant, hipStream_t st) {
@@ -918,62 +984,22 @@ VDA_EXPORT int vda_wq_gemm(void* out, const void* x, const void* qw, const void*
   a.out = out; a.x = x; a.w = qw; a.bias = bias; a.residual = nullptr; a.ws = ws;
   a.M = M; a.N = N; a.K = K; a.x_stride = x_stride; a.out_stride = out_stride; a.res_stride = 0;
   wa.sz = sz; wa.group = group;
-  wa.gshift = -1;
-  if (group == K) wa.gshift = 30;
-  else
-    for (int sh = 0; sh < 16; ++sh) if (group == (32 << sh)) wa.gshift = sh;
+  wa.gshift = wq_group_shift(K, group);
   wa.group_magic = group == 32 ? 0u : (unsigned)(((1ull << 32) + group / 32 - 1) / (group / 32));
-  const bool can_stream = M <= 128 && K % 128 == 0 && wa.gshift >= 0;
+  WqPlan plan;
+  const int code = wq_plan(plan, M, N, K, group, bits, out_stride, ws_bytes, splits, variant);
+  if (code) return code;
+  if (plan.splits > 1 && !ws) return -1;
   wa.per_element = variant == 3;
-  if (variant == 3) variant = 2;
-  if (variant == 2 && !can_stream) return -1;
-  const bool no_split = N % 4 || out_stride % 4 || !ws;
+  a.m_tiles = plan.m_tiles; a.n_tiles = plan.n_tiles; a.splits = plan.splits; a.units_per_split = plan.units_per_split;
   int rc;
-  if (variant == 2 || (variant == 0 && can_stream && !wq_tiles_pay(M, N, K, bits, group, no_split))) {
-    const int nk = K >> 7;
-    const int groups = (N + 127) / 128;
-    const int parts = wq_parts(M, N, K, bits);
-    // (layers that the kernel below takes in one part with a workgroup on most CUs lead there at any number of rows: 28672 x 4096 in 8 bits, 4, 8
-    // and 13 rows, slices 31.9, 35.0 and 38.1 us, this 30.1, 30.6 and 31.2; with 172 of them, 22016 x 4096, slices 24.9, 26.9 and 29.3, this
-    // 29.0, 29.4 and 29.9)
-    const bool whole = parts == 1 && groups >= 224 && groups <= 256 && wq_unscaled_or_8(N, bits, group);
-    if (variant == 0 && splits < 1 && !whole && wq_slices_pay(M, N, K, bits, group, no_split)) {
-      rc = dtype == VDA_BF16 ? (bits == 4 ? launch_wq_slices<bf16_t, 4>(wa, st) : launch_wq_slices<bf16_t, 8>(wa, st))
-                             : (bits == 4 ? launch_wq_slices<f16_t, 4>(wa, st) : launch_wq_slices<f16_t, 8>(wa, st));
-      VDA_CHECK_LAUNCH();
-      return rc;
-    }
-    if (splits < 1) splits = parts;
-    splits = min(splits, nk);
-    if (no_split) splits = 1;
-    while (splits > 1 && (size_t)splits * M * N * sizeof(float) > ws_bytes) --splits;
-    a.units_per_split = (nk + splits - 1) / splits;
-    a.splits = (nk + a.units_per_split - 1) / a.units_per_split;
-    a.m_tiles = 1; a.n_tiles = groups;
-    if (dtype == VDA_BF16) rc = bits == 4 ? launch_wq_stream<bf16_t, 4>(wa, st) : launch_wq_stream<bf16_t, 8>(wa, st);
-    else rc = bits == 4 ? launch_wq_stream<f16_t, 4>(wa, st) : launch_wq_stream<f16_t, 8>(wa, st);
-  } else {
-    a.m_tiles = (M + 255) / 256;
-    const int nt = ((M + a.m_tiles - 1) / a.m_tiles + 31) / 32;
-    a.n_tiles = (N + 255) / 256;
-    const int nu = (K + 63) >> 6;
-    if (splits < 1) {
-      const long tiles = (long)a.m_tiles * a.n_tiles;
-      const double unit = 0.4 + 0.16 * nt;
-      double best = 1e30;
-      for (int s = 1; s <= min(16, max(nu / 4, 1)); ++s) {
-        const double t = (double)((tiles * s + 255) / 256) * ((nu + s - 1) / s * unit + 2) + (s > 1 ? 5 + s * (double)M * N * 8 / 4e6 : 0);
-        if (t < best) { best = t; splits = s; }
-      }
-    }
-    splits = min(splits, nu);
-    if (no_split) splits = 1;
-    while (splits > 1 && (size_t)splits * M * N * sizeof(float) > ws_bytes) --splits;
-    a.units_per_split = (nu + splits - 1) / splits;
-    a.splits = (nu + a.units_per_split - 1) / a.units_per_split;
-    if (dtype == VDA_BF16) rc = bits == 4 ? launch_wq_tile<bf16_t, 4>(wa, nt, st) : launch_wq_tile<bf16_t, 8>(wa, nt, st);
-    else rc = bits == 4 ? launch_wq_tile<f16_t, 4>(wa, nt, st) : launch_wq_tile<f16_t, 8>(wa, nt, st);
-  }
+#define BY_TYPE(LAUNCH, ...)                                                                                            \
+  (dtype == VDA_BF16 ? (bits == 4 ? LAUNCH<bf16_t, 4>(__VA_ARGS__) : LAUNCH<bf16_t, 8>(__VA_ARGS__))                       \
+                     : (bits == 4 ? LAUNCH<f16_t, 4>(__VA_ARGS__) : LAUNCH<f16_t, 8>(__VA_ARGS__)))
+  if (plan.kernel == WqPlan::SLICES) rc = BY_TYPE(launch_wq_slices, wa, st);
+  else if (plan.kernel == WqPlan::STREAM) rc = BY_TYPE(launch_wq_stream, wa, st);
+  else rc = BY_TYPE(launch_wq_tile, wa, plan.nt, st);
+#undef BY_TYPE
   if (rc) return rc;
   VDA_CHECK_LAUNCH();
   return 0;

@@ -91,6 +91,10 @@ _SIGS = {
     "vda_ep_prep": [P, I, I, I, P, P, P, P, P, P],
     "vda_tile_gemm": [P, P, P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, L, L, L, I, I, I, I, I, I, F, P],
     "vda_decode_gemm": [P, P, P, P, P, L, I, I, I, L, L, I, P],
+    "vda_decode_gemm_slabs": [I, I, I, L, L],
+    "vda_dense_gemm_slabs": [I, I, I, L, I, I, I, I, I, L],
+    "vda_wq_gemm_slabs": [I, I, I, I, I, L, L, I, I],
+    "vda_cb4_slabs": [I, I, I, L, I],
     "vda_wq_gemm": [P, P, P, P, P, P, L, I, I, I, I, I, L, L, I, I, I, P],
     "vda_dense_gemm_stamp": [P, P, P, I, I, I, I, P],
     "vda_dense_gemm": [P, P, P, P, P, P, L, I, I, I, L, L, L, I, I, I, I, I, I, L, L, L, P],
