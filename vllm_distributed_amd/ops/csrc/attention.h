@@ -74,5 +74,5 @@ struct SparseSel {
 };
 
 // Wide prefill form (attention_prefill.hip): 512 threads, 256 query columns per workgroup, heads of 64, 96 (16-bit caches) and 128 values.
-// Returns -100 when the shape is outside what that kernel serves (the caller then takes the 4-wave form).
+// Returns 0, -2 for a page size or -3 for a head size or cache type that it is not built for; the caller passes that on (the 4-wave form has the same).
 int vda_launch_prefill_wide(const AttnParams& p, int D, int block_size, int dtype, int kv_fp8, hipStream_t st);

@@ -322,7 +322,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_kernel(AttnParams p) 
   // batch's; e4m3 33.4 / 30.2).
   const int kvh = blockIdx.x, part = blockIdx.y;
   int seq = blockIdx.z;
-  // (the pages of the first steps, in the same trip: read(), below)
+  // (the pages of the first steps, asked for in the same trip; load_k and load_v below read them)
   int page_k[DEPTH], page_v[DEPTH];
   auto pages_ahead = [&] {
     if (p.table_cols <= 0) return;

@@ -258,7 +258,6 @@ VDA_EXPORT int vda_moe_topk_softmax(float* topk_w, int* topk_id, const void* log
 }
 
 // ---------------------------------------------------------------------------------------------
-// ---------------------------------------------------------------------------------------------
 // Pairs sorted by expert, and the table of m-tiles: for expert e with c rows, ceil(c / rows) tiles; with rows == 256 (the wide tiles) the
 // fewest of at most WIDE_ROWS, of like sizes in 32 rows.  ids[p] in [0, E) or negative (the expert lives on another rank); E <= 1024.
 // Up to ALIGN_ONE pairs one workgroup does it all: it counts in LDS, gathers there (scattered words would leave for memory one line each) and
